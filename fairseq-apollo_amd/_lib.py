@@ -12,6 +12,7 @@ import os
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libmega_hip.so")
+HOST_PATH = os.path.join(HERE, "mega_host.so")
 
 F32, BF16, F16 = 0, 1, 2
 
@@ -45,6 +46,11 @@ SIGNATURES = {
                                   _p, _i64, _i64, _i64, _i64, _p]),
     "mega_norm_ema_steps": (_int, [_p, _p, _p, _int, _i64, _p, _p, _p, _p, _p, _p, _p, _p, C.c_double, _p, _p, _p, _int,
                                    _p, _p, _p, _i64, _i64, _i64, _i64, _p]),
+    "mega_norm_token": (_int, [_p, _p, _int, _p, _p, _p, _p, _p, _p, _p, _p, _p, C.c_double, _i64, _i64, _i64, _p]),
+    "mega_token_linear": (_int, [_p, _int, _i64, _p]),
+    "mega_token_embed": (_int, [_p, _p, _int, C.c_double, _i64, _i64, _i64, _i64, _p, _p, _p]),
+    "mega_token_attention_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64, _i64]),
+    "mega_token_gated_attention": (_int, [_p, _p]),
     "mega_norm_ema_fwd_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64]),
     "mega_norm_ema_fwd_scratch_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64]),
     "mega_norm_ema_fwd": (_int, [_p, _p, _p, _int, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, C.c_double, _p, _p, _p,
@@ -131,6 +137,25 @@ def load() -> C.CDLL:
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+_host = None
+
+
+def load_host():
+    """The extension of native host code (csrc/host.cpp), loaded once; raise if it has not been built."""
+    global _host
+    if _host is None:
+        import importlib.util
+
+        load()                                   # libmega_hip.so, which the extension links against
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(f"{HOST_PATH} is missing: build it with `python fairseq-apollo_amd/build.py`")
+        spec = importlib.util.spec_from_file_location("mega_host", HOST_PATH)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        _host = mod
+    return _host
 
 
 def check(rc: int, what: str) -> None:

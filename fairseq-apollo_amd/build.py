@@ -12,6 +12,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libmega_hip.so")
+HOST = os.path.join(HERE, "mega_host.so")
 
 SOURCES = [
     "capi.hip",
@@ -24,6 +25,7 @@ SOURCES = [
     "ema_rows.hip",
     "ema_bwd.hip", "ema_bwd_tile.hip",
     "decode.hip",
+    "decode_layer.hip",
     "elementwise.hip",
     "gate_glue.hip",
     "attention.hip",
@@ -89,7 +91,26 @@ def build_library(verbose: bool = True, jobs: int = 8) -> str:
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
+    build_host(verbose)
     return LIB
+
+
+def build_host(verbose: bool = True) -> str:
+    """The Python extension of native host code (csrc/host.cpp): C++ against torch's headers, no device code; it
+    finds libmega_hip.so beside itself."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    tlib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[f"-I{d}" for d in (*include_paths(), sysconfig.get_paths()["include"])], os.path.join(CSRC, "host.cpp"), "-o", HOST,
+           f"-L{HERE}", "-l:libmega_hip.so", f"-L{tlib}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.check_call(cmd)
+    return HOST
 
 
 if __name__ == "__main__":

@@ -87,6 +87,13 @@ bool audit_use(const void* p, size_t bytes, const char* what);
 // Clears `bytes` (a multiple of 4) with a small kernel (elementwise.hip).  Used instead of a memset
 // node so that a caller may record any entry point into a HIP graph.
 void zero_async(void* p, size_t bytes, hipStream_t s);
+// One token through TimestepNorm and the moving average's state update with an optional padding mask [B] (decode.hip);
+// shapes mega_norm_ema_step's vector kernel takes.
+int norm_ema_token(const void* x, void* xn, void* y, int dtype, const uint8_t* mask, const int64_t* prev_count,
+                   const float* prev_mean, const float* prev_var, int64_t* count, float* mean, float* var,
+                   const float* norm_gamma, const float* norm_beta, double eps, const float* p, const float* q,
+                   const float* gamma, const float* omega, const float* h_in, float* h_out, int64_t B, int64_t D,
+                   int64_t G, int64_t N, hipStream_t s);
 static inline size_t align_up(size_t a, size_t b) { return (a + b - 1) / b * b; }
 // do the byte ranges [a, a + na) and [b, b + nb) share a byte?
 static inline bool ranges_overlap(const void* a, size_t na, const void* b, size_t nb) {

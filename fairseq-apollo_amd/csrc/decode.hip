@@ -30,6 +30,7 @@ struct StepArgs {
   const float* omega;    // [D]
   const float* h_in;     // [B, D, N, 2] or null
   float* h_out;
+  const uint8_t* mask = nullptr;   // [B], non-zero at padding, or null (vector kernel only)
   int B, D, G, N;
   int K;                 // tokens per stream in this launch (the multi-token kernel)
   int MB;                // tokens per batch staged in LDS
@@ -44,6 +45,55 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   float t = 0.f;
   for (int i = 0; i < kT / 64; ++i) t += red[i];
   return t;
+}
+
+struct StepStats {
+  float mean, var, rstd;
+};
+// One wave folds a token's group of dg channels into the carried statistics (weight 1 against the count): group mean,
+// centred second moment, WelfordCombine.  Up to 512 channels stay in registers between the two passes.
+template <typename T>
+__device__ __forceinline__ StepStats step_stats(const T* xr, int dg, int lane, int64_t c0, float u0, float v0, float eps,
+                                                bool padded) {
+  auto sum64 = [](float v) {
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m);
+    return v;
+  };
+  constexpr int NX = 8;
+  float x[NX];
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < NX; ++i) {
+    x[i] = 0.f;
+    if (i * 64 < dg && i * 64 + lane < dg) x[i] = to_float(xr[i * 64 + lane]);
+    s += x[i];
+  }
+  for (int f = NX * 64 + lane; f < dg; f += 64) s += to_float(xr[f]);
+  const float gm = sum64(s) / (float)dg;
+  float s2 = 0.f;
+#pragma unroll
+  for (int i = 0; i < NX; ++i) {
+    const float d = i * 64 + lane < dg ? x[i] - gm : 0.f;
+    s2 = fmaf(d, d, s2);
+  }
+  for (int f = NX * 64 + lane; f < dg; f += 64) {
+    const float d = to_float(xr[f]) - gm;
+    s2 = fmaf(d, d, s2);
+  }
+  const float gv = sum64(s2) / (float)dg;
+  StepStats r;
+  if (padded) {
+    r.mean = u0;
+    r.var = v0;
+  } else {
+    const float c1 = (float)c0 / (float)(c0 + 1), c2 = 1.0f / (float)(c0 + 1);
+    const float dl = gm - u0;
+    r.mean = c1 * u0 + c2 * gm;
+    r.var = c1 * v0 + c2 * gv + (c1 * dl) * (c2 * dl);
+  }
+  r.rstd = 1.0f / sqrtf(r.var + eps);
+  return r;
 }
 
 template <typename T, bool CPLX>
@@ -107,82 +157,114 @@ __global__ __launch_bounds__(kT) void norm_ema_step_kernel(const StepArgs A) {
 // Same step with the state streamed as 32-byte pieces: NP = N / 4 adjacent lanes own one channel,
 // each lane four states (two 16-byte loads of h, q, gamma, one of p), so a wave reads and writes
 // the state as one contiguous 2 KB block; the output sum is finished across the NP lanes.
+// What bounds the step is the state's way through memory, so its loads (and the coefficients') are issued before
+// anything else: the group's moments (every wave for itself, no workgroup barrier, the values kept in registers
+// for the centred second pass) are formed under them.  64 streams x 2048 channels x 16 states: 10.0 us, 3.4 TB/s of
+// state (the same as with the moments in front and two workgroup barriers: enough workgroups share a CU to hide
+// either order); one stream of 1024 channels: 4.2 us.
 constexpr int kTV = 256;
+constexpr int kStepIT = 2;             // channel parts a thread has in flight: 512 = the 128 channels of a group at N = 16
 
 template <typename T, int NP>
 __global__ __launch_bounds__(kTV) void norm_ema_step_vec_kernel(const StepArgs A) {
-  __shared__ float red[kTV / 64];
   const int g = blockIdx.x % A.G, b = blockIdx.x / A.G;
   const int dg = A.D / A.G;
+  const int lane = threadIdx.x & 63;
   const T* xr = (const T*)A.x + (size_t)b * A.D + (size_t)g * dg;
+  const int items = dg * NP;                     // a multiple of NP, so the lanes of a channel stay together
+  float4 h0[kStepIT], h1[kStepIT], q0[kStepIT], q1[kStepIT], g0[kStepIT], g1[kStepIT], pp[kStepIT];
+  float xi[kStepIT], nw[kStepIT], nb[kStepIT], om[kStepIT];
+  auto load_items = [&](int it0) {
+#pragma unroll
+    for (int i = 0; i < kStepIT; ++i) {
+      const int it = it0 + i * kTV + threadIdx.x;
+      if (it0 + i * kTV >= items) break;         // uniform
+      const int f = it < items ? it / NP : 0, part = it % NP;
+      const int d = g * dg + f;
+      const size_t ho = (((size_t)b * A.D + d) * A.N + 4 * part) * 2;
+      const size_t co = (size_t)d * A.N + 4 * part;
+      h0[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+      h1[i] = h0[i];
+      if (A.h_in) {
+        h0[i] = *(const float4*)(A.h_in + ho);
+        h1[i] = *(const float4*)(A.h_in + ho + 4);
+      }
+      q0[i] = *(const float4*)(A.q + co * 2);
+      q1[i] = *(const float4*)(A.q + co * 2 + 4);
+      g0[i] = *(const float4*)(A.g + co * 2);
+      g1[i] = *(const float4*)(A.g + co * 2 + 4);
+      pp[i] = *(const float4*)(A.p + co);
+      xi[i] = to_float(xr[f]);
+      nw[i] = A.nw[d];
+      nb[i] = A.nb[d];
+      om[i] = A.omega[d];
+    }
+  };
+  load_items(0);
   const int64_t c0 = A.prev_count[b];
   const float u0 = A.prev_mean[(size_t)b * A.G + g], v0 = A.prev_var[(size_t)b * A.G + g];
-  auto wg_sum = [&](float v) {
-    for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    float t = 0.f;
-    for (int i = 0; i < kTV / 64; ++i) t += red[i];
-    return t;
-  };
-  float s = 0.f;
-  for (int f = threadIdx.x; f < dg; f += kTV) s += to_float(xr[f]);
-  const float gm = wg_sum(s) / (float)dg;
-  float s2 = 0.f;
-  for (int f = threadIdx.x; f < dg; f += kTV) {
-    const float d = to_float(xr[f]) - gm;
-    s2 += d * d;
-  }
-  const float gv = wg_sum(s2) / (float)dg;
-  const float c1 = (float)c0 / (float)(c0 + 1), c2 = 1.0f / (float)(c0 + 1);
-  const float dl = gm - u0;
-  const float u1 = c1 * u0 + c2 * gm;
-  const float v1 = c1 * v0 + c2 * gv + (c1 * dl) * (c2 * dl);
-  const float rstd = 1.0f / sqrtf(v1 + A.eps);
-  __syncthreads();                               // every thread has read the old state
-  if (threadIdx.x == 0) {
-    A.mean[(size_t)b * A.G + g] = u1;
-    A.var[(size_t)b * A.G + g] = v1;
-    if (g == 0) A.count[b] = c0 + 1;
-  }
-  const int items = dg * NP;                     // a multiple of NP, so the lanes of a channel stay together
-  for (int it0 = 0; it0 < items; it0 += kTV) {
-    const int it = it0 + threadIdx.x;
-    const bool ok = it < items;
-    const int f = ok ? it / NP : 0, part = it % NP;
-    const int d = g * dg + f;
-    const size_t o = (size_t)b * A.D + d;
-    const float xnv_full = (to_float(xr[f]) - u1) * rstd * A.nw[d] + A.nb[d];
-    const T xn_t = from_float<T>(xnv_full);
-    const float xv = to_float(xn_t);             // the moving average sees the rounded activation
-    const size_t ho = (o * A.N + 4 * part) * 2;
-    const size_t co = (size_t)d * A.N + 4 * part;
-    float4 h0 = make_float4(0.f, 0.f, 0.f, 0.f), h1 = h0;
-    if (A.h_in) {
-      h0 = *(const float4*)(A.h_in + ho);
-      h1 = *(const float4*)(A.h_in + ho + 4);
-    }
-    const float4 q0 = *(const float4*)(A.q + co * 2), q1 = *(const float4*)(A.q + co * 2 + 4);
-    const float4 g0 = *(const float4*)(A.g + co * 2), g1 = *(const float4*)(A.g + co * 2 + 4);
-    const float4 pp = *(const float4*)(A.p + co);
-    float4 n0, n1;
-    n0.x = q0.x * h0.x - q0.y * h0.y + pp.x * xv;  n0.y = q0.x * h0.y + q0.y * h0.x;
-    n0.z = q0.z * h0.z - q0.w * h0.w + pp.y * xv;  n0.w = q0.z * h0.w + q0.w * h0.z;
-    n1.x = q1.x * h1.x - q1.y * h1.y + pp.z * xv;  n1.y = q1.x * h1.y + q1.y * h1.x;
-    n1.z = q1.z * h1.z - q1.w * h1.w + pp.w * xv;  n1.w = q1.z * h1.w + q1.w * h1.z;
-    float acc = (g0.x * n0.x - g0.y * n0.y) + (g0.z * n0.z - g0.w * n0.w) + (g1.x * n1.x - g1.y * n1.y) +
-                (g1.z * n1.z - g1.w * n1.w);
+  const bool padded = A.mask != nullptr && A.mask[b] != 0;
+  const StepStats st = step_stats(xr, dg, lane, c0, u0, v0, A.eps, padded);
+  for (int it0 = 0; it0 < items; it0 += kTV * kStepIT) {
+    if (it0 > 0) load_items(it0);
 #pragma unroll
-    for (int m = 1; m < NP; m <<= 1) acc += __shfl_xor(acc, m);
-    if (ok) {
-      *(float4*)(A.h_out + ho) = n0;
-      *(float4*)(A.h_out + ho + 4) = n1;
-      if (part == 0) {
-        ((T*)A.xn)[o] = xn_t;
-        ((T*)A.y)[o] = from_float<T>(acc + A.omega[d] * xv);
+    for (int i = 0; i < kStepIT; ++i) {
+      const int it = it0 + i * kTV + threadIdx.x;
+      if (it0 + i * kTV >= items) break;         // uniform
+      const bool ok = it < items;
+      const int f = ok ? it / NP : 0, part = it % NP;
+      const size_t o = (size_t)b * A.D + g * dg + f;
+      const size_t ho = (o * A.N + 4 * part) * 2;
+      // a padded token leaves as zeros and adds nothing to the state
+      const T xn_t = from_float<T>(padded ? 0.f : (xi[i] - st.mean) * st.rstd * nw[i] + nb[i]);
+      const float xv = to_float(xn_t);           // the moving average sees the rounded activation
+      float4 n0, n1;
+      n0.x = q0[i].x * h0[i].x - q0[i].y * h0[i].y + pp[i].x * xv;  n0.y = q0[i].x * h0[i].y + q0[i].y * h0[i].x;
+      n0.z = q0[i].z * h0[i].z - q0[i].w * h0[i].w + pp[i].y * xv;  n0.w = q0[i].z * h0[i].w + q0[i].w * h0[i].z;
+      n1.x = q1[i].x * h1[i].x - q1[i].y * h1[i].y + pp[i].z * xv;  n1.y = q1[i].x * h1[i].y + q1[i].y * h1[i].x;
+      n1.z = q1[i].z * h1[i].z - q1[i].w * h1[i].w + pp[i].w * xv;  n1.w = q1[i].z * h1[i].w + q1[i].w * h1[i].z;
+      float acc = (g0[i].x * n0.x - g0[i].y * n0.y) + (g0[i].z * n0.z - g0[i].w * n0.w) +
+                  (g1[i].x * n1.x - g1[i].y * n1.y) + (g1[i].z * n1.z - g1[i].w * n1.w);
+#pragma unroll
+      for (int m = 1; m < NP; m <<= 1) acc += __shfl_xor(acc, m);
+      if (ok) {
+        *(float4*)(A.h_out + ho) = n0;
+        *(float4*)(A.h_out + ho + 4) = n1;
+        if (part == 0) {
+          ((T*)A.xn)[o] = xn_t;
+          ((T*)A.y)[o] = from_float<T>(acc + om[i] * xv);
+        }
       }
     }
+  }
+  __syncthreads();                               // every wave has read the old statistics (they may be updated in place)
+  if (threadIdx.x == 0) {
+    A.mean[(size_t)b * A.G + g] = st.mean;
+    A.var[(size_t)b * A.G + g] = st.var;
+    if (g == 0) A.count[b] = c0 + (padded ? 0 : 1);
+  }
+}
+
+// TimestepNorm alone: one wave per (stream, group)
+template <typename T>
+__global__ __launch_bounds__(kTV) void norm_token_kernel(const StepArgs A) {
+  const int id = blockIdx.x * (kTV / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (id >= A.B * A.G) return;
+  const int g = id % A.G, b = id / A.G;
+  const int dg = A.D / A.G;
+  const size_t base = (size_t)b * A.D + (size_t)g * dg;
+  const T* xr = (const T*)A.x + base;
+  const int64_t c0 = A.prev_count[b];
+  const bool padded = A.mask != nullptr && A.mask[b] != 0;
+  const StepStats st = step_stats(xr, dg, lane, c0, A.prev_mean[id], A.prev_var[id], A.eps, padded);
+  for (int f = lane; f < dg; f += 64) {
+    const int d = g * dg + f;
+    ((T*)A.xn)[base + f] = from_float<T>(padded ? 0.f : (to_float(xr[f]) - st.mean) * st.rstd * A.nw[d] + A.nb[d]);
+  }
+  if (lane == 0) {
+    A.mean[id] = st.mean;
+    A.var[id] = st.var;
+    if (g == 0) A.count[b] = c0 + (padded ? 0 : 1);
   }
 }
 
@@ -350,7 +432,56 @@ __global__ __launch_bounds__(kTV) void norm_ema_steps_kernel(const StepArgs A) {
   }
 }
 
+// vector path: complex coefficient storage, 4 | N, N / 4 a power of two, aligned pointers
+bool step_vec_covers(const StepArgs& A) {
+  const int np = A.N / 4;
+  return A.N % 4 == 0 && (np & (np - 1)) == 0 && A.N <= 32 && ((uintptr_t)A.h_out % 16) == 0 &&
+         (!A.h_in || ((uintptr_t)A.h_in % 16) == 0) && ((uintptr_t)A.q % 16) == 0 && ((uintptr_t)A.g % 16) == 0 &&
+         ((uintptr_t)A.p % 16) == 0;
+}
+
+void launch_step_vec(const StepArgs& A, int dtype, hipStream_t s) {
+  const dim3 grid((unsigned)(A.B * A.G));
+  const int np = A.N / 4;
+#define LAUNCH_NV(T)                                                                                     \
+  switch (np) {                                                                                          \
+    case 1: hipLaunchKernelGGL((norm_ema_step_vec_kernel<T, 1>), grid, dim3(kTV), 0, s, A); break;       \
+    case 2: hipLaunchKernelGGL((norm_ema_step_vec_kernel<T, 2>), grid, dim3(kTV), 0, s, A); break;       \
+    case 4: hipLaunchKernelGGL((norm_ema_step_vec_kernel<T, 4>), grid, dim3(kTV), 0, s, A); break;       \
+    default: hipLaunchKernelGGL((norm_ema_step_vec_kernel<T, 8>), grid, dim3(kTV), 0, s, A); break;      \
+  }
+  if (dtype == MEGA_F32) { LAUNCH_NV(float) }
+  else if (dtype == MEGA_BF16) { LAUNCH_NV(bf16_t) }
+  else { LAUNCH_NV(f16_t) }
+#undef LAUNCH_NV
+}
+
 }  // namespace
+
+// the vector kernel with a padding mask, for the composite step of decode_layer.hip
+int norm_ema_token(const void* x, void* xn, void* y, int dtype, const uint8_t* mask, const int64_t* prev_count,
+                   const float* prev_mean, const float* prev_var, int64_t* count, float* mean, float* var,
+                   const float* norm_gamma, const float* norm_beta, double eps, const float* p, const float* q,
+                   const float* gamma, const float* omega, const float* h_in, float* h_out, int64_t B, int64_t D,
+                   int64_t G, int64_t N, hipStream_t s) {
+  MEGA_REQUIRE(B > 0 && D > 0 && G > 0 && N > 0 && D % G == 0 && B * G < (int64_t)1 << 31, MEGA_ERR_ARG,
+               "norm_ema_token: bad shape B=%ld D=%ld G=%ld N=%ld", (long)B, (long)D, (long)G, (long)N);
+  MEGA_REQUIRE(x && xn && y && prev_count && prev_mean && prev_var && count && mean && var && norm_gamma && norm_beta &&
+                   p && q && gamma && omega && h_out,
+               MEGA_ERR_ARG, "norm_ema_token: null pointer argument");
+  MEGA_REQUIRE(!ranges_overlap(prev_count, (size_t)B * 8, count, (size_t)B * 8), MEGA_ERR_ARG,
+               "norm_ema_token: count must not overlap prev_count");
+  StepArgs A;
+  A.x = x; A.xn = xn; A.y = y; A.prev_count = prev_count; A.prev_mean = prev_mean; A.prev_var = prev_var;
+  A.count = count; A.mean = mean; A.var = var; A.nw = norm_gamma; A.nb = norm_beta; A.p = p; A.q = q; A.g = gamma;
+  A.omega = omega; A.h_in = h_in; A.h_out = h_out; A.mask = mask; A.B = (int)B; A.D = (int)D; A.G = (int)G;
+  A.N = (int)N; A.K = 1; A.eps = (float)eps;
+  MEGA_REQUIRE(step_vec_covers(A), MEGA_ERR_UNSUPPORTED,
+               "norm_ema_token: ndim in {4, 8, 16, 32} with 16-byte aligned coefficients only");
+  launch_step_vec(A, dtype, s);
+  MEGA_CHECK_LAUNCH("norm_ema_token");
+  return MEGA_OK;
+}
 }  // namespace mega
 
 using namespace mega;
@@ -383,23 +514,10 @@ extern "C" int mega_norm_ema_step(const void* x, void* xn, void* y, int dtype, c
   A.omega = omega; A.h_in = h_in; A.h_out = h_out; A.B = (int)B; A.D = (int)D; A.G = (int)G; A.N = (int)N;
   A.K = 1;
   A.eps = (float)eps;
-  const dim3 grid((unsigned)(B * G));
   hipStream_t s = (hipStream_t)stream;
-  // vector path: complex coefficient storage (always), 4 | N, N / 4 a power of two, aligned pointers
-  const int np = (int)(N / 4);
-  if (is_complex && N % 4 == 0 && (np & (np - 1)) == 0 && ((uintptr_t)h_out % 16) == 0 && (!h_in || ((uintptr_t)h_in % 16) == 0) &&
-      ((uintptr_t)q % 16) == 0 && ((uintptr_t)gamma % 16) == 0 && ((uintptr_t)p % 16) == 0) {
-#define LAUNCH_NV(T)                                                                                     \
-  switch (np) {                                                                                          \
-    case 1: hipLaunchKernelGGL((norm_ema_step_vec_kernel<T, 1>), grid, dim3(kTV), 0, s, A); break;       \
-    case 2: hipLaunchKernelGGL((norm_ema_step_vec_kernel<T, 2>), grid, dim3(kTV), 0, s, A); break;       \
-    case 4: hipLaunchKernelGGL((norm_ema_step_vec_kernel<T, 4>), grid, dim3(kTV), 0, s, A); break;       \
-    default: hipLaunchKernelGGL((norm_ema_step_vec_kernel<T, 8>), grid, dim3(kTV), 0, s, A); break;      \
-  }
-    if (dtype == MEGA_F32) { LAUNCH_NV(float) }
-    else if (dtype == MEGA_BF16) { LAUNCH_NV(bf16_t) }
-    else { LAUNCH_NV(f16_t) }
-#undef LAUNCH_NV
+  const dim3 grid((unsigned)(B * G));
+  if (is_complex && step_vec_covers(A)) {
+    launch_step_vec(A, dtype, s);
     MEGA_CHECK_LAUNCH("norm_ema_step");
     return MEGA_OK;
   }
@@ -473,5 +591,31 @@ extern "C" int mega_norm_ema_steps(const void* x, void* xn, void* y, int dtype, 
   else { LAUNCH_NK(f16_t) }
 #undef LAUNCH_NK
   MEGA_CHECK_LAUNCH("norm_ema_steps");
+  return MEGA_OK;
+}
+
+extern "C" int mega_norm_token(const void* x, void* xn, int dtype, const uint8_t* mask, const int64_t* prev_count,
+                               const float* prev_mean, const float* prev_var, int64_t* count, float* mean, float* var,
+                               const float* norm_gamma, const float* norm_beta, double eps, int64_t B, int64_t D, int64_t G,
+                               void* stream) {
+  MEGA_REQUIRE(dtype == MEGA_F32 || dtype == MEGA_BF16 || dtype == MEGA_F16, MEGA_ERR_ARG, "norm_token: unknown dtype %d",
+               dtype);
+  MEGA_REQUIRE(B >= 0 && D > 0 && G > 0 && D % G == 0 && B * G < (int64_t)1 << 30, MEGA_ERR_ARG,
+               "norm_token: bad shape B=%ld D=%ld G=%ld", (long)B, (long)D, (long)G);
+  if (B == 0) return MEGA_OK;
+  MEGA_REQUIRE(x && xn && prev_count && prev_mean && prev_var && count && mean && var && norm_gamma && norm_beta, MEGA_ERR_ARG,
+               "norm_token: null pointer argument");
+  MEGA_REQUIRE(!ranges_overlap(prev_count, (size_t)B * 8, count, (size_t)B * 8), MEGA_ERR_ARG,
+               "norm_token: count must not overlap prev_count");
+  StepArgs A = {};
+  A.x = x; A.xn = xn; A.prev_count = prev_count; A.prev_mean = prev_mean; A.prev_var = prev_var; A.count = count;
+  A.mean = mean; A.var = var; A.nw = norm_gamma; A.nb = norm_beta; A.mask = mask; A.B = (int)B; A.D = (int)D;
+  A.G = (int)G; A.eps = (float)eps;
+  const dim3 grid((unsigned)ceil_div(B * G, kTV / 64));
+  hipStream_t s = (hipStream_t)stream;
+  if (dtype == MEGA_F32) hipLaunchKernelGGL(norm_token_kernel<float>, grid, dim3(kTV), 0, s, A);
+  else if (dtype == MEGA_BF16) hipLaunchKernelGGL(norm_token_kernel<bf16_t>, grid, dim3(kTV), 0, s, A);
+  else hipLaunchKernelGGL(norm_token_kernel<f16_t>, grid, dim3(kTV), 0, s, A);
+  MEGA_CHECK_LAUNCH("norm_token");
   return MEGA_OK;
 }

@@ -1,0 +1,312 @@
+// Host side of the calls whose device work is shorter than their Python would be: allocation of the results, argument
+// checks and the C ABI call in native code, one Python call per composite step.  Tensors in, tensors out; the launch
+// stream's raw handle comes from the caller (ops._stream).  No device code and no state in here.
+#include <ATen/ATen.h>
+#include <Python.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../include/mega_hip.h"
+
+namespace {
+
+using at::Tensor;
+
+struct Args {
+  PyObject* const* a;
+  Py_ssize_t n;
+  const char* who;
+  void want(Py_ssize_t k) const {
+    if (n != k) throw std::runtime_error(std::string(who) + ": " + std::to_string(k) + " arguments expected");
+  }
+  bool none(int i) const { return a[i] == Py_None; }
+  const Tensor& t(int i) const {
+    if (!THPVariable_Check(a[i])) throw std::runtime_error(std::string(who) + ": argument " + std::to_string(i) + " must be a tensor");
+    return THPVariable_Unpack(a[i]);
+  }
+  // a contiguous tensor of the given type, size and device
+  const Tensor& t(int i, at::ScalarType dt, int64_t numel, const at::Device& dev) const {
+    const Tensor& x = t(i);
+    if (x.scalar_type() != dt || x.numel() != numel || x.device() != dev || !x.is_contiguous())
+      throw std::runtime_error(std::string(who) + ": argument " + std::to_string(i) + " must be a contiguous tensor of " +
+                               std::to_string(numel) + " elements of " + at::toString(dt) + " on the input's device");
+    return x;
+  }
+  const void* p(int i, at::ScalarType dt, int64_t numel, const at::Device& dev) const { return t(i, dt, numel, dev).data_ptr(); }
+  const void* opt(int i, at::ScalarType dt, int64_t numel, const at::Device& dev) const {
+    return none(i) ? nullptr : p(i, dt, numel, dev);
+  }
+  double d(int i) const {
+    const double v = PyFloat_AsDouble(a[i]);
+    if (v == -1.0 && PyErr_Occurred()) throw std::runtime_error("");
+    return v;
+  }
+  int64_t i64(int i) const {
+    const int64_t v = PyLong_AsLongLong(a[i]);
+    if (v == -1 && PyErr_Occurred()) throw std::runtime_error("");
+    return v;
+  }
+  void* stream(int i) const { return (void*)(uintptr_t)PyLong_AsUnsignedLongLong(a[i]); }
+};
+
+int dtype_code(const Tensor& x) {
+  switch (x.scalar_type()) {
+    case at::kFloat: return MEGA_F32;
+    case at::kBFloat16: return MEGA_BF16;
+    case at::kHalf: return MEGA_F16;
+    default: throw std::runtime_error("unsupported activation dtype (float32, bfloat16, float16)");
+  }
+}
+
+void check(int rc, const char* who) {
+  if (rc != 0) throw std::runtime_error(std::string(who) + ": " + mega_last_error() + " (code " + std::to_string(rc) + ")");
+}
+
+PyObject* wrap(Tensor t) { return t.defined() ? THPVariable_Wrap(std::move(t)) : (Py_INCREF(Py_None), Py_None); }
+
+template <size_t N>
+PyObject* tuple(Tensor (&ts)[N]) {
+  PyObject* r = PyTuple_New(N);
+  if (!r) return nullptr;
+  for (size_t i = 0; i < N; ++i) PyTuple_SET_ITEM(r, i, wrap(std::move(ts[i])));
+  return r;
+}
+
+Tensor empty(at::IntArrayRef sizes, const Tensor& like, at::ScalarType dt) {
+  return at::empty(sizes, like.options().dtype(dt));
+}
+
+// (x [B, 1, D], mask [B] bytes | None, count, mean, var, h | None, keys | None, values | None, keep, norm gamma, norm beta,
+//  norm eps, groups, p, q, gamma, omega, v weight, v bias, mx weight, mx bias, h weight, gamma, beta, move act,
+//  move weight | None, move eps, cis, heads, stream) -> (out [B, 1, D], count, mean, var, h', keys' | None, values' | None)
+PyObject* token_gated_attention(const Args& A) {
+  A.want(30);
+  const Tensor& x = A.t(0);
+  const at::Device dev = x.device();
+  const at::ScalarType T = x.scalar_type();
+  if (x.dim() != 3 || x.size(1) != 1 || !x.is_contiguous() || !x.is_cuda())
+    throw std::runtime_error("token_gated_attention: x must be a contiguous [B, 1, D] device tensor");
+  const int64_t B = x.size(0), D = x.size(2);
+  const Tensor &p = A.t(13), &hw = A.t(21), &gm = A.t(22);
+  if (p.dim() != 2 || hw.dim() != 2 || gm.dim() != 2) throw std::runtime_error("token_gated_attention: weight shapes");
+  const int64_t N = p.size(1), hidden = hw.size(1), S = gm.size(1), G = A.i64(12), Nh = A.i64(28);
+  const int64_t W = 2 * D + S + hidden;
+  if (G <= 0 || D % G || Nh <= 0) throw std::runtime_error("token_gated_attention: groups / heads");
+  int64_t n = 0;
+  if (!A.none(6)) {
+    const Tensor& k = A.t(6);
+    if (k.dim() != 3 || k.size(0) != B || k.size(2) != S) throw std::runtime_error("token_gated_attention: cached keys must be [B, n, S]");
+    n = k.size(1);
+  }
+  MegaTokenAttention a = {};
+  a.dtype = dtype_code(x); a.B = B; a.D = D; a.S = S; a.hidden = hidden; a.heads = Nh; a.groups = G; a.states = N;
+  a.context = n;
+  a.x = x.data_ptr();
+  a.mask = (const uint8_t*)A.opt(1, at::kByte, B, dev);
+  a.prev_count = (const int64_t*)A.p(2, at::kLong, B, dev);
+  a.prev_mean = (const float*)A.p(3, at::kFloat, B * G, dev);
+  a.prev_var = (const float*)A.p(4, at::kFloat, B * G, dev);
+  a.h_in = (const float*)A.opt(5, at::kComplexFloat, B * D * N, dev);
+  if (n > 0) {                       // keys straight from a prompt are a strided half of the q / k map's result
+    const Tensor& k = A.t(6);
+    if (k.scalar_type() != T || k.device() != dev || k.stride(2) != 1)
+      throw std::runtime_error("token_gated_attention: cached keys must be rows of the activation type");
+    a.k_old = k.data_ptr();
+    a.k_row = k.stride(1);
+    a.k_batch = k.stride(0);
+  }
+  a.v_old = A.opt(7, T, B * n * hidden, dev);
+  const bool keep = PyObject_IsTrue(A.a[8]) == 1;
+  a.norm_gamma = (const float*)A.p(9, at::kFloat, D, dev);
+  a.norm_beta = (const float*)A.p(10, at::kFloat, D, dev);
+  a.norm_eps = A.d(11);
+  a.p = (const float*)A.p(13, at::kFloat, D * N, dev);
+  a.q = (const float*)A.p(14, at::kFloat, D * N * 2, dev);
+  a.ema_gamma = (const float*)A.p(15, at::kFloat, D * N * 2, dev);
+  a.omega = (const float*)A.p(16, at::kFloat, D, dev);
+  a.v_weight = A.p(17, T, hidden * D, dev);
+  a.v_bias = A.p(18, T, hidden, dev);
+  a.mx_weight = A.p(19, T, W * D, dev);
+  a.mx_bias = A.p(20, T, W, dev);
+  a.h_weight = A.p(21, T, D * hidden, dev);
+  a.gamma = A.p(22, T, 2 * S, dev);
+  a.beta = A.p(23, T, 2 * S, dev);
+  a.move_act = A.i64(24);
+  a.move_norm_weight = A.opt(25, T, D, dev);
+  a.move_norm_eps = A.d(26);
+  const Tensor& cis = A.t(27);
+  if (cis.scalar_type() != at::kComplexFloat || cis.dim() != 2 || cis.size(0) <= n || cis.size(1) * 2 * Nh != S ||
+      !cis.is_contiguous() || cis.device() != dev)
+    throw std::runtime_error("token_gated_attention: the rotation table must cover the new position");
+  a.cis = (const float*)cis.data_ptr();
+  Tensor r[7];
+  r[0] = at::empty({B, 1, D}, x.options());
+  r[1] = empty({B}, x, at::kLong);
+  r[2] = empty({B, G}, x, at::kFloat);
+  r[3] = empty({B, G}, x, at::kFloat);
+  r[4] = empty({B, D, N}, x, at::kComplexFloat);
+  if (keep) {
+    r[5] = at::empty({B, n + 1, S}, x.options());
+    r[6] = at::empty({B, n + 1, hidden}, x.options());
+    a.k_out = r[5].data_ptr();
+    a.v_out = r[6].data_ptr();
+  }
+  a.out = r[0].data_ptr();
+  a.count = (int64_t*)r[1].data_ptr();
+  a.mean = (float*)r[2].data_ptr();
+  a.var = (float*)r[3].data_ptr();
+  a.h_out = (float*)r[4].data_ptr();
+  const int64_t nws = (int64_t)mega_token_attention_workspace_bytes(B, n, D, S, hidden, Nh);
+  Tensor ws = empty({nws}, x, at::kByte);
+  a.workspace = ws.data_ptr();
+  a.workspace_bytes = nws;
+  check(mega_token_gated_attention(&a, A.stream(29)), A.who);
+  return tuple(r);
+}
+
+// (x [B, 1, D], norm kind, norm weight | None, norm bias | None, eps, fc1 weight, fc1 bias, fc2 weight, layer scale | None,
+//  stream) -> x + scale fc2(silu(fc1(norm(x))))
+PyObject* token_ffn(const Args& A) {
+  A.want(10);
+  const Tensor& x = A.t(0);
+  const at::Device dev = x.device();
+  const at::ScalarType T = x.scalar_type();
+  const Tensor& w1 = A.t(5);
+  if (x.dim() != 3 || x.size(1) != 1 || !x.is_contiguous() || !x.is_cuda() || w1.dim() != 2)
+    throw std::runtime_error("token_ffn: x must be a contiguous [B, 1, D] device tensor");
+  const int64_t B = x.size(0), D = x.size(2), H = w1.size(0);
+  Tensor hid = at::empty({B, H}, x.options()), rows = at::empty({B, D}, x.options()), out[1] = {at::empty({B, 1, D}, x.options())};
+  MegaTokenLinear f1 = {}, f2 = {};
+  f1.prologue = (int)A.i64(1);
+  f1.scratch = rows.data_ptr();
+  f1.norm_weight = A.opt(2, T, D, dev);
+  f1.norm_bias = A.opt(3, T, D, dev);
+  f1.eps = (float)A.d(4);
+  f1.weight = A.p(5, T, H * D, dev);
+  f1.bias = A.p(6, T, H, dev);
+  f1.x = x.data_ptr(); f1.x_stride = D; f1.out = hid.data_ptr(); f1.out_stride = H; f1.N = H; f1.K = D;
+  f1.epilogue = MEGA_TOKEN_SILU;
+  f2.weight = A.p(7, T, D * H, dev);
+  f2.scale = A.opt(8, T, D, dev);
+  f2.x = hid.data_ptr(); f2.x_stride = H; f2.out = out[0].data_ptr(); f2.out_stride = D; f2.N = D; f2.K = H;
+  f2.epilogue = MEGA_TOKEN_RESIDUAL; f2.residual = x.data_ptr(); f2.residual_stride = D;
+  const int dt = dtype_code(x);
+  void* s = A.stream(9);
+  check(mega_token_linear(&f1, dt, B, s), A.who);
+  check(mega_token_linear(&f2, dt, B, s), A.who);
+  return wrap(out[0]);
+}
+
+// (tokens [B, 1], table [V, D], scale, pad, stream) -> (x [B, 1, D], mask [B] bytes)
+PyObject* token_embed(const Args& A) {
+  A.want(5);
+  const Tensor &tok = A.t(0), &tab = A.t(1);
+  if (tok.scalar_type() != at::kLong || !tok.is_contiguous() || tok.device() != tab.device() || !tab.is_cuda() ||
+      tab.dim() != 2 || !tab.is_contiguous())
+    throw std::runtime_error("token_embed: tokens [B, 1] int64 and a contiguous [V, D] table on one device");
+  const int64_t B = tok.numel(), D = tab.size(1);
+  Tensor r[2] = {at::empty({B, 1, D}, tab.options()), empty({B}, tab, at::kByte)};
+  check(mega_token_embed((const int64_t*)tok.data_ptr(), tab.data_ptr(), dtype_code(tab), A.d(2), A.i64(3), tab.size(0), B, D,
+                         r[0].data_ptr(), (uint8_t*)r[1].data_ptr(), A.stream(4)),
+        A.who);
+  return tuple(r);
+}
+
+// (x [B, 1, D], mask [B] bytes | None, count, mean, var, gamma, beta, eps, groups, stream) -> (xn, count, mean, var)
+PyObject* token_norm(const Args& A) {
+  A.want(10);
+  const Tensor& x = A.t(0);
+  const at::Device dev = x.device();
+  if (x.dim() != 3 || x.size(1) != 1 || !x.is_contiguous() || !x.is_cuda())
+    throw std::runtime_error("token_norm: x must be a contiguous [B, 1, D] device tensor");
+  const int64_t B = x.size(0), D = x.size(2), G = A.i64(8);
+  Tensor r[4] = {at::empty({B, 1, D}, x.options()), empty({B}, x, at::kLong), empty({B, G}, x, at::kFloat),
+                 empty({B, G}, x, at::kFloat)};
+  check(mega_norm_token(x.data_ptr(), r[0].data_ptr(), dtype_code(x), (const uint8_t*)A.opt(1, at::kByte, B, dev),
+                        (const int64_t*)A.p(2, at::kLong, B, dev), (const float*)A.p(3, at::kFloat, B * G, dev),
+                        (const float*)A.p(4, at::kFloat, B * G, dev), (int64_t*)r[1].data_ptr(), (float*)r[2].data_ptr(),
+                        (float*)r[3].data_ptr(), (const float*)A.p(5, at::kFloat, D, dev),
+                        (const float*)A.p(6, at::kFloat, D, dev), A.d(7), B, D, G, A.stream(9)),
+        A.who);
+  return tuple(r);
+}
+
+// (x [B, 1, K], weight [N, K], bias | None, stream) -> [B, 1, N]
+PyObject* token_linear(const Args& A) {
+  A.want(4);
+  const Tensor &x = A.t(0), &w = A.t(1);
+  if (x.dim() != 3 || x.size(1) != 1 || !x.is_contiguous() || !x.is_cuda() || w.dim() != 2)
+    throw std::runtime_error("token_linear: x must be a contiguous [B, 1, K] device tensor");
+  const int64_t B = x.size(0), K = x.size(2), N = w.size(0);
+  Tensor out = at::empty({B, 1, N}, x.options());
+  MegaTokenLinear f = {};
+  f.weight = A.p(1, x.scalar_type(), N * K, x.device());
+  f.bias = A.opt(2, x.scalar_type(), N, x.device());
+  f.x = x.data_ptr(); f.x_stride = K; f.out = out.data_ptr(); f.out_stride = N; f.N = N; f.K = K;
+  check(mega_token_linear(&f, dtype_code(x), B, A.stream(3)), A.who);
+  return wrap(out);
+}
+
+// (x [B, D], count, next count, mean, var, norm weight, norm bias, eps, p, q, gamma, complex, omega, h, groups, stream)
+//   -> (xn, y); count / mean / var / h are the step's own buffers, updated in place (next count takes the new count)
+PyObject* norm_ema_step(const Args& A) {
+  A.want(16);
+  Tensor x = A.t(0).detach().contiguous();
+  const at::Device dev = x.device();
+  const Tensor& p = A.t(8);
+  if (x.dim() != 2 || !x.is_cuda() || p.dim() != 2) throw std::runtime_error("norm_ema_step: x must be a [B, D] device tensor");
+  const int64_t B = x.size(0), D = x.size(1), N = p.size(1), G = A.i64(14);
+  Tensor r[2] = {at::empty_like(x), at::empty_like(x)};
+  float* mean = (float*)A.p(3, at::kFloat, B * G, dev);
+  float* var = (float*)A.p(4, at::kFloat, B * G, dev);
+  float* h = (float*)A.p(13, at::kFloat, B * D * N * 2, dev);
+  check(mega_norm_ema_step(x.data_ptr(), r[0].data_ptr(), r[1].data_ptr(), dtype_code(x), (const int64_t*)A.p(1, at::kLong, B, dev),
+                           mean, var, (int64_t*)A.p(2, at::kLong, B, dev), mean, var, (const float*)A.p(5, at::kFloat, D, dev),
+                           (const float*)A.p(6, at::kFloat, D, dev), A.d(7), (const float*)A.p(8, at::kFloat, D * N, dev),
+                           (const float*)A.p(9, at::kFloat, D * N * 2, dev), (const float*)A.p(10, at::kFloat, D * N * 2, dev),
+                           (int)A.i64(11), (const float*)A.p(12, at::kFloat, D, dev), h, h, B, D, G, N, A.stream(15)),
+        A.who);
+  return tuple(r);
+}
+
+// (dict, ...) -> bytes: storage address and in-place version of every tensor in the dictionaries' values, in order
+PyObject* tensor_versions(const Args& A) {
+  int64_t buf[128];
+  size_t n = 0;
+  for (int i = 0; i < A.n; ++i) {
+    if (!PyDict_Check(A.a[i])) throw std::runtime_error("tensor_versions: dictionaries expected");
+    PyObject *key, *value;
+    Py_ssize_t pos = 0;
+    while (PyDict_Next(A.a[i], &pos, &key, &value)) {
+      if (value == Py_None) continue;
+      if (!THPVariable_Check(value) || n + 2 > sizeof(buf) / sizeof(buf[0])) throw std::runtime_error("tensor_versions: up to 64 tensors");
+      const Tensor& t = THPVariable_Unpack(value);
+      buf[n++] = (int64_t)(uintptr_t)t.data_ptr();
+      buf[n++] = (int64_t)t._version();
+    }
+  }
+  return PyBytes_FromStringAndSize((const char*)buf, (Py_ssize_t)(n * 8));
+}
+
+PyObject* guarded(PyObject* (*f)(const Args&), const Args& args) {
+  try {
+    return f(args);
+  } catch (const std::exception& e) {
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
+    return nullptr;
+  }
+}
+
+#define MEGA_ENTRY(f)                                                                                              \
+  {#f,                                                                                                             \
+   (PyCFunction)(void (*)(void))(PyObject * (*)(PyObject*, PyObject* const*, Py_ssize_t))                          \
+       [](PyObject*, PyObject* const* a, Py_ssize_t n) -> PyObject* { return guarded(f, Args{a, n, #f}); },        \
+   METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {MEGA_ENTRY(token_gated_attention), MEGA_ENTRY(token_ffn),  MEGA_ENTRY(token_embed),
+                         MEGA_ENTRY(token_norm),            MEGA_ENTRY(token_linear), MEGA_ENTRY(norm_ema_step),
+                         MEGA_ENTRY(tensor_versions),
+                         {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "mega_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_mega_host(void) { return PyModule_Create(&module); }

@@ -24,7 +24,8 @@ from torch.nn import Parameter
 from . import ops
 from .modules import (AttentionSoftmax, EfficientAttention, GateMulFunc, GateOutFunc, GateQKFunc, IncrementalState,
                       MultiHeadComplexEMA, MultiHeadEMA, SequenceNorm, SplitFunc, SplitGrads, SwiGLU, TimestepNorm,
-                      _tensor_versions, _training_call, linear, linear_residual, norm_then_move, silu)
+                      _tensor_versions, _training_call, linear, linear_residual, mask_bytes, mask_bytes_ok,
+                      norm_then_move, silu)
 
 
 class RMSNorm(nn.Module):
@@ -121,6 +122,9 @@ class NormalizedFeedForwardNetwork(nn.Module):
         # (normalized_feedforward_network.py:81-83)
         if _training_call(self, x) or (self.training and self.hidden_dropout_p > 0):
             h = F.dropout(silu(linear(self.fc1, self.norm(x))), self.hidden_dropout_p, self.training)
+        elif ops.token_rows(x, normalised=True) and self.hidden_dim % 32 == 0 and self.fc1.weight.dtype == x.dtype and \
+                not (self.training and self.dropout_p > 0):
+            return self._few_rows(x)
         else:
             h = ops.silu(self.fc1(self.norm(x)), inplace=True)
         if self.layerscale_weight is None and not (self.training and self.dropout_p > 0):
@@ -129,6 +133,16 @@ class NormalizedFeedForwardNetwork(nn.Module):
         if self.layerscale_weight is not None:
             h = h * self.layerscale_weight
         return h + x
+
+    def _few_rows(self, x: Tensor) -> Tensor:
+        """The block on one token per stream: two launches (norm, first projection and activation; second projection,
+        layer scale and residual)."""
+        rms = isinstance(self.norm, RMSNorm)
+        with ops._on_device(x.device):
+            return ops._lib.load_host().token_ffn(
+                x, ops.TOKEN_RMSNORM if rms else ops.TOKEN_LAYERNORM, self.norm.weight, None if rms else self.norm.bias,
+                self.norm.eps, self.fc1.weight, self.fc1.bias, self.fc2.weight, self.layerscale_weight,
+                ops._stream(x.device))
 
     def extra_repr(self) -> str:
         return 'edim={}, hdim={}, act={}, init={}, layerscale={}'.format(self.embedding_dim, self.hidden_dim,
@@ -293,6 +307,10 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
         bsz, seq_len, embed_dim = x.size()
         assert embed_dim == self.embed_dim
         saved_state = self._get_input_buffer(incremental_state) if incremental_state is not None else None
+        if saved_state is not None and seq_len == 1 and self._token_covers(x, padding_mask, saved_state):
+            out = self._token_step(x, padding_mask, saved_state, incremental_state)
+            if out is not None:
+                return out, None
         residual = x
         if self.bidirectional:
             assert incremental_state is None, 'a bidirectional layer has no incremental state'
@@ -331,6 +349,60 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
         # projection, u and the residual mix after it
         hp = self.h_proj(ops.gate_mul_fwd(attn.reshape(bsz, seq_len, self.hdim), r))
         return ops.gate_out_fwd(residual, u, hx, hp), None
+
+    def _token_covers(self, x: Tensor, padding_mask: Optional[Tensor], saved_state) -> bool:
+        """One new token per stream on the composite step (decode_layer.hip): few streams, 16-bit, the layer form of the
+        language model (softmax, rotary, complex moving average without truncation, group norm)."""
+        move, key = self.move, saved_state.get("prev_key")
+        z, h, Nh = self.zdim, self.hdim, self.num_heads
+        return (ops.token_rows(x, normalised=True) and mask_bytes_ok(padding_mask) and self.v_proj.weight.dtype == x.dtype
+                and self.attention_activation == 'softmax' and isinstance(self.rel_pos_bias, RotaryEmbedding)
+                and self.norm.num_groups is not None and isinstance(move, MultiHeadComplexEMA)
+                and (move.truncation is None or move.truncation < 1) and self.ndim in (4, 8, 16, 32)
+                and h % 32 == 0 and h % (8 * Nh) == 0 and z % (8 * Nh) == 0 and z // Nh <= 512
+                and (key is None or (key.dtype == x.dtype and key.stride(2) == 1 and key.stride(1) % 8 == 0
+                                     and key.stride(0) % 8 == 0 and key.data_ptr() % 16 == 0
+                                     and saved_state["prev_value"].is_contiguous()
+                                     and (self.chunk_size < 0 or key.size(1) < self.chunk_size))))
+
+    def _token_step(self, x: Tensor, padding_mask: Optional[Tensor], saved_state, incremental_state) -> Optional[Tensor]:
+        """The layer on one new token per stream in one native call (7 launches): the same state entries in and out as
+        the operators one by one keep."""
+        norm, move = self.norm, self.move
+        norm_state, move_state = norm._get_input_buffer(incremental_state), move._get_input_buffer(incremental_state)
+        count, mean, var = norm_state.get('prev_count'), norm_state.get('prev_mean'), norm_state.get('prev_var')
+        if count is None or mean is None or var is None:
+            count, mean, var = norm._prior_state(x.size(0))
+        h = move_state.get('prev_state')
+        if h is not None and not (h.dtype is torch.complex64 and h.is_contiguous() and not h.is_conj()):
+            return None
+        gamma, beta = norm._affine()
+        ema = move._prepared_layer()
+        key, value = saved_state.get("prev_key"), saved_state.get("prev_value")
+        n = 0 if key is None else key.size(1)
+        keep = self.chunk_size < 0 or (n + 1) % self.chunk_size != 0
+        act = self.move_act
+        rms = isinstance(act, RMSNorm)
+        mine, mods = self._parameters, self._modules          # (attribute by attribute: 0.25 us each through nn.Module)
+        pv, pm, ph = (mods[k]._parameters for k in ('v_proj', 'mx_proj', 'h_proj'))
+        with ops._on_device(x.device):
+            out, count, mean, var, h, key, value = ops._lib.load_host().token_gated_attention(
+                x, mask_bytes(padding_mask), count, ops._f32c(mean), ops._f32c(var), h, key, value, keep, gamma, beta,
+                norm.eps, norm.num_groups, ema.p, ema.q, ema.gamma, ema.omega, pv['weight'], pv['bias'], pm['weight'],
+                pm['bias'], ph['weight'], mine['gamma'], mine['beta'], ops.TOKEN_RMSNORM if rms else ops.TOKEN_SILU,
+                act._parameters['weight'] if rms else None, act.eps if rms else 0.0,
+                self.rel_pos_bias._freqs_cis(0, n + 1), self.num_heads, ops._stream(x.device))
+        norm_state['prev_mean'], norm_state['prev_var'], norm_state['prev_count'] = mean, var, count
+        norm._set_input_buffer(incremental_state, norm_state)
+        move_state['prev_state'] = h
+        move._set_input_buffer(incremental_state, move_state)
+        if keep:
+            saved_state["prev_key"], saved_state["prev_value"] = key, value
+        else:
+            saved_state.pop("prev_key", None)
+            saved_state.pop("prev_value", None)
+        self._set_input_buffer(incremental_state, saved_state)
+        return out
 
     def _drops(self) -> bool:
         return self.dropout_p > 0 or self.hidden_dropout_p > 0 or self.attention_dropout_p > 0

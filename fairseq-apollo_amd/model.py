@@ -73,6 +73,9 @@ class MegaDecoderNoCrossAttn(nn.Module):
 
     def output_layer(self, features: Tensor) -> Tensor:
         """Project features to the vocabulary (mega_lm.py:379-385)."""
+        w = self.output_projection.weight
+        if not torch.is_grad_enabled() and ops.token_rows(features) and w.dtype == features.dtype:
+            return ops.token_linear(features, w)
         return self.output_projection(features)
 
     def max_positions(self) -> int:
@@ -84,6 +87,8 @@ class MegaDecoderNoCrossAttn(nn.Module):
         masked in every layer and zeroed at the end."""
         bsz, seq_len = prev_output_tokens.size()
         num_paddings = 0
+        if seq_len == 1 and incremental_state is not None and self._token_covers(prev_output_tokens):
+            return self._token_features(prev_output_tokens, incremental_state)
         if seq_len > self.chunk_size > 0 and seq_len % self.chunk_size != 0:
             num_paddings = math.ceil(seq_len / self.chunk_size) * self.chunk_size - seq_len
             prev_output_tokens = F.pad(prev_output_tokens, (0, num_paddings), value=self.padding_idx)
@@ -104,6 +109,33 @@ class MegaDecoderNoCrossAttn(nn.Module):
             x = x * (~decoder_padding_mask).to(x.dtype).unsqueeze(-1)
         if num_paddings > 0:
             x = x[:, :seq_len]
+        return x, {"inner_states": inner_states}
+
+    def _token_covers(self, tokens: Tensor) -> bool:
+        w = self.embed_tokens.weight
+        return (not torch.is_grad_enabled() and w.is_cuda and w.dtype in (torch.bfloat16, torch.float16)
+                and w.is_contiguous() and w.shape[1] % 8 == 0 and tokens.dtype is torch.int64 and tokens.is_contiguous()
+                and tokens.device == w.device and not (self.training and self.embedding_dropout.p > 0))
+
+    def _token_features(self, tokens: Tensor, incremental_state):
+        """extract_features for one new token per stream: which streams are padded stays on the device (asking the
+        host to look would make it wait for everything enqueued before), the layers take the mask as it is."""
+        dev = tokens.device
+        pad = -1 if self.padding_idx is None else self.padding_idx
+        with ops._on_device(dev):
+            x, mask = ops._lib.load_host().token_embed(tokens, self.embed_tokens.weight,
+                                                       1.0 if self.embed_scale is None else self.embed_scale, pad,
+                                                       ops._stream(dev))
+        mask = None if self.padding_idx is None else mask.view(-1, 1)
+        inner_states: List[Tensor] = [x]
+        for layer in self.layers:
+            x, _, _ = layer(x, incremental_state=incremental_state, decoder_padding_mask=mask)
+            inner_states.append(x)
+        x = self.final_norm(x, padding_mask=mask, incremental_state=incremental_state)      # zeros at padding
+        if not isinstance(self.pre_logits, nn.Identity):
+            x = self.pre_logits(x)
+            if mask is not None:
+                x = x * (mask == 0).to(x.dtype).unsqueeze(-1)
         return x, {"inner_states": inner_states}
 
     def reorder_incremental_state(self, incremental_state, new_order: Tensor) -> None:

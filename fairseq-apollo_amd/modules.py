@@ -80,7 +80,7 @@ def _training_call(module: nn.Module, *tensors) -> bool:
                                         or any(p.requires_grad for p in module.parameters()))
 
 
-def _tensor_versions(*modules: nn.Module) -> tuple:
+def _tensor_versions(*modules: nn.Module) -> bytes:
     """Storage address and in-place version of the modules' own parameters and buffers.  An eval-mode cache
     derived from them is stale once this tuple changes: load_state_dict copies into the parameters, an
     optimiser step or an in-place edit under no_grad bumps the version, `.to()` moves the storage.  (The
@@ -92,8 +92,7 @@ def _tensor_versions(*modules: nn.Module) -> tuple:
     utilities do) changes neither the address nor the version counter of `p`, so it is not seen here; after such an
     edit call `module.train(); module.eval()` (every mode switch drops the caches) or edit under `torch.no_grad()`
     through the parameter itself."""
-    return tuple((t.data_ptr(), t._version) for m in modules
-                 for t in (*m._parameters.values(), *m._buffers.values()) if t is not None)
+    return ops._lib.load_host().tensor_versions(*[d for m in modules for d in (m._parameters, m._buffers)])
 
 
 class EMACoeffsFunc(torch.autograd.Function):
@@ -462,6 +461,14 @@ class TimestepNormFunc(torch.autograd.Function):
 timestep_norm = TimestepNormFunc.apply
 
 
+def mask_bytes_ok(mask: Optional[Tensor]) -> bool:
+    return mask is None or (mask.dtype in (torch.bool, torch.uint8) and mask.is_contiguous())
+
+
+def mask_bytes(mask: Optional[Tensor]) -> Optional[Tensor]:
+    return mask.view(torch.uint8) if mask is not None and mask.dtype is torch.bool else mask
+
+
 class TimestepNorm(nn.Module, IncrementalState):
     """Streaming cumulative (group) normalisation with a carried (count, mean, var) state
     (fairseq/modules/norm_layer/timestep_norm.py:71-167).  mean / var are carried in fp32."""
@@ -525,7 +532,14 @@ class TimestepNorm(nn.Module, IncrementalState):
                 self._set_input_buffer(incremental_state, saved_state)
             return out
         gamma, beta = self._affine()
-        if self.num_groups is None:
+        if incremental_state is not None and x.size(1) == 1 and self.num_groups is not None and x.is_cuda and \
+                x.is_contiguous() and mask_bytes_ok(padding_mask):
+            # one token per stream: no look-back over time, one wave per (stream, group)
+            with ops._on_device(x.device):
+                out, count, mean, var = ops._lib.load_host().token_norm(
+                    x, mask_bytes(padding_mask), prev_count, ops._f32c(prev_mean), ops._f32c(prev_var), gamma, beta,
+                    self.eps, self.num_groups, ops._stream(x.device))
+        elif self.num_groups is None:
             out, count, mean, var, _, _ = ops.timestep_norm_fwd(x, prev_count, prev_mean, prev_var, gamma, beta,
                                                                 padding_mask, self.eps, need_stats=False)
         else:

@@ -149,6 +149,30 @@ def check_lookback(where: str = "") -> None:
 
 
 # --------------------------------------------------------------------------------------
+# steps of few rows (one token per stream): native composites
+# --------------------------------------------------------------------------------------
+TOKEN_NONE, TOKEN_SILU, TOKEN_RMSNORM, TOKEN_LAYERNORM = 0, 1, 2, 3
+TOKEN_ROWS = 64                       # rows the one-token kernels take
+_TOKEN_LDS = 144 * 1024               # bytes of normalised input rows a projection workgroup can stage
+
+
+def token_rows(x: torch.Tensor, normalised: bool = False) -> bool:
+    """True when the projections of x [rows, 1, K] run on the one-token kernels: 16-bit activations on the GPU, few
+    rows, whole 16-byte pieces; `normalised`: the rows are staged in LDS by every workgroup."""
+    if not (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and x.dim() == 3 and x.shape[1] == 1):
+        return False
+    B, K = x.shape[0], x.shape[2]
+    return 0 < B <= TOKEN_ROWS and K % 32 == 0 and x.is_contiguous() and \
+        (not normalised or B * (2 * K + 16) <= _TOKEN_LDS)
+
+
+def token_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """F.linear of few rows x [rows, 1, K] (token_rows(x) holds)."""
+    with _on_device(x.device):
+        return _lib.load_host().token_linear(x, weight, bias, _stream(x.device))
+
+
+# --------------------------------------------------------------------------------------
 # ops with the reference's names
 # --------------------------------------------------------------------------------------
 
@@ -1011,17 +1035,10 @@ class DecodeStep:
 
     def __call__(self, x_t: torch.Tensor):
         """x_t: [B, D] -> (xn_t, y_t), both [B, D]."""
-        lib = _lib.load()
-        xd = x_t.detach().contiguous()
-        xn = torch.empty_like(xd)
-        y = torch.empty_like(xd)
         with _on_device(self.dev):
-            rc = lib.mega_norm_ema_step(_ptr(xd), _ptr(xn), _ptr(y), _dtype_code(xd), _ptr(self.count), _ptr(self.mean),
-                                        _ptr(self.var), _ptr(self._count_next), _ptr(self.mean), _ptr(self.var), _ptr(self.nw),
-                                        _ptr(self.nb), self.eps, _ptr(self.p), _ptr(self.q), _ptr(self.gamma),
-                                        1 if self.is_complex else 0, _ptr(self.omega), _ptr(self.h), _ptr(self.h),
-                                        self.B, self.D, self.G, self.N, _stream(self.dev))
-        _lib.check(rc, "norm_ema_step")
+            xn, y = _lib.load_host().norm_ema_step(x_t, self.count, self._count_next, self.mean, self.var, self.nw, self.nb,
+                                                   self.eps, self.p, self.q, self.gamma, 1 if self.is_complex else 0,
+                                                   self.omega, self.h, self.G, _stream(self.dev))
         self.count, self._count_next = self._count_next, self.count
         return xn, y
 

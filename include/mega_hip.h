@@ -213,6 +213,95 @@ int mega_norm_ema_step(const void* x, void* xn, void* y, int dtype, const int64_
                        int is_complex, const float* omega, const float* h_in, float* h_out,
                        int64_t B, int64_t D, int64_t G, int64_t N, void* stream);
 
+/* TimestepNorm of one token of every stream (TimestepNorm.forward with L = 1, timestep_norm.py:100-139):
+ *   x, xn [B,D]; mask [B] (non-zero at padding: the token leaves as zeros and the statistics stay) or NULL;
+ *   prev_* / count, mean, var as mega_norm_ema_step.                                                     */
+int mega_norm_token(const void* x, void* xn, int dtype, const uint8_t* mask, const int64_t* prev_count,
+                    const float* prev_mean, const float* prev_var, int64_t* count, float* mean, float* var,
+                    const float* norm_gamma, const float* norm_beta, double eps, int64_t B, int64_t D, int64_t G,
+                    void* stream);
+
+/* ---- one token of every stream through a whole layer (incremental_state with one new position:
+ * MovingAverageGatedAttention.forward, moving_average_gated_attention.py:263-417; NormalizedFeedForwardNetwork.forward,
+ * normalized_feedforward_network.py:77-93; MegaDecoderNoCrossAttn.extract_features, models/mega_lm.py:313-386).
+ * 16-bit activations, at most 64 streams, weights of the activations' type.                             */
+enum {
+  MEGA_TOKEN_NONE = 0,
+  MEGA_TOKEN_SILU = 1,
+  MEGA_TOKEN_RMSNORM = 2,     /* prologue: x / sqrt(mean(x^2) + eps) * (norm_weight + 1) */
+  MEGA_TOKEN_LAYERNORM = 3,   /* prologue: (x - mean) / sqrt(var + eps) * (norm_weight + 1) + norm_bias */
+  MEGA_TOKEN_RESIDUAL = 4,    /* epilogue: scale * value + residual */
+  MEGA_TOKEN_GATE = 5         /* epilogue: residual + sigmoid(gate_u) (silu(gate_hx + value) - residual) */
+};
+
+/* out[b, n] = epilogue(sum_k weight[n, k] prologue(x[b])[k] + bias[n]), b < B <= 64 */
+typedef struct {
+  const void* weight;         /* [N, K] */
+  const void* bias;           /* [N] or NULL */
+  const void* x;              /* [B, K], rows x_stride elements apart */
+  void* out;                  /* [B, N], rows out_stride elements apart */
+  const void* norm_weight;    /* [K] offsets from one, or NULL */
+  const void* norm_bias;      /* [K] or NULL */
+  const void* residual;       /* [B, N], rows residual_stride elements apart */
+  const void* scale;          /* [N] or NULL (layer scale) */
+  const void* gate_u;         /* [B, N], rows gate_stride elements apart */
+  const void* gate_hx;
+  void* scratch;              /* [B, K] or NULL: lets a call with a prologue normalise many rows once */
+  int64_t x_stride, out_stride, residual_stride, gate_stride, N, K;
+  float eps;
+  int prologue, epilogue;
+} MegaTokenLinear;
+
+int mega_token_linear(const MegaTokenLinear* p, int dtype, int64_t B, void* stream);
+
+/* x[b] = scale table[tokens[b]], mask[b] = tokens[b] == pad (mask may be NULL); an index outside the table gives NaN */
+int mega_token_embed(const int64_t* tokens, const void* table, int dtype, double scale, int64_t pad, int64_t vocab,
+                     int64_t B, int64_t D, void* x, uint8_t* mask, void* stream);
+
+/* The gated attention of one new token behind `context` cached ones of the current chunk (softmax, rotary). */
+typedef struct {
+  int64_t dtype, B, D, S, hidden, heads, groups, states, context;
+  const void* x;              /* [B, D] */
+  void* out;                  /* [B, D] */
+  const uint8_t* mask;        /* [B] or NULL */
+  const int64_t* prev_count;  /* carried state in and out, as mega_norm_ema_step */
+  const float* prev_mean;
+  const float* prev_var;
+  int64_t* count;
+  float* mean;
+  float* var;
+  const float* h_in;          /* [B, D, states, 2] or NULL */
+  float* h_out;
+  const void* k_old;          /* [B, context, S] rows k_row / k_batch elements apart, unrotated keys */
+  const void* v_old;          /* [B, context, hidden] */
+  int64_t k_row, k_batch;
+  void* k_out;                /* [B, context + 1, S], [B, context + 1, hidden], or both NULL (the chunk is full) */
+  void* v_out;
+  const float* norm_gamma;    /* [D] fp32: weight + 1, bias */
+  const float* norm_beta;
+  const float* p;             /* moving-average coefficients, fp32, complex storage */
+  const float* q;
+  const float* ema_gamma;
+  const float* omega;
+  const void* v_weight;       /* [hidden, D], [hidden] */
+  const void* v_bias;
+  const void* mx_weight;      /* [2 D + S + hidden, D], [...]: u | z | r | hx */
+  const void* mx_bias;
+  const void* h_weight;       /* [D, hidden] */
+  const void* gamma;          /* [2, S] offsets from one */
+  const void* beta;           /* [2, S] */
+  const void* move_norm_weight; /* [D] or NULL */
+  const float* cis;           /* [> context, S / heads / 2, 2] */
+  void* workspace;
+  int64_t workspace_bytes;
+  double norm_eps, move_norm_eps;
+  int64_t move_act;           /* MEGA_TOKEN_SILU or MEGA_TOKEN_RMSNORM */
+} MegaTokenAttention;
+
+size_t mega_token_attention_workspace_bytes(int64_t B, int64_t context, int64_t D, int64_t S, int64_t hidden,
+                                            int64_t heads);
+int mega_token_gated_attention(const MegaTokenAttention* a, void* stream);
+
 /* K consecutive tokens of every stream in one launch: the same result as K calls of
  * mega_norm_ema_step on x[:, k] (the reference's chunk-wise streaming, fairseq_cli/train.py:406-417,
  * with chunks of K tokens through TimestepNorm.forward and BaseMovingLayer.forward with incremental

@@ -1,0 +1,99 @@
+"""One token of every stream with carried state on the composite step (csrc/decode_layer.hip) against the operators one by
+one in fp32 with the same (16-bit rounded) weights, which is the route the oracle pins (test_gpu_model.py): logits after
+every token, the carried state after the last one, and the composite step is what ran.
+
+Tolerance (root mean square of the difference over that of the result): a logit is reached through about 30 roundings
+to the activation type, each uniform with rms 2^-9 / sqrt(3) relative for bf16 (2^-12 / sqrt(3) for fp16); sqrt(30) of
+them is 6.2e-3 (7.7e-4); three times that."""
+import copy
+import types
+
+import pytest
+import torch
+
+import fairseq_apollo_amd as M
+from gpu_util import DEV
+
+pytestmark = pytest.mark.gpu
+TOL = {torch.bfloat16: 1.9e-2, torch.float16: 2.4e-3}
+
+
+def _model(D, z, h, heads, ffn, chunk, norm_type, dtype, seed):
+    args = types.SimpleNamespace(decoder_embed_dim=D, decoder_layers=2, decoder_z_dim=z, decoder_hidden_dim=h,
+                                 decoder_n_dim=16, decoder_ffn_embed_dim=ffn, decoder_chunk_size=chunk,
+                                 norm_num_groups=4, num_heads=heads, moving_layer="cema", norm_type=norm_type,
+                                 layer_scale=norm_type == "rmsnorm")
+    torch.manual_seed(seed)
+    model = M.MegaDecoderNoCrossAttn(args, 72, torch.nn.Embedding(72, D, padding_idx=1))
+    with torch.no_grad():
+        for p in model.parameters():
+            if not bool(p.any()):
+                p.normal_(0, 0.1)
+    half = model.to(DEV).to(dtype).eval()
+    return half, copy.deepcopy(half).float()
+
+
+def _rms(a, b):
+    a = torch.view_as_real(a) if a.is_complex() else a
+    b = torch.view_as_real(b) if b.is_complex() else b
+    return float((a.double() - b.double()).norm() / b.double().norm().clamp(min=1e-30))
+
+
+# streams around the row tiles (16, 32) and the rows normalised in the projection (4); contexts around the positions per
+# workgroup (32), the first token, the token that fills the chunk, the one after it; head widths 8, 24, 64; one slab and
+# more (hidden / heads > 512), a width of whole 32-element but not 64-element pieces
+@pytest.mark.parametrize("dtype,B,D,z,h,heads,ffn,chunk,prompt,norm_type", [
+    (torch.bfloat16, 1, 64, 16, 96, 1, 96, 64, 0, "layernorm"),
+    (torch.bfloat16, 4, 96, 32, 1056, 1, 160, 64, 30, "rmsnorm"),
+    (torch.float16, 5, 96, 48, 96, 2, 96, 64, 62, "layernorm"),
+    (torch.bfloat16, 17, 128, 64, 128, 1, 64, 128, 127, "rmsnorm"),
+    (torch.float16, 33, 64, 32, 64, 4, 64, 256, 160, "layernorm"),
+    (torch.bfloat16, 64, 64, 16, 64, 2, 64, -1, 33, "layernorm"),
+])
+def test_token_by_token_logits(dtype, B, D, z, h, heads, ffn, chunk, prompt, norm_type):
+    half, full = _model(D, z, h, heads, ffn, chunk, norm_type, dtype, 7 + B)
+    tokens = torch.randint(2, 72, (B, prompt + 4), device=DEV)
+    tokens[0, prompt + 1] = 1                              # a padded token in one stream
+    layer = half.layers[0].mega_layer
+    ran = []
+    step = layer._token_step
+    layer._token_step = lambda *a: ran.append(1) or step(*a)
+    sa, sb = {}, {}
+    with torch.no_grad():
+        for a in range(0, prompt, chunk if chunk > 0 else max(prompt, 1)):
+            sl = tokens[:, a:min(prompt, a + chunk) if chunk > 0 else prompt]
+            half(sl, incremental_state=sa)
+            full(sl, incremental_state=sb)
+        for t in range(prompt, prompt + 4):
+            la, lb = (m(tokens[:, t:t + 1], incremental_state=s)[0] for m, s in ((half, sa), (full, sb)))
+            assert la.shape == lb.shape == (B, 1, 72) and la.dtype == dtype
+            assert _rms(la, lb) < TOL[dtype], (t, _rms(la, lb))
+    assert len(ran) == 4
+    for ea, eb in zip(sa.values(), sb.values()):
+        assert sorted(ea) == sorted(eb)
+        for k in ea:
+            assert ea[k].shape == eb[k].shape, k
+            if k == "prev_count":
+                assert torch.equal(ea[k], eb[k])
+            else:
+                assert _rms(ea[k], eb[k]) < TOL[dtype], (k, _rms(ea[k], eb[k]))
+    assert M.ops.timestep_norm_status() == 0
+
+
+def test_state_of_an_earlier_token_survives_the_next():
+    """Two continuations of one carried state (beam search keeps such a state): the step writes new state tensors, the
+    old ones stay, and the second continuation equals the first."""
+    half, _ = _model(64, 16, 64, 1, 64, 64, "layernorm", torch.bfloat16, 3)
+    tokens = torch.randint(2, 72, (3, 20), device=DEV)
+    state = {}
+    with torch.no_grad():
+        half(tokens[:, :19], incremental_state=state)
+        before = {n: {k: v.clone() for k, v in e.items()} for n, e in state.items()}
+        outs = []
+        for _ in range(2):
+            mine = {n: dict(e) for n, e in state.items()}
+            outs.append(half(tokens[:, 19:], incremental_state=mine)[0])
+    assert torch.equal(outs[0], outs[1])
+    for n, e in state.items():
+        for k, v in e.items():
+            assert torch.equal(v, before[n][k]), k
