@@ -46,6 +46,13 @@ SIGNATURES = {
                                   _p, _i64, _i64, _i64, _i64, _p]),
     "mega_norm_ema_steps": (_int, [_p, _p, _p, _int, _i64, _p, _p, _p, _p, _p, _p, _p, _p, C.c_double, _p, _p, _p, _int,
                                    _p, _p, _p, _i64, _i64, _i64, _i64, _p]),
+    "mega_train_prepare": (_int, [_p, _p, _int, _int, _p, _p, _p, _p, _p, _sz, _p]),
+    "mega_ema_param_sums": (_int, [_p, _p, _int, _i64, _i64, _i64, _i64, _i64, _i64, _p, _p, _i64, _i64, _i64, _i64, _int,
+                                   _int, _p, _p, _p]),
+    "mega_ema_param_finish": (_int, [_p, _p, _p, _i64, _p, _p, _p]),
+    "mega_timestep_norm_bwd_adds": (_int, [_int, _i64, _i64, _i64, _i64]),
+    "mega_group_timestep_norm_bwd_add": (_int, [_p, _p, _p, _p, _p, _int, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64,
+                                                _i64, _p, _p, _p, _p, _p, _p, _sz, _p]),
     "mega_norm_token": (_int, [_p, _p, _int, _p, _p, _p, _p, _p, _p, _p, _p, _p, C.c_double, _i64, _i64, _i64, _p]),
     "mega_token_linear": (_int, [_p, _int, _i64, _p]),
     "mega_token_embed": (_int, [_p, _p, _int, C.c_double, _i64, _i64, _i64, _i64, _p, _p, _p]),

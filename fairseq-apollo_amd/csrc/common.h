@@ -6,6 +6,8 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include <math.h>
+
 #include "../../include/mega_hip.h"
 
 namespace mega {

@@ -213,7 +213,7 @@ extern "C" size_t mega_ema_param_grad_workspace_bytes(int64_t B, int64_t D, int6
   return align_up((size_t)B * D * N * 16, 256) + align_up((size_t)B * D * 4, 256);
 }
 
-extern "C" int mega_ema_param_grad(const void* dy, const void* x, int dtype, int64_t sgb, int64_t sgd, int64_t sgl,
+static int param_grad(float* dyx_out, const void* dy, const void* x, int dtype, int64_t sgb, int64_t sgd, int64_t sgl,
                                    int64_t sxb, int64_t sxd, int64_t sxl, const float* p, const float* q,
                                    const float* gamma, const uint8_t* mask, int64_t B, int64_t D, int64_t N,
                                    int64_t L, int reverse_time, int lag_one, float* dp, float* dq, float* dgamma,
@@ -225,9 +225,16 @@ extern "C" int mega_ema_param_grad(const void* dy, const void* x, int dtype, int
   MEGA_REQUIRE(N <= kNs, MEGA_ERR_UNSUPPORTED, "ema_param_grad: ndim=%ld > %d is not supported", (long)N, kNs);
   MEGA_REQUIRE(B * ceil_div(D, 8) < (int64_t)1 << 31 && L < (int64_t)1 << 30 && D * N < (int64_t)1 << 31,
                MEGA_ERR_UNSUPPORTED, "ema_param_grad: shape too large");
-  MEGA_REQUIRE(p && q && gamma && dp && dq && dgamma && domega, MEGA_ERR_ARG, "ema_param_grad: null pointer argument");
+  const bool finish = dyx_out == nullptr;
+  MEGA_REQUIRE(q && (!finish || (p && gamma && dp && dq && dgamma && domega)), MEGA_ERR_ARG,
+               "ema_param_grad: null pointer argument");
   hipStream_t s = (hipStream_t)stream;
   if (B == 0 || L == 0) {
+    if (!finish) {
+      zero_async(workspace, (size_t)B * D * N * 16, s);
+      zero_async(dyx_out, (size_t)B * D * 4, s);
+      return MEGA_OK;
+    }
     zero_async(dp, (size_t)D * N * 4, s);
     zero_async(dq, (size_t)D * N * 8, s);
     zero_async(dgamma, (size_t)D * N * 8, s);
@@ -235,7 +242,7 @@ extern "C" int mega_ema_param_grad(const void* dy, const void* x, int dtype, int
     return MEGA_OK;
   }
   MEGA_REQUIRE(dy && x, MEGA_ERR_ARG, "ema_param_grad: null dy / x");
-  const size_t need = mega_ema_param_grad_workspace_bytes(B, D, N);
+  const size_t need = finish ? mega_ema_param_grad_workspace_bytes(B, D, N) : (size_t)B * D * N * 16;
   MEGA_REQUIRE(workspace && workspace_bytes >= need && ((uintptr_t)workspace % 16) == 0, MEGA_ERR_WORKSPACE,
                "ema_param_grad: workspace of %zu bytes (16-byte aligned) needed", need);
   EmaGradArgs A;
@@ -249,7 +256,7 @@ extern "C" int mega_ema_param_grad(const void* dy, const void* x, int dtype, int
     A.sxl = -sxl;
   }
   A.sums = (float*)workspace;
-  A.dyx = (float*)((char*)workspace + align_up((size_t)B * D * N * 16, 256));
+  A.dyx = finish ? (float*)((char*)workspace + align_up((size_t)B * D * N * 16, 256)) : dyx_out;
   A.B = (int)B; A.D = (int)D; A.N = (int)N; A.L = (int)L;
   if (audit_on()) {
     // both forms of the kernel leave (b, channel, state) -> 4 floats and (b, channel) -> 1 float; the activations are
@@ -260,6 +267,7 @@ extern "C" int mega_ema_param_grad(const void* dy, const void* x, int dtype, int
     const int64_t hi_g = (B - 1) * sgb + (D - 1) * sgd + (L - 1) * sgl, hi_x = (B - 1) * sxb + (D - 1) * sxd + (L - 1) * sxl;
     audit_use(dy, (size_t)(hi_g + 1) * es, "ema_param_grad: dy");
     audit_use(x, (size_t)(hi_x + 1) * es, "ema_param_grad: x");
+    if (!finish) return MEGA_OK;
     audit_use(dp, (size_t)D * N * 4, "ema_param_grad: dp");
     audit_use(dq, (size_t)D * N * 8, "ema_param_grad: dq");
     audit_use(dgamma, (size_t)D * N * 8, "ema_param_grad: dgamma");
@@ -270,6 +278,7 @@ extern "C" int mega_ema_param_grad(const void* dy, const void* x, int dtype, int
                                  lag_one)) {
     ema_param_grad_tile_launch(A.dy, A.x, A.sgb, A.sgd, A.sgl, A.sxb, A.sxd, A.sxl, q, B, D, N, L, A.sums, A.dyx, s);
     MEGA_CHECK_LAUNCH("ema_param_grad (matrix-core form)");
+    if (!finish) return MEGA_OK;
     hipLaunchKernelGGL(ema_grad_finalize_kernel, dim3((unsigned)ceil_div(D * N, 256)), dim3(256), 0, s, A.sums, A.dyx,
                        p, gamma, (int)B, (int)D, (int)N, dp, dq, dgamma, domega);
     MEGA_CHECK_LAUNCH("ema_param_grad (finalize)");
@@ -305,8 +314,27 @@ extern "C" int mega_ema_param_grad(const void* dy, const void* x, int dtype, int
   }
 #undef LAUNCH_PG
   MEGA_CHECK_LAUNCH("ema_param_grad");
+  if (!finish) return MEGA_OK;
   hipLaunchKernelGGL(ema_grad_finalize_kernel, dim3((unsigned)ceil_div(D * N, 256)), dim3(256), 0, s, A.sums, A.dyx, p,
                      gamma, (int)B, (int)D, (int)N, dp, dq, dgamma, domega);
   MEGA_CHECK_LAUNCH("ema_param_grad (finalize)");
   return MEGA_OK;
+}
+
+extern "C" int mega_ema_param_grad(const void* dy, const void* x, int dtype, int64_t sgb, int64_t sgd, int64_t sgl,
+                                   int64_t sxb, int64_t sxd, int64_t sxl, const float* p, const float* q,
+                                   const float* gamma, const uint8_t* mask, int64_t B, int64_t D, int64_t N,
+                                   int64_t L, int reverse_time, int lag_one, float* dp, float* dq, float* dgamma,
+                                   float* domega, void* workspace, size_t workspace_bytes, void* stream) {
+  return param_grad(nullptr, dy, x, dtype, sgb, sgd, sgl, sxb, sxd, sxl, p, q, gamma, mask, B, D, N, L, reverse_time, lag_one,
+                    dp, dq, dgamma, domega, workspace, workspace_bytes, stream);
+}
+
+extern "C" int mega_ema_param_sums(const void* dy, const void* x, int dtype, int64_t sgb, int64_t sgd, int64_t sgl,
+                                   int64_t sxb, int64_t sxd, int64_t sxl, const float* q, const uint8_t* mask, int64_t B,
+                                   int64_t D, int64_t N, int64_t L, int reverse_time, int lag_one, float* sums,
+                                   float* dyx, void* stream) {
+  MEGA_REQUIRE(sums && dyx, MEGA_ERR_ARG, "ema_param_sums: null pointer argument");
+  return param_grad(dyx, dy, x, dtype, sgb, sgd, sgl, sxb, sxd, sxl, nullptr, q, nullptr, mask, B, D, N, L, reverse_time,
+                    lag_one, nullptr, nullptr, nullptr, nullptr, sums, (size_t)B * D * N * 16, stream);
 }

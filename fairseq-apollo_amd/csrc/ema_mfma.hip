@@ -28,6 +28,7 @@
 //   scan   : 16-step serial scan over the segments per state (lanes 0..15, values in registers)
 //   sweep 2: K, P, C products with the true start states; y overwrites x in LDS
 #include "ema_mfma.h"
+#include "param_formulas.h"
 
 // Phase markers of the streaming kernel: a profiling build defines MEGA_TR(k) to stamp the
 // shader clock; here they expand to nothing.
@@ -64,6 +65,14 @@ struct ImageArgs {
   int is_complex;
   int lag_back;          // rows >= D exclude the current sample (backward half with shift)
   int parts;             // 1: the bf16 K / P / C operands are wanted, 2: the fp16 ones (the tables always are)
+  // from the stored parameters (RAW): the coefficients are formed here, p, q, gamma, omega are results; workgroups past
+  // the K rows form the norm's operands
+  CoeffSource S;
+  float* p_out;
+  float* q_out;
+  float* g_out;
+  float* om_out;
+  NormParamArgs norm;    // norm.gamma null: none
 };
 
 __device__ __forceinline__ float bf_split(float v, __bf16* h) {
@@ -86,10 +95,15 @@ __device__ __forceinline__ cdouble cmuld(cdouble a, cdouble b) {
 }
 __device__ __forceinline__ cfloat to_cfloat(cdouble a) { return {(float)a.re, (float)a.im}; }
 
+template <bool RAW>
 __global__ __launch_bounds__(kPrepWaves * 64) void ema_image_kernel(const ImageArgs A) {
   __shared__ __attribute__((aligned(16))) char smem[kPrepWaves * (kPowB + kAuxB)];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int kr = blockIdx.x;                        // one coefficient row per workgroup, shared by its four waves
+  if (RAW && kr >= A.K) {
+    norm_params_fwd_at(A.norm, (kr - A.K) * (kPrepWaves * 64) + (int)threadIdx.x);
+    return;
+  }
   const int lag = (kr >= A.D && A.lag_back) ? 1 : 0;
   float2* pw = (float2*)(smem + wave * kPowB);
   float* kkt = (float*)(smem + kPrepWaves * kPowB + wave * kAuxB);   // [64]: k[idx] at kkt[32 + idx]
@@ -100,7 +114,17 @@ __global__ __launch_bounds__(kPrepWaves * 64) void ema_image_kernel(const ImageA
   {
     const int n = lane & 15, blk = lane >> 4;
     float qr = 0.f, qi = 0.f, pv = 0.f, gr = 0.f, gi = 0.f;
-    if (n < A.N) {
+    if (RAW && n < A.N) {
+      const size_t o = ((size_t)kr * A.N + n);
+      const Coeff c = coeff_at(A.S, kr, n);
+      pv = c.p; qr = c.qr; qi = c.qi; gr = c.gr; gi = c.gi;
+      if (wave == 0 && blk == 0) {
+        A.p_out[o] = pv;
+        *(float2*)(A.q_out + 2 * o) = make_float2(qr, qi);
+        *(float2*)(A.g_out + 2 * o) = make_float2(gr, gi);
+        if (n == 0 && kr < A.D) A.om_out[kr] = ld(A.S.omega, A.S.dtype, kr);
+      }
+    } else if (n < A.N) {
       const size_t o = ((size_t)kr * A.N + n);
       qr = A.q[o * 2];
       qi = A.is_complex ? A.q[o * 2 + 1] : 0.f;
@@ -145,7 +169,8 @@ __global__ __launch_bounds__(kPrepWaves * 64) void ema_image_kernel(const ImageA
   __syncthreads();
   if (lane == 0) {
     if (lag) kkt[32] = 0.f;
-    if (A.omega && kr < A.D) kkt[32] += A.omega[kr];
+    if (RAW && kr < A.D) kkt[32] += ld(A.S.omega, A.S.dtype, kr);
+    else if (A.omega && kr < A.D) kkt[32] += A.omega[kr];
   }
   __syncthreads();
   uint4* img = A.image + (size_t)kr * kImgSlots * 64;
@@ -934,12 +959,12 @@ size_t ema_image_bytes(int64_t D, int64_t N, int bidirectional) {
 
 int ema_image_build(const float* p, const float* q, const float* gamma, int is_complex, const float* omega, int64_t D,
                     int64_t N, int bidirectional, int shift, void* image, hipStream_t s, int parts) {
-  ImageArgs A;
+  ImageArgs A = {};
   A.parts = parts;
   A.p = p; A.q = q; A.gamma = gamma; A.omega = omega; A.image = (uint4*)image;
   A.K = (int)(bidirectional ? 2 * D : D); A.D = (int)D; A.N = (int)N; A.is_complex = is_complex;
   A.lag_back = shift ? 1 : 0;
-  hipLaunchKernelGGL(ema_image_kernel, dim3((unsigned)A.K), dim3(kPrepWaves * 64), 0, s, A);
+  hipLaunchKernelGGL(ema_image_kernel<false>, dim3((unsigned)A.K), dim3(kPrepWaves * 64), 0, s, A);
   MEGA_CHECK_LAUNCH("ema kernel generation");
   return MEGA_OK;
 }
@@ -1017,3 +1042,47 @@ bool ema_mfma_covers(int dtype, int64_t sxb, int64_t sxd, int64_t sxl, int64_t s
 }
 
 }  // namespace mega
+
+using namespace mega;
+
+// Everything a training forward derives from its parameters, in one launch: coefficients, operand images (only the
+// operands that kernels for `act_dtype` read: 24 of the 36 KB of a row for bf16), the norm's operands.  Three launches
+// before (coefficients 4.0, images 11.0, norm 2.9 us at 1024 channels; here 11.7).
+extern "C" int mega_train_prepare(const MegaEmaParams* e, const MegaNormParams* norm, int act_dtype, int shift, float* p,
+                                  float* q, float* gamma, float* omega, void* image, size_t image_bytes, void* stream) {
+  MEGA_REQUIRE(e && p && q && gamma && omega && image, MEGA_ERR_ARG, "train_prepare: null pointer argument");
+  auto known = [](int64_t d) { return d == MEGA_F32 || d == MEGA_BF16 || d == MEGA_F16; };
+  MEGA_REQUIRE(known(e->dtype) && known(act_dtype) && e->D > 0 && e->N > 0 && (e->K == e->D || e->K == 2 * e->D) &&
+                   e->K < (1ll << 26),
+               MEGA_ERR_ARG, "train_prepare: bad sizes");
+  MEGA_REQUIRE(e->alpha && e->delta && e->third && e->gamma && e->omega, MEGA_ERR_ARG, "train_prepare: null pointer argument");
+  const size_t need = ema_image_bytes(e->D, e->N, e->K == 2 * e->D ? 1 : 0);
+  MEGA_REQUIRE(need > 0, MEGA_ERR_UNSUPPORTED, "train_prepare: ndim=%ld has no operand image (ndim <= 16 only)", (long)e->N);
+  MEGA_REQUIRE(image_bytes >= need && ((uintptr_t)image % 16) == 0 && ((uintptr_t)q % 8) == 0 && ((uintptr_t)gamma % 8) == 0,
+               MEGA_ERR_WORKSPACE, "train_prepare: image of %zu bytes (16-byte aligned) needed", need);
+  ImageArgs A = {};
+  A.S = coeff_source(e->alpha, e->delta, e->third, e->gamma, e->omega, (int)e->dtype, (int)e->is_complex, e->K, e->N, e->D);
+  A.image = (uint4*)image; A.K = (int)e->K; A.D = (int)e->D; A.N = (int)e->N; A.is_complex = (int)e->is_complex;
+  A.lag_back = shift ? 1 : 0;
+  A.parts = act_dtype == MEGA_BF16 ? kImgAll & ~kImgF16 : kImgAll;
+  A.p_out = p; A.q_out = q; A.g_out = gamma; A.om_out = omega;
+  int64_t blocks = e->K;
+  if (norm) {
+    MEGA_REQUIRE(known(norm->dtype) && known(norm->prior_dtype) && norm->H > 0 && norm->G > 0 && norm->B > 0 &&
+                     norm->H < (1ll << 30) && norm->B * norm->G < (1ll << 30),
+                 MEGA_ERR_ARG, "train_prepare: bad norm sizes");
+    MEGA_REQUIRE(norm->weight && norm->bias && norm->prior_mean && norm->prior_logv && norm->gamma && norm->beta &&
+                     norm->prev_mean && norm->prev_var && (!norm->prior_count || norm->prev_count),
+                 MEGA_ERR_ARG, "train_prepare: null pointer argument");
+    NormParamArgs& P = A.norm;
+    P.weight = norm->weight; P.bias = norm->bias; P.prior_mean = norm->prior_mean; P.prior_logv = norm->prior_logv;
+    P.wdtype = (int)norm->dtype; P.pdtype = (int)norm->prior_dtype; P.H = (int)norm->H; P.G = (int)norm->G; P.B = (int)norm->B;
+    P.gamma = norm->gamma; P.beta = norm->beta; P.prev_mean = norm->prev_mean; P.prev_var = norm->prev_var;
+    P.prior_count = norm->prior_count; P.prev_count = norm->prev_count;
+    const int64_t n = norm->H > norm->B * norm->G ? norm->H : norm->B * norm->G;
+    blocks += ceil_div(n > norm->B ? n : norm->B, kPrepWaves * 64);
+  }
+  hipLaunchKernelGGL(ema_image_kernel<true>, dim3((unsigned)blocks), dim3(kPrepWaves * 64), 0, (hipStream_t)stream, A);
+  MEGA_CHECK_LAUNCH("train_prepare");
+  return MEGA_OK;
+}

@@ -48,6 +48,8 @@ struct Args {
   void* stream(int i) const { return (void*)(uintptr_t)PyLong_AsUnsignedLongLong(a[i]); }
 };
 
+bool truth(PyObject* o) { return PyObject_IsTrue(o) == 1; }
+
 int dtype_code(const Tensor& x) {
   switch (x.scalar_type()) {
     case at::kFloat: return MEGA_F32;
@@ -115,7 +117,7 @@ PyObject* token_gated_attention(const Args& A) {
     a.k_batch = k.stride(0);
   }
   a.v_old = A.opt(7, T, B * n * hidden, dev);
-  const bool keep = PyObject_IsTrue(A.a[8]) == 1;
+  const bool keep = truth(A.a[8]);
   a.norm_gamma = (const float*)A.p(9, at::kFloat, D, dev);
   a.norm_beta = (const float*)A.p(10, at::kFloat, D, dev);
   a.norm_eps = A.d(11);
@@ -268,6 +270,236 @@ PyObject* norm_ema_step(const Args& A) {
   return tuple(r);
 }
 
+// ---- training: TimestepNorm -> moving average, and the moving average alone, from the stored parameters
+struct EmaIn {
+  MegaEmaParams e = {};
+  at::Device dev = at::kCPU;
+};
+// alpha, delta, third, gamma, omega at a[i..i+4]
+EmaIn ema_params(const Args& A, int i, bool is_complex, bool two_sided) {
+  EmaIn r;
+  const Tensor& alpha = A.t(i);
+  if (alpha.dim() < 2 || !alpha.is_cuda()) throw std::runtime_error(std::string(A.who) + ": alpha must be [K, N, 1] on the device");
+  r.dev = alpha.device();
+  const at::ScalarType T = alpha.scalar_type();
+  MegaEmaParams& e = r.e;
+  e.dtype = dtype_code(alpha);
+  e.is_complex = is_complex;
+  e.K = alpha.size(0);
+  e.N = alpha.size(1);
+  e.D = two_sided ? e.K / 2 : e.K;
+  e.alpha = A.p(i, T, e.K * e.N, r.dev);
+  e.delta = A.p(i + 1, T, e.K * e.N, r.dev);
+  e.third = A.p(i + 2, T, is_complex ? e.K : e.K * e.N, r.dev);
+  e.gamma = A.p(i + 3, T, e.K * e.N * (is_complex ? 2 : 1), r.dev);
+  e.omega = A.p(i + 4, T, e.D, r.dev);
+  return r;
+}
+
+// (alpha, delta, third, gamma, omega, is_complex, two_sided, shift, activations (a tensor of their type),
+//  weight | None, bias, prior mean, prior log-variance, prior count, batch, stream)
+//   -> (p, q, gamma, omega, image, norm gamma, norm beta, prior mean [B, G], prior var [B, G], count [B])
+PyObject* train_prepare(const Args& A) {
+  A.want(16);
+  const bool cplx = truth(A.a[5]), two = truth(A.a[6]);
+  const EmaIn in = ema_params(A, 0, cplx, two);
+  const MegaEmaParams& e = in.e;
+  const Tensor& like = A.t(0);
+  Tensor r[10];
+  r[0] = empty({e.K, e.N}, like, at::kFloat);
+  r[1] = empty({e.K, e.N, 2}, like, at::kFloat);
+  r[2] = empty({e.K, e.N, 2}, like, at::kFloat);
+  r[3] = empty({e.D}, like, at::kFloat);
+  const int64_t nimg = (int64_t)mega_ema_image_bytes(e.D, e.N, two ? 1 : 0);
+  if (nimg <= 0) throw std::runtime_error("train_prepare: more than 16 states have no operand image");
+  r[4] = empty({nimg}, like, at::kByte);
+  MegaNormParams n = {};
+  const bool norm = !A.none(9);
+  if (norm) {
+    const Tensor &w = A.t(9), &pm = A.t(11);
+    n.dtype = dtype_code(w);
+    n.prior_dtype = dtype_code(pm);
+    n.H = w.numel();
+    n.G = pm.numel();
+    n.B = A.i64(14);
+    n.weight = A.p(9, w.scalar_type(), n.H, in.dev);
+    n.bias = A.p(10, w.scalar_type(), n.H, in.dev);
+    n.prior_mean = A.p(11, pm.scalar_type(), n.G, in.dev);
+    n.prior_logv = A.p(12, pm.scalar_type(), n.G, in.dev);
+    n.prior_count = (const int64_t*)A.p(13, at::kLong, 1, in.dev);
+    r[5] = empty({n.H}, like, at::kFloat);
+    r[6] = empty({n.H}, like, at::kFloat);
+    r[7] = empty({n.B, n.G}, like, at::kFloat);
+    r[8] = empty({n.B, n.G}, like, at::kFloat);
+    r[9] = empty({n.B}, like, at::kLong);
+    n.gamma = (float*)r[5].data_ptr();
+    n.beta = (float*)r[6].data_ptr();
+    n.prev_mean = (float*)r[7].data_ptr();
+    n.prev_var = (float*)r[8].data_ptr();
+    n.prev_count = (int64_t*)r[9].data_ptr();
+  }
+  check(mega_train_prepare(&e, norm ? &n : nullptr, dtype_code(A.t(8)), truth(A.a[7]), (float*)r[0].data_ptr(),
+                           (float*)r[1].data_ptr(), (float*)r[2].data_ptr(), (float*)r[3].data_ptr(), r[4].data_ptr(), nimg,
+                           A.stream(15)),
+        A.who);
+  return tuple(r);
+}
+
+// (x [B, L, D], mask bytes | None, count, mean, var, norm gamma, norm beta, eps, p, q, gamma, omega, image, is_complex,
+//  y in x's layout, norm workspace, stream) -> (xn, y [B, D, L], count, cummean, cumrstd)
+PyObject* norm_move_forward(const Args& A) {
+  A.want(17);
+  const Tensor& x = A.t(0);
+  const at::Device dev = x.device();
+  if (x.dim() != 3 || !x.is_contiguous() || !x.is_cuda()) throw std::runtime_error("norm_move_forward: x must be a contiguous [B, L, D] device tensor");
+  const int64_t B = x.size(0), L = x.size(1), D = x.size(2), N = A.t(8).size(1), G = A.t(3).numel() / (B > 0 ? B : 1);
+  if (G <= 0 || D % G) throw std::runtime_error("norm_move_forward: groups");
+  const bool input = truth(A.a[14]);
+  Tensor r[5] = {at::empty_like(x), input ? at::empty({B, L, D}, x.options()).transpose(1, 2) : at::empty({B, D, L}, x.options()),
+                 empty({B}, x, at::kLong), empty({B, L, G}, x, at::kFloat), empty({B, L, G}, x, at::kFloat)};
+  Tensor stats = empty({2, B, G}, x, at::kFloat);
+  const int64_t nsc = (int64_t)mega_norm_ema_fwd_scratch_bytes(B, L, D, G, N);
+  Tensor sc = empty({nsc}, x, at::kByte);
+  const Tensor &ws = A.t(15), &img = A.t(12);
+  check(mega_norm_ema_fwd_train(
+            x.data_ptr(), r[0].data_ptr(), r[1].data_ptr(), dtype_code(x), r[1].stride(0), r[1].stride(1), r[1].stride(2),
+            (const int64_t*)A.p(2, at::kLong, B, dev), (const float*)A.p(3, at::kFloat, B * G, dev),
+            (const float*)A.p(4, at::kFloat, B * G, dev), (const float*)A.p(5, at::kFloat, D, dev),
+            (const float*)A.p(6, at::kFloat, D, dev), (const uint8_t*)A.opt(1, at::kByte, B * L, dev), A.d(7),
+            (int64_t*)r[2].data_ptr(), (float*)stats.data_ptr(), (float*)stats.data_ptr() + B * G, (float*)r[3].data_ptr(),
+            (float*)r[4].data_ptr(), (const float*)A.p(8, at::kFloat, D * N, dev), (const float*)A.p(9, at::kFloat, D * N * 2, dev),
+            (const float*)A.p(10, at::kFloat, D * N * 2, dev), truth(A.a[13]), (const float*)A.p(11, at::kFloat, D, dev), nullptr,
+            nullptr, B, L, D, G, N, img.data_ptr(), ws.data_ptr(), ws.numel(), sc.data_ptr(), nsc, A.stream(16)),
+        A.who);
+  return tuple(r);
+}
+
+// The gradient with respect to the moving average's input, [B, L, D] memory: the layer run backwards in time on the
+// output's gradient (which already lies time-major)
+Tensor adjoint(const Tensor& g, const float* p, const float* q, const float* gamma, const float* omega, const void* image,
+               int cplx, int two, int shift, int64_t N, void* stream, const char* who) {
+  const int64_t B = g.size(0), L = g.size(1), D = g.size(2), es = g.element_size();
+  Tensor dx = at::empty_like(g);
+  const int64_t nws = (int64_t)mega_ema_fwd_workspace_bytes(B, D, N, L, two, 0);
+  Tensor ws = empty({nws}, g, at::kByte);
+  const int64_t back = (L - 1) * D * es;
+  check(mega_ema_fwd((const char*)g.data_ptr() + back, (char*)dx.data_ptr() + back, dtype_code(g), L * D, 1, -D, L * D, 1, -D,
+                     p, q, gamma, cplx, omega, nullptr, nullptr, nullptr, B, D, N, L, two, 0, shift, image, ws.data_ptr(), nws,
+                     stream),
+        who);
+  return dx;
+}
+
+struct ParamGrads {
+  Tensor r[5];
+  MegaEmaParamGrads g;
+  explicit ParamGrads(const Args& A, int i) {
+    void** out[5] = {&g.alpha, &g.delta, &g.third, &g.gamma, &g.omega};
+    for (int k = 0; k < 5; ++k) {
+      r[k] = at::empty_like(A.t(i + k));
+      *out[k] = r[k].data_ptr();
+    }
+  }
+};
+
+// (xn gradient | None, y gradient [B, D, L], x, xn, mask bytes | None, prior mean, count, cummean, cumrstd, norm gamma, p, q,
+//  gamma, omega, image, weight, prior log-variance, prior needs gradients, alpha, delta, third, gamma, omega, is_complex,
+//  stream) -> (x gradient, weight, bias, prior mean | None, prior log-variance | None, alpha, delta, third, gamma, omega)
+PyObject* norm_move_backward(const Args& A) {
+  A.want(25);
+  const Tensor &x = A.t(2), &xn = A.t(3);
+  const at::Device dev = x.device();
+  const at::ScalarType T = x.scalar_type();
+  const int64_t B = x.size(0), L = x.size(1), D = x.size(2), N = A.t(10).size(1);
+  if (B <= 0 || L <= 0) throw std::runtime_error("norm_move_backward: empty input");
+  const int64_t G = A.t(5).numel() / B;
+  const int cplx = truth(A.a[23]), dt = dtype_code(x);
+  void* s = A.stream(24);
+  const EmaIn in = ema_params(A, 18, cplx, false);
+  Tensor g = A.t(1).detach();
+  if (g.scalar_type() != T) g = g.to(T);
+  if (g.dim() != 3 || g.size(0) != B || g.size(1) != D || g.size(2) != L) throw std::runtime_error("norm_move_backward: y gradient must be [B, D, L]");
+  g = g.transpose(1, 2).contiguous();                          // free when it already lies time-major
+  const float *p = (const float*)A.p(10, at::kFloat, D * N, dev), *q = (const float*)A.p(11, at::kFloat, D * N * 2, dev);
+  // The padding mask plays no part here: xn is zero at padding, so the sums over time see the masked input as it is, and
+  // what flows back to a padded token ends in the norm, which hands no gradient through it.
+  Tensor dxn = adjoint(g, p, q, (const float*)A.p(12, at::kFloat, D * N * 2, dev), (const float*)A.p(13, at::kFloat, D, dev),
+                       A.t(14).data_ptr(), cplx, 0, 1, N, s, A.who);
+  Tensor sums = empty({B * D * N * 4 + B * D}, x, at::kFloat);
+  float *sp = (float*)sums.data_ptr(), *dyx = sp + B * D * N * 4;
+  check(mega_ema_param_sums(g.data_ptr(), xn.data_ptr(), dt, L * D, 1, D, L * D, 1, D, q, nullptr, B, D, N, L, 0, 0, sp, dyx, s), A.who);
+  // the norm's backward pass on the sum of both gradients of xn
+  Tensor other;
+  if (!A.none(0)) {
+    other = A.t(0).detach();
+    if (other.scalar_type() != T) other = other.to(T);
+    other = other.contiguous();
+    if (!mega_timestep_norm_bwd_adds(dt, B, L, D, G) || (uintptr_t)other.data_ptr() % 16 || (uintptr_t)x.data_ptr() % 16) {
+      dxn.add_(other);
+      other = Tensor();
+    }
+  }
+  Tensor dx = at::empty_like(x), ng = empty({2, D}, x, at::kFloat), pg = empty({2, B, G}, x, at::kFloat);
+  const int64_t nws = (int64_t)mega_timestep_norm_bwd_workspace_bytes(dt, B, L, D, G);
+  Tensor ws = empty({nws}, x, at::kByte);
+  float *dg = (float*)ng.data_ptr(), *dpm = (float*)pg.data_ptr();
+  check(mega_group_timestep_norm_bwd_add(
+            dxn.data_ptr(), other.defined() ? other.data_ptr() : nullptr, nullptr, nullptr, x.data_ptr(), dt,
+            (const float*)A.p(5, at::kFloat, B * G, dev), (const int64_t*)A.p(6, at::kLong, B, dev), nullptr,
+            (const float*)A.p(7, at::kFloat, B * L * G, dev), (const float*)A.p(8, at::kFloat, B * L * G, dev),
+            (const float*)A.p(9, at::kFloat, D, dev), (const uint8_t*)A.opt(4, at::kByte, B * L, dev), B, L, D, G, dx.data_ptr(),
+            dpm, dpm + B * G, dg, dg + D, ws.data_ptr(), nws, s),
+        A.who);
+  const Tensor &w = A.t(15), &pl = A.t(16);
+  Tensor r[10];
+  MegaNormParamGrads n = {};
+  n.gamma_grad = dg; n.beta_grad = dg + D; n.mean_grad = dpm; n.var_grad = dpm + B * G;
+  n.prior_logv = pl.data_ptr();
+  n.dtype = dtype_code(w); n.prior_dtype = dtype_code(pl); n.H = D; n.G = G;
+  r[0] = dx;
+  r[1] = at::empty_like(w);
+  r[2] = at::empty_like(w);
+  n.weight = r[1].data_ptr();
+  n.bias = r[2].data_ptr();
+  if (truth(A.a[17])) {
+    r[3] = at::empty_like(pl);
+    r[4] = at::empty_like(pl);
+    n.prior_mean = r[3].data_ptr();
+    n.prior_logv_grad = r[4].data_ptr();
+  }
+  ParamGrads eg(A, 18);
+  check(mega_ema_param_finish(sp, dyx, &in.e, B, &eg.g, &n, s), A.who);
+  for (int k = 0; k < 5; ++k) r[5 + k] = eg.r[k];
+  return tuple(r);
+}
+
+// (y gradient, x, both with any strides of [B, D, L], mask bytes | None, q, alpha, delta, third, gamma, omega, is_complex,
+//  two_sided, shift, stream) -> gradients of (alpha, delta, third, gamma, omega)
+PyObject* ema_param_backward(const Args& A) {
+  A.want(13);
+  const Tensor &g = A.t(0), &x = A.t(1);
+  const int cplx = truth(A.a[9]), two = truth(A.a[10]), shift = truth(A.a[11]);
+  void* s = A.stream(12);
+  const EmaIn in = ema_params(A, 4, cplx, two);
+  const int64_t B = x.size(0), D = x.size(1), L = x.size(2), N = in.e.N;
+  if (x.dim() != 3 || g.sizes() != x.sizes() || g.scalar_type() != x.scalar_type() || D != in.e.D || B <= 0 || L <= 0 ||
+      x.device() != in.dev || g.device() != in.dev)
+    throw std::runtime_error("ema_param_backward: shapes");
+  const float* q = (const float*)A.p(3, at::kFloat, in.e.K * N * 2, in.dev);
+  const uint8_t* mask = (const uint8_t*)A.opt(2, at::kByte, B * L, in.dev);
+  const int halves = two ? 2 : 1;
+  Tensor sums = empty({halves * (B * D * N * 4 + B * D)}, x, at::kFloat);
+  float* dyx = (float*)sums.data_ptr() + halves * B * D * N * 4;
+  for (int h = 0; h < halves; ++h)
+    check(mega_ema_param_sums(g.data_ptr(), x.data_ptr(), dtype_code(x), g.stride(0), g.stride(1), g.stride(2), x.stride(0),
+                              x.stride(1), x.stride(2), q + h * D * N * 2, mask, B, D, N, L, h, h && shift ? 1 : 0,
+                              (float*)sums.data_ptr() + h * B * D * N * 4, dyx + h * B * D, s),
+          A.who);
+  ParamGrads eg(A, 4);
+  check(mega_ema_param_finish((const float*)sums.data_ptr(), dyx, &in.e, B, &eg.g, nullptr, s), A.who);
+  return tuple(eg.r);
+}
+
 // (dict, ...) -> bytes: storage address and in-place version of every tensor in the dictionaries' values, in order
 PyObject* tensor_versions(const Args& A) {
   int64_t buf[128];
@@ -303,7 +535,8 @@ PyObject* guarded(PyObject* (*f)(const Args&), const Args& args) {
    METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {MEGA_ENTRY(token_gated_attention), MEGA_ENTRY(token_ffn),  MEGA_ENTRY(token_embed),
                          MEGA_ENTRY(token_norm),            MEGA_ENTRY(token_linear), MEGA_ENTRY(norm_ema_step),
-                         MEGA_ENTRY(tensor_versions),
+                         MEGA_ENTRY(tensor_versions),       MEGA_ENTRY(train_prepare), MEGA_ENTRY(norm_move_forward),
+                         MEGA_ENTRY(norm_move_backward),    MEGA_ENTRY(ema_param_backward),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "mega_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

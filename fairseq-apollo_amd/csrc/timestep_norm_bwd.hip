@@ -42,6 +42,7 @@ constexpr int kMaxTileCells = 4096;   // tokens-per-tile * groups held in LDS
 
 struct TsnBwdParams {
   const void* dy;
+  const void* dy2 = nullptr;   // a second gradient of the output, added to dy (one-launch form only), or null
   const void* x;
   void* dx;
   const float* mean_grad;
@@ -607,7 +608,10 @@ __device__ __forceinline__ TileMap shfl32(const TileMap v, int l) {
 // Workgroups are handed out in the order of their ids, so tile = nt - 1 - id / B: whatever a tile waits for was
 // started before it.  512 threads: for the loads thread = (token of a round, slot of 8 channels), always the same
 // channels; for the walk thread = (group, position in walk order).
-template <typename T>
+// ADD: the output's gradient is the sum of two tensors (the moving average's and the value projection's share in the
+// layer); they are added while they are loaded, rounded once to the activation type as a separate addition would, which
+// would be one more pass over three tensors (16 us at 4 x 4096 x 1024 in bf16; here 5 us on top of 38).
+template <typename T, bool ADD>
 __global__ __launch_bounds__(kOpThreads, 4) void tsn_bwd_onepass_kernel(const TsnBwdParams P) {
   constexpr int VEC = 8;
   using V = Vec<T, VEC>;
@@ -646,6 +650,23 @@ __global__ __launch_bounds__(kOpThreads, 4) void tsn_bwd_onepass_kernel(const Ts
     const int tok = min(tokb + j * tps, ntok - 1);
     dq[j] = *(const uint4*)(dy + (size_t)tok * H + cc);
     xq[j] = *(const uint4*)(x + (size_t)tok * H + cc);
+  }
+  if (ADD) {
+    const T* dy2 = (const T*)P.dy2 + ((size_t)b * P.L + t0) * H;
+#pragma unroll
+    for (int j0 = 0; j0 < kOpNV; j0 += 2) {      // two at a time: the registers are full
+      uint4 d2[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) d2[j] = *(const uint4*)(dy2 + (size_t)min(tokb + (j0 + j) * tps, ntok - 1) * H + cc);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const V a = __builtin_bit_cast(V, dq[j0 + j]), c = __builtin_bit_cast(V, d2[j]);
+        V o;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) o.v[e] = from_float<T>(to_float(a.v[e]) + to_float(c.v[e]));
+        dq[j0 + j] = __builtin_bit_cast(uint4, o);
+      }
+    }
   }
   float gw[VEC];
   load_params<VEC>(P.gamma + cc, gw);
@@ -1152,11 +1173,17 @@ int launch_onepass(const TsnBwdParams& P, size_t rec_bytes, hipStream_t s) {
     const size_t cells = (size_t)P.TT * P.G;
     const size_t lds = (5 * cells + P.G + 2 * (size_t)P.H) * 4 + (P.TT + 2) * 4;
     static uint64_t seen = 0;
-    if (first_on_device(&seen))
-      (void)hipFuncSetAttribute((const void*)tsn_bwd_onepass_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    if (first_on_device(&seen)) {
+      (void)hipFuncSetAttribute((const void*)tsn_bwd_onepass_kernel<T, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 160 * 1024);
+      (void)hipFuncSetAttribute((const void*)tsn_bwd_onepass_kernel<T, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                160 * 1024);
+    }
     zero_async(P.rec, rec_bytes, s);       // tile and block records (one range): no word carries the tag
-    hipLaunchKernelGGL((tsn_bwd_onepass_kernel<T>), dim3((unsigned)(P.B * P.nt)), dim3(kOpThreads), lds, s, P);
+    if (P.dy2)
+      hipLaunchKernelGGL((tsn_bwd_onepass_kernel<T, true>), dim3((unsigned)(P.B * P.nt)), dim3(kOpThreads), lds, s, P);
+    else
+      hipLaunchKernelGGL((tsn_bwd_onepass_kernel<T, false>), dim3((unsigned)(P.B * P.nt)), dim3(kOpThreads), lds, s, P);
     MEGA_CHECK_LAUNCH("timestep_norm_bwd (one launch)");
     hipLaunchKernelGGL(tsn_bwd_param_kernel, dim3((unsigned)ceil_div(2 * (int64_t)P.H, 32)), dim3(256), 0, s, P);
     MEGA_CHECK_LAUNCH("timestep_norm_bwd (parameters)");
@@ -1183,7 +1210,14 @@ extern "C" size_t mega_timestep_norm_bwd_workspace_bytes(int dtype, int64_t B, i
 
 extern "C" void mega_test_timestep_norm_bwd_onepass(int on) { g_onepass.store(on ? 1 : 0); }
 
-extern "C" int mega_group_timestep_norm_bwd(const void* y_grad, const float* mean_grad, const float* var_grad,
+// the shapes mega_group_timestep_norm_bwd_add takes a second gradient for: the one-launch form
+extern "C" int mega_timestep_norm_bwd_adds(int dtype, int64_t B, int64_t L, int64_t H, int64_t G) {
+  BwdGeom g;
+  if (B <= 0 || L <= 0 || H <= 0 || G <= 0 || H % G != 0 || !bwd_geometry(dtype, B, L, H, G, &g)) return 0;
+  return g.onepass && g.vec == 8 && g_onepass.load() != 0 ? 1 : 0;
+}
+
+extern "C" int mega_group_timestep_norm_bwd_add(const void* y_grad, const void* y_grad2, const float* mean_grad, const float* var_grad,
                                             const void* x, int dtype, const float* prev_mean, const int64_t* count,
                                             const float* group_mean, const float* cummean, const float* cumrstd,
                                             const float* gamma, const uint8_t* mask, int64_t B, int64_t L, int64_t H,
@@ -1215,6 +1249,10 @@ extern "C" int mega_group_timestep_norm_bwd(const void* y_grad, const float* mea
   MEGA_REQUIRE(bwd_geometry(dtype, B, L, H, G, &g), MEGA_ERR_UNSUPPORTED,
                "timestep_norm_bwd: H=%ld G=%ld outside the supported envelope (H <= 8192, G <= %d)", (long)H, (long)G,
                kMaxTileCells);
+  MEGA_REQUIRE(!y_grad2 || ((uintptr_t)y_grad2 % 16 == 0 && (uintptr_t)y_grad % 16 == 0 && (uintptr_t)x % 16 == 0 &&
+                            (uintptr_t)x_grad % 16 == 0 && (uintptr_t)gamma % 16 == 0 &&
+                            mega_timestep_norm_bwd_adds(dtype, B, L, H, G)),
+               MEGA_ERR_UNSUPPORTED, "timestep_norm_bwd: a second gradient is taken by the one-launch form only");
   if (g.vec > 1 && ((((uintptr_t)y_grad | (uintptr_t)x | (uintptr_t)x_grad | (uintptr_t)gamma) % 16) != 0))
     g.vec = 1;                             // element-wise tiling when a buffer is not 16-byte aligned
   const size_t need = bwd_workspace_need(g);
@@ -1226,6 +1264,7 @@ extern "C" int mega_group_timestep_norm_bwd(const void* y_grad, const float* mea
   if (onepass) {
     if (!audit_on())
       if (const int rc = lookback_pending("timestep_norm_bwd")) return rc;
+    P.dy2 = y_grad2;
     P.dy = y_grad; P.x = x; P.dx = x_grad; P.mean_grad = mean_grad; P.var_grad = var_grad; P.prev_mean = prev_mean;
     P.count = count; P.group_mean = group_mean; P.cummean = cummean; P.cumrstd = cumrstd; P.gamma = gamma; P.mask = mask;
     P.agg = nullptr; P.state = nullptr;
@@ -1244,6 +1283,7 @@ extern "C" int mega_group_timestep_norm_bwd(const void* y_grad, const float* mea
       else audit_use(P.rec, 32, "timestep_norm_bwd: block records (none)");
       audit_use(P.part, (size_t)B * g.op_nt * 2 * H * 4, "timestep_norm_bwd: parameter-gradient shares");
       audit_use(y_grad, (size_t)B * L * H * 2, "timestep_norm_bwd: y_grad");
+      if (y_grad2) audit_use(y_grad2, (size_t)B * L * H * 2, "timestep_norm_bwd: second y_grad");
       audit_use(x, (size_t)B * L * H * 2, "timestep_norm_bwd: x");
       audit_use(x_grad, (size_t)B * L * H * 2, "timestep_norm_bwd: x_grad");
       audit_use(cummean, (size_t)B * L * G * 4, "timestep_norm_bwd: cummean");
@@ -1313,6 +1353,18 @@ extern "C" int mega_group_timestep_norm_bwd(const void* y_grad, const float* mea
     case MEGA_BF16: return launch_bwd<bf16_t>(P, g.vec, s);
     default: return launch_bwd<f16_t>(P, g.vec, s);
   }
+}
+
+extern "C" int mega_group_timestep_norm_bwd(const void* y_grad, const float* mean_grad, const float* var_grad,
+                                            const void* x, int dtype, const float* prev_mean, const int64_t* count,
+                                            const float* group_mean, const float* cummean, const float* cumrstd,
+                                            const float* gamma, const uint8_t* mask, int64_t B, int64_t L, int64_t H,
+                                            int64_t G, void* x_grad, float* prev_mean_grad, float* prev_var_grad,
+                                            float* gamma_grad, float* beta_grad, void* workspace,
+                                            size_t workspace_bytes, void* stream) {
+  return mega_group_timestep_norm_bwd_add(y_grad, nullptr, mean_grad, var_grad, x, dtype, prev_mean, count, group_mean,
+                                          cummean, cumrstd, gamma, mask, B, L, H, G, x_grad, prev_mean_grad,
+                                          prev_var_grad, gamma_grad, beta_grad, workspace, workspace_bytes, stream);
 }
 
 extern "C" int mega_timestep_norm_bwd(const void* y_grad, const float* mean_grad, const float* var_grad, const void* x,

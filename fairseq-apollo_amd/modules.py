@@ -52,26 +52,37 @@ class IncrementalState(object):
 
 
 class MovingAverageFunc(torch.autograd.Function):
-    """The whole moving-average layer (one- or two-sided) as one differentiable operator: the
-    reference chains EMAParametersFunc (fused_ops/ema_parameters.py:11-33) and FFTConvFunc
-    (fused_ops/fftconv.py:13-41) plus the residual; here neither the kernel nor its gradient is
-    materialised.  Inputs (x [B, D, L], p, q, gamma, omega) as BaseMovingLayer holds them."""
+    """The whole moving-average layer (one- or two-sided) from its stored parameters as one differentiable operator:
+    the reference chains the coefficient formulas (complex_exponential_moving_average.py:79-96,
+    exponential_moving_average.py:71-80), EMAParametersFunc (fused_ops/ema_parameters.py:11-33) and FFTConvFunc
+    (fused_ops/fftconv.py:13-41) plus the residual; here neither the kernel nor its gradient is materialised, and the
+    formulas are one launch each way.  x [B, D, L]; alpha, delta, third (theta | beta), gamma, omega as BaseMovingLayer
+    holds them."""
 
     @staticmethod
-    def forward(ctx, x, p, q, gamma, omega, padding_mask, out_layout, bidirectional=False, shift=True):
-        layer = ops.PreparedEMA(p.squeeze(-1), q.squeeze(-1), gamma, omega.reshape(-1), bidirectional, None, shift)
+    def forward(ctx, x, alpha, delta, third, gamma, omega, is_complex, padding_mask, out_layout, bidirectional=False,
+                shift=True):
+        layer, _ = ops.PreparedEMA.of_parameters((alpha, delta, third, gamma, omega), is_complex, bidirectional, shift, x)
         y, _ = layer(x, padding_mask, None, want_state=False, out_layout=out_layout)
         ctx.layer = layer
-        ctx.save_for_backward(x, p, q, gamma, omega, padding_mask)
+        ctx.save_for_backward(x, alpha, delta, third, gamma, omega, padding_mask)
         return y
 
     @staticmethod
     def backward(ctx, y_grad):
-        x, p, q, gamma, omega, padding_mask = ctx.saved_tensors
-        dx, dp, dq, dg, dom = ops.ema_backward(y_grad, x, p.squeeze(-1), q.squeeze(-1), gamma, omega.reshape(-1),
-                                               padding_mask, layer=ctx.layer)
-        return (dx, dp.to(p.dtype).view_as(p), dq.to(q.dtype).view_as(q), dg.to(gamma.dtype).view_as(gamma),
-                dom.to(omega.dtype).view_as(omega), None, None, None, None)
+        x, *params, padding_mask = ctx.saved_tensors
+        layer = ctx.layer
+        g = y_grad.detach().to(x.dtype)
+        if 0 in g.stride() and g.numel() > 0:
+            g = g.contiguous()
+        dx = layer.adjoint(g, padding_mask)
+        if x.numel() == 0:
+            return (dx, *[torch.zeros_like(p) for p in params]) + (None,) * 5
+        with ops._on_device(x.device):
+            grads = ops._lib.load_host().ema_param_backward(
+                g, x.detach(), ops._mask_u8(padding_mask, x.shape[0], x.shape[2]), layer.q, *params, layer.is_complex,
+                layer.bidirectional, layer.shift, ops._stream(x.device))
+        return (dx, *grads, None, None, None, None, None)
 
 
 def _training_call(module: nn.Module, *tensors) -> bool:
@@ -93,6 +104,27 @@ def _tensor_versions(*modules: nn.Module) -> bytes:
     edit call `module.train(); module.eval()` (every mode switch drops the caches) or edit under `torch.no_grad()`
     through the parameter itself."""
     return ops._lib.load_host().tensor_versions(*[d for m in modules for d in (m._parameters, m._buffers)])
+
+
+class CoeffMovingAverageFunc(torch.autograd.Function):
+    """The same operator from coefficients (p, q, gamma, omega) that are in the graph themselves: layers of more than 16
+    states, or parameters of mixed types."""
+
+    @staticmethod
+    def forward(ctx, x, p, q, gamma, omega, padding_mask, out_layout, bidirectional=False, shift=True):
+        layer = ops.PreparedEMA(p.squeeze(-1), q.squeeze(-1), gamma, omega.reshape(-1), bidirectional, None, shift)
+        y, _ = layer(x, padding_mask, None, want_state=False, out_layout=out_layout)
+        ctx.layer = layer
+        ctx.save_for_backward(x, p, q, gamma, omega, padding_mask)
+        return y
+
+    @staticmethod
+    def backward(ctx, y_grad):
+        x, p, q, gamma, omega, padding_mask = ctx.saved_tensors
+        dx, dp, dq, dg, dom = ops.ema_backward(y_grad, x, p.squeeze(-1), q.squeeze(-1), gamma, omega.reshape(-1),
+                                               padding_mask, layer=ctx.layer)
+        return (dx, dp.to(p.dtype).view_as(p), dq.to(q.dtype).view_as(q), dg.to(gamma.dtype).view_as(gamma),
+                dom.to(omega.dtype).view_as(omega), None, None, None, None)
 
 
 class EMACoeffsFunc(torch.autograd.Function):
@@ -186,6 +218,15 @@ class BaseMovingLayer(nn.Module, IncrementalState):
                 self._coeffs = self._calc_coeffs()
             return self._coeffs
 
+    def _stored(self):
+        """(alpha, delta, theta | beta, gamma, omega)"""
+        return self.alpha, self.delta, self.theta if self.complex else self.beta, self.gamma, self.omega
+
+    def _one_launch(self) -> bool:
+        """The stored parameters go to the kernels as they are: one type, on the GPU, contiguous, at most 16 states."""
+        ts = self._stored()
+        return self.ndim <= 16 and _one_cuda_dtype(*ts) and all(t.is_contiguous() for t in ts)
+
     def _drop_stale_cache(self):
         """The eval-mode caches follow the parameters they were computed from."""
         key = _tensor_versions(self)
@@ -235,9 +276,12 @@ class BaseMovingLayer(nn.Module, IncrementalState):
         if torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in self.parameters())):
             if incremental_state is not None or (self.truncation is not None and self.truncation >= 1):
                 return self._chained_forward(x, padding_mask, incremental_state, out_layout)
+            if self._one_launch():
+                return MovingAverageFunc.apply(x, *self._stored(), self.complex, padding_mask, out_layout,
+                                               self.bidirectional, self.shift)
             p, q, gamma, omega = self._calc_all()       # stays in the graph
-            return MovingAverageFunc.apply(x, p, q, gamma, omega, padding_mask, out_layout, self.bidirectional,
-                                           self.shift)
+            return CoeffMovingAverageFunc.apply(x, p, q, gamma, omega, padding_mask, out_layout, self.bidirectional,
+                                                self.shift)
         layer = self._prepared_layer()
         if incremental_state is not None:
             saved_state = self._get_input_buffer(incremental_state)
@@ -633,43 +677,72 @@ class TimestepNorm(nn.Module, IncrementalState):
 
 
 class NormThenMoveFunc(torch.autograd.Function):
-    """x = norm(x); mx = move(x^T) as one differentiable operator whose forward is one library call
+    """x = norm(x); mx = move(x^T) from the two modules' stored parameters as one differentiable operator
     (moving_average_gated_attention.py:304-315; the reference chains GroupTimestepNormFunc,
-    norm_layer/timestep_norm.py:14-66, EMAParametersFunc and FFTConvFunc).  The forward keeps x, xn and the
-    norm's running statistics; the backward runs the moving average backwards in time on mx's gradient, adds
-    the result to xn's own gradient and hands the sum to the norm's backward pass."""
+    norm_layer/timestep_norm.py:14-66, the coefficient formulas, EMAParametersFunc and FFTConvFunc).  The forward is one
+    launch for everything derived from the parameters and one for the pair (where it has a one-kernel form); it keeps x,
+    xn and the norm's running statistics.  The backward runs the moving average backwards in time on mx's gradient and
+    hands the sum with xn's own gradient to the norm's backward pass."""
 
     ENABLED = True          # False: training runs the two modules' own operators one after the other
 
     @staticmethod
-    def forward(ctx, x, prev_count, prev_mean, prev_var, norm_gamma, norm_beta, p, q, gamma, omega, padding_mask,
-                num_groups, eps, out_layout, shift):
-        layer = ops.PreparedEMA(p.squeeze(-1), q.squeeze(-1), gamma, omega.reshape(-1), False, None, shift)
-        xn, y, count, _, _, _, cummean, cumrstd = layer.norm_forward(
-            x, prev_count, prev_mean, prev_var, norm_gamma, norm_beta, num_groups, eps, padding_mask, None,
-            want_state=False, out_layout=out_layout, want_stats=True)
+    def forward(ctx, x, weight, bias, prior_mean, prior_logv, prior_count, alpha, delta, third, gamma, omega, is_complex,
+                padding_mask, eps, out_layout):
+        B = x.shape[0]
+        xd = x.detach() if x.is_contiguous() else x.detach().contiguous()
+        layer, (ng, nb, pm, pv, pc) = ops.PreparedEMA.of_parameters(
+            (alpha, delta, third, gamma, omega), is_complex, False, True, xd,
+            (weight, bias, prior_mean, prior_logv, prior_count), B)
+        if xd.dtype is torch.bfloat16:
+            G, N, (_, L, D) = prior_mean.numel(), layer.N, xd.shape
+            stream = ops._stream(xd.device)
+            ws = ops._tsn_workspace(xd.device, ops.norm_ema_workspace_bytes(B, L, D, G, N), stream)
+            with ops._on_device(xd.device):
+                xn, y, count, cummean, cumrstd = ops._lib.load_host().norm_move_forward(
+                    xd, ops._mask_u8(padding_mask, B, L), pc, pm, pv, ng, nb, eps, layer.p, layer.q, layer.gamma,
+                    layer.omega, layer.image, is_complex, out_layout == "input", ws, stream)
+        else:
+            xn, y, count, _, _, _, cummean, cumrstd = layer.norm_forward(
+                xd, pc, pm, pv, ng, nb, prior_mean.numel(), eps, padding_mask, None, want_state=False,
+                out_layout=out_layout, want_stats=True)
         ctx.layer = layer
-        ctx.num_groups = num_groups
-        ctx.save_for_backward(x, xn, prev_mean, count, cummean, cumrstd, norm_gamma, p, q, gamma, omega, padding_mask)
+        ctx.save_for_backward(xd, xn, pm, count, cummean, cumrstd, ng, weight, prior_mean, prior_logv, alpha, delta, third,
+                              gamma, omega, padding_mask)
+        ctx.set_materialize_grads(False)
         return xn, y
 
     @staticmethod
     def backward(ctx, xn_grad, y_grad):
-        x, xn, prev_mean, count, cummean, cumrstd, norm_gamma, p, q, gamma, omega, padding_mask = ctx.saved_tensors
-        total = xn_grad
-        dp = dq = dg = dom = None
-        if y_grad is not None:
-            dxe, dp, dq, dg, dom = ops.ema_backward(y_grad, xn.transpose(1, 2), p.squeeze(-1), q.squeeze(-1), gamma,
-                                                    omega.reshape(-1), padding_mask, layer=ctx.layer)
-            dxe = dxe.transpose(1, 2)
-            total = dxe if total is None else total + dxe
-            dp, dq = dp.to(p.dtype).view_as(p), dq.to(q.dtype).view_as(q)
-            dg, dom = dg.to(gamma.dtype).view_as(gamma), dom.to(omega.dtype).view_as(omega)
-        x_grad, pm_grad, pv_grad, ng_grad, nb_grad = ops.group_timestep_norm_bwd(
-            total.contiguous(), None, None, x, prev_mean, count, None, cummean, cumrstd, norm_gamma, padding_mask,
-            ctx.num_groups)
-        return (x_grad, None, pm_grad.to(prev_mean.dtype).view_as(prev_mean), pv_grad.view_as(prev_mean),
-                ng_grad.to(norm_gamma.dtype), nb_grad, dp, dq, dg, dom, None, None, None, None, None)
+        (x, xn, pm, count, cummean, cumrstd, ng, weight, prior_mean, prior_logv, *params, padding_mask) = ctx.saved_tensors
+        layer = ctx.layer
+        if y_grad is None:
+            y_grad = torch.zeros_like(xn).transpose(1, 2)
+        B, L, _ = x.shape
+        prior = prior_mean.requires_grad or prior_logv.requires_grad
+        if layer.adjoint_in_place(y_grad):
+            with ops._on_device(x.device):
+                g = ops._lib.load_host().norm_move_backward(
+                    xn_grad, y_grad, x, xn, ops._mask_u8(padding_mask, B, L), pm, count, cummean, cumrstd, ng, layer.p,
+                    layer.q, layer.gamma, layer.omega, layer.image, weight, prior_logv, prior, *params, layer.is_complex,
+                    ops._stream(x.device))
+        else:
+            # types whose moving average runs on rows in time: the operators one by one.  The mask plays no part in the
+            # moving average's share: xn is zero at padding, and the norm hands no gradient to a padded token.
+            gy = y_grad.detach().to(x.dtype)
+            if 0 in gy.stride():
+                gy = gy.contiguous()
+            dxn = layer.adjoint(gy).transpose(1, 2)
+            if xn_grad is not None:
+                dxn = dxn + xn_grad
+            dx, dpm, dpv, dng, dnb = ops.group_timestep_norm_bwd(dxn.contiguous(), None, None, x, pm, count, None, cummean,
+                                                                 cumrstd, ng, padding_mask, prior_mean.numel())
+            dn = ops.norm_params_bwd(dng, dnb, dpm, dpv, weight, prior_mean, prior_logv, B, prior)
+            with ops._on_device(x.device):
+                de = ops._lib.load_host().ema_param_backward(gy, xn.transpose(1, 2), None, layer.q, *params,
+                                                             layer.is_complex, False, True, ops._stream(x.device))
+            g = (dx, *dn, *de)
+        return (*g[:5], None, *g[5:], None, None, None, None)
 
 
 def norm_then_move(norm: nn.Module, move: nn.Module, x: Tensor, padding_mask: Optional[Tensor] = None,
@@ -685,11 +758,10 @@ def norm_then_move(norm: nn.Module, move: nn.Module, x: Tensor, padding_mask: Op
                 and not move.bidirectional and (move.truncation is None or move.truncation < 1)
                 and x.is_cuda and x.dim() == 3 and x.size(0) > 0 and x.size(1) > 0)
     training = one_call and (_training_call(norm, x) or _training_call(move, x))
-    if training and incremental_state is None and NormThenMoveFunc.ENABLED:
-        prev_count, norm_gamma, norm_beta, prev_mean, prev_var = norm._training_operands(x.size(0))
-        p, q, gamma, omega = move._calc_all()           # stay in the graph
-        return NormThenMoveFunc.apply(x, prev_count, prev_mean, prev_var, norm_gamma, norm_beta, p, q, gamma, omega,
-                                      padding_mask, norm.num_groups, norm.eps, out_layout, move.shift)
+    if training and incremental_state is None and NormThenMoveFunc.ENABLED and move._one_launch() and \
+            _one_cuda_dtype(norm.weight, norm.bias) and _one_cuda_dtype(norm.prior_mean, norm.prior_logv):
+        return NormThenMoveFunc.apply(x, norm.weight, norm.bias, norm.prior_mean, norm.prior_logv, norm.prior_count,
+                                      *move._stored(), move.complex, padding_mask, norm.eps, out_layout)
     if not one_call or training:
         xn = norm(x, padding_mask=padding_mask, incremental_state=incremental_state)
         return xn, move(xn.transpose(1, 2), padding_mask, incremental_state, out_layout=out_layout)

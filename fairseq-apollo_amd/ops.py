@@ -728,6 +728,14 @@ def transpose_2d(x: torch.Tensor, reverse_rows: bool = False, reverse_cols: bool
     return out
 
 
+def norm_ema_workspace_bytes(B: int, L: int, D: int, G: int, N: int) -> int:
+    key = ("norm_ema_ws", B, L, D, G, N)
+    n = _ws_bytes_cache.get(key)
+    if n is None:
+        n = _ws_bytes_cache[key] = _lib.load().mega_norm_ema_fwd_workspace_bytes(B, L, D, G, N)
+    return n
+
+
 class PreparedEMA:
     """Coefficients of one moving-average layer converted once to the layout the library
     takes (fp32, complex as (re, im) pairs); calling it runs the fused layer forward.
@@ -759,6 +767,26 @@ class PreparedEMA:
                                           _ptr(self.omega), self.D, self.N, 1 if self.bidirectional else 0,
                                           1 if self.shift else 0, _ptr(self.image), nimg, _stream(self.dev))
             _lib.check(rc, "ema_prepare")
+
+    @classmethod
+    def of_parameters(cls, params, is_complex: bool, bidirectional: bool, shift: bool, act: torch.Tensor, norm=None,
+                      batch: int = 0):
+        """The prepared layer of a training step, in one launch from the stored parameters: params = (alpha, delta, theta |
+        beta, gamma, omega); norm = (weight, bias, prior_mean, prior_logv, prior_count) or None.  The operand image holds
+        what kernels for activations of act's type read.  -> (layer, (norm gamma, norm beta, prior mean [B, G], prior
+        var [B, G], count [B]))."""
+        dev = act.device
+        n = (None,) * 5 if norm is None else norm
+        with _on_device(dev):
+            p, q, g, om, image, *ops_ = _lib.load_host().train_prepare(*params, is_complex, bidirectional, shift, act, *n,
+                                                                      batch, _stream(dev))
+        self = cls.__new__(cls)
+        self.dev = dev
+        self.K, self.N = p.shape
+        self.D = self.K // 2 if bidirectional else self.K
+        self.is_complex, self.bidirectional, self.trunc, self.shift = bool(is_complex), bool(bidirectional), 0, bool(shift)
+        self.p, self.q, self.gamma, self.omega, self.image = p, q, g, om, image
+        return self, ops_
 
     def __call__(self, x: torch.Tensor, padding_mask: Optional[torch.Tensor] = None,
                  h: Optional[torch.Tensor] = None, want_state: bool = False,
@@ -904,6 +932,11 @@ class PreparedEMA:
         if want_stats:
             return xn, y, count, mean, var, hc, cm, cr
         return xn, y, count, mean, var, hc
+
+    def adjoint_in_place(self, y_grad: torch.Tensor) -> bool:
+        """True when the backward of the norm -> moving average pair runs on time-major memory as it is (the streaming
+        kernels for bf16); fp32 / fp16 go through rows in time."""
+        return y_grad.dtype is torch.bfloat16 and self.image is not None
 
     def adjoint(self, y_grad: torch.Tensor, padding_mask: Optional[torch.Tensor] = None) -> torch.Tensor:
         """Gradient of the layer output with respect to its input x:

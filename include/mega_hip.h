@@ -213,6 +213,52 @@ int mega_norm_ema_step(const void* x, void* xn, void* y, int dtype, const int64_
                        int is_complex, const float* omega, const float* h_in, float* h_out,
                        int64_t B, int64_t D, int64_t G, int64_t N, void* stream);
 
+/* ---- a training step's parameter work (MultiHeadEMA / MultiHeadComplexEMA and TimestepNorm) in one launch each way.
+ * The stored parameters: alpha, delta [K,N]; third = theta [K] (complex) or beta [K,N] (real); gamma [K,N,2] or [K,N];
+ * omega [D]; one element type for all of them; K = D or 2 D (two-sided).                                        */
+typedef struct {
+  const void *alpha, *delta, *third, *gamma, *omega;
+  int64_t dtype, is_complex, K, N, D;
+} MegaEmaParams;
+typedef struct {
+  void *alpha, *delta, *third, *gamma, *omega;      /* parameter gradients, the parameters' type and shapes */
+} MegaEmaParamGrads;
+typedef struct {
+  const void *weight, *bias, *prior_mean, *prior_logv;
+  int64_t dtype, prior_dtype, H, G, B;
+  float *gamma, *beta, *prev_mean, *prev_var;       /* [H], [H], [B,G], [B,G]: as mega_norm_params_fwd */
+  const int64_t* prior_count;                       /* one number spread over prev_count [B], or NULL */
+  int64_t* prev_count;
+} MegaNormParams;
+typedef struct {
+  const float *gamma_grad, *beta_grad, *mean_grad, *var_grad;   /* [H], [H], [B,G], [B,G] */
+  const void* prior_logv;
+  int64_t dtype, prior_dtype, H, G;
+  void *weight, *bias, *prior_mean, *prior_logv_grad;           /* prior gradients: both or NULL */
+} MegaNormParamGrads;
+/* -> p [K,N], q, gamma [K,N,2], omega [D] (fp32) and the operand image of mega_ema_prepare, restricted to what the
+ * kernels for activations of act_dtype read; `norm` may be NULL.                                               */
+int mega_train_prepare(const MegaEmaParams* e, const MegaNormParams* norm, int act_dtype, int shift, float* p, float* q,
+                       float* gamma, float* omega, void* image, size_t image_bytes, void* stream);
+/* The sums over time of mega_ema_param_grad (one half of a two-sided layer per call): sums [B,D,N,4] (16-byte aligned)
+ * and dy . x [B,D].                                                                                            */
+int mega_ema_param_sums(const void* dy, const void* x, int dtype, int64_t sgb, int64_t sgd, int64_t sgl, int64_t sxb,
+                        int64_t sxd, int64_t sxl, const float* q, const uint8_t* mask, int64_t B, int64_t D, int64_t N,
+                        int64_t L, int reverse_time, int lag_one, float* sums, float* dyx, void* stream);
+/* sums [halves,B,D,N,4] and the first half's dy . x [B,D] -> parameter gradients; `norm` may be NULL */
+int mega_ema_param_finish(const float* sums, const float* dyx, const MegaEmaParams* e, int64_t B,
+                          const MegaEmaParamGrads* grads, const MegaNormParamGrads* norm, void* stream);
+/* mega_group_timestep_norm_bwd with the output's gradient given as the sum of two tensors (y_grad2 may be NULL); a
+ * second tensor is taken where mega_timestep_norm_bwd_adds says 1 and the buffers are 16-byte aligned.          */
+int mega_timestep_norm_bwd_adds(int dtype, int64_t B, int64_t L, int64_t H, int64_t G);
+int mega_group_timestep_norm_bwd_add(const void* y_grad, const void* y_grad2, const float* mean_grad,
+                                     const float* var_grad, const void* x, int dtype, const float* prev_mean,
+                                     const int64_t* count, const float* group_mean, const float* cummean,
+                                     const float* cumrstd, const float* gamma, const uint8_t* mask, int64_t B, int64_t L,
+                                     int64_t H, int64_t G, void* x_grad, float* prev_mean_grad, float* prev_var_grad,
+                                     float* gamma_grad, float* beta_grad, void* workspace, size_t workspace_bytes,
+                                     void* stream);
+
 /* TimestepNorm of one token of every stream (TimestepNorm.forward with L = 1, timestep_norm.py:100-139):
  *   x, xn [B,D]; mask [B] (non-zero at padding: the token leaves as zeros and the statistics stay) or NULL;
  *   prev_* / count, mean, var as mega_norm_ema_step.                                                     */
