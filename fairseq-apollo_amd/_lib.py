@@ -46,6 +46,15 @@ SIGNATURES = {
                                   _p, _i64, _i64, _i64, _i64, _p]),
     "mega_norm_ema_steps": (_int, [_p, _p, _p, _int, _i64, _p, _p, _p, _p, _p, _p, _p, _p, C.c_double, _p, _p, _p, _int,
                                    _p, _p, _p, _i64, _i64, _i64, _i64, _p]),
+    "mega_row_norm_covers": (_int, [_int, _i64]),
+    "mega_row_norm_fwd": (_int, [_p, _i64, _p, _p, _p, _int, _int, _i64, _i64, C.c_double, _p]),
+    "mega_row_norm_bwd_workspace_bytes": (_sz, [_i64, _i64]),
+    "mega_row_norm_bwd": (_int, [_p, _p, _i64, _p, _p, _p, _p, _p, _int, _int, _i64, _i64, C.c_double, _p, _sz, _p]),
+    "mega_sum_rows_workspace_bytes": (_sz, [_int, _i64, _i64]),
+    "mega_sum_rows": (_int, [_p, _i64, _p, _p, _int, _i64, _i64, _p, _p, _sz, _p]),
+    "mega_gate_qk_fwd_raw": (_int, [_p, _i64, _p, _p, _p, _p, _p, _int, _i64, _i64, _i64, _i64, _i64, C.c_double, _p]),
+    "mega_gate_qk_bwd_raw": (_int, [_p, _p, _p, _i64, _p, _p, _p, _i64, _p, _p, _int, _i64, _i64, _i64, _i64, _i64,
+                                    C.c_double, _p, _sz, _p]),
     "mega_train_prepare": (_int, [_p, _p, _int, _int, _p, _p, _p, _p, _p, _sz, _p]),
     "mega_ema_param_sums": (_int, [_p, _p, _int, _i64, _i64, _i64, _i64, _i64, _i64, _p, _p, _i64, _i64, _i64, _i64, _int,
                                    _int, _p, _p, _p]),

@@ -28,6 +28,7 @@ SOURCES = [
     "decode_layer.hip",
     "elementwise.hip",
     "gate_glue.hip",
+    "row_norm.hip",
     "attention.hip",
     "attention_mfma.hip",
     "long_conv.hip",

@@ -65,13 +65,16 @@ __global__ __launch_bounds__(kRowThreads) void rms_norm_kernel(const T* __restri
 // pos = pos0 + token index within its chunk.
 template <typename T, int VEC>
 __global__ __launch_bounds__(kRowThreads) void gate_qk_kernel(const T* __restrict__ z, int64_t zs,
-                                                              const float* __restrict__ gamma,
-                                                              const float* __restrict__ beta,
+                                                              const void* __restrict__ gamma_,
+                                                              const void* __restrict__ beta_, int raw,
                                                               const float* __restrict__ freqs, T* __restrict__ q,
                                                               T* __restrict__ k, int64_t T_, int S, int Hd,
                                                               int64_t chunk, int64_t pos0, float eps) {
   using V = Vec<T, VEC>;
   static_assert(VEC % 2 == 0, "pairs of features stay inside one vector");
+  // raw: the stored parameters (gamma as its offset from one) in the activation type; otherwise fp32 multipliers
+  auto gamma = [&](int i) { return raw ? to_float(((const T*)gamma_)[i]) + 1.0f : ((const float*)gamma_)[i]; };
+  auto beta = [&](int i) { return raw ? to_float(((const T*)beta_)[i]) : ((const float*)beta_)[i]; };
   const int lane = threadIdx.x & 63;
   const int64_t t = (int64_t)blockIdx.x * kRowsPerWg + (threadIdx.x >> 6);
   if (t >= T_) return;
@@ -98,8 +101,8 @@ __global__ __launch_bounds__(kRowThreads) void gate_qk_kernel(const T* __restric
       float sn, cs;
       sincosf(pos * freqs[(f % Hd) >> 1], &sn, &cs);
       const float z0 = to_float(v.v[i]) * inv, z1 = to_float(v.v[i + 1]) * inv;
-      const float q0 = fmaf(z0, gamma[f], beta[f]), q1 = fmaf(z1, gamma[f + 1], beta[f + 1]);
-      const float k0 = fmaf(z0, gamma[S + f], beta[S + f]), k1 = fmaf(z1, gamma[S + f + 1], beta[S + f + 1]);
+      const float q0 = fmaf(z0, gamma(f), beta(f)), q1 = fmaf(z1, gamma(f + 1), beta(f + 1));
+      const float k0 = fmaf(z0, gamma(S + f), beta(S + f)), k1 = fmaf(z1, gamma(S + f + 1), beta(S + f + 1));
       oq.v[i] = from_float<T>(q0 * cs - q1 * sn);
       oq.v[i + 1] = from_float<T>(q0 * sn + q1 * cs);
       ok.v[i] = from_float<T>(k0 * cs - k1 * sn);
@@ -122,12 +125,13 @@ __global__ __launch_bounds__(kRowThreads) void gate_qk_kernel(const T* __restric
 template <typename T, int VEC, int NV>
 __global__ __launch_bounds__(kRowThreads) void gate_qk_bwd_kernel(
     const T* __restrict__ dq, const T* __restrict__ dk, const T* __restrict__ z, int64_t zs,
-    const float* __restrict__ gamma, const float* __restrict__ freqs, T* __restrict__ dz, int64_t dzs,
+    const void* __restrict__ gamma_, int raw, const float* __restrict__ freqs, T* __restrict__ dz, int64_t dzs,
     float* __restrict__ part, int64_t T_, int S, int Hd, int64_t chunk, int64_t pos0, float eps) {
   using V = Vec<T, VEC>;
   static_assert(VEC % 2 == 0, "pairs of features stay inside one vector");
   extern __shared__ float s_acc[];                     // [4][S]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  auto gamma = [&](int i) { return raw ? to_float(((const T*)gamma_)[i]) + 1.0f : ((const float*)gamma_)[i]; };
   float agq[NV][VEC], abq[NV][VEC], agk[NV][VEC], abk[NV][VEC];
   float gq[NV][VEC], gk[NV][VEC], fr[NV][VEC / 2];
 #pragma unroll
@@ -136,8 +140,8 @@ __global__ __launch_bounds__(kRowThreads) void gate_qk_bwd_kernel(
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
       agq[u][i] = abq[u][i] = agk[u][i] = abk[u][i] = 0.f;
-      gq[u][i] = j + i < S ? gamma[j + i] : 0.f;
-      gk[u][i] = j + i < S ? gamma[S + j + i] : 0.f;
+      gq[u][i] = j + i < S ? gamma(j + i) : 0.f;
+      gk[u][i] = j + i < S ? gamma(S + j + i) : 0.f;
     }
 #pragma unroll
     for (int i = 0; i < VEC / 2; ++i) fr[u][i] = j + 2 * i < S ? freqs[((j + 2 * i) % Hd) >> 1] : 0.f;
@@ -235,9 +239,10 @@ __global__ __launch_bounds__(kRowThreads) void gate_qk_bwd_kernel(
 // columns; its 16 waves each add every 16th row (independent loads in flight, a fixed order inside
 // the wave), then the 16 sums of a column are added in wave order.
 constexpr int kParamSlices = 16;
+template <typename TO>
 __global__ __launch_bounds__(64 * kParamSlices) void gate_qk_param_kernel(const float* __restrict__ part, int rows,
-                                                                          int S, float* __restrict__ dgamma,
-                                                                          float* __restrict__ dbeta) {
+                                                                          int S, TO* __restrict__ dgamma,
+                                                                          TO* __restrict__ dbeta) {
   __shared__ float s_sum[kParamSlices][64];
   const int lane = threadIdx.x & 63, slice = threadIdx.x >> 6;
   const int i = blockIdx.x * 64 + lane;
@@ -259,8 +264,8 @@ __global__ __launch_bounds__(64 * kParamSlices) void gate_qk_param_kernel(const 
     float a = 0.f;
 #pragma unroll
     for (int w = 0; w < kParamSlices; ++w) a += s_sum[w][lane];
-    if (i < 2 * S) dgamma[i] = a;
-    else dbeta[i - 2 * S] = a;
+    if (i < 2 * S) dgamma[i] = from_float<TO>(a);
+    else dbeta[i - 2 * S] = from_float<TO>(a);
   }
 }
 
@@ -436,18 +441,18 @@ int launch_rms_norm(const void* x, int64_t xs, const float* w, void* y, int64_t 
 }
 
 template <typename T>
-int launch_gate_qk(const void* z, int64_t zs, const float* gamma, const float* beta, const float* freqs, void* q,
+int launch_gate_qk(const void* z, int64_t zs, const void* gamma, const void* beta, int raw, const float* freqs, void* q,
                    void* k, int64_t T_, int64_t S, int64_t Hd, int64_t chunk, int64_t pos0, float eps,
                    hipStream_t s) {
   constexpr int VEC = 16 / (int)sizeof(T);
   const unsigned grid = (unsigned)ceil_div(T_, kRowsPerWg);
   if (S % VEC == 0 && vec_ok(z, zs, sizeof(T), VEC) && vec_ok(q, S, sizeof(T), VEC) && vec_ok(k, S, sizeof(T), VEC))
-    hipLaunchKernelGGL((gate_qk_kernel<T, VEC>), dim3(grid), dim3(kRowThreads), 0, s, (const T*)z, zs, gamma, beta,
+    hipLaunchKernelGGL((gate_qk_kernel<T, VEC>), dim3(grid), dim3(kRowThreads), 0, s, (const T*)z, zs, gamma, beta, raw,
                        freqs, (T*)q, (T*)k, T_, (int)S, (int)Hd, chunk, pos0, eps);
   else {
     MEGA_REQUIRE(vec_ok(z, zs, sizeof(T), 2) && vec_ok(q, S, sizeof(T), 2) && vec_ok(k, S, sizeof(T), 2), MEGA_ERR_ARG,
                  "gate_qk_fwd: rows must start on an even element (feature pairs are moved together)");
-    hipLaunchKernelGGL((gate_qk_kernel<T, 2>), dim3(grid), dim3(kRowThreads), 0, s, (const T*)z, zs, gamma, beta,
+    hipLaunchKernelGGL((gate_qk_kernel<T, 2>), dim3(grid), dim3(kRowThreads), 0, s, (const T*)z, zs, gamma, beta, raw,
                        freqs, (T*)q, (T*)k, T_, (int)S, (int)Hd, chunk, pos0, eps);
   }
   MEGA_CHECK_LAUNCH("gate_qk_fwd");
@@ -462,8 +467,8 @@ inline int64_t gate_qk_bwd_wgs(int64_t T_) {
 }
 
 template <typename T>
-int launch_gate_qk_bwd(const void* dq, const void* dk, const void* z, int64_t zs, const float* gamma,
-                       const float* freqs, void* dz, int64_t dzs, float* dgamma, float* dbeta, float* part, int64_t T_,
+int launch_gate_qk_bwd(const void* dq, const void* dk, const void* z, int64_t zs, const void* gamma, int raw,
+                       const float* freqs, void* dz, int64_t dzs, void* dgamma, void* dbeta, float* part, int64_t T_,
                        int64_t S, int64_t Hd, int64_t chunk, int64_t pos0, float eps, hipStream_t s) {
   constexpr int VEC = 16 / (int)sizeof(T);
   MEGA_REQUIRE(S % VEC == 0 && S <= 2 * 64 * VEC && vec_ok(z, zs, sizeof(T), VEC) && vec_ok(dq, S, sizeof(T), VEC) &&
@@ -480,20 +485,24 @@ int launch_gate_qk_bwd(const void* dq, const void* dk, const void* z, int64_t zs
     audit_use(dk, (size_t)T_ * S * sizeof(T), "gate_qk_bwd: k_grad");
     audit_use(dz, (size_t)((T_ - 1) * dzs + S) * sizeof(T), "gate_qk_bwd: z_grad");
     audit_use(z, (size_t)((T_ - 1) * zs + S) * sizeof(T), "gate_qk_bwd: z");
-    audit_use(dgamma, (size_t)2 * S * 4, "gate_qk_bwd: gamma_grad");
-    audit_use(dbeta, (size_t)2 * S * 4, "gate_qk_bwd: beta_grad");
+    audit_use(dgamma, (size_t)2 * S * (raw ? sizeof(T) : 4), "gate_qk_bwd: gamma_grad");
+    audit_use(dbeta, (size_t)2 * S * (raw ? sizeof(T) : 4), "gate_qk_bwd: beta_grad");
     return MEGA_OK;
   }
   if (S <= 64 * VEC)
     hipLaunchKernelGGL((gate_qk_bwd_kernel<T, VEC, 1>), dim3(grid), dim3(kRowThreads), lds, s, (const T*)dq,
-                       (const T*)dk, (const T*)z, zs, gamma, freqs, (T*)dz, dzs, part, T_, (int)S, (int)Hd, chunk, pos0, eps);
+                       (const T*)dk, (const T*)z, zs, gamma, raw, freqs, (T*)dz, dzs, part, T_, (int)S, (int)Hd, chunk, pos0, eps);
   else
     hipLaunchKernelGGL((gate_qk_bwd_kernel<T, VEC, 2>), dim3(grid), dim3(kRowThreads), lds, s, (const T*)dq,
-                       (const T*)dk, (const T*)z, zs, gamma, freqs, (T*)dz, dzs, part, T_, (int)S, (int)Hd, chunk, pos0, eps);
+                       (const T*)dk, (const T*)z, zs, gamma, raw, freqs, (T*)dz, dzs, part, T_, (int)S, (int)Hd, chunk, pos0, eps);
   MEGA_CHECK_LAUNCH("gate_qk_bwd");
-  hipLaunchKernelGGL(gate_qk_param_kernel, dim3((unsigned)ceil_div(4 * S, 64)), dim3(64 * kParamSlices), 0, s, part,
-                     (int)grid,
-                     (int)S, dgamma, dbeta);
+  const dim3 pgrid((unsigned)ceil_div(4 * S, 64));
+  if (raw)
+    hipLaunchKernelGGL(gate_qk_param_kernel<T>, pgrid, dim3(64 * kParamSlices), 0, s, part, (int)grid, (int)S, (T*)dgamma,
+                       (T*)dbeta);
+  else
+    hipLaunchKernelGGL(gate_qk_param_kernel<float>, pgrid, dim3(64 * kParamSlices), 0, s, part, (int)grid, (int)S,
+                       (float*)dgamma, (float*)dbeta);
   MEGA_CHECK_LAUNCH("gate_qk_bwd (parameter sums)");
   return MEGA_OK;
 }
@@ -608,7 +617,7 @@ extern "C" int mega_rms_norm_fwd(const void* x, int64_t x_stride, const float* w
   MEGA_GLUE_DISPATCH(launch_rms_norm, x, x_stride, weight, y, T_, D, (float)eps, s);
 }
 
-extern "C" int mega_gate_qk_fwd(const void* z, int64_t z_stride, const float* gamma, const float* beta,
+static int gate_qk_fwd(int raw, const void* z, int64_t z_stride, const void* gamma, const void* beta,
                                 const float* freqs, void* q, void* k, int dtype, int64_t T_, int64_t S,
                                 int64_t heads, int64_t chunk, int64_t pos0, double eps, void* stream) {
   MEGA_REQUIRE(known_dtype(dtype), MEGA_ERR_ARG, "gate_qk_fwd: unknown dtype %d", dtype);
@@ -623,8 +632,20 @@ extern "C" int mega_gate_qk_fwd(const void* z, int64_t z_stride, const float* ga
                (long long)z_stride, (long long)S);
   MEGA_REQUIRE(ceil_div(T_, kRowsPerWg) < (1ll << 31), MEGA_ERR_ARG, "gate_qk_fwd: too many rows");
   hipStream_t s = (hipStream_t)stream;
-  MEGA_GLUE_DISPATCH(launch_gate_qk, z, z_stride, gamma, beta, freqs, q, k, T_, S, S / heads, chunk, pos0, (float)eps,
+  MEGA_GLUE_DISPATCH(launch_gate_qk, z, z_stride, gamma, beta, raw, freqs, q, k, T_, S, S / heads, chunk, pos0, (float)eps,
                      s);
+}
+
+extern "C" int mega_gate_qk_fwd(const void* z, int64_t z_stride, const float* gamma, const float* beta,
+                                const float* freqs, void* q, void* k, int dtype, int64_t T_, int64_t S,
+                                int64_t heads, int64_t chunk, int64_t pos0, double eps, void* stream) {
+  return gate_qk_fwd(0, z, z_stride, gamma, beta, freqs, q, k, dtype, T_, S, heads, chunk, pos0, eps, stream);
+}
+
+extern "C" int mega_gate_qk_fwd_raw(const void* z, int64_t z_stride, const void* gamma, const void* beta,
+                                    const float* freqs, void* q, void* k, int dtype, int64_t T_, int64_t S,
+                                    int64_t heads, int64_t chunk, int64_t pos0, double eps, void* stream) {
+  return gate_qk_fwd(1, z, z_stride, gamma, beta, freqs, q, k, dtype, T_, S, heads, chunk, pos0, eps, stream);
 }
 
 extern "C" size_t mega_gate_qk_bwd_workspace_bytes(int64_t T_, int64_t S) {
@@ -632,9 +653,9 @@ extern "C" size_t mega_gate_qk_bwd_workspace_bytes(int64_t T_, int64_t S) {
   return align_up((size_t)gate_qk_bwd_wgs(T_) * 4 * (size_t)S * sizeof(float), 256);
 }
 
-extern "C" int mega_gate_qk_bwd_strided(const void* q_grad, const void* k_grad, const void* z, int64_t z_stride,
-                                        const float* gamma, const float* freqs, void* z_grad, int64_t z_grad_stride,
-                                        float* gamma_grad, float* beta_grad, int dtype, int64_t T_, int64_t S,
+static int gate_qk_bwd(int raw, const void* q_grad, const void* k_grad, const void* z, int64_t z_stride,
+                                        const void* gamma, const float* freqs, void* z_grad, int64_t z_grad_stride,
+                                        void* gamma_grad, void* beta_grad, int dtype, int64_t T_, int64_t S,
                                         int64_t heads, int64_t chunk, int64_t pos0, double eps, void* workspace,
                                         size_t workspace_bytes, void* stream) {
   MEGA_REQUIRE(known_dtype(dtype), MEGA_ERR_ARG, "gate_qk_bwd: unknown dtype %d", dtype);
@@ -646,8 +667,9 @@ extern "C" int mega_gate_qk_bwd_strided(const void* q_grad, const void* k_grad, 
   MEGA_REQUIRE(gamma_grad && beta_grad, MEGA_ERR_ARG, "gate_qk_bwd: null pointer argument");
   hipStream_t s = (hipStream_t)stream;
   if (T_ == 0) {
-    zero_async(gamma_grad, (size_t)2 * S * 4, s);
-    zero_async(beta_grad, (size_t)2 * S * 4, s);
+    const size_t pb = (size_t)2 * S * (raw && dtype != MEGA_F32 ? 2 : 4);        // S is even: whole words
+    zero_async(gamma_grad, pb, s);
+    zero_async(beta_grad, pb, s);
     return MEGA_OK;
   }
   MEGA_REQUIRE(q_grad && k_grad && z && gamma && freqs && z_grad, MEGA_ERR_ARG, "gate_qk_bwd: null pointer argument");
@@ -657,8 +679,26 @@ extern "C" int mega_gate_qk_bwd_strided(const void* q_grad, const void* k_grad, 
   const size_t need = mega_gate_qk_bwd_workspace_bytes(T_, S);
   MEGA_REQUIRE(workspace && workspace_bytes >= need && ((uintptr_t)workspace % 16) == 0, MEGA_ERR_WORKSPACE,
                "gate_qk_bwd: workspace of %zu bytes (16-byte aligned) needed", need);
-  MEGA_GLUE_DISPATCH(launch_gate_qk_bwd, q_grad, k_grad, z, z_stride, gamma, freqs, z_grad, z_grad_stride, gamma_grad,
+  MEGA_GLUE_DISPATCH(launch_gate_qk_bwd, q_grad, k_grad, z, z_stride, gamma, raw, freqs, z_grad, z_grad_stride, gamma_grad,
                      beta_grad, (float*)workspace, T_, S, S / heads, chunk, pos0, (float)eps, s);
+}
+
+extern "C" int mega_gate_qk_bwd_strided(const void* q_grad, const void* k_grad, const void* z, int64_t z_stride,
+                                        const float* gamma, const float* freqs, void* z_grad, int64_t z_grad_stride,
+                                        float* gamma_grad, float* beta_grad, int dtype, int64_t T_, int64_t S,
+                                        int64_t heads, int64_t chunk, int64_t pos0, double eps, void* workspace,
+                                        size_t workspace_bytes, void* stream) {
+  return gate_qk_bwd(0, q_grad, k_grad, z, z_stride, gamma, freqs, z_grad, z_grad_stride, gamma_grad, beta_grad, dtype, T_,
+                     S, heads, chunk, pos0, eps, workspace, workspace_bytes, stream);
+}
+
+extern "C" int mega_gate_qk_bwd_raw(const void* q_grad, const void* k_grad, const void* z, int64_t z_stride,
+                                        const void* gamma, const float* freqs, void* z_grad, int64_t z_grad_stride,
+                                        void* gamma_grad, void* beta_grad, int dtype, int64_t T_, int64_t S,
+                                        int64_t heads, int64_t chunk, int64_t pos0, double eps, void* workspace,
+                                        size_t workspace_bytes, void* stream) {
+  return gate_qk_bwd(1, q_grad, k_grad, z, z_stride, gamma, freqs, z_grad, z_grad_stride, gamma_grad, beta_grad, dtype, T_,
+                     S, heads, chunk, pos0, eps, workspace, workspace_bytes, stream);
 }
 
 extern "C" int mega_gate_qk_bwd(const void* q_grad, const void* k_grad, const void* z, int64_t z_stride,

@@ -3,6 +3,7 @@
 // stream's raw handle comes from the caller (ops._stream).  No device code and no state in here.
 #include <ATen/ATen.h>
 #include <Python.h>
+#include <c10/core/GradMode.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "../../include/mega_hip.h"
@@ -500,6 +501,271 @@ PyObject* ema_param_backward(const Args& A) {
   return tuple(eg.r);
 }
 
+// ---- training: the layer around its norm, moving average and attention, forwards and backwards in few calls.  The
+// products are library GEMMs; what lies between them runs in libmega_hip.  Activations and weights share one type.
+Tensor rows2(const Tensor& t) { return t.reshape({-1, t.size(-1)}); }
+
+const void* ptr_or_null(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+Tensor opt_t(const Args& A, int i) { return A.none(i) ? Tensor() : A.t(i); }
+void same_type(const Args& A, std::initializer_list<int> at, const Tensor& x) {
+  for (int i : at)
+    if (!A.none(i) && (A.t(i).scalar_type() != x.scalar_type() || A.t(i).device() != x.device() || !A.t(i).is_contiguous()))
+      throw std::runtime_error(std::string(A.who) + ": argument " + std::to_string(i) + " must be contiguous, of the activations' type and on their device");
+}
+
+Tensor row_norm(const Tensor& x, const Tensor& w, const Tensor& b, int kind, double eps, void* s, const char* who) {
+  Tensor y = at::empty_like(x);
+  if (x.numel()) check(mega_row_norm_fwd(x.data_ptr(), x.size(-1), ptr_or_null(w), ptr_or_null(b), y.data_ptr(), dtype_code(x), kind, x.numel() / x.size(-1), x.size(-1), eps, s), who);
+  return y;
+}
+
+// (dx, dw, db); dw / db undefined where there is no parameter
+std::tuple<Tensor, Tensor, Tensor> row_norm_back(const Tensor& dy, const Tensor& x, const Tensor& w, const Tensor& b,
+                                                 const Tensor& add, int kind, double eps, void* s, const char* who) {
+  Tensor dx = at::empty_like(x), dw, db;
+  if (w.defined()) dw = at::empty_like(w);
+  if (b.defined()) db = at::empty_like(b);
+  const int64_t D = x.size(-1), T = x.numel() / D;
+  const int64_t nws = (int64_t)mega_row_norm_bwd_workspace_bytes(T, D);
+  Tensor ws = empty({nws}, x, at::kByte);
+  check(mega_row_norm_bwd(dy.data_ptr(), x.data_ptr(), D, ptr_or_null(w), ptr_or_null(add), dx.data_ptr(),
+                          dw.defined() ? dw.data_ptr() : nullptr, db.defined() ? db.data_ptr() : nullptr, dtype_code(x), kind, T,
+                          D, eps, ws.data_ptr(), nws, s),
+        who);
+  return {dx, dw, db};
+}
+
+// dx = dy silu'(x) and its sum over the tokens (x undefined: the sum of dy alone)
+std::pair<Tensor, Tensor> sum_rows(const Tensor& dy, const Tensor& x, void* s, const char* who) {
+  const int64_t W = dy.size(-1), T = dy.numel() / W;
+  Tensor dx, out = at::empty({W}, dy.options());
+  if (x.defined()) dx = at::empty_like(x);
+  const int64_t nws = (int64_t)mega_sum_rows_workspace_bytes(dtype_code(dy), T, W);
+  Tensor ws = empty({nws}, dy, at::kByte);
+  check(mega_sum_rows(dy.data_ptr(), W, ptr_or_null(x), dx.defined() ? dx.data_ptr() : nullptr, dtype_code(dy), T, W, out.data_ptr(),
+                      ws.data_ptr(), nws, s),
+        who);
+  return {dx, out};
+}
+
+Tensor silu(const Tensor& x, void* s, const char* who) {
+  Tensor y = at::empty_like(x);
+  check(mega_silu_fwd(x.data_ptr(), y.data_ptr(), dtype_code(x), x.numel(), s), who);
+  return y;
+}
+
+// (x, tensor | None, ...) -> bool: x is a GPU activation and every tensor is contiguous, of its type and device, on 16
+// bytes; `graph`: and every one asks for its gradient (the composites' backward passes form all of them)
+PyObject* same_storage(const Args& A, bool graph) {
+  const Tensor& x = A.t(0);
+  const at::ScalarType dt = x.scalar_type();
+  bool ok = x.is_cuda() && (dt == at::kFloat || dt == at::kBFloat16 || dt == at::kHalf) && x.dim() > 1 && x.numel() > 0 && !x.is_neg() &&
+            (uintptr_t)x.data_ptr() % 16 == 0;
+  for (int i = 1; ok && i < A.n; ++i)
+    if (!A.none(i)) {
+      const Tensor& t = A.t(i);
+      ok = t.scalar_type() == dt && t.device() == x.device() && t.is_contiguous() && (uintptr_t)t.data_ptr() % 16 == 0 && !t.is_neg() &&
+           (!graph || t.requires_grad());
+    }
+  return PyBool_FromLong(ok);
+}
+PyObject* uniform(const Args& A) { return same_storage(A, false); }
+PyObject* trainable(const Args& A) { return same_storage(A, true); }
+
+// (x, kind, weight | None, bias | None, eps, stream) -> y
+PyObject* row_norm_forward(const Args& A) {
+  A.want(6);
+  same_type(A, {0, 2, 3}, A.t(0));
+  return wrap(row_norm(A.t(0), opt_t(A, 2), opt_t(A, 3), (int)A.i64(1), A.d(4), A.stream(5), A.who));
+}
+
+// (dy, x, kind, weight | None, bias | None, eps, stream) -> (dx, dw, db)
+PyObject* row_norm_backward(const Args& A) {
+  A.want(7);
+  same_type(A, {0, 1, 3, 4}, A.t(1));
+  auto [dx, dw, db] = row_norm_back(A.t(0), A.t(1), opt_t(A, 3), opt_t(A, 4), Tensor(), (int)A.i64(2), A.d(5), A.stream(6), A.who);
+  Tensor r[3] = {dx, dw, db};
+  return tuple(r);
+}
+
+// x + fc2(silu(fc1(norm(x)))): (x, kind, norm weight | None, norm bias | None, eps, fc1 weight, fc1 bias, fc2 weight, stream)
+//   -> (out, n, pre, h)
+PyObject* ffn_forward(const Args& A) {
+  A.want(9);
+  const Tensor& x = A.t(0);
+  same_type(A, {0, 2, 3, 5, 6, 7}, x);
+  void* s = A.stream(8);
+  Tensor n = row_norm(x, opt_t(A, 2), opt_t(A, 3), (int)A.i64(1), A.d(4), s, A.who);
+  Tensor pre = at::addmm(A.t(6), rows2(n), A.t(5).t());
+  Tensor h = silu(pre, s, A.who);
+  Tensor out = at::addmm(rows2(x), h, A.t(7).t()).view(x.sizes());
+  Tensor r[4] = {out, n, pre, h};
+  return tuple(r);
+}
+
+// (dout, x, n, pre, h, kind, norm weight | None, norm bias | None, eps, fc1 weight, fc2 weight, stream)
+//   -> (dx, d norm weight, d norm bias, d fc1 weight, d fc1 bias, d fc2 weight)
+PyObject* ffn_backward(const Args& A) {
+  A.want(12);
+  const Tensor &x = A.t(1), &n = A.t(2), &pre = A.t(3), &h = A.t(4);
+  const Tensor dout = A.t(0).to(x.scalar_type()).contiguous();
+  same_type(A, {1, 2, 3, 4, 6, 7, 9, 10}, x);
+  void* s = A.stream(11);
+  const Tensor d2 = rows2(dout);
+  Tensor dw2 = at::mm(d2.t(), h);
+  Tensor dh = at::mm(d2, A.t(10));
+  auto [dpre, db1] = sum_rows(dh, pre, s, A.who);
+  Tensor dw1 = at::mm(dpre.t(), rows2(n));
+  Tensor dn = at::mm(dpre, A.t(9));
+  auto [dx, dnw, dnb] = row_norm_back(dn, x, opt_t(A, 6), opt_t(A, 7), dout, (int)A.i64(5), A.d(8), s, A.who);
+  Tensor r[6] = {dx, dnw, dnb, dw1, db1, dw2};
+  return tuple(r);
+}
+
+// W2 (silu(W1 n) * W3 n) + residual: (n, residual | None, W1, W3, W2, stream) -> (out, a, b, g)
+PyObject* swiglu_forward(const Args& A) {
+  A.want(6);
+  const Tensor& n = A.t(0);
+  same_type(A, {0, 1, 2, 3, 4}, n);
+  void* s = A.stream(5);
+  const Tensor n2 = rows2(n);
+  Tensor a = at::mm(n2, A.t(2).t()), b = at::mm(n2, A.t(3).t()), g = at::empty_like(a);
+  check(mega_swiglu_fwd(a.data_ptr(), b.data_ptr(), g.data_ptr(), dtype_code(n), a.numel(), s), A.who);
+  Tensor out = A.none(1) ? at::mm(g, A.t(4).t()) : at::addmm(rows2(A.t(1)), g, A.t(4).t());
+  auto sizes = n.sizes().vec();
+  sizes.back() = A.t(4).size(0);
+  Tensor r[4] = {out.view(sizes), a, b, g};
+  return tuple(r);
+}
+
+// (dout, n, a, b, g, W1, W3, W2, stream) -> (dn, dW1, dW3, dW2)
+PyObject* swiglu_backward(const Args& A) {
+  A.want(9);
+  const Tensor &n = A.t(1), &a = A.t(2), &b = A.t(3), &g = A.t(4);
+  same_type(A, {1, 2, 3, 4, 5, 6, 7}, n);
+  void* s = A.stream(8);
+  const Tensor d2 = rows2(A.t(0).to(n.scalar_type()).contiguous()), n2 = rows2(n);
+  Tensor dw2 = at::mm(d2.t(), g);
+  Tensor dg = at::mm(d2, A.t(7));
+  Tensor da = at::empty_like(a), db = at::empty_like(b);
+  check(mega_swiglu_bwd(dg.data_ptr(), a.data_ptr(), b.data_ptr(), da.data_ptr(), db.data_ptr(), dtype_code(n), a.numel(), s), A.who);
+  Tensor dw1 = at::mm(da.t(), n2), dw3 = at::mm(db.t(), n2);
+  Tensor dn = at::mm(da, A.t(5));
+  dn.addmm_(db, A.t(6));                         // both branches into one gradient: no third pass to add them
+  Tensor r[4] = {dn.view(n.sizes()), dw1, dw3, dw2};
+  return tuple(r);
+}
+
+// The gated attention between its norm / moving average and the attention product.
+// (xn [B, L, D], mx [B, D, L] view of time-major memory, v weight, v bias, mx weight, mx bias, gamma, beta, freqs, heads,
+//  chunk, move act, move weight | None, move eps, stream) -> (vp, v, mx (time-major), act, base, q, k)
+PyObject* mix_forward(const Args& A) {
+  A.want(15);
+  const Tensor& xn = A.t(0);
+  same_type(A, {0, 2, 3, 4, 5, 6, 7, 12}, xn);
+  void* s = A.stream(14);
+  const int dt = dtype_code(xn);
+  const int64_t D = xn.size(2), S = A.t(6).size(1), E = A.t(2).size(0), heads = A.i64(9), chunk = A.i64(10);
+  const int64_t T = xn.numel() / D, W = 2 * D + S + E;
+  const Tensor mx = A.t(1).transpose(1, 2).contiguous();
+  if (mx.scalar_type() != xn.scalar_type() || mx.sizes() != xn.sizes()) throw std::runtime_error("mix_forward: mx must be [B, D, L]");
+  Tensor vp = at::addmm(A.t(3), rows2(xn), A.t(2).t());
+  Tensor v = silu(vp, s, A.who);
+  const int act_kind = (int)A.i64(11);
+  Tensor act = act_kind == MEGA_TOKEN_RMSNORM ? row_norm(mx, opt_t(A, 12), Tensor(), act_kind, A.d(13), s, A.who) : silu(mx, s, A.who);
+  Tensor base = at::addmm(A.t(5), rows2(act), A.t(4).t());
+  Tensor q = at::empty({T, S}, xn.options()), k = at::empty({T, S}, xn.options());
+  check(mega_gate_qk_fwd_raw((const char*)base.data_ptr() + D * xn.element_size(), W, A.t(6).data_ptr(), A.t(7).data_ptr(),
+                             (const float*)A.p(8, at::kFloat, S / heads / 2, xn.device()), q.data_ptr(), k.data_ptr(), dt, T, S, heads,
+                             chunk, 0, 1e-5, s),
+        A.who);
+  Tensor r[7] = {vp, v, mx, act, base, q, k};
+  return tuple(r);
+}
+
+// (residual [B, L, D], base, attention [T, E], h weight, S, stream) -> (out, gated, hp)
+PyObject* mix_out_forward(const Args& A) {
+  A.want(6);
+  const Tensor &x = A.t(0), &base = A.t(1), &attn = A.t(2);
+  same_type(A, {0, 1, 2, 3}, x);
+  void* s = A.stream(5);
+  const int dt = dtype_code(x);
+  const int64_t D = x.size(2), E = attn.size(-1), S = A.i64(4), W = base.size(1), T = x.numel() / D, es = x.element_size();
+  const char* b = (const char*)base.data_ptr();
+  Tensor gated = at::empty({T, E}, x.options());
+  check(mega_gate_mul_fwd(attn.data_ptr(), E, b + (D + S) * es, W, gated.data_ptr(), dt, T, E, s), A.who);
+  Tensor hp = at::mm(gated, A.t(3).t());
+  Tensor out = at::empty_like(x);
+  check(mega_gate_out_fwd(x.data_ptr(), D, b, W, b + (D + S + E) * es, W, hp.data_ptr(), D, out.data_ptr(), dt, T, D, s), A.who);
+  Tensor r[3] = {out, gated, hp};
+  return tuple(r);
+}
+
+// (dout, residual, base, attention [T, E], gated, hp, h weight, S, stream) -> (d residual, d base (u, r, hx slots), d attention, d h weight)
+PyObject* mix_out_backward(const Args& A) {
+  A.want(9);
+  const Tensor &x = A.t(1), &base = A.t(2), &attn = A.t(3), &gated = A.t(4), &hp = A.t(5), &hw = A.t(6);
+  same_type(A, {1, 2, 3, 4, 5, 6}, x);
+  const Tensor dout = A.t(0).to(x.scalar_type()).contiguous();
+  void* s = A.stream(8);
+  const int dt = dtype_code(x);
+  const int64_t D = x.size(2), E = attn.size(-1), S = A.i64(7), W = base.size(1), T = x.numel() / D, es = x.element_size();
+  const char* b = (const char*)base.data_ptr();
+  Tensor dbase = at::empty_like(base), dres = at::empty_like(x);
+  char* db = (char*)dbase.data_ptr();
+  check(mega_gate_out_bwd_strided(dout.data_ptr(), x.data_ptr(), D, b, W, b + (D + S + E) * es, W, hp.data_ptr(), D, dres.data_ptr(), db,
+                                  W, db + (D + S + E) * es, W, dt, T, D, s),
+        A.who);
+  const Tensor dh = dbase.narrow(1, D + S + E, D);
+  Tensor dhw = at::mm(dh.t(), gated);
+  Tensor dgated = at::mm(dh, hw), dattn = at::empty_like(attn);
+  check(mega_gate_mul_bwd_strided(dgated.data_ptr(), attn.data_ptr(), E, b + (D + S) * es, W, dattn.data_ptr(), db + (D + S) * es, W, dt,
+                                  T, E, s),
+        A.who);
+  Tensor r[4] = {dres, dbase, dattn, dhw};
+  return tuple(r);
+}
+
+// (dq [T, S], dk, dv [T, E], dbase, xn, vp, mx, act, base, v weight, mx weight, gamma, freqs, heads, chunk, move act,
+//  move weight | None, move eps, stream)
+//   -> (d xn, d mx (time-major), d v weight, d v bias, d mx weight, d mx bias, d gamma, d beta, d move weight)
+PyObject* mix_backward(const Args& A) {
+  A.want(19);
+  const Tensor &dbase = A.t(3), &xn = A.t(4), &vp = A.t(5), &mx = A.t(6), &act = A.t(7), &base = A.t(8);
+  same_type(A, {3, 4, 5, 6, 7, 8, 9, 10, 11, 16}, xn);
+  void* s = A.stream(18);
+  const int dt = dtype_code(xn);
+  const Tensor dq = A.t(0).to(xn.scalar_type()).contiguous(), dk = A.t(1).to(xn.scalar_type()).contiguous();
+  const Tensor dv = A.t(2).to(xn.scalar_type()).contiguous();
+  const int64_t D = xn.size(2), S = A.t(11).size(1), heads = A.i64(13), chunk = A.i64(14), T = xn.numel() / D;
+  const int64_t W = base.size(1), es = xn.element_size();
+  Tensor dgamma = at::empty_like(A.t(11)), dbeta = at::empty_like(A.t(11));
+  {
+    const int64_t nws = (int64_t)mega_gate_qk_bwd_workspace_bytes(T, S);
+    Tensor ws = empty({nws}, xn, at::kByte);
+    check(mega_gate_qk_bwd_raw(dq.data_ptr(), dk.data_ptr(), (const char*)base.data_ptr() + D * es, W, A.t(11).data_ptr(),
+                               (const float*)A.p(12, at::kFloat, S / heads / 2, xn.device()), (char*)dbase.data_ptr() + D * es, W,
+                               dgamma.data_ptr(), dbeta.data_ptr(), dt, T, S, heads, chunk, 0, 1e-5, ws.data_ptr(), nws, s),
+          A.who);
+  }
+  Tensor dmxw = at::mm(dbase.t(), rows2(act));
+  Tensor dmxb = sum_rows(dbase, Tensor(), s, A.who).second;
+  Tensor dact = at::mm(dbase, A.t(10)).view(mx.sizes()), dmx, dmw;
+  const int act_kind = (int)A.i64(15);
+  if (act_kind == MEGA_TOKEN_RMSNORM) {
+    Tensor none;
+    std::tie(dmx, dmw, none) = row_norm_back(dact, mx, opt_t(A, 16), Tensor(), Tensor(), act_kind, A.d(17), s, A.who);
+  } else {
+    dmx = at::empty_like(mx);
+    check(mega_silu_bwd(dact.data_ptr(), mx.data_ptr(), dmx.data_ptr(), dt, mx.numel(), s), A.who);
+  }
+  auto [dvp, dvb] = sum_rows(dv.view(vp.sizes()), vp, s, A.who);
+  Tensor dvw = at::mm(dvp.t(), rows2(xn));
+  Tensor dxn = at::mm(dvp, A.t(9)).view(xn.sizes());
+  Tensor r[9] = {dxn, dmx, dvw, dvb, dmxw, dmxb, dgamma, dbeta, dmw};
+  return tuple(r);
+}
+
 // (dict, ...) -> bytes: storage address and in-place version of every tensor in the dictionaries' values, in order
 PyObject* tensor_versions(const Args& A) {
   int64_t buf[128];
@@ -521,6 +787,7 @@ PyObject* tensor_versions(const Args& A) {
 
 PyObject* guarded(PyObject* (*f)(const Args&), const Args& args) {
   try {
+    c10::AutoGradMode no_graph(false);
     return f(args);
   } catch (const std::exception& e) {
     if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
@@ -537,6 +804,10 @@ PyMethodDef methods[] = {MEGA_ENTRY(token_gated_attention), MEGA_ENTRY(token_ffn
                          MEGA_ENTRY(token_norm),            MEGA_ENTRY(token_linear), MEGA_ENTRY(norm_ema_step),
                          MEGA_ENTRY(tensor_versions),       MEGA_ENTRY(train_prepare), MEGA_ENTRY(norm_move_forward),
                          MEGA_ENTRY(norm_move_backward),    MEGA_ENTRY(ema_param_backward),
+                         MEGA_ENTRY(row_norm_forward),      MEGA_ENTRY(row_norm_backward), MEGA_ENTRY(ffn_forward),
+                         MEGA_ENTRY(ffn_backward),          MEGA_ENTRY(swiglu_forward), MEGA_ENTRY(swiglu_backward),
+                         MEGA_ENTRY(mix_forward),           MEGA_ENTRY(mix_out_forward), MEGA_ENTRY(mix_out_backward),
+                         MEGA_ENTRY(mix_backward),          MEGA_ENTRY(uniform),    MEGA_ENTRY(trainable),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "mega_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

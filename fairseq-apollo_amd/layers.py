@@ -22,10 +22,11 @@ from torch import Tensor, nn
 from torch.nn import Parameter
 
 from . import ops
-from .modules import (AttentionSoftmax, EfficientAttention, GateMulFunc, GateOutFunc, GateQKFunc, IncrementalState,
-                      MultiHeadComplexEMA, MultiHeadEMA, SequenceNorm, SplitFunc, SplitGrads, SwiGLU, TimestepNorm,
-                      _tensor_versions, _training_call, linear, linear_residual, mask_bytes, mask_bytes_ok,
-                      norm_then_move, silu)
+from .modules import (AttentionSoftmax, EfficientAttention, FeedForwardFunc, GateMulFunc, GateOutFunc, GateQKFunc,
+                      IncrementalState, MixInFunc, MixOutFunc, MultiHeadComplexEMA, MultiHeadEMA, SequenceNorm, SplitFunc,
+                      SplitGrads, SwiGLU, TimestepNorm, _plain, _tensor_versions, _training_call, linear, linear_residual,
+                      mask_bytes, mask_bytes_ok, norm_then_move, one_graph, row_norm, row_norm_covers, row_norm_formula,
+                      silu)
 
 
 class RMSNorm(nn.Module):
@@ -43,20 +44,17 @@ class RMSNorm(nn.Module):
             self.register_parameter("weight", None)
 
     def forward(self, x: Tensor) -> Tensor:
-        w = None if self.weight is None else self.weight.float() + 1.0
+        if row_norm_covers(x, self.weight):
+            return row_norm(x, ops.TOKEN_RMSNORM, self.weight, None, self.eps)
         if _training_call(self, x):
-            y = x.float()
-            y = y * torch.rsqrt(y.pow(2).mean(-1, keepdim=True) + self.eps)
-            if w is not None:
-                y = y * w
-            return y.to(x.dtype)
-        return ops.rms_norm_fwd(x, w, self.eps)
+            return row_norm_formula(x, ops.TOKEN_RMSNORM, self.weight, None, self.eps)
+        return ops.rms_norm_fwd(x, None if self.weight is None else self.weight.float() + 1.0, self.eps)
 
 
 class LayerNorm(nn.Module):
     """Layer normalisation with the affine weight stored as its offset from one (zero-initialised weight and bias,
     `weight + 1` in the forward): fairseq/modules/norm_layer/layer_norm.py:85-111 (FairseqLayerNorm; the fused
-    variant at :19-39 does the same).  A torch operation: it is not on the measured path."""
+    variant at :19-39 does the same).  The HIP library's row kernel on the GPU, a torch operation elsewhere."""
 
     def __init__(self, dim: int, eps: float = 1e-5, elementwise_affine: bool = True):
         super().__init__()
@@ -70,8 +68,9 @@ class LayerNorm(nn.Module):
             self.register_parameter("bias", None)
 
     def forward(self, x: Tensor) -> Tensor:
-        w = None if self.weight is None else self.weight + 1.0
-        return F.layer_norm(x, self.normalized_shape, w, self.bias, self.eps)
+        if row_norm_covers(x, self.weight, self.bias):
+            return row_norm(x, ops.TOKEN_LAYERNORM, self.weight, self.bias, self.eps)
+        return row_norm_formula(x, ops.TOKEN_LAYERNORM, self.weight, self.bias, self.eps)
 
 
 class NormalizedFeedForwardNetwork(nn.Module):
@@ -118,6 +117,10 @@ class NormalizedFeedForwardNetwork(nn.Module):
 
     def forward(self, x: Tensor, consume_input: bool = False) -> Tensor:
         """consume_input: the caller owns x and does not use it again (the residual sum may be formed in it)."""
+        if self._one_operator(x):
+            rms = isinstance(self.norm, RMSNorm)
+            return FeedForwardFunc.apply(x, self.norm.weight, None if rms else self.norm.bias, self.fc1.weight, self.fc1.bias,
+                                         self.fc2.weight, ops.TOKEN_RMSNORM if rms else ops.TOKEN_LAYERNORM, self.norm.eps)
         # hidden dropout acts whenever the module is in training mode, with or without a graph
         # (normalized_feedforward_network.py:81-83)
         if _training_call(self, x) or (self.training and self.hidden_dropout_p > 0):
@@ -133,6 +136,16 @@ class NormalizedFeedForwardNetwork(nn.Module):
         if self.layerscale_weight is not None:
             h = h * self.layerscale_weight
         return h + x
+
+    def _one_operator(self, x: Tensor) -> bool:
+        """A training call the composite operator takes (no layer scale, no active dropout, whole 16-byte rows)."""
+        norm = self.norm
+        vec = 16 // x.element_size()
+        return (one_graph(x, norm.weight, getattr(norm, 'bias', None), self.fc1.weight, self.fc1.bias, self.fc2.weight)
+                and self.layerscale_weight is None and x.shape[-1] % vec == 0 and x.shape[-1] <= 2048
+                and self.hidden_dim % vec == 0 and _plain(self.fc1, self.fc2) and type(norm) in (RMSNorm, LayerNorm)
+                and not norm._forward_hooks and not norm._forward_pre_hooks
+                and not (self.training and (self.dropout_p > 0 or self.hidden_dropout_p > 0)))
 
     def _few_rows(self, x: Tensor) -> Tensor:
         """The block on one token per stream: two launches (norm, first projection and activation; second projection,
@@ -492,6 +505,8 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
         else:
             x, mx = norm_then_move(self.norm, self.move, x, padding_mask, None, out_layout="input")
             mx = mx.transpose(1, 2)
+        if self._mix_covers(x, mx, residual):
+            return self._mix_autograd(residual, x, mx, padding_mask)
         v = silu(linear(self.v_proj, x))
         mx = self.move_act(mx) if isinstance(self.move_act, RMSNorm) else silu(mx)
         base = linear(self.mx_proj, F.dropout(mx, self.hidden_dropout_p, self.training))
@@ -522,26 +537,7 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
                 q4 = self.rel_pos_bias.rotary(q4.transpose(1, 2), 0).transpose(1, 2)
                 k4 = self.rel_pos_bias.rotary(k4.transpose(1, 2), 0).transpose(1, 2)
             q4, k4 = q4.to(z.dtype), k4.to(z.dtype)
-        if self.attention_activation != 'softmax':
-            attn = self._element_attention(q4, k4, v4, None if padding_mask is None
-                                           else padding_mask.reshape(bsz * nc, C))
-        elif simple or self._keep_weights or (self.bidirectional and padding_mask is not None) or \
-                (self._weight_dropout and self.training):
-            s = torch.einsum('bqnh,bknh->bnqk', q4, k4)
-            if simple:
-                s = s + self.rel_pos_bias(C).to(s.dtype)
-            if self.bidirectional and padding_mask is not None:
-                pad = padding_mask.reshape(bsz * nc, C).to(torch.bool)
-                pad = torch.logical_and(pad, ~pad.all(dim=-1, keepdim=True))
-                s = s.masked_fill(pad[:, None, None, :], float('-inf'))
-            w = self.attn_softmax(s)
-            if self._weight_dropout:
-                w = F.dropout(w, self.attention_dropout_p, self.training)
-            if self._keep_weights:
-                self._last_weights = w
-            attn = torch.einsum('bnqk,bknh->bqnh', w, v4)
-        else:
-            attn = self.efficient_attn(q4, k4, v4)
+        attn = self._attention_autograd(q4, k4, v4, padding_mask)
         gated = GateMulFunc.apply(attn.reshape(bsz, seq_len, self.hdim), r, (arena, 2))
         hp = linear(self.h_proj, F.dropout(gated, self.hidden_dropout_p, self.training))
         if self.training and self.dropout_p > 0:
@@ -550,6 +546,61 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
             h = F.dropout(F.silu(hx + hp), self.dropout_p, True)
             return torch.addcmul(residual, torch.sigmoid(u), h - residual)
         return GateOutFunc.apply(residual, u, hx, hp, (arena, 0, 3))
+
+    def _mix_covers(self, xn: Tensor, mx: Tensor, residual: Tensor) -> bool:
+        """The layer between its norm and its output as two operators around the attention (MixInFunc, MixOutFunc): one
+        type throughout, whole 16-byte slices, nothing dropped between them."""
+        vec = 16 // xn.element_size()
+        act = self.move_act
+        rms = isinstance(act, RMSNorm)
+        return (one_graph(xn, self.v_proj.weight, self.v_proj.bias, self.mx_proj.weight, self.mx_proj.bias, self.h_proj.weight,
+                          self.gamma, self.beta, act.weight if rms else None)
+                and mx.dtype == xn.dtype and residual.dtype == xn.dtype and residual.data_ptr() % 16 == 0
+                and self.embed_dim % vec == 0 and self.zdim % vec == 0 and self.hdim % vec == 0 and self.zdim <= 128 * vec
+                and (not rms or self.embed_dim <= 2048) and type(act) in (RMSNorm, nn.SiLU)
+                and not act._forward_hooks and not act._forward_pre_hooks
+                and _plain(self.v_proj, self.mx_proj, self.h_proj)
+                and not (self.training and (self.dropout_p > 0 or self.hidden_dropout_p > 0)))
+
+    def _mix_autograd(self, residual: Tensor, xn: Tensor, mx: Tensor, padding_mask: Optional[Tensor]) -> Tensor:
+        bsz, seq_len, _ = xn.size()
+        Nh = self.num_heads
+        C = self.chunk_size if 1 < self.chunk_size < seq_len else seq_len
+        nc = seq_len // C
+        simple = isinstance(self.rel_pos_bias, SimpleRelativePositionalBias)
+        freqs = self._no_rotation if simple else self.rel_pos_bias.freqs
+        rms = isinstance(self.move_act, RMSNorm)
+        v, base, q, k = MixInFunc.apply(
+            xn, mx.transpose(1, 2), self.v_proj.weight, self.v_proj.bias, self.mx_proj.weight, self.mx_proj.bias, self.gamma,
+            self.beta, ops._f32c(freqs), self.move_act.weight if rms else None,
+            ops.TOKEN_RMSNORM if rms else ops.TOKEN_SILU, self.move_act.eps if rms else 0.0, Nh, C)
+        attn = self._attention_autograd(q.view(bsz * nc, C, Nh, -1), k.view(bsz * nc, C, Nh, -1),
+                                        v.view(bsz * nc, C, Nh, -1), padding_mask)
+        return MixOutFunc.apply(residual, base, attn.reshape(bsz, seq_len, self.hdim), self.h_proj.weight, self.zdim)
+
+    def _attention_autograd(self, q4: Tensor, k4: Tensor, v4: Tensor, padding_mask: Optional[Tensor]) -> Tensor:
+        """Attention of whole chunks q4, k4, v4 [B chunks, C, heads, H] under autograd."""
+        simple = isinstance(self.rel_pos_bias, SimpleRelativePositionalBias)
+        if self.attention_activation != 'softmax':
+            return self._element_attention(q4, k4, v4, None if padding_mask is None
+                                           else padding_mask.reshape(q4.shape[:2]))
+        elif simple or self._keep_weights or (self.bidirectional and padding_mask is not None) or \
+                (self._weight_dropout and self.training):
+            s = torch.einsum('bqnh,bknh->bnqk', q4, k4)
+            if simple:
+                s = s + self.rel_pos_bias(q4.size(1)).to(s.dtype)
+            if self.bidirectional and padding_mask is not None:
+                pad = padding_mask.reshape(q4.shape[:2]).to(torch.bool)
+                pad = torch.logical_and(pad, ~pad.all(dim=-1, keepdim=True))
+                s = s.masked_fill(pad[:, None, None, :], float('-inf'))
+            w = self.attn_softmax(s)
+            if self._weight_dropout:
+                w = F.dropout(w, self.attention_dropout_p, self.training)
+            if self._keep_weights:
+                self._last_weights = w
+            return torch.einsum('bnqk,bknh->bqnh', w, v4)
+        else:
+            return self.efficient_attn(q4, k4, v4)
 
     def _cached_attention(self, z: Tensor, v: Tensor, saved_state, incremental_state) -> Tensor:
         """Attention with the partial-chunk key / value cache

@@ -1008,6 +1008,93 @@ def linear(lin: nn.Linear, x: Tensor) -> Tensor:
     return lin(x)
 
 
+def _plain(*layers) -> bool:
+    """Linear layers as torch defines them, nobody looking at their inputs or outputs: what reads their weights directly
+    may stand in for the calls."""
+    return all(type(m) is nn.Linear and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                                             or m._backward_pre_hooks) for m in layers)
+
+
+def one_graph(x: Tensor, *params) -> bool:
+    """True when a composite training operator may run on x and these parameters (None: absent): a graph is being built,
+    all of one type, contiguous and aligned, every parameter wants its gradient, no autocast."""
+    return torch.is_grad_enabled() and x.is_cuda and not torch.is_autocast_enabled() and \
+        ops._lib.load_host().trainable(x, *params)
+
+
+def row_norm_covers(x: Tensor, *params) -> bool:
+    D = x.shape[-1]
+    return x.is_cuda and D % (16 // x.element_size()) == 0 and D <= 2048 and not torch.is_autocast_enabled() and \
+        ops._lib.load_host().uniform(x, *params)
+
+
+class RowNormFunc(torch.autograd.Function):
+    """RMSNorm / LayerNorm over the last axis with the affine weight stored as its offset from one: one pass each way
+    (norm_layer/layer_norm.py:41-59, 85-111).  kind: ops.TOKEN_RMSNORM or ops.TOKEN_LAYERNORM."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias, kind, eps):
+        xd = x.detach().contiguous()
+        ctx.save_for_backward(x, weight, bias)
+        ctx.kind, ctx.eps = kind, eps
+        with ops._on_device(x.device):
+            return ops._lib.load_host().row_norm_forward(xd, kind, weight, bias, eps, ops._stream(x.device))
+
+    @staticmethod
+    def backward(ctx, y_grad):
+        x, weight, bias = ctx.saved_tensors
+        if torch.is_grad_enabled():                    # a graph over the backward pass: the formula in torch operations
+            ins = [t for t in (x, weight, bias) if t is not None and t.requires_grad]
+            got = iter(torch.autograd.grad(row_norm_formula(x, ctx.kind, weight, bias, ctx.eps), ins, y_grad,
+                                           create_graph=True))
+            return (*[next(got) if t is not None and t.requires_grad else None for t in (x, weight, bias)], None, None)
+        g = y_grad.to(x.dtype).contiguous()
+        with ops._on_device(x.device):
+            dx, dw, db = ops._lib.load_host().row_norm_backward(g, x.contiguous(), ctx.kind, weight, bias, ctx.eps,
+                                                                ops._stream(x.device))
+        return dx, dw, db, None, None
+
+
+def row_norm_formula(x: Tensor, kind: int, weight: Optional[Tensor], bias: Optional[Tensor], eps: float) -> Tensor:
+    w = None if weight is None else weight + 1.0
+    if kind == ops.TOKEN_LAYERNORM:
+        return F.layer_norm(x, (x.shape[-1],), w, bias, eps)
+    y = x.float()
+    y = y * torch.rsqrt(y.pow(2).mean(-1, keepdim=True) + eps)
+    return (y if w is None else y * w.float()).to(x.dtype)
+
+
+def row_norm(x: Tensor, kind: int, weight: Optional[Tensor], bias: Optional[Tensor], eps: float) -> Tensor:
+    """The norm where row_norm_covers(x, weight, bias)."""
+    if _wants_grad(x, weight, bias):
+        return RowNormFunc.apply(x, weight, bias, kind, eps)
+    with ops._on_device(x.device):
+        return ops._lib.load_host().row_norm_forward(x.contiguous(), kind, weight, bias, eps, ops._stream(x.device))
+
+
+class FeedForwardFunc(torch.autograd.Function):
+    """x + fc2(silu(fc1(norm(x)))) as one operator (normalized_feedforward_network.py:77-93): the bias gradient rides on
+    the activation's backward pass, the residual's gradient joins in the norm's."""
+
+    @staticmethod
+    def forward(ctx, x, norm_weight, norm_bias, w1, b1, w2, kind, eps):
+        xd = x.detach().contiguous()
+        with ops._on_device(x.device):
+            out, n, pre, h = ops._lib.load_host().ffn_forward(xd, kind, norm_weight, norm_bias, eps, w1, b1, w2,
+                                                              ops._stream(x.device))
+        ctx.save_for_backward(xd, n, pre, h, norm_weight, norm_bias, w1, w2)
+        ctx.kind, ctx.eps = kind, eps
+        return out
+
+    @staticmethod
+    def backward(ctx, y_grad):
+        x, n, pre, h, norm_weight, norm_bias, w1, w2 = ctx.saved_tensors
+        with ops._on_device(x.device):
+            dx, dnw, dnb, dw1, db1, dw2 = ops._lib.load_host().ffn_backward(
+                y_grad, x, n, pre, h, ctx.kind, norm_weight, norm_bias, ctx.eps, w1, w2, ops._stream(x.device))
+        return dx, dnw, dnb, dw1, db1, dw2, None, None
+
+
 class SwiGLUFunc(torch.autograd.Function):
     """silu(a) * b with its own backward."""
 
@@ -1019,6 +1106,77 @@ class SwiGLUFunc(torch.autograd.Function):
     @staticmethod
     def backward(ctx, y_grad):
         return ops.swiglu_bwd(y_grad, *ctx.saved_tensors)
+
+
+class SwiGLUBlockFunc(torch.autograd.Function):
+    """W2 (silu(W1 x) * W3 x) + residual as one operator: the two branches' gradients of x meet in a product's
+    accumulator."""
+
+    @staticmethod
+    def forward(ctx, x, residual, w1, w3, w2):
+        xd = x.detach().contiguous()
+        with ops._on_device(x.device):
+            out, a, b, g = ops._lib.load_host().swiglu_forward(xd, residual, w1, w3, w2, ops._stream(x.device))
+        ctx.save_for_backward(xd, a, b, g, w1, w3, w2)
+        ctx.residual = residual is not None
+        return out
+
+    @staticmethod
+    def backward(ctx, y_grad):
+        with ops._on_device(y_grad.device):
+            dx, dw1, dw3, dw2 = ops._lib.load_host().swiglu_backward(y_grad, *ctx.saved_tensors, ops._stream(y_grad.device))
+        return dx, y_grad if ctx.residual else None, dw1, dw3, dw2
+
+
+class MixInFunc(torch.autograd.Function):
+    """From the layer's norm and moving average to the attention's operands
+    (moving_average_gated_attention.py:313-328): v = silu(v_proj(xn)), base = mx_proj(act(mx)), q and k from base's
+    second slice.  `base` has one consumer, MixOutFunc, whose backward returns its gradient as one buffer with q's and
+    k's slice still open: this backward fills that slice in place."""
+
+    @staticmethod
+    def forward(ctx, xn, mx, v_weight, v_bias, mx_weight, mx_bias, gamma, beta, freqs, act_weight, act, eps, heads, chunk):
+        xd = xn.detach().contiguous()
+        stream = ops._stream(xn.device)
+        with ops._on_device(xn.device):
+            vp, v, mxt, a, base, q, k = ops._lib.load_host().mix_forward(
+                xd, mx.detach(), v_weight, v_bias, mx_weight, mx_bias, gamma, beta, freqs, heads, chunk, act, act_weight,
+                eps, stream)
+        ctx.save_for_backward(xd, vp, mxt, a, base, v_weight, mx_weight, gamma, freqs, act_weight)
+        ctx.consts = heads, chunk, act
+        ctx.eps = eps
+        return v, base, q, k
+
+    @staticmethod
+    def backward(ctx, dv, dbase, dq, dk):
+        xn, vp, mx, a, base, v_weight, mx_weight, gamma, freqs, act_weight = ctx.saved_tensors
+        SplitGrads.taken += 1                          # the four slices' gradients lie in one buffer
+        with ops._on_device(xn.device):
+            dxn, dmx, dvw, dvb, dmw, dmb, dgamma, dbeta, daw = ops._lib.load_host().mix_backward(
+                dq, dk, dv, dbase, xn, vp, mx, a, base, v_weight, mx_weight, gamma, freqs, *ctx.consts, act_weight, ctx.eps,
+                ops._stream(xn.device))
+        return dxn, dmx.transpose(1, 2), dvw, dvb, dmw, dmb, dgamma, dbeta, None, daw, None, None, None, None
+
+
+class MixOutFunc(torch.autograd.Function):
+    """residual + sigmoid(u) (silu(hx + h_proj(attention * silu(r))) - residual)
+    (moving_average_gated_attention.py:330, 407-412); u, r, hx are slices of MixInFunc's base [T, 2 D + S + E]."""
+
+    @staticmethod
+    def forward(ctx, residual, base, attn, h_weight, S):
+        res, at = residual.detach().contiguous(), attn.detach().contiguous()
+        with ops._on_device(res.device):
+            out, gated, hp = ops._lib.load_host().mix_out_forward(res, base, at, h_weight, S, ops._stream(res.device))
+        ctx.save_for_backward(res, base, at, gated, hp, h_weight)
+        ctx.S, ctx.attn_shape = S, attn.shape
+        return out
+
+    @staticmethod
+    def backward(ctx, y_grad):
+        with ops._on_device(y_grad.device):
+            dres, dbase, dattn, dhw = ops._lib.load_host().mix_out_backward(y_grad, *ctx.saved_tensors, ctx.S,
+                                                                            ops._stream(y_grad.device))
+        return dres, dbase, dattn.view(ctx.attn_shape), dhw, None
 
 
 class AttentionSoftmaxFunc(torch.autograd.Function):
@@ -1153,5 +1311,12 @@ class SwiGLU(nn.Module):
     def forward(self, x: Tensor, residual: Optional[Tensor] = None, consume_residual: bool = False) -> Tensor:
         """W2 (silu(W1 x) * W3 x) (+ residual, which then enters the last product as its accumulator start: no
         separate addition pass over the activations; consume_residual: see linear_residual)."""
+        w1, w3, w2 = self.w1, self.w3, self.w2
+        if one_graph(x, w1.weight, w3.weight, w2.weight) and w1.bias is None and w3.bias is None and w2.bias is None and \
+                _plain(w1, w3, w2) and (residual is None or (residual.dtype == x.dtype and residual.is_contiguous()
+                                                             and residual.device == x.device
+                                                             and residual.shape[:-1] == x.shape[:-1]
+                                                             and residual.shape[-1] == w2.out_features)):
+            return SwiGLUBlockFunc.apply(x, residual, w1.weight, w3.weight, w2.weight)
         gate = SwiGLUFunc.apply(self.w1(x), self.w3(x)) if _training_call(self, x) else ops.swiglu(self.w1(x), self.w3(x))
         return linear_residual(self.w2, gate, residual, consume_residual)

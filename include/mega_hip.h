@@ -213,6 +213,40 @@ int mega_norm_ema_step(const void* x, void* xn, void* y, int dtype, const int64_
                        int is_complex, const float* omega, const float* h_in, float* h_out,
                        int64_t B, int64_t D, int64_t G, int64_t N, void* stream);
 
+enum {
+  MEGA_TOKEN_NONE = 0,
+  MEGA_TOKEN_SILU = 1,
+  MEGA_TOKEN_RMSNORM = 2,     /* prologue: x / sqrt(mean(x^2) + eps) * (norm_weight + 1) */
+  MEGA_TOKEN_LAYERNORM = 3,   /* prologue: (x - mean) / sqrt(var + eps) * (norm_weight + 1) + norm_bias */
+  MEGA_TOKEN_RESIDUAL = 4,    /* epilogue: scale * value + residual */
+  MEGA_TOKEN_GATE = 5         /* epilogue: residual + sigmoid(gate_u) (silu(gate_hx + value) - residual) */
+};
+
+/* ---- per-token normalisations with their backward (csrc/row_norm.hip); kind: MEGA_TOKEN_RMSNORM or
+ * MEGA_TOKEN_LAYERNORM; weight [D] is stored as its offset from one, in the activations' type like bias [D] (either may be
+ * NULL); rows of at most 2048 values in whole 16-byte pieces (mega_row_norm_covers).
+ *   bwd: dx = norm's gradient + add (add may be NULL), dw, db in the activations' type (NULL: not wanted)        */
+int mega_row_norm_covers(int dtype, int64_t D);
+int mega_row_norm_fwd(const void* x, int64_t x_stride, const void* weight, const void* bias, void* y, int dtype, int kind,
+                      int64_t T, int64_t D, double eps, void* stream);
+size_t mega_row_norm_bwd_workspace_bytes(int64_t T, int64_t D);
+int mega_row_norm_bwd(const void* dy, const void* x, int64_t x_stride, const void* weight, const void* add, void* dx, void* dw,
+                      void* db, int dtype, int kind, int64_t T, int64_t D, double eps, void* workspace,
+                      size_t workspace_bytes, void* stream);
+/* out [W] = sum over the T rows of dy (x = dx = NULL), or of dx = dy silu'(x), which is written too (x, dx contiguous) */
+size_t mega_sum_rows_workspace_bytes(int dtype, int64_t T, int64_t W);
+int mega_sum_rows(const void* dy, int64_t row_stride, const void* x, void* dx, int dtype, int64_t T, int64_t W, void* out,
+                  void* workspace, size_t workspace_bytes, void* stream);
+/* mega_gate_qk_fwd / mega_gate_qk_bwd_strided on the stored parameters: gamma [2,S] as its offset from one and beta [2,S]
+ * in the activations' type; their gradients in that type                                                        */
+int mega_gate_qk_fwd_raw(const void* z, int64_t z_stride, const void* gamma, const void* beta, const float* freqs, void* q,
+                         void* k, int dtype, int64_t T, int64_t S, int64_t heads, int64_t chunk, int64_t pos0, double eps,
+                         void* stream);
+int mega_gate_qk_bwd_raw(const void* q_grad, const void* k_grad, const void* z, int64_t z_stride, const void* gamma,
+                         const float* freqs, void* z_grad, int64_t z_grad_stride, void* gamma_grad, void* beta_grad,
+                         int dtype, int64_t T, int64_t S, int64_t heads, int64_t chunk, int64_t pos0, double eps,
+                         void* workspace, size_t workspace_bytes, void* stream);
+
 /* ---- a training step's parameter work (MultiHeadEMA / MultiHeadComplexEMA and TimestepNorm) in one launch each way.
  * The stored parameters: alpha, delta [K,N]; third = theta [K] (complex) or beta [K,N] (real); gamma [K,N,2] or [K,N];
  * omega [D]; one element type for all of them; K = D or 2 D (two-sided).                                        */
@@ -271,15 +305,6 @@ int mega_norm_token(const void* x, void* xn, int dtype, const uint8_t* mask, con
  * MovingAverageGatedAttention.forward, moving_average_gated_attention.py:263-417; NormalizedFeedForwardNetwork.forward,
  * normalized_feedforward_network.py:77-93; MegaDecoderNoCrossAttn.extract_features, models/mega_lm.py:313-386).
  * 16-bit activations, at most 64 streams, weights of the activations' type.                             */
-enum {
-  MEGA_TOKEN_NONE = 0,
-  MEGA_TOKEN_SILU = 1,
-  MEGA_TOKEN_RMSNORM = 2,     /* prologue: x / sqrt(mean(x^2) + eps) * (norm_weight + 1) */
-  MEGA_TOKEN_LAYERNORM = 3,   /* prologue: (x - mean) / sqrt(var + eps) * (norm_weight + 1) + norm_bias */
-  MEGA_TOKEN_RESIDUAL = 4,    /* epilogue: scale * value + residual */
-  MEGA_TOKEN_GATE = 5         /* epilogue: residual + sigmoid(gate_u) (silu(gate_hx + value) - residual) */
-};
-
 /* out[b, n] = epilogue(sum_k weight[n, k] prologue(x[b])[k] + bias[n]), b < B <= 64 */
 typedef struct {
   const void* weight;         /* [N, K] */

@@ -1,0 +1,107 @@
+"""RMSNorm / LayerNorm rows and the column sums of the training composites against fp64: widths of one to the most
+vectors per lane and with idle lanes, tokens around the waves of a launch, with and without parameters, joined gradient;
+and the composites (feed-forward block, SwiGLU block, the gated attention between norm and output) against the same
+layers with one parameter frozen, which runs them operator by operator."""
+import numpy as np
+import pytest
+import torch
+import torch.nn.functional as F
+
+import fairseq_apollo_amd as M
+from gpu_util import DEV
+
+pytestmark = pytest.mark.gpu
+# one rounding of the result (2^-9 bf16, 2^-11 fp16) on values up to a few times the rms; fp32: sums of up to 8200 terms
+# in fp32, sqrt(8200) 2^-24 of the sum of magnitudes at worst
+ULP = {torch.bfloat16: 2 ** -8, torch.float16: 2 ** -10, torch.float32: 4e-6}
+
+
+def _close(got, ref, dtype, scale=None):
+    ref = ref.double().cpu()
+    scale = ref.abs() + ref.pow(2).mean().sqrt() if scale is None else scale.double().cpu()
+    assert got.dtype == dtype and got.shape == ref.shape
+    assert bool(((got.double().cpu() - ref).abs() <= ULP[dtype] * scale + 1e-12).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,D,affine", [(1, 8, True), (5, 520, True), (2100, 1024, True), (67, 2048, True), (8200, 256, False)])
+@pytest.mark.parametrize("kind", [M.ops.TOKEN_RMSNORM, M.ops.TOKEN_LAYERNORM])
+def test_row_norm_both_ways(dtype, T, D, affine, kind):
+    torch.manual_seed(T + D)
+    x, dy, add = (torch.randn(T, D, device=DEV).to(dtype) + (0.5 if i == 0 else 0) for i in range(3))
+    w = (torch.randn(D, device=DEV) * 0.3).to(dtype) if affine else None
+    b = torch.randn(D, device=DEV).to(dtype) if affine and kind == M.ops.TOKEN_LAYERNORM else None
+    leaves = [t.double().cpu().requires_grad_(True) if t is not None else None for t in (x, w, b)]
+    x64, w64, b64 = leaves
+    c64 = x64 - x64.mean(-1, keepdim=True) if kind == M.ops.TOKEN_LAYERNORM else x64
+    y64 = c64 * torch.rsqrt(c64.pow(2).mean(-1, keepdim=True) + 1e-5)
+    y64 = y64 if w64 is None else y64 * (w64 + 1)
+    y64 = y64 if b64 is None else y64 + b64
+    y64.backward(dy.double().cpu())
+    args = [t.clone().requires_grad_(True) if t is not None else None for t in (x, w, b)]
+    assert M.modules.row_norm_covers(*args)
+    y = M.modules.row_norm(args[0], kind, args[1], args[2], 1e-5)
+    _close(y, y64.detach(), dtype)
+    y.backward(dy)
+    _close(args[0].grad, x64.grad, dtype)
+    with torch.no_grad():
+        hat = ((c64 * torch.rsqrt(c64.pow(2).mean(-1, keepdim=True) + 1e-5)).detach().abs() * dy.double().cpu().abs()).sum(0)
+    if w is not None:
+        _close(args[1].grad, w64.grad, dtype, hat + w64.grad.abs())
+    if b is not None:
+        _close(args[2].grad, b64.grad, dtype, dy.double().cpu().abs().sum(0))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("D,ffn,T,norm", [(64, 96, 33, 'layernorm'), (256, 520, 700, 'rmsnorm')])
+def test_feed_forward_composite(dtype, D, ffn, T, norm):
+    """Against fp64 of the same formula."""
+    torch.manual_seed(D)
+    block = M.NormalizedFeedForwardNetwork(D, ffn, norm_type=norm).to(DEV).to(dtype).train()
+    with torch.no_grad():
+        for p in block.parameters():
+            p.normal_(0, 0.1)
+    x = torch.randn(2, T, D, device=DEV).to(dtype).requires_grad_(True)
+    dy = torch.randn(2, T, D, device=DEV).to(dtype)
+    assert block._one_operator(x)
+    y = block(x)
+    y.backward(dy)
+    P = {k: v.detach().double().cpu().requires_grad_(True) for k, v in block.named_parameters()}
+    x64 = x.detach().double().cpu().requires_grad_(True)
+    n = M.modules.row_norm_formula(x64, M.ops.TOKEN_LAYERNORM, P['norm.weight'], P['norm.bias'], 1e-5) if norm == 'layernorm' \
+        else x64 * torch.rsqrt(x64.pow(2).mean(-1, keepdim=True) + 1e-5) * (P['norm.weight'] + 1)
+    y64 = x64 + F.silu(n @ P['fc1.weight'].t() + P['fc1.bias']) @ P['fc2.weight'].t()
+    y64.backward(dy.double().cpu())
+    # four roundings in a row on the way to any result: 4 ulp of the rms and of the value
+    for got, ref in [(y, y64), (x.grad, x64.grad)] + [(p.grad, P[k].grad) for k, p in block.named_parameters()]:
+        _close(got.detach(), ref.detach(), dtype, 4 * (ref.detach().abs() + ref.detach().pow(2).mean().sqrt()))
+
+
+@pytest.mark.parametrize("dtype,D,S,E,heads,L,chunk,act,two", [
+    (torch.bfloat16, 64, 32, 128, 1, 96, 32, 'rmsnorm', False), (torch.float16, 128, 64, 64, 2, 130, -1, 'silu', False),
+    (torch.float32, 64, 16, 96, 1, 70, -1, 'rmsnorm', True)])
+def test_mix_composite_matches_the_operators(dtype, D, S, E, heads, L, chunk, act, two):
+    """The composite against the operators one by one (taken when a parameter is frozen): the same values in other
+    kernels, roundings apart."""
+    torch.manual_seed(S)
+    layer = M.MovingAverageGatedAttention(D, S, E, 8, chunk_size=chunk, moving_act=act, norm_num_groups=4, num_heads=heads,
+                                          bidirectional=two).to(DEV).to(dtype).train()
+    with torch.no_grad():
+        for p in layer.parameters():
+            if not bool(p.any()):
+                p.normal_(0, 0.2)
+    x0, dy = (torch.randn(2, L, D, device=DEV).to(dtype) for _ in range(2))
+    mask = torch.arange(L, device=DEV)[None, :] >= torch.tensor([[L], [L - 9]], device=DEV) if two else None
+    out = []
+    for freeze in (False, True):
+        layer.h_proj.weight.requires_grad_(not freeze)
+        layer.zero_grad()
+        x = x0.clone().requires_grad_(True)
+        y, _ = layer(x, mask)
+        assert ("MixOut" in type(y.grad_fn).__name__) == (not freeze)
+        y.backward(dy if mask is None else dy * (~mask)[..., None])
+        out.append([y.detach(), x.grad] + [p.grad for n, p in layer.named_parameters() if n != 'h_proj.weight'])
+    for a, b in zip(*out):
+        # the same formulas in both: a handful of roundings of intermediate results apart, 8 ulp of the rms and of the value
+        b64 = b.double().cpu()
+        _close(a, b64, dtype, 8 * (b64.abs() + b64.pow(2).mean().sqrt()))
