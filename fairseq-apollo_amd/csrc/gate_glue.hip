@@ -8,6 +8,8 @@
 //   gate_qk    q, k = rotary(normalize(z) * gamma[i] + beta[i])             (one wave per token)
 //   gate_mul   y = a * silu(r)
 //   gate_out   y = residual + sigmoid(u) * (silu(hx + hp) - residual)
+#include <type_traits>
+
 #include "common.h"
 
 namespace mega {
@@ -113,7 +115,137 @@ __global__ __launch_bounds__(kRowThreads) void gate_qk_kernel(const T* __restric
   }
 }
 
-// Backward of the q / k map.  One wave per token, a wave walks tokens t, t + waves, ...; lane l owns
+// The walk of the two kernels below: the tokens ordered by position first and chunk second, cut into runs of `per`, one
+// run per wave.  The tokens of all chunks at one position turn by the same angles, so the sines and cosines (four
+// sincosf per lane and token, most of the instructions of the map) are formed once per position of a run.  `nc` counts a
+// partial last chunk; its missing positions are skipped (none in a call shorter than a chunk).
+struct QkWalk {
+  int64_t i, end, chunk;
+  int nc, c;
+  int64_t pos;
+  __device__ __forceinline__ QkWalk(int64_t wave, int per, int64_t T_, int64_t chunk_)
+      : chunk(chunk_ < T_ ? chunk_ : T_) {
+    nc = (int)((T_ + chunk - 1) / chunk);
+    const int64_t all = chunk * nc;
+    i = wave * per;
+    end = i + per < all ? i + per : all;
+    pos = i / nc;
+    c = (int)(i - pos * nc);
+  }
+  __device__ __forceinline__ bool more() const { return i < end; }
+  __device__ __forceinline__ int64_t token() const { return c * chunk + pos; }
+  __device__ __forceinline__ void next() {
+    ++i;
+    if (++c == nc) {
+      c = 0;
+      ++pos;
+    }
+  }
+};
+
+// the stored parameter row (raw: activation type, `plus` added; otherwise fp32 multipliers) of VEC features from j
+template <typename T, int VEC>
+__device__ __forceinline__ void qk_params(const void* base, int raw, int j, float plus, float (&f)[VEC]) {
+  if (raw) {
+    const Vec<T, VEC> v = *(const Vec<T, VEC>*)((const T*)base + j);
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) f[i] = to_float(v.v[i]) + plus;
+  } else {
+    const Vec<float, VEC> v = *(const Vec<float, VEC>*)((const float*)base + j);
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) f[i] = v.v[i];
+  }
+}
+
+// gate_qk on rows of at most NV vectors per lane: a lane owns the same features at every token of its run, so the affine
+// parameters and the frequencies are loaded once (whole vectors; gate_qk_kernel loads 32 single values per vector and
+// token, 2 KB apart per wave), and the next token's row is on its way while this one is worked on.  Bound by the sines
+// and the row traffic.  8192 tokens of 512 features in 4 chunks, bf16: 11.7 us (25 MB, 2.1 TB/s;
+// token by token 39.8); 8192 of 256 in 8 chunks: 8.8 us (17.7).
+template <typename T, int VEC, int NV>
+__global__ __launch_bounds__(kRowThreads) void gate_qk_run_kernel(const T* __restrict__ z, int64_t zs,
+                                                                  const void* __restrict__ gamma,
+                                                                  const void* __restrict__ beta, int raw,
+                                                                  const float* __restrict__ freqs, T* __restrict__ q,
+                                                                  T* __restrict__ k, int64_t T_, int S, int Hd,
+                                                                  int64_t chunk, int64_t pos0, float eps, int per) {
+  using V = Vec<T, VEC>;
+  static_assert(VEC % 2 == 0, "pairs of features stay inside one vector");
+  const int lane = threadIdx.x & 63;
+  QkWalk walk((int64_t)blockIdx.x * kRowsPerWg + (threadIdx.x >> 6), per, T_, chunk);
+  if (!walk.more()) return;
+  float gq[NV][VEC], gk[NV][VEC], bq[NV][VEC], bk[NV][VEC], fr[NV][VEC / 2], sn[NV][VEC / 2], cs[NV][VEC / 2];
+  V nz[NV];
+  auto fetch = [&](int64_t t) {
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+      const int j = (u * 64 + lane) * VEC;
+      if (j < S && t < T_) nz[u] = *(const V*)(z + t * zs + j);
+    }
+  };
+  fetch(walk.token());
+#pragma unroll
+  for (int u = 0; u < NV; ++u) {
+    const int j = (u * 64 + lane) * VEC;
+    if (j < S) {
+      qk_params<T, VEC>(gamma, raw, j, 1.0f, gq[u]);
+      qk_params<T, VEC>(gamma, raw, S + j, 1.0f, gk[u]);
+      qk_params<T, VEC>(beta, raw, j, 0.0f, bq[u]);
+      qk_params<T, VEC>(beta, raw, S + j, 0.0f, bk[u]);
+#pragma unroll
+      for (int i = 0; i < VEC / 2; ++i) fr[u][i] = freqs[((j + 2 * i) % Hd) >> 1];
+    }
+  }
+  int64_t at = -1;                                     // position the sines are those of
+  while (walk.more()) {
+    const int64_t t = walk.token(), pos = walk.pos;
+    float f[NV][VEC];
+    float ss = 0.f;
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+      const bool in = (u * 64 + lane) * VEC < S && t < T_;
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) {
+        f[u][i] = in ? to_float(nz[u].v[i]) : 0.f;
+        ss = fmaf(f[u][i], f[u][i], ss);
+      }
+    }
+    walk.next();
+    if (walk.more()) fetch(walk.token());
+    if (t >= T_) continue;                             // (uniform in the wave)
+    if (pos != at) {
+      at = pos;
+#pragma unroll
+      for (int u = 0; u < NV; ++u)
+        if ((u * 64 + lane) * VEC < S)
+#pragma unroll
+          for (int i = 0; i < VEC / 2; ++i) sincosf((float)(pos0 + pos) * fr[u][i], &sn[u][i], &cs[u][i]);
+    }
+    const float inv = 1.0f / fmaxf(sqrtf(wave_sum(ss)), eps);   // F.normalize: x / max(|x|, eps)
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+      const int j = (u * 64 + lane) * VEC;
+      if (j < S) {
+        V oq, ok;
+#pragma unroll
+        for (int i = 0; i < VEC; i += 2) {
+          const float s = sn[u][i >> 1], c = cs[u][i >> 1];
+          const float z0 = f[u][i] * inv, z1 = f[u][i + 1] * inv;
+          const float q0 = fmaf(z0, gq[u][i], bq[u][i]), q1 = fmaf(z1, gq[u][i + 1], bq[u][i + 1]);
+          const float k0 = fmaf(z0, gk[u][i], bk[u][i]), k1 = fmaf(z1, gk[u][i + 1], bk[u][i + 1]);
+          oq.v[i] = from_float<T>(q0 * c - q1 * s);
+          oq.v[i + 1] = from_float<T>(q0 * s + q1 * c);
+          ok.v[i] = from_float<T>(k0 * c - k1 * s);
+          ok.v[i + 1] = from_float<T>(k0 * s + k1 * c);
+        }
+        *(V*)(q + t * (int64_t)S + j) = oq;
+        *(V*)(k + t * (int64_t)S + j) = ok;
+      }
+    }
+  }
+}
+
+// Backward of the q / k map.  A wave walks its run of tokens (QkWalk), the next token's rows on their way; lane l owns
 // the same NV vectors of features at every token, so the four parameter sums (d gamma, d beta of the
 // q and of the k map) stay in registers until the end:
 //   dq_pre = rot^T(dq), dk_pre = rot^T(dk)                         (rotation by -pos * freq)
@@ -122,64 +254,93 @@ __global__ __launch_bounds__(kRowThreads) void gate_qk_kernel(const T* __restric
 //   dz  = (dzn - zn (zn . dzn)) / |z|      (|z| > eps)      or      dzn / eps      (|z| <= eps)
 // The workgroup's four waves then add their sums in LDS, one after the other, and leave one row
 // per workgroup in `part` [workgroups][4][S]; gate_qk_param_kernel adds the rows in order.
+// 8192 tokens of 256 features in 8 chunks, bf16: 15.8 us (17.8 token by token).
 template <typename T, int VEC, int NV>
 __global__ __launch_bounds__(kRowThreads) void gate_qk_bwd_kernel(
     const T* __restrict__ dq, const T* __restrict__ dk, const T* __restrict__ z, int64_t zs,
     const void* __restrict__ gamma_, int raw, const float* __restrict__ freqs, T* __restrict__ dz, int64_t dzs,
-    float* __restrict__ part, int64_t T_, int S, int Hd, int64_t chunk, int64_t pos0, float eps) {
+    float* __restrict__ part, int64_t T_, int S, int Hd, int64_t chunk, int64_t pos0, float eps, int per, int wide) {
   using V = Vec<T, VEC>;
   static_assert(VEC % 2 == 0, "pairs of features stay inside one vector");
   extern __shared__ float s_acc[];                     // [4][S]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   auto gamma = [&](int i) { return raw ? to_float(((const T*)gamma_)[i]) + 1.0f : ((const float*)gamma_)[i]; };
   float agq[NV][VEC], abq[NV][VEC], agk[NV][VEC], abk[NV][VEC];
-  float gq[NV][VEC], gk[NV][VEC], fr[NV][VEC / 2];
+  float gq[NV][VEC], gk[NV][VEC], fr[NV][VEC / 2], sn[NV][VEC / 2], cs[NV][VEC / 2];
+  QkWalk walk((int64_t)blockIdx.x * kRowsPerWg + wave, per, T_, chunk);
+  V nz[NV], na[NV], nb[NV];
+  auto fetch = [&](int64_t t) {
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+      const int j = (u * 64 + lane) * VEC;
+      if (j < S && t < T_) {
+        nz[u] = *(const V*)(z + t * zs + j);
+        na[u] = *(const V*)(dq + t * (int64_t)S + j);
+        nb[u] = *(const V*)(dk + t * (int64_t)S + j);
+      }
+    }
+  };
+  if (walk.more()) fetch(walk.token());
 #pragma unroll
   for (int u = 0; u < NV; ++u) {
     const int j = (u * 64 + lane) * VEC;
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
       agq[u][i] = abq[u][i] = agk[u][i] = abk[u][i] = 0.f;
-      gq[u][i] = j + i < S ? gamma(j + i) : 0.f;
-      gk[u][i] = j + i < S ? gamma(S + j + i) : 0.f;
+      gq[u][i] = gk[u][i] = 0.f;
     }
-#pragma unroll
-    for (int i = 0; i < VEC / 2; ++i) fr[u][i] = j + 2 * i < S ? freqs[((j + 2 * i) % Hd) >> 1] : 0.f;
-  }
-  const int64_t stride = (int64_t)gridDim.x * kRowsPerWg;
-  for (int64_t t = (int64_t)blockIdx.x * kRowsPerWg + wave; t < T_; t += stride) {
-    const T* row = z + t * zs;
-    float zf[NV][VEC], aq[NV][VEC], ak[NV][VEC];
-    float ss = 0.f;
-    const float pos = (float)(pos0 + t % chunk);
-#pragma unroll
-    for (int u = 0; u < NV; ++u) {
-      const int j = (u * 64 + lane) * VEC;
-      if (j < S) {
-        const V v = *(const V*)(row + j);
-        const V a = *(const V*)(dq + t * (int64_t)S + j);
-        const V b = *(const V*)(dk + t * (int64_t)S + j);
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) {
-          zf[u][i] = to_float(v.v[i]);
-          ss = fmaf(zf[u][i], zf[u][i], ss);
-        }
-#pragma unroll
-        for (int i = 0; i < VEC; i += 2) {
-          float sn, cs;
-          sincosf(pos * fr[u][i >> 1], &sn, &cs);
-          const float a0 = to_float(a.v[i]), a1 = to_float(a.v[i + 1]);
-          const float b0 = to_float(b.v[i]), b1 = to_float(b.v[i + 1]);
-          aq[u][i] = a0 * cs + a1 * sn;
-          aq[u][i + 1] = a1 * cs - a0 * sn;
-          ak[u][i] = b0 * cs + b1 * sn;
-          ak[u][i + 1] = b1 * cs - b0 * sn;
-        }
+    if (j < S) {
+      if (wide) {
+        qk_params<T, VEC>(gamma_, raw, j, 1.0f, gq[u]);
+        qk_params<T, VEC>(gamma_, raw, S + j, 1.0f, gk[u]);
       } else {
 #pragma unroll
-        for (int i = 0; i < VEC; ++i) zf[u][i] = aq[u][i] = ak[u][i] = 0.f;
+        for (int i = 0; i < VEC; ++i) {
+          gq[u][i] = gamma(j + i);
+          gk[u][i] = gamma(S + j + i);
+        }
       }
     }
+#pragma unroll
+    for (int i = 0; i < VEC / 2; ++i) {
+      fr[u][i] = j + 2 * i < S ? freqs[((j + 2 * i) % Hd) >> 1] : 0.f;
+      sn[u][i] = cs[u][i] = 0.f;
+    }
+  }
+  int64_t at = -1;                                     // position the sines are those of
+  while (walk.more()) {
+    const int64_t t = walk.token(), pos = walk.pos;
+    float zf[NV][VEC], aq[NV][VEC], ak[NV][VEC];
+    float ss = 0.f;
+    if (pos != at) {
+      at = pos;
+#pragma unroll
+      for (int u = 0; u < NV; ++u)
+#pragma unroll
+        for (int i = 0; i < VEC / 2; ++i) sincosf((float)(pos0 + pos) * fr[u][i], &sn[u][i], &cs[u][i]);
+    }
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+      const bool in = (u * 64 + lane) * VEC < S && t < T_;
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) {
+        zf[u][i] = in ? to_float(nz[u].v[i]) : 0.f;
+        ss = fmaf(zf[u][i], zf[u][i], ss);
+      }
+#pragma unroll
+      for (int i = 0; i < VEC; i += 2) {
+        const float s = sn[u][i >> 1], c = cs[u][i >> 1];
+        const float a0 = in ? to_float(na[u].v[i]) : 0.f, a1 = in ? to_float(na[u].v[i + 1]) : 0.f;
+        const float b0 = in ? to_float(nb[u].v[i]) : 0.f, b1 = in ? to_float(nb[u].v[i + 1]) : 0.f;
+        aq[u][i] = a0 * c + a1 * s;
+        aq[u][i + 1] = a1 * c - a0 * s;
+        ak[u][i] = b0 * c + b1 * s;
+        ak[u][i + 1] = b1 * c - b0 * s;
+      }
+    }
+    walk.next();
+    if (walk.more()) fetch(walk.token());
+    if (t >= T_) continue;                             // (uniform in the wave)
     const float nrm = sqrtf(wave_sum(ss));
     const bool clamped = !(nrm > eps);
     const float inv = 1.0f / fmaxf(nrm, eps);
@@ -440,11 +601,43 @@ int launch_rms_norm(const void* x, int64_t xs, const float* w, void* y, int64_t 
   return MEGA_OK;
 }
 
+constexpr int64_t kQkFwdWaves = 4096;            // 16 per CU
+
+// positions of a walk over T_ tokens (QkWalk), and how many of them a wave takes when about `waves` share them
+inline int64_t qk_walk_length(int64_t T_, int64_t chunk) { return chunk < T_ ? ceil_div(T_, chunk) * chunk : T_; }
+inline int qk_run(int64_t all, int64_t waves) {
+  const int64_t per = ceil_div(all, waves);
+  return (int)(per < 1 ? 1 : per);
+}
+
 template <typename T>
 int launch_gate_qk(const void* z, int64_t zs, const void* gamma, const void* beta, int raw, const float* freqs, void* q,
                    void* k, int64_t T_, int64_t S, int64_t Hd, int64_t chunk, int64_t pos0, float eps,
                    hipStream_t s) {
   constexpr int VEC = 16 / (int)sizeof(T);
+  // Rows of up to two vectors per lane with parameters on whole vectors: runs of tokens.  Half vectors where they still
+  // cover the row with one per lane (more lanes at work on the sines).  16 waves per CU are the launch's target: longer
+  // runs share more sines, but leave CUs short of rows in flight.
+  const auto runs = [&](auto vec, auto nv) -> bool {
+    constexpr int VC = decltype(vec)::value, NV = decltype(nv)::value;
+    const size_t ps = raw ? sizeof(T) : 4;
+    if (S % VC || S > 64 * VC * NV || !vec_ok(z, zs, sizeof(T), VC) || !vec_ok(q, S, sizeof(T), VC) ||
+        !vec_ok(k, S, sizeof(T), VC) || !vec_ok(gamma, S, ps, VC) || !vec_ok(beta, S, ps, VC))
+      return false;
+    const int64_t all = qk_walk_length(T_, chunk);
+    const int per = qk_run(all, kQkFwdWaves);
+    hipLaunchKernelGGL((gate_qk_run_kernel<T, VC, NV>), dim3((unsigned)ceil_div(ceil_div(all, per), kRowsPerWg)),
+                       dim3(kRowThreads), 0, s, (const T*)z, zs, gamma, beta, raw, freqs, (T*)q, (T*)k, T_, (int)S, (int)Hd,
+                       chunk, pos0, eps, per);
+    return true;
+  };
+  using std::integral_constant;
+  if (runs(integral_constant<int, VEC / 2>(), integral_constant<int, 1>()) ||
+      runs(integral_constant<int, VEC>(), integral_constant<int, 1>()) ||
+      runs(integral_constant<int, VEC>(), integral_constant<int, 2>())) {
+    MEGA_CHECK_LAUNCH("gate_qk_fwd");
+    return MEGA_OK;
+  }
   const unsigned grid = (unsigned)ceil_div(T_, kRowsPerWg);
   if (S % VEC == 0 && vec_ok(z, zs, sizeof(T), VEC) && vec_ok(q, S, sizeof(T), VEC) && vec_ok(k, S, sizeof(T), VEC))
     hipLaunchKernelGGL((gate_qk_kernel<T, VEC>), dim3(grid), dim3(kRowThreads), 0, s, (const T*)z, zs, gamma, beta, raw,
@@ -489,12 +682,18 @@ int launch_gate_qk_bwd(const void* dq, const void* dk, const void* z, int64_t zs
     audit_use(dbeta, (size_t)2 * S * (raw ? sizeof(T) : 4), "gate_qk_bwd: beta_grad");
     return MEGA_OK;
   }
-  if (S <= 64 * VEC)
-    hipLaunchKernelGGL((gate_qk_bwd_kernel<T, VEC, 1>), dim3(grid), dim3(kRowThreads), lds, s, (const T*)dq,
-                       (const T*)dk, (const T*)z, zs, gamma, raw, freqs, (T*)dz, dzs, part, T_, (int)S, (int)Hd, chunk, pos0, eps);
-  else
-    hipLaunchKernelGGL((gate_qk_bwd_kernel<T, VEC, 2>), dim3(grid), dim3(kRowThreads), lds, s, (const T*)dq,
-                       (const T*)dk, (const T*)z, zs, gamma, raw, freqs, (T*)dz, dzs, part, T_, (int)S, (int)Hd, chunk, pos0, eps);
+  const int per = qk_run(qk_walk_length(T_, chunk), (int64_t)grid * kRowsPerWg);
+  const auto run = [&](auto vec, auto nv) {
+    constexpr int VC = decltype(vec)::value, NV = decltype(nv)::value;
+    const int wide = vec_ok(gamma, S, raw ? sizeof(T) : 4, VC) ? 1 : 0;
+    hipLaunchKernelGGL((gate_qk_bwd_kernel<T, VC, NV>), dim3(grid), dim3(kRowThreads), lds, s, (const T*)dq, (const T*)dk,
+                       (const T*)z, zs, gamma, raw, freqs, (T*)dz, dzs, part, T_, (int)S, (int)Hd, chunk, pos0, eps, per,
+                       wide);
+  };
+  using std::integral_constant;
+  if (S <= 64 * VEC / 2) run(integral_constant<int, VEC / 2>(), integral_constant<int, 1>());
+  else if (S <= 64 * VEC) run(integral_constant<int, VEC>(), integral_constant<int, 1>());
+  else run(integral_constant<int, VEC>(), integral_constant<int, 2>());
   MEGA_CHECK_LAUNCH("gate_qk_bwd");
   const dim3 pgrid((unsigned)ceil_div(4 * S, 64));
   if (raw)

@@ -609,6 +609,14 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
         simple = isinstance(self.rel_pos_bias, SimpleRelativePositionalBias)
         bsz, seq_len = z.shape[:2]
         Nh = self.num_heads
+        if (self.chunk_size > 1 and seq_len % self.chunk_size == 0 and "prev_key" not in saved_state and not simple
+                and not self.bidirectional and self.attention_activation == 'softmax'):
+            # whole chunks behind whole chunks: nothing cached, nothing to cache
+            self._set_input_buffer(incremental_state, saved_state)
+            q, k = ops.gate_qk_fwd(z, *self._qk_constants(False), Nh, self.chunk_size)
+            shape = (bsz * (seq_len // self.chunk_size), self.chunk_size, Nh)
+            return self.efficient_attn(q.view(*shape, self.zdim // Nh), k.view(*shape, self.zdim // Nh),
+                                       v.reshape(*shape, self.hdim // Nh))
         z = F.normalize(z, p=2, dim=-1, eps=1e-5)
         z = z.unsqueeze(2) * (self.gamma + 1.0) + self.beta
         q, k = torch.unbind(z, dim=2)
