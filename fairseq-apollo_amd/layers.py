@@ -24,7 +24,7 @@ from torch.nn import Parameter
 from . import ops
 from .modules import (AttentionSoftmax, EfficientAttention, FeedForwardFunc, GateMulFunc, GateOutFunc, GateQKFunc,
                       IncrementalState, MixInFunc, MixOutFunc, MultiHeadComplexEMA, MultiHeadEMA, SequenceNorm, SplitFunc,
-                      SplitGrads, SwiGLU, TimestepNorm, _plain, _tensor_versions, _training_call, linear, linear_residual,
+                      SplitGrads, SwiGLU, TimestepNorm, _plain, _tensor_versions, _training_call, _unhooked, linear, linear_residual,
                       mask_bytes, mask_bytes_ok, norm_then_move, one_graph, row_norm, row_norm_covers, row_norm_formula,
                       silu)
 
@@ -125,8 +125,7 @@ class NormalizedFeedForwardNetwork(nn.Module):
         # (normalized_feedforward_network.py:81-83)
         if _training_call(self, x) or (self.training and self.hidden_dropout_p > 0):
             h = F.dropout(silu(linear(self.fc1, self.norm(x))), self.hidden_dropout_p, self.training)
-        elif ops.token_rows(x, normalised=True) and self.hidden_dim % 32 == 0 and self.fc1.weight.dtype == x.dtype and \
-                not (self.training and self.dropout_p > 0):
+        elif ops.token_rows(x, normalised=True) and self._few_rows_cover(x):
             return self._few_rows(x)
         else:
             h = ops.silu(self.fc1(self.norm(x)), inplace=True)
@@ -143,9 +142,15 @@ class NormalizedFeedForwardNetwork(nn.Module):
         vec = 16 // x.element_size()
         return (one_graph(x, norm.weight, getattr(norm, 'bias', None), self.fc1.weight, self.fc1.bias, self.fc2.weight)
                 and self.layerscale_weight is None and x.shape[-1] % vec == 0 and x.shape[-1] <= 2048
-                and self.hidden_dim % vec == 0 and _plain(self.fc1, self.fc2) and type(norm) in (RMSNorm, LayerNorm)
-                and not norm._forward_hooks and not norm._forward_pre_hooks
+                and self.hidden_dim % vec == 0 and _plain(self.fc1, self.fc2) and _unhooked((RMSNorm, LayerNorm), norm)
                 and not (self.training and (self.dropout_p > 0 or self.hidden_dropout_p > 0)))
+
+    def _few_rows_cover(self, x: Tensor) -> bool:
+        norm = self.norm
+        return (self.hidden_dim % 32 == 0 and not (self.training and self.dropout_p > 0) and _plain(self.fc1, self.fc2)
+                and _unhooked((RMSNorm, LayerNorm), norm)
+                and ops._lib.load_host().uniform(x, norm.weight, getattr(norm, 'bias', None), self.fc1.weight, self.fc1.bias,
+                                                 self.fc2.weight, self.layerscale_weight))
 
     def _few_rows(self, x: Tensor) -> Tensor:
         """The block on one token per stream: two launches (norm, first projection and activation; second projection,
@@ -368,7 +373,13 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
         language model (softmax, rotary, complex moving average without truncation, group norm)."""
         move, key = self.move, saved_state.get("prev_key")
         z, h, Nh = self.zdim, self.hdim, self.num_heads
-        return (ops.token_rows(x, normalised=True) and mask_bytes_ok(padding_mask) and self.v_proj.weight.dtype == x.dtype
+        mine, mods = self._parameters, self._modules
+        v_proj, mx_proj, h_proj, act = (mods[k] for k in ('v_proj', 'mx_proj', 'h_proj', 'move_act'))
+        return (ops.token_rows(x, normalised=True) and mask_bytes_ok(padding_mask) and _plain(v_proj, mx_proj, h_proj)
+                and _unhooked((RMSNorm, nn.SiLU), act)
+                and ops._lib.load_host().uniform(
+                    x, *v_proj._parameters.values(), *mx_proj._parameters.values(), *h_proj._parameters.values(),
+                    mine['gamma'], mine['beta'], act._parameters.get('weight'))
                 and self.attention_activation == 'softmax' and isinstance(self.rel_pos_bias, RotaryEmbedding)
                 and self.norm.num_groups is not None and isinstance(move, MultiHeadComplexEMA)
                 and (move.truncation is None or move.truncation < 1) and self.ndim in (4, 8, 16, 32)
@@ -557,8 +568,7 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
                           self.gamma, self.beta, act.weight if rms else None)
                 and mx.dtype == xn.dtype and residual.dtype == xn.dtype and residual.data_ptr() % 16 == 0
                 and self.embed_dim % vec == 0 and self.zdim % vec == 0 and self.hdim % vec == 0 and self.zdim <= 128 * vec
-                and (not rms or self.embed_dim <= 2048) and type(act) in (RMSNorm, nn.SiLU)
-                and not act._forward_hooks and not act._forward_pre_hooks
+                and (not rms or self.embed_dim <= 2048) and _unhooked((RMSNorm, nn.SiLU), act)
                 and _plain(self.v_proj, self.mx_proj, self.h_proj)
                 and not (self.training and (self.dropout_p > 0 or self.hidden_dropout_p > 0)))
 

@@ -16,7 +16,7 @@ from torch import Tensor, nn
 
 from . import ops
 from .layers import MegaDecoderLayer, _arg
-from .modules import TimestepNorm
+from .modules import TimestepNorm, _plain, _unhooked
 
 
 class MegaDecoderNoCrossAttn(nn.Module):
@@ -73,10 +73,12 @@ class MegaDecoderNoCrossAttn(nn.Module):
 
     def output_layer(self, features: Tensor) -> Tensor:
         """Project features to the vocabulary (mega_lm.py:379-385)."""
-        w = self.output_projection.weight
-        if not torch.is_grad_enabled() and ops.token_rows(features) and w.dtype == features.dtype:
+        proj = self.output_projection
+        w = proj.weight
+        if not torch.is_grad_enabled() and ops.token_rows(features) and _plain(proj) and proj.bias is None and \
+                ops._lib.load_host().uniform(features, w):
             return ops.token_linear(features, w)
-        return self.output_projection(features)
+        return proj(features)
 
     def max_positions(self) -> int:
         """Longest sequence the decoder is configured for (mega_lm.py:387-389)."""
@@ -112,8 +114,9 @@ class MegaDecoderNoCrossAttn(nn.Module):
         return x, {"inner_states": inner_states}
 
     def _token_covers(self, tokens: Tensor) -> bool:
-        w = self.embed_tokens.weight
-        return (not torch.is_grad_enabled() and w.is_cuda and w.dtype in (torch.bfloat16, torch.float16)
+        embed = self.embed_tokens
+        w = embed.weight
+        return (_unhooked((nn.Embedding,), embed) and embed.max_norm is None and not torch.is_grad_enabled() and w.is_cuda and w.dtype in (torch.bfloat16, torch.float16)
                 and w.is_contiguous() and w.shape[1] % 8 == 0 and tokens.dtype is torch.int64 and tokens.is_contiguous()
                 and tokens.device == w.device and not (self.training and self.embedding_dropout.p > 0))
 

@@ -1008,11 +1008,18 @@ def linear(lin: nn.Linear, x: Tensor) -> Tensor:
     return lin(x)
 
 
+def _unhooked(kinds: tuple, *mods) -> bool:
+    """Modules of exactly these types, nobody looking at their inputs or outputs: what reads their parameters directly may
+    stand in for the calls."""
+    for m in mods:
+        if type(m) not in kinds or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks:
+            return False
+    return True
+
+
 def _plain(*layers) -> bool:
-    """Linear layers as torch defines them, nobody looking at their inputs or outputs: what reads their weights directly
-    may stand in for the calls."""
-    return all(type(m) is nn.Linear and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
-                                             or m._backward_pre_hooks) for m in layers)
+    """Linear layers as torch defines them, _unhooked."""
+    return _unhooked((nn.Linear,), *layers)
 
 
 def one_graph(x: Tensor, *params) -> bool:

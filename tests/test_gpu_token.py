@@ -97,3 +97,35 @@ def test_state_of_an_earlier_token_survives_the_next():
     for n, e in state.items():
         for k, v in e.items():
             assert torch.equal(v, before[n][k]), k
+
+
+@pytest.mark.parametrize("change", ["hook", "subclass", "columns"])
+def test_token_of_modules_that_are_not_plain(change):
+    """Projections that someone looks at, replaced by a class of their own or stored column by column are called as
+    modules: the values of the operators one by one, in the composite's tolerance."""
+    half, full = _model(64, 16, 64, 1, 64, 64, "layernorm", torch.bfloat16, 5)
+    tokens = torch.randint(2, 72, (3, 20), device=DEV)
+    calls = []
+
+    class Own(torch.nn.Linear):
+        def forward(self, x):
+            calls.append(1)
+            return super().forward(x)
+
+    # (the feed-forward block's second projection adds its residual in its product: its weight is read everywhere)
+    lins = [m for n, m in half.named_modules() if type(m) is torch.nn.Linear and not n.endswith('fc2')]
+    for m in [*lins, half.embed_tokens]:
+        if change == "hook":
+            m.register_forward_hook(lambda *a: calls.append(1))
+        elif change == "columns":
+            m.weight.data = m.weight.data.t().contiguous().t()
+        elif m is not half.embed_tokens:
+            m.__class__ = Own
+    sa, sb = {}, {}
+    with torch.no_grad():
+        half(tokens[:, :19], incremental_state=sa)
+        full(tokens[:, :19], incremental_state=sb)
+        calls.clear()
+        got, want = half(tokens[:, 19:], incremental_state=sa)[0], full(tokens[:, 19:], incremental_state=sb)[0]
+    assert len(calls) == {"hook": len(lins) + 1, "subclass": len(lins), "columns": 0}[change]
+    assert _rms(got, want) < TOL[torch.bfloat16]
