@@ -2,8 +2,11 @@
 // checks and the C ABI call in native code, one Python call per composite step.  Tensors in, tensors out; the launch
 // stream's raw handle comes from the caller (ops._stream).  No device code and no state in here.
 #include <ATen/ATen.h>
+#include <ATen/TensorSubclassLikeUtils.h>
 #include <Python.h>
 #include <c10/core/GradMode.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "../../include/mega_hip.h"
@@ -554,10 +557,24 @@ Tensor silu(const Tensor& x, void* s, const char* who) {
   return y;
 }
 
+// Operations are only being run, not looked at: no tracing, function transform or dispatch mode, which see torch's own
+// operations and nothing that happens in here.
+bool eager() {
+  return !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer) &&
+         !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) &&
+         !c10::impl::dispatch_mode_enabled();
+}
+
+// Values of its own in memory and no forward-mode tangent beside them.
+bool plain(const Tensor& t) { return !at::isTensorSubclassLike(t) && !t._fw_grad(0).defined(); }
+
 // (x, tensor | None, ...) -> bool: x is a GPU activation and every tensor is contiguous, of its type and device, on 16
 // bytes; `graph`: and every one asks for its gradient (the composites' backward passes form all of them)
 PyObject* same_storage(const Args& A, bool graph) {
   const Tensor& x = A.t(0);
+  if (!eager()) return PyBool_FromLong(false);
+  for (int i = 0; i < A.n; ++i)
+    if (!A.none(i) && !plain(A.t(i))) return PyBool_FromLong(false);
   const at::ScalarType dt = x.scalar_type();
   bool ok = x.is_cuda() && (dt == at::kFloat || dt == at::kBFloat16 || dt == at::kHalf) && x.dim() > 1 && x.numel() > 0 && !x.is_neg() &&
             (uintptr_t)x.data_ptr() % 16 == 0;

@@ -1025,13 +1025,15 @@ def _plain(*layers) -> bool:
 def one_graph(x: Tensor, *params) -> bool:
     """True when a composite training operator may run on x and these parameters (None: absent): a graph is being built,
     all of one type, contiguous and aligned, every parameter wants its gradient, no autocast."""
-    return torch.is_grad_enabled() and x.is_cuda and not torch.is_autocast_enabled() and \
-        ops._lib.load_host().trainable(x, *params)
+    return torch.is_grad_enabled() and not torch.compiler.is_compiling() and x.is_cuda and \
+        not torch.is_autocast_enabled() and ops._lib.load_host().trainable(x, *params)
 
 
 def row_norm_covers(x: Tensor, *params) -> bool:
+    """The row kernels take x: 16-bit or single precision, whole 16-byte rows, and an eager call (tracing, function
+    transforms and forward-mode tangents keep torch's own operations)."""
     D = x.shape[-1]
-    return x.is_cuda and D % (16 // x.element_size()) == 0 and D <= 2048 and not torch.is_autocast_enabled() and \
+    return not torch.compiler.is_compiling() and x.is_cuda and D % (16 // x.element_size()) == 0 and D <= 2048 and not torch.is_autocast_enabled() and \
         ops._lib.load_host().uniform(x, *params)
 
 

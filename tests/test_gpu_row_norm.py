@@ -105,3 +105,32 @@ def test_mix_composite_matches_the_operators(dtype, D, S, E, heads, L, chunk, ac
         # the same formulas in both: a handful of roundings of intermediate results apart, 8 ulp of the rms and of the value
         b64 = b.double().cpu()
         _close(a, b64, dtype, 8 * (b64.abs() + b64.pow(2).mean().sqrt()))
+
+
+@pytest.mark.parametrize("norm", [M.layers.RMSNorm, M.layers.LayerNorm])
+def test_norms_under_transforms(norm):
+    """Function transforms, forward-mode tangents and tracing see torch's own operations: the values of the same module
+    on the CPU, fp32 sums of 64 terms in another order apart (sqrt(64) 2^-24 of the sum of magnitudes)."""
+    torch.manual_seed(3)
+    cpu = norm(64)
+    with torch.no_grad():
+        for p in cpu.parameters():
+            p.normal_(0, 0.3)
+    dev = norm(64).to(DEV)
+    dev.load_state_dict(cpu.state_dict())
+    x, t = torch.randn(4, 7, 64), torch.randn(4, 7, 64)
+    xd, td = x.to(DEV), t.to(DEV)
+
+    def near(got, ref):
+        _close(got.detach(), ref.detach(), torch.float32)
+
+    near(torch.func.vmap(dev)(xd), cpu(x))
+    want = torch.func.jvp(cpu, (x,), (t,))
+    for a, b in zip(torch.func.jvp(dev, (xd,), (td,)), want):
+        near(a, b)
+    near(torch.func.grad(lambda v: (dev(v) * td).sum())(xd), torch.func.grad(lambda v: (cpu(v) * t).sum())(x))
+    with torch.autograd.forward_ad.dual_level():
+        dual = dev(torch.autograd.forward_ad.make_dual(xd, td))
+        near(torch.autograd.forward_ad.unpack_dual(dual).tangent, want[1])
+    traced = torch.jit.trace(dev, xd, check_trace=False)
+    near(traced(td), cpu(t))
