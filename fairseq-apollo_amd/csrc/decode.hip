@@ -159,11 +159,12 @@ __global__ __launch_bounds__(kT) void norm_ema_step_kernel(const StepArgs A) {
 // the state as one contiguous 2 KB block; the output sum is finished across the NP lanes.
 // What bounds the step is the state's way through memory, so its loads (and the coefficients') are issued before
 // anything else: the group's moments (every wave for itself, no workgroup barrier, the values kept in registers
-// for the centred second pass) are formed under them.  64 streams x 2048 channels x 16 states: 10.0 us, 3.4 TB/s of
-// state (the same as with the moments in front and two workgroup barriers: enough workgroups share a CU to hide
-// either order); one stream of 1024 channels: 4.2 us.
+// for the centred second pass) are formed under them.  64 streams x 2048 channels x 16 states: 8.7 us a call, 128 streams 13.2 us
+// (13.7 with the moments in front and two workgroup barriers); one stream of 1024 channels: 4.2 us.
 constexpr int kTV = 256;
-constexpr int kStepIT = 2;             // channel parts a thread has in flight: 512 = the 128 channels of a group at N = 16
+// Channel parts a thread has in flight.  Two (the 128 channels of a group at N = 16) need registers that halve the waves
+// per SIMD: 128 streams of 2048 channels 15.4 us against 13.2, of 1536 channels 12.9 against 10.6, none faster at 1 to 64.
+constexpr int kStepIT = 1;
 
 template <typename T, int NP>
 __global__ __launch_bounds__(kTV) void norm_ema_step_vec_kernel(const StepArgs A) {
