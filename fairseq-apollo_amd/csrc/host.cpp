@@ -39,6 +39,19 @@ struct Args {
   const void* opt(int i, at::ScalarType dt, int64_t numel, const at::Device& dev) const {
     return none(i) ? nullptr : p(i, dt, numel, dev);
   }
+  // a weight matrix [rows, cols]
+  const void* mat(int i, at::ScalarType dt, int64_t rows, int64_t cols, const at::Device& dev) const {
+    shape(i, {rows, cols});
+    return p(i, dt, rows * cols, dev);
+  }
+  // the kernels take every size from one operand: the others must have it
+  void shape(int i, at::IntArrayRef sizes) const {
+    if (!none(i) && t(i).sizes() != sizes) {
+      std::string want;
+      for (int64_t s : sizes) want += (want.empty() ? "" : ", ") + std::to_string(s);
+      throw std::runtime_error(std::string(who) + ": argument " + std::to_string(i) + " must be [" + want + "]");
+    }
+  }
   double d(int i) const {
     const double v = PyFloat_AsDouble(a[i]);
     if (v == -1.0 && PyErr_Occurred()) throw std::runtime_error("");
@@ -129,13 +142,13 @@ PyObject* token_gated_attention(const Args& A) {
   a.q = (const float*)A.p(14, at::kFloat, D * N * 2, dev);
   a.ema_gamma = (const float*)A.p(15, at::kFloat, D * N * 2, dev);
   a.omega = (const float*)A.p(16, at::kFloat, D, dev);
-  a.v_weight = A.p(17, T, hidden * D, dev);
+  a.v_weight = A.mat(17, T, hidden, D, dev);
   a.v_bias = A.p(18, T, hidden, dev);
-  a.mx_weight = A.p(19, T, W * D, dev);
+  a.mx_weight = A.mat(19, T, W, D, dev);
   a.mx_bias = A.p(20, T, W, dev);
-  a.h_weight = A.p(21, T, D * hidden, dev);
-  a.gamma = A.p(22, T, 2 * S, dev);
-  a.beta = A.p(23, T, 2 * S, dev);
+  a.h_weight = A.mat(21, T, D, hidden, dev);
+  a.gamma = A.mat(22, T, 2, S, dev);
+  a.beta = A.mat(23, T, 2, S, dev);
   a.move_act = A.i64(24);
   a.move_norm_weight = A.opt(25, T, D, dev);
   a.move_norm_eps = A.d(26);
@@ -187,11 +200,11 @@ PyObject* token_ffn(const Args& A) {
   f1.norm_weight = A.opt(2, T, D, dev);
   f1.norm_bias = A.opt(3, T, D, dev);
   f1.eps = (float)A.d(4);
-  f1.weight = A.p(5, T, H * D, dev);
+  f1.weight = A.mat(5, T, H, D, dev);
   f1.bias = A.p(6, T, H, dev);
   f1.x = x.data_ptr(); f1.x_stride = D; f1.out = hid.data_ptr(); f1.out_stride = H; f1.N = H; f1.K = D;
   f1.epilogue = MEGA_TOKEN_SILU;
-  f2.weight = A.p(7, T, D * H, dev);
+  f2.weight = A.mat(7, T, D, H, dev);
   f2.scale = A.opt(8, T, D, dev);
   f2.x = hid.data_ptr(); f2.x_stride = H; f2.out = out[0].data_ptr(); f2.out_stride = D; f2.N = D; f2.K = H;
   f2.epilogue = MEGA_TOKEN_RESIDUAL; f2.residual = x.data_ptr(); f2.residual_stride = D;
@@ -245,7 +258,7 @@ PyObject* token_linear(const Args& A) {
   const int64_t B = x.size(0), K = x.size(2), N = w.size(0);
   Tensor out = at::empty({B, 1, N}, x.options());
   MegaTokenLinear f = {};
-  f.weight = A.p(1, x.scalar_type(), N * K, x.device());
+  f.weight = A.mat(1, x.scalar_type(), N, K, x.device());
   f.bias = A.opt(2, x.scalar_type(), N, x.device());
   f.x = x.data_ptr(); f.x_stride = K; f.out = out.data_ptr(); f.out_stride = N; f.N = N; f.K = K;
   check(mega_token_linear(&f, dtype_code(x), B, A.stream(3)), A.who);
@@ -516,7 +529,16 @@ void same_type(const Args& A, std::initializer_list<int> at, const Tensor& x) {
       throw std::runtime_error(std::string(A.who) + ": argument " + std::to_string(i) + " must be contiguous, of the activations' type and on their device");
 }
 
+// a row norm's parameters hold one value per column: the kernels read (and in the backward pass write) that many
+void norm_width(const Tensor& x, const Tensor& w, const Tensor& b, const char* who) {
+  for (const Tensor* p : {&w, &b})
+    if (p->defined() && (p->dim() != 1 || p->numel() != x.size(-1)))
+      throw std::runtime_error(std::string(who) + ": norm parameters of " + std::to_string(p->numel()) + " values on rows of " +
+                               std::to_string(x.size(-1)));
+}
+
 Tensor row_norm(const Tensor& x, const Tensor& w, const Tensor& b, int kind, double eps, void* s, const char* who) {
+  norm_width(x, w, b, who);
   Tensor y = at::empty_like(x);
   if (x.numel()) check(mega_row_norm_fwd(x.data_ptr(), x.size(-1), ptr_or_null(w), ptr_or_null(b), y.data_ptr(), dtype_code(x), kind, x.numel() / x.size(-1), x.size(-1), eps, s), who);
   return y;
@@ -525,6 +547,8 @@ Tensor row_norm(const Tensor& x, const Tensor& w, const Tensor& b, int kind, dou
 // (dx, dw, db); dw / db undefined where there is no parameter
 std::tuple<Tensor, Tensor, Tensor> row_norm_back(const Tensor& dy, const Tensor& x, const Tensor& w, const Tensor& b,
                                                  const Tensor& add, int kind, double eps, void* s, const char* who) {
+  norm_width(x, w, b, who);
+  if (dy.sizes() != x.sizes()) throw std::runtime_error(std::string(who) + ": the gradient must have the rows' shape");
   Tensor dx = at::empty_like(x), dw, db;
   if (w.defined()) dw = at::empty_like(w);
   if (b.defined()) db = at::empty_like(b);
@@ -646,6 +670,7 @@ PyObject* swiglu_forward(const Args& A) {
   same_type(A, {0, 1, 2, 3, 4}, n);
   void* s = A.stream(5);
   const Tensor n2 = rows2(n);
+  A.shape(3, A.t(2).sizes());
   Tensor a = at::mm(n2, A.t(2).t()), b = at::mm(n2, A.t(3).t()), g = at::empty_like(a);
   check(mega_swiglu_fwd(a.data_ptr(), b.data_ptr(), g.data_ptr(), dtype_code(n), a.numel(), s), A.who);
   Tensor out = A.none(1) ? at::mm(g, A.t(4).t()) : at::addmm(rows2(A.t(1)), g, A.t(4).t());
@@ -684,6 +709,11 @@ PyObject* mix_forward(const Args& A) {
   const int dt = dtype_code(xn);
   const int64_t D = xn.size(2), S = A.t(6).size(1), E = A.t(2).size(0), heads = A.i64(9), chunk = A.i64(10);
   const int64_t T = xn.numel() / D, W = 2 * D + S + E;
+  A.shape(2, {E, D});
+  A.shape(4, {W, D});
+  A.shape(6, {2, S});
+  A.shape(7, {2, S});
+  A.shape(12, {D});
   const Tensor mx = A.t(1).transpose(1, 2).contiguous();
   if (mx.scalar_type() != xn.scalar_type() || mx.sizes() != xn.sizes()) throw std::runtime_error("mix_forward: mx must be [B, D, L]");
   Tensor vp = at::addmm(A.t(3), rows2(xn), A.t(2).t());
@@ -708,6 +738,9 @@ PyObject* mix_out_forward(const Args& A) {
   void* s = A.stream(5);
   const int dt = dtype_code(x);
   const int64_t D = x.size(2), E = attn.size(-1), S = A.i64(4), W = base.size(1), T = x.numel() / D, es = x.element_size();
+  A.shape(1, {T, 2 * D + S + E});
+  A.shape(3, {D, E});
+  if (attn.numel() != T * E) throw std::runtime_error("mix_out_forward: attention must be [tokens, E]");
   const char* b = (const char*)base.data_ptr();
   Tensor gated = at::empty({T, E}, x.options());
   check(mega_gate_mul_fwd(attn.data_ptr(), E, b + (D + S) * es, W, gated.data_ptr(), dt, T, E, s), A.who);

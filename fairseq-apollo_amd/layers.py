@@ -25,7 +25,7 @@ from . import ops
 from .modules import (AttentionSoftmax, EfficientAttention, FeedForwardFunc, GateMulFunc, GateOutFunc, GateQKFunc,
                       IncrementalState, MixInFunc, MixOutFunc, MultiHeadComplexEMA, MultiHeadEMA, SequenceNorm, SplitFunc,
                       SplitGrads, SwiGLU, TimestepNorm, _plain, _tensor_versions, _training_call, _unhooked, linear, linear_residual,
-                      mask_bytes, mask_bytes_ok, norm_then_move, one_graph, row_norm, row_norm_covers, row_norm_formula,
+                      mask_bytes, mask_bytes_ok, norm_then_move, norm_width_ok, one_graph, row_norm, row_norm_covers, row_norm_formula,
                       silu)
 
 
@@ -68,9 +68,9 @@ class LayerNorm(nn.Module):
             self.register_parameter("bias", None)
 
     def forward(self, x: Tensor) -> Tensor:
-        if row_norm_covers(x, self.weight, self.bias):
+        if self.normalized_shape == (x.shape[-1],) and row_norm_covers(x, self.weight, self.bias):
             return row_norm(x, ops.TOKEN_LAYERNORM, self.weight, self.bias, self.eps)
-        return row_norm_formula(x, ops.TOKEN_LAYERNORM, self.weight, self.bias, self.eps)
+        return F.layer_norm(x, self.normalized_shape, None if self.weight is None else self.weight + 1.0, self.bias, self.eps)
 
 
 class NormalizedFeedForwardNetwork(nn.Module):
@@ -142,12 +142,13 @@ class NormalizedFeedForwardNetwork(nn.Module):
         vec = 16 // x.element_size()
         return (one_graph(x, norm.weight, getattr(norm, 'bias', None), self.fc1.weight, self.fc1.bias, self.fc2.weight)
                 and self.layerscale_weight is None and x.shape[-1] % vec == 0 and x.shape[-1] <= 2048
-                and self.hidden_dim % vec == 0 and _plain(self.fc1, self.fc2) and _unhooked((RMSNorm, LayerNorm), norm)
+                and self.hidden_dim % vec == 0 and norm_width_ok(norm, x.shape[-1]) and _plain(self.fc1, self.fc2) and _unhooked((RMSNorm, LayerNorm), norm)
                 and not (self.training and (self.dropout_p > 0 or self.hidden_dropout_p > 0)))
 
     def _few_rows_cover(self, x: Tensor) -> bool:
         norm = self.norm
-        return (self.hidden_dim % 32 == 0 and not (self.training and self.dropout_p > 0) and _plain(self.fc1, self.fc2)
+        return (self.hidden_dim % 32 == 0 and norm_width_ok(norm, x.shape[-1])
+                and not (self.training and self.dropout_p > 0) and _plain(self.fc1, self.fc2)
                 and _unhooked((RMSNorm, LayerNorm), norm)
                 and ops._lib.load_host().uniform(x, norm.weight, getattr(norm, 'bias', None), self.fc1.weight, self.fc1.bias,
                                                  self.fc2.weight, self.layerscale_weight))

@@ -1029,12 +1029,18 @@ def one_graph(x: Tensor, *params) -> bool:
         not torch.is_autocast_enabled() and ops._lib.load_host().trainable(x, *params)
 
 
+def norm_width_ok(norm: nn.Module, D: int) -> bool:
+    """A row norm's parameters fit rows of D values (where they do not, the general path says so)."""
+    shape = getattr(norm, 'normalized_shape', None)
+    return (shape is None or tuple(shape) == (D,)) and all(p is None or p.shape == (D,) for p in norm._parameters.values())
+
+
 def row_norm_covers(x: Tensor, *params) -> bool:
-    """The row kernels take x: 16-bit or single precision, whole 16-byte rows, and an eager call (tracing, function
-    transforms and forward-mode tangents keep torch's own operations)."""
+    """The row kernels take x: 16-bit or single precision, whole 16-byte rows, parameters of that width, and an eager call
+    (tracing, function transforms and forward-mode tangents keep torch's own operations)."""
     D = x.shape[-1]
     return not torch.compiler.is_compiling() and x.is_cuda and D % (16 // x.element_size()) == 0 and D <= 2048 and not torch.is_autocast_enabled() and \
-        ops._lib.load_host().uniform(x, *params)
+        all(p is None or p.shape == (D,) for p in params) and ops._lib.load_host().uniform(x, *params)
 
 
 class RowNormFunc(torch.autograd.Function):
