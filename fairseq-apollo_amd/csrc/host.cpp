@@ -548,7 +548,7 @@ Tensor row_norm(const Tensor& x, const Tensor& w, const Tensor& b, int kind, dou
 std::tuple<Tensor, Tensor, Tensor> row_norm_back(const Tensor& dy, const Tensor& x, const Tensor& w, const Tensor& b,
                                                  const Tensor& add, int kind, double eps, void* s, const char* who) {
   norm_width(x, w, b, who);
-  if (dy.sizes() != x.sizes()) throw std::runtime_error(std::string(who) + ": the gradient must have the rows' shape");
+  if (dy.numel() != x.numel() || dy.size(-1) != x.size(-1)) throw std::runtime_error(std::string(who) + ": the gradient must have the rows' shape");
   Tensor dx = at::empty_like(x), dw, db;
   if (w.defined()) dw = at::empty_like(w);
   if (b.defined()) db = at::empty_like(b);
