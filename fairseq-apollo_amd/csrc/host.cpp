@@ -652,6 +652,9 @@ PyObject* ffn_backward(const Args& A) {
   const Tensor dout = A.t(0).to(x.scalar_type()).contiguous();
   same_type(A, {1, 2, 3, 4, 6, 7, 9, 10}, x);
   void* s = A.stream(11);
+  A.shape(4, pre.sizes());
+  if (dout.numel() != x.numel() || n.numel() != x.numel() || pre.numel() != x.numel() / x.size(-1) * A.t(10).size(1))
+    throw std::runtime_error("ffn_backward: gradients and saved operands of other sizes than the forward's");
   const Tensor d2 = rows2(dout);
   Tensor dw2 = at::mm(d2.t(), h);
   Tensor dh = at::mm(d2, A.t(10));
@@ -686,6 +689,8 @@ PyObject* swiglu_backward(const Args& A) {
   const Tensor &n = A.t(1), &a = A.t(2), &b = A.t(3), &g = A.t(4);
   same_type(A, {1, 2, 3, 4, 5, 6, 7}, n);
   void* s = A.stream(8);
+  A.shape(3, a.sizes());
+  A.shape(4, a.sizes());
   const Tensor d2 = rows2(A.t(0).to(n.scalar_type()).contiguous()), n2 = rows2(n);
   Tensor dw2 = at::mm(d2.t(), g);
   Tensor dg = at::mm(d2, A.t(7));
@@ -760,6 +765,11 @@ PyObject* mix_out_backward(const Args& A) {
   void* s = A.stream(8);
   const int dt = dtype_code(x);
   const int64_t D = x.size(2), E = attn.size(-1), S = A.i64(7), W = base.size(1), T = x.numel() / D, es = x.element_size();
+  if (dout.numel() != x.numel() || attn.numel() != T * E) throw std::runtime_error("mix_out_backward: the gradient must have the residual's shape, attention [tokens, E]");
+  A.shape(2, {T, 2 * D + S + E});
+  A.shape(4, {T, E});
+  A.shape(5, {T, D});
+  A.shape(6, {D, E});
   const char* b = (const char*)base.data_ptr();
   Tensor dbase = at::empty_like(base), dres = at::empty_like(x);
   char* db = (char*)dbase.data_ptr();
@@ -788,7 +798,17 @@ PyObject* mix_backward(const Args& A) {
   const Tensor dq = A.t(0).to(xn.scalar_type()).contiguous(), dk = A.t(1).to(xn.scalar_type()).contiguous();
   const Tensor dv = A.t(2).to(xn.scalar_type()).contiguous();
   const int64_t D = xn.size(2), S = A.t(11).size(1), heads = A.i64(13), chunk = A.i64(14), T = xn.numel() / D;
-  const int64_t W = base.size(1), es = xn.element_size();
+  const int64_t W = base.size(1), es = xn.element_size(), E = vp.size(-1);
+  if (dq.numel() != T * S || dk.numel() != T * S || dv.numel() != T * E || act.numel() != T * D || mx.numel() != T * D ||
+      mx.size(-1) != D || act.size(-1) != D || W != 2 * D + S + E)
+    throw std::runtime_error("mix_backward: gradients and saved operands of other sizes than the forward's");
+  A.shape(3, {T, W});
+  A.shape(5, {T, E});
+  A.shape(8, {T, W});
+  A.shape(9, {E, D});
+  A.shape(10, {W, D});
+  A.shape(11, {2, S});
+  A.shape(16, {D});
   Tensor dgamma = at::empty_like(A.t(11)), dbeta = at::empty_like(A.t(11));
   {
     const int64_t nws = (int64_t)mega_gate_qk_bwd_workspace_bytes(T, S);

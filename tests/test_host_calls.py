@@ -43,6 +43,35 @@ def test_composite_operands_of_other_shapes():
         H.swiglu_forward(x[0], None, torch.zeros(12, D), torch.zeros(8, D), torch.zeros(D, 12), 0)
 
 
+def test_backward_operands_of_other_shapes():
+    """The backward passes size their kernels from a saved operand or two: the others must fit."""
+    D, S, E, T = 8, 4, 16, 3
+    W = 2 * D + S + E
+    x, row = torch.zeros(1, T, D), lambda *s: torch.zeros(*s)
+    out = [x, x, row(T, W), row(T, E), row(T, E), row(T, D), row(D, E), S, 0]
+    for i, bad in ((0, row(1, T, D - 1)), (2, row(T, W + 2)), (3, row(T - 1, E)), (4, row(T, E - 2)), (5, row(T, E)), (6, row(D + 1, E))):
+        args = list(out)
+        args[i] = bad
+        with pytest.raises(RuntimeError, match="mix_out_backward: "):
+            H.mix_out_backward(*args)
+    back = [row(T, S), row(T, S), row(T, E), row(T, W), x, row(T, E), x, x, row(T, W), row(E, D), row(W, D), row(2, S), row(S // 2),
+            1, T, RMS, row(D), 1e-5, 0]
+    for i, bad in ((0, row(T, S + 2)), (2, row(T + 1, E)), (3, row(T, W + 1)), (6, row(1, T, D + 8)), (8, row(T + 1, W)),
+                   (10, row(W, D - 1)), (11, row(2, S + 2)), (16, row(D + 8))):
+        args = list(back)
+        args[i] = bad
+        with pytest.raises(RuntimeError, match="mix_backward: "):
+            H.mix_backward(*args)
+    ffn = [x, x, x, row(T, 6), row(T, 6), LN, row(D), row(D), 1e-5, row(6, D), row(D, 6), 0]
+    for i, bad in ((0, row(1, T + 1, D)), (3, row(T, 5)), (4, row(T + 1, 6))):
+        args = list(ffn)
+        args[i] = bad
+        with pytest.raises(RuntimeError, match="ffn_backward: "):
+            H.ffn_backward(*args)
+    with pytest.raises(RuntimeError, match="swiglu_backward: argument 3 must be"):
+        H.swiglu_backward(x, x, row(T, 6), row(T, 5), row(T, 6), row(6, D), row(6, D), row(D, 6), 0)
+
+
 def test_norm_widths():
     """What the gates of the norms and of the feed-forward composites ask: parameters as wide as the rows."""
     for norm in (M.layers.LayerNorm(8), M.layers.RMSNorm(8)):
