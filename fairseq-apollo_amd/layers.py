@@ -142,13 +142,14 @@ class NormalizedFeedForwardNetwork(nn.Module):
         vec = 16 // x.element_size()
         return (one_graph(x, norm.weight, getattr(norm, 'bias', None), self.fc1.weight, self.fc1.bias, self.fc2.weight)
                 and self.layerscale_weight is None and x.shape[-1] % vec == 0 and x.shape[-1] <= 2048
-                and self.hidden_dim % vec == 0 and norm_width_ok(norm, x.shape[-1]) and _plain(self.fc1, self.fc2) and _unhooked((RMSNorm, LayerNorm), norm)
+                and self.hidden_dim % vec == 0 and norm_width_ok(norm, x.shape[-1])
+                and _plain(True, self.fc1) and _plain(False, self.fc2) and _unhooked((RMSNorm, LayerNorm), norm)
                 and not (self.training and (self.dropout_p > 0 or self.hidden_dropout_p > 0)))
 
     def _few_rows_cover(self, x: Tensor) -> bool:
         norm = self.norm
         return (self.hidden_dim % 32 == 0 and norm_width_ok(norm, x.shape[-1])
-                and not (self.training and self.dropout_p > 0) and _plain(self.fc1, self.fc2)
+                and not (self.training and self.dropout_p > 0) and _plain(True, self.fc1) and _plain(False, self.fc2)
                 and _unhooked((RMSNorm, LayerNorm), norm)
                 and ops._lib.load_host().uniform(x, norm.weight, getattr(norm, 'bias', None), self.fc1.weight, self.fc1.bias,
                                                  self.fc2.weight, self.layerscale_weight))
@@ -376,7 +377,8 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
         z, h, Nh = self.zdim, self.hdim, self.num_heads
         mine, mods = self._parameters, self._modules
         v_proj, mx_proj, h_proj, act = (mods[k] for k in ('v_proj', 'mx_proj', 'h_proj', 'move_act'))
-        return (ops.token_rows(x, normalised=True) and mask_bytes_ok(padding_mask) and _plain(v_proj, mx_proj, h_proj)
+        return (ops.token_rows(x, normalised=True) and mask_bytes_ok(padding_mask)
+                and _plain(True, v_proj, mx_proj) and _plain(False, h_proj) and 'gamma' in mine and 'beta' in mine
                 and _unhooked((RMSNorm, nn.SiLU), act)
                 and ops._lib.load_host().uniform(
                     x, *v_proj._parameters.values(), *mx_proj._parameters.values(), *h_proj._parameters.values(),
@@ -570,7 +572,7 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
                 and mx.dtype == xn.dtype and residual.dtype == xn.dtype and residual.data_ptr() % 16 == 0
                 and self.embed_dim % vec == 0 and self.zdim % vec == 0 and self.hdim % vec == 0 and self.zdim <= 128 * vec
                 and (not rms or self.embed_dim <= 2048) and _unhooked((RMSNorm, nn.SiLU), act)
-                and _plain(self.v_proj, self.mx_proj, self.h_proj)
+                and _plain(True, self.v_proj, self.mx_proj) and _plain(False, self.h_proj)
                 and not (self.training and (self.dropout_p > 0 or self.hidden_dropout_p > 0)))
 
     def _mix_autograd(self, residual: Tensor, xn: Tensor, mx: Tensor, padding_mask: Optional[Tensor]) -> Tensor:

@@ -75,7 +75,7 @@ class MegaDecoderNoCrossAttn(nn.Module):
         """Project features to the vocabulary (mega_lm.py:379-385)."""
         proj = self.output_projection
         w = proj.weight
-        if not torch.is_grad_enabled() and ops.token_rows(features) and _plain(proj) and proj.bias is None and \
+        if not torch.is_grad_enabled() and ops.token_rows(features) and _plain(False, proj) and \
                 ops._lib.load_host().uniform(features, w):
             return ops.token_linear(features, w)
         return proj(features)

@@ -1017,9 +1017,16 @@ def _unhooked(kinds: tuple, *mods) -> bool:
     return True
 
 
-def _plain(*layers) -> bool:
-    """Linear layers as torch defines them, _unhooked."""
-    return _unhooked((nn.Linear,), *layers)
+def _plain(bias: bool, *layers) -> bool:
+    """Linear layers as torch defines them, _unhooked, their weights parameters; `bias`: all of them with one, or all without.
+    (A composite reads the biases that its formula has and no others.)"""
+    if not _unhooked((nn.Linear,), *layers):
+        return False
+    for m in layers:
+        p = m._parameters
+        if p.get('weight') is None or (p.get('bias') is None if bias else p.get('bias', p) is not None):
+            return False
+    return True
 
 
 def one_graph(x: Tensor, *params) -> bool:
@@ -1327,8 +1334,8 @@ class SwiGLU(nn.Module):
         """W2 (silu(W1 x) * W3 x) (+ residual, which then enters the last product as its accumulator start: no
         separate addition pass over the activations; consume_residual: see linear_residual)."""
         w1, w3, w2 = self.w1, self.w3, self.w2
-        if one_graph(x, w1.weight, w3.weight, w2.weight) and w1.bias is None and w3.bias is None and w2.bias is None and \
-                _plain(w1, w3, w2) and (residual is None or (residual.dtype == x.dtype and residual.is_contiguous()
+        if one_graph(x, w1.weight, w3.weight, w2.weight) and _plain(False, w1, w3, w2) and \
+                (residual is None or (residual.dtype == x.dtype and residual.is_contiguous()
                                                              and residual.device == x.device
                                                              and residual.shape[:-1] == x.shape[:-1]
                                                              and residual.shape[-1] == w2.out_features)):

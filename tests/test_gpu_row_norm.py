@@ -134,3 +134,63 @@ def test_norms_under_transforms(norm):
         near(torch.autograd.forward_ad.unpack_dual(dual).tangent, want[1])
     traced = torch.jit.trace(dev, xd, check_trace=False)
     near(traced(td), cpu(t))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("first,second", [(True, True), (False, False), (False, True)])
+def test_feed_forward_of_other_projections(dtype, first, second):
+    """Projections with and without a bias where the constructor builds the other form: every bias enters the result and
+    gets its gradient.  Against fp64 of the same formula.  These run operator by operator: eight results in a row are
+    rounded on the longest way (weight + 1, norm, product, activation and back through the product, the activation, the
+    norm and the sum with the residual's share): 8 ulp of the rms and of the value."""
+    D, ffn, T = 64, 96, 33
+    torch.manual_seed(2)
+    block = M.NormalizedFeedForwardNetwork(D, ffn)
+    block.fc1, block.fc2 = torch.nn.Linear(D, ffn, bias=first), torch.nn.Linear(ffn, D, bias=second)
+    block = block.to(DEV).to(dtype).train()
+    with torch.no_grad():
+        for p in block.parameters():
+            p.normal_(0, 0.1)
+    x = torch.randn(2, T, D, device=DEV).to(dtype).requires_grad_(True)
+    dy = torch.randn(2, T, D, device=DEV).to(dtype)
+    y = block(x)
+    y.backward(dy)
+    P = {k: v.detach().double().cpu().requires_grad_(True) for k, v in block.named_parameters()}
+    x64 = x.detach().double().cpu().requires_grad_(True)
+    n = F.layer_norm(x64, (D,), P['norm.weight'] + 1, P['norm.bias'], 1e-5)
+    y64 = x64 + F.linear(F.silu(F.linear(n, P['fc1.weight'], P.get('fc1.bias'))), P['fc2.weight'], P.get('fc2.bias'))
+    y64.backward(dy.double().cpu())
+    for got, ref in [(y, y64), (x.grad, x64.grad)] + [(p.grad, P[k].grad) for k, p in block.named_parameters()]:
+        _close(got.detach(), ref.detach(), dtype, 8 * (ref.detach().abs() + ref.detach().pow(2).mean().sqrt()))
+
+
+@pytest.mark.parametrize("name,bias", [("h_proj", True), ("v_proj", False), ("mx_proj", False)])
+def test_gated_attention_of_other_projections(name, bias):
+    """The gated attention with a projection of the other form against the operators one by one (a frozen parameter) in
+    fp32; sums of up to 300 terms in another order: 8 ulp of the rms and of the value, as in the test above."""
+    torch.manual_seed(4)
+    layer = M.MovingAverageGatedAttention(64, 32, 128, 8, chunk_size=32, norm_num_groups=4)
+    old = getattr(layer, name)
+    setattr(layer, name, torch.nn.Linear(old.in_features, old.out_features, bias=bias))
+    layer = layer.to(DEV).train()
+    with torch.no_grad():
+        for p in layer.parameters():
+            if not bool(p.any()):
+                p.normal_(0, 0.2)
+    x0, dy = (torch.randn(2, 96, 64, device=DEV) for _ in range(2))
+    out = []
+    for freeze in (False, True):
+        layer.gamma.requires_grad_(not freeze)
+        layer.zero_grad()
+        x = x0.clone().requires_grad_(True)
+        y, _ = layer(x)
+        y.backward(dy)
+        out.append([y.detach(), x.grad] + [p.grad for n, p in layer.named_parameters() if n != 'gamma'])
+    for a, b in zip(*out):
+        assert a is not None and b is not None
+        b64 = b.double().cpu()
+        _close(a, b64, torch.float32, 8 * (b64.abs() + b64.pow(2).mean().sqrt()))
+    if bias:                                               # the result without the bias is another one
+        with torch.no_grad():
+            layer.h_proj.bias.zero_()
+        assert not torch.allclose(layer(x0)[0], out[0][0], rtol=1e-3, atol=1e-3)

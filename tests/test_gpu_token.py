@@ -129,3 +129,27 @@ def test_token_of_modules_that_are_not_plain(change):
         got, want = half(tokens[:, 19:], incremental_state=sa)[0], full(tokens[:, 19:], incremental_state=sb)[0]
     assert len(calls) == {"hook": len(lins) + 1, "subclass": len(lins), "columns": 0}[change]
     assert _rms(got, want) < TOL[torch.bfloat16]
+
+
+@pytest.mark.parametrize("name,bias", [("fc2", True), ("fc1", False), ("h_proj", True), ("v_proj", False), ("mx_proj", False)])
+def test_token_of_other_projections(name, bias):
+    """A projection with a bias where the layer's own has none, and without where it has one: the token is that of the
+    operators one by one, in the composite's tolerance, and a bias counts."""
+    half, _ = _model(64, 16, 64, 1, 64, 64, "layernorm", torch.bfloat16, 5)
+    for layer in half.layers:
+        block = layer.nffn if name.startswith("fc") else layer.mega_layer
+        old = getattr(block, name)
+        new = torch.nn.Linear(old.in_features, old.out_features, bias=bias)
+        torch.nn.init.normal_(new.weight, 0, 0.1)
+        if bias:
+            torch.nn.init.normal_(new.bias, 0, 1.0)
+        setattr(block, name, new.to(DEV).to(torch.bfloat16))
+    half.eval()
+    full = copy.deepcopy(half).float()
+    tokens = torch.randint(2, 72, (3, 20), device=DEV)
+    sa, sb = {}, {}
+    with torch.no_grad():
+        half(tokens[:, :19], incremental_state=sa)
+        full(tokens[:, :19], incremental_state=sb)
+        got, want = half(tokens[:, 19:], incremental_state=sa)[0], full(tokens[:, 19:], incremental_state=sb)[0]
+    assert _rms(got, want) < TOL[torch.bfloat16]
