@@ -1008,11 +1008,20 @@ def linear(lin: nn.Linear, x: Tensor) -> Tensor:
     return lin(x)
 
 
+_EVERY_MODULE = [getattr(nn.modules.module, f'_global_{kind}_hooks') for kind in
+                 ('forward', 'forward_pre', 'backward', 'backward_pre')]
+
+
 def _unhooked(kinds: tuple, *mods) -> bool:
-    """Modules of exactly these types, nobody looking at their inputs or outputs: what reads their parameters directly may
-    stand in for the calls."""
+    """Modules of exactly these types whose call is their class's own, nobody looking at their inputs or outputs (hooks of
+    their own or on every module, a `forward` replaced on the instance): what reads their parameters directly may stand
+    in for the calls."""
+    for hooks in _EVERY_MODULE:
+        if hooks:
+            return False
     for m in mods:
-        if type(m) not in kinds or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks:
+        if type(m) not in kinds or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks \
+                or 'forward' in m.__dict__:
             return False
     return True
 

@@ -194,3 +194,29 @@ def test_gated_attention_of_other_projections(name, bias):
         with torch.no_grad():
             layer.h_proj.bias.zero_()
         assert not torch.allclose(layer(x0)[0], out[0][0], rtol=1e-3, atol=1e-3)
+
+
+@pytest.mark.parametrize("change", ["forward", "global"])
+def test_composites_of_replaced_forwards(change):
+    """Modules whose `forward` was replaced on the instance, and hooks on every module of the program, are called in
+    training wherever the operators one by one call them (fc1, v_proj and mx_proj run there as products of their own)."""
+    torch.manual_seed(4)
+    layer = M.Mega2Layer(64, 32, 128, 8, 96, 32, norm_num_groups=4, moving_act='rmsnorm').to(DEV).train()
+    block = M.NormalizedFeedForwardNetwork(64, 96).to(DEV).train()
+    seen = [layer.attn.move_act, layer.attn.h_proj, layer.ffn.w1, layer.ffn.w3, block.norm]
+    x, calls = torch.randn(2, 96, 64, device=DEV), []
+    want = [layer(x).detach(), block(x).detach()]
+    if change == "forward":
+        for m in seen:
+            m.forward = lambda v, m=m, f=m.forward: calls.append(m) or f(v)
+        got = [layer(x), block(x)]
+    else:
+        handle = torch.nn.modules.module.register_module_forward_hook(lambda m, *a: calls.append(m))
+        try:
+            got = [layer(x), block(x)]
+        finally:
+            handle.remove()
+    assert all(sum(c is m for c in calls) == 1 for m in seen)
+    for a, b in zip(got, want):
+        b64 = b.double().cpu()
+        _close(a.detach(), b64, torch.float32, 8 * (b64.abs() + b64.pow(2).mean().sqrt()))

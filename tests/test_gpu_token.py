@@ -153,3 +153,30 @@ def test_token_of_other_projections(name, bias):
         full(tokens[:, :19], incremental_state=sb)
         got, want = half(tokens[:, 19:], incremental_state=sa)[0], full(tokens[:, 19:], incremental_state=sb)[0]
     assert _rms(got, want) < TOL[torch.bfloat16]
+
+
+@pytest.mark.parametrize("change", ["forward", "global"])
+def test_token_of_replaced_forwards(change):
+    """A projection, norm or embedding whose `forward` was replaced on the instance (offloading, adapters), and hooks on
+    every module of the program: each is called, as the operators one by one call it."""
+    half, full = _model(64, 16, 64, 1, 64, 64, "layernorm", torch.bfloat16, 5)
+    tokens = torch.randint(2, 72, (3, 20), device=DEV)
+    sa, sb, calls = {}, {}, []
+    seen = [m for n, m in half.named_modules() if type(m) in (torch.nn.Linear, M.layers.LayerNorm) and not n.endswith('fc2')]
+    seen.append(half.embed_tokens)
+    with torch.no_grad():
+        half(tokens[:, :19], incremental_state=sa)
+        full(tokens[:, :19], incremental_state=sb)
+        want = full(tokens[:, 19:], incremental_state=sb)[0]
+        if change == "forward":
+            for m in seen:
+                m.forward = lambda x, m=m, f=m.forward: calls.append(m) or f(x)
+            got = half(tokens[:, 19:], incremental_state=sa)[0]
+        else:
+            handle = torch.nn.modules.module.register_module_forward_hook(lambda m, *a: calls.append(m))
+            try:
+                got = half(tokens[:, 19:], incremental_state=sa)[0]
+            finally:
+                handle.remove()
+    assert all(sum(c is m for c in calls) == 1 for m in seen)
+    assert _rms(got, want) < TOL[torch.bfloat16]
