@@ -138,21 +138,20 @@ class NormalizedFeedForwardNetwork(nn.Module):
 
     def _one_operator(self, x: Tensor) -> bool:
         """A training call the composite operator takes (no layer scale, no active dropout, whole 16-byte rows)."""
-        norm = self.norm
+        norm, fc1, fc2 = self.norm, self.fc1, self.fc2
         vec = 16 // x.element_size()
-        return (one_graph(x, norm.weight, getattr(norm, 'bias', None), self.fc1.weight, self.fc1.bias, self.fc2.weight)
+        return (torch.is_grad_enabled() and _plain(True, fc1) and _plain(False, fc2) and _unhooked((RMSNorm, LayerNorm), norm)
                 and self.layerscale_weight is None and x.shape[-1] % vec == 0 and x.shape[-1] <= 2048
                 and self.hidden_dim % vec == 0 and norm_width_ok(norm, x.shape[-1])
-                and _plain(True, self.fc1) and _plain(False, self.fc2) and _unhooked((RMSNorm, LayerNorm), norm)
-                and not (self.training and (self.dropout_p > 0 or self.hidden_dropout_p > 0)))
+                and not (self.training and (self.dropout_p > 0 or self.hidden_dropout_p > 0))
+                and one_graph(x, norm.weight, getattr(norm, 'bias', None), fc1.weight, fc1.bias, fc2.weight))
 
     def _few_rows_cover(self, x: Tensor) -> bool:
-        norm = self.norm
-        return (self.hidden_dim % 32 == 0 and norm_width_ok(norm, x.shape[-1])
-                and not (self.training and self.dropout_p > 0) and _plain(True, self.fc1) and _plain(False, self.fc2)
-                and _unhooked((RMSNorm, LayerNorm), norm)
-                and ops._lib.load_host().uniform(x, norm.weight, getattr(norm, 'bias', None), self.fc1.weight, self.fc1.bias,
-                                                 self.fc2.weight, self.layerscale_weight))
+        norm, fc1, fc2 = self.norm, self.fc1, self.fc2
+        return (self.hidden_dim % 32 == 0 and _plain(True, fc1) and _plain(False, fc2) and _unhooked((RMSNorm, LayerNorm), norm)
+                and norm_width_ok(norm, x.shape[-1]) and not (self.training and self.dropout_p > 0)
+                and ops._lib.load_host().uniform(x, norm.weight, getattr(norm, 'bias', None), fc1.weight, fc1.bias, fc2.weight,
+                                                 self.layerscale_weight))
 
     def _few_rows(self, x: Tensor) -> Tensor:
         """The block on one token per stream: two launches (norm, first projection and activation; second projection,
@@ -567,13 +566,14 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
         vec = 16 // xn.element_size()
         act = self.move_act
         rms = isinstance(act, RMSNorm)
-        return (one_graph(xn, self.v_proj.weight, self.v_proj.bias, self.mx_proj.weight, self.mx_proj.bias, self.h_proj.weight,
-                          self.gamma, self.beta, act.weight if rms else None)
-                and mx.dtype == xn.dtype and residual.dtype == xn.dtype and residual.data_ptr() % 16 == 0
+        return (torch.is_grad_enabled() and _plain(True, self.v_proj, self.mx_proj) and _plain(False, self.h_proj)
+                and _unhooked((RMSNorm, nn.SiLU), act) and mx.dtype == xn.dtype and residual.dtype == xn.dtype
+                and residual.data_ptr() % 16 == 0
                 and self.embed_dim % vec == 0 and self.zdim % vec == 0 and self.hdim % vec == 0 and self.zdim <= 128 * vec
-                and (not rms or self.embed_dim <= 2048) and _unhooked((RMSNorm, nn.SiLU), act)
-                and _plain(True, self.v_proj, self.mx_proj) and _plain(False, self.h_proj)
-                and not (self.training and (self.dropout_p > 0 or self.hidden_dropout_p > 0)))
+                and (not rms or self.embed_dim <= 2048)
+                and not (self.training and (self.dropout_p > 0 or self.hidden_dropout_p > 0))
+                and one_graph(xn, self.v_proj.weight, self.v_proj.bias, self.mx_proj.weight, self.mx_proj.bias,
+                              self.h_proj.weight, self.gamma, self.beta, act.weight if rms else None))
 
     def _mix_autograd(self, residual: Tensor, xn: Tensor, mx: Tensor, padding_mask: Optional[Tensor]) -> Tensor:
         bsz, seq_len, _ = xn.size()

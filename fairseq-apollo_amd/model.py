@@ -74,10 +74,9 @@ class MegaDecoderNoCrossAttn(nn.Module):
     def output_layer(self, features: Tensor) -> Tensor:
         """Project features to the vocabulary (mega_lm.py:379-385)."""
         proj = self.output_projection
-        w = proj.weight
         if not torch.is_grad_enabled() and ops.token_rows(features) and _plain(False, proj) and \
-                ops._lib.load_host().uniform(features, w):
-            return ops.token_linear(features, w)
+                ops._lib.load_host().uniform(features, proj.weight):
+            return ops.token_linear(features, proj.weight)
         return proj(features)
 
     def max_positions(self) -> int:
@@ -115,8 +114,10 @@ class MegaDecoderNoCrossAttn(nn.Module):
 
     def _token_covers(self, tokens: Tensor) -> bool:
         embed = self.embed_tokens
+        if not _unhooked((nn.Embedding,), embed):
+            return False
         w = embed.weight
-        return (_unhooked((nn.Embedding,), embed) and embed.max_norm is None and not torch.is_grad_enabled() and w.is_cuda and w.dtype in (torch.bfloat16, torch.float16)
+        return (embed.max_norm is None and not torch.is_grad_enabled() and w.is_cuda and w.dtype in (torch.bfloat16, torch.float16)
                 and w.is_contiguous() and w.shape[1] % 8 == 0 and tokens.dtype is torch.int64 and tokens.is_contiguous()
                 and tokens.device == w.device and not (self.training and self.embedding_dropout.p > 0))
 

@@ -180,3 +180,39 @@ def test_token_of_replaced_forwards(change):
                 handle.remove()
     assert all(sum(c is m for c in calls) == 1 for m in seen)
     assert _rms(got, want) < TOL[torch.bfloat16]
+
+
+class Within(torch.nn.Module):
+    """A module that holds another one, and has no weight of its own."""
+
+    def __init__(self, inner):
+        super().__init__()
+        self.inner = inner
+
+    def forward(self, x):
+        return self.inner(x)
+
+
+def test_modules_without_a_weight():
+    """Projections, norms and embeddings inside other modules: token by token and slice by slice as the operators one by
+    one, and SwiGLU's first two projections in training too."""
+    half, full = _model(64, 16, 64, 1, 64, 64, "layernorm", torch.bfloat16, 5)
+    for m in list(half.modules()):
+        for name in ('fc1', 'norm', 'v_proj', 'mx_proj', 'h_proj', 'output_projection', 'embed_tokens'):
+            old = m._modules.get(name)
+            if type(old) in (torch.nn.Linear, torch.nn.Embedding, M.layers.LayerNorm):
+                setattr(m, name, Within(old))
+    tokens = torch.randint(2, 72, (3, 20), device=DEV)
+    sa, sb = {}, {}
+    with torch.no_grad():
+        for a, b in ((0, 19), (19, 20)):
+            got, want = half(tokens[:, a:b], incremental_state=sa)[0], full(tokens[:, a:b], incremental_state=sb)[0]
+            assert _rms(got, want) < TOL[torch.bfloat16]
+    ffn = M.SwiGLU(64, 96).to(DEV)
+    x = torch.randn(2, 9, 64, device=DEV)
+    want = ffn(x, x)
+    ffn.w1, ffn.w3 = Within(ffn.w1), Within(ffn.w3)
+    # fp32: sums of 96 products in another order
+    assert _rms(ffn(x, x).detach(), want.detach()) < 1e-6
+    with torch.no_grad():
+        assert _rms(ffn(x, x), want) < 1e-6
