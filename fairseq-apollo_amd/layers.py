@@ -623,7 +623,7 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
         bsz, seq_len = z.shape[:2]
         Nh = self.num_heads
         if (self.chunk_size > 1 and seq_len % self.chunk_size == 0 and "prev_key" not in saved_state and not simple
-                and not self.bidirectional and self.attention_activation == 'softmax'):
+                and not self.bidirectional and self.attention_activation == 'softmax' and not torch.is_autocast_enabled()):
             # whole chunks behind whole chunks: nothing cached, nothing to cache
             self._set_input_buffer(incremental_state, saved_state)
             q, k = ops.gate_qk_fwd(z, *self._qk_constants(False), Nh, self.chunk_size)

@@ -159,7 +159,8 @@ _TOKEN_LDS = 144 * 1024               # bytes of normalised input rows a project
 def token_rows(x: torch.Tensor, normalised: bool = False) -> bool:
     """True when the projections of x [rows, 1, K] run on the one-token kernels: 16-bit activations on the GPU, few
     rows, whole 16-byte pieces; `normalised`: the rows are staged in LDS by every workgroup."""
-    if not (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and x.dim() == 3 and x.shape[1] == 1):
+    if not (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and x.dim() == 3 and x.shape[1] == 1) or \
+            torch.is_autocast_enabled():               # (autocast picks the type of every product and norm by itself)
         return False
     B, K = x.shape[0], x.shape[2]
     return 0 < B <= TOKEN_ROWS and K % 32 == 0 and x.is_contiguous() and \

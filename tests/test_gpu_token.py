@@ -216,3 +216,20 @@ def test_modules_without_a_weight():
     assert _rms(ffn(x, x).detach(), want.detach()) < 1e-6
     with torch.no_grad():
         assert _rms(ffn(x, x), want) < 1e-6
+
+
+def test_carried_state_under_autocast():
+    """Autocast picks the type of every operation: one token leaves the state that the operators one by one leave (keys
+    in fp32 behind the normalisation), and mixed types are refused as they are there."""
+    half, _ = _model(64, 16, 64, 1, 64, 64, "layernorm", torch.bfloat16, 5)
+    tokens = torch.randint(2, 72, (3, 20), device=DEV)
+    state = {}
+    with torch.no_grad():
+        half(tokens[:, :19], incremental_state=state)
+        other = {n: dict(e) for n, e in state.items()}
+        with torch.autocast('cuda', dtype=torch.bfloat16):
+            half(tokens[:, 19:], incremental_state=state)
+        with torch.autocast('cuda', dtype=torch.float16), pytest.raises(RuntimeError, match="dtype"):
+            half(tokens[:, 19:], incremental_state=other)
+    keys = [e["prev_key"] for e in state.values() if "prev_key" in e]
+    assert len(keys) == 2 and all(k.dtype == torch.float32 for k in keys)
