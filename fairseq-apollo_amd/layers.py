@@ -29,6 +29,11 @@ from .modules import (AttentionSoftmax, EfficientAttention, FeedForwardFunc, Gat
                       silu)
 
 
+def _cached_rows(t: Tensor, x: Tensor) -> bool:
+    """Cached rows that the one-token kernels read and copy in 16-byte pieces beside activations x."""
+    return t.dtype == x.dtype and t.is_contiguous() and t.data_ptr() % 16 == 0
+
+
 class RMSNorm(nn.Module):
     """x / sqrt(mean(x^2) + eps) * (weight + 1): the parameter is stored as the offset from one and starts at zero, as
     in the reference (fairseq/modules/norm_layer/layer_norm.py:41-59: FusedRMSNorm.reset_parameters zeroes it and
@@ -388,7 +393,7 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
                 and h % 32 == 0 and h % (8 * Nh) == 0 and z % (8 * Nh) == 0 and z // Nh <= 512
                 and (key is None or (key.dtype == x.dtype and key.stride(2) == 1 and key.stride(1) % 8 == 0
                                      and key.stride(0) % 8 == 0 and key.data_ptr() % 16 == 0
-                                     and saved_state["prev_value"].is_contiguous()
+                                     and _cached_rows(saved_state["prev_value"], x)
                                      and (self.chunk_size < 0 or key.size(1) < self.chunk_size))))
 
     def _token_step(self, x: Tensor, padding_mask: Optional[Tensor], saved_state, incremental_state) -> Optional[Tensor]:
@@ -400,7 +405,9 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
         if count is None or mean is None or var is None:
             count, mean, var = norm._prior_state(x.size(0))
         h = move_state.get('prev_state')
-        if h is not None and not (h.dtype is torch.complex64 and h.is_contiguous() and not h.is_conj()):
+        if h is not None and not (h.dtype is torch.complex64 and h.is_contiguous() and not h.is_conj() and h.data_ptr() % 16 == 0):
+            return None
+        if not (count.dtype is torch.int64 and count.is_contiguous()):
             return None
         gamma, beta = norm._affine()
         ema = move._prepared_layer()

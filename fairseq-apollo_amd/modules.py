@@ -577,7 +577,7 @@ class TimestepNorm(nn.Module, IncrementalState):
             return out
         gamma, beta = self._affine()
         if incremental_state is not None and x.size(1) == 1 and self.num_groups is not None and x.is_cuda and \
-                x.is_contiguous() and mask_bytes_ok(padding_mask):
+                x.is_contiguous() and mask_bytes_ok(padding_mask) and prev_count.dtype is torch.int64 and prev_count.is_contiguous():
             # one token per stream: no look-back over time, one wave per (stream, group)
             with ops._on_device(x.device):
                 out, count, mean, var = ops._lib.load_host().token_norm(

@@ -233,3 +233,22 @@ def test_carried_state_under_autocast():
             half(tokens[:, 19:], incremental_state=other)
     keys = [e["prev_key"] for e in state.values() if "prev_key" in e]
     assert len(keys) == 2 and all(k.dtype == torch.float32 for k in keys)
+
+
+@pytest.mark.parametrize("entry", ["prev_value", "prev_key", "prev_state", "prev_count"])
+def test_token_with_state_in_other_storage(entry):
+    """Carried state that starts on no 16 bytes (a view of a packed buffer), counts that are every second of a buffer's:
+    the token is that of the operators one by one, in the composite's tolerance."""
+    half, full = _model(64, 16, 64, 1, 64, 64, "layernorm", torch.bfloat16, 5)
+    tokens = torch.randint(2, 72, (3, 20), device=DEV)
+    state, sb = {}, {}
+    with torch.no_grad():
+        half(tokens[:, :19], incremental_state=state)
+        full(tokens[:, :19], incremental_state=sb)
+        for part in state.values():
+            if entry in part:
+                t = part[entry]
+                part[entry] = t.repeat_interleave(2)[::2] if entry == "prev_count" else \
+                    torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)[1:].view(t.shape).copy_(t)
+        got, want = half(tokens[:, 19:], incremental_state=state)[0], full(tokens[:, 19:], incremental_state=sb)[0]
+    assert _rms(got, want) < TOL[torch.bfloat16]
