@@ -381,7 +381,7 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
         z, h, Nh = self.zdim, self.hdim, self.num_heads
         mine, mods = self._parameters, self._modules
         v_proj, mx_proj, h_proj, act = (mods[k] for k in ('v_proj', 'mx_proj', 'h_proj', 'move_act'))
-        return (ops.token_rows(x, normalised=True) and mask_bytes_ok(padding_mask)
+        return (ops.token_rows(x, normalised=True) and mask_bytes_ok(padding_mask, x)
                 and _plain(True, v_proj, mx_proj) and _plain(False, h_proj) and 'gamma' in mine and 'beta' in mine
                 and _unhooked((RMSNorm, nn.SiLU), act)
                 and ops._lib.load_host().uniform(

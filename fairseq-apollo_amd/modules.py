@@ -505,8 +505,9 @@ class TimestepNormFunc(torch.autograd.Function):
 timestep_norm = TimestepNormFunc.apply
 
 
-def mask_bytes_ok(mask: Optional[Tensor]) -> bool:
-    return mask is None or (mask.dtype in (torch.bool, torch.uint8) and mask.is_contiguous())
+def mask_bytes_ok(mask: Optional[Tensor], x: Tensor) -> bool:
+    """The one-token kernels take this padding mask of x [B, 1, D] (another shape is for the general path to refuse)."""
+    return mask is None or (mask.dtype in (torch.bool, torch.uint8) and mask.is_contiguous() and mask.shape == x.shape[:2])
 
 
 def mask_bytes(mask: Optional[Tensor]) -> Optional[Tensor]:
@@ -577,7 +578,7 @@ class TimestepNorm(nn.Module, IncrementalState):
             return out
         gamma, beta = self._affine()
         if incremental_state is not None and x.size(1) == 1 and self.num_groups is not None and x.is_cuda and \
-                x.is_contiguous() and mask_bytes_ok(padding_mask) and prev_count.dtype is torch.int64 and prev_count.is_contiguous():
+                x.is_contiguous() and mask_bytes_ok(padding_mask, x) and prev_count.dtype is torch.int64 and prev_count.is_contiguous():
             # one token per stream: no look-back over time, one wave per (stream, group)
             with ops._on_device(x.device):
                 out, count, mean, var = ops._lib.load_host().token_norm(

@@ -252,3 +252,13 @@ def test_token_with_state_in_other_storage(entry):
                     torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)[1:].view(t.shape).copy_(t)
         got, want = half(tokens[:, 19:], incremental_state=state)[0], full(tokens[:, 19:], incremental_state=sb)[0]
     assert _rms(got, want) < TOL[torch.bfloat16]
+
+
+def test_token_masks_of_other_shapes_are_refused():
+    """A padding mask is [B, 1] for one token, in the layer and in the norm alone."""
+    half, _ = _model(64, 16, 64, 1, 64, 64, "layernorm", torch.bfloat16, 5)
+    x = torch.randn(3, 1, 64, device=DEV, dtype=torch.bfloat16)
+    for mask in (torch.zeros(3, dtype=torch.bool, device=DEV), torch.zeros(1, 3, dtype=torch.bool, device=DEV)):
+        for module in (half.layers[0].mega_layer, half.final_norm):
+            with torch.no_grad(), pytest.raises(RuntimeError, match="padding_mask"):
+                module(x, mask, incremental_state={})
