@@ -529,6 +529,13 @@ void same_type(const Args& A, std::initializer_list<int> at, const Tensor& x) {
       throw std::runtime_error(std::string(A.who) + ": argument " + std::to_string(i) + " must be contiguous, of the activations' type and on their device");
 }
 
+// A gradient as the row kernels read it: of x's type, contiguous, on 16 bytes (autograd also hands out views that start
+// anywhere in a buffer, behind a concatenation for instance)
+Tensor rows16(const Tensor& t, const Tensor& x) {
+  Tensor r = t.to(x.scalar_type()).contiguous();
+  return (uintptr_t)r.data_ptr() % 16 ? r.clone() : r;
+}
+
 // a row norm's parameters hold one value per column: the kernels read (and in the backward pass write) that many
 void norm_width(const Tensor& x, const Tensor& w, const Tensor& b, const char* who) {
   for (const Tensor* p : {&w, &b})
@@ -623,8 +630,8 @@ PyObject* row_norm_forward(const Args& A) {
 // (dy, x, kind, weight | None, bias | None, eps, stream) -> (dx, dw, db)
 PyObject* row_norm_backward(const Args& A) {
   A.want(7);
-  same_type(A, {0, 1, 3, 4}, A.t(1));
-  auto [dx, dw, db] = row_norm_back(A.t(0), A.t(1), opt_t(A, 3), opt_t(A, 4), Tensor(), (int)A.i64(2), A.d(5), A.stream(6), A.who);
+  same_type(A, {1, 3, 4}, A.t(1));
+  auto [dx, dw, db] = row_norm_back(rows16(A.t(0), A.t(1)), A.t(1), opt_t(A, 3), opt_t(A, 4), Tensor(), (int)A.i64(2), A.d(5), A.stream(6), A.who);
   Tensor r[3] = {dx, dw, db};
   return tuple(r);
 }
@@ -649,7 +656,7 @@ PyObject* ffn_forward(const Args& A) {
 PyObject* ffn_backward(const Args& A) {
   A.want(12);
   const Tensor &x = A.t(1), &n = A.t(2), &pre = A.t(3), &h = A.t(4);
-  const Tensor dout = A.t(0).to(x.scalar_type()).contiguous();
+  const Tensor dout = rows16(A.t(0), x);
   same_type(A, {1, 2, 3, 4, 6, 7, 9, 10}, x);
   void* s = A.stream(11);
   A.shape(4, pre.sizes());
@@ -795,8 +802,7 @@ PyObject* mix_backward(const Args& A) {
   same_type(A, {3, 4, 5, 6, 7, 8, 9, 10, 11, 16}, xn);
   void* s = A.stream(18);
   const int dt = dtype_code(xn);
-  const Tensor dq = A.t(0).to(xn.scalar_type()).contiguous(), dk = A.t(1).to(xn.scalar_type()).contiguous();
-  const Tensor dv = A.t(2).to(xn.scalar_type()).contiguous();
+  const Tensor dq = rows16(A.t(0), xn), dk = rows16(A.t(1), xn), dv = rows16(A.t(2), xn);
   const int64_t D = xn.size(2), S = A.t(11).size(1), heads = A.i64(13), chunk = A.i64(14), T = xn.numel() / D;
   const int64_t W = base.size(1), es = xn.element_size(), E = vp.size(-1);
   if (dq.numel() != T * S || dk.numel() != T * S || dv.numel() != T * E || act.numel() != T * D || mx.numel() != T * D ||

@@ -1080,9 +1080,8 @@ class RowNormFunc(torch.autograd.Function):
             got = iter(torch.autograd.grad(row_norm_formula(x, ctx.kind, weight, bias, ctx.eps), ins, y_grad,
                                            create_graph=True))
             return (*[next(got) if t is not None and t.requires_grad else None for t in (x, weight, bias)], None, None)
-        g = y_grad.to(x.dtype).contiguous()
         with ops._on_device(x.device):
-            dx, dw, db = ops._lib.load_host().row_norm_backward(g, x.contiguous(), ctx.kind, weight, bias, ctx.eps,
+            dx, dw, db = ops._lib.load_host().row_norm_backward(y_grad, x.contiguous(), ctx.kind, weight, bias, ctx.eps,
                                                                 ops._stream(x.device))
         return dx, dw, db, None, None
 

@@ -220,3 +220,30 @@ def test_composites_of_replaced_forwards(change):
     for a, b in zip(got, want):
         b64 = b.double().cpu()
         _close(a.detach(), b64, torch.float32, 8 * (b64.abs() + b64.pow(2).mean().sqrt()))
+
+
+def _through_cat(y):
+    """y on the way to a concatenation behind one element: its gradient is a contiguous view that starts on no 16 bytes."""
+    return torch.cat([torch.zeros(1, dtype=y.dtype, device=y.device), y.flatten()])
+
+
+@pytest.mark.parametrize("what", ["layernorm", "rmsnorm", "feed-forward", "swiglu", "gated attention"])
+def test_gradients_off_16_bytes(what):
+    """The same gradients whether the incoming one starts on 16 bytes or not."""
+    torch.manual_seed(9)
+    module = {"layernorm": lambda: M.layers.LayerNorm(64), "rmsnorm": lambda: M.layers.RMSNorm(64),
+              "feed-forward": lambda: M.NormalizedFeedForwardNetwork(64, 96), "swiglu": lambda: M.SwiGLU(64, 96),
+              "gated attention": lambda: M.MovingAverageGatedAttention(64, 32, 128, 8, chunk_size=32, norm_num_groups=4)}[what]()
+    module = module.to(DEV).train()
+    x0 = torch.randn(2, 96, 64, device=DEV)
+    weight = torch.randn(2 * 96 * 64 + 1, device=DEV)
+    out = []
+    for off in (True, False):
+        module.zero_grad()
+        x = x0.clone().requires_grad_(True)
+        y = module(x)
+        y = y[0] if isinstance(y, tuple) else y
+        ((_through_cat(y) * weight).sum() if off else (y * weight[1:].view(y.shape)).sum()).backward()
+        out.append([x.grad] + [p.grad for p in module.parameters()])
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
