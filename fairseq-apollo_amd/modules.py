@@ -1162,8 +1162,8 @@ class SwiGLUBlockFunc(torch.autograd.Function):
 class MixInFunc(torch.autograd.Function):
     """From the layer's norm and moving average to the attention's operands
     (moving_average_gated_attention.py:313-328): v = silu(v_proj(xn)), base = mx_proj(act(mx)), q and k from base's
-    second slice.  `base` has one consumer, MixOutFunc, whose backward returns its gradient as one buffer with q's and
-    k's slice still open: this backward fills that slice in place."""
+    second slice.  `base` has one consumer, MixOutFunc, whose backward returns its gradient as one buffer with zeros in
+    q's and k's slice: this backward fills that slice in place."""
 
     @staticmethod
     def forward(ctx, xn, mx, v_weight, v_bias, mx_weight, mx_bias, gamma, beta, freqs, act_weight, act, eps, heads, chunk):

@@ -247,3 +247,23 @@ def test_gradients_off_16_bytes(what):
         out.append([x.grad] + [p.grad for p in module.parameters()])
     for a, b in zip(*out):
         assert torch.equal(a, b)
+
+
+def test_gated_attention_under_anomaly_detection():
+    """Every gradient that leaves a backward pass is written whole: with fresh memory filled with NaN, anomaly detection
+    finds none."""
+    torch.manual_seed(4)
+    layer = M.MovingAverageGatedAttention(64, 32, 128, 8, chunk_size=32, norm_num_groups=4).to(DEV).train()
+    x = torch.randn(2, 96, 64, device=DEV, requires_grad=True)
+    filled = torch.utils.deterministic.fill_uninitialized_memory
+    torch.use_deterministic_algorithms(True, warn_only=True)           # new tensors start as NaN
+    torch.utils.deterministic.fill_uninitialized_memory = True
+    try:
+        with torch.autograd.set_detect_anomaly(True):
+            y, _ = layer(x)
+            assert "MixOut" in type(y.grad_fn).__name__
+            y.square().sum().backward()
+    finally:
+        torch.use_deterministic_algorithms(False)
+        torch.utils.deterministic.fill_uninitialized_memory = filled
+    assert all(bool(t.grad.isfinite().all()) for t in (x, *layer.parameters()))
