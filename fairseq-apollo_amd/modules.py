@@ -1060,6 +1060,14 @@ def row_norm_covers(x: Tensor, *params) -> bool:
         all(p is None or p.shape == (D,) for p in params) and ops._lib.load_host().uniform(x, *params)
 
 
+def _through_formula(formula, inputs: tuple, grads) -> list:
+    """A composite's backward pass where a graph over it is asked for (create_graph): the gradients of `inputs` through
+    the formula in torch operations; None for those that want none."""
+    ins = [t for t in inputs if t is not None and t.requires_grad]
+    got = iter(torch.autograd.grad(formula(*inputs), ins, grads, create_graph=True, allow_unused=True))
+    return [next(got) if t is not None and t.requires_grad else None for t in inputs]
+
+
 class RowNormFunc(torch.autograd.Function):
     """RMSNorm / LayerNorm over the last axis with the affine weight stored as its offset from one: one pass each way
     (norm_layer/layer_norm.py:41-59, 85-111).  kind: ops.TOKEN_RMSNORM or ops.TOKEN_LAYERNORM."""
@@ -1075,11 +1083,9 @@ class RowNormFunc(torch.autograd.Function):
     @staticmethod
     def backward(ctx, y_grad):
         x, weight, bias = ctx.saved_tensors
-        if torch.is_grad_enabled():                    # a graph over the backward pass: the formula in torch operations
-            ins = [t for t in (x, weight, bias) if t is not None and t.requires_grad]
-            got = iter(torch.autograd.grad(row_norm_formula(x, ctx.kind, weight, bias, ctx.eps), ins, y_grad,
-                                           create_graph=True))
-            return (*[next(got) if t is not None and t.requires_grad else None for t in (x, weight, bias)], None, None)
+        if torch.is_grad_enabled():
+            return (*_through_formula(lambda x, w, b: row_norm_formula(x, ctx.kind, w, b, ctx.eps), (x, weight, bias), y_grad),
+                    None, None)
         with ops._on_device(x.device):
             dx, dw, db = ops._lib.load_host().row_norm_backward(y_grad, x.contiguous(), ctx.kind, weight, bias, ctx.eps,
                                                                 ops._stream(x.device))
@@ -1109,20 +1115,23 @@ class FeedForwardFunc(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, norm_weight, norm_bias, w1, b1, w2, kind, eps):
-        xd = x.detach().contiguous()
         with ops._on_device(x.device):
-            out, n, pre, h = ops._lib.load_host().ffn_forward(xd, kind, norm_weight, norm_bias, eps, w1, b1, w2,
-                                                              ops._stream(x.device))
-        ctx.save_for_backward(xd, n, pre, h, norm_weight, norm_bias, w1, w2)
-        ctx.kind, ctx.eps = kind, eps
+            out, n, pre, h = ops._lib.load_host().ffn_forward(x.detach().contiguous(), kind, norm_weight, norm_bias, eps, w1, b1,
+                                                              w2, ops._stream(x.device))
+        ctx.save_for_backward(x, n, pre, h, norm_weight, norm_bias, w1, w2)
+        ctx.kind, ctx.eps, ctx.bias = kind, eps, b1        # (the bias is read under create_graph only)
         return out
 
     @staticmethod
     def backward(ctx, y_grad):
         x, n, pre, h, norm_weight, norm_bias, w1, w2 = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            def formula(x, nw, nb, w1, b1, w2):
+                return x + F.linear(F.silu(F.linear(row_norm_formula(x, ctx.kind, nw, nb, ctx.eps), w1, b1)), w2)
+            return (*_through_formula(formula, (x, norm_weight, norm_bias, w1, ctx.bias, w2), y_grad), None, None)
         with ops._on_device(x.device):
             dx, dnw, dnb, dw1, db1, dw2 = ops._lib.load_host().ffn_backward(
-                y_grad, x, n, pre, h, ctx.kind, norm_weight, norm_bias, ctx.eps, w1, w2, ops._stream(x.device))
+                y_grad, x.contiguous(), n, pre, h, ctx.kind, norm_weight, norm_bias, ctx.eps, w1, w2, ops._stream(x.device))
         return dx, dnw, dnb, dw1, db1, dw2, None, None
 
 
@@ -1145,17 +1154,23 @@ class SwiGLUBlockFunc(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, residual, w1, w3, w2):
-        xd = x.detach().contiguous()
         with ops._on_device(x.device):
-            out, a, b, g = ops._lib.load_host().swiglu_forward(xd, residual, w1, w3, w2, ops._stream(x.device))
-        ctx.save_for_backward(xd, a, b, g, w1, w3, w2)
+            out, a, b, g = ops._lib.load_host().swiglu_forward(x.detach().contiguous(), residual, w1, w3, w2,
+                                                               ops._stream(x.device))
+        ctx.save_for_backward(x, a, b, g, w1, w3, w2)
         ctx.residual = residual is not None
         return out
 
     @staticmethod
     def backward(ctx, y_grad):
-        with ops._on_device(y_grad.device):
-            dx, dw1, dw3, dw2 = ops._lib.load_host().swiglu_backward(y_grad, *ctx.saved_tensors, ops._stream(y_grad.device))
+        x, a, b, g, w1, w3, w2 = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            dx, dw1, dw3, dw2 = _through_formula(lambda x, w1, w3, w2: F.linear(F.silu(F.linear(x, w1)) * F.linear(x, w3), w2),
+                                                 (x, w1, w3, w2), y_grad)
+        else:
+            with ops._on_device(y_grad.device):
+                dx, dw1, dw3, dw2 = ops._lib.load_host().swiglu_backward(y_grad, x.contiguous(), a, b, g, w1, w3, w2,
+                                                                         ops._stream(y_grad.device))
         return dx, y_grad if ctx.residual else None, dw1, dw3, dw2
 
 
@@ -1167,26 +1182,50 @@ class MixInFunc(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, xn, mx, v_weight, v_bias, mx_weight, mx_bias, gamma, beta, freqs, act_weight, act, eps, heads, chunk):
-        xd = xn.detach().contiguous()
-        stream = ops._stream(xn.device)
         with ops._on_device(xn.device):
             vp, v, mxt, a, base, q, k = ops._lib.load_host().mix_forward(
-                xd, mx.detach(), v_weight, v_bias, mx_weight, mx_bias, gamma, beta, freqs, heads, chunk, act, act_weight,
-                eps, stream)
-        ctx.save_for_backward(xd, vp, mxt, a, base, v_weight, mx_weight, gamma, freqs, act_weight)
+                xn.detach().contiguous(), mx.detach(), v_weight, v_bias, mx_weight, mx_bias, gamma, beta, freqs, heads, chunk,
+                act, act_weight, eps, ops._stream(xn.device))
+        # mx is a view of time-major memory: its transpose is what the native call read
+        ctx.save_for_backward(xn, mx, vp, a, base, v_weight, mx_weight, gamma, freqs, act_weight)
+        ctx.biases = v_bias, mx_bias, beta                 # (read under create_graph only)
         ctx.consts = heads, chunk, act
         ctx.eps = eps
         return v, base, q, k
 
     @staticmethod
     def backward(ctx, dv, dbase, dq, dk):
-        xn, vp, mx, a, base, v_weight, mx_weight, gamma, freqs, act_weight = ctx.saved_tensors
+        xn, mx, vp, a, base, v_weight, mx_weight, gamma, freqs, act_weight = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            v_bias, mx_bias, beta = ctx.biases
+            got = _through_formula(lambda *t: mix_in_formula(*t, freqs, *ctx.consts, ctx.eps),
+                                   (xn, mx, v_weight, v_bias, mx_weight, mx_bias, gamma, beta, act_weight), (dv, dbase, dq, dk))
+            return (*got[:8], None, got[8], None, None, None, None)
         SplitGrads.taken += 1                          # the four slices' gradients lie in one buffer
         with ops._on_device(xn.device):
             dxn, dmx, dvw, dvb, dmw, dmb, dgamma, dbeta, daw = ops._lib.load_host().mix_backward(
-                dq, dk, dv, dbase, xn, vp, mx, a, base, v_weight, mx_weight, gamma, freqs, *ctx.consts, act_weight, ctx.eps,
-                ops._stream(xn.device))
+                dq, dk, dv, dbase, xn.contiguous(), vp, mx.transpose(1, 2).contiguous(), a, base, v_weight, mx_weight, gamma,
+                freqs, *ctx.consts, act_weight, ctx.eps, ops._stream(xn.device))
         return dxn, dmx.transpose(1, 2), dvw, dvb, dmw, dmb, dgamma, dbeta, None, daw, None, None, None, None
+
+
+def mix_in_formula(xn, mx, v_weight, v_bias, mx_weight, mx_bias, gamma, beta, act_weight, freqs, heads, chunk, act, eps):
+    """MixInFunc in torch operations: (v [T, E], base [T, W], q [T, S], k [T, S]) of the T tokens of all rows."""
+    m = mx.transpose(1, 2)
+    a = row_norm_formula(m, act, act_weight, None, eps) if act == ops.TOKEN_RMSNORM else F.silu(m)
+    v = F.silu(F.linear(xn, v_weight, v_bias)).flatten(0, 1)
+    base = F.linear(a, mx_weight, mx_bias).flatten(0, 1)
+    S, D, T = gamma.shape[1], xn.shape[-1], base.shape[0]
+    z = F.normalize(base[:, D:D + S].float(), p=2, dim=-1, eps=1e-5)
+    pos = torch.arange(T, device=z.device, dtype=torch.float32) % chunk
+    angle = (pos[:, None] * freqs).repeat(1, heads)
+    cos, sin = angle.cos(), angle.sin()
+
+    def turned(i):
+        even, odd = (z * (gamma[i].float() + 1.0) + beta[i].float()).unflatten(-1, (S // 2, 2)).unbind(-1)
+        return torch.stack((even * cos - odd * sin, even * sin + odd * cos), -1).flatten(-2).to(base.dtype)
+
+    return v, base, turned(0), turned(1)
 
 
 class MixOutFunc(torch.autograd.Function):
@@ -1195,19 +1234,26 @@ class MixOutFunc(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, residual, base, attn, h_weight, S):
-        res, at = residual.detach().contiguous(), attn.detach().contiguous()
-        with ops._on_device(res.device):
-            out, gated, hp = ops._lib.load_host().mix_out_forward(res, base, at, h_weight, S, ops._stream(res.device))
-        ctx.save_for_backward(res, base, at, gated, hp, h_weight)
-        ctx.S, ctx.attn_shape = S, attn.shape
+        with ops._on_device(residual.device):
+            out, gated, hp = ops._lib.load_host().mix_out_forward(
+                residual.detach().contiguous(), base, attn.detach().contiguous(), h_weight, S, ops._stream(residual.device))
+        ctx.save_for_backward(residual, base, attn, gated, hp, h_weight)
+        ctx.S = S
         return out
 
     @staticmethod
     def backward(ctx, y_grad):
+        residual, base, attn, gated, hp, h_weight = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            def formula(residual, base, attn, h_weight):
+                D = residual.shape[-1]
+                u, _, r, hx = (t.view(*residual.shape[:-1], -1) for t in base.split([D, ctx.S, attn.shape[-1], D], -1))
+                return residual + torch.sigmoid(u) * (F.silu(hx + F.linear(attn * F.silu(r), h_weight)) - residual)
+            return (*_through_formula(formula, (residual, base, attn, h_weight), y_grad), None)
         with ops._on_device(y_grad.device):
-            dres, dbase, dattn, dhw = ops._lib.load_host().mix_out_backward(y_grad, *ctx.saved_tensors, ctx.S,
-                                                                            ops._stream(y_grad.device))
-        return dres, dbase, dattn.view(ctx.attn_shape), dhw, None
+            dres, dbase, dattn, dhw = ops._lib.load_host().mix_out_backward(
+                y_grad, residual.contiguous(), base, attn.contiguous(), gated, hp, h_weight, ctx.S, ops._stream(y_grad.device))
+        return dres, dbase, dattn.view(attn.shape), dhw, None
 
 
 class AttentionSoftmaxFunc(torch.autograd.Function):

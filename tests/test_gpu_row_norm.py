@@ -267,3 +267,81 @@ def test_gated_attention_under_anomaly_detection():
         torch.use_deterministic_algorithms(False)
         torch.utils.deterministic.fill_uninitialized_memory = filled
     assert all(bool(t.grad.isfinite().all()) for t in (x, *layer.parameters()))
+
+
+def _second_derivatives(call, formula, tensors):
+    """Gradients of sum((d loss / d inputs)^2) by both: `call` on the GPU in fp32, `formula` on the CPU in fp64."""
+    out = []
+    for f, t in ((call, [v.clone().requires_grad_(True) for v in tensors]),
+                 (formula, [v.double().cpu().requires_grad_(True) for v in tensors])):
+        y = f(*t)
+        y = y if isinstance(y, tuple) else (y,)
+        weights = [torch.linspace(-1, 1, v.numel(), dtype=v.dtype).view(v.shape).to(v.device) for v in y]
+        first = torch.autograd.grad(y, t, weights, create_graph=True)
+        second = torch.autograd.grad(sum(g.square().sum() for g in first), t, materialize_grads=True)
+        out.append((first, second))
+    for got, ref in zip(out[0][0] + out[0][1], out[1][0] + out[1][1]):
+        ref = ref.detach()
+        # sums of up to 66 x 100 products in fp32, twice in a row
+        _close(got.detach(), ref, torch.float32, 16 * (ref.abs() + ref.pow(2).mean().sqrt()))
+
+
+@pytest.mark.parametrize("kind", [M.ops.TOKEN_RMSNORM, M.ops.TOKEN_LAYERNORM])
+def test_second_derivatives_feed_forward(kind):
+    torch.manual_seed(6)
+    x, nw, w1, b1, w2 = (torch.randn(*s, device=DEV) * 0.5 for s in ((2, 33, 64), (64,), (96, 64), (96,), (64, 96)))
+    nb = torch.randn(64, device=DEV) if kind == M.ops.TOKEN_LAYERNORM else None
+    tensors = [x, nw, w1 * 0.2, b1, w2 * 0.2] + ([nb] if nb is not None else [])
+
+    def formula(x, nw, w1, b1, w2, nb=None):
+        c = x - x.mean(-1, keepdim=True) if nb is not None else x
+        n = c * torch.rsqrt(c.pow(2).mean(-1, keepdim=True) + 1e-5) * (nw + 1)
+        return x + F.linear(F.silu(F.linear(n if nb is None else n + nb, w1, b1)), w2)
+
+    _second_derivatives(lambda x, nw, w1, b1, w2, nb=None: M.modules.FeedForwardFunc.apply(x, nw, nb, w1, b1, w2, kind, 1e-5),
+                        formula, tensors)
+
+
+@pytest.mark.parametrize("residual", [False, True])
+def test_second_derivatives_swiglu(residual):
+    torch.manual_seed(7)
+    x, res, w1, w3, w2 = (torch.randn(*s, device=DEV) * 0.3 for s in ((2, 33, 64), (2, 33, 64), (96, 64), (96, 64), (64, 96)))
+
+    def formula(x, w1, w3, w2, res=None):
+        y = F.linear(F.silu(F.linear(x, w1)) * F.linear(x, w3), w2)
+        return y if res is None else y + res
+
+    _second_derivatives(lambda x, w1, w3, w2, res=None: M.modules.SwiGLUBlockFunc.apply(x, res, w1, w3, w2), formula,
+                        [x, w1, w3, w2] + ([res] if residual else []))
+
+
+@pytest.mark.parametrize("act,heads", [(M.ops.TOKEN_RMSNORM, 1), (M.ops.TOKEN_SILU, 2)])
+def test_second_derivatives_gated_attention(act, heads):
+    """The two halves of the gated attention around the attention itself (here: the sum of q, k and v columns)."""
+    torch.manual_seed(8)
+    B, L, C, D, S, E = 2, 12, 6, 32, 16, 24
+    W = 2 * D + S + E
+    shapes = ((B, L, D), (B, D, L), (E, D), (E,), (W, D), (W,), (2, S), (2, S), (B, L, D), (D, E))
+    tensors = [torch.randn(*s, device=DEV) * 0.3 for s in shapes]
+    if act == M.ops.TOKEN_RMSNORM:
+        tensors.append(torch.randn(D, device=DEV) * 0.3)
+    freqs = torch.rand(S // heads // 2, device=DEV)
+
+    def call(xn, mx, vw, vb, mw, mb, ga, be, res, hw, aw=None):
+        v, base, q, k = M.modules.MixInFunc.apply(xn, mx, vw, vb, mw, mb, ga, be, freqs, aw, act, 1e-5, heads, C)
+        attn = v.view(B, L, E) + (q * k).sum(-1).view(B, L, 1)
+        return M.modules.MixOutFunc.apply(res, base, attn, hw, S)
+
+    def formula(xn, mx, vw, vb, mw, mb, ga, be, res, hw, aw=None):
+        v, m = F.silu(F.linear(xn, vw, vb)), mx.transpose(1, 2)
+        m = F.silu(m) if aw is None else m * torch.rsqrt(m.pow(2).mean(-1, keepdim=True) + 1e-5) * (aw + 1)
+        u, z, r, hx = F.linear(m, mw, mb).split([D, S, E, D], -1)
+        z = F.normalize(z, p=2, dim=-1, eps=1e-5)
+        ang = (torch.arange(L, dtype=torch.float64) % C)[:, None] * freqs.double().cpu().repeat(heads)
+        turn = torch.polar(torch.ones_like(ang), ang)
+        q, k = (torch.view_as_real(torch.view_as_complex((z * (ga[i] + 1) + be[i]).reshape(B, L, -1, 2)) * turn).flatten(-2)
+                for i in (0, 1))
+        attn = v + (q * k).sum(-1, keepdim=True)
+        return res + torch.sigmoid(u) * (F.silu(hx + F.linear(attn * F.silu(r), hw)) - res)
+
+    _second_derivatives(call, formula, tensors)
