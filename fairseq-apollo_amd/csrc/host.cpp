@@ -265,15 +265,16 @@ PyObject* token_linear(const Args& A) {
   return wrap(out);
 }
 
-// (x [B, D], count, next count, mean, var, norm weight, norm bias, eps, p, q, gamma, complex, omega, h, groups, stream)
-//   -> (xn, y); count / mean / var / h are the step's own buffers, updated in place (next count takes the new count)
+// (x [B, D] in any shape, count, next count, mean, var, norm weight, norm bias, eps, p, q, gamma, complex, omega, h, groups,
+//  stream) -> (xn, y) in x's shape; count / mean / var / h are the step's own buffers, updated in place (next count takes the new count)
 PyObject* norm_ema_step(const Args& A) {
   A.want(16);
   Tensor x = A.t(0).detach().contiguous();
   const at::Device dev = x.device();
   const Tensor& p = A.t(8);
-  if (x.dim() != 2 || !x.is_cuda() || p.dim() != 2) throw std::runtime_error("norm_ema_step: x must be a [B, D] device tensor");
-  const int64_t B = x.size(0), D = x.size(1), N = p.size(1), G = A.i64(14);
+  if (!x.is_cuda() || p.dim() != 2) throw std::runtime_error("norm_ema_step: x must be a device tensor");
+  const int64_t B = A.t(1).numel(), D = p.size(0), N = p.size(1), G = A.i64(14);
+  if (x.numel() != B * D) throw std::runtime_error("norm_ema_step: x must hold [B, D] values, the streams' and channels' of the state");
   Tensor r[2] = {at::empty_like(x), at::empty_like(x)};
   float* mean = (float*)A.p(3, at::kFloat, B * G, dev);
   float* var = (float*)A.p(4, at::kFloat, B * G, dev);

@@ -1068,7 +1068,7 @@ class DecodeStep:
         self.h = torch.zeros(self.B, self.D, self.N, 2, dtype=torch.float32, device=self.dev)
 
     def __call__(self, x_t: torch.Tensor):
-        """x_t: [B, D] -> (xn_t, y_t), both [B, D]."""
+        """x_t: [B, D], or these values in another shape ([B, 1, D]) -> (xn_t, y_t) in the same shape."""
         with _on_device(self.dev):
             xn, y = _lib.load_host().norm_ema_step(x_t, self.count, self._count_next, self.mean, self.var, self.nw, self.nb,
                                                    self.eps, self.p, self.q, self.gamma, 1 if self.is_complex else 0,

@@ -195,3 +195,19 @@ def test_multi_token_launch_other_coefficient_shapes_take_single_steps():
                                  ptr(a._count_next), ptr(a.mean), ptr(a.var), ptr(a.nw), ptr(a.nb), 1e-5, ptr(a.p), ptr(a.q),
                                  ptr(a.gamma), 1, ptr(a.omega), ptr(a.h), ptr(a.h), B, D, G, N, None)
     assert rc == -2 and b"ndim" in lib.mega_last_error()
+
+
+def test_step_takes_its_values_in_any_shape():
+    """[B, 1, D] is the token of B streams as [B, D] is, results in the same shape; another number of values is refused."""
+    B, D, N, G = 3, 96, 16, 4
+    rng, p, q, g, om, nw, nb = _setup(B, D, N, G, 43)
+    x = dev(rng.normal(size=(2, B, D)))
+    a, b = (M.ops.DecodeStep(dev(nw), dev(nb), G, 1e-5, dev(p), dev(q), dev(g), dev(om), B) for _ in range(2))
+    for t in range(2):
+        want, got = a(x[t]), b(x[t].view(B, 1, D))
+        for u, v in zip(want, got):
+            assert v.shape == (B, 1, D) and torch.equal(u, v.view(B, D))
+    for bad in (x[0, :2], x[0, :, :95], x):
+        with pytest.raises(RuntimeError, match=r"\[B, D\] values"):
+            a(bad)
+    assert torch.equal(a.state, b.state) and a.count.tolist() == [2] * B
