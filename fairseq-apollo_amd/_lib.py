@@ -64,7 +64,6 @@ SIGNATURES = {
                                                 _i64, _p, _p, _p, _p, _p, _p, _sz, _p]),
     "mega_norm_token": (_int, [_p, _p, _int, _p, _p, _p, _p, _p, _p, _p, _p, _p, C.c_double, _i64, _i64, _i64, _p]),
     "mega_token_linear": (_int, [_p, _int, _i64, _p]),
-    "mega_token_embed": (_int, [_p, _p, _int, C.c_double, _i64, _i64, _i64, _i64, _p, _p, _p]),
     "mega_token_attention_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64, _i64]),
     "mega_token_gated_attention": (_int, [_p, _p]),
     "mega_norm_ema_fwd_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64]),

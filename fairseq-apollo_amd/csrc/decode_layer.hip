@@ -424,25 +424,6 @@ __global__ __launch_bounds__(256) void token_combine_kernel(const float* __restr
   }
 }
 
-// x[b] = scale embed[token[b]], mask[b] = token[b] == pad
-template <typename T>
-__global__ __launch_bounds__(256) void token_embed_kernel(const int64_t* __restrict__ tok, const T* __restrict__ emb,
-                                                          float scale, int64_t pad, int64_t vocab, int D,
-                                                          T* __restrict__ x, uint8_t* __restrict__ mask) {
-  const int b = blockIdx.x;
-  const int64_t t = tok[b];
-  const bool in = t >= 0 && t < vocab;            // an index outside the table reads nothing (NaN, as a sign)
-  const T* row = emb + (in ? t : 0) * (int64_t)D;
-  for (int c = threadIdx.x * 8; c < D; c += 256 * 8) {
-    const Vec<T, 8> v = *(const Vec<T, 8>*)(row + c);
-    Vec<T, 8> o;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) o.v[e] = from_float<T>(in ? to_float(v.v[e]) * scale : __builtin_nanf(""));
-    *(Vec<T, 8>*)(x + (size_t)b * D + c) = o;
-  }
-  if (threadIdx.x == 0 && mask) mask[b] = t == pad ? 1 : 0;
-}
-
 int check_linear(const MegaTokenLinear& p, int64_t B, const char* who) {
   MEGA_REQUIRE(p.N > 0 && p.K > 0 && p.K % 32 == 0 && p.N < (int64_t)1 << 26 && p.K <= 65536, MEGA_ERR_UNSUPPORTED,
                "%s: N=%ld, K=%ld (K must be a multiple of 32)", who, (long)p.N, (long)p.K);
@@ -545,24 +526,6 @@ extern "C" int mega_token_linear(const MegaTokenLinear* p, int dtype, int64_t B,
   MEGA_REQUIRE(p && B >= 0 && B <= 64, MEGA_ERR_ARG, "token_linear: at most 64 rows (B=%ld)", (long)B);
   if (B == 0) return MEGA_OK;
   return linear_dispatch(*p, nullptr, dtype, B, (hipStream_t)stream);
-}
-
-extern "C" int mega_token_embed(const int64_t* tokens, const void* table, int dtype, double scale, int64_t pad,
-                                int64_t vocab, int64_t B, int64_t D, void* x, uint8_t* mask, void* stream) {
-  MEGA_REQUIRE(dtype == MEGA_BF16 || dtype == MEGA_F16, MEGA_ERR_UNSUPPORTED, "token_embed: 16-bit activations only");
-  MEGA_REQUIRE(B >= 0 && B < (int64_t)1 << 31 && D > 0 && D % 8 == 0 && vocab > 0, MEGA_ERR_ARG,
-               "token_embed: bad shape B=%ld D=%ld vocab=%ld", (long)B, (long)D, (long)vocab);
-  if (B == 0) return MEGA_OK;
-  MEGA_REQUIRE(tokens && table && x && ((uintptr_t)table % 16) == 0 && ((uintptr_t)x % 16) == 0, MEGA_ERR_ARG,
-               "token_embed: null or unaligned pointer");
-  if (dtype == MEGA_BF16)
-    hipLaunchKernelGGL(token_embed_kernel<bf16_t>, dim3((unsigned)B), dim3(256), 0, (hipStream_t)stream, tokens,
-                       (const bf16_t*)table, (float)scale, pad, vocab, (int)D, (bf16_t*)x, mask);
-  else
-    hipLaunchKernelGGL(token_embed_kernel<f16_t>, dim3((unsigned)B), dim3(256), 0, (hipStream_t)stream, tokens,
-                       (const f16_t*)table, (float)scale, pad, vocab, (int)D, (f16_t*)x, mask);
-  MEGA_CHECK_LAUNCH("token_embed");
-  return MEGA_OK;
 }
 
 extern "C" size_t mega_token_attention_workspace_bytes(int64_t B, int64_t n, int64_t D, int64_t S, int64_t hidden,

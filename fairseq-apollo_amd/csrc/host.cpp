@@ -215,18 +215,14 @@ PyObject* token_ffn(const Args& A) {
   return wrap(out[0]);
 }
 
-// (tokens [B, 1], table [V, D], scale, pad, stream) -> (x [B, 1, D], mask [B] bytes)
+// (tokens [B, 1], table [V, D], scale | None, pad | None) -> (x [B, 1, D], mask [B, 1] bool | None): torch's own lookup, which
+// knows what to do with an index outside the table
 PyObject* token_embed(const Args& A) {
-  A.want(5);
-  const Tensor &tok = A.t(0), &tab = A.t(1);
-  if (tok.scalar_type() != at::kLong || !tok.is_contiguous() || tok.device() != tab.device() || !tab.is_cuda() ||
-      tab.dim() != 2 || !tab.is_contiguous())
-    throw std::runtime_error("token_embed: tokens [B, 1] int64 and a contiguous [V, D] table on one device");
-  const int64_t B = tok.numel(), D = tab.size(1);
-  Tensor r[2] = {at::empty({B, 1, D}, tab.options()), empty({B}, tab, at::kByte)};
-  check(mega_token_embed((const int64_t*)tok.data_ptr(), tab.data_ptr(), dtype_code(tab), A.d(2), A.i64(3), tab.size(0), B, D,
-                         r[0].data_ptr(), (uint8_t*)r[1].data_ptr(), A.stream(4)),
-        A.who);
+  A.want(4);
+  const Tensor& tok = A.t(0);
+  Tensor r[2] = {at::embedding(A.t(1), tok), Tensor()};
+  if (!A.none(2)) r[0].mul_(A.d(2));
+  if (!A.none(3)) r[1] = tok.eq(A.i64(3));
   return tuple(r);
 }
 

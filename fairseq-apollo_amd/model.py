@@ -118,19 +118,12 @@ class MegaDecoderNoCrossAttn(nn.Module):
             return False
         w = embed.weight
         return (embed.max_norm is None and not torch.is_grad_enabled() and w.is_cuda and w.dtype in (torch.bfloat16, torch.float16)
-                and w.is_contiguous() and w.shape[1] % 8 == 0 and tokens.dtype is torch.int64 and tokens.is_contiguous()
                 and tokens.device == w.device and not (self.training and self.embedding_dropout.p > 0))
 
     def _token_features(self, tokens: Tensor, incremental_state):
         """extract_features for one new token per stream: which streams are padded stays on the device (asking the
         host to look would make it wait for everything enqueued before), the layers take the mask as it is."""
-        dev = tokens.device
-        pad = -1 if self.padding_idx is None else self.padding_idx
-        with ops._on_device(dev):
-            x, mask = ops._lib.load_host().token_embed(tokens, self.embed_tokens.weight,
-                                                       1.0 if self.embed_scale is None else self.embed_scale, pad,
-                                                       ops._stream(dev))
-        mask = None if self.padding_idx is None else mask.view(-1, 1)
+        x, mask = ops._lib.load_host().token_embed(tokens, self.embed_tokens.weight, self.embed_scale, self.padding_idx)
         inner_states: List[Tensor] = [x]
         for layer in self.layers:
             x, _, _ = layer(x, incremental_state=incremental_state, decoder_padding_mask=mask)
@@ -139,7 +132,7 @@ class MegaDecoderNoCrossAttn(nn.Module):
         if not isinstance(self.pre_logits, nn.Identity):
             x = self.pre_logits(x)
             if mask is not None:
-                x = x * (mask == 0).to(x.dtype).unsqueeze(-1)
+                x = x * (~mask).to(x.dtype).unsqueeze(-1)
         return x, {"inner_states": inner_states}
 
     def reorder_incremental_state(self, incremental_state, new_order: Tensor) -> None:

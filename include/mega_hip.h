@@ -325,10 +325,6 @@ typedef struct {
 
 int mega_token_linear(const MegaTokenLinear* p, int dtype, int64_t B, void* stream);
 
-/* x[b] = scale table[tokens[b]], mask[b] = tokens[b] == pad (mask may be NULL); an index outside the table gives NaN */
-int mega_token_embed(const int64_t* tokens, const void* table, int dtype, double scale, int64_t pad, int64_t vocab,
-                     int64_t B, int64_t D, void* x, uint8_t* mask, void* stream);
-
 /* The gated attention of one new token behind `context` cached ones of the current chunk (softmax, rotary). */
 typedef struct {
   int64_t dtype, B, D, S, hidden, heads, groups, states, context;

@@ -262,3 +262,14 @@ def test_token_masks_of_other_shapes_are_refused():
         for module in (half.layers[0].mega_layer, half.final_norm):
             with torch.no_grad(), pytest.raises(RuntimeError, match="padding_mask"):
                 module(x, mask, incremental_state={})
+
+
+def test_layers_see_the_general_mask():
+    """Layers of a one-token call get the padding mask they get otherwise: [B, 1], bool."""
+    half, _ = _model(64, 16, 64, 1, 64, 64, "layernorm", torch.bfloat16, 5)
+    seen = []
+    half.layers[0].register_forward_pre_hook(lambda m, a, kw: seen.append(kw["decoder_padding_mask"]), with_kwargs=True)
+    tokens = torch.tensor([[3], [1]], device=DEV)
+    with torch.no_grad():
+        half(tokens, incremental_state={})
+    assert len(seen) == 1 and seen[0].dtype == torch.bool and torch.equal(seen[0], tokens.eq(1))

@@ -79,3 +79,18 @@ def test_norm_widths():
     assert not M.modules.norm_width_ok(M.layers.LayerNorm(8, elementwise_affine=False), 16)
     with pytest.raises(RuntimeError):
         M.layers.LayerNorm(8, elementwise_affine=False)(torch.zeros(2, 16))
+
+
+@pytest.mark.parametrize("scale,pad", [(8.0, 1), (None, None)])
+def test_token_embedding(scale, pad):
+    """The one-token step's lookup is torch's: the scaled rows and the mask that the general path forms, and an index
+    outside the table is refused as torch refuses it."""
+    table = torch.randn(7, 8, dtype=torch.bfloat16)
+    tokens = torch.tensor([[3], [1], [6]])
+    x, mask = H.token_embed(tokens, table, scale, pad)
+    want = torch.nn.functional.embedding(tokens, table)
+    assert torch.equal(x, want if scale is None else scale * want)
+    assert mask is None if pad is None else torch.equal(mask, tokens.eq(pad))
+    for bad in (7, -1):
+        with pytest.raises(RuntimeError):
+            H.token_embed(torch.tensor([[bad]]), table, scale, pad)
