@@ -861,6 +861,42 @@ PyObject* tensor_versions(const Args& A) {
   return PyBytes_FromStringAndSize((const char*)buf, (Py_ssize_t)(n * 8));
 }
 
+// What the composites' gates ask of modules, (kinds, hooks on every module, bias, module, ...) -> bool: each is of exactly
+// one of these types with its class's own call, nobody looking at inputs or outputs; `bias` not None: and holds a weight
+// parameter, and a bias parameter or none.  Asked seven times per layer and token: one module 0.52 us, two 0.69, where the
+// same questions in Python take 0.70 and 0.97.
+PyObject* plain_modules(const Args& A) {
+  static PyObject *const forward = PyUnicode_InternFromString("forward"), *const parameters = PyUnicode_InternFromString("_parameters"),
+                  *const weight = PyUnicode_InternFromString("weight"), *const bias = PyUnicode_InternFromString("bias"),
+                  *const hooks[] = {PyUnicode_InternFromString("_forward_hooks"), PyUnicode_InternFromString("_forward_pre_hooks"),
+                                    PyUnicode_InternFromString("_backward_hooks"), PyUnicode_InternFromString("_backward_pre_hooks")};
+  if (A.n < 4 || !PyTuple_Check(A.a[0]) || !PyTuple_Check(A.a[1])) throw std::runtime_error("plain_modules: kinds, hooks, bias, modules");
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(A.a[1]); ++i)
+    if (PyObject_IsTrue(PyTuple_GET_ITEM(A.a[1], i))) return PyBool_FromLong(false);
+  auto absent = [](PyObject* v) { return v == nullptr || v == Py_None; };
+  for (Py_ssize_t k = 3; k < A.n; ++k) {
+    PyObject* m = A.a[k];
+    bool known = false;
+    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(A.a[0]); ++i) known = known || (PyObject*)Py_TYPE(m) == PyTuple_GET_ITEM(A.a[0], i);
+    if (!known) return PyBool_FromLong(false);
+    PyObject* d = PyObject_GenericGetDict(m, nullptr);
+    if (!d) return nullptr;
+    bool ok = !PyDict_GetItem(d, forward);
+    for (PyObject* h : hooks) {
+      PyObject* v = PyDict_GetItem(d, h);
+      ok = ok && (!v || !PyObject_IsTrue(v));
+    }
+    if (ok && !A.none(2)) {
+      PyObject* p = PyDict_GetItem(d, parameters);
+      PyObject* b = p && PyDict_Check(p) ? PyDict_GetItem(p, bias) : nullptr;
+      ok = p && PyDict_Check(p) && !absent(PyDict_GetItem(p, weight)) && (A.a[2] == Py_True ? !absent(b) : b == Py_None);
+    }
+    Py_DECREF(d);
+    if (!ok) return PyBool_FromLong(false);
+  }
+  return PyBool_FromLong(true);
+}
+
 PyObject* guarded(PyObject* (*f)(const Args&), const Args& args) {
   try {
     c10::AutoGradMode no_graph(false);
@@ -884,6 +920,7 @@ PyMethodDef methods[] = {MEGA_ENTRY(token_gated_attention), MEGA_ENTRY(token_ffn
                          MEGA_ENTRY(ffn_backward),          MEGA_ENTRY(swiglu_forward), MEGA_ENTRY(swiglu_backward),
                          MEGA_ENTRY(mix_forward),           MEGA_ENTRY(mix_out_forward), MEGA_ENTRY(mix_out_backward),
                          MEGA_ENTRY(mix_backward),          MEGA_ENTRY(uniform),    MEGA_ENTRY(trainable),
+                         MEGA_ENTRY(plain_modules),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "mega_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

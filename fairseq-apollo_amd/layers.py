@@ -143,29 +143,35 @@ class NormalizedFeedForwardNetwork(nn.Module):
 
     def _one_operator(self, x: Tensor) -> bool:
         """A training call the composite operator takes (no layer scale, no active dropout, whole 16-byte rows)."""
+        if not (x.is_cuda and torch.is_grad_enabled()):
+            return False
         norm, fc1, fc2 = self.norm, self.fc1, self.fc2
         vec = 16 // x.element_size()
-        return (torch.is_grad_enabled() and _plain(True, fc1) and _plain(False, fc2) and _unhooked((RMSNorm, LayerNorm), norm)
+        return (_plain(True, fc1) and _plain(False, fc2) and _unhooked((RMSNorm, LayerNorm), norm)
                 and self.layerscale_weight is None and x.shape[-1] % vec == 0 and x.shape[-1] <= 2048
                 and self.hidden_dim % vec == 0 and norm_width_ok(norm, x.shape[-1])
                 and not (self.training and (self.dropout_p > 0 or self.hidden_dropout_p > 0))
                 and one_graph(x, norm.weight, getattr(norm, 'bias', None), fc1.weight, fc1.bias, fc2.weight))
 
     def _few_rows_cover(self, x: Tensor) -> bool:
-        norm, fc1, fc2 = self.norm, self.fc1, self.fc2
+        mods = self._modules
+        norm, fc1, fc2 = mods['norm'], mods['fc1'], mods['fc2']
         return (self.hidden_dim % 32 == 0 and _plain(True, fc1) and _plain(False, fc2) and _unhooked((RMSNorm, LayerNorm), norm)
                 and norm_width_ok(norm, x.shape[-1]) and not (self.training and self.dropout_p > 0)
-                and ops._lib.load_host().uniform(x, norm.weight, getattr(norm, 'bias', None), fc1.weight, fc1.bias, fc2.weight,
-                                                 self.layerscale_weight))
+                and 'weight' in norm._parameters and 'layerscale_weight' in self._parameters
+                and ops._lib.load_host().uniform(x, *norm._parameters.values(), fc1._parameters['weight'], fc1._parameters['bias'],
+                                                 fc2._parameters['weight'], self._parameters['layerscale_weight']))
 
     def _few_rows(self, x: Tensor) -> Tensor:
         """The block on one token per stream: two launches (norm, first projection and activation; second projection,
         layer scale and residual)."""
-        rms = isinstance(self.norm, RMSNorm)
+        mods = self._modules                               # (attribute by attribute: 0.25 us each through nn.Module)
+        norm, first, second = mods['norm'], mods['fc1']._parameters, mods['fc2']._parameters
+        affine = norm._parameters
         with ops._on_device(x.device):
             return ops._lib.load_host().token_ffn(
-                x, ops.TOKEN_RMSNORM if rms else ops.TOKEN_LAYERNORM, self.norm.weight, None if rms else self.norm.bias,
-                self.norm.eps, self.fc1.weight, self.fc1.bias, self.fc2.weight, self.layerscale_weight,
+                x, ops.TOKEN_RMSNORM if isinstance(norm, RMSNorm) else ops.TOKEN_LAYERNORM, affine['weight'], affine.get('bias'),
+                norm.eps, first['weight'], first['bias'], second['weight'], self._parameters['layerscale_weight'],
                 ops._stream(x.device))
 
     def extra_repr(self) -> str:
@@ -573,7 +579,7 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
         vec = 16 // xn.element_size()
         act = self.move_act
         rms = isinstance(act, RMSNorm)
-        return (torch.is_grad_enabled() and _plain(True, self.v_proj, self.mx_proj) and _plain(False, self.h_proj)
+        return (xn.is_cuda and torch.is_grad_enabled() and _plain(True, self.v_proj, self.mx_proj) and _plain(False, self.h_proj)
                 and _unhooked((RMSNorm, nn.SiLU), act) and mx.dtype == xn.dtype and residual.dtype == xn.dtype
                 and residual.data_ptr() % 16 == 0
                 and self.embed_dim % vec == 0 and self.zdim % vec == 0 and self.hdim % vec == 0 and self.zdim <= 128 * vec

@@ -114,10 +114,10 @@ class MegaDecoderNoCrossAttn(nn.Module):
 
     def _token_covers(self, tokens: Tensor) -> bool:
         embed = self.embed_tokens
-        if not _unhooked((nn.Embedding,), embed):
+        if not tokens.is_cuda or torch.is_grad_enabled() or not _unhooked((nn.Embedding,), embed):
             return False
         w = embed.weight
-        return (embed.max_norm is None and not torch.is_grad_enabled() and w.is_cuda and w.dtype in (torch.bfloat16, torch.float16)
+        return (embed.max_norm is None and w.dtype in (torch.bfloat16, torch.float16)
                 and tokens.device == w.device and not (self.training and self.embedding_dropout.p > 0))
 
     def _token_features(self, tokens: Tensor, incremental_state):

@@ -1009,34 +1009,22 @@ def linear(lin: nn.Linear, x: Tensor) -> Tensor:
     return lin(x)
 
 
-_EVERY_MODULE = [getattr(nn.modules.module, f'_global_{kind}_hooks') for kind in
-                 ('forward', 'forward_pre', 'backward', 'backward_pre')]
+_EVERY_MODULE = tuple(getattr(nn.modules.module, f'_global_{kind}_hooks') for kind in
+                      ('forward', 'forward_pre', 'backward', 'backward_pre'))
+_LINEAR = (nn.Linear,)
 
 
 def _unhooked(kinds: tuple, *mods) -> bool:
     """Modules of exactly these types whose call is their class's own, nobody looking at their inputs or outputs (hooks of
     their own or on every module, a `forward` replaced on the instance): what reads their parameters directly may stand
     in for the calls."""
-    for hooks in _EVERY_MODULE:
-        if hooks:
-            return False
-    for m in mods:
-        if type(m) not in kinds or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks \
-                or 'forward' in m.__dict__:
-            return False
-    return True
+    return ops._lib.load_host().plain_modules(kinds, _EVERY_MODULE, None, *mods)
 
 
 def _plain(bias: bool, *layers) -> bool:
     """Linear layers as torch defines them, _unhooked, their weights parameters; `bias`: all of them with one, or all without.
     (A composite reads the biases that its formula has and no others.)"""
-    if not _unhooked((nn.Linear,), *layers):
-        return False
-    for m in layers:
-        p = m._parameters
-        if p.get('weight') is None or (p.get('bias') is None if bias else p.get('bias', p) is not None):
-            return False
-    return True
+    return ops._lib.load_host().plain_modules(_LINEAR, _EVERY_MODULE, bias, *layers)
 
 
 def one_graph(x: Tensor, *params) -> bool:
@@ -1389,7 +1377,7 @@ class SwiGLU(nn.Module):
         """W2 (silu(W1 x) * W3 x) (+ residual, which then enters the last product as its accumulator start: no
         separate addition pass over the activations; consume_residual: see linear_residual)."""
         w1, w3, w2 = self.w1, self.w3, self.w2
-        if torch.is_grad_enabled() and _plain(False, w1, w3, w2) and one_graph(x, w1.weight, w3.weight, w2.weight) and \
+        if x.is_cuda and torch.is_grad_enabled() and _plain(False, w1, w3, w2) and one_graph(x, w1.weight, w3.weight, w2.weight) and \
                 (residual is None or (residual.dtype == x.dtype and residual.is_contiguous()
                                                              and residual.device == x.device
                                                              and residual.shape[:-1] == x.shape[:-1]
