@@ -157,6 +157,11 @@ def load() -> C.CDLL:
 _host = None
 
 
+def host_built() -> bool:
+    """The extension of native host code is loaded or there to be loaded."""
+    return _host is not None or (os.path.exists(HOST_PATH) and os.path.exists(LIB_PATH))
+
+
 def load_host():
     """The extension of native host code (csrc/host.cpp), loaded once; raise if it has not been built."""
     global _host

@@ -844,21 +844,20 @@ PyObject* mix_backward(const Args& A) {
 
 // (dict, ...) -> bytes: storage address and in-place version of every tensor in the dictionaries' values, in order
 PyObject* tensor_versions(const Args& A) {
-  int64_t buf[128];
-  size_t n = 0;
+  std::vector<int64_t> buf;
   for (int i = 0; i < A.n; ++i) {
     if (!PyDict_Check(A.a[i])) throw std::runtime_error("tensor_versions: dictionaries expected");
     PyObject *key, *value;
     Py_ssize_t pos = 0;
     while (PyDict_Next(A.a[i], &pos, &key, &value)) {
       if (value == Py_None) continue;
-      if (!THPVariable_Check(value) || n + 2 > sizeof(buf) / sizeof(buf[0])) throw std::runtime_error("tensor_versions: up to 64 tensors");
+      if (!THPVariable_Check(value)) throw std::runtime_error("tensor_versions: tensors expected");
       const Tensor& t = THPVariable_Unpack(value);
-      buf[n++] = (int64_t)(uintptr_t)t.data_ptr();
-      buf[n++] = (int64_t)t._version();
+      buf.push_back((int64_t)(uintptr_t)t.data_ptr());
+      buf.push_back((int64_t)t._version());
     }
   }
-  return PyBytes_FromStringAndSize((const char*)buf, (Py_ssize_t)(n * 8));
+  return PyBytes_FromStringAndSize((const char*)buf.data(), (Py_ssize_t)(buf.size() * 8));
 }
 
 // What the composites' gates ask of modules, (kinds, hooks on every module, bias, module, ...) -> bool: each is of exactly

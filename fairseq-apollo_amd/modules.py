@@ -91,7 +91,7 @@ def _training_call(module: nn.Module, *tensors) -> bool:
                                         or any(p.requires_grad for p in module.parameters()))
 
 
-def _tensor_versions(*modules: nn.Module) -> bytes:
+def _tensor_versions(*modules: nn.Module):
     """Storage address and in-place version of the modules' own parameters and buffers.  An eval-mode cache
     derived from them is stale once this tuple changes: load_state_dict copies into the parameters, an
     optimiser step or an in-place edit under no_grad bumps the version, `.to()` moves the storage.  (The
@@ -103,6 +103,9 @@ def _tensor_versions(*modules: nn.Module) -> bytes:
     utilities do) changes neither the address nor the version counter of `p`, so it is not seen here; after such an
     edit call `module.train(); module.eval()` (every mode switch drops the caches) or edit under `torch.no_grad()`
     through the parameter itself."""
+    if not ops._lib.host_built():                      # modules on the CPU need no library
+        return tuple((t.data_ptr(), t._version) for m in modules
+                     for t in (*m._parameters.values(), *m._buffers.values()) if t is not None)
     return ops._lib.load_host().tensor_versions(*[d for m in modules for d in (m._parameters, m._buffers)])
 
 

@@ -94,3 +94,28 @@ def test_token_embedding(scale, pad):
     for bad in (7, -1):
         with pytest.raises(RuntimeError):
             H.token_embed(torch.tensor([[bad]]), table, scale, pad)
+
+
+@pytest.mark.parametrize("native", [True, False])
+def test_tensor_versions(native, monkeypatch):
+    """The key of the eval-mode caches: any number of tensors, with the native library and (modules on the CPU) without;
+    an edit in place and another storage change it."""
+    if not native:
+        monkeypatch.setattr(M._lib, "_host", None)
+        monkeypatch.setattr(M._lib, "HOST_PATH", M._lib.HOST_PATH + ".none")
+    m = torch.nn.Module()
+    for i in range(80):
+        m.register_parameter(f"p{i}", torch.nn.Parameter(torch.zeros(2)) if i != 40 else None)
+    keys = [M.modules._tensor_versions(m)]
+    assert M.modules._tensor_versions(m) == keys[0]
+    with torch.no_grad():
+        m.p79.add_(1)
+    keys.append(M.modules._tensor_versions(m))
+    m.p0.data = torch.zeros(2)
+    keys.append(M.modules._tensor_versions(m))
+    assert len(set(keys)) == 3
+    layer = M.MultiHeadComplexEMA(8, ndim=4).eval()
+    p, q, g = layer.coeffs()
+    with torch.no_grad():
+        layer.alpha.add_(1.0)
+    assert not torch.equal(layer.coeffs()[0], p)
