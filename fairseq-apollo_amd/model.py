@@ -74,9 +74,10 @@ class MegaDecoderNoCrossAttn(nn.Module):
     def output_layer(self, features: Tensor) -> Tensor:
         """Project features to the vocabulary (mega_lm.py:379-385)."""
         proj = self.output_projection
-        if not torch.is_grad_enabled() and ops.token_rows(features) and _plain(False, proj) and \
-                ops._lib.load_host().uniform(features, proj.weight):
-            return ops.token_linear(features, proj.weight)
+        if not torch.is_grad_enabled() and ops.token_rows(features) and _plain(False, proj):
+            w = proj.weight
+            if ops.token_linear_pays(features.size(0), *w.shape) and ops._lib.load_host().uniform(features, w):
+                return ops.token_linear(features, w)
         return proj(features)
 
     def max_positions(self) -> int:

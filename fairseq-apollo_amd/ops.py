@@ -167,6 +167,20 @@ def token_rows(x: torch.Tensor, normalised: bool = False) -> bool:
         (not normalised or B * (2 * K + 16) <= _TOKEN_LDS)
 
 
+def token_linear_pays(rows: int, N: int, K: int) -> bool:
+    """The one-token projection of `rows` tokens onto N columns is the faster one.  Each of its workgroups reads all rows
+    again for 16 columns and owns them alone, so it falls behind the library's product where rows and columns are both
+    many.  One call in bf16, us, here / the library (whose call takes 19 us of host time at least; device time alone in
+    brackets):
+        1 row    264 x 1024 4.8 / 19.3 (3.4 / 4.5)   16000 x 1024 8.8 / 19.2 (9.3 / 10.7)   50264 x 2048 38.7 / 50.6
+        16 rows  8192 x 2048 10.6 / 19.4 (11.0 / 9.3)  32000 x 512 12.1 / 19.1 (12.4 / 11.0)  50264 x 1024 28.5 / 21.5
+        32 rows  8192 x 1024 9.8 / 19.4 (10.1 / 8.8)  16000 x 512 11.7 / 19.3 (12.1 / 7.7)  32000 x 1024 34.9 / 23.9
+        64 rows  2048 x 2048 11.4 / 19.4 (11.9 / 9.1)  8192 x 512 9.2 / 19.0 (9.5 / 7.6)  32000 x 1024 50.9 / 24.7
+    The limits keep every measured call below the library's and its device time at most 6 us above; columns shorter than 512
+    count as that many (a workgroup costs about as much)."""
+    return (rows <= 8 and K >= 2048) or N * max(K, 512) <= (1 << 24 if rows <= 16 else 1 << 23 if rows <= 32 else 1 << 22)
+
+
 def token_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """F.linear of few rows x [rows, 1, K] (token_rows(x) holds)."""
     with _on_device(x.device):

@@ -273,3 +273,19 @@ def test_layers_see_the_general_mask():
     with torch.no_grad():
         half(tokens, incremental_state={})
     assert len(seen) == 1 and seen[0].dtype == torch.bool and torch.equal(seen[0], tokens.eq(1))
+
+
+# around the limits of the one-token projection: the same columns for few and for many rows
+@pytest.mark.parametrize("rows,vocab,native", [(16, 8192, True), (17, 8192, False), (8, 16500, True), (9, 16500, False)])
+def test_output_projection_of_many_columns(rows, vocab, native):
+    """The route follows rows x columns; both routes give the product (fp64 of the same rounded operands; one rounding of
+    the result, 2^-9 of it, and fp32 sums)."""
+    model, _ = _model(64, 16, 64, 1, 64, 64, "layernorm", torch.bfloat16, 5)
+    torch.manual_seed(vocab)
+    model.output_projection = torch.nn.Linear(2048, vocab, bias=False).to(DEV).to(torch.bfloat16)
+    x = torch.randn(rows, 1, 2048, device=DEV).to(torch.bfloat16)
+    assert M.ops.token_linear_pays(rows, vocab, 2048) == native
+    with torch.no_grad():
+        got = model.output_layer(x)
+        want = x.double() @ model.output_projection.weight.double().t()
+    assert got.shape == want.shape and _rms(got, want) < 2 ** -9
