@@ -15,17 +15,51 @@ namespace {
 
 using at::Tensor;
 
+// One Python argument, read while the interpreter lock is held.  Tensors stay where they are: the caller's frame holds
+// them until the call returns.
+struct Value {
+  enum Kind { kOther, kNone, kTensor, kInt, kFloat } kind = kOther;
+  const Tensor* t = nullptr;
+  int64_t i = 0;
+  double d = 0.0;
+};
+// false: a Python error is set
+bool read(PyObject* o, Value* v) {
+  if (o == Py_None) {
+    v->kind = Value::kNone;
+  } else if (THPVariable_Check(o)) {
+    v->kind = Value::kTensor;
+    v->t = &THPVariable_Unpack(o);
+  } else if (!PyFloat_Check(o) && PyIndex_Check(o)) {
+    PyObject* n = PyNumber_Index(o);
+    if (!n) return false;
+    v->i = PyLong_AsLongLong(n);
+    Py_DECREF(n);
+    if (v->i == -1 && PyErr_Occurred()) return false;
+    v->kind = Value::kInt;
+    v->d = (double)v->i;
+  } else if (PyNumber_Check(o)) {
+    v->d = PyFloat_AsDouble(o);
+    if (v->d == -1.0 && PyErr_Occurred()) return false;
+    v->kind = Value::kFloat;
+  }
+  return true;
+}
+
 struct Args {
-  PyObject* const* a;
+  const Value* a;
   Py_ssize_t n;
   const char* who;
   void want(Py_ssize_t k) const {
     if (n != k) throw std::runtime_error(std::string(who) + ": " + std::to_string(k) + " arguments expected");
   }
-  bool none(int i) const { return a[i] == Py_None; }
+  [[noreturn]] void bad(int i, const char* what) const {
+    throw std::runtime_error(std::string(who) + ": argument " + std::to_string(i) + " must be " + what);
+  }
+  bool none(int i) const { return a[i].kind == Value::kNone; }
   const Tensor& t(int i) const {
-    if (!THPVariable_Check(a[i])) throw std::runtime_error(std::string(who) + ": argument " + std::to_string(i) + " must be a tensor");
-    return THPVariable_Unpack(a[i]);
+    if (a[i].kind != Value::kTensor) bad(i, "a tensor");
+    return *a[i].t;
   }
   // a contiguous tensor of the given type, size and device
   const Tensor& t(int i, at::ScalarType dt, int64_t numel, const at::Device& dev) const {
@@ -53,19 +87,16 @@ struct Args {
     }
   }
   double d(int i) const {
-    const double v = PyFloat_AsDouble(a[i]);
-    if (v == -1.0 && PyErr_Occurred()) throw std::runtime_error("");
-    return v;
+    if (a[i].kind != Value::kInt && a[i].kind != Value::kFloat) bad(i, "a number");
+    return a[i].d;
   }
   int64_t i64(int i) const {
-    const int64_t v = PyLong_AsLongLong(a[i]);
-    if (v == -1 && PyErr_Occurred()) throw std::runtime_error("");
-    return v;
+    if (a[i].kind != Value::kInt) bad(i, "an integer");
+    return a[i].i;
   }
-  void* stream(int i) const { return (void*)(uintptr_t)PyLong_AsUnsignedLongLong(a[i]); }
+  bool flag(int i) const { return i64(i) != 0; }
+  void* stream(int i) const { return (void*)(uintptr_t)i64(i); }
 };
-
-bool truth(PyObject* o) { return PyObject_IsTrue(o) == 1; }
 
 int dtype_code(const Tensor& x) {
   switch (x.scalar_type()) {
@@ -80,13 +111,25 @@ void check(int rc, const char* who) {
   if (rc != 0) throw std::runtime_error(std::string(who) + ": " + mega_last_error() + " (code " + std::to_string(rc) + ")");
 }
 
-PyObject* wrap(Tensor t) { return t.defined() ? THPVariable_Wrap(std::move(t)) : (Py_INCREF(Py_None), Py_None); }
-
+// what an entry returns: one tensor, or a tuple of them (undefined: None)
+struct Result {
+  Tensor t[10];
+  int n = 0;
+  bool one = false;
+};
+Result wrap(Tensor t) {
+  Result r;
+  r.t[0] = std::move(t);
+  r.n = 1;
+  r.one = true;
+  return r;
+}
 template <size_t N>
-PyObject* tuple(Tensor (&ts)[N]) {
-  PyObject* r = PyTuple_New(N);
-  if (!r) return nullptr;
-  for (size_t i = 0; i < N; ++i) PyTuple_SET_ITEM(r, i, wrap(std::move(ts[i])));
+Result tuple(Tensor (&ts)[N]) {
+  static_assert(N <= 10, "Result holds ten tensors");
+  Result r;
+  for (size_t i = 0; i < N; ++i) r.t[i] = std::move(ts[i]);
+  r.n = (int)N;
   return r;
 }
 
@@ -97,7 +140,7 @@ Tensor empty(at::IntArrayRef sizes, const Tensor& like, at::ScalarType dt) {
 // (x [B, 1, D], mask [B] bytes | None, count, mean, var, h | None, keys | None, values | None, keep, norm gamma, norm beta,
 //  norm eps, groups, p, q, gamma, omega, v weight, v bias, mx weight, mx bias, h weight, gamma, beta, move act,
 //  move weight | None, move eps, cis, heads, stream) -> (out [B, 1, D], count, mean, var, h', keys' | None, values' | None)
-PyObject* token_gated_attention(const Args& A) {
+Result token_gated_attention(const Args& A) {
   A.want(30);
   const Tensor& x = A.t(0);
   const at::Device dev = x.device();
@@ -134,7 +177,7 @@ PyObject* token_gated_attention(const Args& A) {
     a.k_batch = k.stride(0);
   }
   a.v_old = A.opt(7, T, B * n * hidden, dev);
-  const bool keep = truth(A.a[8]);
+  const bool keep = A.flag(8);
   a.norm_gamma = (const float*)A.p(9, at::kFloat, D, dev);
   a.norm_beta = (const float*)A.p(10, at::kFloat, D, dev);
   a.norm_eps = A.d(11);
@@ -184,7 +227,7 @@ PyObject* token_gated_attention(const Args& A) {
 
 // (x [B, 1, D], norm kind, norm weight | None, norm bias | None, eps, fc1 weight, fc1 bias, fc2 weight, layer scale | None,
 //  stream) -> x + scale fc2(silu(fc1(norm(x))))
-PyObject* token_ffn(const Args& A) {
+Result token_ffn(const Args& A) {
   A.want(10);
   const Tensor& x = A.t(0);
   const at::Device dev = x.device();
@@ -217,7 +260,7 @@ PyObject* token_ffn(const Args& A) {
 
 // (tokens [B, 1], table [V, D], scale | None, pad | None) -> (x [B, 1, D], mask [B, 1] bool | None): torch's own lookup, which
 // knows what to do with an index outside the table
-PyObject* token_embed(const Args& A) {
+Result token_embed(const Args& A) {
   A.want(4);
   const Tensor& tok = A.t(0);
   Tensor r[2] = {at::embedding(A.t(1), tok), Tensor()};
@@ -227,7 +270,7 @@ PyObject* token_embed(const Args& A) {
 }
 
 // (x [B, 1, D], mask [B] bytes | None, count, mean, var, gamma, beta, eps, groups, stream) -> (xn, count, mean, var)
-PyObject* token_norm(const Args& A) {
+Result token_norm(const Args& A) {
   A.want(10);
   const Tensor& x = A.t(0);
   const at::Device dev = x.device();
@@ -246,7 +289,7 @@ PyObject* token_norm(const Args& A) {
 }
 
 // (x [B, 1, K], weight [N, K], bias | None, stream) -> [B, 1, N]
-PyObject* token_linear(const Args& A) {
+Result token_linear(const Args& A) {
   A.want(4);
   const Tensor &x = A.t(0), &w = A.t(1);
   if (x.dim() != 3 || x.size(1) != 1 || !x.is_contiguous() || !x.is_cuda() || w.dim() != 2)
@@ -263,7 +306,7 @@ PyObject* token_linear(const Args& A) {
 
 // (x [B, D] in any shape, count, next count, mean, var, norm weight, norm bias, eps, p, q, gamma, complex, omega, h, groups,
 //  stream) -> (xn, y) in x's shape; count / mean / var / h are the step's own buffers, updated in place (next count takes the new count)
-PyObject* norm_ema_step(const Args& A) {
+Result norm_ema_step(const Args& A) {
   A.want(16);
   Tensor x = A.t(0).detach().contiguous();
   const at::Device dev = x.device();
@@ -313,9 +356,9 @@ EmaIn ema_params(const Args& A, int i, bool is_complex, bool two_sided) {
 // (alpha, delta, third, gamma, omega, is_complex, two_sided, shift, activations (a tensor of their type),
 //  weight | None, bias, prior mean, prior log-variance, prior count, batch, stream)
 //   -> (p, q, gamma, omega, image, norm gamma, norm beta, prior mean [B, G], prior var [B, G], count [B])
-PyObject* train_prepare(const Args& A) {
+Result train_prepare(const Args& A) {
   A.want(16);
-  const bool cplx = truth(A.a[5]), two = truth(A.a[6]);
+  const bool cplx = A.flag(5), two = A.flag(6);
   const EmaIn in = ema_params(A, 0, cplx, two);
   const MegaEmaParams& e = in.e;
   const Tensor& like = A.t(0);
@@ -352,7 +395,7 @@ PyObject* train_prepare(const Args& A) {
     n.prev_var = (float*)r[8].data_ptr();
     n.prev_count = (int64_t*)r[9].data_ptr();
   }
-  check(mega_train_prepare(&e, norm ? &n : nullptr, dtype_code(A.t(8)), truth(A.a[7]), (float*)r[0].data_ptr(),
+  check(mega_train_prepare(&e, norm ? &n : nullptr, dtype_code(A.t(8)), A.flag(7), (float*)r[0].data_ptr(),
                            (float*)r[1].data_ptr(), (float*)r[2].data_ptr(), (float*)r[3].data_ptr(), r[4].data_ptr(), nimg,
                            A.stream(15)),
         A.who);
@@ -361,14 +404,14 @@ PyObject* train_prepare(const Args& A) {
 
 // (x [B, L, D], mask bytes | None, count, mean, var, norm gamma, norm beta, eps, p, q, gamma, omega, image, is_complex,
 //  y in x's layout, norm workspace, stream) -> (xn, y [B, D, L], count, cummean, cumrstd)
-PyObject* norm_move_forward(const Args& A) {
+Result norm_move_forward(const Args& A) {
   A.want(17);
   const Tensor& x = A.t(0);
   const at::Device dev = x.device();
   if (x.dim() != 3 || !x.is_contiguous() || !x.is_cuda()) throw std::runtime_error("norm_move_forward: x must be a contiguous [B, L, D] device tensor");
   const int64_t B = x.size(0), L = x.size(1), D = x.size(2), N = A.t(8).size(1), G = A.t(3).numel() / (B > 0 ? B : 1);
   if (G <= 0 || D % G) throw std::runtime_error("norm_move_forward: groups");
-  const bool input = truth(A.a[14]);
+  const bool input = A.flag(14);
   Tensor r[5] = {at::empty_like(x), input ? at::empty({B, L, D}, x.options()).transpose(1, 2) : at::empty({B, D, L}, x.options()),
                  empty({B}, x, at::kLong), empty({B, L, G}, x, at::kFloat), empty({B, L, G}, x, at::kFloat)};
   Tensor stats = empty({2, B, G}, x, at::kFloat);
@@ -382,7 +425,7 @@ PyObject* norm_move_forward(const Args& A) {
             (const float*)A.p(6, at::kFloat, D, dev), (const uint8_t*)A.opt(1, at::kByte, B * L, dev), A.d(7),
             (int64_t*)r[2].data_ptr(), (float*)stats.data_ptr(), (float*)stats.data_ptr() + B * G, (float*)r[3].data_ptr(),
             (float*)r[4].data_ptr(), (const float*)A.p(8, at::kFloat, D * N, dev), (const float*)A.p(9, at::kFloat, D * N * 2, dev),
-            (const float*)A.p(10, at::kFloat, D * N * 2, dev), truth(A.a[13]), (const float*)A.p(11, at::kFloat, D, dev), nullptr,
+            (const float*)A.p(10, at::kFloat, D * N * 2, dev), A.flag(13), (const float*)A.p(11, at::kFloat, D, dev), nullptr,
             nullptr, B, L, D, G, N, img.data_ptr(), ws.data_ptr(), ws.numel(), sc.data_ptr(), nsc, A.stream(16)),
         A.who);
   return tuple(r);
@@ -419,7 +462,7 @@ struct ParamGrads {
 // (xn gradient | None, y gradient [B, D, L], x, xn, mask bytes | None, prior mean, count, cummean, cumrstd, norm gamma, p, q,
 //  gamma, omega, image, weight, prior log-variance, prior needs gradients, alpha, delta, third, gamma, omega, is_complex,
 //  stream) -> (x gradient, weight, bias, prior mean | None, prior log-variance | None, alpha, delta, third, gamma, omega)
-PyObject* norm_move_backward(const Args& A) {
+Result norm_move_backward(const Args& A) {
   A.want(25);
   const Tensor &x = A.t(2), &xn = A.t(3);
   const at::Device dev = x.device();
@@ -427,7 +470,7 @@ PyObject* norm_move_backward(const Args& A) {
   const int64_t B = x.size(0), L = x.size(1), D = x.size(2), N = A.t(10).size(1);
   if (B <= 0 || L <= 0) throw std::runtime_error("norm_move_backward: empty input");
   const int64_t G = A.t(5).numel() / B;
-  const int cplx = truth(A.a[23]), dt = dtype_code(x);
+  const int cplx = A.flag(23), dt = dtype_code(x);
   void* s = A.stream(24);
   const EmaIn in = ema_params(A, 18, cplx, false);
   Tensor g = A.t(1).detach();
@@ -475,7 +518,7 @@ PyObject* norm_move_backward(const Args& A) {
   r[2] = at::empty_like(w);
   n.weight = r[1].data_ptr();
   n.bias = r[2].data_ptr();
-  if (truth(A.a[17])) {
+  if (A.flag(17)) {
     r[3] = at::empty_like(pl);
     r[4] = at::empty_like(pl);
     n.prior_mean = r[3].data_ptr();
@@ -489,10 +532,10 @@ PyObject* norm_move_backward(const Args& A) {
 
 // (y gradient, x, both with any strides of [B, D, L], mask bytes | None, q, alpha, delta, third, gamma, omega, is_complex,
 //  two_sided, shift, stream) -> gradients of (alpha, delta, third, gamma, omega)
-PyObject* ema_param_backward(const Args& A) {
+Result ema_param_backward(const Args& A) {
   A.want(13);
   const Tensor &g = A.t(0), &x = A.t(1);
-  const int cplx = truth(A.a[9]), two = truth(A.a[10]), shift = truth(A.a[11]);
+  const int cplx = A.flag(9), two = A.flag(10), shift = A.flag(11);
   void* s = A.stream(12);
   const EmaIn in = ema_params(A, 4, cplx, two);
   const int64_t B = x.size(0), D = x.size(1), L = x.size(2), N = in.e.N;
@@ -596,36 +639,15 @@ bool eager() {
 // Values of its own in memory and no forward-mode tangent beside them.
 bool plain(const Tensor& t) { return !at::isTensorSubclassLike(t) && !t._fw_grad(0).defined(); }
 
-// (x, tensor | None, ...) -> bool: x is a GPU activation and every tensor is contiguous, of its type and device, on 16
-// bytes; `graph`: and every one asks for its gradient (the composites' backward passes form all of them)
-PyObject* same_storage(const Args& A, bool graph) {
-  const Tensor& x = A.t(0);
-  if (!eager()) return PyBool_FromLong(false);
-  for (int i = 0; i < A.n; ++i)
-    if (!A.none(i) && !plain(A.t(i))) return PyBool_FromLong(false);
-  const at::ScalarType dt = x.scalar_type();
-  bool ok = x.is_cuda() && (dt == at::kFloat || dt == at::kBFloat16 || dt == at::kHalf) && x.dim() > 1 && x.numel() > 0 && !x.is_neg() &&
-            (uintptr_t)x.data_ptr() % 16 == 0;
-  for (int i = 1; ok && i < A.n; ++i)
-    if (!A.none(i)) {
-      const Tensor& t = A.t(i);
-      ok = t.scalar_type() == dt && t.device() == x.device() && t.is_contiguous() && (uintptr_t)t.data_ptr() % 16 == 0 && !t.is_neg() &&
-           (!graph || t.requires_grad());
-    }
-  return PyBool_FromLong(ok);
-}
-PyObject* uniform(const Args& A) { return same_storage(A, false); }
-PyObject* trainable(const Args& A) { return same_storage(A, true); }
-
 // (x, kind, weight | None, bias | None, eps, stream) -> y
-PyObject* row_norm_forward(const Args& A) {
+Result row_norm_forward(const Args& A) {
   A.want(6);
   same_type(A, {0, 2, 3}, A.t(0));
   return wrap(row_norm(A.t(0), opt_t(A, 2), opt_t(A, 3), (int)A.i64(1), A.d(4), A.stream(5), A.who));
 }
 
 // (dy, x, kind, weight | None, bias | None, eps, stream) -> (dx, dw, db)
-PyObject* row_norm_backward(const Args& A) {
+Result row_norm_backward(const Args& A) {
   A.want(7);
   same_type(A, {1, 3, 4}, A.t(1));
   auto [dx, dw, db] = row_norm_back(rows16(A.t(0), A.t(1)), A.t(1), opt_t(A, 3), opt_t(A, 4), Tensor(), (int)A.i64(2), A.d(5), A.stream(6), A.who);
@@ -635,7 +657,7 @@ PyObject* row_norm_backward(const Args& A) {
 
 // x + fc2(silu(fc1(norm(x)))): (x, kind, norm weight | None, norm bias | None, eps, fc1 weight, fc1 bias, fc2 weight, stream)
 //   -> (out, n, pre, h)
-PyObject* ffn_forward(const Args& A) {
+Result ffn_forward(const Args& A) {
   A.want(9);
   const Tensor& x = A.t(0);
   same_type(A, {0, 2, 3, 5, 6, 7}, x);
@@ -650,7 +672,7 @@ PyObject* ffn_forward(const Args& A) {
 
 // (dout, x, n, pre, h, kind, norm weight | None, norm bias | None, eps, fc1 weight, fc2 weight, stream)
 //   -> (dx, d norm weight, d norm bias, d fc1 weight, d fc1 bias, d fc2 weight)
-PyObject* ffn_backward(const Args& A) {
+Result ffn_backward(const Args& A) {
   A.want(12);
   const Tensor &x = A.t(1), &n = A.t(2), &pre = A.t(3), &h = A.t(4);
   const Tensor dout = rows16(A.t(0), x);
@@ -671,7 +693,7 @@ PyObject* ffn_backward(const Args& A) {
 }
 
 // W2 (silu(W1 n) * W3 n) + residual: (n, residual | None, W1, W3, W2, stream) -> (out, a, b, g)
-PyObject* swiglu_forward(const Args& A) {
+Result swiglu_forward(const Args& A) {
   A.want(6);
   const Tensor& n = A.t(0);
   same_type(A, {0, 1, 2, 3, 4}, n);
@@ -688,7 +710,7 @@ PyObject* swiglu_forward(const Args& A) {
 }
 
 // (dout, n, a, b, g, W1, W3, W2, stream) -> (dn, dW1, dW3, dW2)
-PyObject* swiglu_backward(const Args& A) {
+Result swiglu_backward(const Args& A) {
   A.want(9);
   const Tensor &n = A.t(1), &a = A.t(2), &b = A.t(3), &g = A.t(4);
   same_type(A, {1, 2, 3, 4, 5, 6, 7}, n);
@@ -710,7 +732,7 @@ PyObject* swiglu_backward(const Args& A) {
 // The gated attention between its norm / moving average and the attention product.
 // (xn [B, L, D], mx [B, D, L] view of time-major memory, v weight, v bias, mx weight, mx bias, gamma, beta, freqs, heads,
 //  chunk, move act, move weight | None, move eps, stream) -> (vp, v, mx (time-major), act, base, q, k)
-PyObject* mix_forward(const Args& A) {
+Result mix_forward(const Args& A) {
   A.want(15);
   const Tensor& xn = A.t(0);
   same_type(A, {0, 2, 3, 4, 5, 6, 7, 12}, xn);
@@ -740,7 +762,7 @@ PyObject* mix_forward(const Args& A) {
 }
 
 // (residual [B, L, D], base, attention [T, E], h weight, S, stream) -> (out, gated, hp)
-PyObject* mix_out_forward(const Args& A) {
+Result mix_out_forward(const Args& A) {
   A.want(6);
   const Tensor &x = A.t(0), &base = A.t(1), &attn = A.t(2);
   same_type(A, {0, 1, 2, 3}, x);
@@ -761,7 +783,7 @@ PyObject* mix_out_forward(const Args& A) {
 }
 
 // (dout, residual, base, attention [T, E], gated, hp, h weight, S, stream) -> (d residual, d base (u, r, hx slots), d attention, d h weight)
-PyObject* mix_out_backward(const Args& A) {
+Result mix_out_backward(const Args& A) {
   A.want(9);
   const Tensor &x = A.t(1), &base = A.t(2), &attn = A.t(3), &gated = A.t(4), &hp = A.t(5), &hw = A.t(6);
   same_type(A, {1, 2, 3, 4, 5, 6}, x);
@@ -796,7 +818,7 @@ PyObject* mix_out_backward(const Args& A) {
 // (dq [T, S], dk, dv [T, E], dbase, xn, vp, mx, act, base, v weight, mx weight, gamma, freqs, heads, chunk, move act,
 //  move weight | None, move eps, stream)
 //   -> (d xn, d mx (time-major), d v weight, d v bias, d mx weight, d mx bias, d gamma, d beta, d move weight)
-PyObject* mix_backward(const Args& A) {
+Result mix_backward(const Args& A) {
   A.want(19);
   const Tensor &dbase = A.t(3), &xn = A.t(4), &vp = A.t(5), &mx = A.t(6), &act = A.t(7), &base = A.t(8);
   same_type(A, {3, 4, 5, 6, 7, 8, 9, 10, 11, 16}, xn);
@@ -842,8 +864,42 @@ PyObject* mix_backward(const Args& A) {
   return tuple(r);
 }
 
+// ---- questions about Python objects and tensors: short, nothing is launched, the interpreter lock is held
+struct Held {
+  PyObject* const* a;
+  Py_ssize_t n;
+};
+
+// (x, tensor | None, ...) -> bool: x is a GPU activation and every tensor is contiguous, of its type and device, on 16
+// bytes; `graph`: and every one asks for its gradient (the composites' backward passes form all of them)
+PyObject* same_storage(const Held& A, bool graph) {
+  Value v[32];
+  if (A.n < 1 || A.n > 32) throw std::runtime_error("uniform / trainable: 1 to 32 tensors");
+  for (Py_ssize_t i = 0; i < A.n; ++i) {
+    if (A.a[i] != Py_None && !THPVariable_Check(A.a[i])) throw std::runtime_error("uniform / trainable: tensors expected");
+    read(A.a[i], &v[i]);
+  }
+  if (v[0].kind == Value::kNone) throw std::runtime_error("uniform / trainable: the activations are missing");
+  const Tensor& x = *v[0].t;
+  if (!eager()) return PyBool_FromLong(false);
+  for (int i = 0; i < A.n; ++i)
+    if (v[i].t && !plain(*v[i].t)) return PyBool_FromLong(false);
+  const at::ScalarType dt = x.scalar_type();
+  bool ok = x.is_cuda() && (dt == at::kFloat || dt == at::kBFloat16 || dt == at::kHalf) && x.dim() > 1 && x.numel() > 0 && !x.is_neg() &&
+            (uintptr_t)x.data_ptr() % 16 == 0;
+  for (int i = 1; ok && i < A.n; ++i)
+    if (v[i].t) {
+      const Tensor& t = *v[i].t;
+      ok = t.scalar_type() == dt && t.device() == x.device() && t.is_contiguous() && (uintptr_t)t.data_ptr() % 16 == 0 && !t.is_neg() &&
+           (!graph || t.requires_grad());
+    }
+  return PyBool_FromLong(ok);
+}
+PyObject* uniform(const Held& A) { return same_storage(A, false); }
+PyObject* trainable(const Held& A) { return same_storage(A, true); }
+
 // (dict, ...) -> bytes: storage address and in-place version of every tensor in the dictionaries' values, in order
-PyObject* tensor_versions(const Args& A) {
+PyObject* tensor_versions(const Held& A) {
   std::vector<int64_t> buf;
   for (int i = 0; i < A.n; ++i) {
     if (!PyDict_Check(A.a[i])) throw std::runtime_error("tensor_versions: dictionaries expected");
@@ -864,7 +920,7 @@ PyObject* tensor_versions(const Args& A) {
 // one of these types with its class's own call, nobody looking at inputs or outputs; `bias` not None: and holds a weight
 // parameter, and a bias parameter or none.  Asked seven times per layer and token: one module 0.52 us, two 0.69, where the
 // same questions in Python take 0.70 and 0.97.
-PyObject* plain_modules(const Args& A) {
+PyObject* plain_modules(const Held& A) {
   static PyObject *const forward = PyUnicode_InternFromString("forward"), *const parameters = PyUnicode_InternFromString("_parameters"),
                   *const weight = PyUnicode_InternFromString("weight"), *const bias = PyUnicode_InternFromString("bias"),
                   *const hooks[] = {PyUnicode_InternFromString("_forward_hooks"), PyUnicode_InternFromString("_forward_pre_hooks"),
@@ -885,7 +941,7 @@ PyObject* plain_modules(const Args& A) {
       PyObject* v = PyDict_GetItem(d, h);
       ok = ok && (!v || !PyObject_IsTrue(v));
     }
-    if (ok && !A.none(2)) {
+    if (ok && A.a[2] != Py_None) {
       PyObject* p = PyDict_GetItem(d, parameters);
       PyObject* b = p && PyDict_Check(p) ? PyDict_GetItem(p, bias) : nullptr;
       ok = p && PyDict_Check(p) && !absent(PyDict_GetItem(p, weight)) && (A.a[2] == Py_True ? !absent(b) : b == Py_None);
@@ -896,30 +952,78 @@ PyObject* plain_modules(const Args& A) {
   return PyBool_FromLong(true);
 }
 
-PyObject* guarded(PyObject* (*f)(const Args&), const Args& args) {
-  try {
-    c10::AutoGradMode no_graph(false);
-    return f(args);
-  } catch (const std::exception& e) {
-    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
+// ---- entries.  A composite allocates, multiplies and launches without the interpreter lock (and in checked mode waits for
+// its stream): other Python threads go on.
+constexpr Py_ssize_t kMostArgs = 32;
+
+PyObject* guarded(Result (*f)(const Args&), PyObject* const* a, Py_ssize_t n, const char* who) {
+  Value v[kMostArgs];
+  if (n > kMostArgs) {
+    PyErr_Format(PyExc_RuntimeError, "%s: too many arguments", who);
     return nullptr;
   }
+  for (Py_ssize_t i = 0; i < n; ++i)
+    if (!read(a[i], &v[i])) return nullptr;
+  Result r;
+  std::string error;
+  bool failed = false;
+  PyThreadState* lock = PyEval_SaveThread();
+  try {
+    c10::AutoGradMode no_graph(false);
+    r = f(Args{v, n, who});
+  } catch (const std::exception& e) {
+    failed = true;
+    error = e.what();
+  } catch (...) {
+    failed = true;
+    error = std::string(who) + ": unknown error";
+  }
+  PyEval_RestoreThread(lock);
+  if (failed) {
+    PyErr_SetString(PyExc_RuntimeError, error.c_str());
+    return nullptr;
+  }
+  auto object = [](Tensor& t) { return t.defined() ? THPVariable_Wrap(std::move(t)) : (Py_INCREF(Py_None), Py_None); };
+  if (r.one) return object(r.t[0]);
+  PyObject* out = PyTuple_New(r.n);
+  for (int i = 0; out && i < r.n; ++i) {
+    PyObject* o = object(r.t[i]);
+    if (!o) {
+      Py_DECREF(out);
+      return nullptr;
+    }
+    PyTuple_SET_ITEM(out, i, o);
+  }
+  return out;
 }
 
-#define MEGA_ENTRY(f)                                                                                              \
+PyObject* guarded_held(PyObject* (*f)(const Held&), PyObject* const* a, Py_ssize_t n, const char*) {
+  try {
+    return f(Held{a, n});
+  } catch (const std::exception& e) {
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
+  } catch (...) {
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, "unknown error");
+  }
+  return nullptr;
+}
+
+#define MEGA_METHOD(f, guard)                                                                                      \
   {#f,                                                                                                             \
    (PyCFunction)(void (*)(void))(PyObject * (*)(PyObject*, PyObject* const*, Py_ssize_t))                          \
-       [](PyObject*, PyObject* const* a, Py_ssize_t n) -> PyObject* { return guarded(f, Args{a, n, #f}); },        \
+       [](PyObject*, PyObject* const* a, Py_ssize_t n) -> PyObject* { return guard(f, a, n, #f); },                \
    METH_FASTCALL, nullptr}
+#define MEGA_ENTRY(f) MEGA_METHOD(f, guarded)
+#define MEGA_QUESTION(f) MEGA_METHOD(f, guarded_held)
 PyMethodDef methods[] = {MEGA_ENTRY(token_gated_attention), MEGA_ENTRY(token_ffn),  MEGA_ENTRY(token_embed),
                          MEGA_ENTRY(token_norm),            MEGA_ENTRY(token_linear), MEGA_ENTRY(norm_ema_step),
-                         MEGA_ENTRY(tensor_versions),       MEGA_ENTRY(train_prepare), MEGA_ENTRY(norm_move_forward),
+                         MEGA_QUESTION(tensor_versions),       MEGA_ENTRY(train_prepare), MEGA_ENTRY(norm_move_forward),
                          MEGA_ENTRY(norm_move_backward),    MEGA_ENTRY(ema_param_backward),
                          MEGA_ENTRY(row_norm_forward),      MEGA_ENTRY(row_norm_backward), MEGA_ENTRY(ffn_forward),
                          MEGA_ENTRY(ffn_backward),          MEGA_ENTRY(swiglu_forward), MEGA_ENTRY(swiglu_backward),
                          MEGA_ENTRY(mix_forward),           MEGA_ENTRY(mix_out_forward), MEGA_ENTRY(mix_out_backward),
-                         MEGA_ENTRY(mix_backward),          MEGA_ENTRY(uniform),    MEGA_ENTRY(trainable),
-                         MEGA_ENTRY(plain_modules),
+                         MEGA_ENTRY(mix_backward),          MEGA_QUESTION(uniform),    MEGA_QUESTION(trainable),
+                         MEGA_QUESTION(plain_modules),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "mega_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

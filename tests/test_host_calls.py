@@ -119,3 +119,36 @@ def test_tensor_versions(native, monkeypatch):
     with torch.no_grad():
         layer.alpha.add_(1.0)
     assert not torch.equal(layer.coeffs()[0], p)
+
+
+def test_composites_leave_the_interpreter_to_other_threads():
+    """A composite's work runs without the interpreter lock: another thread goes on under a long product (in host memory;
+    the weight of the next product does not fit, so the call ends before anything is launched)."""
+    import threading
+    import time
+
+    ticks, stop = [], threading.Event()
+
+    def count():
+        while not stop.is_set():
+            ticks.append(time.perf_counter())
+            time.sleep(0.001)
+
+    T, D, N = 40000, 512, 512
+    args = [torch.randn(T, D), torch.randn(T, D), *(torch.randn(T, N) for _ in range(3)), torch.randn(N, D), torch.randn(N, D),
+            torch.randn(D + 1, N), 0]
+    threads = torch.get_num_threads()
+    torch.set_num_threads(1)
+    other = threading.Thread(target=count)
+    other.start()
+    try:
+        begin = time.perf_counter()
+        with pytest.raises(RuntimeError):
+            H.swiglu_backward(*args)
+        end = time.perf_counter()
+    finally:
+        stop.set()
+        other.join()
+        torch.set_num_threads(threads)
+    # about one a millisecond; with the lock held none but at the edges
+    assert sum(begin < t < end for t in ticks) > 100 * (end - begin)
