@@ -1192,7 +1192,6 @@ class MixInFunc(torch.autograd.Function):
             got = _through_formula(lambda *t: mix_in_formula(*t, freqs, *ctx.consts, ctx.eps),
                                    (xn, mx, v_weight, v_bias, mx_weight, mx_bias, gamma, beta, act_weight), (dv, dbase, dq, dk))
             return (*got[:8], None, got[8], None, None, None, None)
-        SplitGrads.taken += 1                          # the four slices' gradients lie in one buffer
         with ops._on_device(xn.device):
             dxn, dmx, dvw, dvb, dmw, dmb, dgamma, dbeta, daw = ops._lib.load_host().mix_backward(
                 dq, dk, dv, dbase, xn.contiguous(), vp, mx.transpose(1, 2).contiguous(), a, base, v_weight, mx_weight, gamma,

@@ -629,9 +629,11 @@ def test_attention_bwd_entry_point_refuses_what_it_does_not_cover():
 
 @pytest.mark.parametrize("heads,act,moving,bidir", [(1, 'rmsnorm', 'cema', False), (2, 'silu', 'ema', False),
                                                     (1, 'silu', 'cema', True), (2, 'rmsnorm', 'cema', "padded")])
-def test_gated_attention_layer_trains(heads, act, moving, bidir):
+@pytest.mark.parametrize("operators", [False, True])
+def test_gated_attention_layer_trains(heads, act, moving, bidir, operators):
     """The whole layer under autograd (fp32), causal and bidirectional (also with padding):
-    parameter and input gradients against central differences of the fp64 layer oracle."""
+    parameter and input gradients against central differences of the fp64 layer oracle.  As two composite
+    operators around the attention, and operator by operator (with a frozen parameter)."""
     from test_gpu_layer import _params
     rng = np.random.default_rng(73)
     B, L, D, S, E, N, C = 2, 32, 16, 8, 24, 4, 16
@@ -652,12 +654,15 @@ def test_gated_attention_layer_trains(heads, act, moving, bidir):
     w64 = rng.normal(size=(B, L, D)).astype(np.float32).astype(np.float64)
     if mask is not None:
         w64 = w64 * (~mask)[..., None]         # padded positions carry no loss
+    layer.beta.requires_grad_(not operators)
     x = dev(x64).requires_grad_(True)
     out, _ = layer(x, None if mask is None else torch.from_numpy(mask).to(DEV))
+    assert ("MixOut" in type(out.grad_fn).__name__) == (not operators)
     in_place = M.modules.SplitGrads.taken
     (out * dev(w64)).sum().backward()
-    # the gradients of the four slices of the mx_proj output were written into one buffer (no concatenation)
-    assert M.modules.SplitGrads.taken == in_place + 1
+    # operator by operator: the gradients of the four slices of the mx_proj output were written into one buffer (no
+    # concatenation); the composites have no slices
+    assert M.modules.SplitGrads.taken == in_place + int(operators)
     P = _params(layer)
     okw = dict(chunk=C, num_heads=heads, moving_act=act, num_groups=4, bidirectional=bool(bidir), padding_mask=mask)
     loss = lambda Pd, xx: (O.gated_attention_layer(xx, Pd, **okw) * w64).sum()
@@ -668,6 +673,8 @@ def test_gated_attention_layer_trains(heads, act, moving, bidir):
               ("h_w", layer.h_proj.weight), ("gamma", layer.gamma), ("beta", layer.beta),
               ("norm_weight", layer.norm.weight), ("norm_bias", layer.norm.bias)]
     for name, prm in checks:
+        if not prm.requires_grad:
+            continue
         grad = host(prm.grad)
         scale = np.abs(grad).max() + 1e-6
         for _ in range(3):
