@@ -289,3 +289,27 @@ def test_output_projection_of_many_columns(rows, vocab, native):
         got = model.output_layer(x)
         want = x.double() @ model.output_projection.weight.double().t()
     assert got.shape == want.shape and _rms(got, want) < 2 ** -9
+
+
+# positions per workgroup of 64, 128 and 256 with a partial last block and several rounds of keys and values, heads of
+# more than 256 features, several slabs of 512 value columns
+@pytest.mark.parametrize("B,z,h,heads,prompt", [
+    (64, 128, 1024, 16, 171), (64, 128, 1024, 16, 300), (64, 128, 1024, 16, 700), (40, 512, 2176, 1, 130),
+    (64, 64, 4096, 8, 300), (1, 1024, 1056, 2, 200)])
+def test_token_attention_of_many_positions(B, z, h, heads, prompt):
+    """One token behind a long context against the operators one by one in fp32."""
+    half, full = _model(64, z, h, heads, 64, -1, "layernorm", torch.bfloat16, 13)
+    tokens = torch.randint(2, 72, (B, prompt + 1), device=DEV)
+    layer, ran = half.layers[0].mega_layer, []
+    step = layer._token_step
+    layer._token_step = lambda *a: ran.append(1) or step(*a)
+    sa, sb = {}, {}
+    with torch.no_grad():
+        half(tokens[:, :prompt], incremental_state=sa)
+        full(tokens[:, :prompt], incremental_state=sb)
+        got, want = half(tokens[:, prompt:], incremental_state=sa)[0], full(tokens[:, prompt:], incremental_state=sb)[0]
+    assert ran and _rms(got, want) < TOL[torch.bfloat16]
+    for ea, eb in zip(sa.values(), sb.values()):
+        for k in ea:
+            if k != "prev_count":
+                assert ea[k].shape == eb[k].shape and _rms(ea[k], eb[k]) < TOL[torch.bfloat16], k
