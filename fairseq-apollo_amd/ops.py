@@ -158,7 +158,9 @@ _TOKEN_LDS = 144 * 1024               # bytes of normalised input rows a project
 
 def token_rows(x: torch.Tensor, normalised: bool = False) -> bool:
     """True when the projections of x [rows, 1, K] run on the one-token kernels: 16-bit activations on the GPU, few
-    rows, whole 16-byte pieces; `normalised`: the rows are staged in LDS by every workgroup."""
+    rows, whole 16-byte pieces; `normalised`: with a norm or an activation of the rows in front.  Up to four such rows are
+    staged in LDS by every workgroup, more are normalised once into memory; the limit is that of the staged form and is
+    asked of any number (36 rows of 2048 channels run operator by operator)."""
     if not (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and x.dim() == 3 and x.shape[1] == 1) or \
             torch.is_autocast_enabled():               # (autocast picks the type of every product and norm by itself)
         return False
