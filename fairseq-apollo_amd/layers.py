@@ -143,7 +143,7 @@ class NormalizedFeedForwardNetwork(nn.Module):
 
     def _one_operator(self, x: Tensor) -> bool:
         """A training call the composite operator takes (no layer scale, no active dropout, whole 16-byte rows)."""
-        if not (x.is_cuda and torch.is_grad_enabled()):
+        if not (x.is_cuda and torch.is_grad_enabled()) or torch.compiler.is_compiling():
             return False
         norm, fc1, fc2 = self.norm, self.fc1, self.fc2
         vec = 16 // x.element_size()
@@ -389,13 +389,13 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
         v_proj, mx_proj, h_proj, act = (mods[k] for k in ('v_proj', 'mx_proj', 'h_proj', 'move_act'))
         return (ops.token_rows(x, normalised=True) and mask_bytes_ok(padding_mask, x)
                 and _plain(True, v_proj, mx_proj) and _plain(False, h_proj) and 'gamma' in mine and 'beta' in mine
-                and _unhooked((RMSNorm, nn.SiLU), act)
+                and _unhooked((RMSNorm, nn.SiLU, EfficientAttention), act, mods['efficient_attn'])
                 and ops._lib.load_host().uniform(
                     x, *v_proj._parameters.values(), *mx_proj._parameters.values(), *h_proj._parameters.values(),
                     mine['gamma'], mine['beta'], act._parameters.get('weight'))
-                and self.attention_activation == 'softmax' and isinstance(self.rel_pos_bias, RotaryEmbedding)
-                and self.norm.num_groups is not None and isinstance(move, MultiHeadComplexEMA)
-                and (move.truncation is None or move.truncation < 1) and self.ndim in (4, 8, 16, 32)
+                and self.attention_activation == 'softmax' and type(mods['rel_pos_bias']) is RotaryEmbedding
+                and isinstance(mods['norm'], TimestepNorm) and mods['norm'].num_groups is not None
+                and isinstance(move, MultiHeadComplexEMA) and (move.truncation is None or move.truncation < 1) and self.ndim in (4, 8, 16, 32)
                 and h % 32 == 0 and h % (8 * Nh) == 0 and z % (8 * Nh) == 0 and z // Nh <= 512
                 and (key is None or (key.dtype == x.dtype and key.stride(2) == 1 and key.stride(1) % 8 == 0
                                      and key.stride(0) % 8 == 0 and key.data_ptr() % 16 == 0
@@ -579,7 +579,7 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
         vec = 16 // xn.element_size()
         act = self.move_act
         rms = isinstance(act, RMSNorm)
-        return (xn.is_cuda and torch.is_grad_enabled() and _plain(True, self.v_proj, self.mx_proj) and _plain(False, self.h_proj)
+        return (xn.is_cuda and torch.is_grad_enabled() and not torch.compiler.is_compiling() and _plain(True, self.v_proj, self.mx_proj) and _plain(False, self.h_proj)
                 and _unhooked((RMSNorm, nn.SiLU), act) and mx.dtype == xn.dtype and residual.dtype == xn.dtype
                 and residual.data_ptr() % 16 == 0
                 and self.embed_dim % vec == 0 and self.zdim % vec == 0 and self.hdim % vec == 0 and self.zdim <= 128 * vec
@@ -635,8 +635,9 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
         simple = isinstance(self.rel_pos_bias, SimpleRelativePositionalBias)
         bsz, seq_len = z.shape[:2]
         Nh = self.num_heads
-        if (self.chunk_size > 1 and seq_len % self.chunk_size == 0 and "prev_key" not in saved_state and not simple
-                and not self.bidirectional and self.attention_activation == 'softmax' and not torch.is_autocast_enabled()):
+        if (self.chunk_size > 1 and seq_len % self.chunk_size == 0 and "prev_key" not in saved_state
+                and type(self.rel_pos_bias) is RotaryEmbedding and not self.bidirectional
+                and self.attention_activation == 'softmax' and not torch.is_autocast_enabled()):
             # whole chunks behind whole chunks: nothing cached, nothing to cache
             self._set_input_buffer(incremental_state, saved_state)
             q, k = ops.gate_qk_fwd(z, *self._qk_constants(False), Nh, self.chunk_size)

@@ -1379,7 +1379,8 @@ class SwiGLU(nn.Module):
         """W2 (silu(W1 x) * W3 x) (+ residual, which then enters the last product as its accumulator start: no
         separate addition pass over the activations; consume_residual: see linear_residual)."""
         w1, w3, w2 = self.w1, self.w3, self.w2
-        if x.is_cuda and torch.is_grad_enabled() and _plain(False, w1, w3, w2) and one_graph(x, w1.weight, w3.weight, w2.weight) and \
+        if x.is_cuda and torch.is_grad_enabled() and not torch.compiler.is_compiling() and _plain(False, w1, w3, w2) and \
+                one_graph(x, w1.weight, w3.weight, w2.weight) and \
                 (residual is None or (residual.dtype == x.dtype and residual.is_contiguous()
                                                              and residual.device == x.device
                                                              and residual.shape[:-1] == x.shape[:-1]

@@ -313,3 +313,42 @@ def test_token_attention_of_many_positions(B, z, h, heads, prompt):
         for k in ea:
             if k != "prev_count":
                 assert ea[k].shape == eb[k].shape and _rms(ea[k], eb[k]) < TOL[torch.bfloat16], k
+
+
+class Backwards(M.layers.RotaryEmbedding):
+    """Turns the other way."""
+    turned = 0
+
+    def rotary(self, x, sidx):
+        self.turned += 1
+        cis = self._freqs_cis(sidx, sidx + x.shape[-2]).conj()
+        return torch.view_as_real(torch.view_as_complex(x.float().unflatten(-1, (-1, 2))) * cis).flatten(-2).to(x.dtype)
+
+
+class Around(Within):
+    """A norm inside another module."""
+    seen = 0
+
+    def forward(self, *args, **kwargs):
+        self.seen += 1
+        return self.inner(*args, **kwargs)
+
+
+@pytest.mark.parametrize("what", ["rotation", "norm"])
+def test_replaced_parts_of_a_layer(what):
+    """A rotation of its own class, and a norm inside another module: whole chunks behind whole chunks and one token are
+    those of the operators one by one, which ask both (the rotation for q and for k)."""
+    half, full = _model(64, 16, 64, 2, 64, 64, "layernorm", torch.bfloat16, 5)
+    for layer in (*half.layers, *full.layers):
+        if what == "rotation":
+            layer.mega_layer.rel_pos_bias.__class__ = Backwards
+        else:
+            layer.mega_layer.norm = Around(layer.mega_layer.norm)
+    tokens = torch.randint(2, 72, (3, 129), device=DEV)
+    sa, sb = {}, {}
+    with torch.no_grad():
+        for a, b in ((0, 64), (64, 128), (128, 129)):
+            got, want = half(tokens[:, a:b], incremental_state=sa)[0], full(tokens[:, a:b], incremental_state=sb)[0]
+            assert _rms(got, want) < TOL[torch.bfloat16]
+    for layer in (*half.layers, *full.layers):
+        assert layer.mega_layer.rel_pos_bias.turned == 6 if what == "rotation" else layer.mega_layer.norm.seen == 3
