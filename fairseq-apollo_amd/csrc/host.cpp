@@ -7,6 +7,7 @@
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <torch/csrc/autograd/python_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "../../include/mega_hip.h"
@@ -670,10 +671,19 @@ Result ffn_forward(const Args& A) {
   return tuple(r);
 }
 
-// (dout, x, n, pre, h, kind, norm weight | None, norm bias | None, eps, fc1 weight, fc2 weight, stream)
+// Which gradients a backward pass is asked for (bit i: input i of the autograd function): the products behind the others are
+// left out, and their places in the result are None.
+struct Wanted {
+  int64_t bits;
+  bool any(int64_t m) const { return (bits & m) != 0; }
+  bool operator()(int i) const { return any((int64_t)1 << i); }
+};
+
+// (dout, x, n, pre, h, kind, norm weight | None, norm bias | None, eps, fc1 weight, fc2 weight, stream, wanted)
 //   -> (dx, d norm weight, d norm bias, d fc1 weight, d fc1 bias, d fc2 weight)
 Result ffn_backward(const Args& A) {
-  A.want(12);
+  A.want(13);
+  const Wanted want{A.i64(12)};               // x, norm weight, norm bias, fc1 weight, fc1 bias, fc2 weight
   const Tensor &x = A.t(1), &n = A.t(2), &pre = A.t(3), &h = A.t(4);
   const Tensor dout = rows16(A.t(0), x);
   same_type(A, {1, 2, 3, 4, 6, 7, 9, 10}, x);
@@ -682,12 +692,15 @@ Result ffn_backward(const Args& A) {
   if (dout.numel() != x.numel() || n.numel() != x.numel() || pre.numel() != x.numel() / x.size(-1) * A.t(10).size(1))
     throw std::runtime_error("ffn_backward: gradients and saved operands of other sizes than the forward's");
   const Tensor d2 = rows2(dout);
-  Tensor dw2 = at::mm(d2.t(), h);
-  Tensor dh = at::mm(d2, A.t(10));
-  auto [dpre, db1] = sum_rows(dh, pre, s, A.who);
-  Tensor dw1 = at::mm(dpre.t(), rows2(n));
-  Tensor dn = at::mm(dpre, A.t(9));
-  auto [dx, dnw, dnb] = row_norm_back(dn, x, opt_t(A, 6), opt_t(A, 7), dout, (int)A.i64(5), A.d(8), s, A.who);
+  Tensor dx, dnw, dnb, dw1, db1, dw2;
+  if (want(5)) dw2 = at::mm(d2.t(), h);
+  if (want.any(0x1f)) {
+    Tensor dpre;
+    std::tie(dpre, db1) = sum_rows(at::mm(d2, A.t(10)), pre, s, A.who);
+    if (want(3)) dw1 = at::mm(dpre.t(), rows2(n));
+    if (want.any(7))
+      std::tie(dx, dnw, dnb) = row_norm_back(at::mm(dpre, A.t(9)), x, opt_t(A, 6), opt_t(A, 7), dout, (int)A.i64(5), A.d(8), s, A.who);
+  }
   Tensor r[6] = {dx, dnw, dnb, dw1, db1, dw2};
   return tuple(r);
 }
@@ -709,23 +722,27 @@ Result swiglu_forward(const Args& A) {
   return tuple(r);
 }
 
-// (dout, n, a, b, g, W1, W3, W2, stream) -> (dn, dW1, dW3, dW2)
+// (dout, n, a, b, g, W1, W3, W2, stream, wanted) -> (dn, dW1, dW3, dW2)
 Result swiglu_backward(const Args& A) {
-  A.want(9);
+  A.want(10);
+  const Wanted want{A.i64(9)};                // n, residual, W1, W3, W2
   const Tensor &n = A.t(1), &a = A.t(2), &b = A.t(3), &g = A.t(4);
   same_type(A, {1, 2, 3, 4, 5, 6, 7}, n);
   void* s = A.stream(8);
   A.shape(3, a.sizes());
   A.shape(4, a.sizes());
   const Tensor d2 = rows2(A.t(0).to(n.scalar_type()).contiguous()), n2 = rows2(n);
-  Tensor dw2 = at::mm(d2.t(), g);
-  Tensor dg = at::mm(d2, A.t(7));
-  Tensor da = at::empty_like(a), db = at::empty_like(b);
-  check(mega_swiglu_bwd(dg.data_ptr(), a.data_ptr(), b.data_ptr(), da.data_ptr(), db.data_ptr(), dtype_code(n), a.numel(), s), A.who);
-  Tensor dw1 = at::mm(da.t(), n2), dw3 = at::mm(db.t(), n2);
-  Tensor dn = at::mm(da, A.t(5));
-  dn.addmm_(db, A.t(6));                         // both branches into one gradient: no third pass to add them
-  Tensor r[4] = {dn.view(n.sizes()), dw1, dw3, dw2};
+  Tensor dn, dw1, dw3, dw2;
+  if (want(4)) dw2 = at::mm(d2.t(), g);
+  if (want.any(0xd)) {
+    const Tensor dg = at::mm(d2, A.t(7));
+    const Tensor da = at::empty_like(a), db = at::empty_like(b);
+    check(mega_swiglu_bwd(dg.data_ptr(), a.data_ptr(), b.data_ptr(), da.data_ptr(), db.data_ptr(), dtype_code(n), a.numel(), s), A.who);
+    if (want(2)) dw1 = at::mm(da.t(), n2);
+    if (want(3)) dw3 = at::mm(db.t(), n2);
+    if (want(0)) dn = at::mm(da, A.t(5)).addmm_(db, A.t(6)).view(n.sizes());    // both branches into one gradient: no third pass to add them
+  }
+  Tensor r[4] = {dn, dw1, dw3, dw2};
   return tuple(r);
 }
 
@@ -782,9 +799,10 @@ Result mix_out_forward(const Args& A) {
   return tuple(r);
 }
 
-// (dout, residual, base, attention [T, E], gated, hp, h weight, S, stream) -> (d residual, d base (u, r, hx slots), d attention, d h weight)
+// (dout, residual, base, attention [T, E], gated, hp, h weight, S, stream, wanted) -> (d residual, d base (u, r, hx slots), d attention, d h weight)
 Result mix_out_backward(const Args& A) {
-  A.want(9);
+  A.want(10);
+  const Wanted want{A.i64(9)};                // residual, base, attention, h weight
   const Tensor &x = A.t(1), &base = A.t(2), &attn = A.t(3), &gated = A.t(4), &hp = A.t(5), &hw = A.t(6);
   same_type(A, {1, 2, 3, 4, 5, 6}, x);
   const Tensor dout = A.t(0).to(x.scalar_type()).contiguous();
@@ -806,20 +824,25 @@ Result mix_out_backward(const Args& A) {
                                   W, db + (D + S + E) * es, W, dt, T, D, s),
         A.who);
   const Tensor dh = dbase.narrow(1, D + S + E, D);
-  Tensor dhw = at::mm(dh.t(), gated);
-  Tensor dgated = at::mm(dh, hw), dattn = at::empty_like(attn);
-  check(mega_gate_mul_bwd_strided(dgated.data_ptr(), attn.data_ptr(), E, b + (D + S) * es, W, dattn.data_ptr(), db + (D + S) * es, W, dt,
-                                  T, E, s),
-        A.who);
-  Tensor r[4] = {dres, dbase, dattn, dhw};
+  Tensor dattn, dhw;
+  if (want(3)) dhw = at::mm(dh.t(), gated);
+  if (want.any(6)) {
+    const Tensor dgated = at::mm(dh, hw);
+    dattn = at::empty_like(attn);
+    check(mega_gate_mul_bwd_strided(dgated.data_ptr(), attn.data_ptr(), E, b + (D + S) * es, W, dattn.data_ptr(), db + (D + S) * es, W,
+                                    dt, T, E, s),
+          A.who);
+  }
+  Tensor r[4] = {dres, want(1) ? dbase : Tensor(), dattn, dhw};
   return tuple(r);
 }
 
 // (dq [T, S], dk, dv [T, E], dbase, xn, vp, mx, act, base, v weight, mx weight, gamma, freqs, heads, chunk, move act,
-//  move weight | None, move eps, stream)
+//  move weight | None, move eps, stream, wanted)
 //   -> (d xn, d mx (time-major), d v weight, d v bias, d mx weight, d mx bias, d gamma, d beta, d move weight)
 Result mix_backward(const Args& A) {
-  A.want(19);
+  A.want(20);
+  const Wanted want{A.i64(19)};               // xn, mx, v weight, v bias, mx weight, mx bias, gamma, beta, freqs, move weight
   const Tensor &dbase = A.t(3), &xn = A.t(4), &vp = A.t(5), &mx = A.t(6), &act = A.t(7), &base = A.t(8);
   same_type(A, {3, 4, 5, 6, 7, 8, 9, 10, 11, 16}, xn);
   void* s = A.stream(18);
@@ -846,20 +869,26 @@ Result mix_backward(const Args& A) {
                                dgamma.data_ptr(), dbeta.data_ptr(), dt, T, S, heads, chunk, 0, 1e-5, ws.data_ptr(), nws, s),
           A.who);
   }
-  Tensor dmxw = at::mm(dbase.t(), rows2(act));
-  Tensor dmxb = sum_rows(dbase, Tensor(), s, A.who).second;
-  Tensor dact = at::mm(dbase, A.t(10)).view(mx.sizes()), dmx, dmw;
-  const int act_kind = (int)A.i64(15);
-  if (act_kind == MEGA_TOKEN_RMSNORM) {
-    Tensor none;
-    std::tie(dmx, dmw, none) = row_norm_back(dact, mx, opt_t(A, 16), Tensor(), Tensor(), act_kind, A.d(17), s, A.who);
-  } else {
-    dmx = at::empty_like(mx);
-    check(mega_silu_bwd(dact.data_ptr(), mx.data_ptr(), dmx.data_ptr(), dt, mx.numel(), s), A.who);
+  Tensor dxn, dmx, dvw, dvb, dmxw, dmxb, dmw;
+  if (want(4)) dmxw = at::mm(dbase.t(), rows2(act));
+  if (want(5)) dmxb = sum_rows(dbase, Tensor(), s, A.who).second;
+  if (want.any(0x202)) {
+    const Tensor dact = at::mm(dbase, A.t(10)).view(mx.sizes());
+    const int act_kind = (int)A.i64(15);
+    if (act_kind == MEGA_TOKEN_RMSNORM) {
+      Tensor none;
+      std::tie(dmx, dmw, none) = row_norm_back(dact, mx, opt_t(A, 16), Tensor(), Tensor(), act_kind, A.d(17), s, A.who);
+    } else {
+      dmx = at::empty_like(mx);
+      check(mega_silu_bwd(dact.data_ptr(), mx.data_ptr(), dmx.data_ptr(), dt, mx.numel(), s), A.who);
+    }
   }
-  auto [dvp, dvb] = sum_rows(dv.view(vp.sizes()), vp, s, A.who);
-  Tensor dvw = at::mm(dvp.t(), rows2(xn));
-  Tensor dxn = at::mm(dvp, A.t(9)).view(xn.sizes());
+  if (want.any(0xd)) {
+    Tensor dvp;
+    std::tie(dvp, dvb) = sum_rows(dv.view(vp.sizes()), vp, s, A.who);
+    if (want(2)) dvw = at::mm(dvp.t(), rows2(xn));
+    if (want(0)) dxn = at::mm(dvp, A.t(9)).view(xn.sizes());
+  }
   Tensor r[9] = {dxn, dmx, dvw, dvb, dmxw, dmxb, dgamma, dbeta, dmw};
   return tuple(r);
 }
@@ -897,6 +926,20 @@ PyObject* same_storage(const Held& A, bool graph) {
 }
 PyObject* uniform(const Held& A) { return same_storage(A, false); }
 PyObject* trainable(const Held& A) { return same_storage(A, true); }
+
+// (autograd function's context) -> int: bit i is set where the running backward pass has use for input i's gradient
+// (torch.autograd.grad of a few tensors has none for the others; needs_input_grad only knows what asked in the forward pass)
+PyObject* wanted(const Held& A) {
+  if (A.n != 1 || !PyObject_TypeCheck(A.a[0], &THPFunctionType)) throw std::runtime_error("wanted: an autograd function's context expected");
+  const THPFunction* f = (const THPFunction*)A.a[0];
+  const auto node = f->cdata.lock();
+  if (!node) throw std::runtime_error("wanted: the context's node is gone");
+  long long bits = 0;
+  size_t edge = 0;
+  for (size_t i = 0; i < f->is_variable_input.size(); ++i)
+    if (f->is_variable_input[i] && node->task_should_compute_output(edge++)) bits |= 1ll << i;
+  return PyLong_FromLongLong(bits);
+}
 
 // (dict, ...) -> bytes: storage address and in-place version of every tensor in the dictionaries' values, in order
 PyObject* tensor_versions(const Held& A) {
@@ -1023,7 +1066,7 @@ PyMethodDef methods[] = {MEGA_ENTRY(token_gated_attention), MEGA_ENTRY(token_ffn
                          MEGA_ENTRY(ffn_backward),          MEGA_ENTRY(swiglu_forward), MEGA_ENTRY(swiglu_backward),
                          MEGA_ENTRY(mix_forward),           MEGA_ENTRY(mix_out_forward), MEGA_ENTRY(mix_out_backward),
                          MEGA_ENTRY(mix_backward),          MEGA_QUESTION(uniform),    MEGA_QUESTION(trainable),
-                         MEGA_QUESTION(plain_modules),
+                         MEGA_QUESTION(plain_modules), MEGA_QUESTION(wanted),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "mega_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -1122,7 +1122,8 @@ class FeedForwardFunc(torch.autograd.Function):
             return (*_through_formula(formula, (x, norm_weight, norm_bias, w1, ctx.bias, w2), y_grad), None, None)
         with ops._on_device(x.device):
             dx, dnw, dnb, dw1, db1, dw2 = ops._lib.load_host().ffn_backward(
-                y_grad, x.contiguous(), n, pre, h, ctx.kind, norm_weight, norm_bias, ctx.eps, w1, w2, ops._stream(x.device))
+                y_grad, x.contiguous(), n, pre, h, ctx.kind, norm_weight, norm_bias, ctx.eps, w1, w2, ops._stream(x.device),
+                ops._lib.load_host().wanted(ctx))
         return dx, dnw, dnb, dw1, db1, dw2, None, None
 
 
@@ -1161,7 +1162,7 @@ class SwiGLUBlockFunc(torch.autograd.Function):
         else:
             with ops._on_device(y_grad.device):
                 dx, dw1, dw3, dw2 = ops._lib.load_host().swiglu_backward(y_grad, x.contiguous(), a, b, g, w1, w3, w2,
-                                                                         ops._stream(y_grad.device))
+                                                                         ops._stream(y_grad.device), ops._lib.load_host().wanted(ctx))
         return dx, y_grad if ctx.residual else None, dw1, dw3, dw2
 
 
@@ -1195,8 +1196,8 @@ class MixInFunc(torch.autograd.Function):
         with ops._on_device(xn.device):
             dxn, dmx, dvw, dvb, dmw, dmb, dgamma, dbeta, daw = ops._lib.load_host().mix_backward(
                 dq, dk, dv, dbase, xn.contiguous(), vp, mx.transpose(1, 2).contiguous(), a, base, v_weight, mx_weight, gamma,
-                freqs, *ctx.consts, act_weight, ctx.eps, ops._stream(xn.device))
-        return dxn, dmx.transpose(1, 2), dvw, dvb, dmw, dmb, dgamma, dbeta, None, daw, None, None, None, None
+                freqs, *ctx.consts, act_weight, ctx.eps, ops._stream(xn.device), ops._lib.load_host().wanted(ctx))
+        return dxn, None if dmx is None else dmx.transpose(1, 2), dvw, dvb, dmw, dmb, dgamma, dbeta, None, daw, None, None, None, None
 
 
 def mix_in_formula(xn, mx, v_weight, v_bias, mx_weight, mx_bias, gamma, beta, act_weight, freqs, heads, chunk, act, eps):
@@ -1242,8 +1243,9 @@ class MixOutFunc(torch.autograd.Function):
             return (*_through_formula(formula, (residual, base, attn, h_weight), y_grad), None)
         with ops._on_device(y_grad.device):
             dres, dbase, dattn, dhw = ops._lib.load_host().mix_out_backward(
-                y_grad, residual.contiguous(), base, attn.contiguous(), gated, hp, h_weight, ctx.S, ops._stream(y_grad.device))
-        return dres, dbase, dattn.view(attn.shape), dhw, None
+                y_grad, residual.contiguous(), base, attn.contiguous(), gated, hp, h_weight, ctx.S, ops._stream(y_grad.device),
+                ops._lib.load_host().wanted(ctx))
+        return dres, dbase, None if dattn is None else dattn.view(attn.shape), dhw, None
 
 
 class AttentionSoftmaxFunc(torch.autograd.Function):

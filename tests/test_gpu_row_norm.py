@@ -345,3 +345,38 @@ def test_second_derivatives_gated_attention(act, heads):
         return res + torch.sigmoid(u) * (F.silu(hx + F.linear(attn * F.silu(r), hw)) - res)
 
     _second_derivatives(call, formula, tensors)
+
+
+@pytest.mark.parametrize("what", ["feed-forward", "swiglu", "gated attention"])
+def test_gradients_asked_for_one_by_one(what):
+    """torch.autograd.grad for one input at a time gives the bits of the whole backward pass, and the products behind the
+    gradients that nobody asks for are left out (the next test)."""
+    torch.manual_seed(9)
+    module = {"feed-forward": lambda: M.NormalizedFeedForwardNetwork(64, 96), "swiglu": lambda: M.SwiGLU(64, 96),
+              "gated attention": lambda: M.MovingAverageGatedAttention(64, 32, 128, 8, chunk_size=32, norm_num_groups=4,
+                                                                       moving_act='rmsnorm')}[what]().to(DEV).train()
+    x = torch.randn(2, 96, 64, device=DEV, requires_grad=True)
+    dy = torch.randn(2, 96, 64, device=DEV)
+    inputs = [x, *(p for p in module.parameters() if p.requires_grad)]
+
+    def run(wanted):
+        y = module(x)
+        y = y[0] if isinstance(y, tuple) else y
+        return torch.autograd.grad(y, wanted, dy)
+
+    whole = run(inputs)
+    for t, g in zip(inputs, whole):
+        assert torch.equal(run([t])[0], g)
+
+
+def test_products_nobody_asks_for():
+    """The composites' backward passes with one gradient wanted: the others' weights come back as None."""
+    H, S = M._lib.load_host(), M.ops._stream(torch.device(DEV))
+    torch.manual_seed(1)
+    x, n, pre, h, w1, w2 = (torch.randn(*s, device=DEV) for s in ((6, 8), (6, 8), (6, 16), (6, 16), (16, 8), (8, 16)))
+    ffn = [x, x, n, pre, h, M.ops.TOKEN_RMSNORM, None, None, 1e-5, w1, w2, S]
+    assert [t is not None for t in H.ffn_backward(*ffn, 1)] == [True, False, False, False, True, False]
+    assert [t is not None for t in H.ffn_backward(*ffn, 1 << 5)] == [False] * 5 + [True]
+    glu = [x, n, pre, h, pre, w1, w1, w2, S]
+    assert [t is not None for t in H.swiglu_backward(*glu, 1)] == [True, False, False, False]
+    assert [t is not None for t in H.swiglu_backward(*glu, 1 << 4)] == [False, False, False, True]

@@ -48,28 +48,28 @@ def test_backward_operands_of_other_shapes():
     D, S, E, T = 8, 4, 16, 3
     W = 2 * D + S + E
     x, row = torch.zeros(1, T, D), lambda *s: torch.zeros(*s)
-    out = [x, x, row(T, W), row(T, E), row(T, E), row(T, D), row(D, E), S, 0]
+    out = [x, x, row(T, W), row(T, E), row(T, E), row(T, D), row(D, E), S, 0, 15]
     for i, bad in ((0, row(1, T, D - 1)), (2, row(T, W + 2)), (3, row(T - 1, E)), (4, row(T, E - 2)), (5, row(T, E)), (6, row(D + 1, E))):
         args = list(out)
         args[i] = bad
         with pytest.raises(RuntimeError, match="mix_out_backward: "):
             H.mix_out_backward(*args)
     back = [row(T, S), row(T, S), row(T, E), row(T, W), x, row(T, E), x, x, row(T, W), row(E, D), row(W, D), row(2, S), row(S // 2),
-            1, T, RMS, row(D), 1e-5, 0]
+            1, T, RMS, row(D), 1e-5, 0, 1023]
     for i, bad in ((0, row(T, S + 2)), (2, row(T + 1, E)), (3, row(T, W + 1)), (6, row(1, T, D + 8)), (8, row(T + 1, W)),
                    (10, row(W, D - 1)), (11, row(2, S + 2)), (16, row(D + 8))):
         args = list(back)
         args[i] = bad
         with pytest.raises(RuntimeError, match="mix_backward: "):
             H.mix_backward(*args)
-    ffn = [x, x, x, row(T, 6), row(T, 6), LN, row(D), row(D), 1e-5, row(6, D), row(D, 6), 0]
+    ffn = [x, x, x, row(T, 6), row(T, 6), LN, row(D), row(D), 1e-5, row(6, D), row(D, 6), 0, 63]
     for i, bad in ((0, row(1, T + 1, D)), (3, row(T, 5)), (4, row(T + 1, 6))):
         args = list(ffn)
         args[i] = bad
         with pytest.raises(RuntimeError, match="ffn_backward: "):
             H.ffn_backward(*args)
     with pytest.raises(RuntimeError, match="swiglu_backward: argument 3 must be"):
-        H.swiglu_backward(x, x, row(T, 6), row(T, 5), row(T, 6), row(6, D), row(6, D), row(D, 6), 0)
+        H.swiglu_backward(x, x, row(T, 6), row(T, 5), row(T, 6), row(6, D), row(6, D), row(D, 6), 0, 31)
 
 
 def test_norm_widths():
@@ -136,7 +136,7 @@ def test_composites_leave_the_interpreter_to_other_threads():
 
     T, D, N = 40000, 512, 512
     args = [torch.randn(T, D), torch.randn(T, D), *(torch.randn(T, N) for _ in range(3)), torch.randn(N, D), torch.randn(N, D),
-            torch.randn(D + 1, N), 0]
+            torch.randn(D + 1, N), 0, 31]
     threads = torch.get_num_threads()
     torch.set_num_threads(1)
     other = threading.Thread(target=count)
