@@ -159,7 +159,8 @@ __global__ __launch_bounds__(kT) void norm_ema_step_kernel(const StepArgs A) {
 // the state as one contiguous 2 KB block; the output sum is finished across the NP lanes.
 // What bounds the step is the state's way through memory, so its loads (and the coefficients') are issued before
 // anything else: the group's moments (every wave for itself, no workgroup barrier, the values kept in registers
-// for the centred second pass) are formed under them.  64 streams x 2048 channels x 16 states: 8.7 us a call, 128 streams 13.2 us
+// for the centred second pass) are formed under them.  64 streams x 2048 channels x 16 states: 8.7 us a call in a
+// loop on one input, 9.5 among inputs that change, 128 streams 13.2 us
 // (13.7 with the moments in front and two workgroup barriers); one stream of 1024 channels: 4.2 us.
 constexpr int kTV = 256;
 // Channel parts a thread has in flight.  Two (the 128 channels of a group at N = 16) need registers that halve the waves

@@ -13,9 +13,9 @@
 //                    the weighted sum of values; the same pass writes the grown key / value cache
 //   token_combine    adds the blocks up, applies the r gate
 // 7 launches per layer where the same step as separate operators took about 45: two layers of 1024 channels, one stream
-// behind 700 cached positions: 17 launches, 107 us of device time and 150 us per token with the host's work, where the
-// operators one by one took 97 launches, 338 us and 1230 us.  40 streams behind 900 positions: 326 us, half of it the
-// copy of the key / value cache (330 MB at 3.8 TB/s).
+// behind 700 cached positions: 19 launches, 111 us of device time and 183 us per token with the host's work, where the
+// operators one by one took 97 launches, 338 us and 1230 us.  40 streams behind 900 positions: 345 us of device time, half
+// of it the copy of the key / value cache (330 MB at 3.5 TB/s).
 #include "common.h"
 
 namespace mega {
