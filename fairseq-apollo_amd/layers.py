@@ -158,7 +158,7 @@ class NormalizedFeedForwardNetwork(nn.Module):
         norm, fc1, fc2 = mods['norm'], mods['fc1'], mods['fc2']
         return (self.hidden_dim % 32 == 0 and _plain(True, fc1) and _plain(False, fc2) and _unhooked((RMSNorm, LayerNorm), norm)
                 and norm_width_ok(norm, x.shape[-1]) and not (self.training and self.dropout_p > 0)
-                and 'weight' in norm._parameters and 'layerscale_weight' in self._parameters
+                and len(norm._parameters) == (1 if type(norm) is RMSNorm else 2) and 'layerscale_weight' in self._parameters
                 and ops._lib.load_host().uniform(x, *norm._parameters.values(), fc1._parameters['weight'], fc1._parameters['bias'],
                                                  fc2._parameters['weight'], self._parameters['layerscale_weight']))
 
@@ -390,6 +390,7 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
         return (ops.token_rows(x, normalised=True) and mask_bytes_ok(padding_mask, x)
                 and _plain(True, v_proj, mx_proj) and _plain(False, h_proj) and 'gamma' in mine and 'beta' in mine
                 and _unhooked((RMSNorm, nn.SiLU, EfficientAttention), act, mods['efficient_attn'])
+                and (type(act) is nn.SiLU or 'weight' in act._parameters)
                 and ops._lib.load_host().uniform(
                     x, *v_proj._parameters.values(), *mx_proj._parameters.values(), *h_proj._parameters.values(),
                     mine['gamma'], mine['beta'], act._parameters.get('weight'))

@@ -352,3 +352,21 @@ def test_replaced_parts_of_a_layer(what):
             assert _rms(got, want) < TOL[torch.bfloat16]
     for layer in (*half.layers, *full.layers):
         assert layer.mega_layer.rel_pos_bias.turned == 6 if what == "rotation" else layer.mega_layer.norm.seen == 3
+
+
+@pytest.mark.parametrize("what", ["bias", "weight", "move_act"])
+def test_norm_values_that_are_no_parameters(what):
+    """A norm's weight or bias kept as a buffer (frozen for good) counts as it does in the operators one by one."""
+    half, full = _model(64, 16, 64, 1, 64, 64, "layernorm", torch.bfloat16, 5)
+    for layer in (*half.layers, *full.layers):
+        norm, name = (layer.mega_layer.move_act, "weight") if what == "move_act" else (layer.nffn.norm, what)
+        value = torch.linspace(-3, 3, 64, device=DEV).to(norm.weight.dtype)
+        delattr(norm, name)
+        norm.register_buffer(name, value)
+    tokens = torch.randint(2, 72, (3, 20), device=DEV)
+    sa, sb = {}, {}
+    with torch.no_grad():
+        half(tokens[:, :19], incremental_state=sa)
+        full(tokens[:, :19], incremental_state=sb)
+        got, want = half(tokens[:, 19:], incremental_state=sa)[0], full(tokens[:, 19:], incremental_state=sb)[0]
+    assert _rms(got, want) < TOL[torch.bfloat16]
