@@ -1,13 +1,15 @@
-// TimestepNorm -> moving-average layer in one kernel (gfx950, bf16 activations, 64 or 128 channels per
+// TimestepNorm -> moving-average layer in one kernel (gfx950, bf16 / fp16 / fp32 activations, 32 to 128 channels per
 // norm group, ndim <= 16, optional padding mask, rows of any length up to 16 blocks): what MovingAverageGatedAttention.forward does at
 // fairseq/modules/moving_average_gated_attention.py:304-315 (x = norm(x); mx = move(x^T)) with
 // TimestepNorm per fairseq/csrc/ops/timestep_norm.cc:218-316 and the layer per
 // fairseq/modules/base_moving_average.py:120-172.  x is read once, xn (the norm's output, which the
 // layer also feeds to v_proj) and y are written once.
 //
-// A workgroup (16 waves) owns one (batch row, 64 channels of a norm group, block of 1024 tokens): whole 128-byte
-// lines of x, xn and -- with [B, D, L] rows -- y.  A group of 128 channels is shared by two workgroups, each of
-// which reads the group's whole lines for the moments.  The blocks are aligned to the end of the row: a row that is
+// A workgroup (16 waves) owns one (batch row, up to 64 channels of a norm group, block of 1024 tokens): with 64
+// channels of 16 bits or 32 of fp32 whole 128-byte lines of x, xn and -- with [B, D, L] rows -- y.  A wider group is
+// shared by two to four workgroups, each of which reads the group's whole lines for the moments.  fp32 / fp16
+// activations take the moving average's products on fp16 operands of two terms, as ema_rows.hip does (fp32 activations
+// as two 16-bit planes of LDS, y back over them as the halves of its words).  The blocks are aligned to the end of the row: a row that is
 // not a whole number of blocks starts inside block 0, behind virtual tokens that count as padding.
 //   1. load the block, per-token moments of the group (packed dot products + DPP), Welford scan over
 //      the block's tokens (padding weighs nothing), publish the block aggregate, fold the earlier blocks'
@@ -59,28 +61,43 @@ namespace mega {
 namespace {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 constexpr int kFW = 16;                       // waves per workgroup
 constexpr int kFT = kFW * 64;                 // threads
-constexpr int kFC = 64;                       // channels per workgroup = per norm group
 constexpr int kFSeg = 1024;                   // tokens per block: 16 segments x 2 tiles x 32
-constexpr int kFCPW = kFC / kFW;              // channels per wave
-constexpr int kFNLD = kFSeg * 8 / kFT;        // 16-byte pieces per thread
-constexpr int kFRow = kFSeg * 2;              // bytes of one channel row in LDS
-constexpr int kFTile = kFC * kFRow + (kFC / 4) * 16;
-constexpr int kFRecW = 4 + kFC * kNS * 2;     // 64-bit words per block record: n, mean, var, pad, end states
+constexpr int kFRow = kFSeg * 2;              // bytes of one channel row of a 16-bit plane in LDS
 constexpr int kFMaxBlocks = 16;               // terms of the look-back sum (earlier blocks + the carried state): one per lane of a row
 constexpr int kFTabs = 2;                     // per-state multiplier tables kept in LDS: q^32, q^64
-constexpr size_t kFSmem = (size_t)kFTile + 2 * kFSeg * 4 + 64 + (size_t)kFTabs * kFC * 128 + kFC * 8;
 
 static_assert(kSEGT == 2, "the fused kernel uses the q^64 segment multipliers of the image");
-static_assert(kFSmem <= 160 * 1024, "LDS of one workgroup");
+
+// What follows from the activation type and the CW channels of a workgroup (PARTS workgroups share a norm group).
+template <typename T, int CW, int PARTS>
+struct Geo {
+  static constexpr bool F16 = !__is_same(T, bf16_t);          // operands of the moving average: fp16 or bf16
+  static constexpr int NX = sizeof(T) == 4 ? 2 : 1;           // 16-bit terms of x, a plane of the tile each
+  static constexpr int NC = F16 ? 2 : kNWC;                   // terms of the C operand
+  static constexpr int VPP = 16 / (int)sizeof(T);             // values of a 16-byte piece
+  static constexpr int PPT = CW / VPP;                        // pieces of a token
+  static constexpr int PL = PPT <= 4 ? 4 : 8;                 // lanes of a token (those beyond PPT idle in the norm)
+  static constexpr int TPR = kFT / PL;                        // tokens per round of loads
+  static constexpr int NLD = kFSeg / TPR;                     // rounds = pieces per thread
+  static constexpr int CPW = CW / kFW;                        // channels per wave
+  static constexpr int GC = CW * PARTS;                       // channels per norm group
+  static constexpr int Plane = CW * kFRow + (CW / 4) * 16;
+  static constexpr int Tile = NX * Plane;
+  static constexpr int RecW = 4 + CW * kNS * 2;               // 64-bit words per block record: n, mean, var, pad, end states
+  static constexpr size_t Smem = (size_t)Tile + 2 * kFSeg * 4 + 64 + (size_t)kFTabs * CW * 128 + CW * 8;
+  static_assert(CW % kFW == 0 && CW <= 64 && PPT <= 8, "one to four channels per wave, at most 128 bytes of a token");
+  static_assert(Smem <= 160 * 1024, "LDS of one workgroup");
+};
 
 struct FusedArgs {
-  const bf16_t* x;       // [B, L, D]
-  bf16_t* xn;            // [B, L, D]
-  bf16_t* y;             // strides (syb, syd, syl): [B, D, L] rows (syl == 1) or [B, L, D] (syd == 1)
+  const void* x;         // [B, L, D]
+  void* xn;              // [B, L, D]
+  void* y;               // strides (syb, syd, syl): [B, D, L] rows (syl == 1) or [B, L, D] (syd == 1)
   int64_t syb, syd, syl;
   const int64_t* prev_count;
   const float* prev_mean;
@@ -97,7 +114,7 @@ struct FusedArgs {
   float* cummean;        // [B, L, G] running mean / rstd of every token, kept for the norm's backward pass; or null
   float* cumrstd;
   TsnHeader* hdr;
-  unsigned long long* rec;   // [B * D / 64][S + 1][kFRecW]; slot S: the caller's carried state, put there by block 0
+  unsigned long long* rec;   // [B * D / CW][S + 1][RecW]; slot S: the caller's carried state, put there by block 0
   int B, L, D, G, N, S;
   int pad;               // S * 1024 - L virtual tokens in front of every row: the block grid ends at the row's last token
   float eps;
@@ -114,9 +131,35 @@ __device__ __forceinline__ uint32_t dpp_u(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
 }
 
-__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
-  bf16x2_t v = {(__bf16)lo, (__bf16)hi};
-  return __builtin_bit_cast(uint32_t, v);
+// a pair of values in the 16-bit operand type, rounded to nearest
+template <bool F16>
+__device__ __forceinline__ uint32_t pack16(float lo, float hi) {
+  if constexpr (F16) {
+    const f16x2_t v = {(_Float16)lo, (_Float16)hi};
+    return __builtin_bit_cast(uint32_t, v);
+  } else {
+    const bf16x2_t v = {(__bf16)lo, (__bf16)hi};
+    return __builtin_bit_cast(uint32_t, v);
+  }
+}
+
+// the two values of a packed pair
+template <bool F16>
+__device__ __forceinline__ float2 unpack16(uint32_t w) {
+  if constexpr (F16) {
+    const f16x2_t v = __builtin_bit_cast(f16x2_t, w);
+    return make_float2((float)v[0], (float)v[1]);
+  } else {
+    return make_float2(__uint_as_float(w << 16), __uint_as_float(w & 0xffff0000u));
+  }
+}
+
+template <bool F16>
+__device__ __forceinline__ f32x4 mma(uint4 a, uint4 b, f32x4 c) {
+  if constexpr (F16)
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
 __device__ __forceinline__ float lane_bcast(float v, int src_lane) {
@@ -183,32 +226,38 @@ __device__ __forceinline__ void load_cmp(const char* base, int tab, uint32_t r_o
   re[3] = __uint_as_float(b.z); im[3] = __uint_as_float(b.w);
 }
 
-// the same from the copy of tables 0..2 in LDS
-__device__ __forceinline__ void lds_cmp(const char* s_tab, int tab, int c, uint32_t r_off, float (&re)[4], float (&im)[4]) {
-  const float4 a = *(const float4*)(s_tab + (tab * kFC + c) * 128 + r_off);
-  const float4 b = *(const float4*)(s_tab + (tab * kFC + c) * 128 + 64 + r_off);
+// the same from the copy of tables 0..1 in LDS; row: table * channels + channel
+__device__ __forceinline__ void lds_cmp(const char* s_tab, int row, uint32_t r_off, float (&re)[4], float (&im)[4]) {
+  const float4 a = *(const float4*)(s_tab + row * 128 + r_off);
+  const float4 b = *(const float4*)(s_tab + row * 128 + 64 + r_off);
   re[0] = a.x; im[0] = a.y; re[1] = a.z; im[1] = a.w;
   re[2] = b.x; im[2] = b.y; re[3] = b.z; im[3] = b.w;
 }
 
-// LOUT 0: y as [B, D, L] rows; 1: y as [B, L, D].  GC: channels per norm group, 64 or 128.  A group of 128 channels
-// is shared by two workgroups: each reads the group's whole lines for the moments (both add in the same order, so
-// both arrive at the same statistics to the last bit) and keeps its own 64 channels.
+// LOUT 0: y as [B, D, L] rows; 1: y as [B, L, D].  CW: channels of a workgroup; PARTS: workgroups that share a norm
+// group: each reads the group's whole lines for the moments (all add in the same order, so all arrive at the same
+// statistics to the last bit) and keeps its own CW channels.
 // STAG: the start of block s is held back by s * A.stagger ticks (an instance of its own: the launches that do not
 // hold anything back run the code without the wait).
-template <int LOUT, int GC, bool STAG>
+template <typename T, int CW, int PARTS, int LOUT, bool STAG>
 __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) {
-  constexpr int kParts = GC / kFC;
-  static_assert(kParts == 1 || kParts == 2, "one or two workgroups per norm group");
+  using Gm = Geo<T, CW, PARTS>;
+  constexpr bool F16 = Gm::F16;
+  constexpr int NX = Gm::NX, NC = Gm::NC, VPP = Gm::VPP, PL = Gm::PL, TPR = Gm::TPR, NLD = Gm::NLD, CPW = Gm::CPW;
+  constexpr bool FINE = NX > 1;              // (merges of running statistics)
+  constexpr int kParts = PARTS, GC = Gm::GC, kPlane = Gm::Plane, kRecW = Gm::RecW;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   char* tile = smem;
-  float* s_gm = (float*)(smem + kFTile);      // [kFSeg] group mean of a token, later the running mean
+  float* s_gm = (float*)(smem + Gm::Tile);    // [kFSeg] group mean of a token, later the running mean
   float* s_gv = s_gm + kFSeg;                 // [kFSeg] group variance, later the running rstd
   float* s_wt = s_gv + kFSeg;                 // [4][4] totals of the four scanning waves
-  float* s_end = s_gm;                        // [kFC][kNS][2] block end states from a zero start (after step 2)
-  char* s_tab = (char*)(s_wt + 16);           // [kFTabs][kFC][kNS] complex: q^32, q^64 of every channel
-  uint2* s_reach = (uint2*)(s_tab + kFTabs * kFC * 128);   // [kFC] reach of every channel's slowest pole
+  float* s_end = s_gm;                        // [CW][kNS][2] block end states from a zero start (after step 2)
+  char* s_tab = (char*)(s_wt + 16);           // [kFTabs][CW][kNS] complex: q^32, q^64 of every channel
+  uint2* s_reach = (uint2*)(s_tab + kFTabs * CW * 128);   // [CW] reach of every channel's slowest pole
 
+  const T* const gx = (const T*)A.x;
+  T* const gxn = (T*)A.xn;
+  T* const gy = (T*)A.y;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // uniform: channel rows and image addresses stay scalar
   const int G = A.G;
@@ -227,20 +276,24 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
     unit = local - b * U;
   }
   const int g = unit / kParts, part = unit - g * kParts;
-  const int cb = g * GC + part * kFC;                    // the workgroup's first channel
+  const int cb = g * GC + part * CW;                     // the workgroup's first channel
   const uint32_t tag = A.hdr->epoch + 1u;
   // The blocks are aligned to the end of the row: block 0 starts `pad` virtual tokens before the first one (they
   // count as padding: no statistics, zeros into the moving average, nothing stored), so the last block ends at the
   // last token and the state handed back is the state after it.
   const int t0 = s * kFSeg - A.pad;
   const bool front = s == 0 && A.pad > 0;                // uniform: this block holds virtual tokens
-  const int piece = tid & 7, tokl = tid >> 3;            // 16-byte piece of the 128-byte line, token 0..127
-  // addresses of the block's lines: a uniform base per 128-token round plus one 32-bit lane offset
+  // 16-byte piece of the token's line, token 0 .. TPR - 1 of a round: the lanes of tokens 2m and 2m + 1 are 8 apart
+  const int lp = tid & (PL - 1);
+  const bool act = Gm::PPT == PL || lp < Gm::PPT;
+  const int piece = act ? lp : 0;
+  const int tokl = PL == 8 ? tid >> 3 : ((tid >> 4) << 2) | ((tid >> 1) & 2) | ((tid >> 3) & 1);
+  // addresses of the block's lines: a uniform base per round of tokens plus one 32-bit lane offset
   const int64_t xblk = ((int64_t)b * A.L + t0) * A.D + (int64_t)cb;      // (negative offsets inside a front block are never used)
-  const uint32_t toff = (uint32_t)tokl * (uint32_t)A.D + piece * 8;
+  const uint32_t toff = (uint32_t)tokl * (uint32_t)A.D + piece * VPP;
   const size_t brow = (size_t)b * G + g;                 // statistics of the group
   const size_t rrow = brow * kParts + part;              // records of the workgroup (its own copy of the statistics too)
-  unsigned long long* const myrec = A.rec + (rrow * (A.S + 1) + s) * kFRecW;
+  unsigned long long* const myrec = A.rec + (rrow * (A.S + 1) + s) * kRecW;
   bool poison = false;
 
   MEGA_FTR(0);
@@ -254,98 +307,165 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
   }
   // ---- everything the norm needs from memory is requested before the block itself
   const Moments prior = {(float)A.prev_count[b], A.prev_mean[brow], A.prev_var[brow]};
-  float gam[8], bet[8];
-  load_params<8>(A.gamma + cb + piece * 8, gam);
-  load_params<8>(A.beta + cb + piece * 8, bet);
-  uint4 xv[kFNLD];
-  uint4 xo[kParts == 2 ? kFNLD : 1];
-  const int64_t oblk = ((int64_t)b * A.L + t0) * A.D + (int64_t)(g * GC + (1 - part) * kFC);
-  // padding flags of the thread's eight tokens (bit k: token k * 128 + tokl): the caller's mask and the virtual
+  float gam[VPP], bet[VPP];
+  load_params<VPP>(A.gamma + cb + piece * VPP, gam);
+  load_params<VPP>(A.beta + cb + piece * VPP, bet);
+  uint4 xv[NLD];
+  uint4 xo[kParts > 1 ? NLD : 1];
+  // the thread's pieces of the lines that begin at element `base`; virtual tokens and idle lanes read as zeros
+  auto load_lines = [&](const int64_t base, uint4 (&v)[NLD]) {
+    if (!front) {
+#pragma unroll
+      for (int k = 0; k < NLD; ++k) {
+        v[k] = Gm::PPT == PL || act ? *(const uint4*)(gx + base + (int64_t)k * TPR * A.D + toff) : make_uint4(0u, 0u, 0u, 0u);
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < NLD; ++k)
+        v[k] = act && k * TPR + tokl >= A.pad ? *(const uint4*)(gx + base + (int64_t)k * TPR * A.D + toff) : make_uint4(0u, 0u, 0u, 0u);
+    }
+  };
+  const int64_t gblk = xblk - (int64_t)part * CW;        // first channel of the group
+  load_lines(xblk, xv);
+  // the other half of the group's lines, for the moments only (the workgroup of that half reads the same lines on
+  // the same XCD)
+  if constexpr (kParts == 2) load_lines(gblk + (1 - part) * CW, xo);
+  // padding flags of the thread's tokens (bit k: token k * TPR + tokl): the caller's mask and the virtual
   // tokens of a front block
   uint32_t mbits = 0;
   if (!front) {
-#pragma unroll
-    for (int k = 0; k < kFNLD; ++k) xv[k] = *(const uint4*)(A.x + xblk + (int64_t)k * 128 * A.D + toff);
-    // the other half of the group's lines, for the moments only (the workgroup of that half reads the same lines on
-    // the same XCD)
-    if (kParts == 2) {
-#pragma unroll
-      for (int k = 0; k < kFNLD; ++k) xo[k] = *(const uint4*)(A.x + oblk + (int64_t)k * 128 * A.D + toff);
-    }
     if (A.mask) {
       const uint8_t* mrow = A.mask + (int64_t)b * A.L + t0 + tokl;
 #pragma unroll
-      for (int k = 0; k < kFNLD; ++k) mbits |= (mrow[k * 128] != 0 ? 1u : 0u) << k;
+      for (int k = 0; k < NLD; ++k) mbits |= (mrow[k * TPR] != 0 ? 1u : 0u) << k;
     }
   } else {
 #pragma unroll
-    for (int k = 0; k < kFNLD; ++k) {
-      const bool real = k * 128 + tokl >= A.pad;
-      const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
-      xv[k] = real ? *(const uint4*)(A.x + xblk + (int64_t)k * 128 * A.D + toff) : zero;
-      if (kParts == 2) xo[k] = real ? *(const uint4*)(A.x + oblk + (int64_t)k * 128 * A.D + toff) : zero;
-      const bool padded = !real || (A.mask && A.mask[(int64_t)b * A.L + t0 + k * 128 + tokl] != 0);
+    for (int k = 0; k < NLD; ++k) {
+      const bool real = k * TPR + tokl >= A.pad;
+      const bool padded = !real || (A.mask && A.mask[(int64_t)b * A.L + t0 + k * TPR + tokl] != 0);
       mbits |= (padded ? 1u : 0u) << k;
     }
   }
 
-  // the per-state multipliers of the group's 64 channels (three lines per channel) go to LDS once
+  // the per-state multipliers of the workgroup's channels (two lines per channel) go to LDS once
   {
     static_assert(kCmpQ32 == 0 && kCmpRS == 1 && kFTabs == 2, "tables 0..1 of the compact slot are staged");
     const char* ibase = (const char*)A.image + (size_t)cb * kImgRowBytes + kSlotCmp * 1024;
 #pragma unroll
     for (int it = 0; it < 2; ++it) {
       const int idx = it * kFT + tid;               // (table, channel, 16-byte piece)
-      if (idx < kFTabs * kFC * 8) {
-        const int t = idx / (kFC * 8), rem = idx - t * (kFC * 8), c = rem >> 3, pc = rem & 7;
-        *(uint4*)(s_tab + (t * kFC + c) * 128 + pc * 16) =
+      if (idx < kFTabs * CW * 8) {
+        const int t = idx / (CW * 8), rem = idx - t * (CW * 8), c = rem >> 3, pc = rem & 7;
+        *(uint4*)(s_tab + (t * CW + c) * 128 + pc * 16) =
             *(const uint4*)(ibase + (size_t)c * kImgRowBytes + t * 128 + pc * 16);
       }
     }
     // and how far every channel's slowest pole reaches (asked for here, used after the norm: no wave waits for it)
-    if (tid < kFC) s_reach[tid] = *(const uint2*)(ibase + (size_t)tid * kImgRowBytes + kCmpReach * 128);
+    if (tid < CW) s_reach[tid] = *(const uint2*)(ibase + (size_t)tid * kImgRowBytes + kCmpReach * 128);
   }
 
   // ---- the caller's carried state joins the records the later look-ups read: slot S of the row, written by block 0
-  if (s == 0 && A.h_in) {
+  if (s == 0 && A.h_in && tid < CW * 16) {
     const int c = tid >> 4, n = tid & 15;
     float2 v = make_float2(0.f, 0.f);
     if (n < A.N) {
       v = *(const float2*)(A.h_in + (((size_t)b * A.D + cb + c) * A.N + n) * 2);
       if (!A.is_complex) v.y = 0.f;
     }
-    unsigned long long* e = A.rec + (rrow * (A.S + 1) + A.S) * kFRecW + 4 + ((size_t)c * kNS + n) * 2;
+    unsigned long long* e = A.rec + (rrow * (A.S + 1) + A.S) * kRecW + 4 + ((size_t)c * kNS + n) * 2;
     put_rec(e, tagged(__float_as_uint(v.x), tag));
     put_rec(e + 1, tagged(__float_as_uint(v.y), tag));
   }
 
-  // ---- moments of every token's group (64 channels = the 8 lanes of a line)
-#pragma unroll
-  for (int k = 0; k < kFNLD; ++k) {
-    const uint32_t w[4] = {xv[k].x, xv[k].y, xv[k].z, xv[k].w};
-    float sm = 0.f, sq = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      sm = dot2_ones<bf16_t>(w[i], sm);
-      sq = dot2_self<bf16_t>(w[i], sq);
+  // ---- moments of every token's group (the PL lanes of a line)
+  auto keep_moments = [&](const int k, const float m, const float v) {
+    if (lp == 0) {
+      const bool pad = (mbits >> k) & 1u;
+      s_gm[k * TPR + tokl] = pad ? 0.f : m;                         // (whatever x holds there)
+      s_gv[k * TPR + tokl] = pad ? -1.f : v;                        // a negative variance marks padding
     }
-    if (kParts == 2) {
-      const uint32_t wo[4] = {xo[k].x, xo[k].y, xo[k].z, xo[k].w};
-      float so = 0.f, qo = 0.f;
+  };
+  if constexpr (NX == 1) {
+    // sum and sum of squares by packed dot products; E[x^2] - mean^2 in fp32 resolves more than the inputs carry
+#pragma unroll
+    for (int k = 0; k < NLD; ++k) {
+      const uint32_t w[4] = {xv[k].x, xv[k].y, xv[k].z, xv[k].w};
+      float sm = 0.f, sq = 0.f;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        so = dot2_ones<bf16_t>(wo[i], so);
-        qo = dot2_self<bf16_t>(wo[i], qo);
+        sm = dot2_ones<T>(w[i], sm);
+        sq = dot2_self<T>(w[i], sq);
       }
-      // lower half first in both workgroups
-      sm = part == 0 ? sm + so : so + sm;
-      sq = part == 0 ? sq + qo : qo + sq;
+      if constexpr (kParts == 2) {
+        const uint32_t wo[4] = {xo[k].x, xo[k].y, xo[k].z, xo[k].w};
+        float so = 0.f, qo = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          so = dot2_ones<T>(wo[i], so);
+          qo = dot2_self<T>(wo[i], qo);
+        }
+        // lower half first in both workgroups
+        sm = part == 0 ? sm + so : so + sm;
+        sq = part == 0 ? sq + qo : qo + sq;
+      }
+      const float m = group_sum<PL>(sm) * (1.0f / GC);
+      const float v = fmaxf(group_sum<PL>(sq) * (1.0f / GC) - m * m, 0.f);
+      keep_moments(k, m, v);
     }
-    const float m = group_sum<8>(sm) * (1.0f / GC);
-    const float v = fmaxf(group_sum<8>(sq) * (1.0f / GC) - m * m, 0.f);
-    if (piece == 0) {
-      s_gm[k * 128 + tokl] = m;
-      s_gv[k * 128 + tokl] = ((mbits >> k) & 1u) ? -1.f : v;        // a negative variance marks padding
+  } else {
+    // fp32: the mean of a part first, then its squares around that mean; the later parts of a group (in the order of
+    // their channels) by how far their means lie from the first part's
+    static_assert(Gm::PPT == PL, "every lane of a line holds values");
+    float gmean[NLD], gdist[NLD], gvar[NLD];
+    auto add_part = [&](const int i, const uint4 (&v)[NLD]) {     // i: parts before this one
+#pragma unroll
+      for (int k = 0; k < NLD; ++k) {
+        const float f[4] = {__uint_as_float(v[k].x), __uint_as_float(v[k].y), __uint_as_float(v[k].z), __uint_as_float(v[k].w)};
+        const float m = group_sum<PL>((f[0] + f[1]) + (f[2] + f[3])) * (1.0f / CW);
+        float q = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float d = f[e] - m;
+          q = fmaf(d, d, q);
+        }
+        q = group_sum<PL>(q);
+        if (i == 0) {
+          gmean[k] = m;
+          gdist[k] = 0.f;
+          gvar[k] = q;
+        } else {
+          const float d = m - gmean[k];
+          gdist[k] += d;
+          gvar[k] += fmaf(d * d, (float)CW, q);
+        }
+      }
+    };
+    if constexpr (kParts == 1) {
+      add_part(0, xv);
+    } else if constexpr (kParts == 2) {
+      if (part == 0) {
+        add_part(0, xv);
+        add_part(1, xo);
+      } else {
+        add_part(0, xo);
+        add_part(1, xv);
+      }
+    } else {
+#pragma unroll 1
+      for (int i = 0; i < kParts; ++i) {       // (the workgroup's own part again: one order for all, and registers for one)
+        load_lines(gblk + i * CW, xo);
+        add_part(i, xo);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < NLD; ++k) {
+      if constexpr (kParts == 1) {
+        keep_moments(k, gmean[k], gvar[k] * (1.0f / GC));
+      } else {
+        const float shift = gdist[k] * (1.0f / kParts);
+        keep_moments(k, gmean[k] + shift, fmaxf(fmaf(-shift, shift, gvar[k] * (1.0f / GC)), 0.f));
+      }
     }
   }
   __syncthreads();
@@ -362,10 +482,10 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
     pref[0] = st;
 #pragma unroll
     for (int u = 1; u < 4; ++u) {
-      st = merge(st, Moments{vv[u] >= 0.f ? 1.f : 0.f, mm[u], fmaxf(vv[u], 0.f)});
+      st = merge<FINE>(st, Moments{vv[u] >= 0.f ? 1.f : 0.f, mm[u], fmaxf(vv[u], 0.f)});
       pref[u] = st;
     }
-    const Moments inc = row_scan(st);
+    const Moments inc = row_scan<FINE>(st);
     const Moments exc = dpp_m<0x111>(inc);
     Moments acc = {0.f, 0.f, 0.f}, rp = {0.f, 0.f, 0.f};
 #pragma unroll
@@ -374,9 +494,9 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
                          __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, inc.mean), 16 * r + 15)),
                          __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, inc.var), 16 * r + 15))};
       if ((lane >> 4) == r) rp = acc;
-      acc = merge(acc, t);
+      acc = merge<FINE>(acc, t);
     }
-    lane_exc = merge(rp, exc);
+    lane_exc = merge<FINE>(rp, exc);
     if (lane == 0) {
       s_wt[wave * 4] = acc.n;
       s_wt[wave * 4 + 1] = acc.mean;
@@ -389,7 +509,7 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       if (w == wave) wpre = tot;
-      tot = merge(tot, Moments{s_wt[w * 4], s_wt[w * 4 + 1], s_wt[w * 4 + 2]});
+      tot = merge<FINE>(tot, Moments{s_wt[w * 4], s_wt[w * 4 + 1], s_wt[w * 4 + 2]});
     }
     if (wave == 0 && lane == 0 && !(A.lb.withhold_first && s == 0)) {
       put_rec(myrec, tagged((uint32_t)tot.n, tag));
@@ -400,7 +520,7 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
     // earlier blocks of this (row, group): lane i fetches block i's aggregate
     Moments accp = {0.f, 0.f, 0.f};
     if (s > 0) {
-      const unsigned long long* rp = A.rec + (rrow * (A.S + 1) + (lane < s ? lane : s - 1)) * kFRecW;
+      const unsigned long long* rp = A.rec + (rrow * (A.S + 1) + (lane < s ? lane : s - 1)) * kRecW;
       unsigned long long w0, w1, w2;
       uint32_t spins = 0;
       for (;;) {
@@ -419,20 +539,20 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
         const Moments t = {(float)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)w0, i),
                            __builtin_bit_cast(float, __builtin_amdgcn_readlane((int)(uint32_t)w1, i)),
                            __builtin_bit_cast(float, __builtin_amdgcn_readlane((int)(uint32_t)w2, i))};
-        accp = merge(accp, t);
+        accp = merge<FINE>(accp, t);
       }
     }
     MEGA_FTR(3);
-    Moments carry = merge(prior, accp);
+    Moments carry = merge<FINE>(prior, accp);
     if (poison) {
       carry.mean = __builtin_nanf("");
       if (lane == 0) report_give_up(A.hdr, A.lb.status);
     }
-    const Moments base = merge(carry, merge(wpre, lane_exc));
+    const Moments base = merge<FINE>(carry, merge<FINE>(wpre, lane_exc));
     Moments full = base;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      full = merge(base, pref[u]);
+      full = merge<FINE>(base, pref[u]);
       const float rstd = __builtin_amdgcn_rsqf(full.var + A.eps);
       s_gm[wave * 256 + lane * 4 + u] = full.mean;
       s_gv[wave * 256 + lane * 4 + u] = rstd;
@@ -459,83 +579,107 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
   // as the previous channel's have been used, and travel under the rest of that channel's work)
   const uint32_t loff0 = (uint32_t)lane * 16;
   const uint32_t koff0 = (uint32_t)(((lane & 15) - 8 * (lane >> 4) + 24) * 16);
-  auto load_p = [&](const int c, bf16x8 (&P)[kNWP][2]) {
+  constexpr int kSP = F16 ? kSlotP16 : kSlotP, kSC = F16 ? kSlotC16 : kSlotC;
+  auto load_p = [&](const int c, uint4 (&P)[kNWP][2]) {
     const char* img = (const char*)A.image + (size_t)(cb + c) * kImgRowBytes;
     uint32_t loff = loff0;
     asm volatile("" : "+v"(loff));
 #pragma unroll
     for (int w = 0; w < kNWP; ++w)
 #pragma unroll
-      for (int mb = 0; mb < 2; ++mb) P[w][mb] = __builtin_bit_cast(bf16x8, img_slot(img, kSlotP + 2 * w + mb, loff));
+      for (int mb = 0; mb < 2; ++mb) P[w][mb] = img_slot(img, kSP + 2 * w + mb, loff);
   };
-  auto load_kc = [&](const int c, bf16x8 (&K)[kNWK][2], bf16x8 (&C)[kNWC][2]) {
+  auto load_kc = [&](const int c, uint4 (&K)[kNWK][2], uint4 (&C)[NC][2]) {
     const char* img = (const char*)A.image + (size_t)(cb + c) * kImgRowBytes;
     uint32_t loff = loff0;
     asm volatile("" : "+v"(loff));
-    // K from the slot that holds each distinct vector once: 7 lines per term leave the cache instead of 16
-    uint32_t koff = koff0;
-    asm volatile("" : "+v"(koff));
+    if constexpr (F16) {
 #pragma unroll
-    for (int w = 0; w < kNWK; ++w)
+      for (int w = 0; w < kNWK; ++w)
 #pragma unroll
-      for (int mb = 0; mb < 2; ++mb)
-        K[w][mb] = __builtin_bit_cast(bf16x8, *(const uint4*)(img + ((kSlotKT + w) * 1024 + mb * 256) + koff));
+        for (int mb = 0; mb < 2; ++mb) K[w][mb] = img_slot(img, kSlotK16 + 2 * w + mb, loff);
+    } else {
+      // K from the slot that holds each distinct vector once: 7 lines per term leave the cache instead of 16
+      uint32_t koff = koff0;
+      asm volatile("" : "+v"(koff));
 #pragma unroll
-    for (int w = 0; w < kNWC; ++w)
+      for (int w = 0; w < kNWK; ++w)
 #pragma unroll
-      for (int mb = 0; mb < 2; ++mb) C[w][mb] = __builtin_bit_cast(bf16x8, img_slot(img, kSlotC + 2 * w + mb, loff));
+        for (int mb = 0; mb < 2; ++mb) K[w][mb] = *(const uint4*)(img + ((kSlotKT + w) * 1024 + mb * 256) + koff);
+    }
+#pragma unroll
+    for (int w = 0; w < NC; ++w)
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb) C[w][mb] = img_slot(img, kSC + 2 * w + mb, loff);
   };
   // the P operand of the wave's first channel travels under the normalisation
-  bf16x8 Pa[kNWP][2];
+  uint4 Pa[kNWP][2];
   load_p(wave, Pa);
 
-  // ---- normalise from registers and stage xn (bf16, as the layer sees it) transposed: channel rows of 16
-  // segments x 128 bytes, 16-byte chunk c of segment j at chunk c ^ (j >> 1) (the 16 lanes of a matrix-core
-  // operand load then cover all banks); the lanes of tokens (2m, 2m+1) swap halves so that each writes dwords
-  // (even token | odd token << 16) of four channels
+  // ---- normalise from registers and stage xn (as the layer sees it) transposed: channel rows of 16 segments x
+  // 128 bytes, 16-byte chunk c of segment j at chunk c ^ (j >> 1) (the 16 lanes of a matrix-core operand load then
+  // cover all banks); the lanes of tokens (2m, 2m+1) swap halves so that each writes dwords (even token | odd token
+  // << 16) of four channels.  fp32: the two 16-bit terms of x are the halves, a plane each.
   {
     const int odd = tokl & 1;
     const uint32_t sel_lo = odd ? 0x01000504u : 0x05040100u;
     const uint32_t sel_hi = odd ? 0x03020706u : 0x07060302u;
     const int tl = tokl & ~1;
-    char* wbase = tile + row_base(piece * 8 + odd * 4) + (tl >> 6) * 128 + ((tl & 7) >> 1) * 4;
+    char* wbase = tile + (NX == 1 ? row_base(piece * 8 + odd * 4) : odd * kPlane + row_base(piece * 4)) + (tl >> 6) * 128 +
+                  ((tl & 7) >> 1) * 4;
     const int c8 = (tl & 63) >> 3;
     // weight + 1 = 1 and bias = 0 for every channel of the group (the module's initial values): the affine step
-    // is skipped, one multiply-add per element less (a wave sees all 64 channels, so the branch is uniform)
+    // is skipped, one multiply-add per element less (a wave sees all channels, so the branch is uniform)
     bool plain = true;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) plain = plain && gam[i] == 1.f && bet[i] == 0.f;
+    for (int i = 0; i < VPP; ++i) plain = plain && gam[i] == 1.f && bet[i] == 0.f;
     const bool ident = __all(plain);
     auto stage = [&](auto IDENT, auto MASKED, auto FRONT) {
 #pragma unroll
-    for (int k = 0; k < kFNLD; ++k) {
-      const int tok = k * 128 + tokl;
+    for (int k = 0; k < NLD; ++k) {
+      const int tok = k * TPR + tokl;
       const float m = s_gm[tok], r = s_gv[tok];
       const float mr = m * r;
       const uint32_t w[4] = {xv[k].x, xv[k].y, xv[k].z, xv[k].w};
-      uint32_t o[4];
+      uint32_t o[4], h[4];               // what leaves as xn, and the halves the moving average takes
+      const bool pad = decltype(MASKED)::value && ((mbits >> k) & 1u);      // padding leaves as zeros, whatever x holds there
+      if constexpr (NX == 1) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float lo = fmaf(__uint_as_float(w[i] << 16), r, -mr);
-        const float hi = fmaf(__uint_as_float(w[i] & 0xffff0000u), r, -mr);
-        o[i] = decltype(IDENT)::value ? pack_bf16(lo, hi)
-                                      : pack_bf16(fmaf(lo, gam[2 * i], bet[2 * i]), fmaf(hi, gam[2 * i + 1], bet[2 * i + 1]));
-      }
-      if (decltype(MASKED)::value) {
-        const bool pad = (mbits >> k) & 1u;                 // padding leaves as zeros, whatever x holds there
+        for (int i = 0; i < 4; ++i) {
+          const float2 v = unpack16<F16>(w[i]);
+          const float lo = fmaf(v.x, r, -mr), hi = fmaf(v.y, r, -mr);
+          o[i] = decltype(IDENT)::value ? pack16<F16>(lo, hi)
+                                        : pack16<F16>(fmaf(lo, gam[2 * i], bet[2 * i]), fmaf(hi, gam[2 * i + 1], bet[2 * i + 1]));
+          o[i] = pad ? 0u : o[i];
+          h[i] = o[i];
+        }
+      } else {
+        float f[4], lo[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = pad ? 0u : o[i];
+        for (int i = 0; i < 4; ++i) {
+          f[i] = fmaf(__uint_as_float(w[i]), r, -mr);
+          if (!decltype(IDENT)::value) f[i] = fmaf(f[i], gam[i], bet[i]);
+          f[i] = pad ? 0.f : f[i];
+          o[i] = __float_as_uint(f[i]);
+          lo[i] = f[i] - (float)(_Float16)f[i];
+        }
+        h[0] = pack16<true>(f[0], f[1]);
+        h[1] = pack16<true>(f[2], f[3]);
+        h[2] = pack16<true>(lo[0], lo[1]);
+        h[3] = pack16<true>(lo[2], lo[3]);
       }
-      if (!decltype(FRONT)::value || k * 128 + tokl >= A.pad)              // virtual tokens have no place in xn
-        store_stream((uint4*)(A.xn + xblk + (int64_t)k * 128 * A.D + toff), make_uint4(o[0], o[1], o[2], o[3]));
-      const uint32_t s0 = odd ? o[0] : o[2], s1 = odd ? o[1] : o[3];
+      if (act && (!decltype(FRONT)::value || tok >= A.pad))                // virtual tokens have no place in xn
+        store_stream((uint4*)(gxn + xblk + (int64_t)k * TPR * A.D + toff), make_uint4(o[0], o[1], o[2], o[3]));
+      const uint32_t s0 = odd ? h[0] : h[2], s1 = odd ? h[1] : h[3];
       const uint32_t r0 = dpp_u<0x128>(s0), r1 = dpp_u<0x128>(s1);       // row_ror:8 = the partner token's lane
-      const uint32_t m0 = odd ? o[2] : o[0], m1 = odd ? o[3] : o[1];
-      char* wp = wbase + (2 * k) * 128 + ((c8 ^ k) << 4);
-      *(uint32_t*)(wp) = __builtin_amdgcn_perm(r0, m0, sel_lo);
-      *(uint32_t*)(wp + kFRow) = __builtin_amdgcn_perm(r0, m0, sel_hi);
-      *(uint32_t*)(wp + 2 * kFRow) = __builtin_amdgcn_perm(r1, m1, sel_lo);
-      *(uint32_t*)(wp + 3 * kFRow) = __builtin_amdgcn_perm(r1, m1, sel_hi);
+      const uint32_t m0 = odd ? h[2] : h[0], m1 = odd ? h[3] : h[1];
+      if (act) {
+        char* wp = wbase + k * (TPR * 2) + ((c8 ^ ((k * TPR + tl) >> 7)) << 4);
+        *(uint32_t*)(wp) = __builtin_amdgcn_perm(r0, m0, sel_lo);
+        *(uint32_t*)(wp + kFRow) = __builtin_amdgcn_perm(r0, m0, sel_hi);
+        *(uint32_t*)(wp + 2 * kFRow) = __builtin_amdgcn_perm(r1, m1, sel_lo);
+        *(uint32_t*)(wp + 3 * kFRow) = __builtin_amdgcn_perm(r1, m1, sel_hi);
+      }
     }
     };
     if (front) {
@@ -567,9 +711,9 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
   const int nterms = s + (A.h_in ? 1 : 0);
   const uint32_t roff0 = (uint32_t)r * 16;
   // how far the channels' slowest poles reach (figures of the operand image, uniform per wave and channel)
-  int nsteps[kFCPW], nlook[kFCPW];
+  int nsteps[CPW], nlook[CPW];
 #pragma unroll
-  for (int i = 0; i < kFCPW; ++i) {
+  for (int i = 0; i < CPW; ++i) {
     const uint2 rw = s_reach[wave + kFW * i];
     nsteps[i] = __builtin_amdgcn_readfirstlane((int)rw.x);
     nlook[i] = __builtin_amdgcn_readfirstlane((int)rw.y);
@@ -583,12 +727,26 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
     asm volatile("" ::: "memory");
     __builtin_amdgcn_wave_barrier();
     const char* rb = tile + row_base(c);
-    bf16_t* yr = A.y + (int64_t)b * A.syb + (int64_t)(cb + c) * A.syd + t0;
+    T* yr = gy + (int64_t)b * A.syb + (int64_t)(cb + c) * A.syd + t0;
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const int q = k * 64 + lane;                 // 16-byte chunk of the row: segment q >> 3, chunk q & 7
-      const uint4 v = *(const uint4*)(rb + (q >> 3) * 128 + (((q & 7) ^ (q >> 4)) << 4));
-      if (q * 8 >= -t0) store_stream((uint4*)(yr + q * 8), v);      // (a front block: the row begins inside it, at a multiple of 8)
+      const char* at = rb + (q >> 3) * 128 + (((q & 7) ^ (q >> 4)) << 4);
+      const uint4 v = *(const uint4*)at;
+      // (a front block: the row begins inside it, at a multiple of 8)
+      if constexpr (NX == 1) {
+        if (q * 8 >= -t0) store_stream((uint4*)(yr + q * 8), v);
+      } else {
+        const uint4 u = *(const uint4*)(at + kPlane);          // the low halves of the same eight values
+        if (q * 8 >= -t0) {
+          store_stream((uint4*)(yr + q * 8),
+                       make_uint4(__builtin_amdgcn_perm(v.x, u.x, 0x05040100u), __builtin_amdgcn_perm(v.x, u.x, 0x07060302u),
+                                  __builtin_amdgcn_perm(v.y, u.y, 0x05040100u), __builtin_amdgcn_perm(v.y, u.y, 0x07060302u)));
+          store_stream((uint4*)(yr + q * 8 + 4),
+                       make_uint4(__builtin_amdgcn_perm(v.z, u.z, 0x05040100u), __builtin_amdgcn_perm(v.z, u.z, 0x07060302u),
+                                  __builtin_amdgcn_perm(v.w, u.w, 0x05040100u), __builtin_amdgcn_perm(v.w, u.w, 0x07060302u)));
+        }
+      }
     }
   };
 
@@ -596,16 +754,23 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
   // tile), scanned across the row by doubling: E becomes the state after segment j with the block started from
   // zero.  A step over d segments is skipped (uniform branch) when |q|^(64 d) < 2^-24 for every state of the
   // channel: what it would add is below fp32 resolution.
-  auto segment_scan = [&](const int c, const int steps, const bf16x8 (&P)[kNWP][2], const bf16x8& X0, const bf16x8& X1,
-                          const float (&Qr)[4], const float (&Qi)[4], float (&Er)[4], float (&Ei)[4], float (&Fr)[4],
-                          float (&Fi)[4], const uint32_t roff) {
+  auto segment_scan = [&](const int c, const int steps, const uint4 (&P)[kNWP][2], const char* row, const float (&Qr)[4], const float (&Qi)[4],
+                          float (&Er)[4], float (&Ei)[4], float (&Fr)[4], float (&Fi)[4], const uint32_t roff) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
+      const char* at = row + (((4 * t + r) ^ (j >> 1)) << 4);
+      const uint4 X = *(const uint4*)at;
       f32x4 S0 = {0.f, 0.f, 0.f, 0.f}, S1 = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (NX > 1) {                     // (the small terms of a sum first)
+        const uint4 Xl = *(const uint4*)(at + kPlane);
+        S0 = mma<F16>(P[0][0], Xl, S0);
+        S1 = mma<F16>(P[0][1], Xl, S1);
+      }
 #pragma unroll
       for (int w = 0; w < kNWP; ++w) {
-        S0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(P[w][0], t == 0 ? X0 : X1, S0, 0, 0, 0);
-        S1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(P[w][1], t == 0 ? X0 : X1, S1, 0, 0, 0);
+        const int v = F16 ? kNWP - 1 - w : w;
+        S0 = mma<F16>(P[v][0], X, S0);
+        S1 = mma<F16>(P[v][1], X, S1);
       }
       const float sr[4] = {S0[0], S0[2], S1[0], S1[2]};
       const float si[4] = {S0[1], S0[3], S1[1], S1[3]};
@@ -622,7 +787,7 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
     }
     if (steps > 0) {
       float Rr[4], Ri[4], R2r[4], R2i[4];
-      lds_cmp(s_tab, kCmpRS, c, roff, Rr, Ri);
+      lds_cmp(s_tab, kCmpRS * CW + c, roff, Rr, Ri);
       scan_step<0x111>(Er, Ei, Rr, Ri);
       if (steps > 1) {
         csquare(Rr, Ri, R2r, R2i);
@@ -645,41 +810,41 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
   // it goes before the other waves' phase B
   __builtin_amdgcn_s_setprio(2);
 #pragma unroll
-  for (int i = 0; i < kFCPW; ++i) {
+  for (int i = 0; i < CPW; ++i) {
     const int c = wave + kFW * i;
     uint32_t roff = roff0;
     asm volatile("" : "+v"(roff));
     float Qr[4], Qi[4];
-    lds_cmp(s_tab, kCmpQ32, c, roff, Qr, Qi);
+    lds_cmp(s_tab, kCmpQ32 * CW + c, roff, Qr, Qi);
     const char* row = tile + row_base(c) + j * 128;
-    const bf16x8 X0 = *(const bf16x8*)(row + (((r) ^ (j >> 1)) << 4));
-    const bf16x8 X1 = *(const bf16x8*)(row + (((4 + r) ^ (j >> 1)) << 4));
     float Er[4], Ei[4], Fr[4], Fi[4];
-    segment_scan(c, nsteps[i], Pa, X0, X1, Qr, Qi, Er, Ei, Fr, Fi, roff);
+    segment_scan(c, nsteps[i], Pa, row, Qr, Qi, Er, Ei, Fr, Fi, roff);
     if (j == 15) {
       *(float4*)(s_end + (c * kNS + 2 * r) * 2) = make_float4(Er[0], Ei[0], Er[1], Ei[1]);
       *(float4*)(s_end + (c * kNS + 8 + 2 * r) * 2) = make_float4(Er[2], Ei[2], Er[3], Ei[3]);
     }
     // the next channel's P operand (after the last channel: the first one's again, for phase B)
     __builtin_amdgcn_sched_barrier(0);
-    load_p(i + 1 < kFCPW ? wave + kFW * (i + 1) : wave, Pa);
+    load_p(i + 1 < CPW ? wave + kFW * (i + 1) : wave, Pa);
     __builtin_amdgcn_sched_barrier(0);
     MEGA_FTR(6 + i);
   }
   if (!last_block && !(A.lb.withhold_first && s == 0)) {
-    // the wave's four channels x 16 states x (re, im) = 128 words: two per lane
+    // the wave's channels x 16 states x (re, im): two words per lane (four channels: every lane)
     asm volatile("" ::: "memory");
     __builtin_amdgcn_wave_barrier();
-    const int cp = wave + kFW * (lane >> 4);
-    const float2 v = *(const float2*)(s_end + (cp * kNS + (lane & 15)) * 2);
-    unsigned long long* e = myrec + 4 + ((size_t)cp * kNS + (lane & 15)) * 2;
-    put_rec(e, tagged(__float_as_uint(v.x), tag));
-    put_rec(e + 1, tagged(__float_as_uint(v.y), tag));
+    if (CPW == 4 || (lane >> 4) < CPW) {
+      const int cp = wave + kFW * (lane >> 4);
+      const float2 v = *(const float2*)(s_end + (cp * kNS + (lane & 15)) * 2);
+      unsigned long long* e = myrec + 4 + ((size_t)cp * kNS + (lane & 15)) * 2;
+      put_rec(e, tagged(__float_as_uint(v.x), tag));
+      put_rec(e + 1, tagged(__float_as_uint(v.y), tag));
+    }
   }
   __builtin_amdgcn_s_setprio(0);
 
   // the operands of phase B's first channel travel under the wait for the earlier blocks
-  bf16x8 Ka[kNWK][2], Ca[kNWC][2];
+  uint4 Ka[kNWK][2], Ca[NC][2];
   load_kc(wave, Ka, Ca);
   float Jr[4] = {0.f, 0.f, 0.f, 0.f}, Ji[4] = {0.f, 0.f, 0.f, 0.f};
   auto load_j = [&](const int c) {
@@ -691,25 +856,27 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
   load_j(wave);
 
   // ---- start state of the block: h_start = sum_{d >= 0} (q^1024)^d E_{s-1-d}, E_{-1} being the caller's carried
-  // state (slot S of the row's records).  Lane (j, r) works for channel wave + 16 (j >> 2) and takes the terms
-  // d = (j & 3) + 4 k; the four lanes of a quad add up.
+  // state (slot S of the row's records).  Lane (j, r) works for channel wave + 16 (j >> 2) (idle when the wave has no
+  // such channel) and takes the terms d = (j & 3) + 4 k; the four lanes of a quad add up.
+  const int ci = j >> 2;
+  const bool cown = CPW == 4 || ci < CPW;
+  const int cl = wave + kFW * (cown ? ci : 0);
   float Cr[4] = {0.f, 0.f, 0.f, 0.f}, Ci[4] = {0.f, 0.f, 0.f, 0.f};
   if (nterms > 0) {
-    const int cl = wave + kFW * (j >> 2);
     const int chl = cb + cl;
     int look = 0;                                  // blocks back that still reach this lane's channel
 #pragma unroll
-    for (int i = 0; i < kFCPW; ++i) look = (j >> 2) == i ? nlook[i] : look;
+    for (int i = 0; i < CPW; ++i) look = ci == i ? nlook[i] : look;
     const char* wimg = (const char*)A.image + (size_t)chl * kImgRowBytes;
     int maxlook = 0;
 #pragma unroll
-    for (int i = 0; i < kFCPW; ++i) maxlook = nlook[i] > maxlook ? nlook[i] : maxlook;
+    for (int i = 0; i < CPW; ++i) maxlook = nlook[i] > maxlook ? nlook[i] : maxlook;
     const int nrounds = nterms < maxlook ? nterms : maxlook;
     for (int d0 = 0; d0 < nrounds; d0 += 4) {
       const int d = d0 + (j & 3);
       const bool have = d < nterms && d < look;
       const int slot = have ? (d < s ? s - 1 - d : A.S) : 0;
-      const unsigned long long* e = A.rec + (rrow * (A.S + 1) + slot) * kFRecW + 4 + (size_t)cl * kNS * 2 + 4 * r;
+      const unsigned long long* e = A.rec + (rrow * (A.S + 1) + slot) * kRecW + 4 + (size_t)cl * kNS * 2 + 4 * r;
       float Wr[4], Wi[4];
       load_c4(wimg, kSlotRWJ, (uint32_t)(((r << 4) | (have ? d : 0)) * 16), Wr, Wi);      // (q^1024)^d
       unsigned long long w[8];
@@ -751,8 +918,7 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
   // first returns the state after its last token: end state from a zero start + (q^1024) h_start
   asm volatile("" ::: "memory");
   __builtin_amdgcn_wave_barrier();
-  if (last_block && A.h_out && (j & 3) == 0) {
-    const int cl = wave + kFW * (j >> 2);
+  if (last_block && A.h_out && (j & 3) == 0 && cown) {
     const int ch = cb + cl;
     float Rr[4], Ri[4];
     load_cmp((const char*)A.image + (size_t)ch * kImgRowBytes, kCmpRW, roff0, Rr, Ri);
@@ -768,8 +934,7 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
   }
   asm volatile("" ::: "memory");
   __builtin_amdgcn_wave_barrier();
-  if ((j & 3) == 0) {
-    const int cl = wave + kFW * (j >> 2);
+  if ((j & 3) == 0 && cown) {
     *(float4*)(s_end + (cl * kNS + 2 * r) * 2) = make_float4(Cr[0], Ci[0], Cr[1], Ci[1]);
     *(float4*)(s_end + (cl * kNS + 8 + 2 * r) * 2) = make_float4(Cr[2], Ci[2], Cr[3], Ci[3]);
   }
@@ -783,29 +948,27 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
   // one would show; at a segment's second tile h = q^32 h + F), bf16,
   // back into LDS over x, and out as whole rows.
 #pragma unroll
-  for (int i = 0; i < kFCPW; ++i) {
+  for (int i = 0; i < CPW; ++i) {
     const int c = wave + kFW * i;
     // One bf16 term for the states leaves an error of 2^-9 of sum |gamma q h| at the first tokens of every tile.  It
     // shows where the states dwarf y (slow poles: |q|^128 >= 2^-24 for some state of the channel), in layers of few
     // states, whose rounding errors do not average out in the sum over the states, and in real-valued layers, whose
     // input weights alternate in sign along the states so that the states cancel by construction: those take a
-    // second term (hi + lo).  MEGA_FUSED_TWO_TERMS=1 gives every channel the second term (+ 0.7 us at the headline
+    // second term (hi + lo), and fp16 operands always do.  MEGA_FUSED_TWO_TERMS=1 gives every channel the second term (+ 0.7 us at the headline
     // shape).
-    const bool two_terms = MEGA_FUSED_TWO_TERMS || nsteps[i] >= 2 || A.N <= 8 || !A.is_complex;
+    const bool two_terms = F16 || MEGA_FUSED_TWO_TERMS || nsteps[i] >= 2 || A.N <= 8 || !A.is_complex;
     uint32_t roff = roff0;
     asm volatile("" : "+v"(roff));
     char* row = tile + row_base(c) + j * 128;
-    const bf16x8 X0 = *(const bf16x8*)(row + (((r) ^ (j >> 1)) << 4));
-    const bf16x8 X1 = *(const bf16x8*)(row + (((4 + r) ^ (j >> 1)) << 4));
     float hr[4], hi[4], Fr[4], Fi[4];
     {
       float Qr[4], Qi[4];
-      lds_cmp(s_tab, kCmpQ32, c, roff, Qr, Qi);
-      segment_scan(c, nsteps[i], Pa, X0, X1, Qr, Qi, hr, hi, Fr, Fi, roff);
+      lds_cmp(s_tab, kCmpQ32 * CW + c, roff, Qr, Qi);
+      segment_scan(c, nsteps[i], Pa, row, Qr, Qi, hr, hi, Fr, Fi, roff);
     }
     MEGA_FTR2(0);
     __builtin_amdgcn_sched_barrier(0);
-    if (i + 1 < kFCPW) load_p(wave + kFW * (i + 1), Pa);
+    if (i + 1 < CPW) load_p(wave + kFW * (i + 1), Pa);
     __builtin_amdgcn_sched_barrier(0);
     {
       const float4 b0 = *(const float4*)(s_end + (c * kNS + 2 * r) * 2);
@@ -819,46 +982,65 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
       }
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (i + 1 < kFCPW) load_j(wave + kFW * (i + 1));
+    if (i + 1 < CPW) load_j(wave + kFW * (i + 1));
     __builtin_amdgcn_sched_barrier(0);
     MEGA_FTR2(1);
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       asm volatile("" ::: "memory");              // x again from LDS: cheaper than eight registers across the scan
-      const bf16x8 X = *(const bf16x8*)(row + (((4 * t + r) ^ (j >> 1)) << 4));
+      const char* xat = row + (((4 * t + r) ^ (j >> 1)) << 4);
+      const uint4 X = *(const uint4*)xat;
       f32x4 Y0 = {0.f, 0.f, 0.f, 0.f}, Y1 = {0.f, 0.f, 0.f, 0.f};
+      uint32_t hp[4];
 #pragma unroll
-      for (int w = 0; w < kNWK; ++w) {
-        Y0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Ka[w][0], X, Y0, 0, 0, 0);
-        Y1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Ka[w][1], X, Y1, 0, 0, 0);
-      }
-      bf16x8 Hop;
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        Hop[2 * u] = (__bf16)hr[u];
-        Hop[2 * u + 1] = (__bf16)hi[u];
-      }
-#pragma unroll
-      for (int w = 0; w < kNWC; ++w) {
-        Y0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Ca[w][0], Hop, Y0, 0, 0, 0);
-        Y1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Ca[w][1], Hop, Y1, 0, 0, 0);
-      }
-      if (two_terms) {
-        bf16x8 Hlo;
+      for (int u = 0; u < 4; ++u) hp[u] = pack16<F16>(hr[u], hi[u]);
+      const uint4 Hop = make_uint4(hp[0], hp[1], hp[2], hp[3]);
+      auto low_states = [&]() {
+        uint32_t hl[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          Hlo[2 * u] = (__bf16)(hr[u] - (float)Hop[2 * u]);
-          Hlo[2 * u + 1] = (__bf16)(hi[u] - (float)Hop[2 * u + 1]);
+          const float2 v = unpack16<F16>(hp[u]);
+          hl[u] = pack16<F16>(hr[u] - v.x, hi[u] - v.y);
         }
+        const uint4 Hlo = make_uint4(hl[0], hl[1], hl[2], hl[3]);
 #pragma unroll
         for (int w = 0; w < kNWC; ++w) {
-          Y0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Ca[w][0], Hlo, Y0, 0, 0, 0);
-          Y1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Ca[w][1], Hlo, Y1, 0, 0, 0);
+          Y0 = mma<F16>(Ca[w][0], Hlo, Y0);
+          Y1 = mma<F16>(Ca[w][1], Hlo, Y1);
         }
+      };
+      if constexpr (F16) {                        // the small terms of the sum first
+        low_states();
+        Y0 = mma<F16>(Ca[NC - 1][0], Hop, Y0);
+        Y1 = mma<F16>(Ca[NC - 1][1], Hop, Y1);
+        if constexpr (NX > 1) {
+          const uint4 Xl = *(const uint4*)(xat + kPlane);
+          Y0 = mma<F16>(Ka[0][0], Xl, Y0);
+          Y1 = mma<F16>(Ka[0][1], Xl, Y1);
+        }
+#pragma unroll
+        for (int w = kNWK - 1; w >= 0; --w) {
+          Y0 = mma<F16>(Ka[w][0], X, Y0);
+          Y1 = mma<F16>(Ka[w][1], X, Y1);
+        }
+        Y0 = mma<F16>(Ca[0][0], Hop, Y0);
+        Y1 = mma<F16>(Ca[0][1], Hop, Y1);
+      } else {
+#pragma unroll
+        for (int w = 0; w < kNWK; ++w) {
+          Y0 = mma<F16>(Ka[w][0], X, Y0);
+          Y1 = mma<F16>(Ka[w][1], X, Y1);
+        }
+#pragma unroll
+        for (int w = 0; w < NC; ++w) {
+          Y0 = mma<F16>(Ca[w][0], Hop, Y0);
+          Y1 = mma<F16>(Ca[w][1], Hop, Y1);
+        }
+        if (two_terms) low_states();
       }
       if (t == 0) {
         float Qr[4], Qi[4];
-        lds_cmp(s_tab, kCmpQ32, c, roff, Qr, Qi);
+        lds_cmp(s_tab, kCmpQ32 * CW + c, roff, Qr, Qi);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const float nr = fmaf(Qr[u], hr[u], fmaf(-Qi[u], hi[u], Fr[u]));
@@ -866,15 +1048,26 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
           hr[u] = nr;
         }
       }
-      // y (bf16) over x: tokens 32 t + 4 r + {0..3} and 32 t + 16 + 4 r + {0..3} of segment j
-      *(uint2*)(row + (((4 * t + (r >> 1)) ^ (j >> 1)) << 4) + (r & 1) * 8) =
-          make_uint2(pack_bf16(Y0[0], Y0[1]), pack_bf16(Y0[2], Y0[3]));
-      *(uint2*)(row + (((4 * t + 2 + (r >> 1)) ^ (j >> 1)) << 4) + (r & 1) * 8) =
-          make_uint2(pack_bf16(Y1[0], Y1[1]), pack_bf16(Y1[2], Y1[3]));
+      // y over x (fp32: the upper and lower halves of its words, a plane each): tokens 32 t + 4 r + {0..3} and
+      // 32 t + 16 + 4 r + {0..3} of segment j
+      char* y0 = row + (((4 * t + (r >> 1)) ^ (j >> 1)) << 4) + (r & 1) * 8;
+      char* y1 = row + (((4 * t + 2 + (r >> 1)) ^ (j >> 1)) << 4) + (r & 1) * 8;
+      if constexpr (NX == 1) {
+        *(uint2*)y0 = make_uint2(pack16<F16>(Y0[0], Y0[1]), pack16<F16>(Y0[2], Y0[3]));
+        *(uint2*)y1 = make_uint2(pack16<F16>(Y1[0], Y1[1]), pack16<F16>(Y1[2], Y1[3]));
+      } else {
+        auto halves = [](const float a, const float c, const uint32_t sel) {
+          return __builtin_amdgcn_perm(__float_as_uint(c), __float_as_uint(a), sel);
+        };
+        *(uint2*)y0 = make_uint2(halves(Y0[0], Y0[1], 0x07060302u), halves(Y0[2], Y0[3], 0x07060302u));
+        *(uint2*)y1 = make_uint2(halves(Y1[0], Y1[1], 0x07060302u), halves(Y1[2], Y1[3], 0x07060302u));
+        *(uint2*)(y0 + kPlane) = make_uint2(halves(Y0[0], Y0[1], 0x05040100u), halves(Y0[2], Y0[3], 0x05040100u));
+        *(uint2*)(y1 + kPlane) = make_uint2(halves(Y1[0], Y1[1], 0x05040100u), halves(Y1[2], Y1[3], 0x05040100u));
+      }
       MEGA_FTR2(2 + t);
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (i + 1 < kFCPW) load_kc(wave + kFW * (i + 1), Ka, Ca);
+    if (i + 1 < CPW) load_kc(wave + kFW * (i + 1), Ka, Ca);
     __builtin_amdgcn_sched_barrier(0);
     MEGA_FTR2(4);
     if (LOUT == 0) store_row(c);
@@ -888,13 +1081,14 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
     const uint32_t sel_keep = odd ? 0x07060302u : 0x05040100u;
     const uint32_t sel_give = odd ? 0x05040100u : 0x07060302u;
     const int tl = tokl & ~1;
-    const char* rbase = tile + row_base(piece * 8 + odd * 4) + (tl >> 6) * 128 + ((tl & 7) >> 1) * 4;
+    const char* rbase = tile + (NX == 1 ? row_base(piece * 8 + odd * 4) : odd * kPlane + row_base(piece * 4)) +
+                        (tl >> 6) * 128 + ((tl & 7) >> 1) * 4;
     const int c8 = (tl & 63) >> 3;
-    bf16_t* yb = A.y + (int64_t)b * A.syb + (int64_t)(cb + piece * 8) * A.syd;
+    T* yb = gy + (int64_t)b * A.syb + (int64_t)(cb + piece * VPP) * A.syd;
 #pragma unroll
-    for (int k = 0; k < kFNLD; ++k) {
-      const int tok = k * 128 + tokl;
-      const char* rp = rbase + (2 * k) * 128 + ((c8 ^ k) << 4);
+    for (int k = 0; k < NLD; ++k) {
+      const int tok = k * TPR + tokl;
+      const char* rp = rbase + k * (TPR * 2) + ((c8 ^ ((k * TPR + tl) >> 7)) << 4);
       uint32_t w[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) w[e] = *(const uint32_t*)(rp + e * kFRow);
@@ -902,12 +1096,19 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
       const uint32_t keep1 = __builtin_amdgcn_perm(w[3], w[2], sel_keep);
       const uint32_t got0 = dpp_u<0x128>(__builtin_amdgcn_perm(w[1], w[0], sel_give));
       const uint32_t got1 = dpp_u<0x128>(__builtin_amdgcn_perm(w[3], w[2], sel_give));
+      // the even token's lane kept (and got the partner's view of) the first half: channels 0..3 of eight, or the
+      // upper halves of four words
+      const uint32_t f0 = odd ? got0 : keep0, f1 = odd ? got1 : keep1, l0 = odd ? keep0 : got0, l1 = odd ? keep1 : got1;
       uint4 o;
-      o.x = odd ? got0 : keep0;
-      o.y = odd ? got1 : keep1;
-      o.z = odd ? keep0 : got0;
-      o.w = odd ? keep1 : got1;
-      if (t0 + tok >= 0) store_stream((uint4*)(yb + (int64_t)(t0 + tok) * A.syl), o);
+      if constexpr (NX == 1) {
+        o = make_uint4(f0, f1, l0, l1);
+      } else {
+        o.x = __builtin_amdgcn_perm(f0, l0, 0x05040100u);
+        o.y = __builtin_amdgcn_perm(f0, l0, 0x07060302u);
+        o.z = __builtin_amdgcn_perm(f1, l1, 0x05040100u);
+        o.w = __builtin_amdgcn_perm(f1, l1, 0x07060302u);
+      }
+      if (act && t0 + tok >= 0) store_stream((uint4*)(yb + (int64_t)(t0 + tok) * A.syl), o);
     }
   }
 
@@ -928,25 +1129,87 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
   }
 }
 
-// R: record rows = workgroups per block = B * D / 64
-size_t fused_ws_bytes(int64_t R, int64_t S) {
-  return align_up(sizeof(TsnHeader), 256) + align_up((size_t)R * (S + 1) * kFRecW * 8, 256);
+// records of B * D channels in workgroups of cw
+size_t fused_ws_bytes(int64_t B, int64_t D, int64_t S, int cw) {
+  return align_up(sizeof(TsnHeader), 256) + align_up((size_t)(B * ceil_div(D, cw)) * (S + 1) * (4 + cw * kNS * 2) * 8, 256);
+}
+
+// Channels of a workgroup for norm groups of gc channels, 0: no instance.  16-bit rows of a block fill the LDS with 64
+// channels, fp32 rows (two planes) with 32; a group that does not fit is shared by equal parts of a multiple of 16.
+// The two operators one after the other (norm, transposition, rows kernels, transposition) take, against one launch
+// here, with y in x's layout: fp16 3 x 1501 x 768 in 48s 79 us, 26 here; fp16 4 x 4096 x 1024 in 64s 101 us, 34; fp16
+// 2 x 8192 x 2048 in 128s 249 us, 76; fp32 4 x 4096 x 1024 138 us, 53 (3.8 TB/s); fp32 2 x 8192 x 2048 in four parts
+// 364 us, 134; fp32 1 x 300 x 512 in 32s 51 us, 24 (the host's call).  bf16 in the widths beside 64 and 128 (norm, then
+// the streaming kernel): 4 x 4096 x 768 in 48s 54 us, 40; 8 x 2048 x 512 in 32s 32 us, 24; 2 x 1333 x 1536 37 us, 25.
+int fused_channels(int dtype, int64_t gc) {
+  const bool wide = dtype == MEGA_F32;
+  switch (gc) {
+    case 32: return 32;
+    case 48: return wide ? 16 : 48;
+    case 64: return wide ? 32 : 64;
+    case 96: return wide ? 32 : 48;
+    case 128: return wide ? 32 : 64;
+    default: return 0;
+  }
+}
+
+template <typename T, int CW, int PARTS, int LOUT, bool STAG>
+void fused_launch(const FusedArgs& A, dim3 grid, hipStream_t s) {
+  static uint64_t attr_seen = 0;
+  const auto kern = norm_ema_fused_kernel<T, CW, PARTS, LOUT, STAG>;
+  constexpr size_t smem = Geo<T, CW, PARTS>::Smem;
+  if (first_on_device(&attr_seen))
+    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+  hipLaunchKernelGGL(kern, grid, dim3(kFT), smem, s, A);
+}
+
+template <typename T, int CW, int PARTS>
+void fused_launch_layout(const FusedArgs& A, int lout, dim3 grid, hipStream_t s) {
+  if constexpr (__is_same(T, bf16_t) && CW == 64) {
+    if (A.stagger > 0)
+      return lout ? fused_launch<T, CW, PARTS, 1, true>(A, grid, s) : fused_launch<T, CW, PARTS, 0, true>(A, grid, s);
+  }
+  return lout ? fused_launch<T, CW, PARTS, 1, false>(A, grid, s) : fused_launch<T, CW, PARTS, 0, false>(A, grid, s);
+}
+
+template <typename T>
+void fused_launch_width(const FusedArgs& A, int gc, int lout, dim3 grid, hipStream_t s) {
+  if constexpr (sizeof(T) == 4) {
+    switch (gc) {
+      case 32: return fused_launch_layout<T, 32, 1>(A, lout, grid, s);
+      case 48: return fused_launch_layout<T, 16, 3>(A, lout, grid, s);
+      case 64: return fused_launch_layout<T, 32, 2>(A, lout, grid, s);
+      case 96: return fused_launch_layout<T, 32, 3>(A, lout, grid, s);
+      default: return fused_launch_layout<T, 32, 4>(A, lout, grid, s);
+    }
+  } else {
+    switch (gc) {
+      case 32: return fused_launch_layout<T, 32, 1>(A, lout, grid, s);
+      case 48: return fused_launch_layout<T, 48, 1>(A, lout, grid, s);
+      case 64: return fused_launch_layout<T, 64, 1>(A, lout, grid, s);
+      case 96: return fused_launch_layout<T, 48, 2>(A, lout, grid, s);
+      default: return fused_launch_layout<T, 64, 2>(A, lout, grid, s);
+    }
+  }
+}
+
+bool fused_sizes(int dtype, int64_t B, int64_t L, int64_t D, int64_t G, int64_t N, bool carried, bool rows) {
+  if (G <= 0 || D <= 0 || D % G || N > kNS || N <= 0 || L <= 0) return false;
+  const int cw = fused_channels(dtype, D / G);
+  if (cw == 0 || ceil_div(L, kFSeg) + (carried ? 1 : 0) > kFMaxBlocks) return false;
+  // a ragged first block (the block grid is aligned to the end of the row): no carried state in (it would have to
+  // enter in the middle of a block), and rows in time must begin at a multiple of 8 inside it
+  if (L % kFSeg != 0 && (carried || (rows && L % 8 != 0))) return false;
+  return B * (D / cw) * ceil_div(L, kFSeg) < (int64_t)1 << 31;
 }
 
 bool fused_covers(int dtype, int64_t B, int64_t L, int64_t D, int64_t G, int64_t N, const void* x, const void* xn,
-                  const void* y, int64_t syb, int64_t syd, int64_t syl, const uint8_t* mask, const float* h_in) {
-  (void)mask;
-  if (dtype != MEGA_BF16 || G <= 0 || (D != G * kFC && D != G * 2 * kFC) || N > kNS || N <= 0) return false;
-  if (L <= 0 || ceil_div(L, kFSeg) + (h_in ? 1 : 0) > kFMaxBlocks) return false;
-  // a ragged first block (the block grid is aligned to the end of the row): no carried state in (it would have to
-  // enter in the middle of a block), and rows in time must begin at a multiple of 8 inside it
-  if (L % kFSeg != 0 && (h_in || (syl == 1 && L % 8 != 0))) return false;
+                  const void* y, int64_t syb, int64_t syd, int64_t syl, const float* h_in) {
+  if (!fused_sizes(dtype, B, L, D, G, N, h_in != nullptr, syl == 1)) return false;
   if (((uintptr_t)x % 16) || ((uintptr_t)xn % 16) || ((uintptr_t)y % 16)) return false;
   const bool rows = syl == 1 && syd % 8 == 0 && syb % 8 == 0;
   const bool lines = syd == 1 && syl % 8 == 0 && syb % 8 == 0;
-  if (!rows && !lines) return false;
-  if (B * (D / kFC) * ceil_div(L, kFSeg) >= (int64_t)1 << 31) return false;
-  return true;
+  return rows || lines;
 }
 
 }  // namespace
@@ -958,9 +1221,15 @@ using namespace mega;
 extern "C" size_t mega_norm_ema_fwd_workspace_bytes(int64_t B, int64_t L, int64_t D, int64_t G, int64_t N) {
   (void)N;
   if (B <= 0 || L <= 0 || D <= 0 || G <= 0) return 256;
-  const size_t fused = fused_ws_bytes(B * ceil_div(D, kFC), ceil_div(L, kFSeg));
+  const size_t fused = fused_ws_bytes(B, D, ceil_div(L, kFSeg), 16);      // (the narrowest workgroups: the most records)
   const size_t tsn = mega_timestep_norm_workspace_bytes(MEGA_BF16, B, L, D, G);
   return fused > tsn ? fused : tsn;
+}
+
+// 1: a call of these sizes (dense operands on 16 bytes) is one launch of the one-kernel route, for any activation type
+extern "C" int mega_norm_ema_fwd_one_kernel(int dtype, int64_t B, int64_t L, int64_t D, int64_t G, int64_t N, int carried,
+                                            int rows_out) {
+  return fused_sizes(dtype, B, L, D, G, N, carried != 0, rows_out != 0) && mega_ema_image_bytes(D, N, 0) > 0 ? 1 : 0;
 }
 
 // scratch (no initialisation, contents never survive a call): the moving average's own workspace when the two
@@ -997,7 +1266,7 @@ extern "C" int mega_norm_ema_fwd_train(const void* x, void* xn, void* y, int dty
   const int64_t S = ceil_div(L > 0 ? L : 1, kFSeg);
   char* w = (char*)workspace;
   const bool one_kernel = L > 0 && (image || mega_ema_image_bytes(D, N, 0) > 0) &&
-                          fused_covers(dtype, B, L, D, G, N, x, xn, y, syb, syd, syl, mask, h_in);
+                          fused_covers(dtype, B, L, D, G, N, x, xn, y, syb, syd, syl, h_in);
   if (!one_kernel || !image) {
     const size_t sneed = mega_norm_ema_fwd_scratch_bytes(B, L > 0 ? L : 1, D, G, N);
     MEGA_REQUIRE(scratch && scratch_bytes >= sneed, MEGA_ERR_WORKSPACE, "norm_ema_fwd: scratch of %zu bytes needed",
@@ -1016,12 +1285,12 @@ extern "C" int mega_norm_ema_fwd_train(const void* x, void* xn, void* y, int dty
     const void* img = image;
     if (!img) {
       // no cached image: kernel generation runs with every call
-      const int rc = ema_image_build(p, q, gamma, is_complex, omega, D, N, 0, 1, scratch, s, kImgPC | kImgKT | kImgBlocks);
+      const int rc = ema_image_build(p, q, gamma, is_complex, omega, D, N, 0, 1, scratch, s, (dtype == MEGA_BF16 ? kImgPC | kImgKT : kImgF16) | kImgBlocks);
       if (rc) return rc;
       img = scratch;
     }
     FusedArgs A;
-    A.x = (const bf16_t*)x; A.xn = (bf16_t*)xn; A.y = (bf16_t*)y; A.syb = syb; A.syd = syd; A.syl = syl;
+    A.x = x; A.xn = xn; A.y = y; A.syb = syb; A.syd = syd; A.syl = syl;
     A.prev_count = prev_count; A.prev_mean = prev_mean; A.prev_var = prev_var; A.count = count; A.mean = mean;
     A.var = var; A.gamma = norm_gamma; A.beta = norm_beta; A.mask = mask; A.image = (const uint4*)img; A.h_in = h_in; A.h_out = h_out;
     A.cummean = cummean; A.cumrstd = cumrstd;
@@ -1029,30 +1298,22 @@ extern "C" int mega_norm_ema_fwd_train(const void* x, void* xn, void* y, int dty
     A.B = (int)B; A.L = (int)L; A.D = (int)D; A.G = (int)G; A.N = (int)N; A.S = (int)S; A.eps = (float)eps;
     A.pad = (int)(S * kFSeg - L);
     A.is_complex = is_complex;
-    const int parts = (int)(D / (G * kFC));              // workgroups per norm group
-    A.xcd_map = ((G * parts) % 8 == 0) ? 1 : 0;
+    const int gc = (int)(D / G), cw = fused_channels(dtype, gc);
+    A.xcd_map = (D / cw) % 8 == 0 ? 1 : 0;
     A.lb = lookback_launch(true);
-    const dim3 grid((unsigned)(B * G * parts * S));
+    const dim3 grid((unsigned)(B * (D / cw) * S));
     // held-back starts only where the launch is one round of workgroups (one per compute unit) and fills most of it
     const int cus = device_cu_count();
     A.stagger = (S > 1 && S <= MEGA_FUSED_STAGGER_BLOCKS && (int64_t)grid.x <= cus &&
                  (int64_t)grid.x * MEGA_FUSED_STAGGER_FILL >= cus * (MEGA_FUSED_STAGGER_FILL - 1))
                     ? MEGA_FUSED_STAGGER
                     : 0;
-    typedef void (*Kern)(const FusedArgs);
     const int lout = syl == 1 ? 0 : 1;
-    const Kern kerns[2][2][2] = {
-        {{norm_ema_fused_kernel<0, 64, false>, norm_ema_fused_kernel<0, 64, true>},
-         {norm_ema_fused_kernel<1, 64, false>, norm_ema_fused_kernel<1, 64, true>}},
-        {{norm_ema_fused_kernel<0, 128, false>, norm_ema_fused_kernel<0, 128, true>},
-         {norm_ema_fused_kernel<1, 128, false>, norm_ema_fused_kernel<1, 128, true>}}};
-    const int stag = A.stagger > 0 ? 1 : 0;
-    const Kern kern = kerns[parts - 1][lout][stag];
-    static uint64_t attr_seen[2][2][2] = {{{0, 0}, {0, 0}}, {{0, 0}, {0, 0}}};
-    if (first_on_device(&attr_seen[parts - 1][lout][stag])) {
-      (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFSmem);
+    switch (dtype) {
+      case MEGA_F32: fused_launch_width<float>(A, gc, lout, grid, s); break;
+      case MEGA_F16: fused_launch_width<f16_t>(A, gc, lout, grid, s); break;
+      default: fused_launch_width<bf16_t>(A, gc, lout, grid, s); break;
     }
-    hipLaunchKernelGGL(kern, grid, dim3(kFT), kFSmem, s, A);
     MEGA_CHECK_LAUNCH("norm_ema_fwd");
     return lookback_verify("norm_ema_fwd", s);
   }

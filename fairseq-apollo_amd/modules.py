@@ -698,8 +698,9 @@ class NormThenMoveFunc(torch.autograd.Function):
         layer, (ng, nb, pm, pv, pc) = ops.PreparedEMA.of_parameters(
             (alpha, delta, third, gamma, omega), is_complex, False, True, xd,
             (weight, bias, prior_mean, prior_logv, prior_count), B)
-        if xd.dtype is torch.bfloat16:
-            G, N, (_, L, D) = prior_mean.numel(), layer.N, xd.shape
+        G, N, (_, L, D) = prior_mean.numel(), layer.N, xd.shape
+        if xd.dtype is torch.bfloat16 or (xd.data_ptr() % 16 == 0 and ops.norm_ema_one_kernel(
+                ops._dtype_code(xd), B, L, D, G, N, False, out_layout == "rows")):
             stream = ops._stream(xd.device)
             ws = ops._tsn_workspace(xd.device, ops.norm_ema_workspace_bytes(B, L, D, G, N), stream)
             with ops._on_device(xd.device):

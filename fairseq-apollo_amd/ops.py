@@ -745,6 +745,15 @@ def transpose_2d(x: torch.Tensor, reverse_rows: bool = False, reverse_cols: bool
     return out
 
 
+def norm_ema_one_kernel(dtype: int, B: int, L: int, D: int, G: int, N: int, carried: bool, rows: bool) -> bool:
+    """Whether TimestepNorm -> moving average of these sizes is one launch (mega_norm_ema_fwd_one_kernel)."""
+    key = ("norm_ema_one", dtype, B, L, D, G, N, carried, rows)
+    n = _ws_bytes_cache.get(key)
+    if n is None:
+        n = _ws_bytes_cache[key] = _lib.load().mega_norm_ema_fwd_one_kernel(dtype, B, L, D, G, N, int(carried), int(rows))
+    return bool(n)
+
+
 def norm_ema_workspace_bytes(B: int, L: int, D: int, G: int, N: int) -> int:
     key = ("norm_ema_ws", B, L, D, G, N)
     n = _ws_bytes_cache.get(key)
@@ -895,8 +904,10 @@ class PreparedEMA:
         if out_layout not in ("rows", "input"):
             raise RuntimeError(f"out_layout must be 'rows' or 'input', got {out_layout!r}")
         if xd.dtype is not torch.bfloat16 and 64 <= L <= 16384 and self.N <= 16 and B > 0 \
-                and not ((want_state or h is not None) and L % 1024):
-            # fp32 / fp16: the two operators, the second through PreparedEMA.__call__, which takes the normalised
+                and not ((want_state or h is not None) and L % 1024) \
+                and not (xd.data_ptr() % 16 == 0 and
+                         norm_ema_one_kernel(dt, B, L, D, G, self.N, h is not None, out_layout == "rows")):
+            # fp32 / fp16 outside the one-kernel sizes: the two operators, the second through PreparedEMA.__call__, which takes the normalised
             # activations (time-major in memory) onto the rows kernels; inside the library's own two-operator
             # route the moving average would read them in place on its vector-ALU path
             if want_stats:

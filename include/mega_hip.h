@@ -397,9 +397,9 @@ int mega_norm_ema_steps(const void* x, void* xn, void* y, int dtype, int64_t K,
  *   norm state / parameters / mask as mega_group_timestep_norm_fwd (norm_gamma = weight + 1);
  *   moving-average coefficients, h_in / h_out and `image` as mega_ema_fwd (unidirectional,
  *   no truncation); h_out must not overlap h_in.
- * bf16 activations with 64 or 128 channels per norm group (D = 64 G or 128 G), ndim <= 16, with or
- * without a mask, ceil(L / 1024) (+ 1 with h_in) <= 16 run as ONE kernel that reads x once and writes xn
- * and y once.  L need not be a multiple of 1024 (the blocks are aligned to the end of the row, so h_out is
+ * Activations of any type with 32, 48, 64, 96 or 128 channels per norm group, ndim <= 16, with or
+ * without a mask, ceil(L / 1024) (+ 1 with h_in) <= 16, operands on 16 bytes run as ONE kernel that reads x once
+ * and writes xn and y once (mega_norm_ema_fwd_one_kernel says whether sizes do).  L need not be a multiple of 1024 (the blocks are aligned to the end of the row, so h_out is
  * the state after the last token), but such a row takes no h_in, and [B,D,L] rows then need L % 8 == 0.
  * Everything else runs the two operators one after the other.
  * `workspace` (launch epoch, block / tile records) must be zero-filled once and then belongs to
@@ -408,6 +408,9 @@ int mega_norm_ema_steps(const void* x, void* xn, void* y, int dtype, int64_t K,
  * other or when image == NULL (kernel generation inside the call).                          */
 size_t mega_norm_ema_fwd_workspace_bytes(int64_t B, int64_t L, int64_t D, int64_t G, int64_t N);
 size_t mega_norm_ema_fwd_scratch_bytes(int64_t B, int64_t L, int64_t D, int64_t G, int64_t N);
+/* 1 when calls of these sizes run as one kernel (carried: with h_in; rows_out: y as [B,D,L] rows), else 0 */
+int mega_norm_ema_fwd_one_kernel(int dtype, int64_t B, int64_t L, int64_t D, int64_t G, int64_t N, int carried,
+                                 int rows_out);
 int mega_norm_ema_fwd(const void* x, void* xn, void* y, int dtype, int64_t syb, int64_t syd,
                       int64_t syl, const int64_t* prev_count, const float* prev_mean,
                       const float* prev_var, const float* norm_gamma, const float* norm_beta,

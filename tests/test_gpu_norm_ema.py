@@ -423,3 +423,52 @@ def test_fp32_fp16_ragged_row_and_training_statistics(dtype, tol):
     assert rel_err(host(cr)[:, -1], 1.0 / np.sqrt(v + 1e-5)) < 1e-4
     yo, _ = O.ema_forward(host(xn).transpose(0, 2, 1), p, q, g, om)
     assert rel_err(host(y), yo) < tol
+
+
+# largest error of xn and of y (given the rounded xn) over the largest value: half a unit in the last place of the
+# activation type against the root mean square times a handful of roundings; fp32 as the row kernels (1.8e-6 measured)
+WIDTH_TOL = {torch.float32: 1e-4, torch.float16: 4e-3, BF: 2e-2}
+
+
+@pytest.mark.parametrize("cpg", [32, 48, 64, 96, 128])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, BF])
+@pytest.mark.parametrize("B,L,G,out_layout,masked,carried", [(2, 1501, 8, "input", True, False), (1, 2048, 3, "rows", False, True),
+                                                             (3, 8, 1, "rows", False, False), (2, 1, 2, "input", False, False),
+                                                             (1, 3072, 2, "input", True, True), (2, 1032, 2, "rows", True, False)])
+def test_one_kernel_widths_and_types(dtype, cpg, B, L, G, out_layout, masked, carried):
+    """Every norm group width and activation type of the one-kernel route: idle lanes (48, 96 channels of 16-bit
+    values), groups shared by two to four workgroups, both fp32 planes, front blocks of virtual tokens, and the
+    statistics and states handed on."""
+    print(f"case {dtype} cpg={cpg} B={B} L={L} G={G} out={out_layout} masked={masked} carried={carried}", flush=True)
+    D, N = cpg * G, 16
+    code = {torch.float32: 0, BF: 1, torch.float16: 2}[dtype]
+    assert M.ops.norm_ema_one_kernel(code, B, L, D, G, N, carried, out_layout == "rows")
+    rng = np.random.default_rng(60)
+    p, q, g, om, nw, nb = _setup(rng, D, N)
+    x, x64 = rounded(rng.normal(size=(B, L, D)) * 1.3 + 0.4, dtype)
+    mask = None
+    if masked:
+        mask = np.zeros((B, L), bool)
+        mask[0, : L // 5] = True
+        # (a short tail: behind some hundreds of padded tokens the states are below fp32's range, 1e-43 of q^438)
+        mask[B - 1, L - min(L // 7, 9):] = True
+        x[torch.from_numpy(mask).to(DEV)] = float("nan")          # whatever padding holds
+    layer = M.ops.PreparedEMA(dev(p), dev(q), dev(g), dev(om))
+    h0 = (rng.normal(size=(B, D, N)) + 1j * rng.normal(size=(B, D, N))) * 0.1
+    h = torch.from_numpy(h0.astype(np.complex64)).to(DEV) if carried else None
+    prior = (rng.integers(1, 50, B), rng.normal(size=(B, G)) * 0.2, rng.uniform(0.5, 1.5, (B, G)))
+    tp = (torch.from_numpy(prior[0]).to(DEV), dev(prior[1]), dev(prior[2]))
+    xn, y, cnt, mean, var, h1, cm, cr = _run(layer, x, G, nw, nb, prior=tp, h=h, want_state=carried or L % 8 == 0,
+                                             padding_mask=None if mask is None else dev(mask, torch.bool),
+                                             out_layout=out_layout, want_stats=True)
+    tol = WIDTH_TOL[dtype]
+    xno, c, mu, v = O.timestep_norm(x64, *prior, nw + 1, nb, mask, G)
+    assert rel_err(host(xn), xno) < tol
+    assert cnt.tolist() == c.tolist()
+    assert rel_err(host(mean), mu) < 1e-4 and rel_err(host(var), v) < 1e-4
+    assert rel_err(host(cm)[:, -1], mu) < 1e-4 and rel_err(host(cr)[:, -1], 1.0 / np.sqrt(v + 1e-5)) < 1e-4
+    yo, ho = O.ema_forward(host(xn).transpose(0, 2, 1), p, q, g, om, mask, *((h0,) if carried else ()), incremental=True)
+    _check_y(y, yo, tol, tol)
+    if h1 is not None:
+        e = rel_err(np.real(host(h1)), np.real(ho)), rel_err(np.imag(host(h1)), np.imag(ho))
+        assert max(e) < 2e-3, e
