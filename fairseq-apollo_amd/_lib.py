@@ -68,6 +68,8 @@ SIGNATURES = {
     "mega_token_gated_attention": (_int, [_p, _p]),
     "mega_norm_ema_fwd_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64]),
     "mega_norm_ema_fwd_scratch_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64]),
+    "mega_gemm_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64]),
+    "mega_gemm_f32": (_int, [_p, _p, _sz, _p]),
     "mega_norm_ema_fwd_one_kernel": (_int, [_int, _i64, _i64, _i64, _i64, _i64, _int, _int]),
     "mega_norm_ema_fwd": (_int, [_p, _p, _p, _int, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, C.c_double, _p, _p, _p,
                                  _p, _p, _p, _int, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p, _p, _sz, _p, _sz, _p]),

@@ -27,6 +27,7 @@ SOURCES = [
     "decode.hip",
     "decode_layer.hip",
     "elementwise.hip",
+    "gemm.hip",
     "gate_glue.hip",
     "row_norm.hip",
     "attention.hip",

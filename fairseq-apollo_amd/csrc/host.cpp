@@ -559,8 +559,66 @@ Result ema_param_backward(const Args& A) {
 }
 
 // ---- training: the layer around its norm, moving average and attention, forwards and backwards in few calls.  The
-// products are library GEMMs; what lies between them runs in libmega_hip.  Activations and weights share one type.
+// products of 16-bit activations are library GEMMs; those of fp32 and what lies between them run in libmega_hip.
+// Activations and weights share one type.
 Tensor rows2(const Tensor& t) { return t.reshape({-1, t.size(-1)}); }
+
+// A matrix whose elements follow each other along one of its axes: that axis and the other one's stride
+struct Matrix {
+  int64_t ld;
+  bool first;                                   // the contiguous axis is the first one
+};
+bool matrix(const Tensor& t, Matrix* m) {
+  if (t.dim() != 2) return false;
+  const int64_t r = t.size(0), c = t.size(1), sr = t.stride(0), sc = t.stride(1);
+  if ((sc == 1 || c == 1) && (sr >= c || r == 1)) return *m = {r == 1 ? c : sr, false}, true;
+  if ((sr == 1 || r == 1) && (sc >= r || c == 1)) return *m = {c == 1 ? r : sc, true}, true;
+  return false;
+}
+
+// a [M, K] b [K, N] (+ bias) (+ residual) as fp32 products on the matrix cores (mega_gemm_f32), silu of it with the value
+// before in `pre`; `out` (optional) receives the result and may be the residual.  False: not of this kind.
+bool product_f32(const Tensor& a, const Tensor& b, const Tensor& bias, const Tensor& residual, bool silu, Tensor* pre, Tensor* out,
+                 void* s, const char* who) {
+  Matrix ma, mb, mr = {0, false};
+  if (a.scalar_type() != at::kFloat || b.scalar_type() != at::kFloat || !a.is_cuda() || a.device() != b.device() || !matrix(a, &ma) ||
+      !matrix(b, &mb) || a.size(1) != b.size(0) || a.numel() == 0 || b.numel() == 0)
+    return false;
+  const int64_t M = a.size(0), K = a.size(1), N = b.size(1);
+  auto fits = [&](const Tensor& t) { return t.scalar_type() == at::kFloat && t.device() == a.device(); };
+  if (bias.defined() && (!fits(bias) || bias.numel() != N || !bias.is_contiguous())) return false;
+  if (residual.defined() && (!fits(residual) || !matrix(residual, &mr) || mr.first || residual.size(0) != M || residual.size(1) != N)) return false;
+  if (!out->defined()) *out = at::empty({M, N}, a.options());
+  if (pre) *pre = at::empty({M, N}, a.options());
+  MegaGemm g = {};
+  g.a = a.data_ptr(); g.b = b.data_ptr(); g.c = out->data_ptr();
+  g.bias = bias.defined() ? bias.data_ptr() : nullptr;
+  g.residual = residual.defined() ? residual.data_ptr() : nullptr;
+  g.pre = pre ? pre->data_ptr() : nullptr;
+  g.lda = ma.ld; g.a_kmajor = ma.first;
+  g.ldb = mb.ld; g.b_kmajor = !mb.first;
+  g.ldc = N; g.ldr = mr.ld;
+  g.M = M; g.N = N; g.K = K; g.batch = g.inner = 1;
+  g.silu = silu; g.alpha = 1.f;
+  const int64_t nws = (int64_t)mega_gemm_workspace_bytes(M, N, K, 1);
+  Tensor ws;
+  if (nws) ws = at::empty({nws}, a.options().dtype(at::kByte));
+  check(mega_gemm_f32(&g, nws ? ws.data_ptr() : nullptr, (size_t)nws, s), who);
+  return true;
+}
+
+Tensor mm(const Tensor& a, const Tensor& b, void* s, const char* who) {
+  Tensor out;
+  return product_f32(a, b, Tensor(), Tensor(), false, nullptr, &out, s, who) ? out : at::mm(a, b);
+}
+// a b + c, c a row of biases or a whole matrix
+Tensor addmm(const Tensor& c, const Tensor& a, const Tensor& b, void* s, const char* who) {
+  Tensor out;
+  const bool row = c.dim() == 1;
+  return product_f32(a, b, row ? c : Tensor(), row ? Tensor() : c, false, nullptr, &out, s, who) ? out : at::addmm(c, a, b);
+}
+// silu(a b + bias) and the value before
+std::pair<Tensor, Tensor> silu_mm(const Tensor& bias, const Tensor& a, const Tensor& b, void* s, const char* who);
 
 const void* ptr_or_null(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 Tensor opt_t(const Args& A, int i) { return A.none(i) ? Tensor() : A.t(i); }
@@ -629,6 +687,62 @@ Tensor silu(const Tensor& x, void* s, const char* who) {
   return y;
 }
 
+std::pair<Tensor, Tensor> silu_mm(const Tensor& bias, const Tensor& a, const Tensor& b, void* s, const char* who) {
+  Tensor pre, out;
+  if (!product_f32(a, b, bias, Tensor(), true, &pre, &out, s, who)) {
+    pre = at::addmm(bias, a, b);
+    out = silu(pre, s, who);
+  }
+  return {pre, out};
+}
+
+// a linear layer outside training: (x [.., K] contiguous fp32, weight [N, K], bias | None, residual [.., N] | None, silu,
+// the residual's memory may take the result, stream) -> [.., N]
+Result linear_f32(const Args& A) {
+  A.want(7);
+  const Tensor &x = A.t(0), &w = A.t(1);
+  same_type(A, {0, 1, 2, 3}, x);
+  auto sizes = x.sizes().vec();
+  if (w.dim() != 2 || sizes.back() != w.size(1)) throw std::runtime_error("linear_f32: rows of another width than the weight's");
+  sizes.back() = w.size(0);
+  A.shape(2, {w.size(0)});
+  A.shape(3, sizes);
+  const Tensor r = A.none(3) ? Tensor() : rows2(A.t(3));
+  Tensor out = !A.none(3) && A.flag(5) ? r : Tensor();
+  if (!product_f32(rows2(x), w.t(), opt_t(A, 2), r, A.flag(4), nullptr, &out, A.stream(6), A.who))
+    throw std::runtime_error("linear_f32: fp32 device tensors expected");
+  return wrap(out.view(sizes));
+}
+
+// Batched fp32 products over the positions and heads of attention: (a, b, c, M, N, K, batch, heads, a's row stride, batch
+// stride, head stride, reduction along its rows, the same four of b, c's row, batch and head stride, causal, alpha, stream)
+Result attention_product(const Args& A) {
+  A.want(22);
+  MegaGemm g = {};
+  const Tensor& a = A.t(0);
+  same_type(A, {0, 1, 2}, a);
+  if (a.scalar_type() != at::kFloat || !a.is_cuda()) throw std::runtime_error("attention_product: fp32 device tensors expected");
+  g.a = a.data_ptr(); g.b = A.t(1).data_ptr(); g.c = A.t(2).data_ptr();
+  g.M = A.i64(3); g.N = A.i64(4); g.K = A.i64(5); g.batch = A.i64(6) * A.i64(7); g.inner = A.i64(7);
+  g.lda = A.i64(8); g.sa = A.i64(9); g.sai = A.i64(10); g.a_kmajor = A.flag(11);
+  g.ldb = A.i64(12); g.sb = A.i64(13); g.sbi = A.i64(14); g.b_kmajor = A.flag(15);
+  g.ldc = A.i64(16); g.sc = A.i64(17); g.sci = A.i64(18);
+  g.causal = (int)A.i64(19); g.alpha = (float)A.d(20);
+  auto inside = [&](const Tensor& t, int64_t rows, int64_t cols, int64_t ld, int64_t sb, int64_t si) {
+    return ld >= 0 && sb >= 0 && si >= 0 &&
+           (A.i64(6) - 1) * sb + (g.inner - 1) * si + (rows - 1) * ld + cols <= t.numel();
+  };
+  if (g.M < 1 || g.N < 1 || g.K < 1 || A.i64(6) < 1 || g.inner < 1 ||
+      !inside(a, g.a_kmajor ? g.K : g.M, g.a_kmajor ? g.M : g.K, g.lda, g.sa, g.sai) ||
+      !inside(A.t(1), g.b_kmajor ? g.K : g.N, g.b_kmajor ? g.N : g.K, g.ldb, g.sb, g.sbi) || !inside(A.t(2), g.M, g.N, g.ldc, g.sc, g.sci))
+    throw std::runtime_error("attention_product: sizes beyond an operand");
+  const int64_t nws = (int64_t)mega_gemm_workspace_bytes(g.M, g.N, g.K, g.batch);
+  Tensor ws;
+  if (nws) ws = at::empty({nws}, a.options().dtype(at::kByte));
+  check(mega_gemm_f32(&g, nws ? ws.data_ptr() : nullptr, (size_t)nws, A.stream(21)), A.who);
+  return Result();
+}
+
 // Operations are only being run, not looked at: no tracing, function transform or dispatch mode, which see torch's own
 // operations and nothing that happens in here.
 bool eager() {
@@ -664,9 +778,8 @@ Result ffn_forward(const Args& A) {
   same_type(A, {0, 2, 3, 5, 6, 7}, x);
   void* s = A.stream(8);
   Tensor n = row_norm(x, opt_t(A, 2), opt_t(A, 3), (int)A.i64(1), A.d(4), s, A.who);
-  Tensor pre = at::addmm(A.t(6), rows2(n), A.t(5).t());
-  Tensor h = silu(pre, s, A.who);
-  Tensor out = at::addmm(rows2(x), h, A.t(7).t()).view(x.sizes());
+  auto [pre, h] = silu_mm(A.t(6), rows2(n), A.t(5).t(), s, A.who);
+  Tensor out = addmm(rows2(x), h, A.t(7).t(), s, A.who).view(x.sizes());
   Tensor r[4] = {out, n, pre, h};
   return tuple(r);
 }
@@ -693,13 +806,13 @@ Result ffn_backward(const Args& A) {
     throw std::runtime_error("ffn_backward: gradients and saved operands of other sizes than the forward's");
   const Tensor d2 = rows2(dout);
   Tensor dx, dnw, dnb, dw1, db1, dw2;
-  if (want(5)) dw2 = at::mm(d2.t(), h);
+  if (want(5)) dw2 = mm(d2.t(), h, s, A.who);
   if (want.any(0x1f)) {
     Tensor dpre;
-    std::tie(dpre, db1) = sum_rows(at::mm(d2, A.t(10)), pre, s, A.who);
-    if (want(3)) dw1 = at::mm(dpre.t(), rows2(n));
+    std::tie(dpre, db1) = sum_rows(mm(d2, A.t(10), s, A.who), pre, s, A.who);
+    if (want(3)) dw1 = mm(dpre.t(), rows2(n), s, A.who);
     if (want.any(7))
-      std::tie(dx, dnw, dnb) = row_norm_back(at::mm(dpre, A.t(9)), x, opt_t(A, 6), opt_t(A, 7), dout, (int)A.i64(5), A.d(8), s, A.who);
+      std::tie(dx, dnw, dnb) = row_norm_back(mm(dpre, A.t(9), s, A.who), x, opt_t(A, 6), opt_t(A, 7), dout, (int)A.i64(5), A.d(8), s, A.who);
   }
   Tensor r[6] = {dx, dnw, dnb, dw1, db1, dw2};
   return tuple(r);
@@ -713,9 +826,9 @@ Result swiglu_forward(const Args& A) {
   void* s = A.stream(5);
   const Tensor n2 = rows2(n);
   A.shape(3, A.t(2).sizes());
-  Tensor a = at::mm(n2, A.t(2).t()), b = at::mm(n2, A.t(3).t()), g = at::empty_like(a);
+  Tensor a = mm(n2, A.t(2).t(), s, A.who), b = mm(n2, A.t(3).t(), s, A.who), g = at::empty_like(a);
   check(mega_swiglu_fwd(a.data_ptr(), b.data_ptr(), g.data_ptr(), dtype_code(n), a.numel(), s), A.who);
-  Tensor out = A.none(1) ? at::mm(g, A.t(4).t()) : at::addmm(rows2(A.t(1)), g, A.t(4).t());
+  Tensor out = A.none(1) ? mm(g, A.t(4).t(), s, A.who) : addmm(rows2(A.t(1)), g, A.t(4).t(), s, A.who);
   auto sizes = n.sizes().vec();
   sizes.back() = A.t(4).size(0);
   Tensor r[4] = {out.view(sizes), a, b, g};
@@ -733,14 +846,15 @@ Result swiglu_backward(const Args& A) {
   A.shape(4, a.sizes());
   const Tensor d2 = rows2(A.t(0).to(n.scalar_type()).contiguous()), n2 = rows2(n);
   Tensor dn, dw1, dw3, dw2;
-  if (want(4)) dw2 = at::mm(d2.t(), g);
+  if (want(4)) dw2 = mm(d2.t(), g, s, A.who);
   if (want.any(0xd)) {
-    const Tensor dg = at::mm(d2, A.t(7));
+    const Tensor dg = mm(d2, A.t(7), s, A.who);
     const Tensor da = at::empty_like(a), db = at::empty_like(b);
     check(mega_swiglu_bwd(dg.data_ptr(), a.data_ptr(), b.data_ptr(), da.data_ptr(), db.data_ptr(), dtype_code(n), a.numel(), s), A.who);
-    if (want(2)) dw1 = at::mm(da.t(), n2);
-    if (want(3)) dw3 = at::mm(db.t(), n2);
-    if (want(0)) dn = at::mm(da, A.t(5)).addmm_(db, A.t(6)).view(n.sizes());    // both branches into one gradient: no third pass to add them
+    if (want(2)) dw1 = mm(da.t(), n2, s, A.who);
+    if (want(3)) dw3 = mm(db.t(), n2, s, A.who);
+    if (want(0)) dn = n.scalar_type() == at::kFloat ? addmm(mm(da, A.t(5), s, A.who), db, A.t(6), s, A.who).view(n.sizes())
+                                                    : at::mm(da, A.t(5)).addmm_(db, A.t(6)).view(n.sizes());    // both branches into one gradient: no third pass to add them
   }
   Tensor r[4] = {dn, dw1, dw3, dw2};
   return tuple(r);
@@ -764,11 +878,10 @@ Result mix_forward(const Args& A) {
   A.shape(12, {D});
   const Tensor mx = A.t(1).transpose(1, 2).contiguous();
   if (mx.scalar_type() != xn.scalar_type() || mx.sizes() != xn.sizes()) throw std::runtime_error("mix_forward: mx must be [B, D, L]");
-  Tensor vp = at::addmm(A.t(3), rows2(xn), A.t(2).t());
-  Tensor v = silu(vp, s, A.who);
+  auto [vp, v] = silu_mm(A.t(3), rows2(xn), A.t(2).t(), s, A.who);
   const int act_kind = (int)A.i64(11);
   Tensor act = act_kind == MEGA_TOKEN_RMSNORM ? row_norm(mx, opt_t(A, 12), Tensor(), act_kind, A.d(13), s, A.who) : silu(mx, s, A.who);
-  Tensor base = at::addmm(A.t(5), rows2(act), A.t(4).t());
+  Tensor base = addmm(A.t(5), rows2(act), A.t(4).t(), s, A.who);
   Tensor q = at::empty({T, S}, xn.options()), k = at::empty({T, S}, xn.options());
   check(mega_gate_qk_fwd_raw((const char*)base.data_ptr() + D * xn.element_size(), W, A.t(6).data_ptr(), A.t(7).data_ptr(),
                              (const float*)A.p(8, at::kFloat, S / heads / 2, xn.device()), q.data_ptr(), k.data_ptr(), dt, T, S, heads,
@@ -792,7 +905,7 @@ Result mix_out_forward(const Args& A) {
   const char* b = (const char*)base.data_ptr();
   Tensor gated = at::empty({T, E}, x.options());
   check(mega_gate_mul_fwd(attn.data_ptr(), E, b + (D + S) * es, W, gated.data_ptr(), dt, T, E, s), A.who);
-  Tensor hp = at::mm(gated, A.t(3).t());
+  Tensor hp = mm(gated, A.t(3).t(), s, A.who);
   Tensor out = at::empty_like(x);
   check(mega_gate_out_fwd(x.data_ptr(), D, b, W, b + (D + S + E) * es, W, hp.data_ptr(), D, out.data_ptr(), dt, T, D, s), A.who);
   Tensor r[3] = {out, gated, hp};
@@ -825,9 +938,9 @@ Result mix_out_backward(const Args& A) {
         A.who);
   const Tensor dh = dbase.narrow(1, D + S + E, D);
   Tensor dattn, dhw;
-  if (want(3)) dhw = at::mm(dh.t(), gated);
+  if (want(3)) dhw = mm(dh.t(), gated, s, A.who);
   if (want.any(6)) {
-    const Tensor dgated = at::mm(dh, hw);
+    const Tensor dgated = mm(dh, hw, s, A.who);
     dattn = at::empty_like(attn);
     check(mega_gate_mul_bwd_strided(dgated.data_ptr(), attn.data_ptr(), E, b + (D + S) * es, W, dattn.data_ptr(), db + (D + S) * es, W,
                                     dt, T, E, s),
@@ -870,10 +983,10 @@ Result mix_backward(const Args& A) {
           A.who);
   }
   Tensor dxn, dmx, dvw, dvb, dmxw, dmxb, dmw;
-  if (want(4)) dmxw = at::mm(dbase.t(), rows2(act));
+  if (want(4)) dmxw = mm(dbase.t(), rows2(act), s, A.who);
   if (want(5)) dmxb = sum_rows(dbase, Tensor(), s, A.who).second;
   if (want.any(0x202)) {
-    const Tensor dact = at::mm(dbase, A.t(10)).view(mx.sizes());
+    const Tensor dact = mm(dbase, A.t(10), s, A.who).view(mx.sizes());
     const int act_kind = (int)A.i64(15);
     if (act_kind == MEGA_TOKEN_RMSNORM) {
       Tensor none;
@@ -886,8 +999,8 @@ Result mix_backward(const Args& A) {
   if (want.any(0xd)) {
     Tensor dvp;
     std::tie(dvp, dvb) = sum_rows(dv.view(vp.sizes()), vp, s, A.who);
-    if (want(2)) dvw = at::mm(dvp.t(), rows2(xn));
-    if (want(0)) dxn = at::mm(dvp, A.t(9)).view(xn.sizes());
+    if (want(2)) dvw = mm(dvp.t(), rows2(xn), s, A.who);
+    if (want(0)) dxn = mm(dvp, A.t(9), s, A.who).view(xn.sizes());
   }
   Tensor r[9] = {dxn, dmx, dvw, dvb, dmxw, dmxb, dgamma, dbeta, dmw};
   return tuple(r);
@@ -1066,7 +1179,8 @@ PyMethodDef methods[] = {MEGA_ENTRY(token_gated_attention), MEGA_ENTRY(token_ffn
                          MEGA_ENTRY(ffn_backward),          MEGA_ENTRY(swiglu_forward), MEGA_ENTRY(swiglu_backward),
                          MEGA_ENTRY(mix_forward),           MEGA_ENTRY(mix_out_forward), MEGA_ENTRY(mix_out_backward),
                          MEGA_ENTRY(mix_backward),          MEGA_QUESTION(uniform),    MEGA_QUESTION(trainable),
-                         MEGA_QUESTION(plain_modules), MEGA_QUESTION(wanted),
+                         MEGA_QUESTION(plain_modules), MEGA_QUESTION(wanted),     MEGA_ENTRY(linear_f32),
+                         MEGA_ENTRY(attention_product),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "mega_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

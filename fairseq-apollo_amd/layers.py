@@ -24,7 +24,7 @@ from torch.nn import Parameter
 from . import ops
 from .modules import (AttentionSoftmax, EfficientAttention, FeedForwardFunc, GateMulFunc, GateOutFunc, GateQKFunc,
                       IncrementalState, MixInFunc, MixOutFunc, MultiHeadComplexEMA, MultiHeadEMA, SequenceNorm, SplitFunc,
-                      SplitGrads, SwiGLU, TimestepNorm, _plain, _tensor_versions, _training_call, _unhooked, linear, linear_residual,
+                      SplitGrads, SwiGLU, TimestepNorm, _plain, _tensor_versions, _training_call, _unhooked, linear, linear_residual, project,
                       mask_bytes, mask_bytes_ok, norm_then_move, norm_width_ok, one_graph, row_norm, row_norm_covers, row_norm_formula,
                       silu)
 
@@ -133,7 +133,7 @@ class NormalizedFeedForwardNetwork(nn.Module):
         elif ops.token_rows(x, normalised=True) and self._few_rows_cover(x):
             return self._few_rows(x)
         else:
-            h = ops.silu(self.fc1(self.norm(x)), inplace=True)
+            h = project(self.fc1, self.norm(x), True)
         if self.layerscale_weight is None and not (self.training and self.dropout_p > 0):
             return linear_residual(self.fc2, h, x, consume_input)      # the residual rides in the product
         h = F.dropout(self.fc2(h), self.dropout_p, self.training)
@@ -348,12 +348,12 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
             mx = None
         else:
             x, mx = norm_then_move(self.norm, self.move, x, padding_mask, incremental_state, out_layout="input")
-        v = ops.silu(self.v_proj(x), inplace=True)
+        v = project(self.v_proj, x, True)
         if mx is None:
             mx = self.move(x.transpose(1, 2), padding_mask, incremental_state, out_layout="input")
         mx = mx.transpose(1, 2)
         mx = self.move_act(mx) if isinstance(self.move_act, RMSNorm) else ops.silu(mx, inplace=True)
-        base = self.mx_proj(mx)
+        base = project(self.mx_proj, mx)
         u, z, r, hx = torch.split(base, [self.embed_dim, self.zdim, self.hdim, self.embed_dim], dim=-1)
         Nh = self.num_heads
         if saved_state is None:
@@ -377,7 +377,7 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
             attn = self._cached_attention(z, v, saved_state, incremental_state)
         # the gates are applied where their operands are consumed: r on the way into the output
         # projection, u and the residual mix after it
-        hp = self.h_proj(ops.gate_mul_fwd(attn.reshape(bsz, seq_len, self.hdim), r))
+        hp = project(self.h_proj, ops.gate_mul_fwd(attn.reshape(bsz, seq_len, self.hdim), r))
         return ops.gate_out_fwd(residual, u, hx, hp), None
 
     def _token_covers(self, x: Tensor, padding_mask: Optional[Tensor], saved_state) -> bool:

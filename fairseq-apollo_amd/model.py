@@ -16,7 +16,7 @@ from torch import Tensor, nn
 
 from . import ops
 from .layers import MegaDecoderLayer, _arg
-from .modules import TimestepNorm, _plain, _unhooked
+from .modules import TimestepNorm, _plain, _unhooked, project
 
 
 class MegaDecoderNoCrossAttn(nn.Module):
@@ -78,7 +78,7 @@ class MegaDecoderNoCrossAttn(nn.Module):
             w = proj.weight
             if ops.token_linear_pays(features.size(0), *w.shape) and ops._lib.load_host().uniform(features, w):
                 return ops.token_linear(features, w)
-        return proj(features)
+        return project(proj, features)
 
     def max_positions(self) -> int:
         """Longest sequence the decoder is configured for (mega_lm.py:387-389)."""

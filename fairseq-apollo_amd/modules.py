@@ -1352,6 +1352,23 @@ class EfficientAttention(nn.Module):
         return 'causal={}, dropout={}'.format(self._causal, self._dropout)
 
 
+def own_product(lin: nn.Linear, x: Tensor, *more) -> bool:
+    """lin(x) outside training as one of the library's own fp32 products (16-bit activations keep the GEMM library)."""
+    w, b = lin._parameters.get('weight'), lin._parameters.get('bias')
+    return (x.dtype is torch.float32 and x.is_cuda and x.dim() > 1 and w is not None and not torch.is_grad_enabled()
+            and not torch.compiler.is_compiling() and not torch.is_autocast_enabled() and x.is_contiguous() and x.shape[-1] == w.shape[1]
+            and _plain(b is not None, lin) and ops._lib.load_host().uniform(x, w, b, *more))
+
+
+def project(lin: nn.Linear, x: Tensor, act: bool = False) -> Tensor:
+    """lin(x), or silu(lin(x)), outside training."""
+    if own_product(lin, x):
+        with ops._on_device(x.device):
+            return ops._lib.load_host().linear_f32(x, lin.weight, lin.bias, None, act, False, ops._stream(x.device))
+    y = lin(x)
+    return ops.silu(y, inplace=True) if act else y
+
+
 def linear_residual(lin: nn.Linear, h: Tensor, residual: Optional[Tensor], consume: bool = False) -> Tensor:
     """lin(h) + residual as one library GEMM (the residual is the accumulator's start, rounded once with the
     product); lin(h) when there is no residual.  consume: the caller owns `residual` and has no further use for
@@ -1361,6 +1378,10 @@ def linear_residual(lin: nn.Linear, h: Tensor, residual: Optional[Tensor], consu
         return lin(h)
     if lin.bias is not None or residual.dtype != h.dtype or not residual.is_contiguous():
         return lin(h) + residual
+    if own_product(lin, h, residual) and residual.shape[:-1] == h.shape[:-1] and residual.shape[-1] == lin.weight.shape[0]:
+        with ops._on_device(h.device):
+            return ops._lib.load_host().linear_f32(h, lin.weight, None, residual, False, consume and not residual.requires_grad,
+                                                   ops._stream(h.device))
     r2, h2 = residual.reshape(-1, residual.shape[-1]), h.reshape(-1, h.shape[-1])
     if consume and not torch.is_grad_enabled() and not residual.requires_grad:
         r2.addmm_(h2, lin.weight.t())
@@ -1389,5 +1410,5 @@ class SwiGLU(nn.Module):
                                                              and residual.shape[:-1] == x.shape[:-1]
                                                              and residual.shape[-1] == w2.out_features)):
             return SwiGLUBlockFunc.apply(x, residual, w1.weight, w3.weight, w2.weight)
-        gate = SwiGLUFunc.apply(self.w1(x), self.w3(x)) if _training_call(self, x) else ops.swiglu(self.w1(x), self.w3(x))
+        gate = SwiGLUFunc.apply(self.w1(x), self.w3(x)) if _training_call(self, x) else ops.swiglu(project(w1, x), project(w3, x))
         return linear_residual(self.w2, gate, residual, consume_residual)

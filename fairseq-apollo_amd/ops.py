@@ -631,11 +631,21 @@ def attention_fwd(q, k, v, scale: float, dropout: float, use_causal_mask: bool, 
         # library GEMMs around this library's softmax, which is what the reference does for every shape
         # (attention_kernel.cu:40-131); the library's own fallback is a kernel of one thread per score.  The scores
         # are rounded to the activation type before the softmax, as the reference's are.
-        s = torch.einsum('bqnh,bknh->bnqk', qd, kd)
-        if float(scale) != 1.0:
-            s.mul_(float(scale))
+        own = own_attention_products(L, H1, H2, qd, kd, vd)
+        if own:
+            # (what lies above the diagonal is not formed, and the causal softmax does not read it)
+            s = torch.empty(B, Nh, L, L, dtype=qd.dtype, device=dev)
+            _position_product((qd, 0), (kd, 0), (s, 1), L, L, H1, 1 if use_causal_mask else 0, float(scale))
+        else:
+            s = torch.einsum('bqnh,bknh->bnqk', qd, kd)
+            if float(scale) != 1.0:
+                s.mul_(float(scale))
         wts = attention_softmax_fwd(s, dropout, use_causal_mask, seed)
         del s
+        if own:
+            if not weights_only:
+                _position_product((wts, 1), (vd, 0), (y, 0), L, H2, L, 2 if use_causal_mask else 0, b_rows=True)
+            return y, (wts if need_weights else None)
         y = None if weights_only else torch.einsum('bnqk,bknh->bqnh', wts, vd).contiguous()
         return y, (wts if need_weights else None)
     ws = _scratch_buffer(dev, nws) if nws else None
@@ -645,6 +655,28 @@ def attention_fwd(q, k, v, scale: float, dropout: float, use_causal_mask: bool, 
                                     ws.numel() if nws else 0, _stream(dev))
     _lib.check(rc, "attention_fwd")
     return y, w
+
+
+def _position_product(a, b, c, M, N, K, causal=0, alpha=1.0, a_rows=False, b_rows=False):
+    """c = alpha a b per batch entry and head, fp32.  Operands (tensor, kind), contiguous: kind 0 [B, L, Nh, H] (positions by
+    features), 1 [B, Nh, L, L] (weights); a(m, k), b(n, k): the reduction runs along the last axis, or with a_rows / b_rows
+    along the positions before it."""
+    def of(t, weights):
+        B, d1, d2, d3 = t.shape
+        return (d3, d1 * d2 * d3, d2 * d3) if weights else (d2 * d3, d1 * d2 * d3, d3)
+    (a, aw), (b, bw), (c, cw) = a, b, c
+    Nh = a.shape[1] if aw else a.shape[2]
+    with _on_device(a.device):
+        _lib.load_host().attention_product(a, b, c, M, N, K, a.shape[0], Nh, *of(a, aw), a_rows, *of(b, bw), b_rows, *of(c, cw),
+                                           causal, alpha, _stream(a.device))
+    return c
+
+
+def own_attention_products(L: int, H1: int, H2: int, *ts) -> bool:
+    """fp32 attention of whole 16-byte rows: its products run on the library's matrix-core kernel.  Sizes that 16-byte
+    accesses do not fit keep the GEMM library (element-wise loads are slower than its kernels, if not than its call)."""
+    return all(t.dtype is torch.float32 for t in ts) and L >= 64 and not (L % 4 or H1 % 4 or H2 % 4) and \
+        not torch.compiler.is_compiling() and not torch.is_autocast_enabled() and _lib.load_host().uniform(*ts)
 
 
 def attention_softmax_bwd(y_grad: torch.Tensor, y: torch.Tensor, use_causal_mask: bool, scale: float = 1.0,
@@ -715,6 +747,15 @@ def attention_bwd(y_grad, q, k, v, w, scale: float, use_causal_mask: bool, y=Non
                                         _ptr(v_grad), _dtype_code(qd), B, L, Nh, H1, H2, float(scale),
                                         1 if use_causal_mask else 0, _ptr(ws), ws.numel(), _stream(dev))
         _lib.check(rc, "attention_bwd")
+        return q_grad, k_grad, v_grad
+    if qd.numel() and own_attention_products(L, H1, H2, qd, kd, vd, wd, g):
+        c = use_causal_mask
+        q_grad, k_grad, v_grad, ds = (torch.empty_like(t) for t in (qd, kd, vd, wd))
+        _position_product((wd, 1), (g, 0), (v_grad, 0), L, H2, L, 3 if c else 0, a_rows=True, b_rows=True)
+        _position_product((g, 0), (vd, 0), (ds, 1), L, L, H2, 1 if c else 0)
+        attention_softmax_bwd(ds, wd, c, scale=float(scale), inplace=True)
+        _position_product((ds, 1), (qd, 0), (k_grad, 0), L, H1, L, 3 if c else 0, a_rows=True, b_rows=True)
+        _position_product((ds, 1), (kd, 0), (q_grad, 0), L, H1, L, 2 if c else 0, b_rows=True)
         return q_grad, k_grad, v_grad
     v_grad = torch.einsum('bnqk,bqnh->bknh', wd, g)
     w_grad = torch.einsum('bqnh,bknh->bnqk', g, vd).contiguous()

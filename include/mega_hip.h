@@ -408,6 +408,27 @@ int mega_norm_ema_steps(const void* x, void* xn, void* y, int dtype, int64_t K,
  * other or when image == NULL (kernel generation inside the call).                          */
 size_t mega_norm_ema_fwd_workspace_bytes(int64_t B, int64_t L, int64_t D, int64_t G, int64_t N);
 size_t mega_norm_ema_fwd_scratch_bytes(int64_t B, int64_t L, int64_t D, int64_t G, int64_t N);
+/* ---- single-precision matrix products on the matrix cores (csrc/gemm.hip).
+ * C[m][n] = alpha sum_k A(m, k) B(n, k) (+ bias[n]) (+ residual[m][n]); silu: C = silu of that, and `pre` (optional)
+ * gets the value before it.  A(m, k) lies at m lda + k, or with a_kmajor at k lda + m; B(n, k) alike.  fp32 throughout,
+ * any sizes and strides (16-byte accesses where they fit).  Batched: entry o inner + i adds o s? + i s?i to the bases
+ * (no bias, residual or activation then).  causal: 1: elements with n > m need not be formed; 2: A(m, k) is zero for
+ * k > m; 3: A(m, k) is zero for k < m (positions of M against N or K).
+ * Workspace: mega_gemm_workspace_bytes (no initialisation; 0: none), for products split along K.               */
+typedef struct {
+  const void *a, *b;
+  void* c;
+  const void *bias, *residual;
+  void* pre;
+  int64_t lda, ldb, ldc, ldr;
+  int64_t sa, sai, sb, sbi, sc, sci;
+  int64_t M, N, K, batch, inner;
+  int32_t a_kmajor, b_kmajor, causal, silu;
+  float alpha;
+} MegaGemm;
+size_t mega_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t batch);
+int mega_gemm_f32(const MegaGemm* g, void* workspace, size_t workspace_bytes, void* stream);
+
 /* 1 when calls of these sizes run as one kernel (carried: with h_in; rows_out: y as [B,D,L] rows), else 0 */
 int mega_norm_ema_fwd_one_kernel(int dtype, int64_t B, int64_t L, int64_t D, int64_t G, int64_t N, int carried,
                                  int rows_out);

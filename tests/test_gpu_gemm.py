@@ -1,0 +1,126 @@
+"""fp32 products on the matrix cores (mega_gemm_f32) against 64-bit products: every storage order, tile and step
+remainders, products split along the reduction, epilogues, batched causal forms, values that are not finite; and the
+callers that hand their products over (linear layers outside training, attention)."""
+import ctypes as C
+import math
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+import fairseq_apollo_amd as M
+from gpu_util import DEV
+
+pytestmark = pytest.mark.gpu
+
+
+class _Gemm(C.Structure):
+    _fields_ = [(n, C.c_void_p) for n in ("a", "b", "c", "bias", "residual", "pre")] + \
+        [(n, C.c_int64) for n in ("lda", "ldb", "ldc", "ldr", "sa", "sai", "sb", "sbi", "sc", "sci", "M", "N", "K", "batch", "inner")] + \
+        [(n, C.c_int32) for n in ("a_kmajor", "b_kmajor", "causal", "silu")] + [("alpha", C.c_float)]
+
+
+def _tol(K):
+    """Roundings of the running sum, six for every 32 reduction indices and of either sign, beside the result's own."""
+    return 2.0 ** -24 * (2 + math.sqrt(6 * (K / 32 + 1)))
+
+
+def _gemm(a, b, ka, kb, bias=None, residual=None, silu=False, pre=False, alpha=1.0):
+    """a [M, K], b [N, K] as given or (ka / kb) stored transposed, rows cut out of wider memory where `wide` made them"""
+    lib = M._lib.load()
+    m, k = (a.shape[1], a.shape[0]) if ka else a.shape
+    n = b.shape[1] if kb else b.shape[0]
+    c = torch.full((m, n), float("nan"), device=DEV)
+    p = torch.full((m, n), float("nan"), device=DEV) if pre else None
+    ptr = lambda t: None if t is None else t.data_ptr()
+    g = _Gemm(ptr(a), ptr(b), ptr(c), ptr(bias), ptr(residual), ptr(p), a.stride(0), b.stride(0), n,
+              residual.stride(0) if residual is not None else 0, 0, 0, 0, 0, 0, 0, m, n, k, 1, 1, ka, kb, 0, silu, alpha)
+    nws = lib.mega_gemm_workspace_bytes(m, n, k, 1)
+    ws = torch.empty(max(nws, 16), dtype=torch.uint8, device=DEV)
+    rc = lib.mega_gemm_f32(C.byref(g), ws.data_ptr(), nws, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib.mega_last_error()
+    torch.cuda.synchronize()
+    return (c, p) if pre else c
+
+
+def _rel(x, r):
+    return ((x.double() - r).norm() / r.norm().clamp_min(1e-300)).item()
+
+
+@pytest.mark.parametrize("ka,kb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("m,n,k,wide", [(1, 1, 1, 0), (3, 5, 7, 0), (64, 64, 32, 0), (68, 60, 36, 0), (65, 63, 33, 1), (132, 260, 100, 4),
+                                        (36, 4, 132, 0), (300, 140, 2052, 0), (64, 128, 8000, 0), (4100, 4100, 36, 0), (4096, 4224, 64, 4)])
+def test_products_of_every_order_and_remainder(m, n, k, wide, ka, kb):
+    """wide: columns beside the operands' own in memory (1: rows off 16 bytes)."""
+    print(f"case m={m} n={n} k={k} wide={wide} ka={ka} kb={kb}", flush=True)
+    gen = torch.Generator(DEV).manual_seed(m + n + k)
+    mk = lambda r, c: torch.randn(r, c + wide, generator=gen, device=DEV)[:, :c] * 3
+    a, b = mk(k, m) if ka else mk(m, k), mk(k, n) if kb else mk(n, k)
+    r = (a.double().t() if ka else a.double()) @ (b.double() if kb else b.double().t())
+    assert _rel(_gemm(a, b, ka, kb), r) < _tol(k)
+
+
+@pytest.mark.parametrize("m,n,k", [(70, 66, 40), (40, 96, 2048), (129, 7, 65)])
+def test_epilogues(m, n, k):
+    gen = torch.Generator(DEV).manual_seed(5)
+    mk = lambda *s: torch.randn(*s, generator=gen, device=DEV)
+    a, b, bias, res = mk(m, k), mk(n, k), mk(n), mk(m, n)
+    r = 0.5 * (a.double() @ b.double().t()) + bias.double() + res.double()
+    c, pre = _gemm(a, b, 0, 0, bias, res, True, True, 0.5)
+    assert _rel(pre, r) < _tol(k)
+    assert _rel(c, F.silu(r)) < _tol(k) + 2.0 ** -22          # (expf and the division: a few units more)
+
+
+@pytest.mark.parametrize("L,H1,H2", [(64, 8, 12), (100, 16, 20), (260, 64, 128), (1000, 32, 64)])
+def test_attention_products_and_gradients(L, H1, H2):
+    """q k^T, w v and the four products behind them, causal and not, two heads, against 64 bits."""
+    B, Nh = 2, 2
+    gen = torch.Generator(DEV).manual_seed(L)
+    mk = lambda h: torch.randn(B, L, Nh, h, generator=gen, device=DEV)
+    q, k, v, g = mk(H1), mk(H1), mk(H2), mk(H2)
+    for causal in (True, False):
+        print(f"case L={L} H1={H1} H2={H2} causal={causal}", flush=True)
+        assert M.ops.own_attention_products(L, H1, H2, q, k, v)
+        y, w = M.ops.attention_fwd(q, k, v, 0.3, 0.0, causal, need_weights=True)
+        t = [x.double().transpose(1, 2).contiguous().requires_grad_() for x in (q, k, v)]
+        s = 0.3 * (t[0] @ t[1].transpose(-1, -2))
+        if causal:
+            s = s.masked_fill(torch.ones(L, L, dtype=torch.bool, device=DEV).triu(1), float("-inf"))
+        ref = s.softmax(-1) @ t[2]
+        ref.backward(g.double().transpose(1, 2))
+        got = M.ops.attention_bwd(g, q, k, v, w, 0.3, causal)
+        torch.cuda.synchronize()
+        # exp of scores with an absolute error of |s| 2^-23 or so, through two more products
+        assert _rel(y.transpose(1, 2), ref) < 4e-6
+        for x, r in zip(got, t):
+            assert _rel(x.transpose(1, 2), r.grad) < 1e-5
+
+
+def test_values_that_are_not_finite():
+    gen = torch.Generator(DEV).manual_seed(9)
+    a, b = torch.randn(200, 300, generator=gen, device=DEV), torch.randn(150, 300, generator=gen, device=DEV)
+    a[3, 5], a[7, 9], b[11, 100], a[20, 100], b[12, 7] = float("inf"), float("nan"), 3.4e38, 0.25, float("-inf")
+    c, r = _gemm(a, b, 0, 0), (a.double() @ b.double().t()).float()
+    assert torch.equal(torch.isnan(c), torch.isnan(r)) and torch.equal(torch.isposinf(c), torch.isposinf(r))
+    ok = torch.isfinite(r)
+    assert _rel(c[ok], r[ok].double()) < _tol(300)
+
+
+def test_linear_layers_outside_training():
+    """project / linear_residual: bias, silu, a residual consumed in place; hooked and replaced layers keep their own call."""
+    x, res = torch.randn(3, 50, 96, device=DEV), torch.randn(3, 50, 72, device=DEV)
+    lin, nob = torch.nn.Linear(96, 72).to(DEV), torch.nn.Linear(96, 72, bias=False).to(DEV)
+    with torch.no_grad():
+        r = F.linear(x.double(), lin.weight.double(), lin.bias.double())
+        assert M.modules.own_product(lin, x)
+        assert _rel(M.modules.project(lin, x), r) < _tol(96)
+        assert _rel(M.modules.project(lin, x, True), F.silu(r)) < _tol(96) + 2.0 ** -22
+        want = F.linear(x.double(), nob.weight.double()) + res.double()
+        assert _rel(M.modules.linear_residual(nob, x, res), want) < _tol(96)
+        out = M.modules.linear_residual(nob, x, res, True)
+        assert out.data_ptr() == res.data_ptr() and _rel(out, want) < _tol(96)
+        hook = lin.register_forward_hook(lambda m, i, o: o * 0)
+        assert not M.modules.own_product(lin, x) and not M.modules.project(lin, x).any()
+        hook.remove()
+        assert not M.modules.own_product(lin, x.transpose(0, 1)) and not M.modules.own_product(lin, x.half())
+    assert not M.modules.own_product(lin, x)
