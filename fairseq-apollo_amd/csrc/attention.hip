@@ -48,33 +48,89 @@ __device__ __forceinline__ float drop_key(float v, float dropout, uint64_t seed,
   return (dropout > 0.f && hash_uniform(seed, idx) < dropout) ? -INFINITY : v;
 }
 
-// one workgroup per row
-template <typename T>
-__global__ __launch_bounds__(kBlock) void softmax_kernel(const T* __restrict__ x, T* __restrict__ y,
-                                                         int64_t outer, int64_t inner, int causal, float dropout,
-                                                         uint64_t seed) {
+// One workgroup per row of pitch ld; columns beyond `inner` become zeros.  mask: [rows / per, inner], nonzero = the key is
+// left out (a row of it that leaves out every key is no mask).  R > 0: the row's values stay in registers, R to a
+// thread, between the three passes over them (inner <= R * kBlock; x may be y).  Bound by memory: 8000 rows x 1000 fp32
+// 24 us with three reads of every value, 16 us so.
+template <typename T, int R>
+__global__ __launch_bounds__(kBlock) void softmax_kernel(const T* x, T* y, int64_t outer, int64_t inner, int64_t ld, int causal,
+                                                         float dropout, uint64_t seed, const uint8_t* __restrict__ mask,
+                                                         int64_t per) {
   __shared__ float red[kBlock / 64];
   const int64_t row = blockIdx.x;
   const int64_t r = row % outer;
   int64_t n = causal ? inner - outer + r + 1 : inner;
   if (n < 0) n = 0;
-  const T* xp = x + row * inner;
-  T* yp = y + row * inner;
+  const T* xp = x + row * ld;
+  T* yp = y + row * ld;
   const uint64_t e0 = (uint64_t)row * (uint64_t)inner;
+  const uint8_t* mp = mask ? mask + (row / per) * inner : nullptr;
+  if (mp) {
+    float open = 0.f;
+    for (int64_t j = threadIdx.x; j < n; j += kBlock) open = mp[j] ? open : 1.f;
+    if (block_reduce(open, red, true) == 0.f) mp = nullptr;
+  }
+  auto value = [&](int64_t j) {
+    return mp && mp[j] ? -INFINITY : drop_key(to_float(xp[j]), dropout, seed, e0 + j);
+  };
+  float v[R > 0 ? R : 1];
   float m = -INFINITY;
-  for (int64_t j = threadIdx.x; j < n; j += kBlock) m = fmaxf(m, drop_key(to_float(xp[j]), dropout, seed, e0 + j));
+  if constexpr (R > 0) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int64_t j = threadIdx.x + i * kBlock;
+      v[i] = j < n ? value(j) : -INFINITY;
+      m = fmaxf(m, v[i]);
+    }
+  } else {
+    for (int64_t j = threadIdx.x; j < n; j += kBlock) m = fmaxf(m, value(j));
+  }
   m = block_reduce(m, red, true);
   const bool dead = !(m > -INFINITY) || !(m < INFINITY);
   float s = 0.f;
-  if (!dead)
-    for (int64_t j = threadIdx.x; j < n; j += kBlock)
-      s += __expf(drop_key(to_float(xp[j]), dropout, seed, e0 + j) - m);
+  if (!dead) {
+    if constexpr (R > 0) {
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        v[i] = threadIdx.x + i * kBlock < n ? __expf(v[i] - m) : 0.f;
+        s += v[i];
+      }
+    } else {
+      for (int64_t j = threadIdx.x; j < n; j += kBlock) s += __expf(value(j) - m);
+    }
+  }
   s = block_reduce(s, red, false);
   const float c = (dead || s == 0.f) ? 0.f : 1.0f / s;
-  for (int64_t j = threadIdx.x; j < inner; j += kBlock) {
-    const float e = (j < n && !dead) ? __expf(drop_key(to_float(xp[j]), dropout, seed, e0 + j) - m) * c : 0.f;
-    yp[j] = from_float<T>(e);
+  if constexpr (R > 0) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int64_t j = threadIdx.x + i * kBlock;
+      if (j < ld) yp[j] = from_float<T>(dead ? 0.f : v[i] * c);
+    }
+    for (int64_t j = threadIdx.x + R * kBlock; j < ld; j += kBlock) yp[j] = from_float<T>(0.f);
+  } else {
+    for (int64_t j = threadIdx.x; j < ld; j += kBlock) {
+      const float e = (j < n && !dead) ? __expf(value(j) - m) * c : 0.f;
+      yp[j] = from_float<T>(e);
+    }
   }
+}
+
+template <typename T>
+int launch_softmax(const void* x, void* y, int64_t rows, int64_t outer, int64_t inner, int64_t ld, int causal, float dropout,
+                   uint64_t seed, const uint8_t* mask, int64_t per, hipStream_t s) {
+  const dim3 grid((unsigned)rows);
+  if (inner <= 4 * kBlock)
+    hipLaunchKernelGGL((softmax_kernel<T, 4>), grid, dim3(kBlock), 0, s, (const T*)x, (T*)y, outer, inner, ld, causal, dropout,
+                       seed, mask, per);
+  else if (inner <= 8 * kBlock)
+    hipLaunchKernelGGL((softmax_kernel<T, 8>), grid, dim3(kBlock), 0, s, (const T*)x, (T*)y, outer, inner, ld, causal, dropout,
+                       seed, mask, per);
+  else
+    hipLaunchKernelGGL((softmax_kernel<T, 0>), grid, dim3(kBlock), 0, s, (const T*)x, (T*)y, outer, inner, ld, causal, dropout,
+                       seed, mask, per);
+  MEGA_CHECK_LAUNCH("attention_softmax_fwd");
+  return MEGA_OK;
 }
 
 // Plain attention: one workgroup per (b, head, query row); scores of the row live in LDS.
@@ -134,7 +190,7 @@ __global__ __launch_bounds__(kBlock) void attention_row_kernel(const T* __restri
 // written as zeros without being read.  dx may alias dy.
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void softmax_bwd_kernel(const T* dy, const T* __restrict__ y,
-                                                          T* dx, int64_t rows, int outer, int inner, int causal,
+                                                          T* dx, int64_t rows, int outer, int inner, int ld, int causal,
                                                           float scale) {
   using V = Vec<T, VEC>;
   const int lane = threadIdx.x & 63;
@@ -144,9 +200,9 @@ __global__ __launch_bounds__(256) void softmax_bwd_kernel(const T* dy, const T* 
   int limit = causal ? inner - outer + r + 1 : inner;     // columns that can be non-zero
   if (limit < 0) limit = 0;
   if (limit > inner) limit = inner;
-  const T* dyr = dy + row * inner;
-  const T* yr = y + row * inner;
-  T* dxr = dx + row * inner;
+  const T* dyr = dy + row * ld;
+  const T* yr = y + row * ld;
+  T* dxr = dx + row * ld;
   float dot = 0.f;
   for (int c = lane * VEC; c < limit; c += 64 * VEC) {
     const V a = *(const V*)(dyr + c);
@@ -157,7 +213,7 @@ __global__ __launch_bounds__(256) void softmax_bwd_kernel(const T* dy, const T* 
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) dot += __shfl_xor(dot, o);
-  for (int c = lane * VEC; c < inner; c += 64 * VEC) {
+  for (int c = lane * VEC; c < ld; c += 64 * VEC) {
     V o;
     if (c < limit) {
       const V a = *(const V*)(dyr + c);
@@ -174,17 +230,17 @@ __global__ __launch_bounds__(256) void softmax_bwd_kernel(const T* dy, const T* 
 }
 
 template <typename T>
-int launch_softmax_bwd(const void* dy, const void* y, void* dx, int64_t rows, int64_t outer, int64_t inner, int causal,
-                       float scale, hipStream_t s) {
+int launch_softmax_bwd(const void* dy, const void* y, void* dx, int64_t rows, int64_t outer, int64_t inner, int64_t ld,
+                       int causal, float scale, hipStream_t s) {
   constexpr int FULL = 16 / (int)sizeof(T);
   const dim3 grid((unsigned)ceil_div(rows, 4));
-  const bool vec = inner % FULL == 0 && ((((uintptr_t)dy | (uintptr_t)y | (uintptr_t)dx) % 16) == 0);
+  const bool vec = ld % FULL == 0 && ((((uintptr_t)dy | (uintptr_t)y | (uintptr_t)dx) % 16) == 0);
   if (vec)
     hipLaunchKernelGGL((softmax_bwd_kernel<T, FULL>), grid, dim3(256), 0, s, (const T*)dy, (const T*)y, (T*)dx, rows,
-                       (int)outer, (int)inner, causal, scale);
+                       (int)outer, (int)inner, (int)ld, causal, scale);
   else
     hipLaunchKernelGGL((softmax_bwd_kernel<T, 1>), grid, dim3(256), 0, s, (const T*)dy, (const T*)y, (T*)dx, rows,
-                       (int)outer, (int)inner, causal, scale);
+                       (int)outer, (int)inner, (int)ld, causal, scale);
   MEGA_CHECK_LAUNCH("attention_softmax_bwd");
   return MEGA_OK;
 }
@@ -206,23 +262,47 @@ extern "C" int mega_attention_softmax_fwd(const void* x, void* y, int dtype, int
   MEGA_REQUIRE(x && y, MEGA_ERR_ARG, "attention_softmax_fwd: null pointer argument");
   MEGA_REQUIRE(rows < (int64_t)1 << 31, MEGA_ERR_UNSUPPORTED, "attention_softmax_fwd: too many rows");
   hipStream_t s = (hipStream_t)stream;
-  const dim3 grid((unsigned)rows);
   switch (dtype) {
-    case MEGA_F32:
-      hipLaunchKernelGGL(softmax_kernel<float>, grid, dim3(kBlock), 0, s, (const float*)x, (float*)y, outer, inner, causal,
-                         dropout, seed);
-      break;
-    case MEGA_BF16:
-      hipLaunchKernelGGL(softmax_kernel<bf16_t>, grid, dim3(kBlock), 0, s, (const bf16_t*)x, (bf16_t*)y, outer, inner, causal,
-                         dropout, seed);
-      break;
-    default:
-      hipLaunchKernelGGL(softmax_kernel<f16_t>, grid, dim3(kBlock), 0, s, (const f16_t*)x, (f16_t*)y, outer, inner, causal,
-                         dropout, seed);
-      break;
+    case MEGA_F32: return launch_softmax<float>(x, y, rows, outer, inner, inner, causal, dropout, seed, nullptr, 1, s);
+    case MEGA_BF16: return launch_softmax<bf16_t>(x, y, rows, outer, inner, inner, causal, dropout, seed, nullptr, 1, s);
+    default: return launch_softmax<f16_t>(x, y, rows, outer, inner, inner, causal, dropout, seed, nullptr, 1, s);
   }
-  MEGA_CHECK_LAUNCH("attention_softmax_fwd");
+}
+
+static int softmax_rows_ok(const char* who, int dtype, int64_t batch, int64_t outer, int64_t inner, int64_t ld) {
+  MEGA_REQUIRE(dtype == MEGA_F32 || dtype == MEGA_BF16 || dtype == MEGA_F16, MEGA_ERR_ARG, "%s: unknown dtype %d", who, dtype);
+  MEGA_REQUIRE(batch >= 0 && outer >= 0 && inner >= 0 && ld >= inner, MEGA_ERR_ARG, "%s: bad size", who);
+  MEGA_REQUIRE(batch * outer < (int64_t)1 << 31 && ld < (int64_t)1 << 30, MEGA_ERR_UNSUPPORTED, "%s: too many rows or columns", who);
   return MEGA_OK;
+}
+
+extern "C" int mega_attention_softmax_keys_fwd(const void* x, void* y, int dtype, int64_t batch, int64_t outer, int64_t inner,
+                                               int64_t ld, const uint8_t* mask, int64_t heads, void* stream) {
+  if (const int rc = softmax_rows_ok("attention_softmax_keys_fwd", dtype, batch, outer, inner, ld)) return rc;
+  MEGA_REQUIRE(heads >= 1 && batch % heads == 0, MEGA_ERR_ARG, "attention_softmax_keys_fwd: batch counts whole sets of heads");
+  const int64_t rows = batch * outer, per = heads * outer;
+  if (rows == 0 || inner == 0) return MEGA_OK;
+  MEGA_REQUIRE(x && y, MEGA_ERR_ARG, "attention_softmax_keys_fwd: null pointer argument");
+  hipStream_t s = (hipStream_t)stream;
+  switch (dtype) {
+    case MEGA_F32: return launch_softmax<float>(x, y, rows, outer, inner, ld, 0, 0.f, 0, mask, per, s);
+    case MEGA_BF16: return launch_softmax<bf16_t>(x, y, rows, outer, inner, ld, 0, 0.f, 0, mask, per, s);
+    default: return launch_softmax<f16_t>(x, y, rows, outer, inner, ld, 0, 0.f, 0, mask, per, s);
+  }
+}
+
+extern "C" int mega_attention_softmax_ld_bwd(const void* dy, const void* y, void* dx, int dtype, int64_t batch, int64_t outer,
+                                             int64_t inner, int64_t ld, float scale, void* stream) {
+  if (const int rc = softmax_rows_ok("attention_softmax_ld_bwd", dtype, batch, outer, inner, ld)) return rc;
+  const int64_t rows = batch * outer;
+  if (rows == 0 || inner == 0) return MEGA_OK;
+  MEGA_REQUIRE(dy && y && dx, MEGA_ERR_ARG, "attention_softmax_ld_bwd: null pointer argument");
+  hipStream_t s = (hipStream_t)stream;
+  switch (dtype) {
+    case MEGA_F32: return launch_softmax_bwd<float>(dy, y, dx, rows, outer, inner, ld, 0, scale, s);
+    case MEGA_BF16: return launch_softmax_bwd<bf16_t>(dy, y, dx, rows, outer, inner, ld, 0, scale, s);
+    default: return launch_softmax_bwd<f16_t>(dy, y, dx, rows, outer, inner, ld, 0, scale, s);
+  }
 }
 
 extern "C" size_t mega_attention_workspace_bytes(int dtype, int64_t B, int64_t L, int64_t Nh, int64_t H1,
@@ -287,9 +367,9 @@ extern "C" int mega_attention_softmax_bwd(const void* y_grad, const void* y, voi
                "attention_softmax_bwd: shape too large");
   hipStream_t s = (hipStream_t)stream;
   switch (dtype) {
-    case MEGA_F32: return launch_softmax_bwd<float>(y_grad, y, x_grad, rows, outer, inner, causal, scale, s);
-    case MEGA_BF16: return launch_softmax_bwd<bf16_t>(y_grad, y, x_grad, rows, outer, inner, causal, scale, s);
-    default: return launch_softmax_bwd<f16_t>(y_grad, y, x_grad, rows, outer, inner, causal, scale, s);
+    case MEGA_F32: return launch_softmax_bwd<float>(y_grad, y, x_grad, rows, outer, inner, inner, causal, scale, s);
+    case MEGA_BF16: return launch_softmax_bwd<bf16_t>(y_grad, y, x_grad, rows, outer, inner, inner, causal, scale, s);
+    default: return launch_softmax_bwd<f16_t>(y_grad, y, x_grad, rows, outer, inner, inner, causal, scale, s);
   }
 }
 

@@ -100,8 +100,9 @@ struct Side {
   static __device__ __forceinline__ uint32_t offset(int64_t ld, int tid, int h, int room, int left) {
     int w, k;
     piece(tid, h, w, k);
-    w = min(w, KM ? room - 4 : room - 1);
-    k = min(k, KM ? left - 1 : left - 4);
+    // (sizes that are no multiple of four come with padded rows: the last piece is whole in memory)
+    w = min(w, KM ? ((room + 3) & ~3) - 4 : room - 1);
+    k = min(k, KM ? left - 1 : ((left + 3) & ~3) - 4);
     return (uint32_t)((KM ? (int64_t)k * ld + w : (int64_t)w * ld + k) * 4);
   }
   static __device__ __forceinline__ void load(const float* tile, const uint32_t (&off)[NP], float4 (&v)[NP]) {
@@ -113,7 +114,14 @@ struct Side {
     for (int h = 0; h < NP; ++h) {
       int w, k;
       piece(tid, h, w, k);
-      if (k >= left) v[h] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if constexpr (KM) {
+        if (k >= left) v[h] = make_float4(0.f, 0.f, 0.f, 0.f);
+      } else {
+        v[h].x = k < left ? v[h].x : 0.f;
+        v[h].y = k + 1 < left ? v[h].y : 0.f;
+        v[h].z = k + 2 < left ? v[h].z : 0.f;
+        v[h].w = k + 3 < left ? v[h].w : 0.f;
+      }
     }
   }
   // the same for operands off 16 bytes or of odd sizes, element by element
@@ -473,7 +481,7 @@ extern "C" int mega_gemm_f32(const MegaGemm* g, void* workspace, size_t workspac
   };
   // (whole pieces along the contiguous axis, a tile's rows within 4 GB of its first element)
   const int64_t far = ((int64_t)1 << 32) / 4 / 128;
-  const bool edge = !(on16(g->a, g->lda, g->sa, g->sai) && (g->a_kmajor ? g->M : g->K) % 4 == 0 && g->lda < far &&
+  const bool edge = !(on16(g->a, g->lda, g->sa, g->sai) && (g->a_padded || (g->a_kmajor ? g->M : g->K) % 4 == 0) && g->lda < far &&
                       on16(g->b, g->ldb, g->sb, g->sbi) && (g->b_kmajor ? g->N : g->K) % 4 == 0 && g->ldb < far);
   G.vc = on16(g->c, g->ldc, g->sc, g->sci) && (uintptr_t)g->pre % 16 == 0;
   Plan p = gemm_plan(g->M, g->N, g->K, g->batch);

@@ -715,9 +715,10 @@ Result linear_f32(const Args& A) {
 }
 
 // Batched fp32 products over the positions and heads of attention: (a, b, c, M, N, K, batch, heads, a's row stride, batch
-// stride, head stride, reduction along its rows, the same four of b, c's row, batch and head stride, causal, alpha, stream)
+// stride, head stride, reduction along its rows, the same four of b, c's row, batch and head stride, causal, alpha, a's rows
+// are padded to whole pieces of four, stream)
 Result attention_product(const Args& A) {
-  A.want(22);
+  A.want(23);
   MegaGemm g = {};
   const Tensor& a = A.t(0);
   same_type(A, {0, 1, 2}, a);
@@ -727,19 +728,20 @@ Result attention_product(const Args& A) {
   g.lda = A.i64(8); g.sa = A.i64(9); g.sai = A.i64(10); g.a_kmajor = A.flag(11);
   g.ldb = A.i64(12); g.sb = A.i64(13); g.sbi = A.i64(14); g.b_kmajor = A.flag(15);
   g.ldc = A.i64(16); g.sc = A.i64(17); g.sci = A.i64(18);
-  g.causal = (int)A.i64(19); g.alpha = (float)A.d(20);
+  g.causal = (int)A.i64(19); g.alpha = (float)A.d(20); g.a_padded = A.flag(21);
   auto inside = [&](const Tensor& t, int64_t rows, int64_t cols, int64_t ld, int64_t sb, int64_t si) {
     return ld >= 0 && sb >= 0 && si >= 0 &&
            (A.i64(6) - 1) * sb + (g.inner - 1) * si + (rows - 1) * ld + cols <= t.numel();
   };
+  if (g.a_padded && g.lda % 4) throw std::runtime_error("attention_product: padded rows are whole pieces");
   if (g.M < 1 || g.N < 1 || g.K < 1 || A.i64(6) < 1 || g.inner < 1 ||
-      !inside(a, g.a_kmajor ? g.K : g.M, g.a_kmajor ? g.M : g.K, g.lda, g.sa, g.sai) ||
+      !inside(a, g.a_kmajor ? g.K : g.M, g.a_padded ? g.lda : g.a_kmajor ? g.M : g.K, g.lda, g.sa, g.sai) ||
       !inside(A.t(1), g.b_kmajor ? g.K : g.N, g.b_kmajor ? g.N : g.K, g.ldb, g.sb, g.sbi) || !inside(A.t(2), g.M, g.N, g.ldc, g.sc, g.sci))
     throw std::runtime_error("attention_product: sizes beyond an operand");
   const int64_t nws = (int64_t)mega_gemm_workspace_bytes(g.M, g.N, g.K, g.batch);
   Tensor ws;
   if (nws) ws = at::empty({nws}, a.options().dtype(at::kByte));
-  check(mega_gemm_f32(&g, nws ? ws.data_ptr() : nullptr, (size_t)nws, A.stream(21)), A.who);
+  check(mega_gemm_f32(&g, nws ? ws.data_ptr() : nullptr, (size_t)nws, A.stream(22)), A.who);
   return Result();
 }
 

@@ -23,7 +23,7 @@ from torch.nn import Parameter
 
 from . import ops
 from .modules import (AttentionSoftmax, EfficientAttention, FeedForwardFunc, GateMulFunc, GateOutFunc, GateQKFunc,
-                      IncrementalState, MixInFunc, MixOutFunc, MultiHeadComplexEMA, MultiHeadEMA, SequenceNorm, SplitFunc,
+                      IncrementalState, MixInFunc, MixOutFunc, PaddedAttentionFunc, MultiHeadComplexEMA, MultiHeadEMA, SequenceNorm, SplitFunc,
                       SplitGrads, SwiGLU, TimestepNorm, _plain, _tensor_versions, _training_call, _unhooked, linear, linear_residual, project,
                       mask_bytes, mask_bytes_ok, norm_then_move, norm_width_ok, one_graph, row_norm, row_norm_covers, row_norm_formula,
                       silu)
@@ -475,6 +475,8 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
         learned relative bias is added to the scores, scores of padded keys are -inf except in chunks
         that consist of padding only; library GEMMs around the softmax op (causal for one-sided
         layers)."""
+        if self._padded_product(q4, k4, v4, key_padding):
+            return ops.padded_attention_fwd(q4, k4, v4, key_padding)[0]
         s = torch.einsum('bqnh,bknh->bnqk', q4, k4)
         if isinstance(self.rel_pos_bias, SimpleRelativePositionalBias):
             s = s + self.rel_pos_bias(q4.size(1)).to(s.dtype)
@@ -613,6 +615,9 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
                                            else padding_mask.reshape(q4.shape[:2]))
         elif simple or self._keep_weights or (self.bidirectional and padding_mask is not None) or \
                 (self._weight_dropout and self.training):
+            pad = None if padding_mask is None or not self.bidirectional else padding_mask.reshape(q4.shape[:2])
+            if not self._keep_weights and not self._weight_dropout and self._padded_product(q4, k4, v4, pad):
+                return PaddedAttentionFunc.apply(q4, k4, v4, pad)
             s = torch.einsum('bqnh,bknh->bnqk', q4, k4)
             if simple:
                 s = s + self.rel_pos_bias(q4.size(1)).to(s.dtype)
@@ -628,6 +633,14 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
             return torch.einsum('bnqk,bknh->bqnh', w, v4)
         else:
             return self.efficient_attn(q4, k4, v4)
+
+    def _padded_product(self, q4: Tensor, k4: Tensor, v4: Tensor, key_padding: Optional[Tensor]) -> bool:
+        """Two-sided fp32 attention with padded keys whose products, mask and softmax are the library's own."""
+        soft = self.attn_softmax
+        return (key_padding is not None and self.bidirectional and type(self.rel_pos_bias) is not SimpleRelativePositionalBias
+                and _unhooked((AttentionSoftmax,), soft) and not soft._causal and not (self.training and soft._dropout > 0)
+                and key_padding.shape == q4.shape[:2] and q4.dim() == 4 and q4.is_contiguous() and k4.is_contiguous() and v4.is_contiguous()
+                and ops.own_attention_products((q4.size(1) + 3) // 4 * 4, q4.size(3), v4.size(3), q4, k4, v4))
 
     def _cached_attention(self, z: Tensor, v: Tensor, saved_state, incremental_state) -> Tensor:
         """Attention with the partial-chunk key / value cache

@@ -1303,6 +1303,20 @@ class AttentionFunc(torch.autograd.Function):
         return q_grad, k_grad, v_grad, None, None, None, None, None
 
 
+class PaddedAttentionFunc(torch.autograd.Function):
+    """softmax(q k^T, padded keys left out) v of fp32 operands (ops.padded_attention_fwd); mask: [B, L] bytes."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, mask):
+        y, w = ops.padded_attention_fwd(q, k, v, mask)
+        ctx.save_for_backward(q, k, v, w)
+        return y
+
+    @staticmethod
+    def backward(ctx, y_grad):
+        return (*ops.padded_attention_bwd(y_grad, *ctx.saved_tensors), None)
+
+
 attention_softmax = AttentionSoftmaxFunc.apply
 attention = AttentionFunc.apply
 

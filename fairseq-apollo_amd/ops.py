@@ -659,7 +659,7 @@ def attention_fwd(q, k, v, scale: float, dropout: float, use_causal_mask: bool, 
 
 def _position_product(a, b, c, M, N, K, causal=0, alpha=1.0, a_rows=False, b_rows=False):
     """c = alpha a b per batch entry and head, fp32.  Operands (tensor, kind), contiguous: kind 0 [B, L, Nh, H] (positions by
-    features), 1 [B, Nh, L, L] (weights); a(m, k), b(n, k): the reduction runs along the last axis, or with a_rows / b_rows
+    features), 1 [B, Nh, L, P] (weights, rows padded to P >= L); a(m, k), b(n, k): the reduction runs along the last axis, or with a_rows / b_rows
     along the positions before it."""
     def of(t, weights):
         B, d1, d2, d3 = t.shape
@@ -668,15 +668,51 @@ def _position_product(a, b, c, M, N, K, causal=0, alpha=1.0, a_rows=False, b_row
     Nh = a.shape[1] if aw else a.shape[2]
     with _on_device(a.device):
         _lib.load_host().attention_product(a, b, c, M, N, K, a.shape[0], Nh, *of(a, aw), a_rows, *of(b, bw), b_rows, *of(c, cw),
-                                           causal, alpha, _stream(a.device))
+                                           causal, alpha, aw == 1 and a.shape[3] != a.shape[2], _stream(a.device))
     return c
 
 
 def own_attention_products(L: int, H1: int, H2: int, *ts) -> bool:
     """fp32 attention of whole 16-byte rows: its products run on the library's matrix-core kernel.  Sizes that 16-byte
-    accesses do not fit keep the GEMM library (element-wise loads are slower than its kernels, if not than its call)."""
+    accesses do not fit keep the GEMM library (element-wise loads are slower than its kernels, if not than its call);
+    the length counts where the weights' rows are not padded."""
     return all(t.dtype is torch.float32 for t in ts) and L >= 64 and not (L % 4 or H1 % 4 or H2 % 4) and \
         not torch.compiler.is_compiling() and not torch.is_autocast_enabled() and _lib.load_host().uniform(*ts)
+
+
+def padded_attention_fwd(q, k, v, mask):
+    """softmax(q k^T over the keys that `mask` ([B, L] bytes, nonzero = padding) leaves) v for fp32 [B, L, Nh, H] operands;
+    a chunk that is padding throughout attends as if it were not masked
+    (moving_average_gated_attention.py:222-232).  -> (y, weights [B, Nh, L, P], rows padded with zeros to whole pieces)."""
+    dev = _need_gpu(q, k, v, mask)
+    B, L, Nh, H1 = q.shape
+    H2, P = v.shape[3], (L + 3) // 4 * 4
+    w, y = torch.empty(B, Nh, L, P, dtype=q.dtype, device=dev), torch.empty(B, L, Nh, H2, dtype=q.dtype, device=dev)
+    _position_product((q, 0), (k, 0), (w, 1), L, L, H1)
+    with _on_device(dev):
+        rc = _lib.load().mega_attention_softmax_keys_fwd(_ptr(w), _ptr(w), _dtype_code(w), B * Nh, L, L, P, _ptr(_mask_u8(mask, B, L)),
+                                                         Nh, _stream(dev))
+    _lib.check(rc, "attention_softmax_keys_fwd")
+    return _position_product((w, 1), (v, 0), (y, 0), L, H2, L, b_rows=True), w
+
+
+def padded_attention_bwd(y_grad, q, k, v, w):
+    """-> (q_grad, k_grad, v_grad) of padded_attention_fwd (a masked key's weight is zero, and so is its score's gradient)."""
+    dev = _need_gpu(y_grad, q, k, v, w)
+    B, L, Nh, H1 = q.shape
+    H2, P = v.shape[3], w.shape[3]
+    g = y_grad.detach().to(q.dtype).contiguous()
+    if g.data_ptr() % 16:
+        g = g.clone()
+    dq, dk, dv, ds = (torch.empty_like(t) for t in (q, k, v, w))
+    _position_product((w, 1), (g, 0), (dv, 0), L, H2, L, a_rows=True, b_rows=True)
+    _position_product((g, 0), (v, 0), (ds, 1), L, L, H2)
+    with _on_device(dev):
+        rc = _lib.load().mega_attention_softmax_ld_bwd(_ptr(ds), _ptr(w), _ptr(ds), _dtype_code(w), B * Nh, L, L, P, 1.0, _stream(dev))
+    _lib.check(rc, "attention_softmax_ld_bwd")
+    _position_product((ds, 1), (q, 0), (dk, 0), L, H1, L, a_rows=True, b_rows=True)
+    _position_product((ds, 1), (k, 0), (dq, 0), L, H1, L, b_rows=True)
+    return dq, dk, dv
 
 
 def attention_softmax_bwd(y_grad: torch.Tensor, y: torch.Tensor, use_causal_mask: bool, scale: float = 1.0,

@@ -425,6 +425,7 @@ typedef struct {
   int64_t M, N, K, batch, inner;
   int32_t a_kmajor, b_kmajor, causal, silu;
   float alpha;
+  int32_t a_padded;      /* A's rows in memory are whole multiples of four elements, readable to their end */
 } MegaGemm;
 size_t mega_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t batch);
 int mega_gemm_f32(const MegaGemm* g, void* workspace, size_t workspace_bytes, void* stream);
@@ -679,6 +680,14 @@ int mega_group_sequence_norm_bwd(const void* y_grad, const void* x, int dtype, c
 int mega_attention_softmax_fwd(const void* x, void* y, int dtype, int64_t batch, int64_t outer,
                                int64_t inner, int causal, float dropout, uint64_t seed,
                                void* stream);
+/* The same over rows of pitch ld >= inner (the columns beyond inner become zeros; y may be x), without DropKey and causal
+ * limit, with masked keys: mask [batch / heads, inner] bytes, nonzero = left out, unless a row of it masks every key
+ * (batch counts the heads of every entry).  And the backward pass over such rows (dx may be dy).           */
+int mega_attention_softmax_keys_fwd(const void* x, void* y, int dtype, int64_t batch, int64_t outer, int64_t inner,
+                                    int64_t ld, const uint8_t* mask, int64_t heads, void* stream);
+int mega_attention_softmax_ld_bwd(const void* dy, const void* y, void* dx, int dtype, int64_t batch, int64_t outer,
+                                  int64_t inner, int64_t ld, float scale, void* stream);
+
 /* stands in for attention_softmax_bwd (fairseq/csrc/ops/attention_softmax.cc:20-26,
  * softmax.cuh AttentionSoftmaxBwdKernel; also the middle step of attention_bwd,
  * ops/attention_kernel.cu:195-203):

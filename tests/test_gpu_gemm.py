@@ -124,3 +124,29 @@ def test_linear_layers_outside_training():
         hook.remove()
         assert not M.modules.own_product(lin, x.transpose(0, 1)) and not M.modules.own_product(lin, x.half())
     assert not M.modules.own_product(lin, x)
+
+
+@pytest.mark.parametrize("L", [64, 65, 130, 511, 1003])
+def test_padded_attention(L):
+    """Two-sided attention with padded keys, one row of it padding throughout, at lengths that are whole pieces and not:
+    softmax(q k^T) v and its gradients against 64 bits, padded keys getting none."""
+    print(f"case L={L}", flush=True)
+    B, Nh, H1, H2 = 3, 2, 16, 24
+    gen = torch.Generator(DEV).manual_seed(L)
+    q, k, v, g = (torch.randn(B, L, Nh, h, generator=gen, device=DEV) for h in (H1, H1, H2, H2))
+    mask = torch.zeros(B, L, dtype=torch.bool, device=DEV)
+    mask[0, L - L // 3:] = True
+    mask[1] = True
+    ins = [t.clone().requires_grad_() for t in (q, k, v)]
+    y = M.modules.PaddedAttentionFunc.apply(*ins, mask)
+    y.backward(g)
+    torch.cuda.synchronize()
+    ref = [t.double().transpose(1, 2).contiguous().requires_grad_() for t in (q, k, v)]
+    s = ref[0] @ ref[1].transpose(-1, -2)
+    s = s.masked_fill((mask & ~mask.all(-1, keepdim=True))[:, None, None, :], float("-inf"))
+    out = s.softmax(-1) @ ref[2]
+    out.backward(g.double().transpose(1, 2))
+    assert _rel(y.transpose(1, 2), out) < 4e-6
+    for t, r in zip(ins, ref):
+        assert _rel(t.grad.transpose(1, 2), r.grad) < 1e-5
+    assert not ins[2].grad[0, mask[0]].any() and not ins[1].grad[0, mask[0]].any()
