@@ -68,6 +68,9 @@ SIGNATURES = {
     "mega_token_gated_attention": (_int, [_p, _p]),
     "mega_norm_ema_fwd_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64]),
     "mega_norm_ema_fwd_scratch_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64]),
+    "mega_gemm16_pays": (_int, [_i64, _i64, _i64, _int, _int]),
+    "mega_gemm16_workspace_bytes": (_sz, [_i64, _i64, _i64]),
+    "mega_gemm16": (_int, [_p, _int, _p, _sz, _p]),
     "mega_gemm_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64]),
     "mega_gemm_f32": (_int, [_p, _p, _sz, _p]),
     "mega_norm_ema_fwd_one_kernel": (_int, [_int, _i64, _i64, _i64, _i64, _i64, _int, _int]),

@@ -27,7 +27,7 @@ SOURCES = [
     "decode.hip",
     "decode_layer.hip",
     "elementwise.hip",
-    "gemm.hip",
+    "gemm.hip", "gemm16.hip",
     "gate_glue.hip",
     "row_norm.hip",
     "attention.hip",

@@ -1,0 +1,354 @@
+// Matrix products of bf16 / fp16 activations for the sizes the GEMM library serves badly: C = op(A) op(B) (+ bias)
+// (+ residual), and silu of the rounded value.  A library call costs 26 us of host time, more than most products of a
+// few thousand tokens take, and its weight gradients (both operands stored along the other axis, a reduction over
+// thousands of tokens onto a small matrix) run at a third to a half of its forward products' rate.  Which sizes come here:
+// gemm16_wins.
+//
+// A workgroup of four waves owns a 128 x 128 or 64 x 64 tile, 32 or 64 reduction indices a step: 16-byte pieces go from memory
+// to registers two steps ahead and from there to one of two LDS stages, k-contiguous operands as rows of a step's indices,
+// the others as they lie in memory, their fragments read by transposing LDS loads.  Sums are fp32 throughout, also
+// between the parts of a product that is split along the reduction.
+#include <type_traits>
+
+#include "common.h"
+
+namespace mega {
+namespace {
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((ext_vector_type(4))) short s16x4;
+
+constexpr int kHT = 256;          // threads
+
+struct Gemm16P {
+  const void *A, *B;   // element (m, k): m * lda + k, or (K-major) k * lda + m; (n, k) alike
+  void* C;             // m * ldc + n
+  const void* bias;    // [N] or null
+  const void* R;       // added: m * ldr + n, or null
+  void* pre;           // the value before the activation, or null
+  int64_t lda, ldb, ldc, ldr;
+  int M, N, K, silu;
+  int mt, nt;
+  int kstep;           // reduction indices of a split
+  float* part;         // [splits][M][N], or null
+};
+
+template <typename T>
+__device__ __forceinline__ f32x4 mma16(uint4 a, uint4 b, f32x4 c) {
+  if constexpr (__is_same(T, bf16_t))
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+
+__device__ __forceinline__ float silu_h(float v) { return v / (1.f + __expf(-v)); }
+
+// One operand's side of the tile: W rows (of A) or columns (of B), KM: stored K-major.
+template <int W, bool KM, int kHK>
+struct Side16 {
+  static constexpr int Row = KM ? W * 2 : kHK * 2;                // bytes of a row
+  static constexpr int Bytes = W * kHK * 2;
+  static constexpr int NP = W * kHK / 8 / kHT;                    // 16-byte pieces per thread
+
+  static __device__ __forceinline__ void piece(int tid, int h, int& w, int& k) {
+    const int p = tid + h * kHT;
+    if constexpr (KM) {
+      w = (p % (W / 8)) * 8;
+      k = p / (W / 8);
+    } else {
+      w = p / (kHK / 8);
+      k = (p % (kHK / 8)) * 8;
+    }
+  }
+  static __device__ __forceinline__ int turn(int row) {
+    if constexpr (KM) return W == 128 ? (row & 3) + 4 * ((row >> 3) & 1) : ((row >> 1) & 1) + 2 * ((row >> 3) & 1);
+    else return kHK == 64 ? (row >> 1) & 7 : (row >> 2) & 3;
+  }
+  // byte offset of piece h from the tile's first element in a step of `left` indices; what lies beyond the matrix is
+  // replaced by the last piece inside it (rows are never stored, indices are cleared below)
+  static __device__ __forceinline__ uint32_t offset(int64_t ld, int tid, int h, int room, int left) {
+    int w, k;
+    piece(tid, h, w, k);
+    w = min(w, KM ? room - 8 : room - 1);
+    k = min(k, KM ? left - 1 : left - 8);
+    return (uint32_t)((KM ? (int64_t)k * ld + w : (int64_t)w * ld + k) * 2);
+  }
+  static __device__ __forceinline__ void load(const char* tile, const uint32_t (&off)[NP], uint4 (&v)[NP]) {
+#pragma unroll
+    for (int h = 0; h < NP; ++h) v[h] = *(const uint4*)(tile + off[h]);
+  }
+  static __device__ __forceinline__ void store(char* lds, int tid, int left, const uint4 (&v)[NP]) {
+#pragma unroll
+    for (int h = 0; h < NP; ++h) {
+      int w, k;
+      piece(tid, h, w, k);
+      const bool in = k < left;                                    // (left = 64 at compile time in whole steps)
+      const uint4 x = make_uint4(in ? v[h].x : 0u, in ? v[h].y : 0u, in ? v[h].z : 0u, in ? v[h].w : 0u);
+      char* at = KM ? lds + k * Row + (((w >> 4) ^ turn(k)) << 5) + (w & 15) * 2 : lds + w * Row + (((k >> 3) ^ turn(w)) << 4);
+      *(uint4*)at = x;
+    }
+  }
+  // fragment of 32 indices (kk-th of the step): lane (n, g) gets indices 8 g .. 8 g + 7 of row / column w16 * 16 + n
+  static __device__ __forceinline__ uint4 frag(const char* lds, int w16, int kk, int lane) {
+    const int n = lane & 15, g = lane >> 4;
+    if constexpr (KM) {
+      const int row = 8 * g + (n >> 2);
+      const char* q = lds + (kk * 32 + row) * Row + ((w16 ^ turn(row)) << 5) + (n & 3) * 8;
+      const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(q));
+      const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(q + 4 * Row));
+      const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
+      return make_uint4(l2.x, l2.y, h2.x, h2.y);
+    } else {
+      const int row = w16 * 16 + n;
+      return *(const uint4*)(lds + row * Row + (((kk * 4 + g) ^ turn(row)) << 4));
+    }
+  }
+};
+
+template <typename T>
+__device__ __forceinline__ void finish16(const Gemm16P& G, int m, int n, float (&v)[4]) {
+  T* const C = (T*)G.C;
+  if (G.bias) {
+    const Vec<T, 4> b = *(const Vec<T, 4>*)((const T*)G.bias + n);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] += to_float(b.v[u]);
+  }
+  if (G.R) {
+    const Vec<T, 4> r = *(const Vec<T, 4>*)((const T*)G.R + (int64_t)m * G.ldr + n);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] += to_float(r.v[u]);
+  }
+  Vec<T, 4> o;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) o.v[u] = from_float<T>(v[u]);
+  if (G.pre) *(Vec<T, 4>*)((T*)G.pre + (int64_t)m * G.ldc + n) = o;
+  if (G.silu) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) o.v[u] = from_float<T>(silu_h(to_float(o.v[u])));
+  }
+  *(Vec<T, 4>*)(C + (int64_t)m * G.ldc + n) = o;
+}
+
+// TT: edge of the tile (a wave forms a quarter of it); RAG: a partial last step
+template <typename T, int TT, bool KA, bool KB, bool RAG>
+__global__ __launch_bounds__(kHT, 2) void gemm16_kernel(const Gemm16P G) {
+  constexpr int kHK = TT == 128 ? 32 : 64;                       // reduction indices a step
+  using SA = Side16<TT, KA, kHK>;
+  using SB = Side16<TT, KB, kHK>;
+  constexpr int F = TT / 32;
+  constexpr int kStage = SA::Bytes + SB::Bytes;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tiles = G.mt * G.nt, total = (int)gridDim.x;
+  const int id = total % 8 == 0 ? ((int)blockIdx.x & 7) * (total >> 3) + ((int)blockIdx.x >> 3) : (int)blockIdx.x;
+  const int z = id / tiles, tl = id - z * tiles;
+  const int mi = tl / G.nt, m0 = mi * TT, n0 = (tl - mi * G.nt) * TT;
+  const int kb = G.part ? z * G.kstep : 0, ke = G.part ? min(G.K, kb + G.kstep) : G.K;
+  f32x4 acc[F][F];
+#pragma unroll
+  for (int i = 0; i < F; ++i)
+#pragma unroll
+    for (int j = 0; j < F; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int wm = (wave >> 1) * F, wn = (wave & 1) * F;
+  uint4 ra[2][SA::NP], rb[2][SB::NP];
+  uint32_t oa[SA::NP], ob[SB::NP];
+  auto offsets = [&](const int left) {
+#pragma unroll
+    for (int h = 0; h < SA::NP; ++h) oa[h] = SA::offset(G.lda, tid, h, G.M - m0, left);
+#pragma unroll
+    for (int h = 0; h < SB::NP; ++h) ob[h] = SB::offset(G.ldb, tid, h, G.N - n0, left);
+  };
+  offsets(kHK);
+  const char* const ta = (const char*)G.A + (KA ? (int64_t)kb * G.lda + m0 : (int64_t)m0 * G.lda + kb) * 2;
+  const char* const tb = (const char*)G.B + (KB ? (int64_t)kb * G.ldb + n0 : (int64_t)n0 * G.ldb + kb) * 2;
+  const int64_t da = (KA ? kHK * G.lda : kHK) * 2, db = (KB ? kHK * G.ldb : kHK) * 2;
+  const int steps = (ke - kb + kHK - 1) / kHK;
+  auto load = [&](int s, uint4 (&va)[SA::NP], uint4 (&vb)[SB::NP]) {
+    s = min(s, steps - 1);
+    if (RAG) offsets(min(kHK, ke - kb - s * kHK));
+    SA::load(ta + s * da, oa, va);
+    SB::load(tb + s * db, ob, vb);
+  };
+  auto store = [&](int s, char* stage, uint4 (&va)[SA::NP], uint4 (&vb)[SB::NP]) {
+    const int left = RAG ? ke - kb - s * kHK : kHK;
+    SA::store(stage, tid, left, va);
+    SB::store(stage + SA::Bytes, tid, left, vb);
+  };
+  auto step = [&](auto P, const int s) {
+    constexpr int p = decltype(P)::value;
+    const char* la = lds + p * kStage;
+    const char* lb = la + SA::Bytes;
+#pragma unroll
+    for (int kk = 0; kk < kHK / 32; ++kk) {
+      uint4 fa[F], fb[F];
+#pragma unroll
+      for (int i = 0; i < F; ++i) fa[i] = SA::frag(la, wm + i, kk, lane);
+#pragma unroll
+      for (int j = 0; j < F; ++j) fb[j] = SB::frag(lb, wn + j, kk, lane);
+      // the operands swapped: a lane ends up with four consecutive columns of a row
+#pragma unroll
+      for (int j = 0; j < F; ++j)
+#pragma unroll
+        for (int i = 0; i < F; ++i) acc[i][j] = mma16<T>(fb[j], fa[i], acc[i][j]);
+    }
+    store(s + 1, lds + (1 - p) * kStage, ra[1 - p], rb[1 - p]);
+    __builtin_amdgcn_sched_barrier(0);
+    load(s + 3, ra[1 - p], rb[1 - p]);
+    __syncthreads();
+  };
+  if (steps > 0) {
+    load(0, ra[0], rb[0]);
+    load(1, ra[1], rb[1]);
+    store(0, lds, ra[0], rb[0]);
+    load(2, ra[0], rb[0]);
+    __syncthreads();
+  }
+  for (int s = 0; s < steps; s += 2) {
+    step(std::integral_constant<int, 0>{}, s);
+    if (s + 1 >= steps) break;
+    step(std::integral_constant<int, 1>{}, s + 1);
+  }
+  float* part = G.part ? G.part + (int64_t)z * G.M * G.N : nullptr;
+#pragma unroll
+  for (int i = 0; i < F; ++i) {
+    const int m = m0 + (wm + i) * 16 + (lane & 15);
+#pragma unroll
+    for (int j = 0; j < F; ++j) {
+      const int n = n0 + (wn + j) * 16 + (lane >> 4) * 4;
+      if (m >= G.M || n >= G.N) continue;                          // (N is a multiple of eight)
+      float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+      if (part) *(float4*)(part + (int64_t)m * G.N + n) = make_float4(v[0], v[1], v[2], v[3]);
+      else finish16<T>(G, m, n, v);
+    }
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void gemm16_sum_kernel(const Gemm16P G, int splits) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4, total = (int64_t)G.M * G.N;
+  if (i >= total) return;
+  float v[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < splits; ++s) {
+    const float4 p = *(const float4*)(G.part + s * total + i);
+    v[0] += p.x; v[1] += p.y; v[2] += p.z; v[3] += p.w;
+  }
+  const int m = (int)(i / G.N);
+  finish16<T>(G, m, (int)(i - (int64_t)m * G.N), v);
+}
+
+struct Plan16 {
+  int tile, splits, kstep;
+};
+
+// Tiles of 128 (32 indices a step: 196 registers, no spills; 64 indices spill) where a long reduction makes two
+// workgroups for every compute unit of them, of 64 otherwise; a product of few tiles is split along the reduction.
+Plan16 gemm16_plan(int64_t M, int64_t N, int64_t K) {
+  const int cus = device_cu_count();
+  Plan16 p = {64, 1, 0};
+  const int64_t t128 = ceil_div(M, 128) * ceil_div(N, 128), parts = K / 2048 > 4 ? 4 : K / 2048;
+  if (t128 * parts >= 2 * cus) p.tile = 128;
+  const int64_t tiles = ceil_div(M, p.tile) * ceil_div(N, p.tile);
+  if (tiles <= cus / 2) {
+    int64_t s = ceil_div(2 * cus, tiles);
+    const int64_t most = K / 512;
+    if (s > most) s = most;
+    if (s > 32) s = 32;
+    if (s > 1) {
+      p.kstep = (int)(ceil_div(ceil_div(K, s), 64) * 64);
+      p.splits = (int)ceil_div(K, p.kstep);
+    }
+  }
+  return p;
+}
+
+// Sizes this kernel serves better than the library, us of device time (its call costs the host 20 us less, and a pass
+// over so few tokens is bound by the host):
+//   at most 6 GFLOP    1000 x 2048 x 1024  12   library 11      1000 x 1024 x 2048  15   library 11
+//                       300 x 2048 x 1024  7.6  library 7.7     2000 x 1088 x 512  9.5   library 10.5
+//   and not          1000 x 4352 x 1024 (9 GFLOP)  25   library 15      8192 x 2048 x 1024  50   library 30
+//   weight gradients (both K-major) onto at most 2 M elements over 2048 tokens and more
+//                    2048 x 1024 x 8192  55   library 70       264 x 1024 x 8192  22   library 52
+//   and not          2816 x 1024 x 8192  80   library 80      4096 x 2048 x 8192 160   library 135
+bool gemm16_wins(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor) {
+  return 2.0 * (double)M * (double)N * (double)K <= 6e9 || (a_kmajor && b_kmajor && M * N <= (int64_t)1 << 21 && K >= 2048);
+}
+
+template <typename T, int TT, bool KA, bool KB, bool RAG>
+void launch16(const Gemm16P& G, unsigned blocks, hipStream_t s) {
+  static uint64_t attr_seen = 0;
+  const auto kern = gemm16_kernel<T, TT, KA, KB, RAG>;
+  constexpr int smem = 2 * 2 * TT * (TT == 128 ? 32 : 64) * 2;
+  if (smem > 64 * 1024 && first_on_device(&attr_seen))
+    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(kHT), smem, s, G);
+}
+template <typename T, int TT, bool RAG>
+void launch16_order(const Gemm16P& G, int ka, int kb, unsigned blocks, hipStream_t s) {
+  if (ka && kb) launch16<T, TT, true, true, RAG>(G, blocks, s);
+  else if (ka) launch16<T, TT, true, false, RAG>(G, blocks, s);
+  else if (kb) launch16<T, TT, false, true, RAG>(G, blocks, s);
+  else launch16<T, TT, false, false, RAG>(G, blocks, s);
+}
+template <typename T>
+void launch16_type(const Gemm16P& G, const Plan16& p, int ka, int kb, unsigned blocks, hipStream_t s) {
+  const bool rag = G.K % 64 != 0;
+  if (p.tile == 128) rag ? launch16_order<T, 128, true>(G, ka, kb, blocks, s) : launch16_order<T, 128, false>(G, ka, kb, blocks, s);
+  else rag ? launch16_order<T, 64, true>(G, ka, kb, blocks, s) : launch16_order<T, 64, false>(G, ka, kb, blocks, s);
+  if (p.splits > 1)
+    hipLaunchKernelGGL((gemm16_sum_kernel<T>), dim3((unsigned)ceil_div((int64_t)G.M * G.N, 1024)), dim3(256), 0, s, G, p.splits);
+}
+
+}  // namespace
+}  // namespace mega
+
+using namespace mega;
+
+extern "C" int mega_gemm16_pays(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor) {
+  return gemm16_wins(M, N, K, a_kmajor, b_kmajor) ? 1 : 0;
+}
+
+extern "C" size_t mega_gemm16_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  const Plan16 p = gemm16_plan(M, N, K);
+  return p.splits > 1 ? (size_t)p.splits * M * N * 4 : 0;
+}
+
+extern "C" int mega_gemm16(const MegaGemm* g, int dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  MEGA_REQUIRE(g && (dtype == MEGA_BF16 || dtype == MEGA_F16), MEGA_ERR_ARG, "gemm16: bf16 or fp16 operands");
+  MEGA_REQUIRE(g->M > 0 && g->N > 0 && g->K > 0 && g->batch == 1 && !g->causal && g->alpha == 1.f, MEGA_ERR_UNSUPPORTED,
+               "gemm16: single products without a factor");
+  MEGA_REQUIRE(g->a && g->b && g->c, MEGA_ERR_ARG, "gemm16: null pointer argument");
+  MEGA_REQUIRE(g->M < (int64_t)1 << 30 && g->N < (int64_t)1 << 30 && g->K < (int64_t)1 << 30, MEGA_ERR_UNSUPPORTED,
+               "gemm16: sizes below 2^30");
+  MEGA_REQUIRE(g->lda >= (g->a_kmajor ? g->M : g->K) && g->ldb >= (g->b_kmajor ? g->N : g->K) && g->ldc >= g->N &&
+                   (!g->residual || g->ldr >= g->N),
+               MEGA_ERR_ARG, "gemm16: a leading dimension is shorter than its row");
+  const int64_t far = ((int64_t)1 << 32) / 2 / 128;
+  auto on16 = [](const void* p) { return (uintptr_t)p % 16 == 0; };
+  MEGA_REQUIRE(on16(g->a) && on16(g->b) && on16(g->c) && on16(g->bias) && on16(g->residual) && on16(g->pre) && g->lda % 8 == 0 &&
+                   g->ldb % 8 == 0 && g->ldc % 8 == 0 && (!g->residual || g->ldr % 8 == 0) && g->N % 8 == 0 &&
+                   (g->a_kmajor ? g->M : g->K) % 8 == 0 && (g->b_kmajor ? g->N : g->K) % 8 == 0 && g->lda < far && g->ldb < far,
+               MEGA_ERR_UNSUPPORTED, "gemm16: rows of whole 16-byte pieces");
+  Gemm16P G = {};
+  G.A = g->a; G.B = g->b; G.C = g->c; G.bias = g->bias; G.R = g->residual; G.pre = g->pre;
+  G.lda = g->lda; G.ldb = g->ldb; G.ldc = g->ldc; G.ldr = g->ldr;
+  G.M = (int)g->M; G.N = (int)g->N; G.K = (int)g->K; G.silu = g->silu;
+  const Plan16 p = gemm16_plan(g->M, g->N, g->K);
+  G.mt = (int)ceil_div(g->M, p.tile);
+  G.nt = (int)ceil_div(g->N, p.tile);
+  if (p.splits > 1) {
+    const size_t need = (size_t)p.splits * g->M * g->N * 4;
+    MEGA_REQUIRE(workspace && workspace_bytes >= need && on16(workspace), MEGA_ERR_WORKSPACE, "gemm16: workspace of %zu bytes needed",
+                 need);
+    G.part = (float*)workspace;
+    G.kstep = p.kstep;
+  }
+  const int64_t blocks = (int64_t)G.mt * G.nt * p.splits;
+  MEGA_REQUIRE(blocks < (int64_t)1 << 31, MEGA_ERR_UNSUPPORTED, "gemm16: too many tiles");
+  if (dtype == MEGA_BF16) launch16_type<bf16_t>(G, p, g->a_kmajor, g->b_kmajor, (unsigned)blocks, (hipStream_t)stream);
+  else launch16_type<f16_t>(G, p, g->a_kmajor, g->b_kmajor, (unsigned)blocks, (hipStream_t)stream);
+  MEGA_CHECK_LAUNCH("gemm16");
+  return MEGA_OK;
+}

@@ -559,7 +559,7 @@ Result ema_param_backward(const Args& A) {
 }
 
 // ---- training: the layer around its norm, moving average and attention, forwards and backwards in few calls.  The
-// products of 16-bit activations are library GEMMs; those of fp32 and what lies between them run in libmega_hip.
+// products of 16-bit activations are library GEMMs beyond some size; the others and what lies between them run in libmega_hip.
 // Activations and weights share one type.
 Tensor rows2(const Tensor& t) { return t.reshape({-1, t.size(-1)}); }
 
@@ -576,18 +576,28 @@ bool matrix(const Tensor& t, Matrix* m) {
   return false;
 }
 
-// a [M, K] b [K, N] (+ bias) (+ residual) as fp32 products on the matrix cores (mega_gemm_f32), silu of it with the value
-// before in `pre`; `out` (optional) receives the result and may be the residual.  False: not of this kind.
-bool product_f32(const Tensor& a, const Tensor& b, const Tensor& bias, const Tensor& residual, bool silu, Tensor* pre, Tensor* out,
-                 void* s, const char* who) {
+// a [M, K] b [K, N] (+ bias) (+ residual) on the library's own products, silu of it with the value before in `pre`; `out`
+// (optional) receives the result and may be the residual.  fp32 always (mega_gemm_f32), 16-bit types at the sizes where they
+// win (mega_gemm16).  False: not of this kind.
+bool product(const Tensor& a, const Tensor& b, const Tensor& bias, const Tensor& residual, bool silu, Tensor* pre, Tensor* out,
+             void* s, const char* who) {
   Matrix ma, mb, mr = {0, false};
-  if (a.scalar_type() != at::kFloat || b.scalar_type() != at::kFloat || !a.is_cuda() || a.device() != b.device() || !matrix(a, &ma) ||
-      !matrix(b, &mb) || a.size(1) != b.size(0) || a.numel() == 0 || b.numel() == 0)
+  const at::ScalarType dt = a.scalar_type();
+  const bool wide = dt == at::kFloat;
+  if ((!wide && dt != at::kBFloat16 && dt != at::kHalf) || b.scalar_type() != dt || !a.is_cuda() || a.device() != b.device() ||
+      !matrix(a, &ma) || !matrix(b, &mb) || a.size(1) != b.size(0) || a.numel() == 0 || b.numel() == 0)
     return false;
   const int64_t M = a.size(0), K = a.size(1), N = b.size(1);
-  auto fits = [&](const Tensor& t) { return t.scalar_type() == at::kFloat && t.device() == a.device(); };
+  auto fits = [&](const Tensor& t) { return t.scalar_type() == dt && t.device() == a.device(); };
   if (bias.defined() && (!fits(bias) || bias.numel() != N || !bias.is_contiguous())) return false;
   if (residual.defined() && (!fits(residual) || !matrix(residual, &mr) || mr.first || residual.size(0) != M || residual.size(1) != N)) return false;
+  if (!wide) {
+    auto on16 = [](const Tensor& t) { return !t.defined() || (uintptr_t)t.data_ptr() % 16 == 0; };
+    const int64_t far = ((int64_t)1 << 32) / 2 / 128;
+    if (!mega_gemm16_pays(M, N, K, ma.first, !mb.first) || N % 8 || ma.ld % 8 || mb.ld % 8 || mr.ld % 8 || (ma.first ? M : K) % 8 ||
+        (mb.first ? K : N) % 8 || ma.ld >= far || mb.ld >= far || !on16(a) || !on16(b) || !on16(bias) || !on16(residual) || !on16(*out))
+      return false;
+  }
   if (!out->defined()) *out = at::empty({M, N}, a.options());
   if (pre) *pre = at::empty({M, N}, a.options());
   MegaGemm g = {};
@@ -600,22 +610,23 @@ bool product_f32(const Tensor& a, const Tensor& b, const Tensor& bias, const Ten
   g.ldc = N; g.ldr = mr.ld;
   g.M = M; g.N = N; g.K = K; g.batch = g.inner = 1;
   g.silu = silu; g.alpha = 1.f;
-  const int64_t nws = (int64_t)mega_gemm_workspace_bytes(M, N, K, 1);
+  const int64_t nws = (int64_t)(wide ? mega_gemm_workspace_bytes(M, N, K, 1) : mega_gemm16_workspace_bytes(M, N, K));
   Tensor ws;
   if (nws) ws = at::empty({nws}, a.options().dtype(at::kByte));
-  check(mega_gemm_f32(&g, nws ? ws.data_ptr() : nullptr, (size_t)nws, s), who);
+  void* w = nws ? ws.data_ptr() : nullptr;
+  check(wide ? mega_gemm_f32(&g, w, (size_t)nws, s) : mega_gemm16(&g, dtype_code(a), w, (size_t)nws, s), who);
   return true;
 }
 
 Tensor mm(const Tensor& a, const Tensor& b, void* s, const char* who) {
   Tensor out;
-  return product_f32(a, b, Tensor(), Tensor(), false, nullptr, &out, s, who) ? out : at::mm(a, b);
+  return product(a, b, Tensor(), Tensor(), false, nullptr, &out, s, who) ? out : at::mm(a, b);
 }
 // a b + c, c a row of biases or a whole matrix
 Tensor addmm(const Tensor& c, const Tensor& a, const Tensor& b, void* s, const char* who) {
   Tensor out;
   const bool row = c.dim() == 1;
-  return product_f32(a, b, row ? c : Tensor(), row ? Tensor() : c, false, nullptr, &out, s, who) ? out : at::addmm(c, a, b);
+  return product(a, b, row ? c : Tensor(), row ? Tensor() : c, false, nullptr, &out, s, who) ? out : at::addmm(c, a, b);
 }
 // silu(a b + bias) and the value before
 std::pair<Tensor, Tensor> silu_mm(const Tensor& bias, const Tensor& a, const Tensor& b, void* s, const char* who);
@@ -689,28 +700,27 @@ Tensor silu(const Tensor& x, void* s, const char* who) {
 
 std::pair<Tensor, Tensor> silu_mm(const Tensor& bias, const Tensor& a, const Tensor& b, void* s, const char* who) {
   Tensor pre, out;
-  if (!product_f32(a, b, bias, Tensor(), true, &pre, &out, s, who)) {
+  if (!product(a, b, bias, Tensor(), true, &pre, &out, s, who)) {
     pre = at::addmm(bias, a, b);
     out = silu(pre, s, who);
   }
   return {pre, out};
 }
 
-// a linear layer outside training: (x [.., K] contiguous fp32, weight [N, K], bias | None, residual [.., N] | None, silu,
-// the residual's memory may take the result, stream) -> [.., N]
-Result linear_f32(const Args& A) {
+// a linear layer outside training: (x [.., K] contiguous, weight [N, K], bias | None, residual [.., N] | None, silu,
+// the residual's memory may take the result, stream) -> [.., N], or None where the product is left to the GEMM library
+Result linear_own(const Args& A) {
   A.want(7);
   const Tensor &x = A.t(0), &w = A.t(1);
   same_type(A, {0, 1, 2, 3}, x);
   auto sizes = x.sizes().vec();
-  if (w.dim() != 2 || sizes.back() != w.size(1)) throw std::runtime_error("linear_f32: rows of another width than the weight's");
+  if (w.dim() != 2 || sizes.back() != w.size(1)) throw std::runtime_error("linear_own: rows of another width than the weight's");
   sizes.back() = w.size(0);
   A.shape(2, {w.size(0)});
   A.shape(3, sizes);
   const Tensor r = A.none(3) ? Tensor() : rows2(A.t(3));
   Tensor out = !A.none(3) && A.flag(5) ? r : Tensor();
-  if (!product_f32(rows2(x), w.t(), opt_t(A, 2), r, A.flag(4), nullptr, &out, A.stream(6), A.who))
-    throw std::runtime_error("linear_f32: fp32 device tensors expected");
+  if (!product(rows2(x), w.t(), opt_t(A, 2), r, A.flag(4), nullptr, &out, A.stream(6), A.who)) return wrap(Tensor());
   return wrap(out.view(sizes));
 }
 
@@ -855,8 +865,11 @@ Result swiglu_backward(const Args& A) {
     check(mega_swiglu_bwd(dg.data_ptr(), a.data_ptr(), b.data_ptr(), da.data_ptr(), db.data_ptr(), dtype_code(n), a.numel(), s), A.who);
     if (want(2)) dw1 = mm(da.t(), n2, s, A.who);
     if (want(3)) dw3 = mm(db.t(), n2, s, A.who);
-    if (want(0)) dn = n.scalar_type() == at::kFloat ? addmm(mm(da, A.t(5), s, A.who), db, A.t(6), s, A.who).view(n.sizes())
-                                                    : at::mm(da, A.t(5)).addmm_(db, A.t(6)).view(n.sizes());    // both branches into one gradient: no third pass to add them
+    if (want(0)) {                            // both branches into one gradient: no third pass to add them
+      Tensor both = mm(da, A.t(5), s, A.who), out = both;
+      if (!product(db, A.t(6), Tensor(), both, false, nullptr, &out, s, A.who)) both.addmm_(db, A.t(6));
+      dn = both.view(n.sizes());
+    }
   }
   Tensor r[4] = {dn, dw1, dw3, dw2};
   return tuple(r);
@@ -1181,7 +1194,7 @@ PyMethodDef methods[] = {MEGA_ENTRY(token_gated_attention), MEGA_ENTRY(token_ffn
                          MEGA_ENTRY(ffn_backward),          MEGA_ENTRY(swiglu_forward), MEGA_ENTRY(swiglu_backward),
                          MEGA_ENTRY(mix_forward),           MEGA_ENTRY(mix_out_forward), MEGA_ENTRY(mix_out_backward),
                          MEGA_ENTRY(mix_backward),          MEGA_QUESTION(uniform),    MEGA_QUESTION(trainable),
-                         MEGA_QUESTION(plain_modules), MEGA_QUESTION(wanted),     MEGA_ENTRY(linear_f32),
+                         MEGA_QUESTION(plain_modules), MEGA_QUESTION(wanted),     MEGA_ENTRY(linear_own),
                          MEGA_ENTRY(attention_product),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "mega_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

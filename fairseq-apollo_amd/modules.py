@@ -1366,10 +1366,14 @@ class EfficientAttention(nn.Module):
         return 'causal={}, dropout={}'.format(self._causal, self._dropout)
 
 
+OWN_16BIT_FLOPS = 6e9             # mega_gemm16_pays of products along the rows: no native call is made to be told no
+
+
 def own_product(lin: nn.Linear, x: Tensor, *more) -> bool:
-    """lin(x) outside training as one of the library's own fp32 products (16-bit activations keep the GEMM library)."""
+    """lin(x) outside training may be one of the library's own products (fp32, and 16-bit types at some sizes)."""
     w, b = lin._parameters.get('weight'), lin._parameters.get('bias')
-    return (x.dtype is torch.float32 and x.is_cuda and x.dim() > 1 and w is not None and not torch.is_grad_enabled()
+    return (x.is_cuda and x.dim() > 1 and w is not None and w.dim() == 2
+            and (x.dtype is torch.float32 or 2 * x.numel() * w.shape[0] <= OWN_16BIT_FLOPS) and not torch.is_grad_enabled()
             and not torch.compiler.is_compiling() and not torch.is_autocast_enabled() and x.is_contiguous() and x.shape[-1] == w.shape[1]
             and _plain(b is not None, lin) and ops._lib.load_host().uniform(x, w, b, *more))
 
@@ -1378,7 +1382,9 @@ def project(lin: nn.Linear, x: Tensor, act: bool = False) -> Tensor:
     """lin(x), or silu(lin(x)), outside training."""
     if own_product(lin, x):
         with ops._on_device(x.device):
-            return ops._lib.load_host().linear_f32(x, lin.weight, lin.bias, None, act, False, ops._stream(x.device))
+            y = ops._lib.load_host().linear_own(x, lin.weight, lin.bias, None, act, False, ops._stream(x.device))
+        if y is not None:
+            return y
     y = lin(x)
     return ops.silu(y, inplace=True) if act else y
 
@@ -1394,8 +1400,10 @@ def linear_residual(lin: nn.Linear, h: Tensor, residual: Optional[Tensor], consu
         return lin(h) + residual
     if own_product(lin, h, residual) and residual.shape[:-1] == h.shape[:-1] and residual.shape[-1] == lin.weight.shape[0]:
         with ops._on_device(h.device):
-            return ops._lib.load_host().linear_f32(h, lin.weight, None, residual, False, consume and not residual.requires_grad,
-                                                   ops._stream(h.device))
+            y = ops._lib.load_host().linear_own(h, lin.weight, None, residual, False, consume and not residual.requires_grad,
+                                                ops._stream(h.device))
+        if y is not None:
+            return y
     r2, h2 = residual.reshape(-1, residual.shape[-1]), h.reshape(-1, h.shape[-1])
     if consume and not torch.is_grad_enabled() and not residual.requires_grad:
         r2.addmm_(h2, lin.weight.t())

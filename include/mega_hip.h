@@ -429,6 +429,11 @@ typedef struct {
 } MegaGemm;
 size_t mega_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t batch);
 int mega_gemm_f32(const MegaGemm* g, void* workspace, size_t workspace_bytes, void* stream);
+/* The same for single bf16 / fp16 products (operands, bias, residual, pre and C of `dtype`, fp32 sums, alpha 1, silu of the
+ * rounded value): rows of whole 16-byte pieces on 16 bytes, N a multiple of eight (csrc/gemm16.hip).           */
+int mega_gemm16_pays(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor);   /* faster here than in a GEMM library */
+size_t mega_gemm16_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int mega_gemm16(const MegaGemm* g, int dtype, void* workspace, size_t workspace_bytes, void* stream);
 
 /* 1 when calls of these sizes run as one kernel (carried: with h_in; rows_out: y as [B,D,L] rows), else 0 */
 int mega_norm_ema_fwd_one_kernel(int dtype, int64_t B, int64_t L, int64_t D, int64_t G, int64_t N, int carried,

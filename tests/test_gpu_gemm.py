@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
 class _Gemm(C.Structure):
     _fields_ = [(n, C.c_void_p) for n in ("a", "b", "c", "bias", "residual", "pre")] + \
         [(n, C.c_int64) for n in ("lda", "ldb", "ldc", "ldr", "sa", "sai", "sb", "sbi", "sc", "sci", "M", "N", "K", "batch", "inner")] + \
-        [(n, C.c_int32) for n in ("a_kmajor", "b_kmajor", "causal", "silu")] + [("alpha", C.c_float)]
+        [(n, C.c_int32) for n in ("a_kmajor", "b_kmajor", "causal", "silu")] + [("alpha", C.c_float), ("a_padded", C.c_int32)]
 
 
 def _tol(K):
@@ -25,21 +25,29 @@ def _tol(K):
     return 2.0 ** -24 * (2 + math.sqrt(6 * (K / 32 + 1)))
 
 
-def _gemm(a, b, ka, kb, bias=None, residual=None, silu=False, pre=False, alpha=1.0):
-    """a [M, K], b [N, K] as given or (ka / kb) stored transposed, rows cut out of wider memory where `wide` made them"""
+def _call(a, b, c, ka, kb, bias=None, residual=None, silu=False, p=None, alpha=1.0):
     lib = M._lib.load()
-    m, k = (a.shape[1], a.shape[0]) if ka else a.shape
-    n = b.shape[1] if kb else b.shape[0]
-    c = torch.full((m, n), float("nan"), device=DEV)
-    p = torch.full((m, n), float("nan"), device=DEV) if pre else None
+    m, n = c.shape
+    k = a.shape[0] if ka else a.shape[1]
     ptr = lambda t: None if t is None else t.data_ptr()
     g = _Gemm(ptr(a), ptr(b), ptr(c), ptr(bias), ptr(residual), ptr(p), a.stride(0), b.stride(0), n,
               residual.stride(0) if residual is not None else 0, 0, 0, 0, 0, 0, 0, m, n, k, 1, 1, ka, kb, 0, silu, alpha)
-    nws = lib.mega_gemm_workspace_bytes(m, n, k, 1)
+    wide = a.dtype is torch.float32
+    nws = lib.mega_gemm_workspace_bytes(m, n, k, 1) if wide else lib.mega_gemm16_workspace_bytes(m, n, k)
     ws = torch.empty(max(nws, 16), dtype=torch.uint8, device=DEV)
-    rc = lib.mega_gemm_f32(C.byref(g), ws.data_ptr(), nws, torch.cuda.current_stream().cuda_stream)
+    s = torch.cuda.current_stream().cuda_stream
+    rc = lib.mega_gemm_f32(C.byref(g), ws.data_ptr(), nws, s) if wide else \
+        lib.mega_gemm16(C.byref(g), 1 if a.dtype is torch.bfloat16 else 2, ws.data_ptr(), nws, s)
     assert rc == 0, lib.mega_last_error()
     torch.cuda.synchronize()
+
+
+def _gemm(a, b, ka, kb, bias=None, residual=None, silu=False, pre=False, alpha=1.0):
+    """a [M, K], b [N, K] as given or (ka / kb) stored transposed"""
+    m, n = a.shape[1] if ka else a.shape[0], b.shape[1] if kb else b.shape[0]
+    c = torch.full((m, n), float("nan"), device=DEV, dtype=a.dtype)
+    p = torch.full_like(c, float("nan")) if pre else None
+    _call(a, b, c, ka, kb, bias, residual, silu, p, alpha)
     return (c, p) if pre else c
 
 
@@ -150,3 +158,30 @@ def test_padded_attention(L):
     for t, r in zip(ins, ref):
         assert _rel(t.grad.transpose(1, 2), r.grad) < 1e-5
     assert not ins[2].grad[0, mask[0]].any() and not ins[1].grad[0, mask[0]].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("ka,kb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("m,n,k,wide", [(8, 8, 8, 0), (64, 64, 64, 0), (72, 56, 40, 8), (136, 264, 104, 0), (1000, 264, 72, 0),
+                                        (40, 96, 2056, 0), (264, 1024, 8192, 0), (2048, 1032, 8200, 8)])
+def test_16bit_products(dtype, ka, kb, m, n, k, wide):
+    """Tile and step remainders, tiles of 128 (the long reductions), parts along the reduction, both types: one rounding
+    of a 64-bit product away (2^-9 / 2^-12 of the largest a value can be from its neighbour, half of that on average)."""
+    print(f"case {dtype} m={m} n={n} k={k} wide={wide} ka={ka} kb={kb}", flush=True)
+    gen = torch.Generator(DEV).manual_seed(m + n + k)
+    mk = lambda r, c: torch.randn(r, c + wide, generator=gen, device=DEV).to(dtype)[:, :c]
+    a, b = mk(k, m) if ka else mk(m, k), mk(k, n) if kb else mk(n, k)
+    r = (a.double().t() if ka else a.double()) @ (b.double() if kb else b.double().t())
+    assert _rel(_gemm(a, b, ka, kb), r) < (2.0 ** -9 if dtype is torch.bfloat16 else 2.0 ** -12) + _tol(k)
+
+
+@pytest.mark.parametrize("m,n,k", [(72, 64, 40), (40, 96, 2048)])
+def test_16bit_epilogues(m, n, k):
+    """Bias and residual enter before the one rounding, silu acts on the rounded value."""
+    gen = torch.Generator(DEV).manual_seed(6)
+    mk = lambda *s: torch.randn(*s, generator=gen, device=DEV).to(torch.bfloat16)
+    a, b, bias, res = mk(m, k), mk(n, k), mk(n), mk(m, n)
+    r = a.double() @ b.double().t() + bias.double() + res.double()
+    c, pre = _gemm(a, b, 0, 0, bias, res, True, True)
+    assert _rel(pre, r) < 2.0 ** -9 + _tol(k)
+    assert _rel(c, F.silu(pre.double())) < 2.0 ** -9 + 2.0 ** -22
