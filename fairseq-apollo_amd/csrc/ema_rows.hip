@@ -118,9 +118,10 @@ __device__ __forceinline__ int plane_off(int i) {
 
 // STATE: only the block's end state is wanted (first kernel; with A.both the grid holds both directions).  NX: terms
 // of x; F16: fp16 operands; VEC: rows, mask and partial sums are aligned for four tokens per access and L is a
-// multiple of 4.  BOTH (second kernel, L a multiple of 1024, VEC): a wave forms both directions of its 1024 tokens
-// of memory, backward first, and adds them up in LDS, so that y is written once and no partial sums pass
-// through memory.
+// multiple of 4.  BOTH (second kernel, L a multiple of 1024, VEC): two waves form the two directions of the same 1024
+// tokens of memory and add them up in LDS, so that y is written once and no partial sums pass through memory.  (One
+// wave for both, backward first, is a chain of twice the length at 150 registers instead of 110: a call of 1 x 256 x
+// 16384 in fp32 24.7 us, 23.4 so; 8 x 1024 x 4096 209, 191; 2 x 512 x 8192 in bf16, masked 39.0, 35.4.)
 // Workgroups per CU the register budget is set for.  The apply kernel wants about 150 registers per lane: at four
 // workgroups (128 registers) it spills inside the block loop, and every reload of a spilled register waits
 // (vmcnt(0)) for the row loads in flight as well; at three it keeps everything in registers.
@@ -129,11 +130,11 @@ __device__ __forceinline__ int plane_off(int i) {
 #endif
 template <typename T, int NX, bool F16, bool STATE, bool VEC, bool BOTH>
 __global__ __launch_bounds__(64 * kRW, MEGA_ROWS_MINB) void ema_rows_kernel(const RowsArgs A) {
-  constexpr int kWaveLds = (BOTH ? 2 : 1) * kRWaveLds;
-  __shared__ __attribute__((aligned(16))) char lds[kRW * kWaveLds];
+  constexpr int kRows = BOTH ? kRW / 2 : kRW;            // rows of a workgroup
+  __shared__ __attribute__((aligned(16))) char lds[kRW * kRWaveLds];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int nrg = (A.R + kRW - 1) / kRW;
+  const int nrg = (A.R + kRows - 1) / kRows;
   int bid = (int)blockIdx.x, dirsel = 0;
   if (STATE && A.both) {
     const int per = nrg * (A.S - 1);
@@ -141,29 +142,27 @@ __global__ __launch_bounds__(64 * kRW, MEGA_ROWS_MINB) void ema_rows_kernel(cons
     bid -= dirsel * per;
   }
   const int sm = bid / nrg;                             // time-major: the early blocks of all rows first
-  const int row = (bid - sm * nrg) * kRW + wave;
-  if (row >= A.R) return;
+  const int wrow = (bid - sm * nrg) * kRows + (BOTH ? wave >> 1 : wave);
+  if (!BOTH && wrow >= A.R) return;
+  const int row = BOTH ? min(wrow, A.R - 1) : wrow;     // (two waves meet at barriers: one of no row repeats the last)
   const int b = row / A.D, d = row - b * A.D;
   const int j = lane & 15, r = lane >> 4;
-  char* plane = lds + wave * kWaveLds;                  // hi plane at 0, lo plane at 2048
-  float* ys = (float*)(plane + (BOTH ? kRWaveLds : 0)); // y as fp32 (over the used-up x unless both directions meet here)
+  char* plane = lds + wave * kRWaveLds;                 // hi plane at 0, lo plane at 2048
+  float* ys = (float*)(BOTH ? lds + (wave & ~1) * kRWaveLds : plane);      // y as fp32, over the used-up x (of the backward wave)
   const T* xr = (const T*)A.x + (size_t)b * A.sxb + (size_t)d * A.sxd;
   const uint32_t loff = (uint32_t)lane * 16, roff = (uint32_t)r * 16;
   constexpr int NL = 8;                                // loads in flight per lane and round (element-wise path)
   const uint8_t* mrow = A.mask ? A.mask + (size_t)b * A.L : nullptr;
-  int reverse = 0, i0 = 0;
-#pragma unroll 1
-  for (int pass = 0; pass < (BOTH ? 2 : 1); ++pass) {
-  // this pass's direction: its block in walking order, coefficient rows, records and carried states
-  const bool back = BOTH ? pass == 0 : (STATE && dirsel) ? true : A.reverse != 0;
+  // this wave's direction: its block in walking order, coefficient rows, records and carried states
+  const bool back = BOTH ? (wave & 1) == 0 : (STATE && dirsel) ? true : A.reverse != 0;
   const bool second = BOTH || (STATE && A.both);         // the launch covers both directions
-  reverse = back ? 1 : 0;
+  const int reverse = back ? 1 : 0;
   const int s = (BOTH && back) ? A.S - 1 - sm : sm;
   const int koff = second ? (back ? A.D : 0) : A.koff;
   float* rec = A.rec + ((second && back) ? A.rec_dir : 0);
   const float* h_in = (second && back) ? nullptr : A.h_in;
   float* h_out = (second && back) ? nullptr : A.h_out;
-  i0 = s * kRBlk;                                       // first token of the block in walking order
+  const int i0 = s * kRBlk;                             // first token of the block in walking order
   const char* img = (const char*)A.image + (size_t)(koff + d) * kImgRowBytes;
 
   // ---- the block of x into LDS as two 16-bit planes (masked and out-of-range tokens as zeros); every load of
@@ -434,7 +433,7 @@ __global__ __launch_bounds__(64 * kRW, MEGA_ROWS_MINB) void ema_rows_kernel(cons
   // ---- y through LDS (fp32, in walking order; x is used up; the 16-byte pieces of a segment's 256 bytes are
   // XOR-swizzled by the segment so that the 16 segments' stores fall on different banks) and out in whole runs
   // of 64 tokens
-  __builtin_amdgcn_wave_barrier();
+  if (BOTH) __syncthreads(); else __builtin_amdgcn_wave_barrier();
   if (BOTH && back) {
     // in the order of memory: walking piece (j, c) is piece (15 - j, 15 - c) there, its four tokens reversed
 #pragma unroll
@@ -444,7 +443,9 @@ __global__ __launch_bounds__(64 * kRW, MEGA_ROWS_MINB) void ema_rows_kernel(cons
         const int jm = 15 - j, cm = 15 - (t * 8 + h * 4 + r);
         *(float4*)(ys + jm * 64 + ((cm ^ jm) & 15) * 4) = make_float4(Y[t][h][3], Y[t][h][2], Y[t][h][1], Y[t][h][0]);
       }
-  } else {
+  }
+  if (BOTH) __syncthreads();
+  if (!BOTH || !back) {
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -458,8 +459,34 @@ __global__ __launch_bounds__(64 * kRW, MEGA_ROWS_MINB) void ema_rows_kernel(cons
         *at = v;
       }
   }
+  if (BOTH) {
+    __syncthreads();
+    // both waves write: the backward one the first half of the block, in the order of memory
+    const bool live = wrow < A.R;
+    const int f0 = sm * kRBlk;
+    T* yo = (T*)A.y + (size_t)b * A.syb + (size_t)d * A.syd;
+    const bool keep = A.omega && A.mask;                 // masked tokens keep their residual omega x
+    const float omv = keep ? A.omega[d] : 0.f;
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      const int i = ((wave & 1) * 2 + m) * 256 + 4 * lane, w = f0 + i;
+      float4 v = *(const float4*)(ys + (i & ~63) + (((((i & 63) >> 2) ^ (i >> 6)) & 15) << 2));
+      if (keep) {
+        const Vec<T, 4> xo = *(const Vec<T, 4>*)(xr + w);
+        const uint32_t mm = *(const uint32_t*)(mrow + w);
+        v.x += (mm & 0xffu) ? omv * to_float(xo.v[0]) : 0.f;
+        v.y += (mm & 0xff00u) ? omv * to_float(xo.v[1]) : 0.f;
+        v.z += (mm & 0xff0000u) ? omv * to_float(xo.v[2]) : 0.f;
+        v.w += (mm & 0xff000000u) ? omv * to_float(xo.v[3]) : 0.f;
+      }
+      Vec<T, 4> o;
+      o.v[0] = from_float<T>(v.x); o.v[1] = from_float<T>(v.y); o.v[2] = from_float<T>(v.z); o.v[3] = from_float<T>(v.w);
+      if (live) *(Vec<T, 4>*)(yo + w) = o;
+    }
+    return;
+  }
   __builtin_amdgcn_wave_barrier();
-  }  // pass
+  // the wave's own rows
   T* yr = (T*)A.y + (size_t)b * A.syb + (size_t)d * A.syd;
   float* ar = A.acc ? A.acc + ((size_t)b * A.D + d) * A.L : nullptr;
   const bool resid = A.omega && A.mask;                  // masked tokens keep their residual omega x
@@ -537,6 +564,7 @@ template <typename T, int NX, bool F16, bool VEC>
 int launch_rows_v(const RowsArgs& A, hipStream_t s) {
   const int nrg = (A.R + kRW - 1) / kRW;
   const unsigned per_state = (unsigned)(nrg * (A.S - 1)), per_apply = (unsigned)(nrg * A.S);
+  const unsigned per_both = (unsigned)((A.R + kRW / 2 - 1) / (kRW / 2) * A.S);
   if (A.S > 1) {
     // end states of the blocks 0 .. S - 2 (nobody inherits from the last one), of both directions when asked
     hipLaunchKernelGGL((ema_rows_kernel<T, NX, F16, true, VEC, false>), dim3(per_state * (A.both ? 2 : 1)), dim3(64 * kRW),
@@ -544,7 +572,7 @@ int launch_rows_v(const RowsArgs& A, hipStream_t s) {
   }
   if (A.both) {
     if constexpr (VEC)
-      hipLaunchKernelGGL((ema_rows_kernel<T, NX, F16, false, true, true>), dim3(per_apply), dim3(64 * kRW), 0, s, A);
+      hipLaunchKernelGGL((ema_rows_kernel<T, NX, F16, false, true, true>), dim3(per_both), dim3(64 * kRW), 0, s, A);
   } else {
     hipLaunchKernelGGL((ema_rows_kernel<T, NX, F16, false, VEC, false>), dim3(per_apply), dim3(64 * kRW), 0, s, A);
   }
