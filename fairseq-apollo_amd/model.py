@@ -15,7 +15,7 @@ import torch.nn.functional as F
 from torch import Tensor, nn
 
 from . import ops
-from .layers import MegaDecoderLayer, _arg
+from .layers import MegaDecoderLayer, MovingAverageGatedAttention, _arg
 from .modules import TimestepNorm, _plain, _unhooked, project
 
 
@@ -98,7 +98,9 @@ class MegaDecoderNoCrossAttn(nn.Module):
         if self.embed_scale is not None:
             x = self.embed_scale * x
         decoder_padding_mask = prev_output_tokens.eq(self.padding_idx) if self.padding_idx is not None else None
-        if decoder_padding_mask is not None and not decoder_padding_mask.any():
+        # Outside training the mask goes along as it is: whether anything in it is set would have the host wait for all the
+        # work before (and the masked kernels cost no more).  Positions appended above are known to be padding.
+        if decoder_padding_mask is not None and num_paddings == 0 and not self._mask_stays(x) and not decoder_padding_mask.any():
             decoder_padding_mask = None
         x = self.embedding_dropout(x)
         inner_states: List[Tensor] = [x]
@@ -107,11 +109,24 @@ class MegaDecoderNoCrossAttn(nn.Module):
             inner_states.append(x)
         x = self.final_norm(x, padding_mask=decoder_padding_mask, incremental_state=incremental_state)
         x = self.pre_logits(x)
-        if decoder_padding_mask is not None:
+        if decoder_padding_mask is not None and not self._norm_clears(x):
             x = x * (~decoder_padding_mask).to(x.dtype).unsqueeze(-1)
         if num_paddings > 0:
             x = x[:, :seq_len]
         return x, {"inner_states": inner_states}
+
+    def _mask_stays(self, x: Tensor) -> bool:
+        """A call whose padding mask need not be looked at: on the device, nothing recorded, layers whose only use of the
+        mask is in the norm and the moving average."""
+        return (x.is_cuda and not torch.is_grad_enabled() and not torch.compiler.is_compiling() and self._norm_clears(x)
+                and all(type(layer) is MegaDecoderLayer and layer.mega_layer.attention_activation == 'softmax' and
+                        _unhooked((MegaDecoderLayer, MovingAverageGatedAttention), layer, layer.mega_layer) for layer in self.layers))
+
+    def _norm_clears(self, x: Tensor) -> bool:
+        """The features are the final norm's output as it is, which is zero at padding."""
+        norm = self.final_norm
+        return (x.is_cuda and not torch.is_grad_enabled() and type(self.pre_logits) is nn.Identity and norm.num_groups is not None
+                and _unhooked((TimestepNorm,), norm) and _unhooked((nn.Identity,), self.pre_logits))
 
     def _token_covers(self, tokens: Tensor) -> bool:
         embed = self.embed_tokens

@@ -114,3 +114,21 @@ def test_logits_streamed_against_the_model_oracle(name, T):
     want = _oracle(model, args, tokens)
     assert rel_err(host(got), want) < 5e-4, (name, rel_err(host(got), want))
     assert M.ops.timestep_norm_status() == 0
+
+
+@pytest.mark.parametrize("name", sorted(TABLE))
+@pytest.mark.parametrize("L,padded", [(16, 0), (16, 5), (21, 0), (21, 3)])
+def test_a_mask_that_is_not_looked_at_changes_nothing(name, L, padded, monkeypatch):
+    """Outside training the padding mask stays on the device: the same logits, bit for bit, as with the host asking
+    whether anything in it is set and clearing the features once more, padded tokens or none, whole chunks or not."""
+    model, args, vocab = _build(name, 3)
+    tok = torch.randint(2, vocab, (3, L), generator=torch.Generator().manual_seed(4)).to(DEV)
+    if padded:
+        tok[1, L - padded:] = 1
+    with torch.no_grad():
+        got = model(tok)[0]
+        monkeypatch.setattr(type(model), "_mask_stays", lambda self, x: False)
+        monkeypatch.setattr(type(model), "_norm_clears", lambda self, x: False)
+        want = model(tok)[0]
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
