@@ -386,7 +386,46 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
       s_gv[k * TPR + tokl] = pad ? -1.f : v;                        // a negative variance marks padding
     }
   };
-  if constexpr (NX == 1) {
+  if constexpr (NX == 1 && CW == 32 && kParts > 1) {
+    // Quarters of 64 channels' lines: the sums of four lanes each, added as the wider workgroups' eight lanes are (the
+    // statistics of a row do not depend on how its launch was split).
+    float sm[2][NLD], sq[2][NLD];
+    auto add_quarter = [&](const int i, const uint4 (&v)[NLD]) {   // i: which four pieces of a line
+#pragma unroll
+      for (int k = 0; k < NLD; ++k) {
+        const uint32_t w[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+        float s = 0.f, q = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          s = dot2_ones<T>(w[e], s);
+          q = dot2_self<T>(w[e], q);
+        }
+        sm[i & 1][k] = i < 2 ? s : sm[i & 1][k] + s;
+        sq[i & 1][k] = i < 2 ? q : sq[i & 1][k] + q;
+      }
+    };
+    if constexpr (kParts == 2) {
+      if (part == 0) {
+        add_quarter(0, xv);
+        add_quarter(1, xo);
+      } else {
+        add_quarter(0, xo);
+        add_quarter(1, xv);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < kParts; ++i) {
+        load_lines(gblk + i * CW, xo);
+        add_quarter(i, xo);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < NLD; ++k) {
+      const float m = (group_sum<PL>(sm[0][k]) + group_sum<PL>(sm[1][k])) * (1.0f / GC);
+      const float v = fmaxf((group_sum<PL>(sq[0][k]) + group_sum<PL>(sq[1][k])) * (1.0f / GC) - m * m, 0.f);
+      keep_moments(k, m, v);
+    }
+  } else if constexpr (NX == 1) {
     // sum and sum of squares by packed dot products; E[x^2] - mean^2 in fp32 resolves more than the inputs carry
 #pragma unroll
     for (int k = 0; k < NLD; ++k) {
@@ -1141,8 +1180,13 @@ size_t fused_ws_bytes(int64_t B, int64_t D, int64_t S, int cw) {
 // 2 x 8192 x 2048 in 128s 249 us, 76; fp32 4 x 4096 x 1024 138 us, 53 (3.8 TB/s); fp32 2 x 8192 x 2048 in four parts
 // 364 us, 134; fp32 1 x 300 x 512 in 32s 51 us, 24 (the host's call).  bf16 in the widths beside 64 and 128 (norm, then
 // the streaming kernel): 4 x 4096 x 768 in 48s 54 us, 40; 8 x 2048 x 512 in 32s 32 us, 24; 2 x 1333 x 1536 37 us, 25.
-int fused_channels(int dtype, int64_t gc) {
+// 16-bit groups of 64 and 128 channels go to workgroups of 32 where even those are no more than the compute units: the
+// launch lasts one workgroup's chain, which half the channels shorten (the moments' lines are read by every workgroup of
+// the group): bf16 2 x 2991 x 1024 32.1 us of device time with 64, 28.1 with 32; 4 x 2048 x 1024 30.0, 26.1; the values
+// are the same bit for bit.
+int fused_channels(int dtype, int64_t gc, int64_t rows_blocks_channels) {
   const bool wide = dtype == MEGA_F32;
+  if (!wide && (gc == 64 || gc == 128) && rows_blocks_channels <= (int64_t)32 * device_cu_count()) return 32;
   switch (gc) {
     case 32: return 32;
     case 48: return wide ? 16 : 48;
@@ -1173,7 +1217,7 @@ void fused_launch_layout(const FusedArgs& A, int lout, dim3 grid, hipStream_t s)
 }
 
 template <typename T>
-void fused_launch_width(const FusedArgs& A, int gc, int lout, dim3 grid, hipStream_t s) {
+void fused_launch_width(const FusedArgs& A, int gc, int cw, int lout, dim3 grid, hipStream_t s) {
   if constexpr (sizeof(T) == 4) {
     switch (gc) {
       case 32: return fused_launch_layout<T, 32, 1>(A, lout, grid, s);
@@ -1186,16 +1230,18 @@ void fused_launch_width(const FusedArgs& A, int gc, int lout, dim3 grid, hipStre
     switch (gc) {
       case 32: return fused_launch_layout<T, 32, 1>(A, lout, grid, s);
       case 48: return fused_launch_layout<T, 48, 1>(A, lout, grid, s);
-      case 64: return fused_launch_layout<T, 64, 1>(A, lout, grid, s);
+      case 64:
+        return cw == 32 ? fused_launch_layout<T, 32, 2>(A, lout, grid, s) : fused_launch_layout<T, 64, 1>(A, lout, grid, s);
       case 96: return fused_launch_layout<T, 48, 2>(A, lout, grid, s);
-      default: return fused_launch_layout<T, 64, 2>(A, lout, grid, s);
+      default:
+        return cw == 32 ? fused_launch_layout<T, 32, 4>(A, lout, grid, s) : fused_launch_layout<T, 64, 2>(A, lout, grid, s);
     }
   }
 }
 
 bool fused_sizes(int dtype, int64_t B, int64_t L, int64_t D, int64_t G, int64_t N, bool carried, bool rows) {
   if (G <= 0 || D <= 0 || D % G || N > kNS || N <= 0 || L <= 0) return false;
-  const int cw = fused_channels(dtype, D / G);
+  const int cw = fused_channels(dtype, D / G, B * D * ceil_div(L, kFSeg));
   if (cw == 0 || ceil_div(L, kFSeg) + (carried ? 1 : 0) > kFMaxBlocks) return false;
   // a ragged first block (the block grid is aligned to the end of the row): no carried state in (it would have to
   // enter in the middle of a block), and rows in time must begin at a multiple of 8 inside it
@@ -1298,7 +1344,7 @@ extern "C" int mega_norm_ema_fwd_train(const void* x, void* xn, void* y, int dty
     A.B = (int)B; A.L = (int)L; A.D = (int)D; A.G = (int)G; A.N = (int)N; A.S = (int)S; A.eps = (float)eps;
     A.pad = (int)(S * kFSeg - L);
     A.is_complex = is_complex;
-    const int gc = (int)(D / G), cw = fused_channels(dtype, gc);
+    const int gc = (int)(D / G), cw = fused_channels(dtype, gc, B * D * S);
     A.xcd_map = (D / cw) % 8 == 0 ? 1 : 0;
     A.lb = lookback_launch(true);
     const dim3 grid((unsigned)(B * (D / cw) * S));
@@ -1310,9 +1356,9 @@ extern "C" int mega_norm_ema_fwd_train(const void* x, void* xn, void* y, int dty
                     : 0;
     const int lout = syl == 1 ? 0 : 1;
     switch (dtype) {
-      case MEGA_F32: fused_launch_width<float>(A, gc, lout, grid, s); break;
-      case MEGA_F16: fused_launch_width<f16_t>(A, gc, lout, grid, s); break;
-      default: fused_launch_width<bf16_t>(A, gc, lout, grid, s); break;
+      case MEGA_F32: fused_launch_width<float>(A, gc, cw, lout, grid, s); break;
+      case MEGA_F16: fused_launch_width<f16_t>(A, gc, cw, lout, grid, s); break;
+      default: fused_launch_width<bf16_t>(A, gc, cw, lout, grid, s); break;
     }
     MEGA_CHECK_LAUNCH("norm_ema_fwd");
     return lookback_verify("norm_ema_fwd", s);
