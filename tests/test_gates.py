@@ -1,0 +1,31 @@
+"""Rules that send a call to a fused operator instead of the modules' own calls: what they must leave alone.  No GPU: the
+rules only look at modules and shapes (where a rule asks for device tensors, that question is answered for it)."""
+import pytest
+import torch
+
+import fairseq_apollo_amd as M
+from fairseq_apollo_amd import layers
+
+
+def _two_sided(**kw):
+    return M.MovingAverageGatedAttention(16, 8, 32, 4, norm_num_groups=4, bidirectional=True, **kw)
+
+
+def _padded(layer, monkeypatch):
+    """Whether attention with padded keys would run as the one fused operator (shapes and types taken as fitting)."""
+    monkeypatch.setattr(M.ops, "own_attention_products", lambda *a: True)
+    q, v = torch.zeros(2, 64, 1, 8), torch.zeros(2, 64, 1, 32)
+    return layer._padded_product(q, q, v, torch.zeros(2, 64, dtype=torch.bool))
+
+
+class _OwnBias(layers.SimpleRelativePositionalBias):
+    pass
+
+
+@pytest.mark.parametrize("bias,fused", [(None, True), (layers.SimpleRelativePositionalBias, False), (_OwnBias, False)])
+def test_padded_attention_adds_every_learned_bias(bias, fused, monkeypatch):
+    """A learned bias, of the class itself or one derived from it, belongs to the scores: the fused operator has none."""
+    layer = _two_sided()
+    if bias is not None:
+        layer.rel_pos_bias = bias(64)
+    assert _padded(layer, monkeypatch) == fused
