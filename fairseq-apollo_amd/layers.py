@@ -638,7 +638,7 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
         """Two-sided fp32 attention with padded keys whose products, mask and softmax are the library's own."""
         soft = self.attn_softmax
         return (key_padding is not None and self.bidirectional and not isinstance(self.rel_pos_bias, SimpleRelativePositionalBias)
-                and _unhooked((AttentionSoftmax,), soft) and not soft._causal and not (self.training and soft._dropout > 0)
+                and _unhooked((AttentionSoftmax,), soft) and not soft._causal and not (soft.training and soft._dropout > 0)
                 and key_padding.shape == q4.shape[:2] and q4.dim() == 4 and q4.is_contiguous() and k4.is_contiguous() and v4.is_contiguous()
                 and ops.own_attention_products((q4.size(1) + 3) // 4 * 4, q4.size(3), v4.size(3), q4, k4, v4))
 

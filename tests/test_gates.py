@@ -29,3 +29,13 @@ def test_padded_attention_adds_every_learned_bias(bias, fused, monkeypatch):
     if bias is not None:
         layer.rel_pos_bias = bias(64)
     assert _padded(layer, monkeypatch) == fused
+
+
+@pytest.mark.parametrize("layer_trains,softmax_trains,fused", [(False, False, True), (True, True, False), (False, True, False),
+                                                               (True, False, True)])
+def test_padded_attention_drops_what_its_softmax_drops(layer_trains, softmax_trains, fused, monkeypatch):
+    """Dropped keys follow the softmax module's own mode (sampling with dropout keeps the layer in eval mode)."""
+    layer = _two_sided(attention_dropout=0.5).train(layer_trains)
+    layer.attn_softmax.train(softmax_trains)
+    assert layer.attn_softmax._dropout > 0
+    assert _padded(layer, monkeypatch) == fused
