@@ -126,8 +126,7 @@ class MegaDecoderNoCrossAttn(nn.Module):
         """The features are the final norm's output as it is, which is zero at padding."""
         norm = self.final_norm
         return (x.is_cuda and not torch.is_grad_enabled() and not torch.compiler.is_compiling()
-                and type(self.pre_logits) is nn.Identity and norm.num_groups is not None
-                and _unhooked((TimestepNorm,), norm) and _unhooked((nn.Identity,), self.pre_logits))
+                and _unhooked((nn.Identity,), self.pre_logits) and _unhooked((TimestepNorm,), norm) and norm.num_groups is not None)
 
     def _token_covers(self, tokens: Tensor) -> bool:
         embed = self.embed_tokens

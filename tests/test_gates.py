@@ -1,5 +1,7 @@
 """Rules that send a call to a fused operator instead of the modules' own calls: what they must leave alone.  No GPU: the
 rules only look at modules and shapes (where a rule asks for device tensors, that question is answered for it)."""
+import types
+
 import pytest
 import torch
 
@@ -39,3 +41,21 @@ def test_padded_attention_drops_what_its_softmax_drops(layer_trains, softmax_tra
     layer.attn_softmax.train(softmax_trains)
     assert layer.attn_softmax._dropout > 0
     assert _padded(layer, monkeypatch) == fused
+
+
+def _language_model():
+    args = types.SimpleNamespace(decoder_embed_dim=16, decoder_layers=2, decoder_z_dim=8, decoder_hidden_dim=32, decoder_n_dim=4,
+                                 decoder_ffn_embed_dim=16, decoder_chunk_size=8, norm_num_groups=4, moving_layer="cema")
+    return M.MegaDecoderNoCrossAttn(args, 32, torch.nn.Embedding(32, 16, padding_idx=1)).eval()
+
+
+_ON_DEVICE = types.SimpleNamespace(is_cuda=True)
+
+
+def test_replaced_final_norm_keeps_the_general_path():
+    """A norm of another kind (no groups to speak of) in the place of the last one: its output is cleared at padding."""
+    model = _language_model()
+    with torch.no_grad():
+        assert model._norm_clears(_ON_DEVICE) and model._mask_stays(_ON_DEVICE)
+        model.final_norm = torch.nn.LayerNorm(16)
+        assert not model._norm_clears(_ON_DEVICE) and not model._mask_stays(_ON_DEVICE)
