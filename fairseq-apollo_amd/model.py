@@ -16,7 +16,7 @@ from torch import Tensor, nn
 
 from . import ops
 from .layers import MegaDecoderLayer, MovingAverageGatedAttention, _arg
-from .modules import TimestepNorm, _plain, _unhooked, project
+from .modules import MultiHeadComplexEMA, MultiHeadEMA, TimestepNorm, _plain, _unhooked, project
 
 
 class MegaDecoderNoCrossAttn(nn.Module):
@@ -119,8 +119,10 @@ class MegaDecoderNoCrossAttn(nn.Module):
         """A call whose padding mask need not be looked at: on the device, nothing recorded, layers whose only use of the
         mask is in the norm and the moving average."""
         return (x.is_cuda and not torch.is_grad_enabled() and not torch.compiler.is_compiling() and self._norm_clears(x)
-                and all(type(layer) is MegaDecoderLayer and layer.mega_layer.attention_activation == 'softmax' and
-                        _unhooked((MegaDecoderLayer, MovingAverageGatedAttention), layer, layer.mega_layer) for layer in self.layers))
+                and all(_unhooked((MegaDecoderLayer,), layer) and _unhooked((MovingAverageGatedAttention,), layer.mega_layer)
+                        and layer.mega_layer.attention_activation == 'softmax'
+                        and _unhooked((TimestepNorm, MultiHeadEMA, MultiHeadComplexEMA), layer.mega_layer.norm, layer.mega_layer.move)
+                        for layer in self.layers))
 
     def _norm_clears(self, x: Tensor) -> bool:
         """The features are the final norm's output as it is, which is zero at padding."""

@@ -59,3 +59,28 @@ def test_replaced_final_norm_keeps_the_general_path():
         assert model._norm_clears(_ON_DEVICE) and model._mask_stays(_ON_DEVICE)
         model.final_norm = torch.nn.LayerNorm(16)
         assert not model._norm_clears(_ON_DEVICE) and not model._mask_stays(_ON_DEVICE)
+
+
+class _Other(torch.nn.Module):
+    """A layer's part with its call's signature and nothing else."""
+
+    def forward(self, x, *args, **kw):
+        return x
+
+
+@pytest.mark.parametrize("part", ["", "norm", "move"])
+def test_replaced_parts_of_a_layer_get_no_mask_of_zeros(part):
+    """The mask of a call without padding goes to the layers only where every module that receives it is the package's
+    own, unwatched: another one keeps getting None."""
+    model = _language_model()
+    layer = model.layers[1]
+    with torch.no_grad():
+        if part:
+            hook = getattr(layer.mega_layer, part).register_forward_pre_hook(lambda m, i: None)
+            assert not model._mask_stays(_ON_DEVICE)
+            hook.remove()
+            assert model._mask_stays(_ON_DEVICE)
+            setattr(layer.mega_layer, part, _Other())
+        else:
+            layer.mega_layer = _Other()
+        assert not model._mask_stays(_ON_DEVICE)
