@@ -1304,17 +1304,25 @@ class AttentionFunc(torch.autograd.Function):
 
 
 class PaddedAttentionFunc(torch.autograd.Function):
-    """softmax(q k^T, padded keys left out) v of fp32 operands (ops.padded_attention_fwd); mask: [B, L] bytes."""
+    """softmax(q k^T, padded keys left out) v of fp32 operands (ops.padded_attention_fwd); mask: [B, L], nonzero = padding."""
 
     @staticmethod
     def forward(ctx, q, k, v, mask):
         y, w = ops.padded_attention_fwd(q, k, v, mask)
-        ctx.save_for_backward(q, k, v, w)
+        ctx.save_for_backward(q, k, v, w, mask)
         return y
 
     @staticmethod
     def backward(ctx, y_grad):
-        return (*ops.padded_attention_bwd(y_grad, *ctx.saved_tensors), None)
+        q, k, v, w, mask = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            def formula(q, k, v):
+                pad = mask.to(torch.bool)
+                pad = (pad & ~pad.all(dim=-1, keepdim=True))[:, None, None, :]
+                return torch.einsum('bnqk,bknh->bqnh',
+                                    torch.einsum('bqnh,bknh->bnqk', q, k).masked_fill(pad, float('-inf')).softmax(-1), v)
+            return (*_through_formula(formula, (q, k, v), y_grad), None)
+        return (*ops.padded_attention_bwd(y_grad, q, k, v, w, ops._lib.load_host().wanted(ctx)), None)
 
 
 attention_softmax = AttentionSoftmaxFunc.apply

@@ -696,22 +696,28 @@ def padded_attention_fwd(q, k, v, mask):
     return _position_product((w, 1), (v, 0), (y, 0), L, H2, L, b_rows=True), w
 
 
-def padded_attention_bwd(y_grad, q, k, v, w):
-    """-> (q_grad, k_grad, v_grad) of padded_attention_fwd (a masked key's weight is zero, and so is its score's gradient)."""
+def padded_attention_bwd(y_grad, q, k, v, w, want: int = 7):
+    """-> (q_grad, k_grad, v_grad) of padded_attention_fwd (a masked key's weight is zero, and so is its score's gradient);
+    None for those whose bit (1, 2, 4) is not set in `want`."""
     dev = _need_gpu(y_grad, q, k, v, w)
     B, L, Nh, H1 = q.shape
     H2, P = v.shape[3], w.shape[3]
     g = y_grad.detach().to(q.dtype).contiguous()
     if g.data_ptr() % 16:
         g = g.clone()
-    dq, dk, dv, ds = (torch.empty_like(t) for t in (q, k, v, w))
-    _position_product((w, 1), (g, 0), (dv, 0), L, H2, L, a_rows=True, b_rows=True)
-    _position_product((g, 0), (v, 0), (ds, 1), L, L, H2)
-    with _on_device(dev):
-        rc = _lib.load().mega_attention_softmax_ld_bwd(_ptr(ds), _ptr(w), _ptr(ds), _dtype_code(w), B * Nh, L, L, P, 1.0, _stream(dev))
-    _lib.check(rc, "attention_softmax_ld_bwd")
-    _position_product((ds, 1), (q, 0), (dk, 0), L, H1, L, a_rows=True, b_rows=True)
-    _position_product((ds, 1), (k, 0), (dq, 0), L, H1, L, b_rows=True)
+    dq = dk = dv = None
+    if want & 4:
+        dv = _position_product((w, 1), (g, 0), (torch.empty_like(v), 0), L, H2, L, a_rows=True, b_rows=True)
+    if want & 3:
+        ds = _position_product((g, 0), (v, 0), (torch.empty_like(w), 1), L, L, H2)
+        with _on_device(dev):
+            rc = _lib.load().mega_attention_softmax_ld_bwd(_ptr(ds), _ptr(w), _ptr(ds), _dtype_code(w), B * Nh, L, L, P, 1.0,
+                                                           _stream(dev))
+        _lib.check(rc, "attention_softmax_ld_bwd")
+        if want & 2:
+            dk = _position_product((ds, 1), (q, 0), (torch.empty_like(k), 0), L, H1, L, a_rows=True, b_rows=True)
+        if want & 1:
+            dq = _position_product((ds, 1), (k, 0), (torch.empty_like(q), 0), L, H1, L, b_rows=True)
     return dq, dk, dv
 
 

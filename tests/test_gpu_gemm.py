@@ -185,3 +185,34 @@ def test_16bit_epilogues(m, n, k):
     c, pre = _gemm(a, b, 0, 0, bias, res, True, True)
     assert _rel(pre, r) < 2.0 ** -9 + _tol(k)
     assert _rel(c, F.silu(pre.double())) < 2.0 ** -9 + 2.0 ** -22
+
+
+def _padded_reference(q, k, v, mask):
+    s = q.transpose(1, 2).contiguous() @ k.permute(0, 2, 3, 1).contiguous()
+    s = s.masked_fill((mask & ~mask.all(-1, keepdim=True))[:, None, None, :], float("-inf"))
+    return (s.softmax(-1) @ v.transpose(1, 2).contiguous()).transpose(1, 2)
+
+
+def test_padded_attention_differentiates_twice_and_in_part():
+    """A graph over the backward pass (create_graph) is the formula's, and gradients of some operands are the same values
+    as when all are formed; one row is padding throughout."""
+    B, L, Nh, H1, H2 = 2, 66, 2, 8, 12
+    gen = torch.Generator(DEV).manual_seed(4)
+    mk = lambda h: torch.randn(B, L, Nh, h, generator=gen, device=DEV)
+    mask = torch.zeros(B, L, dtype=torch.bool, device=DEV)
+    mask[0, 50:], mask[1] = True, True
+    ins, g, c = [mk(h).requires_grad_() for h in (H1, H1, H2)], mk(H2), mk(H1)
+    full = torch.autograd.grad(M.modules.PaddedAttentionFunc.apply(*ins, mask), ins, g)
+    for i in range(3):
+        part, = torch.autograd.grad(M.modules.PaddedAttentionFunc.apply(*ins, mask), [ins[i]], g)
+        assert torch.equal(part, full[i])
+
+    def second(f, ins, g, c):
+        dq, = torch.autograd.grad(f(*ins, mask), [ins[0]], g, create_graph=True)
+        return torch.autograd.grad((dq * c).sum(), ins)
+
+    got = second(M.modules.PaddedAttentionFunc.apply, ins, g, c)
+    ref = [t.detach().double().requires_grad_() for t in ins]
+    want = second(_padded_reference, ref, g.double(), c.double())
+    for a, b in zip(got, want):
+        assert _rel(a, b) < 1e-5                # (as the first derivatives: fp32 products of a softmax's differences)
