@@ -105,7 +105,7 @@ __global__ __launch_bounds__(kBlock) void softmax_kernel(const T* x, T* y, int64
 #pragma unroll
     for (int i = 0; i < R; ++i) {
       const int64_t j = threadIdx.x + i * kBlock;
-      if (j < ld) yp[j] = from_float<T>(dead ? 0.f : v[i] * c);
+      if (j < ld) yp[j] = from_float<T>(j < n && !dead ? v[i] * c : 0.f);      // (a NaN score makes c NaN)
     }
     for (int64_t j = threadIdx.x + R * kBlock; j < ld; j += kBlock) yp[j] = from_float<T>(0.f);
   } else {

@@ -447,3 +447,32 @@ def test_time_major_rows_route(dtype, bidirectional, B, D, L, masked):
     dx_ref = layer.adjoint(gt.transpose(1, 2).contiguous(), tm)
     assert dx.stride() == (L * D, 1, D)
     assert rel_err(host(dx), host(dx_ref)) < 1e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n", [60, 1021, 1500, 2100])
+def test_softmax_zeros_beyond_a_row_with_nan(dtype, n):
+    """A NaN score spoils the weights of its row up to the causal limit and none behind it; columns that pad a row
+    (ld > inner) are zeros whatever the row holds.  Rows short enough to stay in registers (4 and 8 values a thread) and
+    longer ones."""
+    print(f"case {dtype} n={n}", flush=True)
+    x = torch.randn(2, 1, n, n, generator=torch.Generator().manual_seed(n)).to(dtype).to(DEV)
+    row = n // 2
+    x[1, 0, row, 3] = float("nan")
+    y = M.ops.attention_softmax_fwd(x, 0.0, True)
+    torch.cuda.synchronize()
+    assert torch.isnan(y[1, 0, row, :row + 1]).all() and not y[1, 0, row, row + 1:].any()
+    assert torch.isfinite(y[0]).all() and not y[0, 0].triu(1).any()
+    ld = n + 7
+    buf = torch.full((2, n, ld), 7.0, dtype=dtype, device=DEV)
+    buf[..., :n] = x[:, 0]
+    mask = torch.zeros(2, n, dtype=torch.uint8, device=DEV)
+    mask[0, n - 5:] = 1
+    rc = M._lib.load().mega_attention_softmax_keys_fwd(buf.data_ptr(), buf.data_ptr(), M.ops._dtype_code(buf), 2, n, n, ld, mask.data_ptr(), 1,
+                                                       torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert rc == 0
+    assert torch.isnan(buf[1, row, :n]).all() and not buf[..., n:].any() and not buf[0, :, n - 5:].any()
+    want = x[0, 0].double().masked_fill(mask[0].bool(), float("-inf")).softmax(-1)
+    # half a unit in the last place of the type, and expf's few of fp32
+    assert ((buf[0, :, :n].double() - want).norm() / want.norm()).item() < {torch.float32: 1e-6, torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12}[dtype] * 1.01
