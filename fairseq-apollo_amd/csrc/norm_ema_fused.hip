@@ -500,7 +500,7 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
 #pragma unroll
     for (int k = 0; k < NLD; ++k) {
       if constexpr (kParts == 1) {
-        keep_moments(k, gmean[k], gvar[k] * (1.0f / GC));
+        keep_moments(k, gmean[k], fmaxf(gvar[k] * (1.0f / GC), 0.f));       // (NaN is no padding: it counts, as in the other widths)
       } else {
         const float shift = gdist[k] * (1.0f / kParts);
         keep_moments(k, gmean[k] + shift, fmaxf(fmaf(-shift, shift, gvar[k] * (1.0f / GC)), 0.f));

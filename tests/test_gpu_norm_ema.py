@@ -472,3 +472,23 @@ def test_one_kernel_widths_and_types(dtype, cpg, B, L, G, out_layout, masked, ca
     if h1 is not None:
         e = rel_err(np.real(host(h1)), np.real(ho)), rel_err(np.imag(host(h1)), np.imag(ho))
         assert max(e) < 2e-3, e
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, BF])
+@pytest.mark.parametrize("cpg", [32, 48, 64, 96, 128])
+def test_a_token_that_is_not_a_number_counts(dtype, cpg):
+    """NaN in one group of one token: the token counts (only padding does not), the group is NaN from there on, the other
+    group and the earlier tokens are what they are without it."""
+    print(f"case {dtype} cpg={cpg}", flush=True)
+    B, L, G, at = 1, 128, 2, 70
+    D = cpg * G
+    p, q, g, om, nw, nb = _setup(np.random.default_rng(70), D, 16)
+    x = torch.randn(B, L, D, generator=torch.Generator().manual_seed(70)).to(dtype).to(DEV)
+    layer = M.ops.PreparedEMA(dev(p), dev(q), dev(g), dev(om))
+    xn0, y0, cnt0, _, _, _ = _run(layer, x, G, nw, nb, out_layout="input")
+    x[0, at, cpg + 5] = float("nan")
+    xn, y, cnt, mean, var, _ = _run(layer, x, G, nw, nb, out_layout="input")
+    assert cnt.tolist() == cnt0.tolist() == [L]
+    assert torch.equal(xn[:, :, :cpg], xn0[:, :, :cpg]) and torch.equal(xn[:, :at], xn0[:, :at])
+    assert torch.equal(y[:, :cpg], y0[:, :cpg]) and torch.isnan(xn[:, at:, cpg:]).all()
+    assert torch.isnan(mean[0, 1]) and not torch.isnan(mean[0, 0])
