@@ -389,9 +389,7 @@ void launch_gemm(GemmArgs G, int64_t M, int64_t N, int64_t batches, bool xcd, hi
   constexpr int smem = 2 * (TM + TN) * PITCH;
   auto kern = gemm_nt_kernel<TIn, TOut, WM, WN, AT, BT, EPI, FM, FN>;
   static uint64_t attr_seen = 0;
-  if (smem > 64 * 1024 && first_on_device(&attr_seen)) {
-    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-  }
+  if (smem > 64 * 1024) raise_lds_limit(&attr_seen, smem, kern);
   if (audit_on()) {
     // the last element each operand is addressed at, from the kernel's own indexing: 16-byte pieces whose first
     // element passes the bounds test, rows below M / N, reduction steps below K; batch bz = bo nin + bi
@@ -1092,9 +1090,7 @@ void launch_flash(const void* q, const void* k, const void* v, void* y, int64_t 
   {                                                                                                           \
     auto kern = flash_fwd_kernel<T, KS_, fqb, fbd>;                                                           \
     static uint64_t attr_seen = 0;                                                                            \
-    if (first_on_device(&attr_seen)) {                                                                        \
-      (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);    \
-    }                                                                                                         \
+    raise_lds_limit(&attr_seen, (int)smem, kern);                                                             \
     hipLaunchKernelGGL(kern, grid, dim3(64 * FNW), smem, s, F);                                               \
   }
   if (ks == 2) MEGA_FLASH(2) else MEGA_FLASH(4)

@@ -9,6 +9,7 @@
 #include <math.h>
 
 #include "../../include/mega_hip.h"
+#include "lds_limit.h"
 
 namespace mega {
 
@@ -49,18 +50,6 @@ int lookback_verify(const char* entry, hipStream_t stream);
   } while (0)
 
 static inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
-
-// Function attributes (the dynamic shared memory limit of a kernel) belong to a device: a call site sets them the
-// first time it launches on each device.  `seen` is the call site's own mask of devices.
-static inline bool first_on_device(uint64_t* seen) {
-  int d = 0;
-  if (hipGetDevice(&d) != hipSuccess) {
-    (void)hipGetLastError();
-    d = 0;
-  }
-  const uint64_t bit = 1ull << (d & 63);
-  return !(__atomic_fetch_or(seen, bit, __ATOMIC_RELAXED) & bit);
-}
 
 // Compute units of the current device, queried once per device (256 when the query fails).
 static inline int device_cu_count() {

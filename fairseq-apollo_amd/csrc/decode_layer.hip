@@ -450,9 +450,7 @@ int launch_linear(const MegaTokenLinear& p0, const MegaTokenLinear* p1, int64_t 
 #define MEGA_TL(MT_)                                                                                            \
   {                                                                                                             \
     static uint64_t seen = 0;                                                                                   \
-    if (first_on_device(&seen))                                                                                 \
-      (void)hipFuncSetAttribute((const void*)token_linear_kernel<T, MT_>,                                       \
-                                hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024);                        \
+    raise_lds_limit(&seen, 144 * 1024, token_linear_kernel<T, MT_>);                                            \
     hipLaunchKernelGGL((token_linear_kernel<T, MT_>), dim3(blocks), dim3(kLinThreads), smem, s, p0, q, blocks0, (int)B); \
   }
   if (mt == 1) MEGA_TL(1) else if (mt == 2) MEGA_TL(2) else MEGA_TL(4)

@@ -1001,9 +1001,7 @@ int ema_mfma_try(const void* x, void* y, int dtype, int64_t sxb, int64_t sxd, in
     const int mode = fast ? ((L / G::SC) % 2 == 0 ? 2 : 1) : 0;
     const int ki = (lin * 2 + lout) * 3 + mode;
     const Kern kern = table[ki];
-    if (first_on_device(&attr_seen[ki])) {
-      (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, G::TOTAL);
-    }
+    raise_lds_limit(&attr_seen[ki], G::TOTAL, kern);
     hipLaunchKernelGGL(kern, grid, dim3(kThreadsM), G::TOTAL, s, a);
     MEGA_CHECK_LAUNCH("ema_fwd (matrix-core path)");
     return MEGA_OK;

@@ -431,8 +431,7 @@ void gemm_launch_form(const GemmP& G, unsigned blocks, hipStream_t s) {
   static uint64_t attr_seen = 0;
   const auto kern = gemm_f32_kernel<TM, TN, WN, KA, KB, FORM>;
   constexpr int smem = 2 * kTerms * (TM + TN) * kGK * 2;
-  if (smem > 64 * 1024 && first_on_device(&attr_seen))
-    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+  if (smem > 64 * 1024) raise_lds_limit(&attr_seen, smem, kern);
   hipLaunchKernelGGL(kern, dim3(blocks), dim3(128 * WN), smem, s, G);
 }
 

@@ -277,11 +277,9 @@ bool gemm16_wins(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor) {
 
 template <typename T, int TT, bool KA, bool KB, bool RAG>
 void launch16(const Gemm16P& G, unsigned blocks, hipStream_t s) {
-  static uint64_t attr_seen = 0;
   const auto kern = gemm16_kernel<T, TT, KA, KB, RAG>;
   constexpr int smem = 2 * 2 * TT * (TT == 128 ? 32 : 64) * 2;
-  if (smem > 64 * 1024 && first_on_device(&attr_seen))
-    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+  static_assert(smem <= 64 * 1024, "within the LDS that every launch may ask for");
   hipLaunchKernelGGL(kern, dim3(blocks), dim3(kHT), smem, s, G);
 }
 template <typename T, int TT, bool RAG>

@@ -281,9 +281,7 @@ int launch_long_conv_fft(const void* x, void* y, const float* k, int64_t B, int6
   auto kern = long_conv_fft_kernel<T>;
   const size_t smem = ((size_t)9) << logm;             // M + M / 8 slots of 8 bytes
   static uint64_t attr_seen = 0;
-  if (first_on_device(&attr_seen)) {
-    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 9 << kFftMaxLog);
-  }
+  raise_lds_limit(&attr_seen, 9 << kFftMaxLog, kern);
   // enough workgroups to fill the chip: split the batch when there are few channels
   int64_t nb = 1;
   while (D * nb < 512 && nb * 2 <= (B + 1) / 2) nb *= 2;

@@ -1202,8 +1202,7 @@ void fused_launch(const FusedArgs& A, dim3 grid, hipStream_t s) {
   static uint64_t attr_seen = 0;
   const auto kern = norm_ema_fused_kernel<T, CW, PARTS, LOUT, STAG>;
   constexpr size_t smem = Geo<T, CW, PARTS>::Smem;
-  if (first_on_device(&attr_seen))
-    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+  raise_lds_limit(&attr_seen, (int)smem, kern);
   hipLaunchKernelGGL(kern, grid, dim3(kFT), smem, s, A);
 }
 

@@ -1118,17 +1118,9 @@ int launch_tiles(const TsnBwdParams& P, hipStream_t s) {
   const size_t cells = (size_t)P.TT * P.G;
   const size_t lds0 = (5 * cells + P.G + 2 * (size_t)P.H) * 4 + (P.TT + 1) * 4;
   const size_t lds1 = (5 * cells + P.G) * 4 + (P.TT + 1) * 4;
-  static uint64_t seen0 = 0, seen1 = 0;
-  if (first_on_device(&seen0)) {
-    (void)hipFuncSetAttribute((const void*)tsn_bwd_tile_kernel<T, VEC, 0, false>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    (void)hipFuncSetAttribute((const void*)tsn_bwd_tile_kernel<T, VEC, 0, true>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-  }
-  if (first_on_device(&seen1)) {
-    (void)hipFuncSetAttribute((const void*)tsn_bwd_tile_kernel<T, VEC, 1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              160 * 1024);
-  }
+  static uint64_t seen = 0;
+  raise_lds_limit(&seen, 160 * 1024, tsn_bwd_tile_kernel<T, VEC, 0, false>, tsn_bwd_tile_kernel<T, VEC, 0, true>,
+                  tsn_bwd_tile_kernel<T, VEC, 1>);
   const dim3 grid((unsigned)(P.B * P.nt));
   const bool fixed = P.R.PER == 1 && P.R.slots <= kThreads && kThreads % P.R.slots == 0;
   if (fixed) {
@@ -1173,12 +1165,7 @@ int launch_onepass(const TsnBwdParams& P, size_t rec_bytes, hipStream_t s) {
     const size_t cells = (size_t)P.TT * P.G;
     const size_t lds = (5 * cells + P.G + 2 * (size_t)P.H) * 4 + (P.TT + 2) * 4;
     static uint64_t seen = 0;
-    if (first_on_device(&seen)) {
-      (void)hipFuncSetAttribute((const void*)tsn_bwd_onepass_kernel<T, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                160 * 1024);
-      (void)hipFuncSetAttribute((const void*)tsn_bwd_onepass_kernel<T, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                160 * 1024);
-    }
+    raise_lds_limit(&seen, 160 * 1024, tsn_bwd_onepass_kernel<T, false>, tsn_bwd_onepass_kernel<T, true>);
     zero_async(P.rec, rec_bytes, s);       // tile and block records (one range): no word carries the tag
     if (P.dy2)
       hipLaunchKernelGGL((tsn_bwd_onepass_kernel<T, true>), dim3((unsigned)(P.B * P.nt)), dim3(kOpThreads), lds, s, P);
