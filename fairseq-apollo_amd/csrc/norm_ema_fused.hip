@@ -1238,19 +1238,29 @@ void fused_launch_width(const FusedArgs& A, int gc, int cw, int lout, dim3 grid,
   }
 }
 
-bool fused_sizes(int dtype, int64_t B, int64_t L, int64_t D, int64_t G, int64_t N, bool carried, bool rows) {
+// state: 1: a state comes in, 2: one is handed on (bits).
+// No call is less accurate here than as two operators.  fp32 / fp16 rows of at least 64 tokens go through the rows kernels
+// there, whose operands are the same two fp16 terms (errors of y 1.6e-7 here, 1.9e-7 there, fp32, 2 x 700 x 512); shorter
+// ones, and those that hand a state on behind a partial block, through the fp32 recurrence of ema_scan.hip: 1.3e-7 here
+// and 0.8e-7 there at 2 x 40 x 256, and a channel whose norm weight is 1e-3 of the others' 7e-5 and 4e-7.  bf16 in the
+// widths beside 64 and 128 likewise below 256 tokens (errors of y 1.9e-3 and 1.66e-3, 2 x 200; of the state 2.4e-6 and
+// 1e-7, 2 x 40), and the streaming kernel's states behind a partial block are closer than the ones here (1.96e-6, 2.4e-6).
+bool fused_sizes(int dtype, int64_t B, int64_t L, int64_t D, int64_t G, int64_t N, int state, bool rows) {
   if (G <= 0 || D <= 0 || D % G || N > kNS || N <= 0 || L <= 0) return false;
-  const int cw = fused_channels(dtype, D / G, B * D * ceil_div(L, kFSeg));
-  if (cw == 0 || ceil_div(L, kFSeg) + (carried ? 1 : 0) > kFMaxBlocks) return false;
+  const int64_t gc = D / G;
+  const int cw = fused_channels(dtype, gc, B * D * ceil_div(L, kFSeg));
+  if (cw == 0 || ceil_div(L, kFSeg) + (state & 1) > kFMaxBlocks) return false;
+  const bool bf16_lines = dtype == MEGA_BF16 && (gc == 64 || gc == 128);
+  if (!bf16_lines && (L < (dtype == MEGA_BF16 ? 256 : 64) || (state != 0 && L % kFSeg != 0))) return false;
   // a ragged first block (the block grid is aligned to the end of the row): no carried state in (it would have to
   // enter in the middle of a block), and rows in time must begin at a multiple of 8 inside it
-  if (L % kFSeg != 0 && (carried || (rows && L % 8 != 0))) return false;
+  if (L % kFSeg != 0 && ((state & 1) || (rows && L % 8 != 0))) return false;
   return B * (D / cw) * ceil_div(L, kFSeg) < (int64_t)1 << 31;
 }
 
 bool fused_covers(int dtype, int64_t B, int64_t L, int64_t D, int64_t G, int64_t N, const void* x, const void* xn,
-                  const void* y, int64_t syb, int64_t syd, int64_t syl, const float* h_in) {
-  if (!fused_sizes(dtype, B, L, D, G, N, h_in != nullptr, syl == 1)) return false;
+                  const void* y, int64_t syb, int64_t syd, int64_t syl, const float* h_in, const float* h_out) {
+  if (!fused_sizes(dtype, B, L, D, G, N, (h_in ? 1 : 0) | (h_out ? 2 : 0), syl == 1)) return false;
   if (((uintptr_t)x % 16) || ((uintptr_t)xn % 16) || ((uintptr_t)y % 16)) return false;
   const bool rows = syl == 1 && syd % 8 == 0 && syb % 8 == 0;
   const bool lines = syd == 1 && syl % 8 == 0 && syb % 8 == 0;
@@ -1274,7 +1284,7 @@ extern "C" size_t mega_norm_ema_fwd_workspace_bytes(int64_t B, int64_t L, int64_
 // 1: a call of these sizes (dense operands on 16 bytes) is one launch of the one-kernel route, for any activation type
 extern "C" int mega_norm_ema_fwd_one_kernel(int dtype, int64_t B, int64_t L, int64_t D, int64_t G, int64_t N, int carried,
                                             int rows_out) {
-  return fused_sizes(dtype, B, L, D, G, N, carried != 0, rows_out != 0) && mega_ema_image_bytes(D, N, 0) > 0 ? 1 : 0;
+  return fused_sizes(dtype, B, L, D, G, N, carried, rows_out != 0) && mega_ema_image_bytes(D, N, 0) > 0 ? 1 : 0;
 }
 
 // scratch (no initialisation, contents never survive a call): the moving average's own workspace when the two
@@ -1311,7 +1321,7 @@ extern "C" int mega_norm_ema_fwd_train(const void* x, void* xn, void* y, int dty
   const int64_t S = ceil_div(L > 0 ? L : 1, kFSeg);
   char* w = (char*)workspace;
   const bool one_kernel = L > 0 && (image || mega_ema_image_bytes(D, N, 0) > 0) &&
-                          fused_covers(dtype, B, L, D, G, N, x, xn, y, syb, syd, syl, h_in);
+                          fused_covers(dtype, B, L, D, G, N, x, xn, y, syb, syd, syl, h_in, h_out);
   if (!one_kernel || !image) {
     const size_t sneed = mega_norm_ema_fwd_scratch_bytes(B, L > 0 ? L : 1, D, G, N);
     MEGA_REQUIRE(scratch && scratch_bytes >= sneed, MEGA_ERR_WORKSPACE, "norm_ema_fwd: scratch of %zu bytes needed",

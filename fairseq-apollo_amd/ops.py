@@ -828,8 +828,9 @@ def transpose_2d(x: torch.Tensor, reverse_rows: bool = False, reverse_cols: bool
     return out
 
 
-def norm_ema_one_kernel(dtype: int, B: int, L: int, D: int, G: int, N: int, carried: bool, rows: bool) -> bool:
-    """Whether TimestepNorm -> moving average of these sizes is one launch (mega_norm_ema_fwd_one_kernel)."""
+def norm_ema_one_kernel(dtype: int, B: int, L: int, D: int, G: int, N: int, carried: int, rows: bool) -> bool:
+    """Whether TimestepNorm -> moving average of these sizes is one launch (mega_norm_ema_fwd_one_kernel); carried: 1 with a
+    state in, 2 with one out, 3 with both."""
     key = ("norm_ema_one", dtype, B, L, D, G, N, carried, rows)
     n = _ws_bytes_cache.get(key)
     if n is None:
@@ -989,10 +990,11 @@ class PreparedEMA:
         if xd.dtype is not torch.bfloat16 and 64 <= L <= 16384 and self.N <= 16 and B > 0 \
                 and not ((want_state or h is not None) and L % 1024) \
                 and not (xd.data_ptr() % 16 == 0 and
-                         norm_ema_one_kernel(dt, B, L, D, G, self.N, h is not None, out_layout == "rows")):
-            # fp32 / fp16 outside the one-kernel sizes: the two operators, the second through PreparedEMA.__call__, which takes the normalised
-            # activations (time-major in memory) onto the rows kernels; inside the library's own two-operator
-            # route the moving average would read them in place on its vector-ALU path
+                         norm_ema_one_kernel(dt, B, L, D, G, self.N, 3 if h is not None else 2 if want_state else 0,
+                                             out_layout == "rows")):
+            # fp32 / fp16 outside the one-kernel sizes: the two operators, the second through PreparedEMA.__call__, which
+            # takes the normalised activations (time-major in memory) onto the rows kernels; inside the library's own
+            # two-operator route the moving average would read them in place on its vector-ALU path
             if want_stats:
                 xn, count, mean, var, _, cm, cr = group_timestep_norm_fwd(xd, prev_count, prev_mean, prev_var, norm_gamma,
                                                                           norm_beta, padding_mask, G, eps)

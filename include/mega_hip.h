@@ -399,8 +399,12 @@ int mega_norm_ema_steps(const void* x, void* xn, void* y, int dtype, int64_t K,
  *   no truncation); h_out must not overlap h_in.
  * Activations of any type with 32, 48, 64, 96 or 128 channels per norm group, ndim <= 16, with or
  * without a mask, ceil(L / 1024) (+ 1 with h_in) <= 16, operands on 16 bytes run as ONE kernel that reads x once
- * and writes xn and y once (mega_norm_ema_fwd_one_kernel says whether sizes do).  L need not be a multiple of 1024 (the blocks are aligned to the end of the row, so h_out is
- * the state after the last token), but such a row takes no h_in, and [B,D,L] rows then need L % 8 == 0.
+ * and writes xn and y once (mega_norm_ema_fwd_one_kernel says whether sizes do).  L need not be a multiple of 1024
+ * (the blocks are aligned to the end of the row, so h_out is the state after the last token), but such a row takes no
+ * h_in, and [B,D,L] rows then need L % 8 == 0.  Unless they are bf16 with 64 or 128 channels per group, such rows take
+ * no h_out either, and rows are at least 64 tokens long (bf16: 256).  fp32 / fp16 activations enter the moving average
+ * as two and one fp16 terms there, as in mega_ema_fwd on [B,D,L] rows: |xn| and the states stay below 65504, and what
+ * is below 2^-14 keeps an absolute 2^-25.
  * Everything else runs the two operators one after the other.
  * `workspace` (launch epoch, block / tile records) must be zero-filled once and then belongs to
  * these calls, exactly like the TimestepNorm workspace (the two may be the same buffer);
@@ -435,7 +439,8 @@ int mega_gemm16_pays(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor
 size_t mega_gemm16_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int mega_gemm16(const MegaGemm* g, int dtype, void* workspace, size_t workspace_bytes, void* stream);
 
-/* 1 when calls of these sizes run as one kernel (carried: with h_in; rows_out: y as [B,D,L] rows), else 0 */
+/* 1 when calls of these sizes run as one kernel (carried: 1 with h_in, 2 with h_out, 3 with both; rows_out: y as [B,D,L]
+ * rows), else 0 */
 int mega_norm_ema_fwd_one_kernel(int dtype, int64_t B, int64_t L, int64_t D, int64_t G, int64_t N, int carried,
                                  int rows_out);
 int mega_norm_ema_fwd(const void* x, void* xn, void* y, int dtype, int64_t syb, int64_t syd,

@@ -152,3 +152,18 @@ def test_composites_leave_the_interpreter_to_other_threads():
         torch.set_num_threads(threads)
     # about one a millisecond; with the lock held none but at the edges
     assert sum(begin < t < end for t in ticks) > 100 * (end - begin)
+
+
+@pytest.mark.parametrize("cpg", [32, 48, 64, 96, 128])
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+def test_sizes_of_the_one_kernel_pair(dtype, cpg):
+    """TimestepNorm -> moving average in one launch (dtype: 0 fp32, 1 bf16, 2 fp16): not where the two operators are more
+    accurate, which short rows are and, behind a partial block, the state handed on; bf16 in whole lines always was."""
+    one = lambda L, state=0, rows=False: M.ops.norm_ema_one_kernel(dtype, 2, L, 4 * cpg, 4, 16, state, rows)
+    always = dtype == 1 and cpg in (64, 128)
+    shortest = 256 if dtype == 1 else 64
+    assert one(2048) and one(2048, 3) and one(1000) and one(1000, 0, True) and one(1024, 2) and one(shortest)
+    assert one(shortest - 1) == one(1) == one(1000, 2) == one(2049, 2) == always
+    assert not one(1000, 1) and not one(1000, 3) and not one(1001, 0, True)
+    assert one(16 * 1024) and not one(16 * 1024, 1) and not one(17 * 1024)
+    assert not M.ops.norm_ema_one_kernel(dtype, 2, 2048, 4 * 24, 4, 16, 0, False)
