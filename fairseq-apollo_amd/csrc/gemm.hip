@@ -1,5 +1,6 @@
 // Matrix products of single-precision activations on the matrix cores: C = alpha op(A) op(B) (+ bias) (+ residual), and
-// silu of it.  Every linear layer, its three training products and the attention's products of fp32 models come here.
+// silu of it.  The attention's products of fp32 models come here, and linear layers and their three training products at
+// the sizes of gemm_wins.
 //
 // The matrix cores' fp32 form runs at 157 TFLOP/s, their bf16 form at 2.5 PFLOP/s.  An fp32 value is the sum of three
 // bf16 values exactly (3 x 8 significant bits, each term rounded to nearest), so a product of two matrices is the sum
@@ -399,15 +400,11 @@ struct Plan {
 // Tiles of 128 (half the LDS traffic of a product) where there are several of them for every compute unit, of 64
 // otherwise.  A product of fewer tiles than compute units is split along the reduction, 256 indices and more each, into
 // partial sums that a second kernel adds up in order.
-// Against the library's fp32 products, us, both from a queue that is kept full (its host call, 26 us, is longer than
-// most of them; the one here takes 6), errors in 1e-7 of the result:
-//   x W^T     8000 x 512 x 256    23 (2.3)   library 23 (2.9)      8000 x 1088 x 256   44 (2.3)   library 62 (2.8)
-//             2048 x 2176 x 512   43 (2.3)   library 64 (4.1)      2048 x 512 x 1024   28 (3.4)   library 20 (5.7)
-//             4096 x 4096 x 4096 800 (10)    library 910 (11.5)
-//   dY^T X    512 x 256 x 8000    30 (3.6)   library 47 (16)       1088 x 256 x 8000   52 (5.0)   library 64 (16)
 // What bounds a step of a tile is LDS: three planes are written and read for every fp32 operand (72 KB a step of a
 // 64 x 64 tile, 576 cycles at 128 bytes a cycle beside 384 of matrix products on each SIMD), and the waves of a
 // workgroup read, multiply and write in step; the 128 tile's waves do so for twice the products.
+// Errors against 64 bits in 1e-7 of the result, the library's fp32 products behind the comma: x W^T 8000 x 512 x 256 2.3,
+// 2.9; 2048 x 512 x 1024 3.4, 5.7; 4096 x 4096 x 4096 10, 11.5; dY^T X 512 x 256 x 8000 3.6, 16; 1088 x 256 x 8000 5.0, 16.
 Plan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t batch) {
   const int cus = device_cu_count();
   Plan p = {64, 1, 0};
@@ -424,6 +421,30 @@ Plan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t batch) {
     }
   }
   return p;
+}
+
+// Sizes that come here, us of device time, one kernel after the other, beside the GEMM library's.  A library call takes
+// 24 - 26 us of host time, one here 6; what loses more than 9 us and a tenth of device time against that is left to it.
+//   two and more workgroups a compute unit, two only for short reductions (one alone waits at every barrier: 0.70 us a
+//   step of 32, two 0.51 a piece, three 0.46, the library's rate is 0.45):
+//     8000 x 512 x 256     24, library 23       2048 x 2176 x 512    42, 63       2048 x 1024 x 1024    35, 35
+//     8000 x 1024 x 2816  311, 318              4096 x 1024 x 2816  164, 157
+//   tiles of 128:  16384 x 2048 x 1024  397, 479      4096 x 4096 x 2048   365, 479
+//   up to 3 GFLOP, counted in whole tiles (small ones are a launch's latency, 10 us here and 5 there):
+//     2048 x 512 x 1024    24, 21       512 x 1024 x 2816    33, 27       300 x 2048 x 1024    26, 18
+//     512 x 512 x 1024     15, 10       64 x 4096 x 2048     19, 16       1 x 4096 x 2048      18, 9
+//   weight gradients (both K-major) onto at most 300,000 elements, whose long reductions the library hardly splits:
+//     512 x 256 x 8000     29, 46       1088 x 256 x 8000    53, 63       128 x 128 x 1000     17, 62
+//   and not (the library's):
+//     512 x 2048 x 4096    89, 63       1000 x 1024 x 4352   97, 68       2048 x 1024 x 2816   88, 80
+//     1024 x 1024 x 8000 177, 112       2048 x 1024 x 8000  255, 229       512 x 1024 x 8000   72, 65 (both K-major)
+// Operands that 16-byte accesses do not fit go to the library (element-wise loads: 1000 x 1022 x 1026 57, 24).
+bool gemm_wins(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor) {
+  const Plan p = gemm_plan(M, N, K, 1);
+  if (p.tile == 128) return true;
+  const int64_t tiles = ceil_div(M, 64) * ceil_div(N, 64), two = 2 * device_cu_count();
+  if (2.0 * 64 * 64 * (double)tiles * (double)K <= 3e9) return true;
+  return tiles * p.splits > two || (tiles * p.splits == two && K / p.splits <= 1024) || (a_kmajor && b_kmajor && M * N <= 300000);
 }
 
 template <int TM, int TN, int WN, bool KA, bool KB, int FORM>
@@ -447,6 +468,10 @@ void gemm_launch(const GemmP& G, int ka, int kb, unsigned blocks, hipStream_t s)
 }  // namespace mega
 
 using namespace mega;
+
+extern "C" int mega_gemm_f32_pays(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor) {
+  return M > 0 && N > 0 && K > 0 && gemm_wins(M, N, K, a_kmajor, b_kmajor) ? 1 : 0;
+}
 
 extern "C" size_t mega_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t batch) {
   if (M <= 0 || N <= 0 || K <= 0 || batch != 1) return 0;

@@ -577,8 +577,8 @@ bool matrix(const Tensor& t, Matrix* m) {
 }
 
 // a [M, K] b [K, N] (+ bias) (+ residual) on the library's own products, silu of it with the value before in `pre`; `out`
-// (optional) receives the result and may be the residual.  fp32 always (mega_gemm_f32), 16-bit types at the sizes where they
-// win (mega_gemm16).  False: not of this kind.
+// (optional) receives the result and may be the residual.  Rows of whole 16-byte pieces, at the sizes where mega_gemm_f32 and
+// mega_gemm16 are worth a call (their own rules).  False: not of this kind.
 bool product(const Tensor& a, const Tensor& b, const Tensor& bias, const Tensor& residual, bool silu, Tensor* pre, Tensor* out,
              void* s, const char* who) {
   Matrix ma, mb, mr = {0, false};
@@ -591,13 +591,12 @@ bool product(const Tensor& a, const Tensor& b, const Tensor& bias, const Tensor&
   auto fits = [&](const Tensor& t) { return t.scalar_type() == dt && t.device() == a.device(); };
   if (bias.defined() && (!fits(bias) || bias.numel() != N || !bias.is_contiguous())) return false;
   if (residual.defined() && (!fits(residual) || !matrix(residual, &mr) || mr.first || residual.size(0) != M || residual.size(1) != N)) return false;
-  if (!wide) {
-    auto on16 = [](const Tensor& t) { return !t.defined() || (uintptr_t)t.data_ptr() % 16 == 0; };
-    const int64_t far = ((int64_t)1 << 32) / 2 / 128;
-    if (!mega_gemm16_pays(M, N, K, ma.first, !mb.first) || N % 8 || ma.ld % 8 || mb.ld % 8 || mr.ld % 8 || (ma.first ? M : K) % 8 ||
-        (mb.first ? K : N) % 8 || ma.ld >= far || mb.ld >= far || !on16(a) || !on16(b) || !on16(bias) || !on16(residual) || !on16(*out))
-      return false;
-  }
+  auto on16 = [](const Tensor& t) { return !t.defined() || (uintptr_t)t.data_ptr() % 16 == 0; };
+  const int64_t vec = 16 / a.element_size(), far = ((int64_t)1 << 32) / a.element_size() / 128;
+  if (!(wide ? mega_gemm_f32_pays : mega_gemm16_pays)(M, N, K, ma.first, !mb.first) || ma.ld % vec || mb.ld % vec || (ma.first ? M : K) % vec ||
+      (mb.first ? K : N) % vec || ma.ld >= far || mb.ld >= far || !on16(a) || !on16(b))
+    return false;
+  if (!wide && (N % vec || mr.ld % vec || !on16(bias) || !on16(residual) || !on16(*out))) return false;
   if (!out->defined()) *out = at::empty({M, N}, a.options());
   if (pre) *pre = at::empty({M, N}, a.options());
   MegaGemm g = {};

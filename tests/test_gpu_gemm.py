@@ -216,3 +216,15 @@ def test_padded_attention_differentiates_twice_and_in_part():
     want = second(_padded_reference, ref, g.double(), c.double())
     for a, b in zip(got, want):
         assert _rel(a, b) < 1e-5                # (as the first derivatives: fp32 products of a softmax's differences)
+
+
+@pytest.mark.parametrize("m,n,k,own", [(64, 72, 96, True), (64, 70, 96, True), (64, 72, 94, False), (512, 2048, 4096, False)])
+def test_fp32_linear_layers_of_sizes_left_to_the_library(m, n, k, own):
+    """Odd widths (no whole 16-byte rows) and sizes that the matrix-core kernel serves slower: the module's own call."""
+    lin, x = torch.nn.Linear(k, n).to(DEV), torch.randn(m, k, device=DEV)
+    with torch.no_grad():
+        y = M._lib.load_host().linear_own(x, lin.weight, lin.bias, None, False, False, torch.cuda.current_stream().cuda_stream)
+        assert (y is not None) == own
+        out = M.modules.project(lin, x)
+        assert torch.equal(out, y if own else lin(x))
+        assert _rel(out, F.linear(x.double(), lin.weight.double(), lin.bias.double())) < max(_tol(k), 1e-6 * math.sqrt(k / 1024))

@@ -167,3 +167,12 @@ def test_sizes_of_the_one_kernel_pair(dtype, cpg):
     assert not one(1000, 1) and not one(1000, 3) and not one(1001, 0, True)
     assert one(16 * 1024) and not one(16 * 1024, 1) and not one(17 * 1024)
     assert not M.ops.norm_ema_one_kernel(dtype, 2, 2048, 4 * 24, 4, 16, 0, False)
+
+
+@pytest.mark.parametrize("m,n,k,gradient,own", [
+    (8000, 512, 256, 0, 1), (2048, 2176, 512, 0, 1), (16384, 2048, 1024, 0, 1), (4096, 4096, 2048, 0, 1), (1, 128, 128, 0, 1),
+    (300, 2048, 1024, 0, 1), (512, 256, 8000, 1, 1), (1088, 256, 8000, 1, 1), (512, 2048, 4096, 0, 0), (1000, 1024, 4352, 0, 0),
+    (2048, 1024, 2816, 0, 0), (2048, 512, 1024, 0, 1), (2048, 1024, 1024, 0, 1), (1024, 1024, 8000, 1, 0), (2048, 1024, 8000, 1, 0), (512, 512, 16384, 0, 0), (512, 512, 16384, 1, 1), (1, 16384, 4096, 0, 0)])
+def test_sizes_of_the_fp32_products(m, n, k, gradient, own):
+    """fp32 products that the matrix-core kernel serves clearly slower than the GEMM library are left to it."""
+    assert M._lib.load().mega_gemm_f32_pays(m, n, k, gradient, gradient) == own
