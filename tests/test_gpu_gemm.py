@@ -228,3 +228,26 @@ def test_fp32_linear_layers_of_sizes_left_to_the_library(m, n, k, own):
         out = M.modules.project(lin, x)
         assert torch.equal(out, y if own else lin(x))
         assert _rel(out, F.linear(x.double(), lin.weight.double(), lin.bias.double())) < max(_tol(k), 1e-6 * math.sqrt(k / 1024))
+
+
+@pytest.mark.parametrize("ka,kb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("m,n,k", [(37, 50, 61), (68, 72, 100), (64, 96, 2056), (4096, 4224, 64)])
+def test_values_that_are_not_finite_in_every_form(m, n, k, ka, kb):
+    """NaN, infinities of either sign and finite values beyond bf16's largest, in every storage order, in element-wise and
+    partial steps, in parts along the reduction and in the wide tile: NaN and infinities where the arithmetic has them, the
+    other elements as ever."""
+    print(f"case m={m} n={n} k={k} ka={ka} kb={kb}", flush=True)
+    gen = torch.Generator(DEV).manual_seed(m)
+    a, b = torch.randn(m, k, generator=gen, device=DEV), torch.randn(n, k, generator=gen, device=DEV)
+    a[3, 5], a[7, k - 1], a[20, 10], b[11, 2], b[n - 1, 7] = float("inf"), float("nan"), 3.4e38, float("-inf"), -3.4e38
+    a[20] *= 0.1
+    a[20, 10] = 3.4e38
+    b[:, 10] *= 0.1
+    c = _gemm(a.t().contiguous() if ka else a, b.t().contiguous() if kb else b, ka, kb)
+    r = (a.double() @ b.double().t()).float()
+    assert torch.equal(torch.isnan(c), torch.isnan(r)) and torch.equal(torch.isposinf(c), torch.isposinf(r))
+    assert torch.equal(torch.isneginf(c), torch.isneginf(r))
+    ok = torch.isfinite(r)
+    big = r.abs() > 1e30
+    assert big[ok].any()
+    assert _rel(c[ok & ~big], r[ok & ~big].double()) < _tol(k) and ((c - r).abs() <= 1e-6 * r.abs())[ok & big].all()
