@@ -352,14 +352,10 @@ __global__ __launch_bounds__(kFT) void norm_ema_fused_kernel(const FusedArgs A) 
   {
     static_assert(kCmpQ32 == 0 && kCmpRS == 1 && kFTabs == 2, "tables 0..1 of the compact slot are staged");
     const char* ibase = (const char*)A.image + (size_t)cb * kImgRowBytes + kSlotCmp * 1024;
-#pragma unroll
-    for (int it = 0; it < 2; ++it) {
-      const int idx = it * kFT + tid;               // (table, channel, 16-byte piece)
-      if (idx < kFTabs * CW * 8) {
-        const int t = idx / (CW * 8), rem = idx - t * (CW * 8), c = rem >> 3, pc = rem & 7;
-        *(uint4*)(s_tab + (t * CW + c) * 128 + pc * 16) =
-            *(const uint4*)(ibase + (size_t)c * kImgRowBytes + t * 128 + pc * 16);
-      }
+    static_assert(kFTabs * CW * 8 <= kFT, "one piece a thread");
+    if (tid < kFTabs * CW * 8) {                    // (table, channel, 16-byte piece)
+      const int t = tid / (CW * 8), rem = tid - t * (CW * 8), c = rem >> 3, pc = rem & 7;
+      *(uint4*)(s_tab + (t * CW + c) * 128 + pc * 16) = *(const uint4*)(ibase + (size_t)c * kImgRowBytes + t * 128 + pc * 16);
     }
     // and how far every channel's slowest pole reaches (asked for here, used after the norm: no wave waits for it)
     if (tid < CW) s_reach[tid] = *(const uint2*)(ibase + (size_t)tid * kImgRowBytes + kCmpReach * 128);
@@ -1182,8 +1178,9 @@ size_t fused_ws_bytes(int64_t B, int64_t D, int64_t S, int cw) {
 // the streaming kernel): 4 x 4096 x 768 in 48s 54 us, 40; 8 x 2048 x 512 in 32s 32 us, 24; 2 x 1333 x 1536 37 us, 25.
 // 16-bit groups of 64 and 128 channels go to workgroups of 32 where even those are no more than the compute units: the
 // launch lasts one workgroup's chain, which half the channels shorten (the moments' lines are read by every workgroup of
-// the group): bf16 2 x 2991 x 1024 32.1 us of device time with 64, 28.1 with 32; 4 x 2048 x 1024 30.0, 26.1; the values
-// are the same bit for bit.
+// the group): bf16 2 x 2991 x 1024 32.1 us of device time with 64, 28.1 with 32; 4 x 2048 x 1024 30.0, 26.1; the bf16
+// values are the same bit for bit, of fp16 ones about two in a million differ by a unit in the last place (whether the
+// compiler rounds fma and conversion once or twice differs from instance to instance).
 int fused_channels(int dtype, int64_t gc, int64_t rows_blocks_channels) {
   const bool wide = dtype == MEGA_F32;
   if (!wide && (gc == 64 || gc == 128) && rows_blocks_channels <= (int64_t)32 * device_cu_count()) return 32;
