@@ -154,6 +154,10 @@ def test_timestep_norm_module_autograd(groups, prior_count):
     (torch.bfloat16, 1, 2048, 256, 2, 16, False, "input"),     # groups of 128 channels, two blocks
     (torch.bfloat16, 2, 1000, 64, 1, 8, True, "input"),        # ragged row with padding
     (torch.float32, 2, 70, 32, 4, 4, True, "rows"),            # outside the one-kernel envelope
+    (torch.float32, 2, 1000, 96, 2, 16, True, "rows"),         # fp32 / fp16 inside it: ragged and whole blocks
+    (torch.float32, 1, 2048, 256, 4, 16, False, "input"),
+    (torch.float16, 2, 777, 96, 2, 16, True, "input"),
+    (torch.float16, 1, 1024, 128, 2, 8, False, "rows"),
 ])
 def test_norm_then_move_trains_as_one_operator(dtype, B, L, D, G, N, masked, layout):
     """norm_then_move under autograd is one operator whose forward is the one-kernel block (with the norm's
@@ -190,7 +194,8 @@ def test_norm_then_move_trains_as_one_operator(dtype, B, L, D, G, N, masked, lay
 
     xn_a, y_a, dx_a, g_a = run(True)
     xn_b, y_b, dx_b, g_b = run(False)
-    tol = 2e-4 if dtype == torch.float32 else 3e-2
+    # (fp16: eight times closer than bf16)
+    tol = {torch.float32: 2e-4, torch.float16: 4e-3}.get(dtype, 3e-2)
     assert rel_err(host(xn_a), host(xn_b)) < tol and rel_err(host(y_a), host(y_b)) < tol
     assert rel_err(host(dx_a), host(dx_b)) < tol
     for (name, _), ga, gb in zip(list(norm.named_parameters()) + list(move.named_parameters()), g_a, g_b):

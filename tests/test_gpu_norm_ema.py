@@ -202,9 +202,14 @@ def test_slowly_decaying_poles_across_blocks(mixed):
     assert rel_err(np.real(host(h)), np.real(ho)) < 2e-3
 
 
-@pytest.mark.parametrize("dtype,B,L,D,G,masked", [(BF, 2, 700, 128, 2, False), (BF, 2, 1000, 128, 2, True),
-                                                  (torch.float32, 1, 1024, 64, 1, False), (BF, 1, 2048, 96, 3, False)])
-def test_outside_the_envelope_runs_two_operators(dtype, B, L, D, G, masked):
+@pytest.mark.parametrize("dtype,B,L,D,G,masked,inside", [
+    (BF, 2, 700, 128, 2, False, False), (BF, 2, 1000, 128, 2, True, True), (torch.float32, 1, 1024, 64, 1, False, True),
+    (BF, 1, 2048, 96, 3, False, True), (BF, 1, 2048, 96, 4, False, False), (torch.float32, 2, 700, 64, 4, True, False),
+    (torch.float32, 1, 2048, 96, 4, False, False), (torch.float16, 2, 1024, 48, 3, True, False)])
+def test_outside_the_envelope_runs_two_operators(dtype, B, L, D, G, masked, inside):
+    """Group widths of 16 and 24, rows in time of a length that is no multiple of 8; and the same call on sizes that run as
+    one kernel (inside)."""
+    assert M.ops.norm_ema_one_kernel(M.ops._DT[dtype], B, L, D, G, 16, 0, True) == inside
     rng = np.random.default_rng(54)
     N = 16
     p, q, g, om, nw, nb = _setup(rng, D, N)
@@ -224,7 +229,7 @@ def test_outside_the_envelope_runs_two_operators(dtype, B, L, D, G, masked):
     assert rel_err(host(y), yo) < tol
 
 
-M_TOL = {torch.float32: 1e-4, BF: 2e-2}
+M_TOL = {torch.float32: 1e-4, torch.float16: 4e-3, BF: 2e-2}
 
 
 @pytest.mark.parametrize("L,out_layout,masked", [(1000, "rows", False), (1032, "rows", True), (2056, "input", False),
@@ -425,9 +430,17 @@ def test_fp32_fp16_ragged_row_and_training_statistics(dtype, tol):
     assert rel_err(host(y), yo) < tol
 
 
-# largest error of xn and of y (given the rounded xn) over the largest value: half a unit in the last place of the
-# activation type against the root mean square times a handful of roundings; fp32 as the row kernels (1.8e-6 measured)
-WIDTH_TOL = {torch.float32: 1e-4, torch.float16: 4e-3, BF: 2e-2}
+def _as_stored(*arrays):
+    """Values as single precision holds them (what the layer is given), in 64 bits."""
+    return [np.asarray(a, np.complex64 if np.iscomplexobj(a) else np.float32).astype(np.complex128 if np.iscomplexobj(a) else np.float64)
+            for a in arrays]
+
+
+# bounds of xn and of y given xn, of the statistics and of the state, each an element's error over its own size or the root
+# mean square.  About four times the largest measured: fp32 1.2e-6, 16-bit types half a unit in the last place (4.9e-4,
+# 3.9e-3; y in bf16 1.65e-2, states of one term); statistics 3.6e-7; states 8e-6 (behind a padded tail, which shrinks them;
+# 1e-6 without), bf16 1.9e-5
+WIDTH_TOL = {torch.float32: (5e-6, 1.5e-6, 4e-5), torch.float16: (1e-3, 1.5e-6, 4e-5), BF: (2e-2, 1.5e-6, 1e-4)}
 
 
 @pytest.mark.parametrize("cpg", [32, 48, 64, 96, 128])
@@ -442,12 +455,12 @@ def test_one_kernel_widths_and_types(dtype, cpg, B, L, G, out_layout, masked, ca
     print(f"case {dtype} cpg={cpg} B={B} L={L} G={G} out={out_layout} masked={masked} carried={carried}", flush=True)
     D, N = cpg * G, 16
     code = {torch.float32: 0, BF: 1, torch.float16: 2}[dtype]
-    want_state = carried or L % 8 == 0
+    want_state = carried or L % 8 == 0 and not masked
     # (short rows and states behind a partial block: two operators, except for bf16 in groups of 64 and 128)
     one = dtype is BF and cpg in (64, 128) or L >= (256 if dtype is BF else 64) and not (want_state and L % 1024)
     assert M.ops.norm_ema_one_kernel(code, B, L, D, G, N, carried + 2 * want_state, out_layout == "rows") == one
     rng = np.random.default_rng(60)
-    p, q, g, om, nw, nb = _setup(rng, D, N)
+    p, q, g, om, nw, nb = _as_stored(*_setup(rng, D, N))
     x, x64 = rounded(rng.normal(size=(B, L, D)) * 1.3 + 0.4, dtype)
     mask = None
     if masked:
@@ -457,24 +470,41 @@ def test_one_kernel_widths_and_types(dtype, cpg, B, L, G, out_layout, masked, ca
         mask[B - 1, L - min(L // 7, 9):] = True
         x[torch.from_numpy(mask).to(DEV)] = float("nan") if one else 1e4          # whatever padding holds
     layer = M.ops.PreparedEMA(dev(p), dev(q), dev(g), dev(om))
-    h0 = (rng.normal(size=(B, D, N)) + 1j * rng.normal(size=(B, D, N))) * 0.1
+    h0, = _as_stored((rng.normal(size=(B, D, N)) + 1j * rng.normal(size=(B, D, N))) * 0.1)
     h = torch.from_numpy(h0.astype(np.complex64)).to(DEV) if carried else None
-    prior = (rng.integers(1, 50, B), rng.normal(size=(B, G)) * 0.2, rng.uniform(0.5, 1.5, (B, G)))
+    prior = (rng.integers(1, 50, B), *_as_stored(rng.normal(size=(B, G)) * 0.2, rng.uniform(0.5, 1.5, (B, G))))
     tp = (torch.from_numpy(prior[0]).to(DEV), dev(prior[1]), dev(prior[2]))
     xn, y, cnt, mean, var, h1, cm, cr = _run(layer, x, G, nw, nb, prior=tp, h=h, want_state=want_state,
                                              padding_mask=None if mask is None else dev(mask, torch.bool),
                                              out_layout=out_layout, want_stats=True)
-    tol = WIDTH_TOL[dtype]
+    tol, stat, state = WIDTH_TOL[dtype]
     xno, c, mu, v = O.timestep_norm(x64, *prior, nw + 1, nb, mask, G)
     assert rel_err(host(xn), xno) < tol
     assert cnt.tolist() == c.tolist()
-    assert rel_err(host(mean), mu) < 1e-4 and rel_err(host(var), v) < 1e-4
-    assert rel_err(host(cm)[:, -1], mu) < 1e-4 and rel_err(host(cr)[:, -1], 1.0 / np.sqrt(v + 1e-5)) < 1e-4
+    assert rel_err(host(mean), mu) < stat and rel_err(host(var), v) < stat
+    assert rel_err(host(cm)[:, -1], mu) < stat and rel_err(host(cr)[:, -1], 1.0 / np.sqrt(v + 1e-5)) < stat
     yo, ho = O.ema_forward(host(xn).transpose(0, 2, 1), p, q, g, om, mask, *((h0,) if carried else ()), incremental=True)
     _check_y(y, yo, tol, tol)
     if h1 is not None:
         e = rel_err(np.real(host(h1)), np.real(ho)), rel_err(np.imag(host(h1)), np.imag(ho))
-        assert max(e) < 2e-3, e
+        assert max(e) < state, e
+
+
+@pytest.mark.parametrize("cpg", [32, 96])
+def test_fp32_slowly_decaying_poles(cpg):
+    """States two orders of magnitude above y that cancel in the sum over the states: y as far from 64 bits as two fp16
+    terms of every operand leave it (2.3e-6 measured; one term of the states would leave 2^-12 of sum |gamma q h|)."""
+    rng = np.random.default_rng(53)
+    B, G, N, L = 1, 2, 16, 3000
+    D = cpg * G
+    q = (1 - 10 ** rng.uniform(-4, -1.5, size=(D, N))) * np.exp(1j * rng.uniform(0, np.pi, size=(D, N)))
+    p, g = rng.random((D, N)) * 0.5, (rng.normal(size=(D, N)) + 1j * rng.normal(size=(D, N))) / 4
+    p, q, g, om = _as_stored(p, q, g, rng.normal(size=D))
+    x, _ = rounded(rng.normal(size=(B, L, D)), torch.float32)
+    assert M.ops.norm_ema_one_kernel(0, B, L, D, G, N, 0, False)
+    xn, y, _, _, _, _ = _run(M.ops.PreparedEMA(dev(p), dev(q), dev(g), dev(om)), x, G, np.zeros(D), np.zeros(D), out_layout="input")
+    yo, _ = O.ema_forward(host(xn).transpose(0, 2, 1), p, q, g, om)
+    assert rel_err(host(y), yo) < 1e-5
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, BF])
@@ -520,3 +550,46 @@ def test_accuracy_of_short_rows_and_handed_on_states(dtype, L, want_state, tol, 
         assert e.max() < tol, e.max()
     if want_state:
         assert np.linalg.norm(host(h) - ho) / np.linalg.norm(ho) < state_tol
+
+
+@pytest.mark.parametrize("dtype,cpg,L,out_layout,masked,carried", [
+    (BF, 64, 5120, "input", False, True), (BF, 64, 4104, "rows", True, False), (BF, 128, 5000, "input", True, False),
+    (BF, 128, 5120, "rows", False, True), (torch.float16, 64, 5120, "rows", True, True), (torch.float16, 64, 4999, "input", True, False),
+    (torch.float16, 128, 5120, "input", False, True), (torch.float16, 128, 4104, "rows", False, False)])
+def test_wide_workgroups_of_large_launches(dtype, cpg, L, out_layout, masked, carried):
+    """Launches with more channel blocks than compute units keep 64 channels a workgroup, without held-back starts (five
+    blocks a row): bit for bit what half the batch gives in workgroups of 32, kept training statistics among it; the last
+    row against the oracle.  (fp16: some of the compiled forms round a normalised value to fp32 before fp16, some at once; in
+    the first block of a row of 4999 tokens that tells 12 of five million values apart, by one unit in the last place.)"""
+    print(f"case {dtype} cpg={cpg} L={L} out={out_layout} masked={masked} carried={carried}", flush=True)
+    B, D = 2, 1024
+    S, cus, G = -(-L // 1024), torch.cuda.get_device_properties(DEV).multi_processor_count, D // cpg
+    assert S > 4 and B * D * S > 32 * cus >= B * D * S // 2
+    rng = np.random.default_rng(72)
+    p, q, g, om, nw, nb = _setup(rng, D, 16)
+    x = torch.randn(B, L, D, generator=torch.Generator().manual_seed(72)).to(dtype).to(DEV)
+    mask = None
+    if masked:
+        mask = torch.zeros(B, L, dtype=torch.bool, device=DEV)
+        mask[0, L - 300:], mask[1, :37] = True, True
+    layer = M.ops.PreparedEMA(dev(p), dev(q), dev(g), dev(om))
+    h = torch.view_as_complex(torch.randn(B, D, 16, 2, generator=torch.Generator().manual_seed(73)).to(DEV)) if carried else None
+    cut = lambda t, s: None if t is None else t[s].contiguous()
+    run = lambda s: _run(layer, cut(x, s), G, nw, nb, out_layout=out_layout, padding_mask=cut(mask, s), h=cut(h, s), want_stats=True)
+    full = run(slice(None))
+    for b in range(B):
+        for u, v, name in zip(full, run(slice(b, b + 1)), ("xn", "y", "count", "mean", "var", "h", "cummean", "cumrstd")):
+            if u is not None:
+                f = torch.view_as_real if u.is_complex() else (lambda t: t)
+                u, v = f(u)[b:b + 1], f(v)
+                if u.dtype is torch.float16:
+                    # y: what a unit of xn (up to 5 here) comes to times a lag's weight (up to 5 with omega's)
+                    unit = 2.0 ** -10 * v.float().abs() + (2.0 ** -10 * 25 if name == "y" else 2.0 ** -24)
+                    assert (u != v).float().mean().item() < 1e-4 and ((u.float() - v.float()).abs() <= unit).all(), (name, b)
+                else:
+                    assert torch.equal(u, v), (name, b)
+    sel = np.r_[0:3, 60:68, D - 3:D]
+    m = None if mask is None else host(mask)[1:]
+    yo, _ = O.ema_forward(host(full[0])[1:, :, sel].transpose(0, 2, 1), p[sel], q[sel], g[sel], om[sel], m,
+                          *(() if h is None else (host(h)[1:, sel],)))
+    _check_y(full[1][1:, sel], yo)

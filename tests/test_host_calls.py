@@ -176,3 +176,10 @@ def test_sizes_of_the_one_kernel_pair(dtype, cpg):
 def test_sizes_of_the_fp32_products(m, n, k, gradient, own):
     """fp32 products that the matrix-core kernel serves clearly slower than the GEMM library are left to it."""
     assert M._lib.load().mega_gemm_f32_pays(m, n, k, gradient, gradient) == own
+
+
+def test_the_limit_of_16bit_products_stands_once():
+    """modules.own_product asks no native call beyond the size at which mega_gemm16_pays says no."""
+    flops, (m, n) = M.modules.OWN_16BIT_FLOPS, (1000, 1000)
+    k = int(flops / (2 * m * n))
+    assert M._lib.load().mega_gemm16_pays(m, n, k, 0, 0) == 1 and M._lib.load().mega_gemm16_pays(m, n, k + 1, 0, 0) == 0
