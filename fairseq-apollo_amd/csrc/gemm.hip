@@ -1,6 +1,6 @@
 // Matrix products of single-precision activations on the matrix cores: C = alpha op(A) op(B) (+ bias) (+ residual), and
-// silu of it.  The attention's products of fp32 models come here, and linear layers and their three training products at
-// the sizes of gemm_wins.
+// silu of it.  fp32 models' linear layers and their three training products come here at the sizes of gemm_wins, the
+// attention's products at those of gemm_batched_wins.
 //
 // The matrix cores' fp32 form runs at 157 TFLOP/s, their bf16 form at 2.5 PFLOP/s.  An fp32 value is the sum of three
 // bf16 values (3 x 8 significant bits, each term rounded to nearest; exactly from 2^-110 on, below that the last term
@@ -470,6 +470,29 @@ bool gemm_wins(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor) {
   return tiles * p.splits > two || (tiles * p.splits == two && K / p.splits <= 1024) || (a_kmajor && b_kmajor && M * N <= 300000);
 }
 
+// The same for a batch of products over positions (attention's; `heads` of them interleaved in every row of the operands,
+// which the library's call copies apart first), from replayed graphs:
+//   fewer workgroups than twice the compute units are a chain of steps (batches are not split): only short ones
+//     q k^T   8 x 512 x 512 x 128       own 12, library 13       w v   8 x 1000 x 64 x 1000   own 31, library 15 (not)
+//             1 x 512 x 512 x 1024          25, 9 (not)                2 x 4096 x 64 x 4096      101, 37 (not)
+//     just as many: up to 1024 indices, or half of them (causal w v 2 x 1024 x 1024 x 1024 37, 34; full 8 x 2048 x 128 x 2048
+//     74, 63 (not))
+//   several heads: own (4 x 1000 x 4 heads x 64: q k^T 16, 36)
+//   tiles of 128: own from 256 reduction indices on (4 x 2048 x 2048 x 1024 208, 245); little reduction onto 2^25 scores
+//     and more, or 64 rows, waste it (8 x 2048 x 2048 x 32 57, 41; 64 x 64 x 2048 x 64 36, 20)
+//   tiles of 64: own (8 x 1000 x 1000 x 512 69, 72), unless the second operand's rows overflow an XCD's 4 MB of L2
+//     (2 x 2048 x 2048 x 512 78, 66) and no causal limit saves half of it
+bool gemm_batched_wins(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t heads, int causal, int a_kmajor) {
+  const Plan p = gemm_plan(M, N, K, batch);
+  const int64_t tiles = ceil_div(M, 64) * ceil_div(N, 64) * batch, splits = causal ? 1 : p.splits, two = 2 * device_cu_count();
+  if (tiles * splits < two) return K / splits <= 512;
+  if (tiles * splits == two) return causal >= 2 || K <= 1024;
+  if (heads > 1) return true;
+  if (p.tile == 128) return M > 64 && (K > 128 || tiles < 8192);
+  if (N * K >= 1 << 20 && !a_kmajor) return causal == 2 || (causal == 1 && batch > 1);
+  return true;
+}
+
 template <int TM, int TN, int WN, bool KA, bool KB, int FORM>
 void gemm_launch_form(const GemmP& G, unsigned blocks, hipStream_t s) {
   static uint64_t attr_seen = 0;
@@ -494,6 +517,10 @@ using namespace mega;
 
 extern "C" int mega_gemm_f32_pays(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor) {
   return M > 0 && N > 0 && K > 0 && gemm_wins(M, N, K, a_kmajor, b_kmajor) ? 1 : 0;
+}
+
+extern "C" int mega_gemm_f32_batched_pays(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t heads, int causal, int a_kmajor) {
+  return M > 0 && N > 0 && K > 0 && batch > 0 && gemm_batched_wins(M, N, K, batch, heads, causal, a_kmajor) ? 1 : 0;
 }
 
 extern "C" size_t mega_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t batch) {

@@ -623,31 +623,17 @@ def attention_fwd(q, k, v, scale: float, dropout: float, use_causal_mask: bool, 
         raise RuntimeError("attention_fwd: q, k, v must share one dtype")
     B, L, Nh, H1 = qd.shape
     H2 = vd.shape[3]
-    y = None if weights_only else torch.empty(B, L, Nh, H2, dtype=qd.dtype, device=dev)
-    w = torch.empty(B, Nh, L, L, dtype=qd.dtype, device=dev) if need_weights else None
     nws = lib.mega_attention_workspace_bytes(_dtype_code(qd), B, L, Nh, H1, H2)
     if not nws and L >= 64 and qd.numel():
-        # outside the matrix-core kernels (fp32, head sizes that are not multiples of 8): the two products as batched
-        # library GEMMs around this library's softmax, which is what the reference does for every shape
-        # (attention_kernel.cu:40-131); the library's own fallback is a kernel of one thread per score.  The scores
-        # are rounded to the activation type before the softmax, as the reference's are.
+        # outside the matrix-core kernels (fp32, head sizes that are not multiples of 8): the two products around this
+        # library's softmax, which is what the reference does for every shape (attention_kernel.cu:40-131); the
+        # library's own fallback is a kernel of one thread per score.  The scores are rounded to the activation type
+        # before the softmax, as the reference's are.
         own = own_attention_products(L, H1, H2, qd, kd, vd)
-        if own:
-            # (what lies above the diagonal is not formed, and the causal softmax does not read it)
-            s = torch.empty(B, Nh, L, L, dtype=qd.dtype, device=dev)
-            _position_product((qd, 0), (kd, 0), (s, 1), L, L, H1, 1 if use_causal_mask else 0, float(scale))
-        else:
-            s = torch.einsum('bqnh,bknh->bnqk', qd, kd)
-            if float(scale) != 1.0:
-                s.mul_(float(scale))
-        wts = attention_softmax_fwd(s, dropout, use_causal_mask, seed)
-        del s
-        if own:
-            if not weights_only:
-                _position_product((wts, 1), (vd, 0), (y, 0), L, H2, L, 2 if use_causal_mask else 0, b_rows=True)
-            return y, (wts if need_weights else None)
-        y = None if weights_only else torch.einsum('bnqk,bknh->bqnh', wts, vd).contiguous()
-        return y, (wts if need_weights else None)
+        wts = attention_softmax_fwd(_scores(qd, kd, L, use_causal_mask, float(scale), own), dropout, use_causal_mask, seed)
+        return None if weights_only else _weighted(wts, vd, use_causal_mask, False, own), (wts if need_weights else None)
+    y = None if weights_only else torch.empty(B, L, Nh, H2, dtype=qd.dtype, device=dev)
+    w = torch.empty(B, Nh, L, L, dtype=qd.dtype, device=dev) if need_weights else None
     ws = _scratch_buffer(dev, nws) if nws else None
     with _on_device(dev):
         rc = lib.mega_attention_fwd(_ptr(qd), _ptr(kd), _ptr(vd), _ptr(y), _ptr(w), _dtype_code(qd), B, L, Nh, H1, H2,
@@ -673,11 +659,40 @@ def _position_product(a, b, c, M, N, K, causal=0, alpha=1.0, a_rows=False, b_row
 
 
 def own_attention_products(L: int, H1: int, H2: int, *ts) -> bool:
-    """fp32 attention of whole 16-byte rows: its products run on the library's matrix-core kernel.  Sizes that 16-byte
+    """fp32 attention of whole 16-byte rows: its products may run on the library's matrix-core kernel.  Sizes that 16-byte
     accesses do not fit keep the GEMM library (element-wise loads are slower than its kernels, if not than its call);
     the length counts where the weights' rows are not padded."""
     return all(t.dtype is torch.float32 for t in ts) and L >= 64 and not (L % 4 or H1 % 4 or H2 % 4) and \
         not torch.compiler.is_compiling() and not torch.is_autocast_enabled() and _lib.load_host().uniform(*ts)
+
+
+def _product_pays(M: int, N: int, K: int, B: int, Nh: int, causal: int, a_rows: bool) -> bool:
+    key = ("gemm_batched", M, N, K, B, Nh, causal, a_rows)
+    n = _ws_bytes_cache.get(key)
+    if n is None:
+        n = _ws_bytes_cache[key] = _lib.load().mega_gemm_f32_batched_pays(M, N, K, B * Nh, Nh, causal, int(a_rows))
+    return bool(n)
+
+
+def _scores(a, b, P: int, causal: bool, alpha: float = 1.0, own: bool = True):
+    """alpha a b^T of [B, L, Nh, H] operands: [B, Nh, L, P], rows padded to P >= L.  Own products (where the sizes pay, and
+    for padded rows) form nothing above the diagonal, which a causal softmax does not read."""
+    B, L, Nh, H = a.shape
+    c = 1 if causal else 0
+    if own and (P != L or _product_pays(L, L, H, B, Nh, c, False)):
+        return _position_product((a, 0), (b, 0), (torch.empty(B, Nh, L, P, dtype=a.dtype, device=a.device), 1), L, L, H, c, alpha)
+    s = torch.einsum('bqnh,bknh->bnqk', a, b).contiguous()
+    return s if alpha == 1.0 else s.mul_(alpha)
+
+
+def _weighted(w, x, causal: bool, transposed: bool, own: bool = True):
+    """w x over the keys, or (transposed) w^T x over the queries; w [B, Nh, L, P] (zero above the diagonal when causal), x
+    and the result [B, L, Nh, H]."""
+    B, L, Nh, H = x.shape
+    c = (3 if transposed else 2) if causal else 0
+    if own and _product_pays(L, H, L, B, Nh, c, transposed):
+        return _position_product((w, 1), (x, 0), (torch.empty_like(x), 0), L, H, L, c, a_rows=transposed, b_rows=True)
+    return torch.einsum('bnqk,bqnh->bknh' if transposed else 'bnqk,bknh->bqnh', w[..., :L], x).contiguous()
 
 
 def padded_attention_fwd(q, k, v, mask):
@@ -685,39 +700,38 @@ def padded_attention_fwd(q, k, v, mask):
     a chunk that is padding throughout attends as if it were not masked
     (moving_average_gated_attention.py:222-232).  -> (y, weights [B, Nh, L, P], rows padded with zeros to whole pieces)."""
     dev = _need_gpu(q, k, v, mask)
-    B, L, Nh, H1 = q.shape
-    H2, P = v.shape[3], (L + 3) // 4 * 4
-    w, y = torch.empty(B, Nh, L, P, dtype=q.dtype, device=dev), torch.empty(B, L, Nh, H2, dtype=q.dtype, device=dev)
-    _position_product((q, 0), (k, 0), (w, 1), L, L, H1)
+    B, L, Nh, _ = q.shape
+    P = (L + 3) // 4 * 4
+    w = _scores(q, k, P, False)
     with _on_device(dev):
         rc = _lib.load().mega_attention_softmax_keys_fwd(_ptr(w), _ptr(w), _dtype_code(w), B * Nh, L, L, P, _ptr(_mask_u8(mask, B, L)),
                                                          Nh, _stream(dev))
     _lib.check(rc, "attention_softmax_keys_fwd")
-    return _position_product((w, 1), (v, 0), (y, 0), L, H2, L, b_rows=True), w
+    return _weighted(w, v, False, False), w
 
 
 def padded_attention_bwd(y_grad, q, k, v, w, want: int = 7):
     """-> (q_grad, k_grad, v_grad) of padded_attention_fwd (a masked key's weight is zero, and so is its score's gradient);
     None for those whose bit (1, 2, 4) is not set in `want`."""
     dev = _need_gpu(y_grad, q, k, v, w)
-    B, L, Nh, H1 = q.shape
-    H2, P = v.shape[3], w.shape[3]
+    B, L, Nh, _ = q.shape
+    P = w.shape[3]
     g = y_grad.detach().to(q.dtype).contiguous()
     if g.data_ptr() % 16:
         g = g.clone()
     dq = dk = dv = None
     if want & 4:
-        dv = _position_product((w, 1), (g, 0), (torch.empty_like(v), 0), L, H2, L, a_rows=True, b_rows=True)
+        dv = _weighted(w, g, False, True)
     if want & 3:
-        ds = _position_product((g, 0), (v, 0), (torch.empty_like(w), 1), L, L, H2)
+        ds = _scores(g, v, P, False)
         with _on_device(dev):
             rc = _lib.load().mega_attention_softmax_ld_bwd(_ptr(ds), _ptr(w), _ptr(ds), _dtype_code(w), B * Nh, L, L, P, 1.0,
                                                            _stream(dev))
         _lib.check(rc, "attention_softmax_ld_bwd")
         if want & 2:
-            dk = _position_product((ds, 1), (q, 0), (torch.empty_like(k), 0), L, H1, L, a_rows=True, b_rows=True)
+            dk = _weighted(ds, q, False, True)
         if want & 1:
-            dq = _position_product((ds, 1), (k, 0), (torch.empty_like(q), 0), L, H1, L, b_rows=True)
+            dq = _weighted(ds, k, False, False)
     return dq, dk, dv
 
 
@@ -760,7 +774,8 @@ def attention_bwd(y_grad, q, k, v, w, scale: float, use_causal_mask: bool, y=Non
     four batched products around the softmax backward; w [B, Nh, L, L] are the forward's weights.
     16-bit activations with head sizes that are multiples of 8 run through the library's own matrix-core
     products (mega_attention_bwd: head-strided operands read in place, the causal half of every product
-    skipped); fp32 and odd head sizes through four batched library GEMMs around mega_attention_softmax_bwd.
+    skipped); fp32 and odd head sizes through four batched products around mega_attention_softmax_bwd (fp32 on the
+    library's own kernel where the sizes pay, the others in the GEMM library).
     `y` (not in the reference's signature): the forward's output; with it the softmax backward's row sums are
     y_grad . y and the L x L weight gradient never reaches memory.  It must be the output the forward produced
     from this very `w` (y = w v); a `y` from anywhere else gives a wrong score gradient without any check --
@@ -790,21 +805,10 @@ def attention_bwd(y_grad, q, k, v, w, scale: float, use_causal_mask: bool, y=Non
                                         1 if use_causal_mask else 0, _ptr(ws), ws.numel(), _stream(dev))
         _lib.check(rc, "attention_bwd")
         return q_grad, k_grad, v_grad
-    if qd.numel() and own_attention_products(L, H1, H2, qd, kd, vd, wd, g):
-        c = use_causal_mask
-        q_grad, k_grad, v_grad, ds = (torch.empty_like(t) for t in (qd, kd, vd, wd))
-        _position_product((wd, 1), (g, 0), (v_grad, 0), L, H2, L, 3 if c else 0, a_rows=True, b_rows=True)
-        _position_product((g, 0), (vd, 0), (ds, 1), L, L, H2, 1 if c else 0)
-        attention_softmax_bwd(ds, wd, c, scale=float(scale), inplace=True)
-        _position_product((ds, 1), (qd, 0), (k_grad, 0), L, H1, L, 3 if c else 0, a_rows=True, b_rows=True)
-        _position_product((ds, 1), (kd, 0), (q_grad, 0), L, H1, L, 2 if c else 0, b_rows=True)
-        return q_grad, k_grad, v_grad
-    v_grad = torch.einsum('bnqk,bqnh->bknh', wd, g)
-    w_grad = torch.einsum('bqnh,bknh->bnqk', g, vd).contiguous()
-    s_grad = attention_softmax_bwd(w_grad, wd, use_causal_mask, scale=float(scale), inplace=True)
-    k_grad = torch.einsum('bnqk,bqnh->bknh', s_grad, qd)
-    q_grad = torch.einsum('bnqk,bknh->bqnh', s_grad, kd)
-    return q_grad, k_grad, v_grad
+    own = qd.numel() > 0 and own_attention_products(L, H1, H2, qd, kd, vd, wd, g)
+    v_grad = _weighted(wd, g, use_causal_mask, True, own)
+    s_grad = attention_softmax_bwd(_scores(g, vd, L, use_causal_mask, own=own), wd, use_causal_mask, scale=float(scale), inplace=True)
+    return _weighted(s_grad, kd, use_causal_mask, False, own), _weighted(s_grad, qd, use_causal_mask, True, own), v_grad
 
 
 # --------------------------------------------------------------------------------------

@@ -432,6 +432,7 @@ typedef struct {
   int32_t a_padded;      /* A's rows in memory are whole multiples of four elements, readable to their end */
 } MegaGemm;
 int mega_gemm_f32_pays(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor);   /* as well served here as by a GEMM library */
+int mega_gemm_f32_batched_pays(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t heads, int causal, int a_kmajor);
 size_t mega_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t batch);
 int mega_gemm_f32(const MegaGemm* g, void* workspace, size_t workspace_bytes, void* stream);
 /* The same for single bf16 / fp16 products (operands, bias, residual, pre and C of `dtype`, fp32 sums, alpha 1, silu of the

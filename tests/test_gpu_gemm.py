@@ -251,3 +251,48 @@ def test_values_that_are_not_finite_in_every_form(m, n, k, ka, kb):
     big = r.abs() > 1e30
     assert big[ok].any()
     assert _rel(c[ok & ~big], r[ok & ~big].double()) < _tol(k) and ((c - r).abs() <= 1e-6 * r.abs())[ok & big].all()
+
+
+@pytest.mark.parametrize("L,P,H", [(68, 68, 8), (1000, 1000, 64), (1003, 1004, 20), (2052, 2052, 12)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_position_products(L, P, H, causal):
+    """The attention's three kinds of product on the matrix-core kernel at sizes that a call may leave to the GEMM library as
+    well: two heads, padded rows (two-sided only), causal limits that leave operands' halves unread."""
+    if causal and P != L:
+        pytest.skip("padded rows are two-sided attention's")
+    B, Nh = 2, 2
+    gen = torch.Generator(DEV).manual_seed(L)
+    x, y = (torch.randn(B, L, Nh, H, generator=gen, device=DEV) for _ in range(2))
+    w = torch.randn(B, Nh, L, P, generator=gen, device=DEV)
+    w[..., L:] = 0
+    if causal:
+        w.tril_()
+    prod, t = M.ops._position_product, lambda a: a.double().transpose(1, 2).contiguous()
+    s = prod((x, 0), (y, 0), (torch.full_like(w, float("nan")), 1), L, L, H, int(causal), 0.5)[..., :L]
+    ref = 0.5 * (t(x) @ t(y).transpose(-1, -2).contiguous())
+    keep = torch.ones(L, L, dtype=torch.bool, device=DEV).tril() if causal else torch.ones(L, L, dtype=torch.bool, device=DEV)
+    assert _rel(s[..., keep], ref[..., keep]) < _tol(H)
+    w64 = w[..., :L].double()
+    for transposed in (False, True):
+        got = prod((w, 1), (x, 0), (torch.full_like(x, float("nan")), 0), L, H, L, (2 + transposed) * causal, a_rows=transposed, b_rows=True)
+        want = (w64.transpose(-1, -2).contiguous() if transposed else w64) @ t(x)
+        assert _rel(t(got), want) < _tol(L)
+
+
+@pytest.mark.parametrize("B,L,Nh,H1,H2", [(2, 1024, 1, 32, 64), (1, 2048, 1, 64, 512)])
+def test_attention_on_both_kinds_of_product(B, L, Nh, H1, H2):
+    """Sizes of which some products run on the matrix-core kernel and the others in the GEMM library: forward and backward
+    against 64 bits."""
+    gen = torch.Generator(DEV).manual_seed(L)
+    q, k, v, g = (torch.randn(B, L, Nh, h, generator=gen, device=DEV) for h in (H1, H1, H2, H2))
+    pays = M.ops._product_pays
+    assert len({pays(L, L, H1, B, Nh, 1, False), pays(L, H1, L, B, Nh, 2, False)}) == 2
+    y, w = M.ops.attention_fwd(q, k, v, 0.2, 0.0, True, need_weights=True)
+    got = M.ops.attention_bwd(g, q, k, v, w, 0.2, True)
+    t = [x.double().transpose(1, 2).contiguous().requires_grad_() for x in (q, k, v)]
+    s = (0.2 * (t[0] @ t[1].transpose(-1, -2))).masked_fill(torch.ones(L, L, dtype=torch.bool, device=DEV).triu(1), float("-inf"))
+    ref = s.softmax(-1) @ t[2]
+    ref.backward(g.double().transpose(1, 2))
+    assert _rel(y.transpose(1, 2), ref) < 4e-6
+    for x, r in zip(got, t):
+        assert _rel(x.transpose(1, 2), r.grad) < 1e-5

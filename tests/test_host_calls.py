@@ -183,3 +183,13 @@ def test_the_limit_of_16bit_products_stands_once():
     flops, (m, n) = M.modules.OWN_16BIT_FLOPS, (1000, 1000)
     k = int(flops / (2 * m * n))
     assert M._lib.load().mega_gemm16_pays(m, n, k, 0, 0) == 1 and M._lib.load().mega_gemm16_pays(m, n, k + 1, 0, 0) == 0
+
+
+@pytest.mark.parametrize("m,n,k,batch,heads,causal,a_kmajor,own", [
+    (512, 512, 128, 8, 1, 0, 0, 1), (1000, 64, 1000, 8, 1, 0, 0, 0), (4096, 64, 4096, 2, 1, 2, 0, 0), (512, 512, 1024, 1, 1, 1, 0, 0),
+    (1000, 1000, 64, 16, 4, 0, 0, 1), (2048, 2048, 1024, 4, 1, 0, 0, 1), (2048, 2048, 32, 8, 1, 0, 0, 0), (1000, 1000, 512, 8, 1, 0, 0, 1),
+    (2048, 2048, 512, 2, 1, 0, 0, 0), (2048, 1024, 2048, 2, 1, 3, 1, 1), (64, 2048, 64, 64, 1, 2, 0, 0), (2048, 64, 2048, 1, 1, 0, 0, 1), (1024, 1024, 1024, 2, 1, 2, 0, 1),
+    (2048, 128, 2048, 8, 1, 0, 0, 0)])
+def test_sizes_of_the_fp32_attention_products(m, n, k, batch, heads, causal, a_kmajor, own):
+    """Batched fp32 products that the matrix-core kernel serves clearly slower than the GEMM library are left to it."""
+    assert M._lib.load().mega_gemm_f32_batched_pays(m, n, k, batch, heads, causal, a_kmajor) == own
