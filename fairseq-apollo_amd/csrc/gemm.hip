@@ -9,7 +9,7 @@
 // formed, accumulation is fp32 throughout.  Measured against 64 bits the result is closer than the library's fp32
 // products (which round after every four reduction indices; here after 32): see the figures at gemm_plan.
 // Infinities, NaN and values that round beyond bf16's largest leave the split as NaN: an output element that is not
-// finite is formed again in plain fp32 (plain_block).
+// finite is formed again with plain fp32 multiply-adds.
 //
 // A workgroup owns a 128 x 128 (eight waves) or 64 x 64 (four) tile of C, 32 reduction indices a step: fp32 pieces go
 // from memory to registers two steps ahead, are split there and wait in LDS as three 16-bit planes per operand, two
@@ -190,37 +190,6 @@ struct Side {
   }
 };
 
-// A 16 x 16 block of the product from row m, column n on, in plain fp32 on the matrix cores' fp32 form, which treats
-// infinities and NaN as the arithmetic does: what the split leaves as NaN is formed again by it.  All lanes of a wave take
-// part; straight from memory, 32 indices a step.  Weight gradient 1024 x 1024 x 8000 without a finite element 1.57 ms, with
-// one row of them 0.87 (of finite values 0.2); a lane by itself for every element took 29.9 and 15.2 ms.
-template <bool KA, bool KB>
-__device__ __forceinline__ f32x4 plain_block(const float* A, const float* B, const GemmP& G, int m, int n, int kb, int ke, int lane) {
-  const int r = lane & 15, g = lane >> 4;
-  m = min(m + r, G.M - 1);
-  n = min(n + r, G.N - 1);
-  const float* pa = A + (KA ? (int64_t)m : (int64_t)m * G.lda);
-  const float* pb = B + (KB ? (int64_t)n : (int64_t)n * G.ldb);
-  const int64_t sa = KA ? G.lda : 1, sb = KB ? G.ldb : 1;
-  f32x4 s = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-  for (int k0 = kb; k0 < ke; k0 += kGK) {
-    float a[kGK / 4], b[kGK / 4];
-#pragma unroll
-    for (int h = 0; h < kGK / 4; ++h) {
-      const int k = min(k0 + h * 4 + g, ke - 1);
-      a[h] = pa[k * sa];
-      b[h] = pb[k * sb];
-    }
-#pragma unroll
-    for (int h = 0; h < kGK / 4; ++h) {
-      const bool in = k0 + h * 4 + g < ke;
-      s = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? b[h] : 0.f, in ? a[h] : 0.f, s, 0, 0, 0);
-    }
-  }
-  return s;
-}
-
 // TM x TN: the tile; two waves along its rows, WN along its columns.  FORM 0: whole steps of 32 reduction indices and
 // 16-byte accesses; 1: a partial last step; 2: operands that 16-byte accesses do not fit
 template <int TM, int TN, int WN, bool KA, bool KB, int FORM>
@@ -346,15 +315,28 @@ __global__ __launch_bounds__(128 * WN, 2) void gemm_f32_kernel(const GemmP G) {
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
       const int n = n0 + (wn + j) * 16 + (lane >> 4) * 4;
+      if (m >= G.M || n >= G.N) continue;
       float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
-      const bool in = m < G.M && n < G.N;
       const float chk = (v[0] - v[0]) + (v[1] - v[1]) + (v[2] - v[2]) + (v[3] - v[3]);
-      if (__any(in && chk != 0.f)) {                               // something is not finite
-        const f32x4 p = plain_block<KA, KB>(A, B, G, m0 + (wm + i) * 16, n0 + (wn + j) * 16, kb, ke, lane);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = v[u] - v[u] == 0.f ? v[u] : p[u];
+      if (chk != 0.f) {
+        // Something is not finite: in plain fp32, lane by lane, eight indices on their way at a time.  Weight gradient 1024 x
+        // 1024 x 8000 (180 us) with one row that is not finite 3.9 ms, without a finite element 7.3 (15 and 30 one index at a
+        // time; 0.9 and 1.6 by the matrix cores' fp32 form, whose code here had the compiler schedule the loop above worse:
+        // every product of finite values 3 - 8 % slower).
+#pragma unroll 1
+        for (int u = 0; u < 4; ++u) {
+          if (n + u >= G.N) break;
+          const float* pa = A + (KA ? (int64_t)m : (int64_t)m * G.lda);
+          const float* pb = B + (KB ? (int64_t)(n + u) : (int64_t)(n + u) * G.ldb);
+          float s = 0.f;
+#pragma unroll 8
+          for (int k = kb; k < ke; ++k) s = fmaf(pa[KA ? (int64_t)k * G.lda : k], pb[KB ? (int64_t)k * G.ldb : k], s);
+          if (u == 0) v[0] = s;
+          if (u == 1) v[1] = s;
+          if (u == 2) v[2] = s;
+          if (u == 3) v[3] = s;
+        }
       }
-      if (!in) continue;
       float* c = C + (int64_t)m * ldc + n;
       if (G.part) {
         if (G.N % 4 == 0) {
