@@ -594,13 +594,21 @@ bool product(const Tensor& a, const Tensor& b, const Tensor& bias, const Tensor&
   auto on16 = [](const Tensor& t) { return !t.defined() || (uintptr_t)t.data_ptr() % 16 == 0; };
   const int64_t vec = 16 / a.element_size(), far = ((int64_t)1 << 32) / a.element_size() / 128;
   if (!(wide ? mega_gemm_f32_pays : mega_gemm16_pays)(M, N, K, ma.first, !mb.first) || ma.ld % vec || mb.ld % vec || (ma.first ? M : K) % vec ||
-      (mb.first ? K : N) % vec || ma.ld >= far || mb.ld >= far || !on16(a) || !on16(b))
+      (mb.first ? K : N) % vec || ma.ld >= far || mb.ld >= far)
     return false;
   if (!wide && (N % vec || mr.ld % vec || !on16(bias) || !on16(residual) || !on16(*out))) return false;
+  // a gradient that starts off 16 bytes gives what the same gradient on 16 bytes gives: from a copy of it
+  auto aligned = [&](const Tensor& t, Matrix* m) {
+    if (on16(t)) return t;
+    const Tensor c = (m->first ? t.t() : t).clone(at::MemoryFormat::Contiguous);
+    m->ld = c.size(1);
+    return m->first ? c.t() : c;
+  };
+  const Tensor a16 = aligned(a, &ma), b16 = aligned(b, &mb);
   if (!out->defined()) *out = at::empty({M, N}, a.options());
   if (pre) *pre = at::empty({M, N}, a.options());
   MegaGemm g = {};
-  g.a = a.data_ptr(); g.b = b.data_ptr(); g.c = out->data_ptr();
+  g.a = a16.data_ptr(); g.b = b16.data_ptr(); g.c = out->data_ptr();
   g.bias = bias.defined() ? bias.data_ptr() : nullptr;
   g.residual = residual.defined() ? residual.data_ptr() : nullptr;
   g.pre = pre ? pre->data_ptr() : nullptr;
