@@ -1379,6 +1379,8 @@ OWN_16BIT_FLOPS = 6e9             # mega_gemm16_pays of products along the rows:
 
 def own_product(lin: nn.Linear, x: Tensor, *more) -> bool:
     """lin(x) outside training may be one of the library's own products (fp32, and 16-bit types at some sizes)."""
+    if type(lin) is not nn.Linear:                     # (a scripted module's parameters are no dictionary)
+        return False
     w, b = lin._parameters.get('weight'), lin._parameters.get('bias')
     return (x.is_cuda and x.dim() > 1 and w is not None and w.dim() == 2
             and (x.dtype is torch.float32 or 2 * x.numel() * w.shape[0] <= OWN_16BIT_FLOPS) and not torch.is_grad_enabled()

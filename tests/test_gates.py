@@ -84,3 +84,9 @@ def test_replaced_parts_of_a_layer_get_no_mask_of_zeros(part):
         else:
             layer.mega_layer = _Other()
         assert not model._mask_stays(_ON_DEVICE)
+
+
+def test_scripted_linear_layers_run_as_they_are():
+    lin, x = torch.nn.Linear(16, 8), torch.randn(3, 5, 16)
+    with torch.no_grad():
+        assert torch.equal(M.modules.project(torch.jit.script(lin), x), lin(x))
