@@ -90,3 +90,19 @@ def test_scripted_linear_layers_run_as_they_are():
     lin, x = torch.nn.Linear(16, 8), torch.randn(3, 5, 16)
     with torch.no_grad():
         assert torch.equal(M.modules.project(torch.jit.script(lin), x), lin(x))
+
+
+class _Scripted(torch.nn.Module):
+    def forward(self, x):
+        return x + 1
+
+
+def test_scripted_layers_get_no_mask_of_zeros():
+    """A scripted module among the layers, or in a layer's place for its attention: the mask rule says no."""
+    model = _language_model()
+    with torch.no_grad():
+        model.layers[1] = torch.jit.script(_Scripted())
+        assert not model._mask_stays(_ON_DEVICE)
+        model.layers[1] = _language_model().layers[1]
+        model.layers[1].mega_layer = torch.jit.script(_Scripted())
+        assert not model._mask_stays(_ON_DEVICE)
