@@ -84,7 +84,7 @@ __device__ __forceinline__ Moments merge(Moments a, Moments b) {
     const float w = (heavy_b ? a.n : b.n) * rn;
     const float d = om - bm, wd = w * d;
     r.mean = bm + wd;
-    r.var = bv + (w * (ov - bv) + wd * (d - wd));
+    r.var = bv < INFINITY ? bv + (w * (ov - bv) + wd * (d - wd)) : bv;      // (inf - inf: a variance beyond fp32 stays that)
   } else {
     const float cb = b.n * rn, ca = a.n * rn;
     const float d = b.mean - a.mean;

@@ -527,6 +527,29 @@ def test_a_token_that_is_not_a_number_counts(dtype, cpg):
     assert torch.isnan(mean[0, 1]) and not torch.isnan(mean[0, 0])
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, BF])
+@pytest.mark.parametrize("cpg", [32, 48, 64, 96, 128])
+@pytest.mark.parametrize("L,at", [(1024, 70), (2600, 1100), (512, 0)])
+def test_a_variance_beyond_fp32(dtype, cpg, L, at):
+    """One token whose values are finite and whose variance is not: the group's values are its bias from there on (their
+    factor is zero), as with the norm by itself; no NaN."""
+    print(f"case {dtype} cpg={cpg} L={L} at={at}", flush=True)
+    B, G = 1, 2
+    D = cpg * G
+    assert M.ops.norm_ema_one_kernel(0 if dtype is torch.float32 else 1, B, L, D, G, 16, 0, False)
+    p, q, g, om, nw, nb = _setup(np.random.default_rng(71), D, 16)
+    x = torch.randn(B, L, D, generator=torch.Generator().manual_seed(71)).to(dtype).to(DEV)
+    layer = M.ops.PreparedEMA(dev(p), dev(q), dev(g), dev(om))
+    x[0, at, cpg:] = torch.tensor([1e20, -1e20], dtype=dtype, device=DEV).repeat(cpg // 2)
+    xn, y, cnt, mean, var, _ = _run(layer, x, G, nw, nb, out_layout="input")
+    alone = M.ops.group_timestep_norm_fwd(x, torch.zeros(B, dtype=torch.int64, device=DEV), torch.zeros(B, G, device=DEV),
+                                          torch.ones(B, G, device=DEV), dev(nw) + 1, dev(nb), None, G, 1e-5)
+    bias = dev(nb)[cpg:].to(dtype)
+    assert torch.equal(alone[0][:, at:, cpg:], bias.expand(B, L - at, cpg)) and torch.equal(xn[:, at:, cpg:], alone[0][:, at:, cpg:])
+    assert cnt.tolist() == [L] and var[0, 1] == float("inf") == alone[3][0, 1] and torch.isfinite(mean).all()
+    assert torch.isfinite(xn).all() and torch.isfinite(y).all()
+
+
 @pytest.mark.parametrize("dtype,L,want_state,tol,state_tol", [(torch.float32, 40, False, 1e-6, 0), (torch.float32, 700, True, 1e-6, 5e-7),
                                                               (torch.float16, 700, True, 0, 5e-7), (BF, 40, True, 0, 5e-7)])
 def test_accuracy_of_short_rows_and_handed_on_states(dtype, L, want_state, tol, state_tol):
