@@ -1,6 +1,6 @@
 """Committed golden vectors (tests/golden/ref_cpu_vectors.npz: outputs of the reference's own CPU
 operators, written by tests/golden/make_golden.py) against the numpy oracle, the C oracle and,
-on a GPU box, the HIP library.  fp32 inputs; tolerance 2e-5 for the fp64/fp32 oracles
+on a GPU, the HIP library.  fp32 inputs; tolerance 2e-5 for the fp64/fp32 oracles
 (the vectors are fp32 results), 1e-4 for the HIP fp32 path."""
 import os
 

@@ -97,7 +97,7 @@ def test_config3_b64_d2048_2048_steps():
 
 
 def test_config3_bf16_full_width():
-    """configs[3] in its own arithmetic: 64 streams, D = 2048, N = 16, bf16 activations, 512 consecutive single-token
+    """The decode step in its own arithmetic: 64 streams, D = 2048, N = 16, bf16 activations, 512 consecutive single-token
     steps and then the same tokens as launches of 64; a sample of streams against the fp64 oracle (the norm on the
     bf16 inputs, the moving average on the bf16 xn the step produced, as a layer behind it would see it), every stream
     against the parallel path in bf16."""

@@ -83,7 +83,7 @@ def test_one_kernel_envelope_against_oracle(out_layout, B, L, G, N, cplx, cpg):
 
 
 def test_config2_headline_shape():
-    """B = 4, L = 4096, D = 1024, N = 16, 16 groups, bf16: the block of configs[2] as one kernel; the norm
+    """B = 4, L = 4096, D = 1024, N = 16, 16 groups, bf16: the headline block as one kernel; the norm
     against the closed form in fp64, the moving average against the FFT oracle on sampled channels."""
     B, L, D, N, G = 4, 4096, 1024, 16, 16
     rng = np.random.default_rng(1236)

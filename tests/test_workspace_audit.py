@@ -4,7 +4,7 @@
 No GPU: under mega_audit_begin() these entry points launch nothing; for every launch they would make they compute the
 last byte each operand is addressed at, from the sizes and strides the kernel would receive, and check it against the
 registered byte ranges of the call's tensors and workspace (made-up addresses here).  The shapes are the ones the GPU
-tests, the sweeps and the training benchmark of configs[4] use, plus ragged ones around the kernels' tile sizes.  The
+tests, the sweeps and the layer's training benchmark use, plus ragged ones around the kernels' tile sizes.  The
 workspace is registered with exactly `*_workspace_bytes` bytes, so a consumer that addresses one byte more fails."""
 import ctypes as C
 
@@ -40,7 +40,7 @@ def _finish(lib, rc, min_checks):
 
 ATT_SHAPES = [
     # B, L, Nh, H1, H2
-    (4, 2048, 4, 128, 1024),      # configs[4]: chunks of the layer's training step
+    (4, 2048, 4, 128, 1024),      # chunks of the layer's training step
     (2, 4096, 4, 128, 1024),
     (1, 512, 1, 64, 64), (2, 256, 2, 64, 128), (3, 64, 2, 8, 8), (1, 72, 1, 16, 24),
     (2, 100, 3, 32, 40),          # L % 8 != 0: the transposed-copy route
