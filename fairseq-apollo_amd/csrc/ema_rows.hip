@@ -634,7 +634,7 @@ int ema_rows_run(const void* x, void* y, int dtype, int64_t sxb, int64_t sxd, in
   if (bidirectional) {
     const bool vec = dtype == MEGA_F32 ? rows_vec_ok<float>(A) : rows_vec_ok<bf16_t>(A);
     if (vec && L % kRBlk == 0) {
-      // whole blocks: the two directions of a block of memory meet inside one wave
+      // whole blocks: the two directions of a block of memory meet in two waves of a workgroup
       A.both = 1;
       return launch(A);
     }

@@ -1170,7 +1170,8 @@ size_t fused_ws_bytes(int64_t B, int64_t D, int64_t S, int cw) {
 }
 
 // Channels of a workgroup for norm groups of gc channels, 0: no instance.  16-bit rows of a block fill the LDS with 64
-// channels, fp32 rows (two planes) with 32; a group that does not fit is shared by equal parts of a multiple of 16.
+// channels, fp32 rows (two planes) with 32; a group that does not fit is shared by equal parts of a multiple of 16.  Only the widths
+// below have instances, each measured against the two operators; others (16, 24, 80, 112, 160 and more) run as two operators.
 // The two operators one after the other (norm, transposition, rows kernels, transposition) take, against one launch
 // here, with y in x's layout: fp16 3 x 1501 x 768 in 48s 79 us, 26 here; fp16 4 x 4096 x 1024 in 64s 101 us, 34; fp16
 // 2 x 8192 x 2048 in 128s 249 us, 76; fp32 4 x 4096 x 1024 138 us, 53 (3.8 TB/s); fp32 2 x 8192 x 2048 in four parts

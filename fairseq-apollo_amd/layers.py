@@ -473,8 +473,9 @@ class MovingAverageGatedAttention(nn.Module, IncrementalState):
     def _padded_attention(self, q4: Tensor, k4: Tensor, v4: Tensor, key_padding: Tensor) -> Tensor:
         """Softmax attention outside the fused op (moving_average_gated_attention.py:210-256): the
         learned relative bias is added to the scores, scores of padded keys are -inf except in chunks
-        that consist of padding only; library GEMMs around the softmax op (causal for one-sided
-        layers)."""
+        that consist of padding only; the padded operator of fp32 layers without a learned bias
+        (ops.padded_attention_fwd), for the others torch products around the softmax op (causal for
+        one-sided layers)."""
         if self._padded_product(q4, k4, v4, key_padding):
             return ops.padded_attention_fwd(q4, k4, v4, key_padding)[0]
         s = torch.einsum('bqnh,bknh->bnqk', q4, k4)

@@ -1271,8 +1271,8 @@ class AttentionFunc(torch.autograd.Function):
     DropKey) for the backward pass.  Here they are kept only with DropKey or outside the matrix-core envelope;
     otherwise the forward is the one-kernel attention (no L x L array at all), q, k, v and y are saved, and the backward
     forms the weights again in scratch memory before its four products: B Nh L^2 elements less to hold per layer
-    between the passes (134 MB at configs[4]), the same gradients.  `KEEP_WEIGHTS = True` restores the reference's
-    behaviour.  `seed` (not in the reference) pins the DropKey mask."""
+    between the passes (134 MB for 4 chunks of 2048 tokens and 4 heads in bf16), the same gradients.
+    `KEEP_WEIGHTS = True` restores the reference's behaviour.  `seed` (not in the reference) pins the DropKey mask."""
 
     KEEP_WEIGHTS = False
 
@@ -1400,8 +1400,8 @@ def project(lin: nn.Linear, x: Tensor, act: bool = False) -> Tensor:
 
 
 def linear_residual(lin: nn.Linear, h: Tensor, residual: Optional[Tensor], consume: bool = False) -> Tensor:
-    """lin(h) + residual as one library GEMM (the residual is the accumulator's start, rounded once with the
-    product); lin(h) when there is no residual.  consume: the caller owns `residual` and has no further use for
+    """lin(h) + residual as one product, the library's own where its rules take it (own_product), else a GEMM library's
+    (the residual is the accumulator's start, rounded once with the product); lin(h) when there is no residual.  consume: the caller owns `residual` and has no further use for
     it, so outside autograd the product is accumulated into it in place (the out-of-place form first copies the
     residual into its result: one more pass over the activations)."""
     if residual is None:
