@@ -1,70 +1,42 @@
-// Matrix products of bf16 / fp16 activations for the sizes the GEMM library serves badly: C = op(A) op(B) (+ bias)
-// (+ residual), and silu of the rounded value.  A library call costs 26 us of host time, more than most products of a
-// few thousand tokens take, and its weight gradients (both operands stored along the other axis, a reduction over
-// thousands of tokens onto a small matrix) run at a third to a half of its forward products' rate.  Which sizes come here:
-// gemm16_wins.
+// Matrix products of bf16 / fp16 activations: C = op(A) op(B) (+ bias) (+ residual), and silu of the rounded value.  A library
+// call costs 26 us of host time, more than most products of a few thousand tokens take, and its weight gradients (both
+// operands stored along the other axis, a reduction over thousands of tokens onto a small matrix) run at a third to a half
+// of its forward products' rate.  Here are the kernel for few tokens and the entry; wide tiles: gemm16_wide.h.
 //
-// A workgroup of four waves owns a 128 x 128 or 64 x 64 tile, 32 or 64 reduction indices a step: 16-byte pieces go from memory
+// A workgroup of four waves owns a 64 x 64 tile, 64 reduction indices a step: 16-byte pieces go from memory
 // to registers two steps ahead and from there to one of two LDS stages, k-contiguous operands as rows of a step's indices,
 // the others as they lie in memory, their fragments read by transposing LDS loads.  Sums are fp32 throughout, also
 // between the parts of a product that is split along the reduction.
 #include <type_traits>
 
-#include "common.h"
+#include "gemm16.h"
 
 namespace mega {
 namespace {
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-typedef __attribute__((ext_vector_type(4))) short s16x4;
-
 constexpr int kHT = 256;          // threads
+constexpr int kTile = 64;         // rows, columns and reduction indices of a step
 
-struct Gemm16P {
-  const void *A, *B;   // element (m, k): m * lda + k, or (K-major) k * lda + m; (n, k) alike
-  void* C;             // m * ldc + n
-  const void* bias;    // [N] or null
-  const void* R;       // added: m * ldr + n, or null
-  void* pre;           // the value before the activation, or null
-  int64_t lda, ldb, ldc, ldr;
-  int M, N, K, silu;
-  int mt, nt;
-  int kstep;           // reduction indices of a split
-  float* part;         // [splits][M][N], or null
-};
-
-template <typename T>
-__device__ __forceinline__ f32x4 mma16(uint4 a, uint4 b, f32x4 c) {
-  if constexpr (__is_same(T, bf16_t))
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
-
-__device__ __forceinline__ float silu_h(float v) { return v / (1.f + __expf(-v)); }
-
-// One operand's side of the tile: W rows (of A) or columns (of B), KM: stored K-major.
-template <int W, bool KM, int kHK>
+// One operand's side of the tile: 64 rows (of A) or columns (of B), KM: stored K-major.
+template <bool KM>
 struct Side16 {
-  static constexpr int Row = KM ? W * 2 : kHK * 2;                // bytes of a row
-  static constexpr int Bytes = W * kHK * 2;
-  static constexpr int NP = W * kHK / 8 / kHT;                    // 16-byte pieces per thread
+  static constexpr int Row = kTile * 2;                           // bytes of a row
+  static constexpr int Bytes = kTile * kTile * 2;
+  static constexpr int NP = kTile * kTile / 8 / kHT;              // 16-byte pieces per thread
 
   static __device__ __forceinline__ void piece(int tid, int h, int& w, int& k) {
     const int p = tid + h * kHT;
     if constexpr (KM) {
-      w = (p % (W / 8)) * 8;
-      k = p / (W / 8);
+      w = (p % (kTile / 8)) * 8;
+      k = p / (kTile / 8);
     } else {
-      w = p / (kHK / 8);
-      k = (p % (kHK / 8)) * 8;
+      w = p / (kTile / 8);
+      k = (p % (kTile / 8)) * 8;
     }
   }
   static __device__ __forceinline__ int turn(int row) {
-    if constexpr (KM) return W == 128 ? (row & 3) + 4 * ((row >> 3) & 1) : ((row >> 1) & 1) + 2 * ((row >> 3) & 1);
-    else return kHK == 64 ? (row >> 1) & 7 : (row >> 2) & 3;
+    if constexpr (KM) return ((row >> 1) & 1) + 2 * ((row >> 3) & 1);
+    else return (row >> 1) & 7;
   }
   // byte offset of piece h from the tile's first element in a step of `left` indices; what lies beyond the matrix is
   // replaced by the last piece inside it (rows are never stored, indices are cleared below)
@@ -107,44 +79,19 @@ struct Side16 {
   }
 };
 
-template <typename T>
-__device__ __forceinline__ void finish16(const Gemm16P& G, int m, int n, float (&v)[4]) {
-  T* const C = (T*)G.C;
-  if (G.bias) {
-    const Vec<T, 4> b = *(const Vec<T, 4>*)((const T*)G.bias + n);
-#pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] += to_float(b.v[u]);
-  }
-  if (G.R) {
-    const Vec<T, 4> r = *(const Vec<T, 4>*)((const T*)G.R + (int64_t)m * G.ldr + n);
-#pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] += to_float(r.v[u]);
-  }
-  Vec<T, 4> o;
-#pragma unroll
-  for (int u = 0; u < 4; ++u) o.v[u] = from_float<T>(v[u]);
-  if (G.pre) *(Vec<T, 4>*)((T*)G.pre + (int64_t)m * G.ldc + n) = o;
-  if (G.silu) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) o.v[u] = from_float<T>(silu_h(to_float(o.v[u])));
-  }
-  *(Vec<T, 4>*)(C + (int64_t)m * G.ldc + n) = o;
-}
-
-// TT: edge of the tile (a wave forms a quarter of it); RAG: a partial last step
-template <typename T, int TT, bool KA, bool KB, bool RAG>
+// RAG: a partial last step
+template <typename T, bool KA, bool KB, bool RAG>
 __global__ __launch_bounds__(kHT, 2) void gemm16_kernel(const Gemm16P G) {
-  constexpr int kHK = TT == 128 ? 32 : 64;                       // reduction indices a step
-  using SA = Side16<TT, KA, kHK>;
-  using SB = Side16<TT, KB, kHK>;
-  constexpr int F = TT / 32;
+  using SA = Side16<KA>;
+  using SB = Side16<KB>;
+  constexpr int F = kTile / 32;                                  // 16 x 16 blocks of a wave each way
   constexpr int kStage = SA::Bytes + SB::Bytes;
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int tiles = G.mt * G.nt, total = (int)gridDim.x;
   const int id = total % 8 == 0 ? ((int)blockIdx.x & 7) * (total >> 3) + ((int)blockIdx.x >> 3) : (int)blockIdx.x;
   const int z = id / tiles, tl = id - z * tiles;
-  const int mi = tl / G.nt, m0 = mi * TT, n0 = (tl - mi * G.nt) * TT;
+  const int mi = tl / G.nt, m0 = mi * kTile, n0 = (tl - mi * G.nt) * kTile;
   const int kb = G.part ? z * G.kstep : 0, ke = G.part ? min(G.K, kb + G.kstep) : G.K;
   f32x4 acc[F][F];
 #pragma unroll
@@ -160,19 +107,19 @@ __global__ __launch_bounds__(kHT, 2) void gemm16_kernel(const Gemm16P G) {
 #pragma unroll
     for (int h = 0; h < SB::NP; ++h) ob[h] = SB::offset(G.ldb, tid, h, G.N - n0, left);
   };
-  offsets(kHK);
+  offsets(kTile);
   const char* const ta = (const char*)G.A + (KA ? (int64_t)kb * G.lda + m0 : (int64_t)m0 * G.lda + kb) * 2;
   const char* const tb = (const char*)G.B + (KB ? (int64_t)kb * G.ldb + n0 : (int64_t)n0 * G.ldb + kb) * 2;
-  const int64_t da = (KA ? kHK * G.lda : kHK) * 2, db = (KB ? kHK * G.ldb : kHK) * 2;
-  const int steps = (ke - kb + kHK - 1) / kHK;
+  const int64_t da = (KA ? kTile * G.lda : kTile) * 2, db = (KB ? kTile * G.ldb : kTile) * 2;
+  const int steps = (ke - kb + kTile - 1) / kTile;
   auto load = [&](int s, uint4 (&va)[SA::NP], uint4 (&vb)[SB::NP]) {
     s = min(s, steps - 1);
-    if (RAG) offsets(min(kHK, ke - kb - s * kHK));
+    if (RAG) offsets(min(kTile, ke - kb - s * kTile));
     SA::load(ta + s * da, oa, va);
     SB::load(tb + s * db, ob, vb);
   };
   auto store = [&](int s, char* stage, uint4 (&va)[SA::NP], uint4 (&vb)[SB::NP]) {
-    const int left = RAG ? ke - kb - s * kHK : kHK;
+    const int left = RAG ? ke - kb - s * kTile : kTile;
     SA::store(stage, tid, left, va);
     SB::store(stage + SA::Bytes, tid, left, vb);
   };
@@ -181,7 +128,7 @@ __global__ __launch_bounds__(kHT, 2) void gemm16_kernel(const Gemm16P G) {
     const char* la = lds + p * kStage;
     const char* lb = la + SA::Bytes;
 #pragma unroll
-    for (int kk = 0; kk < kHK / 32; ++kk) {
+    for (int kk = 0; kk < kTile / 32; ++kk) {
       uint4 fa[F], fb[F];
 #pragma unroll
       for (int i = 0; i < F; ++i) fa[i] = SA::frag(la, wm + i, kk, lane);
@@ -220,7 +167,7 @@ __global__ __launch_bounds__(kHT, 2) void gemm16_kernel(const Gemm16P G) {
       if (m >= G.M || n >= G.N) continue;                          // (N is a multiple of eight)
       float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
       if (part) *(float4*)(part + (int64_t)m * G.N + n) = make_float4(v[0], v[1], v[2], v[3]);
-      else finish16<T>(G, m, n, v);
+      else finish16<T, 4>(G, m, n, v);
     }
   }
 }
@@ -235,65 +182,72 @@ __global__ __launch_bounds__(256) void gemm16_sum_kernel(const Gemm16P G, int sp
     v[0] += p.x; v[1] += p.y; v[2] += p.z; v[3] += p.w;
   }
   const int m = (int)(i / G.N);
-  finish16<T>(G, m, (int)(i - (int64_t)m * G.N), v);
+  finish16<T, 4>(G, m, (int)(i - (int64_t)m * G.N), v);
 }
 
 struct Plan16 {
-  int tile, splits, kstep;
+  int splits, kstep;
 };
 
-// Tiles of 128 (32 indices a step: 196 registers, no spills; 64 indices spill) where a long reduction makes two
-// workgroups for every compute unit of them, of 64 otherwise; a product of few tiles is split along the reduction.
+// A product of few tiles is split along the reduction.
 Plan16 gemm16_plan(int64_t M, int64_t N, int64_t K) {
   const int cus = device_cu_count();
-  Plan16 p = {64, 1, 0};
-  const int64_t t128 = ceil_div(M, 128) * ceil_div(N, 128), parts = K / 2048 > 4 ? 4 : K / 2048;
-  if (t128 * parts >= 2 * cus) p.tile = 128;
-  const int64_t tiles = ceil_div(M, p.tile) * ceil_div(N, p.tile);
+  Plan16 p = {1, 0};
+  const int64_t tiles = ceil_div(M, kTile) * ceil_div(N, kTile);
   if (tiles <= cus / 2) {
     int64_t s = ceil_div(2 * cus, tiles);
     const int64_t most = K / 512;
     if (s > most) s = most;
     if (s > 32) s = 32;
     if (s > 1) {
-      p.kstep = (int)(ceil_div(ceil_div(K, s), 64) * 64);
+      p.kstep = (int)(ceil_div(ceil_div(K, s), kTile) * kTile);
       p.splits = (int)ceil_div(K, p.kstep);
     }
   }
   return p;
 }
 
-// Sizes this kernel serves better than the library, us of device time (its call costs the host 20 us less, and a pass
-// over so few tokens is bound by the host):
-//   at most 6 GFLOP    1000 x 2048 x 1024  12   library 11      1000 x 1024 x 2048  15   library 11
-//                       300 x 2048 x 1024  7.6  library 7.7     2000 x 1088 x 512  9.5   library 10.5
-//   and not          1000 x 4352 x 1024 (9 GFLOP)  25   library 15      8192 x 2048 x 1024  50   library 30
-//   weight gradients (both K-major) onto at most 2 M elements over 2048 tokens and more
-//                    2048 x 1024 x 8192  55   library 70       264 x 1024 x 8192  22   library 52
-//   and not          2816 x 1024 x 8192  80   library 80      4096 x 2048 x 8192 160   library 135
-bool gemm16_wins(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor) {
-  return 2.0 * (double)M * (double)N * (double)K <= 6e9 || (a_kmajor && b_kmajor && M * N <= (int64_t)1 << 21 && K >= 2048);
+// What a product costs here, us of device time: half a microsecond a step of the two workgroups a compute unit holds, the
+// second kernel's 5 and its traffic at 4 TB/s.
+double gemm16_small_us(int64_t M, int64_t N, int64_t K) {
+  const Plan16 p = gemm16_plan(M, N, K);
+  const double tiles = (double)ceil_div(M, kTile) * ceil_div(N, kTile) * p.splits, two = 2.0 * device_cu_count();
+  return 4 + 0.5 * ceil_div(ceil_div(K, p.splits), kTile) * (tiles > two ? tiles / two : 1) +
+         (p.splits > 1 ? 5 + (double)M * N * (4 * p.splits + 2) / 4e6 : 0);
 }
 
-template <typename T, int TT, bool KA, bool KB, bool RAG>
-void launch16(const Gemm16P& G, unsigned blocks, hipStream_t s) {
-  const auto kern = gemm16_kernel<T, TT, KA, KB, RAG>;
-  constexpr int smem = 2 * 2 * TT * (TT == 128 ? 32 : 64) * 2;
-  static_assert(smem <= 64 * 1024, "within the LDS that every launch may ask for");
-  hipLaunchKernelGGL(kern, dim3(blocks), dim3(kHT), smem, s, G);
+// Wide tiles (gemm16_wide.h) where their estimate is the smaller one; us, tiles of 64 and wide ones:
+//     300 x 4352 x 1024   10, 15       600 x 4352 x 1024   16.5, 15     1000 x 4352 x 1024   25, 16
+//    2048 x 2048 x 1024   19, 16      2048 x 4352 x 1024   43, 26       5000 x 1536 x 768    27, 16
+//   both K-major   264 x 1024 x 8192   22, 24     1024 x 2048 x 2000   21, 27     1536 x 768 x 4503   39, 26
+bool gemm16_wide(int64_t M, int64_t N, int64_t K, WidePlan* p) {
+  *p = gemm16_wide_plan(M, N, K);
+  return p->us < gemm16_small_us(M, N, K);
 }
-template <typename T, int TT, bool RAG>
-void launch16_order(const Gemm16P& G, int ka, int kb, unsigned blocks, hipStream_t s) {
-  if (ka && kb) launch16<T, TT, true, true, RAG>(G, blocks, s);
-  else if (ka) launch16<T, TT, true, false, RAG>(G, blocks, s);
-  else if (kb) launch16<T, TT, false, true, RAG>(G, blocks, s);
-  else launch16<T, TT, false, false, RAG>(G, blocks, s);
+
+// Products that come here: all but the largest, whose one library call costs the host nothing against milliseconds on the
+// device.  us of device time beside the library's, whose call costs the host 20 us more and takes no silu:
+//   x W^T      8192 x 2048 x 1024   32.0, 31.1     8192 x 4352 x 1024   80.8, 71.9     8192 x 1024 x 2048   31.5, 33.1
+//              8192 x 2816 x 1024   53.0, 48.8     8192 x 1024 x 2816   43.6, 45.1     6144 x 2816 x 1024   46.3, 53.7
+//              8192 x 8704 x 2048    228, 242      8192 x 5632 x 2048    145, 156      8192 x 2048 x 5632    137, 122
+//   dY W       8192 x 1024 x 4352   67.2, 71.6     8192 x 2048 x 4096   95.7, 103      8192 x 2048 x 8704    193, 208
+//   dY^T X     2048 x 1024 x 8192   43.0, 69.3     4352 x 1024 x 8192   82.2, 116      8704 x 2048 x 8192    224, 307
+//              1024 x 2816 x 8192   59.1, 84.8     2048 x 5632 x 8192    174, 178
+bool gemm16_wins(int64_t M, int64_t N, int64_t K) { return 2.0 * (double)M * (double)N * (double)K <= 1e13; }
+
+template <typename T, bool KA, bool KB>
+void launch16(const Gemm16P& G, unsigned blocks, hipStream_t s) {
+  constexpr int smem = 2 * 2 * kTile * kTile * 2;
+  static_assert(smem <= 64 * 1024, "within the LDS that every launch may ask for");
+  const auto kern = G.K % kTile ? gemm16_kernel<T, KA, KB, true> : gemm16_kernel<T, KA, KB, false>;
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(kHT), smem, s, G);
 }
 template <typename T>
 void launch16_type(const Gemm16P& G, const Plan16& p, int ka, int kb, unsigned blocks, hipStream_t s) {
-  const bool rag = G.K % 64 != 0;
-  if (p.tile == 128) rag ? launch16_order<T, 128, true>(G, ka, kb, blocks, s) : launch16_order<T, 128, false>(G, ka, kb, blocks, s);
-  else rag ? launch16_order<T, 64, true>(G, ka, kb, blocks, s) : launch16_order<T, 64, false>(G, ka, kb, blocks, s);
+  if (ka && kb) launch16<T, true, true>(G, blocks, s);
+  else if (ka) launch16<T, true, false>(G, blocks, s);
+  else if (kb) launch16<T, false, true>(G, blocks, s);
+  else launch16<T, false, false>(G, blocks, s);
   if (p.splits > 1)
     hipLaunchKernelGGL((gemm16_sum_kernel<T>), dim3((unsigned)ceil_div((int64_t)G.M * G.N, 1024)), dim3(256), 0, s, G, p.splits);
 }
@@ -304,13 +258,15 @@ void launch16_type(const Gemm16P& G, const Plan16& p, int ka, int kb, unsigned b
 using namespace mega;
 
 extern "C" int mega_gemm16_pays(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor) {
-  return gemm16_wins(M, N, K, a_kmajor, b_kmajor) ? 1 : 0;
+  return gemm16_wins(M, N, K) ? 1 : 0;
 }
 
 extern "C" size_t mega_gemm16_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const Plan16 p = gemm16_plan(M, N, K);
-  return p.splits > 1 ? (size_t)p.splits * M * N * 4 : 0;
+  const size_t small = p.splits > 1 ? (size_t)p.splits * M * N * 4 : 0;
+  WidePlan w;
+  return gemm16_wide(M, N, K, &w) && w.bytes > small ? w.bytes : small;
 }
 
 extern "C" int mega_gemm16(const MegaGemm* g, int dtype, void* workspace, size_t workspace_bytes, void* stream) {
@@ -333,9 +289,19 @@ extern "C" int mega_gemm16(const MegaGemm* g, int dtype, void* workspace, size_t
   G.A = g->a; G.B = g->b; G.C = g->c; G.bias = g->bias; G.R = g->residual; G.pre = g->pre;
   G.lda = g->lda; G.ldb = g->ldb; G.ldc = g->ldc; G.ldr = g->ldr;
   G.M = (int)g->M; G.N = (int)g->N; G.K = (int)g->K; G.silu = g->silu;
+  WidePlan w;
+  // (rows of a wide tile within 4 GB of its first element)
+  if (gemm16_wide(g->M, g->N, g->K, &w) && g->lda < far / 2 && g->ldb < far / 2) {
+    MEGA_REQUIRE(ceil_div(g->M, kWideM) * ceil_div(g->N, w.tn) < (int64_t)1 << 27, MEGA_ERR_UNSUPPORTED, "gemm16: too many tiles");
+    MEGA_REQUIRE(!w.bytes || (workspace && workspace_bytes >= w.bytes && on16(workspace)), MEGA_ERR_WORKSPACE,
+                 "gemm16: workspace of %zu bytes needed", w.bytes);
+    gemm16_wide_launch(G, w, dtype == MEGA_BF16, g->a_kmajor, g->b_kmajor, workspace, (hipStream_t)stream);
+    MEGA_CHECK_LAUNCH("gemm16 (wide tiles)");
+    return MEGA_OK;
+  }
   const Plan16 p = gemm16_plan(g->M, g->N, g->K);
-  G.mt = (int)ceil_div(g->M, p.tile);
-  G.nt = (int)ceil_div(g->N, p.tile);
+  G.mt = (int)ceil_div(g->M, kTile);
+  G.nt = (int)ceil_div(g->N, kTile);
   if (p.splits > 1) {
     const size_t need = (size_t)p.splits * g->M * g->N * 4;
     MEGA_REQUIRE(workspace && workspace_bytes >= need && on16(workspace), MEGA_ERR_WORKSPACE, "gemm16: workspace of %zu bytes needed",

@@ -1374,7 +1374,7 @@ class EfficientAttention(nn.Module):
         return 'causal={}, dropout={}'.format(self._causal, self._dropout)
 
 
-OWN_16BIT_FLOPS = 6e9             # mega_gemm16_pays of products along the rows: no native call is made to be told no
+OWN_16BIT_FLOPS = 1e13            # mega_gemm16_pays of products along the rows: no native call is made to be told no
 
 
 def own_product(lin: nn.Linear, x: Tensor, *more) -> bool:

@@ -294,3 +294,46 @@ def test_attention_on_both_kinds_of_product(B, L, Nh, H1, H2):
     assert _rel(y.transpose(1, 2), ref) < 4e-6
     for x, r in zip(got, t):
         assert _rel(x.transpose(1, 2), r.grad) < 1e-5
+
+
+# sizes on wide tiles: 256 x 128 with every remainder and whole; the same in parts; 256 x 256 all in parts, whole ones and the
+# last in parts, with remainders and whole
+_WIDE = [(1096, 4360, 1032), (2048, 2048, 1024), (1032, 1048, 8200), (4352, 1032, 8200), (8712, 2056, 4104), (6144, 2816, 1024)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("ka,kb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("m,n,k", _WIDE + [(1032, 1048, 8199)])
+def test_16bit_products_on_wide_tiles(dtype, ka, kb, m, n, k):
+    """As test_16bit_products; columns beside the operands' own hold NaN, and the last rows and columns are checked apart."""
+    if k % 8 and not (ka and kb):
+        pytest.skip("rows of whole 16-byte pieces")
+    print(f"case {dtype} m={m} n={n} k={k} ka={ka} kb={kb}", flush=True)
+    gen = torch.Generator(DEV).manual_seed(m + n + k)
+
+    def mk(r, c):
+        t = torch.full((r, c + 8), float("nan"), device=DEV, dtype=dtype)
+        t[:, :c] = torch.randn(r, c, generator=gen, device=DEV)
+        return t[:, :c]
+
+    a, b = mk(k, m) if ka else mk(m, k), mk(k, n) if kb else mk(n, k)
+    r = (a.double().t() if ka else a.double()) @ (b.double() if kb else b.double().t())
+    c = _gemm(a, b, ka, kb)
+    tol = (2.0 ** -9 if dtype is torch.bfloat16 else 2.0 ** -12) + _tol(k)
+    assert _rel(c, r) < tol and _rel(c[-8:], r[-8:]) < tol and _rel(c[:, -8:], r[:, -8:]) < tol
+
+
+@pytest.mark.parametrize("bias,res,silu,pre", [(1, 0, 0, 0), (0, 1, 0, 0), (1, 0, 1, 0), (1, 1, 1, 1), (0, 0, 1, 1), (1, 0, 0, 1)])
+@pytest.mark.parametrize("m,n,k", [(1096, 4360, 1032), (1032, 1048, 8200), (6144, 2816, 1024)])
+def test_16bit_epilogues_on_wide_tiles(m, n, k, bias, res, silu, pre):
+    gen = torch.Generator(DEV).manual_seed(8)
+    mk = lambda *s: torch.randn(*s, generator=gen, device=DEV).to(torch.bfloat16)
+    a, b, v, x = mk(m, k), mk(n, k), mk(n) * 30, mk(m, n) * 30
+    r = a.double() @ b.double().t() + bias * v.double() + res * x.double()
+    got = _gemm(a, b, 0, 0, v if bias else None, x if res else None, bool(silu), bool(pre))
+    c, p = got if pre else (got, None)
+    tol = 2.0 ** -9 + _tol(k)
+    if pre:
+        assert _rel(p, r) < tol
+    # silu of the rounded value (known where it is written as well; its slope is at most 1.1), rounded again
+    assert _rel(c, F.silu(p.double() if pre else r) if silu else r) < (2.0 ** -9 + 2.0 ** -22 if pre and silu else 3 * tol if silu else tol)
