@@ -164,13 +164,15 @@ __device__ __forceinline__ uint4 eight(const uint32_t (&p)[4]) {
 // SIMD), so instructions count: bias in registers, rows' pointers once, rounded pairs exchanged instead of single values
 // (8192 x 2048 x 1024 with 256-column tiles: 32.0 us, 34.3 through finish16 on eight exchanged floats).
 //
-// KIND 0: the sums alone, 1: with bias or residual, 2: silu and the value before as well
+// Branches between the blocks keep one block's loads and exponentials from running beside the next one's, so the frequent
+// kinds are whole: 0 the sums alone, 1 with a bias, 2 with a residual, 3 silu of 1, 4 anything (8192 x 2048 x 1024: 31, 31, 38,
+// 34 us; residual and silu with branches 41 and 39).
 template <typename T, bool ACC, int KIND, bool EDGE, int FM, int FN>
 __device__ __forceinline__ void store_wave(const Gemm16P& G, const Place& p, int wm, int wn, int lane, const f32x4 (&acc)[FM][FN]) {
   const int g = lane >> 4, row = wm * 16 + (lane & 15), col = wn * 16;
   const int m0 = p.m0 + row, n0 = p.n0 + col, own = n0 + g * 4, mine = n0 + (g & 1) * 16 + (g >> 1) * 8;
   float bias[FN][4];
-  if (KIND && G.bias) {
+  if (KIND && KIND != 2 && G.bias) {
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
       const int n = EDGE ? min(own + j * 16, G.N - 4) : own + j * 16;
@@ -188,7 +190,7 @@ __device__ __forceinline__ void store_wave(const Gemm16P& G, const Place& p, int
   for (int i = 0; i < FM; ++i) {
     const int m = m0 + i * 16, mr = EDGE ? min(m, G.M - 1) : m;
     const int64_t at = (int64_t)mr * G.ldc + mine;
-    const T* r = KIND && G.R ? (const T*)G.R + (int64_t)mr * G.ldr : nullptr;
+    const T* r = KIND == 2 || (KIND == 4 && G.R) ? (const T*)G.R + (int64_t)mr * G.ldr : nullptr;
 #pragma unroll
     for (int j = 0; j < FN; j += 2) {
       const bool in = !EDGE || (m < G.M && mine + j * 16 < G.N);   // (N is a multiple of eight)
@@ -198,8 +200,8 @@ __device__ __forceinline__ void store_wave(const Gemm16P& G, const Place& p, int
         float v[4];
         const f32x4 sum = values<ACC>(acc[i][j + h]);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = KIND ? sum[u] + bias[j + h][u] : sum[u];
-        if (KIND && r) {
+        for (int u = 0; u < 4; ++u) v[u] = KIND && KIND != 2 ? sum[u] + bias[j + h][u] : sum[u];
+        if (KIND == 2 || (KIND == 4 && r)) {
           const int n = own + (j + h) * 16;
           const Vec<T, 4> t = *(const Vec<T, 4>*)(r + (EDGE ? min(n, G.N - 4) : n));
 #pragma unroll
@@ -208,11 +210,11 @@ __device__ __forceinline__ void store_wave(const Gemm16P& G, const Place& p, int
         q[2 * h] = pack16<T>(v[0], v[1]);
         q[2 * h + 1] = pack16<T>(v[2], v[3]);
       }
-      if (KIND == 2 && G.pre) {
+      if (KIND == 4 && G.pre) {
         const uint4 x = eight(q);
         if (in) *(uint4*)((T*)G.pre + at + j * 16) = x;
       }
-      if (KIND == 2 && G.silu) {
+      if (KIND == 3 || (KIND == 4 && G.silu)) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) q[u] = pack16<T>(silu_h(low16<T>(q[u])), silu_h(low16<T>(q[u] >> 16)));
       }
@@ -231,12 +233,13 @@ __device__ __forceinline__ void finish_wave(const Gemm16P& G, const Place& p, in
 #pragma unroll
       for (int j = 0; j < FN; ++j) *(f32x4*)(c + i * 16 * TN + j * 16) = values<ACC>(acc[i][j]);
   } else if (p.m0 + kWideM <= G.M && p.n0 + TN <= G.N) {
-    if (G.silu || G.pre) store_wave<T, ACC, 2, false>(G, p, wm, wn, lane, acc);
-    else if (G.bias || G.R) store_wave<T, ACC, 1, false>(G, p, wm, wn, lane, acc);
+    if (G.pre || (G.R && (G.bias || G.silu))) store_wave<T, ACC, 4, false>(G, p, wm, wn, lane, acc);
+    else if (G.R) store_wave<T, ACC, 2, false>(G, p, wm, wn, lane, acc);
+    else if (G.silu) store_wave<T, ACC, 3, false>(G, p, wm, wn, lane, acc);
+    else if (G.bias) store_wave<T, ACC, 1, false>(G, p, wm, wn, lane, acc);
     else store_wave<T, ACC, 0, false>(G, p, wm, wn, lane, acc);
   } else {
-    if (G.silu || G.pre) store_wave<T, ACC, 2, true>(G, p, wm, wn, lane, acc);
-    else store_wave<T, ACC, 1, true>(G, p, wm, wn, lane, acc);
+    store_wave<T, ACC, 4, true>(G, p, wm, wn, lane, acc);
   }
 }
 
