@@ -94,7 +94,7 @@ struct Side {
   // swizzle of the 32-byte spans of a K-major row / the 16-byte pieces of a k-contiguous one
   static __device__ __forceinline__ int turn(int row) {
     if constexpr (KM) return W == 128 ? (row & 3) + 4 * ((row >> 3) & 1) : ((row >> 1) & 1) + 2 * ((row >> 3) & 1);
-    else return (row >> 2) & 3;
+    else return (0x78 >> (row >> 1 & 6)) & 3;        // 0, 2, 3, 1
   }
 
   // byte offset of piece h from the tile's first element in a step of `left` reduction indices; rows and indices beyond
