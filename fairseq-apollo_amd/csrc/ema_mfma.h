@@ -73,12 +73,10 @@ int ema_mfma_try(const void* x, void* y, int dtype, int64_t sxb, int64_t sxd, in
                  int64_t N, int64_t L, int bidirectional, int64_t Lk, float* acc, float* h_tile, hipStream_t s);
 
 // ---- [B, D, L] rows of any activation type, parallel over blocks of 1024 tokens (csrc/ema_rows.hip)
-size_t ema_rows_record_bytes(int64_t B, int64_t D, int64_t L, int bidirectional);
 bool ema_rows_covers(int dtype, int64_t sxb, int64_t sxd, int64_t sxl, int64_t syb, int64_t syd, int64_t syl,
                      int64_t B, int64_t D, int64_t N, int64_t L, int64_t Lk, const float* h_out);
 int ema_rows_run(const void* x, void* y, int dtype, int64_t sxb, int64_t sxd, int64_t syb, int64_t syd,
                  const void* image, int is_complex, const float* omega, const uint8_t* mask, const float* h_in,
-                 float* h_out, int64_t B, int64_t D, int64_t N, int64_t L, int bidirectional, float* acc, float* rec,
-                 hipStream_t s);
+                 float* h_out, int64_t B, int64_t D, int64_t N, int64_t L, int bidirectional, hipStream_t s);
 
 }  // namespace mega

@@ -1056,7 +1056,7 @@ __global__ void coef_prep_kernel(const float* __restrict__ p, const float* __res
 
 struct Plan {
   int NP, TPR, Tc, nchunks;
-  size_t coef_bytes, st_bytes, acc_bytes, tile_bytes, image_bytes, rows_bytes, total;
+  size_t coef_bytes, st_bytes, acc_bytes, tile_bytes, image_bytes, total;
 };
 
 Plan make_plan(int64_t B, int64_t D, int64_t N, int64_t L, int nsets, bool need_acc, bool bidirectional = false) {
@@ -1084,8 +1084,7 @@ Plan make_plan(int64_t B, int64_t D, int64_t N, int64_t L, int nsets, bool need_
   (void)nsets;
   pl.tile_bytes = align_up((size_t)B * D * 16 * 2 * 4, 256);      // state after the last whole tile
   pl.image_bytes = align_up(ema_image_bytes(D, N, bidirectional ? 1 : 0), 256);   // when the caller brings none
-  pl.rows_bytes = align_up(ema_rows_record_bytes(B, D, L, bidirectional ? 1 : 0), 256);   // block end states of the rows path
-  pl.total = pl.coef_bytes + pl.st_bytes + pl.acc_bytes + pl.tile_bytes + pl.image_bytes + pl.rows_bytes;
+  pl.total = pl.coef_bytes + pl.st_bytes + pl.acc_bytes + pl.tile_bytes + pl.image_bytes;
   return pl;
 }
 
@@ -1387,7 +1386,7 @@ extern "C" int mega_ema_fwd(const void* x, void* y, int dtype, int64_t sxb, int6
       img = wimg;
     }
     return ema_rows_run(x, y, dtype, sxb, sxd, syb, syd, img, is_complex, omega, mask, h_in, h_out, B, D, N, L,
-                        bidirectional, acc, (float*)(wimg + pl.image_bytes), s);
+                        bidirectional, s);
   }
   // rows too long for the rows kernel (more than 16 blocks of 1024 tokens) with fewer than 16 channel blocks: the
   // streaming kernel would run on that many workgroups, the time-parallel vector-ALU passes below are quicker

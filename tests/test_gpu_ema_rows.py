@@ -132,3 +132,21 @@ def test_kernel_generation_inside_the_call(dtype, B, D, layout):
     layer.image = saved
     torch.cuda.synchronize()
     assert torch.equal(y0, y1) and torch.equal(torch.view_as_real(h0), torch.view_as_real(h1))
+
+
+@pytest.mark.parametrize("bidir", [False, True])
+@pytest.mark.parametrize("B,D,L", [(3, 7, 64), (3, 7, 1024), (5, 3, 1025), (3, 5, 2048), (1, 5, 3000), (2, 3, 4096), (1, 3, 4100), (1, 1, 15363)])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_rows_of_every_number_of_blocks(dtype, B, D, L, bidir):
+    """One to fifteen blocks a row; several rows a workgroup, the last one with fewer; lengths in whole and partial blocks, in
+    tokens by four and one by one; padding at the end and inside; states of sixteen poles that reach across the row."""
+    rng = np.random.default_rng(L)
+    p, q, g = _coeffs(rng, 2 * D if bidir else D, 16, True)
+    om = rng.normal(size=D)
+    x, x64 = rounded(rng.normal(size=(B, D, L)), dtype)
+    mask = rng.random((B, L)) < 0.02
+    mask[0, L - L // 5:] = True
+    for m in (mask, None):
+        y, _ = _run(x, p, q, g, om, padding_mask=None if m is None else dev(m, torch.bool), bidirectional=bidir)
+        yo, _ = O.ema_forward(x64, p, q, g, om, m, bidirectional=bidir)
+        assert rel_err(host(y), yo) < TOL[dtype]
