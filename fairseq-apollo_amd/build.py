@@ -15,7 +15,7 @@ LIB = os.path.join(HERE, "libmega_hip.so")
 HOST = os.path.join(HERE, "mega_host.so")
 
 SOURCES = [
-    "gemm16_wide.hip", "gemm16_wide_f16.hip",      # (the longest first)
+    "gemm16_wide.hip", "gemm16_wide_f16.hip", "attention_wide.hip",      # (the longest first)
     "capi.hip",
     "timestep_norm.hip",
     "timestep_norm_bwd.hip",

@@ -19,9 +19,10 @@
 //   (rows of w that are not whole 16-byte pieces: transposed, zero-padded copies of w, dS, dy, q, k instead)
 //
 // The GEMM: (64 WM) x (64 WN) output tile per workgroup of WM x WN waves (64 x 64 each as 4 x 4 MFMA
-// blocks): 128 x 128 for the scores, 256 x 256 for the second product, which carries the flops.
+// blocks), 128 x 128; the long products of rows in whole 16-byte pieces: attention_wide.hip.
 // K step 64, operands staged through LDS as dense 128-byte rows with XOR-swizzled 16-byte pieces (no bank
 // conflicts), register prefetch of the next K step, all tiles of one batch entry on one XCD, epilogue through LDS.
+#include "attention_wide.h"
 #include "common.h"
 
 namespace mega {
@@ -382,6 +383,29 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_nt_kernel(const GemmArgs G)
     }
 }
 
+// the last element each operand is addressed at, from the kernels' own indexing: 16-byte pieces whose first
+// element passes the bounds test, rows below M / N, reduction steps below K; batch bz = bo nin + bi
+template <typename TIn, typename TOut, bool AT, bool BT, int EPI>
+void audit_gemm(const GemmArgs& G, int64_t batches) {
+  const int64_t bo = (batches - 1) / G.nin, bi = batches - 1 < G.nin ? batches - 1 : G.nin - 1;
+  auto pieces = [](int64_t n) { return (n - 1) / 8 * 8 + 8; };
+  const size_t a_el = AT ? (size_t)((G.K - 1) * G.lda + pieces(G.M)) : (size_t)((G.M - 1) * G.lda + pieces(G.K));
+  const size_t b_el = BT ? (size_t)((G.K - 1) * G.ldb + pieces(G.N)) : (size_t)((G.N - 1) * G.ldb + pieces(G.K));
+  const size_t c_el = (size_t)((G.M - 1) * G.ldc + G.N);
+  audit_use((const TIn*)G.A + bo * G.sa + bi * G.sai, a_el * sizeof(TIn), "gemm operand A");
+  audit_use((const TIn*)G.A, 1, "gemm operand A (first batch)");
+  audit_use((const TIn*)G.Bm + bo * G.sb + bi * G.sbi, b_el * sizeof(TIn), "gemm operand B");
+  audit_use((const TIn*)G.Bm, 1, "gemm operand B (first batch)");
+  if (EPI == 1) {
+    audit_use((TIn*)G.C + bo * G.sc + bi * G.sci, c_el * sizeof(TIn), "gemm result (softmax-backward epilogue)");
+    audit_use((const TIn*)G.E + bo * G.se + bi * G.sei, (size_t)((G.M - 1) * G.lde + G.N) * sizeof(TIn),
+              "gemm epilogue operand E");
+    audit_use(G.rowdot, (size_t)batches * G.M * 4, "gemm epilogue row sums");
+  } else {
+    audit_use((TOut*)G.C + bo * G.sc + bi * G.sci, c_el * sizeof(TOut), "gemm result");
+  }
+}
+
 template <typename TIn, typename TOut, int WM, int WN, bool AT = false, bool BT = false, int EPI = 0, int FM = 4,
           int FN = FM>
 void launch_gemm(GemmArgs G, int64_t M, int64_t N, int64_t batches, bool xcd, hipStream_t s) {
@@ -391,25 +415,7 @@ void launch_gemm(GemmArgs G, int64_t M, int64_t N, int64_t batches, bool xcd, hi
   static uint64_t attr_seen = 0;
   if (smem > 64 * 1024) raise_lds_limit(&attr_seen, smem, kern);
   if (audit_on()) {
-    // the last element each operand is addressed at, from the kernel's own indexing: 16-byte pieces whose first
-    // element passes the bounds test, rows below M / N, reduction steps below K; batch bz = bo nin + bi
-    const int64_t bo = (batches - 1) / G.nin, bi = batches - 1 < G.nin ? batches - 1 : G.nin - 1;
-    auto pieces = [](int64_t n) { return (n - 1) / 8 * 8 + 8; };
-    const size_t a_el = AT ? (size_t)((G.K - 1) * G.lda + pieces(G.M)) : (size_t)((G.M - 1) * G.lda + pieces(G.K));
-    const size_t b_el = BT ? (size_t)((G.K - 1) * G.ldb + pieces(G.N)) : (size_t)((G.N - 1) * G.ldb + pieces(G.K));
-    const size_t c_el = (size_t)((G.M - 1) * G.ldc + G.N);
-    audit_use((const TIn*)G.A + bo * G.sa + bi * G.sai, a_el * sizeof(TIn), "gemm operand A");
-    audit_use((const TIn*)G.A, 1, "gemm operand A (first batch)");
-    audit_use((const TIn*)G.Bm + bo * G.sb + bi * G.sbi, b_el * sizeof(TIn), "gemm operand B");
-    audit_use((const TIn*)G.Bm, 1, "gemm operand B (first batch)");
-    if (EPI == 1) {
-      audit_use((TIn*)G.C + bo * G.sc + bi * G.sci, c_el * sizeof(TIn), "gemm result (softmax-backward epilogue)");
-      audit_use((const TIn*)G.E + bo * G.se + bi * G.sei, (size_t)((G.M - 1) * G.lde + G.N) * sizeof(TIn),
-                "gemm epilogue operand E");
-      audit_use(G.rowdot, (size_t)batches * G.M * 4, "gemm epilogue row sums");
-    } else {
-      audit_use((TOut*)G.C + bo * G.sc + bi * G.sci, c_el * sizeof(TOut), "gemm result");
-    }
+    audit_gemm<TIn, TOut, AT, BT, EPI>(G, batches);
     return;
   }
   G.xcd = xcd ? 1 : 0;
@@ -418,6 +424,28 @@ void launch_gemm(GemmArgs G, int64_t M, int64_t N, int64_t batches, bool xcd, hi
   const dim3 grid3((unsigned)G.nt, (unsigned)G.mt, (unsigned)batches);
   const dim3 grid1((unsigned)((int64_t)G.nt * G.mt * batches));
   hipLaunchKernelGGL(kern, xcd ? grid1 : grid3, dim3(64 * WM * WN), smem, s, G);
+}
+
+// The same product on wide tiles; false: not within their limits, nothing is launched.  Rows, columns and reduction are whole
+// 16-byte pieces, on 16 bytes.
+template <typename T, AttnWide KIND>
+bool launch_wide(const GemmArgs& G, int64_t batches, hipStream_t s) {
+  AttnWideP P = {};
+  P.A = G.A; P.B = G.Bm; P.C = G.C;
+  P.lda = G.lda; P.ldb = G.ldb; P.ldc = G.ldc;
+  P.sa = G.sa; P.sb = G.sb; P.sc = G.sc; P.sai = G.sai; P.sbi = G.sbi; P.sci = G.sci;
+  P.nin = G.nin; P.batches = (int)batches; P.M = G.M; P.N = G.N; P.K = G.K;
+  P.E = G.E; P.rowdot = G.rowdot; P.lde = G.lde; P.se = G.se; P.sei = G.sei;
+  P.alpha = G.alpha;
+  P.causal = G.causal != 0;
+  if (!attention_wide_takes(P, KIND)) return false;
+  if (audit_on()) {
+    if (KIND == kScoreGrad) audit_gemm<T, float, false, false, 1>(G, batches);
+    else audit_gemm<T, T, KIND == kValueGrad, true, 0>(G, batches);
+    return true;
+  }
+  attention_wide_launch(P, KIND, __is_same(T, bf16_t), s);
+  return true;
 }
 
 // v [B][L][Nh][H2] -> vt [B][Nh][H2][Lp] (Lp = L rounded up to 8, zero padded).  64 x 64 tiles:
@@ -1150,11 +1178,14 @@ int run_attention(const void* q, const void* k, const void* v, void* y, void* w,
   G.lda = Lp; G.ldc = Nh * H2;
   G.sa = Nh * L * Lp; G.sai = L * Lp; G.sc = L * Nh * H2; G.sci = H2;
   G.M = (int)L; G.N = (int)H2; G.alpha = 1.0f; G.causal = causal ? 2 : 0;
-  // the second product carries the flops: 256 x 256 tiles when the problem has that many rows and columns
+  // the second product carries the flops: wide tiles when the problem has that many rows and columns
   if (v_inplace) {
     G.Bm = v; G.ldb = Nh * H2; G.sb = L * Nh * H2; G.sbi = H2; G.K = (int)L;
-    if (L >= 256 && H2 >= 256) launch_gemm<T, T, 4, 4, false, true>(G, L, H2, BN_, xcd, s);
-    else launch_gemm<T, T, 2, 2, false, true>(G, L, H2, BN_, xcd, s);
+    if (L >= 256 && H2 >= 256) {
+      if (L % 8 || ((uintptr_t)y % 16) || !launch_wide<T, kValues>(G, BN_, s)) launch_gemm<T, T, 4, 4, false, true>(G, L, H2, BN_, xcd, s);
+    } else {
+      launch_gemm<T, T, 2, 2, false, true>(G, L, H2, BN_, xcd, s);
+    }
   } else {
     G.Bm = Vt; G.ldb = Lp; G.sb = Nh * H2 * Lp; G.sbi = H2 * Lp; G.K = (int)Lp;
     if (L >= 256 && H2 >= 256) launch_gemm<T, T, 4, 4>(G, L, H2, BN_, xcd, s);
@@ -1249,8 +1280,7 @@ int run_attention_bwd(const void* dy, const void* q, const void* k, const void* 
                          rd, (int)L, (int)Nh, (int)H2, nrows);
     }
     G.C = dS; G.E = w; G.rowdot = rd; G.lde = L; G.se = Nh * L * L; G.sei = L * L; G.alpha = scale;
-    if (L >= 512) launch_gemm<T, float, 4, 4, false, false, 1>(G, L, L, BN_, xcd, s);
-    else launch_gemm<T, float, 2, 2, false, false, 1>(G, L, L, BN_, xcd, s);
+    if (L < 512 || !launch_wide<T, kScoreGrad>(G, BN_, s)) launch_gemm<T, float, 2, 2, false, false, 1>(G, L, L, BN_, xcd, s);
   } else if (L >= 512) {
     launch_gemm<T, float, 4, 4>(G, L, L, BN_, xcd, s);
   } else {
@@ -1279,8 +1309,7 @@ int run_attention_bwd(const void* dy, const void* q, const void* k, const void* 
     G.lda = L; G.ldb = Nh * H2; G.ldc = Nh * H2;
     G.sa = Nh * L * L; G.sai = L * L; G.sb = L * Nh * H2; G.sbi = H2; G.sc = L * Nh * H2; G.sci = H2;
     G.M = (int)L; G.N = (int)H2; G.K = (int)L; G.alpha = 1.0f; G.causal = causal ? 3 : 0;
-    if (L >= 256 && H2 >= 256) launch_gemm<T, T, 2, 4, true, true, 0, 8, 4>(G, L, H2, BN_, xcd, s);
-    else launch_gemm<T, T, 2, 2, true, true>(G, L, H2, BN_, xcd, s);
+    if (L < 256 || H2 < 256 || !launch_wide<T, kValueGrad>(G, BN_, s)) launch_gemm<T, T, 2, 2, true, true>(G, L, H2, BN_, xcd, s);
     // dq[b,:,n,:] = dS[b,n] k[b,:,n,:] (attention_kernel.cu:205-222): k K-major
     G.A = dS; G.Bm = k; G.C = dq;
     G.lda = Lp; G.ldb = Nh * H1; G.ldc = Nh * H1;

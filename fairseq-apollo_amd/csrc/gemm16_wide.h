@@ -363,101 +363,115 @@ __global__ __launch_bounds__(256, 1) void gemm16_square_kernel(const Gemm16P G) 
   finish_wave<T, true, TN>(G, at_tile, wm, wn, lane, acc);
 }
 
+// A 256 x 128 tile by eight waves.
 template <typename T, bool KA, bool KB, bool RAG>
-__global__ __launch_bounds__(512, 2) void gemm16_tall_kernel(const Gemm16P G) {
-  constexpr int TN = 128, ST = 3, kWT = 512;                       // columns of a tile, stages, threads
+struct Tall {
+  static constexpr int TN = 128, ST = 3, kWT = 512;                // columns of a tile, stages, threads
   using SA = Wide<kWideM, KA, kWT>;
   using SB = Wide<TN, KB, kWT>;
-  constexpr int WN = 2, FM = kWideM / 16 * WN / 8, FN = TN / 16 / WN, KK = kKS / 32;   // waves along N, a wave's blocks each way
-  constexpr int kStage = SA::Bytes + SB::Bytes, LD = SA::NP + SB::NP;
-  extern __shared__ __attribute__((aligned(16))) char lds[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const Place at_tile = place<TN>(G);
-  const int m0 = at_tile.m0, n0 = at_tile.n0, kb = at_tile.kb, ke = at_tile.ke;
-  const int steps = (ke - kb + kKS - 1) / kKS;
-  f32x4 acc[FM][FN];
+  static constexpr int WN = 2, FM = kWideM / 16 * WN / 8, FN = TN / 16 / WN, KK = kKS / 32;   // waves along N, a wave's blocks each way
+  static constexpr int kStage = SA::Bytes + SB::Bytes, LD = SA::NP + SB::NP;
+  static constexpr int kLds = ST * kStage;
+
+  // The sums of the tile whose first row / column start at ta / tb, over `len` indices; rooms: rows / columns to the end of
+  // the matrix.
+  static __device__ __forceinline__ void sums(char* lds, const char* ta, const char* tb, int64_t lda, int64_t ldb, int room_a,
+                                              int room_b, int len, int tid, int wm, int wn, f32x4 (&acc)[FM][FN]) {
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int steps = (len + kKS - 1) / kKS;
 #pragma unroll
-  for (int i = 0; i < FM; ++i)
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int wm = (wave / WN) * FM, wn = (wave % WN) * FN;
-  uint32_t oa[SA::NP], ob[SB::NP];
-  auto offsets = [&](const int left) {
+      for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    uint32_t oa[SA::NP], ob[SB::NP];
+    auto offsets = [&](const int left) {
 #pragma unroll
-    for (int h = 0; h < SA::NP; ++h) oa[h] = SA::offset(G.lda, tid, h, G.M - m0, left);
+      for (int h = 0; h < SA::NP; ++h) oa[h] = SA::offset(lda, tid, h, room_a, left);
 #pragma unroll
-    for (int h = 0; h < SB::NP; ++h) ob[h] = SB::offset(G.ldb, tid, h, G.N - n0, left);
-  };
-  offsets(kKS);
-  const char* ta = (const char*)G.A + (KA ? (int64_t)kb * G.lda + m0 : (int64_t)m0 * G.lda + kb) * 2;
-  const char* tb = (const char*)G.B + (KB ? (int64_t)kb * G.ldb + n0 : (int64_t)n0 * G.ldb + kb) * 2;
-  const int64_t da = (KA ? kKS * G.lda : kKS) * 2, db = (KB ? kKS * G.ldb : kKS) * 2;
-  const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds + wave * 1024;
-  int next = 0;                      // the step that is asked for next, and its stage
-  uint32_t stage = at;
-  auto issue = [&]() {
-    if (RAG && next == steps - 1) offsets(ke - kb - next * kKS);
+      for (int h = 0; h < SB::NP; ++h) ob[h] = SB::offset(ldb, tid, h, room_b, left);
+    };
+    offsets(kKS);
+    const int64_t da = (KA ? kKS * lda : kKS) * 2, db = (KB ? kKS * ldb : kKS) * 2;
+    const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds + wave * 1024;
+    int next = 0;                    // the step that is asked for next, and its stage
+    uint32_t stage = at;
+    auto issue = [&]() {
+      if (RAG && next == steps - 1) offsets(len - next * kKS);
 #pragma unroll
-    for (int h = 0; h < SA::NP; ++h) dma16(stage + h * (kWT * 16), oa[h], ta);
+      for (int h = 0; h < SA::NP; ++h) dma16(stage + h * (kWT * 16), oa[h], ta);
 #pragma unroll
-    for (int h = 0; h < SB::NP; ++h) dma16(stage + SA::Bytes + h * (kWT * 16), ob[h], tb);
-    ta += da;
-    tb += db;
-    ++next;
-    stage = stage == at + (ST - 1) * kStage ? at : stage + kStage;
-  };
-  typename SA::template Frags<FM> fa_at;
-  typename SB::template Frags<FN> fb_at;
-  fa_at.init(wm, lane);
-  fb_at.init(wn, lane);
+      for (int h = 0; h < SB::NP; ++h) dma16(stage + SA::Bytes + h * (kWT * 16), ob[h], tb);
+      ta += da;
+      tb += db;
+      ++next;
+      stage = stage == at + (ST - 1) * kStage ? at : stage + kStage;
+    };
+    typename SA::template Frags<FM> fa_at;
+    typename SB::template Frags<FN> fb_at;
+    fa_at.init(wm, lane);
+    fb_at.init(wn, lane);
 #pragma unroll
-  for (int s = 0; s < ST - 1; ++s)
-    if (s < steps) issue();
-  if (steps >= ST - 1) wait_loads<LD*(ST - 2)>();
-  else wait_loads<0>();
-  barrier();
-  // Two groups of four waves, one of each on every SIMD: while one reads its fragments the other multiplies.
-  if (wave >= 4) barrier();
-  const char* la = lds;
-  for (int s = 0; s < steps; ++s) {
-    __builtin_amdgcn_sched_barrier(0);
-    if (next < steps) issue();
-    uint4 fa[KK][FM], fb[KK][FN];
-#pragma unroll
-    for (int kk = 0; kk < KK; ++kk) {
-#pragma unroll
-      for (int j = 0; j < FN; ++j) fb[kk][j] = fb_at.get(la + SA::Bytes, j, kk);
-#pragma unroll
-      for (int i = 0; i < FM; ++i) fa[kk][i] = fa_at.get(la, i, kk);
-    }
-    la = la == lds + (ST - 1) * kStage ? lds : la + kStage;
-    if (s + ST - 1 < steps) wait_loads<LD*(ST - 2)>();            // the next step's stage has arrived
+    for (int s = 0; s < ST - 1; ++s)
+      if (s < steps) issue();
+    if (steps >= ST - 1) wait_loads<LD*(ST - 2)>();
     else wait_loads<0>();
     barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    if (RAG && s == steps - 1) {
-      const int left = ke - kb - s * kKS, g8 = (lane >> 4) * 8;
+    // Two groups of four waves, one of each on every SIMD: while one reads its fragments the other multiplies.
+    if (wave >= 4) barrier();
+    const char* la = lds;
+    for (int s = 0; s < steps; ++s) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (next < steps) issue();
+      uint4 fa[KK][FM], fb[KK][FN];
 #pragma unroll
       for (int kk = 0; kk < KK; ++kk) {
 #pragma unroll
-        for (int j = 0; j < FN; ++j) fb[kk][j] = keep(fb[kk][j], kk * 32 + g8, left);
+        for (int j = 0; j < FN; ++j) fb[kk][j] = fb_at.get(la + SA::Bytes, j, kk);
 #pragma unroll
-        for (int i = 0; i < FM; ++i) fa[kk][i] = keep(fa[kk][i], kk * 32 + g8, left);
+        for (int i = 0; i < FM; ++i) fa[kk][i] = fa_at.get(la, i, kk);
       }
+      la = la == lds + (ST - 1) * kStage ? lds : la + kStage;
+      if (s + ST - 1 < steps) wait_loads<LD*(ST - 2)>();          // the next step's stage has arrived
+      else wait_loads<0>();
+      barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      if (RAG && s == steps - 1) {
+        const int left = len - s * kKS, g8 = (lane >> 4) * 8;
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) {
+#pragma unroll
+          for (int j = 0; j < FN; ++j) fb[kk][j] = keep(fb[kk][j], kk * 32 + g8, left);
+#pragma unroll
+          for (int i = 0; i < FM; ++i) fa[kk][i] = keep(fa[kk][i], kk * 32 + g8, left);
+        }
+      }
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+          for (int i = 0; i < FM; ++i) acc[i][j] = mma16<T>(fb[kk][j], fa[kk][i], acc[i][j]);
+      __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_sched_barrier(0);
+      barrier();
     }
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int kk = 0; kk < KK; ++kk)
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int i = 0; i < FM; ++i) acc[i][j] = mma16<T>(fb[kk][j], fa[kk][i], acc[i][j]);
-    __builtin_amdgcn_s_setprio(0);
-    __builtin_amdgcn_sched_barrier(0);
-    barrier();
+    if (wave < 4) barrier();
   }
-  if (wave < 4) barrier();
-  finish_wave<T, false, TN>(G, at_tile, wm, wn, lane, acc);
+};
+
+template <typename T, bool KA, bool KB, bool RAG>
+__global__ __launch_bounds__(512, 2) void gemm16_tall_kernel(const Gemm16P G) {
+  using K = Tall<T, KA, KB, RAG>;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const Place p = place<K::TN>(G);
+  const int wm = (wave / K::WN) * K::FM, wn = (wave % K::WN) * K::FN;
+  const char* ta = (const char*)G.A + (KA ? (int64_t)p.kb * G.lda + p.m0 : (int64_t)p.m0 * G.lda + p.kb) * 2;
+  const char* tb = (const char*)G.B + (KB ? (int64_t)p.kb * G.ldb + p.n0 : (int64_t)p.n0 * G.ldb + p.kb) * 2;
+  f32x4 acc[K::FM][K::FN];
+  K::sums(lds, ta, tb, G.lda, G.ldb, G.M - p.m0, G.N - p.n0, p.ke - p.kb, tid, wm, wn, acc);
+  finish_wave<T, false, K::TN>(G, p, wm, wn, tid & 63, acc);
 }
 
 // the tiles behind the first G.full: the parts' sums added in order
@@ -490,7 +504,7 @@ void launch_wide(const Gemm16P& G, const WidePlan& p, hipStream_t s) {
     raise_lds_limit(&square_seen, smem, kern);
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), smem, s, G);
   } else {
-    constexpr int smem = 3 * (kWideM + 128) * kKS * 2;
+    constexpr int smem = Tall<T, KA, KB, RAG>::kLds;
     const auto kern = gemm16_tall_kernel<T, KA, KB, RAG>;
     raise_lds_limit(&tall_seen, smem, kern);
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(512), smem, s, G);

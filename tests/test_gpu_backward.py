@@ -612,6 +612,36 @@ def test_attention_bwd_entry_point(dtype, tol, B, L, Nh, H1, H2, causal):
             assert np.sqrt((e ** 2).mean()) < tol * rms and np.abs(e).max() < 4 * tol * max(rms, np.abs(ref).max()), tag
 
 
+@pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 2e-2), (torch.float16, 4e-3)])
+@pytest.mark.parametrize("B,L,Nh,H1,H2,causal", [
+    (1, 256, 1, 64, 256, True),      # one tile of values and of their gradient
+    (2, 264, 1, 16, 264, True),      # eight rows and columns beyond a tile, remainders of every reduction
+    (8, 512, 1, 32, 256, True),      # the first length of the score gradient's wide tiles; entries spread over the XCDs
+    (1, 632, 3, 8, 320, True),       # the last row of its tiles one short, three entries
+    (4, 1032, 2, 64, 392, True),     # a last row of tiles with eight rows
+    (1, 760, 2, 64, 328, False),     # whole products, edges both ways
+])
+def test_attention_wide_products(dtype, tol, B, L, Nh, H1, H2, causal):
+    """y = P v, dv and dS on wide tiles, against the fp64 oracle; gradients held as for the entry point above, the weights
+    and y to half a unit in the last place (eps / 2) for each rounding, of the weights and of the result."""
+    rng = np.random.default_rng(7000 + L)
+    q, q64 = rounded(rng.normal(size=(B, L, Nh, H1)) * 0.5, dtype)
+    k, k64 = rounded(rng.normal(size=(B, L, Nh, H1)) * 0.5, dtype)
+    v, v64 = rounded(rng.normal(size=(B, L, Nh, H2)), dtype)
+    dy, dy64 = rounded(rng.normal(size=(B, L, Nh, H2)), dtype)
+    scale = 1.0 / np.sqrt(H1)
+    y, w = M.ops.attention_fwd(q, k, v, scale, 0.0, causal, need_weights=True)
+    y64, w64 = O.attention(q64, k64, v64, scale, causal)
+    eps = torch.finfo(dtype).eps
+    assert np.linalg.norm(host(y) - y64) < eps * np.linalg.norm(y64)
+    assert np.linalg.norm(host(w) - w64) < eps / 2 * np.linalg.norm(w64)
+    got = M.ops.attention_bwd(dy, q, k, v, w, scale, causal, y=y)
+    for name, g, ref in zip("qkv", got, O.attention_bwd(dy64, q64, k64, v64, scale, causal)):
+        e = host(g) - ref
+        rms = np.sqrt((ref ** 2).mean())
+        assert np.sqrt((e ** 2).mean()) < tol * rms and np.abs(e).max() < 4 * tol * max(rms, np.abs(ref).max()), name
+
+
 def test_attention_bwd_entry_point_refuses_what_it_does_not_cover():
     """fp32 and head sizes that are not multiples of 8 take the batched library products in ops.attention_bwd; the
     entry point itself says so instead of computing something else."""
