@@ -1158,12 +1158,22 @@ int run_attention(const void* q, const void* k, const void* v, void* y, void* w,
   G.sa = L * Nh * H1; G.sai = H1; G.sb = L * Nh * H1; G.sbi = H1; G.sc = Nh * L * Lp; G.sci = L * Lp;
   G.nin = (int)Nh; G.M = (int)L; G.N = (int)L; G.K = (int)H1; G.alpha = scale; G.causal = causal ? 1 : 0; G.kshift = 0;
   const bool xcd = BN_ % 8 == 0;
-  launch_gemm<T, float, 2, 2>(G, L, L, BN_, xcd, s);
-  if (dropout > 0.f)
-    hipLaunchKernelGGL(dropkey_f32_kernel, dim3((unsigned)ceil_div(BN_ * L, 4)), dim3(256), 0, s, S, (int)L, (int)L, Lp,
-                       causal, dropout, seed, (int64_t)(BN_ * L));
-  hipLaunchKernelGGL(softmax_f32_kernel<T>, dim3((unsigned)ceil_div(BN_ * L, 4)), dim3(256), 0, s, S, P, (int)L, (int)L,
-                     Lp, Lp, (int)Lp, causal, w ? 1 : 0, (int64_t)(BN_ * L));
+  AttnWeightsP W = {};
+  W.q = q; W.k = k; W.P = P;
+  W.L = (int)L; W.Nh = (int)Nh; W.H1 = (int)H1; W.batches = (int)BN_;
+  W.scale_log2 = scale * 1.4426950408889634f;
+  W.causal = causal ? 1 : 0;
+  W.zero_all = w ? 1 : 0;
+  if (dropout <= 0.f && attention_weights_takes(W)) {
+    attention_weights_launch(W, __is_same(T, bf16_t), s);
+  } else {
+    launch_gemm<T, float, 2, 2>(G, L, L, BN_, xcd, s);
+    if (dropout > 0.f)
+      hipLaunchKernelGGL(dropkey_f32_kernel, dim3((unsigned)ceil_div(BN_ * L, 4)), dim3(256), 0, s, S, (int)L, (int)L, Lp,
+                         causal, dropout, seed, (int64_t)(BN_ * L));
+    hipLaunchKernelGGL(softmax_f32_kernel<T>, dim3((unsigned)ceil_div(BN_ * L, 4)), dim3(256), 0, s, S, P, (int)L, (int)L,
+                       Lp, Lp, (int)Lp, causal, w ? 1 : 0, (int64_t)(BN_ * L));
+  }
   if (w && (void*)P != w) {
     // the weights the reference returns: [B, Nh, L, L]
     hipMemcpy2DAsync(w, (size_t)L * sizeof(T), P, (size_t)Lp * sizeof(T), (size_t)L * sizeof(T), (size_t)(BN_ * L),

@@ -32,4 +32,17 @@ enum AttnWide { kScoreGrad, kValues, kValueGrad };
 bool attention_wide_takes(const AttnWideP& P, AttnWide kind);
 void attention_wide_launch(AttnWideP P, AttnWide kind, bool bf16, hipStream_t s);
 
+// The weights themselves: P [batches][L][L] = softmax(scale q k^T) over the visible keys, zeros behind them (causal): to the
+// end of the row, or of the 256 columns that hold the diagonal
+struct AttnWeightsP {
+  const void *q, *k;   // [B][L][Nh][H1]
+  void* P;
+  int L, Nh, H1, batches;
+  float scale_log2;    // scale log2(e)
+  int causal, zero_all;
+  int xcd, qt;         // tiles of queries
+};
+bool attention_weights_takes(const AttnWeightsP& A);
+void attention_weights_launch(AttnWeightsP A, bool bf16, hipStream_t s);
+
 }  // namespace mega

@@ -1,4 +1,4 @@
-// 16-bit attention with its weights in memory: the long products y = P v, dv = w^T dy, and dS, whose
+// 16-bit attention with its weights in memory: the weights (below), and the long products y = P v, dv = w^T dy, and dS, whose
 // epilogue is the softmax's backward (fairseq/csrc/ops/attention_kernel.cu:40-131, 155-203).  The products: tall tiles of gemm16_wide.h (256 x 128, memory straight to
 // LDS, two groups of waves in turn), one product per (row, head).
 //
@@ -136,6 +136,184 @@ int64_t entry_tiles(const AttnWideP& P, AttnWide kind) {
   return mt * (mt + 1) - (nt < 2 * mt ? 1 : 0);
 }
 
+// ---- the weights, without the fp32 scores in memory.
+//
+// A workgroup owns 64 queries of a batch entry, in registers as the matrix instruction's columns; its waves take tiles of 64 keys
+// in turn, fragments straight from memory (k fits an L2).  Scores are formed twice: for the rows' maxima and
+// sums, which the waves exchange once through LDS, and for the weights.  Both are 32-bit throughout, as they were between the
+// three passes over the scores.  What bounds it is a wave's turn (fragments on their way, products, exponentials one after the
+// other) and the writing: 16 x 2048 x 2048 in bf16, 134 MB, 49 us (85 as product and softmax).
+constexpr int kQBlocks = 4;
+template <typename T, int KS>
+__global__ __launch_bounds__(256, 2) void attn_weights_kernel(const AttnWeightsP A) {
+  constexpr int FQ = kQBlocks, KB = 4, NW = 4, BQ = 16 * FQ, BK = 16 * KB;   // blocks of queries, of keys; waves
+  __shared__ float2 stat[NW][BQ];
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // longest rows first, the shortest of them last beside them: two workgroups of a compute unit have about the same keys
+  const int x = A.xcd ? (int)blockIdx.x & 7 : 0, id = A.xcd ? (int)blockIdx.x >> 3 : (int)blockIdx.x;
+  const int here = A.xcd ? A.batches >> 3 : A.batches, total = here * A.qt, half = (total + 1) >> 1;
+  const int o = id < half ? id : total - 1 - (id - half);
+  const int z = (o % here) * (A.xcd ? 8 : 1) + x, q0 = (A.qt - 1 - o / here) * BQ;
+  const int b = z / A.Nh, h = z - b * A.Nh;
+  const int64_t rs = (int64_t)A.Nh * A.H1, base = (int64_t)b * A.L * rs + (int64_t)h * A.H1;
+  const T* const Q = (const T*)A.q + base;
+  const T* const Kp = (const T*)A.k + base;
+  T* const P = (T*)A.P + (int64_t)z * A.L * A.L;
+  uint4 fq[FQ][KS];
+#pragma unroll
+  for (int j = 0; j < FQ; ++j)
+#pragma unroll
+    for (int s = 0; s < KS; ++s) fq[j][s] = *(const uint4*)(Q + min(q0 + 16 * j + n, A.L - 1) * rs + s * 32 + g * 8);
+  const int seen = A.causal ? min(A.L, q0 + BQ) : A.L;             // keys that any of the rows sees
+  const int tiles = (seen + BK - 1) / BK;
+  // scores (times log2 e) of the tile of keys from k0 on: key k0 + 16 kb + 4 g + u of query q0 + 16 j + n; invisible: -inf
+  auto scores = [&](const int k0, f32x4 (&S)[KB][FQ]) {
+    uint4 fk[KB][KS];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int s = 0; s < KS; ++s) fk[kb][s] = *(const uint4*)(Kp + min(k0 + 16 * kb + n, A.L - 1) * rs + s * 32 + g * 8);
+    __builtin_amdgcn_sched_barrier(0);                             // (all in flight together)
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int j = 0; j < FQ; ++j) {
+        S[kb][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < KS; ++s) S[kb][j] = mma16<T>(fk[kb][s], fq[j][s], S[kb][j]);
+      }
+    const bool edge = k0 + BK > A.L || (A.causal && k0 + BK - 1 > q0);
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int j = 0; j < FQ; ++j)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) S[kb][j][u] *= A.scale_log2;
+    if (edge) {
+#pragma unroll
+      for (int j = 0; j < FQ; ++j) {
+        const int last = A.causal ? min(q0 + 16 * j + n, A.L - 1) : A.L - 1;
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) S[kb][j][u] = k0 + 16 * kb + 4 * g + u <= last ? S[kb][j][u] : -INFINITY;
+      }
+    }
+  };
+  float mx[FQ], sum[FQ];
+#pragma unroll
+  for (int j = 0; j < FQ; ++j) {
+    mx[j] = -INFINITY;
+    sum[j] = 0.f;
+  }
+  // two parts of a row: (m, l) takes (m2, l2) in
+  auto join = [](float& m, float& l, float m2, float l2) {
+    const float both = fmaxf(m, m2), from = both == -INFINITY ? 0.f : both;
+    l = l * __builtin_amdgcn_exp2f(m - from) + l2 * __builtin_amdgcn_exp2f(m2 - from);
+    m = both;
+  };
+  f32x4 S[KB][FQ];
+  int t = wave;
+  for (; t < tiles; t += NW) {
+    scores(t * BK, S);
+#pragma unroll
+    for (int j = 0; j < FQ; ++j) {
+      float m = mx[j];
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) m = fmaxf(m, S[kb][j][u]);
+      const float from = m == -INFINITY ? 0.f : m;
+      float l = 0.f;
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) l += __builtin_amdgcn_exp2f(S[kb][j][u] - from);
+      sum[j] = sum[j] * __builtin_amdgcn_exp2f(mx[j] - from) + l;
+      mx[j] = m;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < FQ; ++j) {
+#pragma unroll
+    for (int d = 16; d <= 32; d <<= 1) {
+      const float m2 = __shfl_xor(mx[j], d), l2 = __shfl_xor(sum[j], d);
+      join(mx[j], sum[j], m2, l2);
+    }
+    if (g == 0) stat[wave][16 * j + n] = make_float2(mx[j], sum[j]);
+  }
+  __syncthreads();
+  float from[FQ], inv[FQ];
+  bool odd = false;                                     // a row of zeros or of NaN
+#pragma unroll
+  for (int j = 0; j < FQ; ++j) {
+    float m = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float2 v = stat[w][16 * j + n];
+      join(m, l, v.x, v.y);
+    }
+    // nothing visible, or beyond 32 bits: zeros (a NaN among visible scores makes the row NaN)
+    const bool dead = m == -INFINITY || m == INFINITY || l == 0.f;
+    from[j] = dead ? INFINITY : m;
+    inv[j] = dead ? 0.f : 1.0f / l;
+    odd = odd || dead || !(l == l);
+  }
+  odd = __any(odd);
+  const int width = A.causal && !A.zero_all ? min(A.L, (q0 + BQ + 255) / 256 * 256) : A.L, all = (width + BK - 1) / BK;
+  const int eighth = (g & 1) * 16 + (g >> 1) * 8;
+  T* const row0 = P + (int64_t)(q0 + n) * A.L + eighth;
+  for (int f = t; f < all; f += NW) {
+#pragma unroll
+    for (int j = 0; j < FQ; ++j)
+#pragma unroll
+      for (int kb = 0; kb < KB; kb += 2) {
+        const int c = f * BK + 16 * kb;
+        if (q0 + 16 * j + n < A.L && c + eighth < width) *(uint4*)(row0 + 16 * j * (int64_t)A.L + c) = make_uint4(0, 0, 0, 0);
+      }
+  }
+  // the last tile's scores are still there
+  for (t -= NW; t >= 0;) {
+#pragma unroll
+    for (int j = 0; j < FQ; ++j) {
+      const int r = q0 + 16 * j + n;
+#pragma unroll
+      for (int kb = 0; kb < KB; kb += 2) {
+        const int c = t * BK + 16 * kb;
+        uint32_t p[4];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          float v[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) v[u] = __builtin_amdgcn_exp2f(S[kb + e][j][u] - from[j]) * inv[j];
+          if (odd) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+              if (from[j] == INFINITY || (A.causal && c + 16 * e + 4 * g + u > r)) v[u] = 0.f;
+          }
+          p[2 * e] = pack16<T>(v[0], v[1]);
+          p[2 * e + 1] = pack16<T>(v[2], v[3]);
+        }
+        const uint4 w = eight(p);
+        if (r < A.L && c + eighth < width) *(uint4*)(row0 + 16 * j * (int64_t)A.L + c) = w;
+      }
+    }
+    t -= NW;
+    if (t >= 0) scores(t * BK, S);
+  }
+}
+
+template <typename T, int KS>
+void launch_weights(AttnWeightsP A, hipStream_t s) {
+  A.qt = (int)ceil_div(A.L, 16 * kQBlocks);
+  hipLaunchKernelGGL((attn_weights_kernel<T, KS>), dim3((unsigned)((int64_t)A.batches * A.qt)), dim3(256), 0, s, A);
+}
+template <typename T>
+void launch_weights_type(const AttnWeightsP& A, hipStream_t s) {
+  if (A.H1 == 64) launch_weights<T, 2>(A, s);
+  else launch_weights<T, 4>(A, s);
+}
+
 }  // namespace
 
 bool attention_wide_takes(const AttnWideP& P, AttnWide kind) {
@@ -150,6 +328,25 @@ void attention_wide_launch(AttnWideP P, AttnWide kind, bool bf16, hipStream_t s)
   P.xcd = P.batches % 8 == 0;
   if (bf16) launch_kind<bf16_t>(P, kind, s);
   else launch_kind<f16_t>(P, kind, s);
+}
+
+// Rows of at most 256 keys, which a workgroup's waves take in one turn, and products that give every compute unit a workgroup:
+// fewer workgroups with longer rows are a chain of turns (2.7 us each with one wave on a SIMD), where the scores' own
+// product has more tiles.  us, product and softmax beside this kernel, entries x positions x width (causal, full):
+//      1 x  256 x 128     9.1, 8.9     9.0, 8.8       16 x 1024 x  64    33.8, 20.7    40.9, 21.3
+//      8 x  256 x  64     9.4, 7.5     9.6, 7.2       16 x 2048 x 128    85.4, 49.4     159, 71.9
+//      1 x  512 x 128     9.6, 14.2 (not)              4 x 2048 x 128    30.5, 39.5    39.8, 40.4 (not)
+//      8 x 1024 x 128    24.4, 25.2 (not)              2 x 4096 x 128    99.7, 68.9     156, 71.5 (missed)
+// Width 256: fragments from memory for half as many queries; 8 x 1024 x 256 24.5, 31.3 (not).
+bool attention_weights_takes(const AttnWeightsP& A) {
+  return (A.H1 == 64 || A.H1 == 128) && A.L % 8 == 0 && ((uintptr_t)A.P % 16) == 0 && (int64_t)A.batches * A.L < (int64_t)1 << 31 &&
+         (A.L <= 256 || A.batches * ceil_div(A.L, 64) >= device_cu_count());
+}
+
+void attention_weights_launch(AttnWeightsP A, bool bf16, hipStream_t s) {
+  A.xcd = A.batches % 8 == 0;
+  if (bf16) launch_weights_type<bf16_t>(A, s);
+  else launch_weights_type<f16_t>(A, s);
 }
 
 }  // namespace mega

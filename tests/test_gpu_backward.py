@@ -642,6 +642,38 @@ def test_attention_wide_products(dtype, tol, B, L, Nh, H1, H2, causal):
         assert np.sqrt((e ** 2).mean()) < tol * rms and np.abs(e).max() < 4 * tol * max(rms, np.abs(ref).max()), name
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,L,Nh,H1,causal", [
+    (1, 8, 1, 64, True), (3, 64, 1, 128, True), (1, 72, 2, 64, True), (1, 256, 1, 128, True), (8, 1032, 2, 64, True),
+    (17, 1024, 1, 128, True), (1, 200, 2, 64, False), (32, 520, 1, 128, False),
+])
+def test_attention_weights_in_one_pass(dtype, B, L, Nh, H1, causal):
+    """The weights straight from q and k, at the edges of its tiles of queries and keys: every one within a rounding (eps / 2) and
+    the 32-bit sums' and exponentials' 1e-5 of the fp64 oracle (fp16: and half the smallest step, 2^-25), zeros behind the
+    diagonal.  A query that is not a number leaves its row without a maximum: zeros, and no other row changes; a key that is
+    not makes the rows that see it NaN up to the diagonal."""
+    rng = np.random.default_rng(7100 + L)
+    q, q64 = rounded(rng.normal(size=(B, L, Nh, H1)), dtype)
+    k, k64 = rounded(rng.normal(size=(B, L, Nh, H1)), dtype)
+    v = torch.zeros(B, L, Nh, 8, dtype=dtype, device="cuda:0")
+    scale = -1.5 / np.sqrt(H1)
+    _, w = M.ops.attention_fwd(q, k, v, scale, 0.0, causal, need_weights=True)
+    _, want = O.attention(q64, k64, host(v), scale, causal)
+    close = (torch.finfo(dtype).eps / 2 + 1e-5) * np.abs(want) + 2.0 ** -25
+    assert (np.abs(host(w) - want) <= close).all()
+    bad = L // 2
+    q[0, bad, 0] = float("nan")
+    _, w2 = M.ops.attention_fwd(q, k, v, scale, 0.0, causal, need_weights=True)
+    assert not bool(w2[0, 0, bad].any())
+    seen = bad + 1 if causal else L
+    w2[0, 0, bad] = w[0, 0, bad]
+    assert torch.equal(w, w2)
+    q[0, bad, 0] = 1.0
+    k[0, min(3, L - 1), 0] = float("nan")
+    _, w3 = M.ops.attention_fwd(q, k, v, scale, 0.0, causal, need_weights=True)
+    assert bool(torch.isnan(w3[0, 0, bad, :seen]).all()) and not bool(w3[0, 0, bad, seen:].any())
+
+
 def test_attention_bwd_entry_point_refuses_what_it_does_not_cover():
     """fp32 and head sizes that are not multiples of 8 take the batched library products in ops.attention_bwd; the
     entry point itself says so instead of computing something else."""
