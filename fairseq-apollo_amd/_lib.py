@@ -71,6 +71,8 @@ SIGNATURES = {
     "mega_gemm16_pays": (_int, [_i64, _i64, _i64, _int, _int]),
     "mega_gemm16_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "mega_gemm16": (_int, [_p, _int, _p, _sz, _p]),
+    "mega_embedding_grad_workspace_bytes": (_sz, [_i64, _i64, _i64]),
+    "mega_embedding_grad": (_int, [_p, _p, _p, _int, _i64, _i64, _i64, _i64, _p, _sz, _p]),
     "mega_gemm_f32_pays": (_int, [_i64, _i64, _i64, _int, _int]),
     "mega_gemm_f32_batched_pays": (_int, [_i64, _i64, _i64, _i64, _i64, _int, _int]),
     "mega_gemm_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64]),

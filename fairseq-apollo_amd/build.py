@@ -30,6 +30,7 @@ SOURCES = [
     "elementwise.hip",
     "gemm.hip", "gemm16.hip",
     "gate_glue.hip",
+    "embed_grad.hip",
     "row_norm.hip",
     "attention.hip",
     "attention_mfma.hip",

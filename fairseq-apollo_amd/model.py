@@ -16,7 +16,7 @@ from torch import Tensor, nn
 
 from . import ops
 from .layers import MegaDecoderLayer, MovingAverageGatedAttention, _arg
-from .modules import MultiHeadComplexEMA, MultiHeadEMA, TimestepNorm, _plain, _unhooked, project
+from .modules import MultiHeadComplexEMA, MultiHeadEMA, TimestepNorm, _plain, _unhooked, embed, project
 
 # a decoder layer and what in it receives the padding mask
 _MASK_READERS = (MegaDecoderLayer, MovingAverageGatedAttention, TimestepNorm, MultiHeadEMA, MultiHeadComplexEMA)
@@ -97,7 +97,7 @@ class MegaDecoderNoCrossAttn(nn.Module):
         if seq_len > self.chunk_size > 0 and seq_len % self.chunk_size != 0:
             num_paddings = math.ceil(seq_len / self.chunk_size) * self.chunk_size - seq_len
             prev_output_tokens = F.pad(prev_output_tokens, (0, num_paddings), value=self.padding_idx)
-        x = self.embed_tokens(prev_output_tokens)
+        x = embed(self.embed_tokens, prev_output_tokens)
         if self.embed_scale is not None:
             x = self.embed_scale * x
         decoder_padding_mask = prev_output_tokens.eq(self.padding_idx) if self.padding_idx is not None else None

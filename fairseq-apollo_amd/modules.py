@@ -1374,6 +1374,41 @@ class EfficientAttention(nn.Module):
         return 'causal={}, dropout={}'.format(self._causal, self._dropout)
 
 
+class EmbeddingFunc(torch.autograd.Function):
+    """F.embedding; the table's gradient by the library's kernel, where torch sorts the ids (19 launches)."""
+
+    @staticmethod
+    def forward(ctx, ids, weight, padding_idx):
+        ctx.save_for_backward(ids)
+        ctx.rows, ctx.padding_idx = weight.shape[0], padding_idx
+        return F.embedding(ids, weight, padding_idx)
+
+    @staticmethod
+    def backward(ctx, y_grad):
+        if not ctx.needs_input_grad[1]:
+            return None, None, None
+        ids, = ctx.saved_tensors
+        got = None
+        if not torch.is_grad_enabled():
+            got = ops.embedding_grad(y_grad, ids, ctx.rows, ctx.padding_idx)
+        if got is None:                                # a graph over it is asked for (create_graph), or many rows
+            pad = -1 if ctx.padding_idx is None else ctx.padding_idx
+            got = torch.ops.aten.embedding_dense_backward(y_grad, ids, ctx.rows, pad, False)
+        return None, got, None
+
+
+def embed(table: nn.Embedding, ids: Tensor) -> Tensor:
+    """table(ids)."""
+    if ids.is_cuda and ids.dtype is torch.int64 and ids.numel() and type(table) is nn.Embedding:
+        w = table._parameters.get('weight')
+        if (w is not None and w.dim() == 2 and 0 < w.shape[0] <= EMBED_ROWS and table.max_norm is None
+                and not table.scale_grad_by_freq and not table.sparse and one_graph(w) and ids.device == w.device
+                and w.is_contiguous() and _unhooked((nn.Embedding,), table)):
+            return EmbeddingFunc.apply(ids, w, table.padding_idx)
+    return table(ids)
+
+
+EMBED_ROWS = 318                  # mega_embedding_grad's limit: larger tables keep torch's operation
 OWN_16BIT_FLOPS = 1e13            # mega_gemm16_pays of products along the rows: no native call is made to be told no
 
 

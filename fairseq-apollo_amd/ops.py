@@ -1472,6 +1472,26 @@ def colsum(x: torch.Tensor, out_dtype: Optional[torch.dtype] = None) -> torch.Te
     return out
 
 
+def embedding_grad(y_grad: torch.Tensor, ids: torch.Tensor, rows: int, padding_idx: Optional[int]) -> Optional[torch.Tensor]:
+    """Gradient of an embedding table [rows, D] from the looked-up vectors' [..., D], or None where the kernel does not take
+    it: more rows than the LDS holds."""
+    dev = _need_gpu(y_grad, ids)
+    lib = _lib.load()
+    g, idx = y_grad.detach().contiguous(), ids.detach().contiguous()
+    D = g.shape[-1]
+    need = lib.mega_embedding_grad_workspace_bytes(idx.numel(), rows, D)
+    if not need or idx.dtype is not torch.int64 or g.numel() != idx.numel() * D:
+        return None
+    out = torch.empty(rows, D, dtype=g.dtype, device=dev)
+    stream = _stream(dev)
+    ws = _scratch_buffer(dev, need, stream)
+    with _on_device(dev):
+        rc = lib.mega_embedding_grad(_ptr(idx), _ptr(g), _ptr(out), _dtype_code(g), idx.numel(), rows, D,
+                                     -1 if padding_idx is None else padding_idx, _ptr(ws), ws.numel(), stream)
+    _lib.check(rc, "embedding_grad")
+    return out
+
+
 # ------------------------------------------------------------------------------------------------
 # per-token glue of the gated-attention layer (rows of a wider projection output are passed in
 # place: every input carries its own row stride)

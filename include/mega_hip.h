@@ -441,6 +441,13 @@ int mega_gemm16_pays(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor
 size_t mega_gemm16_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int mega_gemm16(const MegaGemm* g, int dtype, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Gradient of an embedding table of at most 318 rows (csrc/embed_grad.hip): dw[v, :] = sum of dy[t, :] over ids[t] == v, zeros at
+ * padding_id (none: negative); ids outside the table are passed over.  dy and dw of `dtype`, sums fp32 in the order of the
+ * tokens.  workspace_bytes 0: not covered.                                                                            */
+size_t mega_embedding_grad_workspace_bytes(int64_t T, int64_t V, int64_t D);
+int mega_embedding_grad(const int64_t* ids, const void* dy, void* dw, int dtype, int64_t T, int64_t V, int64_t D, int64_t padding_id,
+                        void* workspace, size_t workspace_bytes, void* stream);
+
 /* 1 when calls of these sizes run as one kernel (carried: 1 with h_in, 2 with h_out, 3 with both; rows_out: y as [B,D,L]
  * rows), else 0 */
 int mega_norm_ema_fwd_one_kernel(int dtype, int64_t B, int64_t L, int64_t D, int64_t G, int64_t N, int carried,

@@ -476,3 +476,51 @@ def test_softmax_zeros_beyond_a_row_with_nan(dtype, n):
     want = x[0, 0].double().masked_fill(mask[0].bool(), float("-inf")).softmax(-1)
     # half a unit in the last place of the type, and expf's few of fp32
     assert ((buf[0, :, :n].double() - want).norm() / want.norm()).item() < {torch.float32: 1e-6, torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12}[dtype] * 1.01
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,V,D,pad", [(1, 1, 1, None), (15, 3, 63, 0), (16, 264, 64, 1), (65, 7, 65, None), (4099, 318, 96, 317),
+                                       (8192, 264, 1024, 1)])
+def test_embedding_grad(dtype, T, V, D, pad):
+    """The table's gradient against 64-bit sums: every element within its rounding (eps / 2, fp32: none) and, per addend,
+    2^-24 of the sum of magnitudes (fp32 sums in any order: T 2^-24 at most); equal ids next to each other, ids that do not
+    occur, the padding row, and a value that is not a number, which stays in its row."""
+    gen = torch.Generator().manual_seed(T)
+    ids = torch.randint(0, V, (T,), generator=gen)
+    ids[T // 3:T // 2] = V // 2
+    dy = torch.randn(T, D, generator=gen).to(dtype)
+    got = M.ops.embedding_grad(dy.cuda(), ids.cuda(), V, pad).cpu()
+    want = torch.zeros(V, D, dtype=torch.float64).index_add_(0, ids, dy.double())
+    size = torch.zeros(V, D, dtype=torch.float64).index_add_(0, ids, dy.double().abs())
+    if pad is not None:
+        want[pad] = 0
+    round_off = 0.0 if dtype is torch.float32 else torch.finfo(dtype).eps / 2
+    count = torch.zeros(V, dtype=torch.float64).index_add_(0, ids, torch.ones(T, dtype=torch.float64))[:, None]
+    bound = round_off * want.abs() + 1.01 * (count + 40) * 2.0 ** -24 * size + 2.0 ** -25 * (dtype is torch.float16)
+    assert got.dtype == dtype and bool(((got.double() - want).abs() <= bound).all())
+    dy[T - 1, D - 1] = float("nan")
+    got2 = M.ops.embedding_grad(dy.cuda(), ids.cuda(), V, pad).cpu()
+    row = int(ids[T - 1])
+    assert row == pad or bool(torch.isnan(got2[row, D - 1]))
+    got2[row, D - 1] = got[row, D - 1]
+    assert torch.equal(got, got2)
+
+
+def test_embedding_in_a_graph_of_its_own():
+    """M.modules.embed against torch's embedding: values, gradient, the gradient of the gradient, and what it leaves to torch."""
+    table = torch.nn.Embedding(40, 32, padding_idx=2).cuda()
+    ids = torch.randint(0, 40, (3, 17), device="cuda:0")
+    g = torch.randn(3, 17, 32, device="cuda:0", requires_grad=True)
+    a, b = M.modules.embed(table, ids), table(ids)
+    assert a.grad_fn.name() != b.grad_fn.name() and torch.equal(a, b)
+    ga, = torch.autograd.grad(a, table.weight, g, create_graph=True)
+    gb, = torch.autograd.grad(b, table.weight, g, create_graph=True)
+    assert torch.allclose(ga, gb, rtol=1e-5, atol=1e-6)
+    assert torch.equal(torch.autograd.grad((ga ** 2).sum(), g)[0], torch.autograd.grad((gb ** 2).sum(), g)[0])
+    a.backward(g.detach(), retain_graph=True)
+    assert torch.allclose(table.weight.grad, gb, rtol=1e-5, atol=1e-6) and not bool(table.weight.grad[2].any())
+    with torch.no_grad():
+        assert M.modules.embed(table, ids).grad_fn is None
+    for other in (torch.nn.Embedding(319, 8).cuda(), torch.nn.Embedding(40, 8, max_norm=1.0).cuda(), torch.nn.Embedding(40, 8, sparse=True).cuda(),
+                  torch.nn.Embedding(40, 8, scale_grad_by_freq=True).cuda()):
+        assert M.modules.embed(other, ids).grad_fn.name() == b.grad_fn.name()
