@@ -559,7 +559,7 @@ Result ema_param_backward(const Args& A) {
 }
 
 // ---- training: the layer around its norm, moving average and attention, forwards and backwards in few calls.  The
-// products of 16-bit activations are library GEMMs beyond some size; the others and what lies between them run in libmega_hip.
+// products (but the largest of 16-bit types, and fp32 ones by size) and what lies between them run in libmega_hip.
 // Activations and weights share one type.
 Tensor rows2(const Tensor& t) { return t.reshape({-1, t.size(-1)}); }
 

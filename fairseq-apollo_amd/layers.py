@@ -4,9 +4,9 @@ restricted to the rotary softmax attention through the fused ops (causal with Ti
 one-sided EMA / CEMA, or bidirectional with SequenceNorm and a two-sided one), plus the north-star
 SwiGLU FFN.
 
-The projections are library GEMMs (torch -> hipBLASLt); normalisation, moving average,
+The projections are libmega_hip.so's own products by size and type (torch -> hipBLASLt otherwise); normalisation, moving average,
 attention and the SwiGLU gate run in libmega_hip.so.  Under autograd the normalisation, the
-moving average and the attention (softmax backward in libmega_hip.so, batched library GEMMs) keep
+moving average and the attention (by size and type with its products in libmega_hip.so, else batched library GEMMs) keep
 their own backward operators, and so do the r gate, the output gate and the SwiGLU gate; the
 remaining element-wise steps (q / k map, activations of v and of the moving average) run as torch
 operations so that the graph is complete.
@@ -82,7 +82,7 @@ class NormalizedFeedForwardNetwork(nn.Module):
     """The reference's position-wise block, `x + fc2(silu(fc1(norm(x))))` with an optional
     per-feature layer scale (fairseq/modules/normalized_feedforward_network.py:13-93; same
     constructor arguments, parameter names and initialisation; the two dropouts act in training
-    mode only).  The two projections are library GEMMs; norm and activation are elementwise glue."""
+    mode only).  The two projections are products (above); norm and activation are elementwise glue."""
 
     def __init__(self, embed_dim, ffn_hidden_dim, dropout=0.0, hidden_dropout=0.0, norm_type='layernorm',
                  norm_affine=True, norm_eps=1e-5, layer_scale=None, init_mode='bert', export=False):

@@ -1458,7 +1458,7 @@ def linear_residual(lin: nn.Linear, h: Tensor, residual: Optional[Tensor], consu
 
 class SwiGLU(nn.Module):
     """W2 (silu(W1 x) * W3 x) with the gate evaluated by the HIP kernel; the three
-    projections are library GEMMs."""
+    projections are the library's own products by size and type, a GEMM library's otherwise."""
 
     def __init__(self, embed_dim: int, hidden_dim: int, bias: bool = False) -> None:
         super().__init__()
