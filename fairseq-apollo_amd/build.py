@@ -6,8 +6,11 @@ Run as a script (`python fairseq-apollo_amd/build.py`) or through
 from __future__ import annotations
 
 import os
+import re
+import shutil
 import subprocess
 import sys
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -58,6 +61,87 @@ def hipcc() -> str:
     raise RuntimeError("hipcc not found")
 
 
+def operand_faults(name: str, listing: list) -> list:
+    """What a kernel whose matrix instructions are written as inline assembly must not hold, in its disassembly (lines of
+    llvm-objdump): the compiler pads the matrix instructions it knows with wait states, these it moves values around
+    unpadded.  Two wait states belong between a vector instruction and a matrix instruction that shares a register with it, 19
+    between a matrix instruction and any other use of its result; no registers in scratch memory (fragments would come back
+    through copies); M0 written before a load to LDS and used for nothing else."""
+    code, at = [], {}
+    for line in listing:
+        m = re.match(r"\s+(\S+)\s*(.*?)\s*// ([0-9A-F]+):(.*)", line)
+        if m:
+            at[int(m[3], 16)] = len(code)
+            jump = re.search(r"\+0x([0-9a-f]+)>", m[4]) if m[1].startswith(("s_branch", "s_cbranch")) else None
+            code.append((m[1], m[2], jump and int(jump[1], 16)))
+    start = min(at, default=0)
+    before = [[i - 1] if i and code[i - 1][0] not in ("s_branch", "s_endpgm") else [] for i in range(len(code))]
+    for i, (_, _, jump) in enumerate(code):
+        if jump is not None:
+            before[at[start + jump]].append(i)
+
+    def registers(text):
+        out = set()
+        for kind, low, _, high in re.findall(r"\b([va])\[?(\d+)(:(\d+))?", text):
+            out |= {(kind, r) for r in range(int(low), int(high or low) + 1)}
+        return out
+
+    uses = [registers(args) for _, args, _ in code]
+    results = [registers(args.split(",")[0]) for _, args, _ in code]
+
+    def within(i, states):
+        """Instructions from which fewer than `states` wait states lie before i, along every way there."""
+        seen, todo = {}, [(j, states) for j in before[i]]
+        while todo:
+            j, left = todo.pop()
+            if seen.get(j, 0) >= left:
+                continue
+            seen[j] = left
+            left -= 1 + (int(code[j][1], 0) if code[j][0] == "s_nop" else 0)
+            if left > 0:
+                todo += [(k, left) for k in before[j]]
+        return seen
+
+    faults = []
+    for i, (op, args, _) in enumerate(code):
+        if op.startswith("v_mfma"):
+            for j in within(i, 2):
+                if code[j][0].startswith("v_") and not code[j][0].startswith("v_mfma") and uses[j] & uses[i]:
+                    faults.append(f"{name}: {code[j][0]} {code[j][1]} just before {op} {args}")
+        elif any(kind == "a" for kind, _ in uses[i]):
+            for j in within(i, 19):
+                if code[j][0].startswith("v_mfma") and results[j] & uses[i]:
+                    faults.append(f"{name}: {op} {args} too close behind {code[j][0]} {code[j][1]}")
+        if op.startswith("scratch_"):
+            faults.append(f"{name}: registers in scratch memory: {op} {args}")
+        if re.search(r"\bm0\b", args) and not (op == "s_mov_b32" and args.startswith("m0,") and
+                                               any(code[k][0].startswith("global_load_lds") for k in (i + 1, i + 2) if k < len(code))):
+            faults.append(f"{name}: M0 beside the loads to LDS: {op} {args}")
+    return faults
+
+
+def check_matrix_kernels(lib: str) -> int:
+    """operand_faults of every gemm16_square_kernel in a built library; their number."""
+    objdump = os.path.join(os.path.dirname(os.path.realpath(shutil.which(hipcc()) or hipcc())), "..", "llvm", "bin", "llvm-objdump")
+    faults, kernels = [], 0
+    with tempfile.TemporaryDirectory() as folder:
+        os.symlink(os.path.abspath(lib), os.path.join(folder, "lib"))
+        subprocess.check_call([objdump, "--offloading", "lib"], cwd=folder, stdout=subprocess.DEVNULL)
+        for part in sorted(os.listdir(folder)):
+            path = os.path.join(folder, part)
+            if "gfx950" not in part or b"gemm16_square_kernel" not in open(path, "rb").read():
+                continue
+            text = subprocess.check_output([objdump, "-d", "--no-show-raw-insn", path], text=True)
+            for block in re.split(r"\n(?=[0-9a-f]+ <)", text):
+                head, _, body = block.partition("\n")
+                if "gemm16_square_kernel" in head:
+                    kernels += 1
+                    faults += operand_faults(head.split("<")[1].split(">")[0], body.splitlines())
+    if faults:
+        raise RuntimeError("matrix instructions of the compiled kernels:\n" + "\n".join(faults[:20]))
+    return kernels
+
+
 def build_library(verbose: bool = True, jobs: int = 8) -> str:
     """Compile every source to an object in parallel, then link the shared library."""
     objdir = os.path.join(HERE, "build")
@@ -95,6 +179,7 @@ def build_library(verbose: bool = True, jobs: int = 8) -> str:
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
+    check_matrix_kernels(LIB)
     build_host(verbose)
     return LIB
 

@@ -10,6 +10,7 @@
 #pragma once
 
 #include <type_traits>
+#include <utility>
 
 #include "gemm16.h"
 
@@ -17,9 +18,10 @@ namespace mega {
 namespace {
 
 constexpr int kKS = 64;           // reduction indices a step
-// 16 bytes a lane from memory to LDS: lane l's go to byte lds + 16 l
+// 16 bytes a lane from memory to LDS: lane l's go to byte lds + 16 l.  (That the compiler keeps nothing of its own in M0 is
+// part of the build's check: putting it back each time costs 2 %.)
 __device__ __forceinline__ void dma16(uint32_t lds, uint32_t off, const char* base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
 }
 template <int N>
 __device__ __forceinline__ void wait_loads() {
@@ -94,7 +96,10 @@ __device__ __forceinline__ uint4 keep(uint4 f, int k0, int left) {
 }
 
 // c += a b with the accumulator in the accumulator registers (left to itself the compiler keeps it in the others and moves it
-// to and fro)
+// to and fro).  The compiler pads its own matrix instructions with the wait states that a vector instruction before them, or
+// behind them on their result, calls for; these it does not see.  None is needed where it puts no register copy between them,
+// which the build checks in the compiled kernels (check_matrix_kernels of build.py) instead of paying for it here: two wait
+// states with each cost 3 - 5 % of a product (8192 x 8192 x 8192 705, 730 us), with every fourth as much.
 template <typename T>
 __device__ __forceinline__ void mma_acc(f32x4& c, uint4 a, uint4 b) {
   typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
@@ -243,6 +248,16 @@ __device__ __forceinline__ void finish_wave(const Gemm16P& G, const Place& p, in
   }
 }
 
+// f(0), .. f(N - 1) with their numbers as constants: fragments addressed by them are registers whatever is unrolled when
+template <int... I, typename F>
+__device__ __forceinline__ void each_of(std::integer_sequence<int, I...>, F&& f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void each(F&& f) {
+  each_of(std::make_integer_sequence<int, N>{}, f);
+}
+
 template <typename T, bool KA, bool KB, bool RAG>
 __global__ __launch_bounds__(256, 1) void gemm16_square_kernel(const Gemm16P G) {
   constexpr int TN = 256, ST = 2, kWT = 256;                       // columns of a tile, stages, threads
@@ -303,16 +318,15 @@ __global__ __launch_bounds__(256, 1) void gemm16_square_kernel(const Gemm16P G) 
   const char* la = lds;
   uint4 fa[2][FM], fb[2][FN];
   constexpr int NM = FM * FN, FR = FM + FN, RS = NM * 3 / 4 / FR, DS = NM / LD;
-  auto read = [&](auto Q, const char* from, int f) {                // fragment f of index half Q: fb 0, fa 0 .., fb 1 ..
-    constexpr int q = decltype(Q)::value;
-    if (f == 0) fb[q][0] = fb_at.get(from + SA::Bytes, 0, q);
-    else if (f <= FM) fa[q][f - 1] = fa_at.get(from, f - 1, q);
-    else fb[q][f - FM] = fb_at.get(from + SA::Bytes, f - FM, q);
+  auto read = [&](auto Q, const char* from, auto F) {               // fragment F of index half Q: fb 0, fa 0 .., fb 1 ..
+    constexpr int q = decltype(Q)::value, f = decltype(F)::value;
+    if constexpr (f == 0) fb[q][0] = fb_at.get(from + SA::Bytes, 0, q);
+    else if constexpr (f <= FM) fa[q][f - 1] = fa_at.get(from, f - 1, q);
+    else if constexpr (f < FR) fb[q][f - FM] = fb_at.get(from + SA::Bytes, f - FM, q);
   };
   using zero = std::integral_constant<int, 0>;
   using one = std::integral_constant<int, 1>;
-#pragma unroll
-  for (int f = 0; f < FR; ++f) read(zero{}, la, f);
+  each<FR>([&](auto f) { read(zero{}, la, f); });
   auto step = [&](auto MORE, const int s) {
     constexpr bool more = decltype(MORE)::value;
     const int left = ke - kb - s * kKS, g8 = (lane >> 4) * 8;
@@ -324,13 +338,13 @@ __global__ __launch_bounds__(256, 1) void gemm16_square_kernel(const Gemm16P G) 
       asm volatile("s_nop 4" ::: "memory");
     }
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int t = 0; t < NM; ++t) {
+    each<NM>([&](auto at) {
+      constexpr int t = decltype(at)::value;
       // (all read in the first three quarters: they have arrived when the products are through)
-      if (t % RS == 0 && t / RS < FR) read(one{}, la, t / RS);
+      if constexpr (t % RS == 0) read(one{}, la, std::integral_constant<int, t / RS>{});
       mma_acc<T>(acc[t % FM][t / FM], fb[0][t / FM], fa[0][t % FM]);
       __builtin_amdgcn_sched_barrier(0);
-    }
+    });
     if (more) wait_loads<LD*(ST - 2)>();
     else wait_loads<0>();
     barrier();
@@ -344,13 +358,13 @@ __global__ __launch_bounds__(256, 1) void gemm16_square_kernel(const Gemm16P G) 
     }
     if (RAG && more && next == steps - 1) offsets(ke - kb - next * kKS);
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int t = 0; t < NM; ++t) {
-      if (t % RS == 0 && t / RS < FR) read(zero{}, la, t / RS);
+    each<NM>([&](auto at) {
+      constexpr int t = decltype(at)::value;
+      if constexpr (t % RS == 0) read(zero{}, la, std::integral_constant<int, t / RS>{});
       if (more && t % DS == 1 && t / DS < LD) piece(t / DS);
       mma_acc<T>(acc[t % FM][t / FM], fb[1][t / FM], fa[1][t % FM]);
       __builtin_amdgcn_sched_barrier(0);
-    }
+    });
     if (more) advance();
   };
   int s = 0;
