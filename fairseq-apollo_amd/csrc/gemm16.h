@@ -42,8 +42,14 @@ __device__ __forceinline__ f32x4 mma16(uint4 a, uint4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
 
-// (the reciprocal is good to one unit; the result is rounded to 16 bits)
-__device__ __forceinline__ float silu_h(float v) { return v * __builtin_amdgcn_rcpf(1.f + __expf(-v)); }
+// v / (1 + e^-v): the reciprocal's quotient (scaled, so that it stays a normal number to the end of the exponential's range) and
+// one Newton step from its remainder; an infinite denominator has none.  Of all bf16 values none differs from the division's
+// result (the bare reciprocal's: 4, and nothing below -87.3), of fp16 one tie; on wide tiles 2 us of 8192 x 2048 x 1024 (40.5),
+// the division 5.
+__device__ __forceinline__ float silu_h(float v) {
+  const float n = v * 0x1p-8f, d = fmaf(__expf(-v), 0x1p-8f, 0x1p-8f), y = __builtin_amdgcn_rcpf(d), q = n * y;
+  return fmaf(fminf(fmaf(-d, q, n), 0x1p127f), y, q);
+}
 
 // E consecutive values of row m from column n on: bias and residual, one rounding, silu of the rounded value
 template <typename T, int E>

@@ -337,3 +337,19 @@ def test_16bit_epilogues_on_wide_tiles(m, n, k, bias, res, silu, pre):
         assert _rel(p, r) < tol
     # silu of the rounded value (known where it is written as well; its slope is at most 1.1), rounded again
     assert _rel(c, F.silu(p.double() if pre else r) if silu else r) < (2.0 ** -9 + 2.0 ** -22 if pre and silu else 3 * tol if silu else tol)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,k", [(8, 8), (256, 1024)])                  # tiles of 64; wide ones
+def test_16bit_silu_of_every_value(dtype, n, k):
+    """Half a unit in the last place and 32-bit exp's few units (its argument's rounding: 89 of 2^-24), to the end of exp's range:
+    from e^126 ln 2 on the reciprocal of 1 + e^-v alone is no normal number (bf16 -88: -5.3e-37)."""
+    v = torch.arange(-32768, 32768, device=DEV).to(torch.int16).view(dtype)
+    v = torch.where(v.isfinite(), v, 0)
+    a, b = torch.zeros(65536, k, device=DEV, dtype=dtype), torch.zeros(n, k, device=DEV, dtype=dtype)
+    a[:, 0], b[:, 0] = v, 1
+    c, x = _gemm(a, b, 0, 0, silu=True).double(), v.double()[:, None]
+    r = x * torch.where(x < 0, x.exp() / (1 + x.exp()), 1 / (1 + (-x).exp()))
+    info = torch.finfo(dtype)
+    close = (c - r).abs() <= (info.eps / 2 + 100 * 2.0 ** -24) * r.abs() + info.tiny * info.eps / 2
+    assert bool((close | ((x < -88.7) & (c == 0))).all())
