@@ -235,6 +235,12 @@ bool gemm16_wide(int64_t M, int64_t N, int64_t K, WidePlan* p) {
 //              1024 x 2816 x 8192   59.1, 84.8     2048 x 5632 x 8192    174, 178
 bool gemm16_wins(int64_t M, int64_t N, int64_t K) { return 2.0 * (double)M * (double)N * (double)K <= 1e13; }
 
+// Sizes that the kernels hold in 32 bits, tiles that a launch takes (2^32 threads)
+bool gemm16_launchable(int64_t M, int64_t N, int64_t K) {
+  const int64_t most = (int64_t)1 << 30;
+  return M < most && N < most && K < most && ceil_div(M, kTile) * ceil_div(N, kTile) < ((int64_t)1 << 32) / kHT;
+}
+
 template <typename T, bool KA, bool KB>
 void launch16(const Gemm16P& G, unsigned blocks, hipStream_t s) {
   constexpr int smem = 2 * 2 * kTile * kTile * 2;
@@ -258,7 +264,7 @@ void launch16_type(const Gemm16P& G, const Plan16& p, int ka, int kb, unsigned b
 using namespace mega;
 
 extern "C" int mega_gemm16_pays(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor) {
-  return gemm16_wins(M, N, K) ? 1 : 0;
+  return gemm16_launchable(M, N, K) && gemm16_wins(M, N, K) ? 1 : 0;
 }
 
 extern "C" size_t mega_gemm16_workspace_bytes(int64_t M, int64_t N, int64_t K) {
@@ -274,8 +280,7 @@ extern "C" int mega_gemm16(const MegaGemm* g, int dtype, void* workspace, size_t
   MEGA_REQUIRE(g->M > 0 && g->N > 0 && g->K > 0 && g->batch == 1 && !g->causal && g->alpha == 1.f, MEGA_ERR_UNSUPPORTED,
                "gemm16: single products without a factor");
   MEGA_REQUIRE(g->a && g->b && g->c, MEGA_ERR_ARG, "gemm16: null pointer argument");
-  MEGA_REQUIRE(g->M < (int64_t)1 << 30 && g->N < (int64_t)1 << 30 && g->K < (int64_t)1 << 30, MEGA_ERR_UNSUPPORTED,
-               "gemm16: sizes below 2^30");
+  MEGA_REQUIRE(gemm16_launchable(g->M, g->N, g->K), MEGA_ERR_UNSUPPORTED, "gemm16: sizes below 2^30, fewer than 2^24 tiles of 64 x 64");
   MEGA_REQUIRE(g->lda >= (g->a_kmajor ? g->M : g->K) && g->ldb >= (g->b_kmajor ? g->N : g->K) && g->ldc >= g->N &&
                    (!g->residual || g->ldr >= g->N),
                MEGA_ERR_ARG, "gemm16: a leading dimension is shorter than its row");
@@ -292,7 +297,6 @@ extern "C" int mega_gemm16(const MegaGemm* g, int dtype, void* workspace, size_t
   WidePlan w;
   // (rows of a wide tile within 4 GB of its first element)
   if (gemm16_wide(g->M, g->N, g->K, &w) && g->lda < far / 2 && g->ldb < far / 2) {
-    MEGA_REQUIRE(ceil_div(g->M, kWideM) * ceil_div(g->N, w.tn) < (int64_t)1 << 27, MEGA_ERR_UNSUPPORTED, "gemm16: too many tiles");
     MEGA_REQUIRE(!w.bytes || (workspace && workspace_bytes >= w.bytes && on16(workspace)), MEGA_ERR_WORKSPACE,
                  "gemm16: workspace of %zu bytes needed", w.bytes);
     gemm16_wide_launch(G, w, dtype == MEGA_BF16, g->a_kmajor, g->b_kmajor, workspace, (hipStream_t)stream);
@@ -309,8 +313,7 @@ extern "C" int mega_gemm16(const MegaGemm* g, int dtype, void* workspace, size_t
     G.part = (float*)workspace;
     G.kstep = p.kstep;
   }
-  const int64_t blocks = (int64_t)G.mt * G.nt * p.splits;
-  MEGA_REQUIRE(blocks < (int64_t)1 << 31, MEGA_ERR_UNSUPPORTED, "gemm16: too many tiles");
+  const int64_t blocks = (int64_t)G.mt * G.nt * p.splits;          // (split only where they are few)
   if (dtype == MEGA_BF16) launch16_type<bf16_t>(G, p, g->a_kmajor, g->b_kmajor, (unsigned)blocks, (hipStream_t)stream);
   else launch16_type<f16_t>(G, p, g->a_kmajor, g->b_kmajor, (unsigned)blocks, (hipStream_t)stream);
   MEGA_CHECK_LAUNCH("gemm16");

@@ -185,6 +185,13 @@ def test_the_limit_of_16bit_products_stands_once():
     assert M._lib.load().mega_gemm16_pays(m, n, k, 0, 0) == 1 and M._lib.load().mega_gemm16_pays(m, n, k + 1, 0, 0) == 0
 
 
+@pytest.mark.parametrize("m,n,k,own", [((1 << 30) - 64, 8, 8, 1), (1 << 30, 8, 8, 0), (8, 1 << 30, 8, 0), ((1 << 29) - 64, 128, 8, 1), (1 << 29, 136, 8, 0)])
+@pytest.mark.parametrize("a_kmajor,b_kmajor", [(0, 1), (1, 1)])
+def test_16bit_products_that_no_launch_takes(m, n, k, own, a_kmajor, b_kmajor):
+    """Sizes beyond the kernels' 32 bits or a launch's 2^32 threads are left to the GEMM library, not refused."""
+    assert M._lib.load().mega_gemm16_pays(m, n, k, a_kmajor, b_kmajor) == own
+
+
 @pytest.mark.parametrize("m,n,k,batch,heads,causal,a_kmajor,own", [
     (512, 512, 128, 8, 1, 0, 0, 1), (1000, 64, 1000, 8, 1, 0, 0, 0), (4096, 64, 4096, 2, 1, 2, 0, 0), (512, 512, 1024, 1, 1, 1, 0, 0),
     (1000, 1000, 64, 16, 4, 0, 0, 1), (2048, 2048, 1024, 4, 1, 0, 0, 1), (2048, 2048, 32, 8, 1, 0, 0, 0), (1000, 1000, 512, 8, 1, 0, 0, 1),
