@@ -69,6 +69,7 @@ SIGNATURES = {
     "mega_norm_ema_fwd_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64]),
     "mega_norm_ema_fwd_scratch_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64]),
     "mega_gemm16_pays": (_int, [_i64, _i64, _i64, _int, _int]),
+    "mega_gemm16_silu_pays": (_int, [_i64, _i64, _i64, _int, _int]),
     "mega_gemm16_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "mega_gemm16": (_int, [_p, _int, _p, _sz, _p]),
     "mega_embedding_grad_workspace_bytes": (_sz, [_i64, _i64, _i64]),

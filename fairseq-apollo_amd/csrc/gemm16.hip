@@ -225,15 +225,36 @@ bool gemm16_wide(int64_t M, int64_t N, int64_t K, WidePlan* p) {
   return p->us < gemm16_small_us(M, N, K);
 }
 
-// Products that come here: all but the largest, whose one library call costs the host nothing against milliseconds on the
-// device.  us of device time beside the library's, whose call costs the host 20 us more and takes no silu:
-//   x W^T      8192 x 2048 x 1024   32.0, 31.1     8192 x 4352 x 1024   80.8, 71.9     8192 x 1024 x 2048   31.5, 33.1
-//              8192 x 2816 x 1024   53.0, 48.8     8192 x 1024 x 2816   43.6, 45.1     6144 x 2816 x 1024   46.3, 53.7
-//              8192 x 8704 x 2048    228, 242      8192 x 5632 x 2048    145, 156      8192 x 2048 x 5632    137, 122
-//   dY W       8192 x 1024 x 4352   67.2, 71.6     8192 x 2048 x 4096   95.7, 103      8192 x 2048 x 8704    193, 208
-//   dY^T X     2048 x 1024 x 8192   43.0, 69.3     4352 x 1024 x 8192   82.2, 116      8704 x 2048 x 8192    224, 307
-//              1024 x 2816 x 8192   59.1, 84.8     2048 x 5632 x 8192    174, 178
-bool gemm16_wins(int64_t M, int64_t N, int64_t K) { return 2.0 * (double)M * (double)N * (double)K <= 1e13; }
+// Products that come here.  us of device time beside the library's, between a pass that writes the operand and one that reads
+// the result (x W^T in whole tiles), otherwise operands and results from memory (more than 600 MB of them in turn; *: the same
+// ones each time):
+//   x W^T, whole rounds of tiles or less than two
+//                5000 x 2048 x 1024   28.0, 24.2     8192 x 1024 x 2048   34.2, 35.6     8192 x 2816 x 1024   57.7, 53.3
+//                5000 x 2048 x 4096   88.1, 70.2     8192 x 2048 x 5632    130, 123     32768 x 5632 x 2048    571, 528
+//     more than two, the last one partial    12000 x 2816 x 1024   76.7, 84.6     12000 x 4352 x 1024    115, 147
+//                8192 x 5632 x 2048    156, 163      8192 x 8704 x 2048    246, 260     12000 x 4096 x 4096    284, 443
+//                8192 x 4352 x 1024   82.4, 73.1    10000 x 5632 x 2048    198, 180     16384 x 8704 x 2048    464, 435
+//     N not in whole tiles   8192 x 1032 x 1024   29.6, 29.9     8192 x 3264 x 768   56.3, 67.4    65536 x 776 x 1024    123, 156
+//               20000 x 2056 x 512    61.7, 116      8192 x 8200 x 2048    233, 275     65536 x 2056 x 2048   499, 451
+//     with silu (the library's takes another pass)    2048 x 4096 x 2048   36.5, 43.0    8192 x 4096 x 2048    126, 129
+//               16384 x 1536 x 768    58.7, 63.7    32768 x 8192 x 4096   1551, 1601    16384 x 8192 x 8192   1493, 1464
+//   dY W         8192 x 1024 x 2048   36.2, 39.6     5000 x 2048 x 4096   92.7, 80.9     8192 x 2048 x 8704    223, 232
+//               16384 x 5632 x 2048    321, 362     16384 x 16384 x 16384*  6221, 6574
+//   dY^T X       1024 x 2048 x 8192   44.5, 76.3     4352 x 1024 x 12000   117, 172      8704 x 2048 x 8192    248, 320
+//                2816 x 1024 x 2048   29.3, 26.2    16384 x 16384 x 16384*  6315, 7585
+// x W^T in whole tiles: the library is 6 % ahead on average (127 sizes), but where its tiles leave a partial round behind more than
+// two whole ones, 6 % behind (33 sizes, 0.89 to 1.56).  Its call costs the host 26 us, so that calls made of products below
+// 20 GFLOP (20 us and less) are bound by the host with it: a layer of 2048 tokens of 1024 channels 217 us, 299 with the
+// library; beyond, the device is the bound: 5000 tokens of 2048 channels 1032 with all of them here, 947 in the library.  N not
+// in whole tiles: 10 - 25 % ahead to 200 GFLOP, even to 400.  silu: ahead by the pass, whose share is 1 / K.  dY W is even to
+// 130 GFLOP, 2 - 5 % ahead beyond, dY^T X 20 - 70 % ahead.  Nothing is measured beyond 1e13.
+bool gemm16_wins(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor, bool silu) {
+  const double flops = 2.0 * (double)M * (double)N * (double)K;
+  if (a_kmajor || b_kmajor) return flops <= 1e13;
+  if (silu && K <= 4096) return flops <= 2.5e12;
+  const int64_t tiles = ceil_div(M, kWideM) * ceil_div(N, 256), round = device_cu_count();
+  return flops <= (N % 256 || (tiles > 2 * round && tiles % round) ? 5e11 : 2e10);
+}
 
 // Sizes that the kernels hold in 32 bits, tiles that a launch takes (2^32 threads)
 bool gemm16_launchable(int64_t M, int64_t N, int64_t K) {
@@ -264,7 +285,11 @@ void launch16_type(const Gemm16P& G, const Plan16& p, int ka, int kb, unsigned b
 using namespace mega;
 
 extern "C" int mega_gemm16_pays(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor) {
-  return gemm16_launchable(M, N, K) && gemm16_wins(M, N, K) ? 1 : 0;
+  return gemm16_launchable(M, N, K) && gemm16_wins(M, N, K, a_kmajor, b_kmajor, false) ? 1 : 0;
+}
+
+extern "C" int mega_gemm16_silu_pays(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor) {
+  return gemm16_launchable(M, N, K) && gemm16_wins(M, N, K, a_kmajor, b_kmajor, true) ? 1 : 0;
 }
 
 extern "C" size_t mega_gemm16_workspace_bytes(int64_t M, int64_t N, int64_t K) {

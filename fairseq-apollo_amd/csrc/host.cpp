@@ -559,7 +559,7 @@ Result ema_param_backward(const Args& A) {
 }
 
 // ---- training: the layer around its norm, moving average and attention, forwards and backwards in few calls.  The
-// products (but the largest of 16-bit types, and fp32 ones by size) and what lies between them run in libmega_hip.
+// products (by size, order and type) and what lies between them run in libmega_hip.
 // Activations and weights share one type.
 Tensor rows2(const Tensor& t) { return t.reshape({-1, t.size(-1)}); }
 
@@ -593,7 +593,7 @@ bool product(const Tensor& a, const Tensor& b, const Tensor& bias, const Tensor&
   if (residual.defined() && (!fits(residual) || !matrix(residual, &mr) || mr.first || residual.size(0) != M || residual.size(1) != N)) return false;
   auto on16 = [](const Tensor& t) { return !t.defined() || (uintptr_t)t.data_ptr() % 16 == 0; };
   const int64_t vec = 16 / a.element_size(), far = ((int64_t)1 << 32) / a.element_size() / 128;
-  if (!(wide ? mega_gemm_f32_pays : mega_gemm16_pays)(M, N, K, ma.first, !mb.first) || ma.ld % vec || mb.ld % vec || (ma.first ? M : K) % vec ||
+  if (!(wide ? mega_gemm_f32_pays : silu ? mega_gemm16_silu_pays : mega_gemm16_pays)(M, N, K, ma.first, !mb.first) || ma.ld % vec || mb.ld % vec || (ma.first ? M : K) % vec ||
       (mb.first ? K : N) % vec || ma.ld >= far || mb.ld >= far)
     return false;
   if (!wide && (N % vec || mr.ld % vec || !on16(bias) || !on16(residual) || !on16(*out))) return false;

@@ -1409,23 +1409,24 @@ def embed(table: nn.Embedding, ids: Tensor) -> Tensor:
 
 
 EMBED_ROWS = 318                  # mega_embedding_grad's limit: larger tables keep torch's operation
-OWN_16BIT_FLOPS = 1e13            # mega_gemm16_pays of products along the rows: no native call is made to be told no
+OWN_16BIT_FLOPS = 5e11            # mega_gemm16_pays of products along the rows: no native call is made to be told no
 
 
-def own_product(lin: nn.Linear, x: Tensor, *more) -> bool:
-    """lin(x) outside training may be one of the library's own products (fp32, and 16-bit types at some sizes)."""
+def own_product(lin: nn.Linear, x: Tensor, *more, act: bool = False) -> bool:
+    """lin(x), or silu(lin(x)), outside training may be one of the library's own products (fp32, and 16-bit types at some
+    sizes)."""
     if type(lin) is not nn.Linear:                     # (a scripted module's parameters are no dictionary)
         return False
     w, b = lin._parameters.get('weight'), lin._parameters.get('bias')
     return (x.is_cuda and x.dim() > 1 and w is not None and w.dim() == 2
-            and (x.dtype is torch.float32 or 2 * x.numel() * w.shape[0] <= OWN_16BIT_FLOPS) and not torch.is_grad_enabled()
+            and (act or x.dtype is torch.float32 or 2 * x.numel() * w.shape[0] <= OWN_16BIT_FLOPS) and not torch.is_grad_enabled()
             and not torch.compiler.is_compiling() and not torch.is_autocast_enabled() and x.is_contiguous() and x.shape[-1] == w.shape[1]
             and _plain(b is not None, lin) and ops._lib.load_host().uniform(x, w, b, *more))
 
 
 def project(lin: nn.Linear, x: Tensor, act: bool = False) -> Tensor:
     """lin(x), or silu(lin(x)), outside training."""
-    if own_product(lin, x):
+    if own_product(lin, x, act=act):
         with ops._on_device(x.device):
             y = ops._lib.load_host().linear_own(x, lin.weight, lin.bias, None, act, False, ops._stream(x.device))
         if y is not None:

@@ -438,6 +438,7 @@ int mega_gemm_f32(const MegaGemm* g, void* workspace, size_t workspace_bytes, vo
 /* The same for single bf16 / fp16 products (operands, bias, residual, pre and C of `dtype`, fp32 sums, alpha 1, silu of the
  * rounded value): rows of whole 16-byte pieces on 16 bytes, N a multiple of eight (csrc/gemm16.hip).           */
 int mega_gemm16_pays(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor);   /* faster here than in a GEMM library */
+int mega_gemm16_silu_pays(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor);   /* with silu, the library's as a pass of its own */
 size_t mega_gemm16_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int mega_gemm16(const MegaGemm* g, int dtype, void* workspace, size_t workspace_bytes, void* stream);
 

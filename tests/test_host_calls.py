@@ -185,6 +185,18 @@ def test_the_limit_of_16bit_products_stands_once():
     assert M._lib.load().mega_gemm16_pays(m, n, k, 0, 0) == 1 and M._lib.load().mega_gemm16_pays(m, n, k + 1, 0, 0) == 0
 
 
+@pytest.mark.parametrize("m,n,k,order,silu,own", [
+    (2048, 4096, 1024, 0, 0, 1), (5000, 2048, 1024, 0, 0, 0), (8192, 2816, 1024, 0, 0, 0), (8192, 2048, 5632, 0, 0, 0), (8192, 8192, 8192, 0, 0, 0),
+    (8192, 4096, 2048, 0, 0, 0), (32768, 5632, 2048, 0, 0, 0), (12000, 2816, 1024, 0, 0, 1), (8192, 5632, 2048, 0, 0, 1), (16384, 8704, 2048, 0, 0, 0),
+    (8192, 3264, 768, 0, 0, 1), (65536, 2056, 2048, 0, 0, 0), (5000, 2048, 1024, 0, 1, 1), (8192, 4096, 2048, 0, 1, 1),
+    (8192, 4096, 8192, 0, 1, 0), (2048, 512, 8192, 0, 1, 1), (1 << 29, 136, 8, 0, 1, 0), (8192, 2048, 5632, 1, 0, 1), (8192, 8192, 8192, 3, 0, 1)])
+def test_sizes_of_the_16bit_products(m, n, k, order, silu, own):
+    """x W^T that the device computes clearly faster in the GEMM library, where the device and not its call's host time is the
+    bound, is left to it; with silu, whose pass the library's product does not spare, and the gradients' orders are not."""
+    lib = M._lib.load()
+    assert (lib.mega_gemm16_silu_pays if silu else lib.mega_gemm16_pays)(m, n, k, order >> 1, order & 1) == own
+
+
 @pytest.mark.parametrize("m,n,k,own", [((1 << 30) - 64, 8, 8, 1), (1 << 30, 8, 8, 0), (8, 1 << 30, 8, 0), ((1 << 29) - 64, 128, 8, 1), (1 << 29, 136, 8, 0)])
 @pytest.mark.parametrize("a_kmajor,b_kmajor", [(0, 1), (1, 1)])
 def test_16bit_products_that_no_launch_takes(m, n, k, own, a_kmajor, b_kmajor):
