@@ -207,19 +207,22 @@ Plan16 gemm16_plan(int64_t M, int64_t N, int64_t K) {
   return p;
 }
 
-// What a product costs here, us of device time: half a microsecond a step of the two workgroups a compute unit holds, the
-// second kernel's 5 and its traffic at 4 TB/s.
+// What a product costs here, us of device time: 0.36 a step of a compute unit's only workgroup, half a microsecond of the two it
+// holds, the second kernel's 5 and its traffic at 4 TB/s.  (600 x 1024 x 2816 19.3, 1000 x 1024 x 2816 19.8, 768 x 768 x 2048
+// 15.3, 300 x 2048 x 4096 26.5, 1000 x 2048 x 4096 33.5.)
 double gemm16_small_us(int64_t M, int64_t N, int64_t K) {
   const Plan16 p = gemm16_plan(M, N, K);
   const double tiles = (double)ceil_div(M, kTile) * ceil_div(N, kTile) * p.splits, two = 2.0 * device_cu_count();
-  return 4 + 0.5 * ceil_div(ceil_div(K, p.splits), kTile) * (tiles > two ? tiles / two : 1) +
+  return 4 + (2 * tiles > two ? 0.5 : 0.36) * ceil_div(ceil_div(K, p.splits), kTile) * (tiles > two ? tiles / two : 1) +
          (p.splits > 1 ? 5 + (double)M * N * (4 * p.splits + 2) / 4e6 : 0);
 }
 
 // Wide tiles (gemm16_wide.h) where their estimate is the smaller one; us, tiles of 64 and wide ones:
 //     300 x 4352 x 1024   10, 15       600 x 4352 x 1024   16.5, 15     1000 x 4352 x 1024   25, 16
 //    2048 x 2048 x 1024   19, 16      2048 x 4352 x 1024   43, 26       5000 x 1536 x 768    27, 16
+//     600 x 1024 x 2816   19, 24      1000 x 1024 x 2816   20, 23      1000 x 2048 x 4096   34, 29
 //   both K-major   264 x 1024 x 8192   22, 24     1024 x 2048 x 2000   21, 27     1536 x 768 x 4503   39, 26
+//                  768 x 768 x 2048    15, 22
 bool gemm16_wide(int64_t M, int64_t N, int64_t K, WidePlan* p) {
   *p = gemm16_wide_plan(M, N, K);
   return p->us < gemm16_small_us(M, N, K);

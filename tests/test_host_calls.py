@@ -212,3 +212,10 @@ def test_16bit_products_that_no_launch_takes(m, n, k, own, a_kmajor, b_kmajor):
 def test_sizes_of_the_fp32_attention_products(m, n, k, batch, heads, causal, a_kmajor, own):
     """Batched fp32 products that the matrix-core kernel serves clearly slower than the GEMM library are left to it."""
     assert M._lib.load().mega_gemm_f32_batched_pays(m, n, k, batch, heads, causal, a_kmajor) == own
+
+
+@pytest.mark.parametrize("m,n,k,parts", [(600, 1024, 2816, 0), (1000, 1024, 2816, 0), (768, 768, 2048, 0), (1000, 768, 3264, 0), (1000, 2048, 4096, 1), (300, 2048, 4096, 1)])
+def test_16bit_products_in_parts(m, n, k, parts):
+    """One workgroup of 64 x 64 on every compute unit is not taken for half of two: wide tiles in parts, and their second
+    launch, only where they are the quicker ones."""
+    assert (M._lib.load().mega_gemm16_workspace_bytes(m, n, k) > 0) == parts
