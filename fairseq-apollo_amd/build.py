@@ -61,12 +61,12 @@ def hipcc() -> str:
     raise RuntimeError("hipcc not found")
 
 
-def operand_faults(name: str, listing: list) -> list:
-    """What a kernel whose matrix instructions are written as inline assembly must not hold, in its disassembly (lines of
-    llvm-objdump): the compiler pads the matrix instructions it knows with wait states, these it moves values around
-    unpadded.  Two wait states belong between a vector instruction and a matrix instruction that shares a register with it, 19
-    between a matrix instruction and any other use of its result; no registers in scratch memory (fragments would come back
-    through copies); M0 written before a load to LDS and used for nothing else."""
+def assembly_faults(name: str, listing: list, matrix: bool = True) -> list:
+    """What a kernel with inline assembly must not hold, in its disassembly (lines of llvm-objdump).  Loads to LDS: M0 is
+    written before one and used for nothing else.  Matrix instructions: the compiler pads those it knows with wait states, these
+    it moves values around unpadded.  Two wait states belong between a vector instruction and a matrix instruction that
+    shares a register with it, 19 between a matrix instruction and any other use of its result; no registers in scratch memory
+    (fragments would come back through copies)."""
     code, at = [], {}
     for line in listing:
         m = re.match(r"\s+(\S+)\s*(.*?)\s*// ([0-9A-F]+):(.*)", line)
@@ -104,6 +104,11 @@ def operand_faults(name: str, listing: list) -> list:
 
     faults = []
     for i, (op, args, _) in enumerate(code):
+        if re.search(r"\bm0\b", args) and not (op == "s_mov_b32" and args.startswith("m0,") and
+                                               any(code[k][0].startswith("global_load_lds") for k in (i + 1, i + 2) if k < len(code))):
+            faults.append(f"{name}: M0 beside the loads to LDS: {op} {args}")
+        if not matrix:
+            continue
         if op.startswith("v_mfma"):
             for j in within(i, 2):
                 if code[j][0].startswith("v_") and not code[j][0].startswith("v_mfma") and uses[j] & uses[i]:
@@ -114,31 +119,33 @@ def operand_faults(name: str, listing: list) -> list:
                     faults.append(f"{name}: {op} {args} too close behind {code[j][0]} {code[j][1]}")
         if op.startswith("scratch_"):
             faults.append(f"{name}: registers in scratch memory: {op} {args}")
-        if re.search(r"\bm0\b", args) and not (op == "s_mov_b32" and args.startswith("m0,") and
-                                               any(code[k][0].startswith("global_load_lds") for k in (i + 1, i + 2) if k < len(code))):
-            faults.append(f"{name}: M0 beside the loads to LDS: {op} {args}")
     return faults
 
 
-def check_matrix_kernels(lib: str) -> int:
-    """operand_faults of every gemm16_square_kernel in a built library; their number."""
+# kernels with loads to LDS as assembly (dma16 of gemm16_wide.h), and whether their matrix instructions are assembly too
+ASSEMBLY = {"gemm16_square_kernel": True, "gemm16_tall_kernel": False, "attn_wide_kernel": False}
+
+
+def check_assembly(lib: str) -> dict:
+    """assembly_faults of every kernel in a built library that holds assembly; how many there are of each."""
     objdump = os.path.join(os.path.dirname(os.path.realpath(shutil.which(hipcc()) or hipcc())), "..", "llvm", "bin", "llvm-objdump")
-    faults, kernels = [], 0
+    faults, kernels = [], dict.fromkeys(ASSEMBLY, 0)
     with tempfile.TemporaryDirectory() as folder:
         os.symlink(os.path.abspath(lib), os.path.join(folder, "lib"))
         subprocess.check_call([objdump, "--offloading", "lib"], cwd=folder, stdout=subprocess.DEVNULL)
         for part in sorted(os.listdir(folder)):
             path = os.path.join(folder, part)
-            if "gfx950" not in part or b"gemm16_square_kernel" not in open(path, "rb").read():
+            if "gfx950" not in part or not any(kind.encode() in open(path, "rb").read() for kind in ASSEMBLY):
                 continue
             text = subprocess.check_output([objdump, "-d", "--no-show-raw-insn", path], text=True)
             for block in re.split(r"\n(?=[0-9a-f]+ <)", text):
                 head, _, body = block.partition("\n")
-                if "gemm16_square_kernel" in head:
-                    kernels += 1
-                    faults += operand_faults(head.split("<")[1].split(">")[0], body.splitlines())
+                for kind, matrix in ASSEMBLY.items():
+                    if kind in head:
+                        kernels[kind] += 1
+                        faults += assembly_faults(head.split("<")[1].split(">")[0], body.splitlines(), matrix)
     if faults:
-        raise RuntimeError("matrix instructions of the compiled kernels:\n" + "\n".join(faults[:20]))
+        raise RuntimeError("inline assembly in the compiled kernels:\n" + "\n".join(faults[:20]))
     return kernels
 
 
@@ -179,7 +186,7 @@ def build_library(verbose: bool = True, jobs: int = 8) -> str:
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
-    check_matrix_kernels(LIB)
+    check_assembly(LIB)
     build_host(verbose)
     return LIB
 

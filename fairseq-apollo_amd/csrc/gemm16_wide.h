@@ -18,10 +18,10 @@ namespace mega {
 namespace {
 
 constexpr int kKS = 64;           // reduction indices a step
-// 16 bytes a lane from memory to LDS: lane l's go to byte lds + 16 l.  (That the compiler keeps nothing of its own in M0 is
-// part of the build's check: putting it back each time costs 2 %.)
+// 16 bytes a lane from memory to LDS: lane l's go to byte lds + 16 l.  (The compiler does not honour a clobber of M0.  That it
+// keeps nothing of its own there is part of the build's check: putting it back each time costs 2 % of a product.)
 __device__ __forceinline__ void dma16(uint32_t lds, uint32_t off, const char* base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
 }
 template <int N>
 __device__ __forceinline__ void wait_loads() {
@@ -98,7 +98,7 @@ __device__ __forceinline__ uint4 keep(uint4 f, int k0, int left) {
 // c += a b with the accumulator in the accumulator registers (left to itself the compiler keeps it in the others and moves it
 // to and fro).  The compiler pads its own matrix instructions with the wait states that a vector instruction before them, or
 // behind them on their result, calls for; these it does not see.  None is needed where it puts no register copy between them,
-// which the build checks in the compiled kernels (check_matrix_kernels of build.py) instead of paying for it here: two wait
+// which the build checks in the compiled kernels (check_assembly of build.py) instead of paying for it here: two wait
 // states with each cost 3 - 5 % of a product (8192 x 8192 x 8192 705, 730 us), with every fourth as much.
 template <typename T>
 __device__ __forceinline__ void mma_acc(f32x4& c, uint4 a, uint4 b) {

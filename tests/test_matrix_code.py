@@ -1,5 +1,5 @@
-"""The build's check of matrix instructions written as inline assembly (no GPU): what it finds in listings with a mistake, and
-that the built library holds none."""
+"""The build's check of kernels with inline assembly (no GPU): what it finds in listings with a mistake, and that the built
+library holds none."""
 import importlib.util
 import os
 
@@ -23,7 +23,7 @@ def faults(*code):
         if op.startswith(("s_branch", "s_cbranch")):
             target, args = f" <kernel+0x{4 * int(args):x}>", "1"
         lines.append(f"\t{op} {args}    // {0x100 + 4 * i:012X}: 00000000{target}")
-    return build.operand_faults("kernel", lines)
+    return build.assembly_faults("kernel", lines)
 
 
 @pytest.mark.parametrize("count,code", [
@@ -48,6 +48,6 @@ def test_mistakes_are_found(count, code):
     assert len(faults(*code)) == count
 
 
-def test_the_built_matrix_kernels():
-    """both types, every order of the operands, with and without a partial step"""
-    assert build.check_matrix_kernels(build.LIB) == 16
+def test_the_built_kernels():
+    """both types, every order of the operands (attention: its three products), with and without a partial step"""
+    assert build.check_assembly(build.LIB) == {"gemm16_square_kernel": 16, "gemm16_tall_kernel": 16, "attn_wide_kernel": 12}
