@@ -1161,7 +1161,7 @@ int run_attention(const void* q, const void* k, const void* v, void* y, void* w,
   AttnWeightsP W = {};
   W.q = q; W.k = k; W.P = P;
   W.L = (int)L; W.Nh = (int)Nh; W.H1 = (int)H1; W.batches = (int)BN_;
-  W.scale_log2 = scale * 1.4426950408889634f;
+  W.scale = scale;
   W.causal = causal ? 1 : 0;
   W.zero_all = w ? 1 : 0;
   if (dropout <= 0.f && attention_weights_takes(W)) {

@@ -38,7 +38,7 @@ struct AttnWeightsP {
   const void *q, *k;   // [B][L][Nh][H1]
   void* P;
   int L, Nh, H1, batches;
-  float scale_log2;    // scale log2(e)
+  float scale;
   int causal, zero_all;
   int xcd, qt;         // tiles of queries
 };

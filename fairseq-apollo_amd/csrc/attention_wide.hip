@@ -166,7 +166,7 @@ __global__ __launch_bounds__(256, 2) void attn_weights_kernel(const AttnWeightsP
     for (int s = 0; s < KS; ++s) fq[j][s] = *(const uint4*)(Q + min(q0 + 16 * j + n, A.L - 1) * rs + s * 32 + g * 8);
   const int seen = A.causal ? min(A.L, q0 + BQ) : A.L;             // keys that any of the rows sees
   const int tiles = (seen + BK - 1) / BK;
-  // scores (times log2 e) of the tile of keys from k0 on: key k0 + 16 kb + 4 g + u of query q0 + 16 j + n; invisible: -inf
+  // scores of the tile of keys from k0 on: key k0 + 16 kb + 4 g + u of query q0 + 16 j + n; invisible: -inf
   auto scores = [&](const int k0, f32x4 (&S)[KB][FQ]) {
     uint4 fk[KB][KS];
 #pragma unroll
@@ -188,7 +188,7 @@ __global__ __launch_bounds__(256, 2) void attn_weights_kernel(const AttnWeightsP
 #pragma unroll
       for (int j = 0; j < FQ; ++j)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) S[kb][j][u] *= A.scale_log2;
+        for (int u = 0; u < 4; ++u) S[kb][j][u] *= A.scale;
     if (edge) {
 #pragma unroll
       for (int j = 0; j < FQ; ++j) {
@@ -206,10 +206,12 @@ __global__ __launch_bounds__(256, 2) void attn_weights_kernel(const AttnWeightsP
     mx[j] = -INFINITY;
     sum[j] = 0.f;
   }
+  // e^(s - m), s <= m: the difference is scaled for exp2, not the scores, which may be anything in 32 bits
+  auto expd = [](float s, float m) { return __builtin_amdgcn_exp2f((s - m) * 1.4426950408889634f); };
   // two parts of a row: (m, l) takes (m2, l2) in
-  auto join = [](float& m, float& l, float m2, float l2) {
+  auto join = [&](float& m, float& l, float m2, float l2) {
     const float both = fmaxf(m, m2), from = both == -INFINITY ? 0.f : both;
-    l = l * __builtin_amdgcn_exp2f(m - from) + l2 * __builtin_amdgcn_exp2f(m2 - from);
+    l = l * expd(m, from) + l2 * expd(m2, from);
     m = both;
   };
   f32x4 S[KB][FQ];
@@ -228,8 +230,8 @@ __global__ __launch_bounds__(256, 2) void attn_weights_kernel(const AttnWeightsP
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) l += __builtin_amdgcn_exp2f(S[kb][j][u] - from);
-      sum[j] = sum[j] * __builtin_amdgcn_exp2f(mx[j] - from) + l;
+        for (int u = 0; u < 4; ++u) l += expd(S[kb][j][u], from);
+      sum[j] = sum[j] * expd(mx[j], from) + l;
       mx[j] = m;
     }
   }
@@ -285,7 +287,7 @@ __global__ __launch_bounds__(256, 2) void attn_weights_kernel(const AttnWeightsP
         for (int e = 0; e < 2; ++e) {
           float v[4];
 #pragma unroll
-          for (int u = 0; u < 4; ++u) v[u] = __builtin_amdgcn_exp2f(S[kb + e][j][u] - from[j]) * inv[j];
+          for (int u = 0; u < 4; ++u) v[u] = expd(S[kb + e][j][u], from[j]) * inv[j];
           if (odd) {
 #pragma unroll
             for (int u = 0; u < 4; ++u)
@@ -333,8 +335,8 @@ void attention_wide_launch(AttnWideP P, AttnWide kind, bool bf16, hipStream_t s)
 // Rows of at most 256 keys, which a workgroup's waves take in one turn, and products that give every compute unit a workgroup:
 // fewer workgroups with longer rows are a chain of turns (2.7 us each with one wave on a SIMD), where the scores' own
 // product has more tiles.  us, product and softmax beside this kernel, entries x positions x width (causal, full):
-//      1 x  256 x 128     9.1, 8.9     9.0, 8.8       16 x 1024 x  64    33.8, 20.7    40.9, 21.3
-//      8 x  256 x  64     9.4, 7.5     9.6, 7.2       16 x 2048 x 128    85.4, 49.4     159, 71.9
+//      1 x  256 x 128     9.1, 9.2     9.0, 9.1       16 x 1024 x  64    33.8, 21.1    40.9, 21.6
+//      8 x  256 x  64     9.4, 7.7     9.6, 7.5       16 x 2048 x 128    85.4, 49.1     159, 72.1
 //      1 x  512 x 128     9.6, 14.2 (not)              4 x 2048 x 128    30.5, 39.5    39.8, 40.4 (not)
 //      8 x 1024 x 128    24.4, 25.2 (not)              2 x 4096 x 128    99.7, 68.9     156, 71.5 (missed)
 // Width 256: fragments from memory for half as many queries; 8 x 1024 x 256 24.5, 31.3 (not).

@@ -674,6 +674,28 @@ def test_attention_weights_in_one_pass(dtype, B, L, Nh, H1, causal):
     assert bool(torch.isnan(w3[0, 0, bad, :seen]).all()) and not bool(w3[0, 0, bad, seen:].any())
 
 
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+@pytest.mark.parametrize("B,L,H1,causal", [(2, 64, 64, True), (1, 256, 128, False), (33, 512, 64, True)])
+def test_attention_weights_of_the_largest_scores(B, L, H1, causal, sign):
+    """Scores up to 3.2e38 are numbers like any others (times log2(e) they would not be): equal ones share their rows, one of
+    2^127 beside smaller ones has its row to itself."""
+    q = torch.full((B, L, 1, H1), sign * 2.0 ** 60, dtype=torch.bfloat16, device="cuda:0")
+    k = torch.full((B, L, 1, H1), 1.8125 * 2.0 ** 67 / H1, dtype=torch.bfloat16, device="cuda:0")      # 3.08e38
+    v = torch.zeros(B, L, 1, 8, dtype=torch.bfloat16, device="cuda:0")
+    _, w = M.ops.attention_fwd(q, k, v, 1.0, 0.0, causal, need_weights=True)
+    seen = torch.arange(1, L + 1, device="cuda:0")[:, None] if causal else torch.full((L, 1), L, device="cuda:0")
+    want = torch.where(torch.arange(L, device="cuda:0")[None] < seen, 1.0 / seen, 0.0)
+    assert bool(((w[:, 0].float() - want).abs() <= 2.0 ** -8 * want).all())
+    k[:, 1::2] *= 0.75
+    k[:, 0::4] *= 0.5
+    k[0, 5] = 2.0 ** 67 / H1 * (1.0 if sign > 0 else 0.25)
+    _, w = M.ops.attention_fwd(q, k, v, 1.0, 0.0, causal, need_weights=True)
+    s = (q.double()[:, :, 0] @ k.double()[:, :, 0].transpose(1, 2))
+    if causal:
+        s = s.masked_fill(torch.arange(L, device="cuda:0")[None] >= seen, float("-inf"))
+    assert bool(((w[:, 0].double() - s.softmax(-1)).abs() <= 2.0 ** -8 * s.softmax(-1)).all())
+
+
 def test_attention_bwd_entry_point_refuses_what_it_does_not_cover():
     """fp32 and head sizes that are not multiples of 8 take the batched library products in ops.attention_bwd; the
     entry point itself says so instead of computing something else."""
