@@ -1381,6 +1381,8 @@ class EmbeddingFunc(torch.autograd.Function):
     def forward(ctx, ids, weight, padding_idx):
         ctx.save_for_backward(ids)
         ctx.rows, ctx.padding_idx = weight.shape[0], padding_idx
+        if padding_idx is not None and padding_idx < 0:  # (from the table's end, as F.embedding takes it)
+            ctx.padding_idx += weight.shape[0]
         return F.embedding(ids, weight, padding_idx)
 
     @staticmethod

@@ -222,3 +222,15 @@ def test_split_keeps_its_gradient_buffer_or_concatenates():
     first = b.grad.clone()
     loss.backward()
     assert torch.equal(b.grad, 2 * first)
+
+
+@pytest.mark.parametrize("padding", [None, 2, -1, -7])
+def test_embedding_gradient_of_a_padding_row(padding):
+    """The padding row counts from the table's end where it is negative, in the gradient as in F.embedding (here the form that
+    a graph over the backward pass takes)."""
+    ids = torch.tensor([[0, 2, 6, 6], [5, 2, 0, 3]])
+    w = torch.randn(7, 5, requires_grad=True)
+    dy = torch.randn(2, 4, 5)
+    ours, = torch.autograd.grad(M.modules.EmbeddingFunc.apply(ids, w, padding), w, dy, create_graph=True)
+    theirs, = torch.autograd.grad(torch.nn.functional.embedding(ids, w, padding), w, dy)
+    assert torch.equal(ours, theirs)
