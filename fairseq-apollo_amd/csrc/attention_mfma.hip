@@ -1373,6 +1373,8 @@ bool attention_mfma_covers(int dtype, const void* q, const void* k, const void* 
   return true;
 }
 
+// (what the largest of its ways needs: the weights' one kernel leaves the scores' part unused, weights written where the caller
+// wants them the probabilities', v read in place its transposed copy)
 size_t attention_mfma_workspace_bytes(int dtype, int64_t B, int64_t L, int64_t Nh, int64_t H2) {
   const int64_t Lp = (L + 7) / 8 * 8;
   const size_t es = dtype == MEGA_F32 ? 4 : 2;

@@ -446,7 +446,9 @@ template <typename T, int NX, bool F16, bool VEC, bool BOTH>
 int launch_rows_v(const RowsArgs& A, hipStream_t s) {
   static uint64_t attr_seen = 0;
   // two directions want 150 registers: workgroups of few waves may have them (8 x 256 x 1024, two-sided 8.6 us, 9.9 at 128);
-  // one direction is quicker with more waves beside each other (4 x 1024 x 2048 fp16 15.3, 16.8)
+  // one direction is quicker with more waves beside each other (4 x 1024 x 2048 fp16 15.3, 16.8).  Longer rows have up to 16
+  // waves a workgroup and so 128 registers: with four tokens an access 9 of them (fp32), 10 (fp16) or 4 (bf16) live in scratch
+  // with two directions, 4 with one (fp32, fp16).
   auto kern = ema_rows_kernel<T, NX, F16, VEC, BOTH, kRMost>;
   if constexpr (BOTH) {
     if (A.S <= 4) kern = ema_rows_kernel<T, NX, F16, VEC, BOTH, 4>;

@@ -1059,6 +1059,8 @@ struct Plan {
   size_t coef_bytes, st_bytes, acc_bytes, tile_bytes, image_bytes, total;
 };
 
+// What the largest of the ways needs: the matrix-core rows (ema_rows.hip) use the image alone, neither chunk states nor
+// partial sums.
 Plan make_plan(int64_t B, int64_t D, int64_t N, int64_t L, int nsets, bool need_acc, bool bidirectional = false) {
   Plan pl;
   int tpr = 1;

@@ -171,7 +171,7 @@ __device__ __forceinline__ uint4 eight(const uint32_t (&p)[4]) {
 //
 // Branches between the blocks keep one block's loads and exponentials from running beside the next one's, so the frequent
 // kinds are whole: 0 the sums alone, 1 with a bias, 2 with a residual, 3 silu of 1, 4 anything (8192 x 2048 x 1024: 31, 31, 38,
-// 34 us; residual and silu with branches 41 and 39).
+// 36 us; residual and silu with branches 41 and 39, silu by the bare reciprocal 34).
 template <typename T, bool ACC, int KIND, bool EDGE, int FM, int FN>
 __device__ __forceinline__ void store_wave(const Gemm16P& G, const Place& p, int wm, int wn, int lane, const f32x4 (&acc)[FM][FN]) {
   const int g = lane >> 4, row = wm * 16 + (lane & 15), col = wn * 16;

@@ -9,6 +9,10 @@ extern template void launch_wide_type<f16_t>(const Gemm16P&, const WidePlan&, in
 // The tile and the split with the least estimated time.  Whole rounds of tiles (one on each compute unit) run unsplit; what is
 // left over is split along the reduction over the idle units, into fp32 partial sums that a second kernel adds up.  In us:
 // 1.4 a step and 10 a round with square tiles, 0.85 and 6 with tall ones, 5 and its traffic at 4 TB/s for the second kernel.
+// High by 5 - 25 % of what warm operands take, for both kinds alike (8192 x 4352 x 1024 94.8, 77.3; 8192 x 2816 x 1024 58.8, 47.4;
+// 8192 x 2048 x 2048 54.8, 52.0; 5000 x 1024 x 2048 33.2, 26.1), nearer with operands from memory (88.4, 61.5, -, 31.3): fit to
+// compare plans, with each other and with the 64 x 64 tiles' estimate, not to tell times.  The parts take up to 200 MB of a call's
+// workspace (192 tiles beside whole rounds, in four).
 WidePlan gemm16_wide_plan(int64_t M, int64_t N, int64_t K) {
   const int64_t cus = device_cu_count(), steps = ceil_div(K, kKS);
   WidePlan best = {};

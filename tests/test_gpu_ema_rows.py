@@ -135,11 +135,13 @@ def test_kernel_generation_inside_the_call(dtype, B, D, layout):
 
 
 @pytest.mark.parametrize("bidir", [False, True])
-@pytest.mark.parametrize("B,D,L", [(3, 7, 64), (3, 7, 1024), (5, 3, 1025), (3, 5, 2048), (1, 5, 3000), (2, 3, 4096), (1, 3, 4100), (1, 1, 15363)])
+@pytest.mark.parametrize("B,D,L", [(3, 7, 64), (3, 7, 1024), (5, 3, 1025), (3, 5, 2048), (1, 5, 3000), (2, 3, 4096), (1, 3, 4100), (1, 3, 6000), (2, 1, 9216),
+                                   (1, 1, 15360), (1, 1, 15363)])
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_rows_of_every_number_of_blocks(dtype, B, D, L, bidir):
-    """One to fifteen blocks a row; several rows a workgroup, the last one with fewer; lengths in whole and partial blocks, in
-    tokens by four and one by one; padding at the end and inside; states of sixteen poles that reach across the row."""
+    """One, two, three, four, five, six, nine, fifteen and sixteen blocks a row; several rows a workgroup, the last one with
+    fewer; lengths in whole and partial blocks, in tokens by four and one by one; padding at the end and inside; states of
+    sixteen poles that reach across the row."""
     rng = np.random.default_rng(L)
     p, q, g = _coeffs(rng, 2 * D if bidir else D, 16, True)
     om = rng.normal(size=D)

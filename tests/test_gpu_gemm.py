@@ -325,18 +325,39 @@ def test_16bit_products_on_wide_tiles(dtype, ka, kb, m, n, k):
 
 @pytest.mark.parametrize("bias,res,silu,pre", [(1, 0, 0, 0), (0, 1, 0, 0), (1, 0, 1, 0), (1, 1, 1, 1), (0, 0, 1, 1), (1, 0, 0, 1)])
 @pytest.mark.parametrize("m,n,k", [(1096, 4360, 1032), (1032, 1048, 8200), (6144, 2816, 1024)])
-def test_16bit_epilogues_on_wide_tiles(m, n, k, bias, res, silu, pre):
+@pytest.mark.parametrize("dtype,ka,kb", [(torch.bfloat16, 0, 0), (torch.float16, 0, 0), (torch.bfloat16, 0, 1), (torch.float16, 1, 1)])
+def test_16bit_epilogues_on_wide_tiles(dtype, ka, kb, m, n, k, bias, res, silu, pre):
+    """Every way a value is finished, whole tiles and edges, in both types and three orders; with a residual also into the
+    residual's own memory."""
     gen = torch.Generator(DEV).manual_seed(8)
-    mk = lambda *s: torch.randn(*s, generator=gen, device=DEV).to(torch.bfloat16)
+    mk = lambda *s: torch.randn(*s, generator=gen, device=DEV).to(dtype)
     a, b, v, x = mk(m, k), mk(n, k), mk(n) * 30, mk(m, n) * 30
     r = a.double() @ b.double().t() + bias * v.double() + res * x.double()
-    got = _gemm(a, b, 0, 0, v if bias else None, x if res else None, bool(silu), bool(pre))
+    a, b = a.t().contiguous() if ka else a, b.t().contiguous() if kb else b
+    got = _gemm(a, b, ka, kb, v if bias else None, x if res else None, bool(silu), bool(pre))
     c, p = got if pre else (got, None)
-    tol = 2.0 ** -9 + _tol(k)
+    half = 2.0 ** -9 if dtype is torch.bfloat16 else 2.0 ** -12
+    tol = half + _tol(k)
     if pre:
         assert _rel(p, r) < tol
     # silu of the rounded value (known where it is written as well; its slope is at most 1.1), rounded again
-    assert _rel(c, F.silu(p.double() if pre else r) if silu else r) < (2.0 ** -9 + 2.0 ** -22 if pre and silu else 3 * tol if silu else tol)
+    assert _rel(c, F.silu(p.double() if pre else r) if silu else r) < (half + 2.0 ** -22 if pre and silu else 3 * tol if silu else tol)
+    if res and not pre:
+        _call(a, b, x, ka, kb, v if bias else None, x, bool(silu))
+        assert torch.equal(x, c)
+
+
+def test_16bit_workspace_too_small():
+    """Wide tiles in parts refuse a workspace that does not hold them, and write nothing."""
+    m, n, k = 1032, 1048, 8200
+    lib, need = M._lib.load(), M._lib.load().mega_gemm16_workspace_bytes(m, n, k)
+    a, b, c = torch.ones(m, k, device=DEV, dtype=torch.bfloat16), torch.ones(n, k, device=DEV, dtype=torch.bfloat16), torch.zeros(m, n, device=DEV, dtype=torch.bfloat16)
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    g = _Gemm(a.data_ptr(), b.data_ptr(), c.data_ptr(), None, None, None, k, k, n, 0, 0, 0, 0, 0, 0, 0, m, n, k, 1, 1, 0, 0, 0, 0, 1.0, 0)
+    for have, at in ((need - 1, ws.data_ptr()), (need, None)):
+        assert need > 0 and lib.mega_gemm16(C.byref(g), 1, at, have, torch.cuda.current_stream().cuda_stream) != 0
+    torch.cuda.synchronize()
+    assert not bool(c.any())
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
