@@ -247,8 +247,12 @@ bool gemm16_wide(int64_t M, int64_t N, int64_t K, WidePlan* p) {
 //                2816 x 1024 x 2048   29.3, 26.2    16384 x 16384 x 16384*  6315, 7585
 // x W^T in whole tiles: the library is 6 % ahead on average (127 sizes), but where its tiles leave a partial round behind more than
 // two whole ones, 6 % behind (33 sizes, 0.89 to 1.56).  Its call costs the host 26 us, so that calls made of products below
-// 20 GFLOP (20 us and less) are bound by the host with it: a layer of 2048 tokens of 1024 channels 217 us, 299 with the
-// library; beyond, the device is the bound: 5000 tokens of 2048 channels 1032 with all of them here, 947 in the library.  N not
+// 20 GFLOP (20 us and less) are bound by the host with it, and those of up to 4096 tokens, with less beside the products, below
+// 40 GFLOP; beyond, the device is the bound: 5000 tokens of 2048 channels 1032 with all of them here, 947 in the library.  us of
+// whole calls, those of 20 to 40 GFLOP in the library and here:
+//   model, width 1024   3 x 1000   540, 507     8 x 461   577, 520     4 x 1024   585, 580     1 x 5000   673, 678 (not)     2 x 2991   751, 755 (not)
+//   layer   4096 x 1024   307, 297     1024 x 2048   319, 301     1536 x 2048   355, 377     2560 x 2048   497, 498     5120 x 1024   350, 351 (not)
+// (below: a layer of 2048 tokens of 1024 channels 299 with the library, 217.  Missed: 2048 x 2048, 473, all of them here 448.)  N not
 // in whole tiles: 10 - 25 % ahead to 200 GFLOP, even to 400.  silu: ahead by the pass, whose share is 1 / K.  dY W is even to
 // 130 GFLOP, 2 - 5 % ahead beyond, dY^T X 20 - 70 % ahead.  Nothing is measured beyond 1e13.
 bool gemm16_wins(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor, bool silu) {
@@ -256,7 +260,7 @@ bool gemm16_wins(int64_t M, int64_t N, int64_t K, int a_kmajor, int b_kmajor, bo
   if (a_kmajor || b_kmajor) return flops <= 1e13;
   if (silu && K <= 4096) return flops <= 2.5e12;
   const int64_t tiles = ceil_div(M, kWideM) * ceil_div(N, 256), round = device_cu_count();
-  return flops <= (N % 256 || (tiles > 2 * round && tiles % round) ? 5e11 : 2e10);
+  return flops <= (N % 256 || (tiles > 2 * round && tiles % round) ? 5e11 : M <= 4096 ? 4e10 : 2e10);
 }
 
 // Sizes that the kernels hold in 32 bits, tiles that a launch takes (2^32 threads)

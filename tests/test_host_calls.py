@@ -186,7 +186,7 @@ def test_the_limit_of_16bit_products_stands_once():
 
 
 @pytest.mark.parametrize("m,n,k,order,silu,own", [
-    (2048, 4096, 1024, 0, 0, 1), (5000, 2048, 1024, 0, 0, 0), (8192, 2816, 1024, 0, 0, 0), (8192, 2048, 5632, 0, 0, 0), (8192, 8192, 8192, 0, 0, 0),
+    (2048, 4096, 1024, 0, 0, 1), (5000, 2048, 1024, 0, 0, 0), (4096, 2816, 1024, 0, 0, 1), (4096, 2048, 4096, 0, 0, 0), (8192, 2816, 1024, 0, 0, 0), (8192, 2048, 5632, 0, 0, 0), (8192, 8192, 8192, 0, 0, 0),
     (8192, 4096, 2048, 0, 0, 0), (32768, 5632, 2048, 0, 0, 0), (12000, 2816, 1024, 0, 0, 1), (8192, 5632, 2048, 0, 0, 1), (16384, 8704, 2048, 0, 0, 0),
     (8192, 3264, 768, 0, 0, 1), (65536, 2056, 2048, 0, 0, 0), (5000, 2048, 1024, 0, 1, 1), (8192, 4096, 2048, 0, 1, 1),
     (8192, 4096, 8192, 0, 1, 0), (2048, 512, 8192, 0, 1, 1), (1 << 29, 136, 8, 0, 1, 0), (8192, 2048, 5632, 1, 0, 1), (8192, 8192, 8192, 3, 0, 1)])
